@@ -67,10 +67,14 @@ class Sampler:
         if logits.dtype != torch.float32 or not logits.is_cuda or logits.numel() != self.V:
             raise _lib.RwkvHipError("sample() takes the fp32 logits [vocab] on the GPU")
         logits = logits.contiguous()
+        unif = self.u
         if u is None:
             self.u.uniform_(generator=self.gen)
         elif isinstance(u, torch.Tensor):
-            self.u.copy_(u.reshape(1))
+            if u.device == logits.device and u.dtype == torch.float32 and u.numel() == 1:
+                unif = u                       # read where it is: no copy launch in front of the draw (5 us)
+            else:
+                self.u.copy_(u.reshape(1))
         else:
             self.u.fill_(float(u))
         seen = self.seen.data_ptr() if penalties else None
@@ -80,7 +84,7 @@ class Sampler:
             self.ban.data_ptr() if self.ban is not None else None, 0 if self.ban is None else self.ban.numel(),
             seen, occ, self.weight.data_ptr() if (self.weight is not None and penalties) else None,
             float(alpha_presence), float(alpha_frequency), float(alpha_decay),
-            self.u.data_ptr(), self.probs.data_ptr(), self.token.data_ptr(), _stream())
+            unif.data_ptr(), self.probs.data_ptr(), self.token.data_ptr(), _stream())
         _lib.check(rc, "rwkv_sample_logits")
         return self.token
 

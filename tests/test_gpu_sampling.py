@@ -163,3 +163,41 @@ def test_greedy_token(vocab, dtype):
     assert L.rwkv_greedy_token(None, lib.RWKV_DT_F32, 8, out.data_ptr(), None) == -3
     assert L.rwkv_greedy_token(out.data_ptr(), lib.RWKV_DT_F32, 0, out.data_ptr(), None) == -1
     assert L.rwkv_greedy_token(out.data_ptr(), 7, 8, out.data_ptr(), None) == -5
+
+
+@pytest.mark.parametrize("vocab", [1, 5, 255, 1023, 4096, 4099, 50277, 65536])
+@pytest.mark.parametrize("kind", ["flat", "peaked", "equal", "banned"])
+def test_sample_edges(vocab, kind):
+    """The register groups of four, the last partial group row and both stages of the cut's search: vocabularies around
+    4, 256 and 4096 entries, logits nearly flat (tens of thousands of entries between the first bounds), peaked, all
+    equal, and all but one banned; pointers that are not 16-byte aligned take the scalar loads."""
+    from chatrwkv_amd.sampling import Sampler
+    x = logits_for(vocab, vocab, 0.05 if kind == "flat" else 4.0)
+    ban = ()
+    if kind == "equal":
+        x[:] = 0.75
+    if kind == "banned":
+        ban = [i for i in range(vocab) if i != vocab // 2][:4000]
+        x[vocab // 2] = 30.0
+    buf = torch.zeros(vocab + 1, dtype=torch.float32, device=DEV)
+    buf[1:] = torch.from_numpy(x).to(DEV)
+    adj = osamp.apply_penalties(x, ban)
+    for top_p, top_k in ((0.5, 0), (0.9, 0), (0.9, 20), (0.0, 0)):
+        if kind == "equal" and top_k:
+            continue                       # ties at the k-th place are kept here and cut arbitrarily in the reference
+        ref = osamp.filter_probs(adj, 1.0, top_p, top_k).astype(np.float64)
+        margin = _boundary_margin(adj, top_p, 1.0) if kind != "equal" else 1.0
+        probs = []
+        for logits in (torch.from_numpy(x).to(DEV), buf[1:]):
+            s = Sampler(vocab, device=DEV, token_ban=ban, seed=1)
+            for u in (0.0, 0.4321, 0.99999):
+                tok = int(s.sample(logits, 1.0, top_p, top_k, u=u))
+                got = s.probs.cpu().numpy().astype(np.float64)
+                _check_probs(got, ref, margin)
+                cdf = np.cumsum(got)
+                # fp32 running sums: off by at most the rounding of ~25 additions in a chain, 25 * 2^-24 of the total
+                slack = 25 * 2.0 ** -24 * cdf[-1]
+                assert got[tok] > 0 and cdf[tok] >= u * cdf[-1] - slack and cdf[tok] - got[tok] <= u * cdf[-1] + slack
+                assert int(s.seen[tok]) == 1
+            probs.append(got)
+        assert np.array_equal(probs[0], probs[1])
