@@ -362,19 +362,21 @@ __global__ __launch_bounds__(64 * WT * WM) void gemm_kernel(int T, int N, int M,
 // s_waitcnt: the compiler waits for lgkmcnt(0) wherever older and newer reads are both outstanding.
 // fp16 weights (W_U8 = false): the weight tile is laid out like the A tile (32 KB), a stage is 64 KB and two fit, so
 // one tile is in flight while one multiplies.
-// Tile TM x TN is 256 x 256 (wave tile 128 x 64: the long, wide products) or 128 x 128 (wave tile 64 x 32, a stage of
-// 24 KB: products with too few 256 x 256 tiles for the chip run at full depth with these instead of splitting K).
-// NW (waves per workgroup: 8, or 4 with 64 x 64 wave tiles) and NSTG (stages, 0 = the default above) exist for
-// tuning runs.  Measured on the 128 x 128 tile with uint8 weights: four waves of 64 x 64 (a third fewer fragment
-// reads per MFMA) 45.0 against 41.7 us on [1024 x 4096] x [4096 x 4096] and equal on launches of several rounds;
-// four and five stages (tiles three and four ahead) 42.6 against 42.8 us, and 4-6 % slower on launches of several
-// rounds, where only one workgroup then fits a CU.  Neither fragment reads nor load latency bound that tile.
-constexpr int DT = 256, DM = 256;
+// Tile TM x TN is 256 x 256 (wave tile 128 x 64: the long, wide products), 128 x 128 (wave tile 64 x 32, a stage of
+// 24 KB: products with too few 256 x 256 tiles for the chip run at full depth with these instead of splitting K) or
+// 64 x 128 (four waves of 64 x 32, a stage of 16 KB: calls of up to 64 rows, which are HBM bound -- with 128 rows two
+// thirds of the bytes in flight were copies of the last row).  NSTG: stages, 0 = the default above.
+// Measured (uint8, us, scaling pass included): four stages instead of three on the 128 x 128 tile [256 x 4096] x
+// [4096 x 12288] 46.3 -> 41, [256 x 4096] x [4096 x 4096] at full depth 45.6 -> 37.4, [1024 x 4096] x [4096 x 4096]
+// 51.9 -> 50.0; 5 % slower where the tiles take several rounds, as only one workgroup then fits a CU.  64 x 128 tile at
+// 64 rows: [4096 x 12288] 29.5 -> 24.4, [4096 x 20480] 44.1 -> 35.3, [16384 x 4096] 34.6 -> 29.1, [4096 x 4096] 19.1 -> 17.5.
+// Not faster on the 128 x 128 tile: four waves of 64 x 64 (45.0 against 41.7 us on [1024 x 4096] x [4096 x 4096]), and
+// eight waves of 64 x 64 that halve K between them (40 % fewer fragment reads: 48.1 against 50.0, several rounds slower).
 template <bool W_U8, int TM, int TN, int NW = 8, int NSTG = 0> struct DmaCfg {
     static constexpr int A = TM * BK * 2, W = W_U8 ? TN * BK : TN * BK * 2, STAGE = A + W;
     static constexpr int NST = NSTG ? NSTG : (W_U8 || TM < 256) ? 3 : 2;
     static constexpr int AL = A / 1024 / NW, WL = W / 1024 / NW, LOADS = AL + WL;   // 1 KB loads per wave and tile
-    static constexpr int WR = 2, WC = NW / 2;                            // waves: 2 rows x 4 (or 2) columns
+    static constexpr int WR = TM >= 128 ? 2 : 1, WC = NW / WR;           // waves: 2 rows x 4 columns; 64-row tile: 1 x 4
     static constexpr int MI = TM / (32 * WR), NI = TN / (32 * WC);       // 32 x 32 blocks per wave
     static constexpr int STG_STRIDE = TN + 8;   // epilogue staging: 128 rows of TN floats, padded (see the epilogue)
     static constexpr size_t BODY = (size_t)NST * STAGE > (size_t)128 * STG_STRIDE * 4 ? (size_t)NST * STAGE : (size_t)128 * STG_STRIDE * 4;
@@ -390,7 +392,7 @@ DEV void gemm_dma_body(int T, int N, int M, const h16 *__restrict__ A, int64_t l
                        void *__restrict__ Y, int64_t ldy, const GemmEpi &ep, int nk_split, float *__restrict__ part, int split) {
     using Cfg = DmaCfg<W_U8, TM, TN, NW, NSTG>;
     constexpr int D_A = Cfg::A, D_STAGE = Cfg::STAGE, D_NST = Cfg::NST, AL = Cfg::AL, WL = Cfg::WL, MI = Cfg::MI, NI = Cfg::NI;
-    static_assert((TM == 256 || TM == 128) && (TN == 256 || TN == 128), "tile");
+    static_assert((TM == 256 || TM == 128 || TM == 64) && (TN == 256 || TN == 128), "tile");
     static_assert((NW == 8 || NW == 4) && 2 * TM <= 64 * NW && MI >= 2 && MI <= 4 && NI >= 1 && NI <= 2, "waves");
     extern __shared__ __align__(1024) unsigned char smem[];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -740,7 +742,7 @@ DEV void gemm_dma_body(int T, int N, int M, const h16 *__restrict__ A, int64_t l
         float *stg = (float *)smem;
         __syncthreads();   // every wave has read its last fragments
 #pragma unroll 1
-        for (int h = 0; h < TM / 128; ++h) {
+        for (int h = 0; h < (TM + 127) / 128; ++h) {
             if ((wr * WROWS) / 128 == h) {
 #pragma unroll
                 for (int b = 0; b < NI; ++b)
@@ -753,7 +755,7 @@ DEV void gemm_dma_body(int T, int N, int M, const h16 *__restrict__ A, int64_t l
             }
             __syncthreads();
 #pragma unroll 1
-            for (int it = 0; it < 128 / RPI; ++it) {
+            for (int it = 0; it < (TM < 128 ? TM : 128) / RPI; ++it) {
                 const int row = it * RPI + tid / CPR, t = t0 + h * 128 + row;
                 const bool valid = t < T && col_ok;
                 float a0 = 0.f, a2 = 0.f;
@@ -806,30 +808,30 @@ __global__ __launch_bounds__(64 * WT * WM) void gemm_group_kernel(int T, int N, 
 }
 
 // the same through the direct-to-LDS kernel; blockIdx.z is the k split when the group has too few tiles for the chip
-template <bool W_U8, bool SPLIT, int TM, int TN>
-__global__ __launch_bounds__(512) void gemm_dma_group_kernel(int T, int N, GemmGroup g) {
+template <bool W_U8, bool SPLIT, int TM, int TN, int NW, int NSTG>
+__global__ __launch_bounds__(64 * NW) void gemm_dma_group_kernel(int T, int N, GemmGroup g) {
     const int gi = blockIdx.y, M = g.M[gi];
-    gemm_dma_body<W_U8, SPLIT, TM, TN>(T, N, M, g.A[gi], g.lda, g.W[gi], g.ldw[gi], g.Y[gi], M, g.ep[gi], SPLIT ? g.nk_split : N / BK,
+    gemm_dma_body<W_U8, SPLIT, TM, TN, NW, NSTG>(T, N, M, g.A[gi], g.lda, g.W[gi], g.ldw[gi], g.Y[gi], M, g.ep[gi], SPLIT ? g.nk_split : N / BK,
                                        g.part[gi], SPLIT ? blockIdx.z : 0);
 }
 
-template <bool W_U8, int TM, int TN>
+template <bool W_U8, int TM, int TN, int NW, int NSTG>
 int launch_dma_group(const GemmGroup &g, int n, int64_t T, int64_t N, int64_t grid_x, int ks, hipStream_t st) {
-    constexpr size_t lds = DmaCfg<W_U8, TM, TN>::LDS;
+    constexpr size_t lds = DmaCfg<W_U8, TM, TN, NW, NSTG>::LDS;
     static PerDeviceOnce once;
     bool *attr_done = once.slot();
     if (!attr_done || !*attr_done) {
-        hipError_t e = hipFuncSetAttribute((const void *)gemm_dma_group_kernel<W_U8, false, TM, TN>,
+        hipError_t e = hipFuncSetAttribute((const void *)gemm_dma_group_kernel<W_U8, false, TM, TN, NW, NSTG>,
                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e == hipSuccess)
-            e = hipFuncSetAttribute((const void *)gemm_dma_group_kernel<W_U8, true, TM, TN>, hipFuncAttributeMaxDynamicSharedMemorySize,
+            e = hipFuncSetAttribute((const void *)gemm_dma_group_kernel<W_U8, true, TM, TN, NW, NSTG>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                     (int)lds);
         if (e != hipSuccess) return (int)e;
         if (attr_done) *attr_done = true;
     }
     const dim3 grid((unsigned)grid_x, (unsigned)n, (unsigned)ks);
-    if (ks > 1) hipLaunchKernelGGL((gemm_dma_group_kernel<W_U8, true, TM, TN>), grid, dim3(512), lds, st, (int)T, (int)N, g);
-    else hipLaunchKernelGGL((gemm_dma_group_kernel<W_U8, false, TM, TN>), grid, dim3(512), lds, st, (int)T, (int)N, g);
+    if (ks > 1) hipLaunchKernelGGL((gemm_dma_group_kernel<W_U8, true, TM, TN, NW, NSTG>), grid, dim3(64 * NW), lds, st, (int)T, (int)N, g);
+    else hipLaunchKernelGGL((gemm_dma_group_kernel<W_U8, false, TM, TN, NW, NSTG>), grid, dim3(64 * NW), lds, st, (int)T, (int)N, g);
     return RWKV_OK;
 }
 
@@ -1194,36 +1196,63 @@ bool dma_ok(bool w_u8, int64_t N, int64_t M, const void *A, int64_t lda, const v
     return true;
 }
 
-// Cost model of a direct-to-LDS launch in microseconds, fitted to launches of the 7B shapes (256 to 4096 rows):
+// The direct-to-LDS tiles: rows and columns.  TILE_S4 is TILE_S with four stages.
+enum { TILE_L, TILE_S, TILE_S4, TILE_N, TILES };
+struct TileDim { int tm, tn; };
+constexpr TileDim tile_dim[TILES] = {{256, 256}, {128, 128}, {128, 128}, {64, 128}};
+
+// Cost model of a direct-to-LDS launch in microseconds, fitted to launches of the 7B shapes (20 to 4096 rows):
 // `tiles` tiles of nk k-tiles split c ways run in whole rounds over the 256 CUs; a k-tile step takes 1.75 us with
-// the 256 x 256 tile and 0.573 us with the 128 x 128 one (a quarter of the work in a third of the time); every
-// round adds its fill, drain and epilogue (10 steps; 4.3 for a split launch, whose epilogue is the reduction pass;
-// 12.8 for the small tile, 5.5 where two workgroups per CU overlap); the reduction pass of a split takes 2.5 us
-// + 3.6 us per slab and 16 MB of fp32 output, at least 4.5 us.
-double dma_cost(int64_t tiles, int nk, int c, bool small_tile, size_t out_bytes) {
-    const int64_t rounds = (tiles * c + 255) / 256;
-    const double step = small_tile ? 0.573 : 1.75;
-    const double extra = small_tile ? (rounds > 1 ? 5.5 : 12.8) : (c > 1 ? 4.3 : 10.0);
-    return (double)rounds * (nk / c + extra) * step + (c > 1 ? std::max(4.5, 2.5 + 3.6 * c * (double)out_bytes / (16 << 20)) : 0.0);
+// the 256 x 256 tile, 0.573 us with the 128 x 128 one (a quarter of the work in a third of the time) and 0.327 us with
+// the 64 x 128 one; every round adds its fill, drain and epilogue (10 steps; 4.3 for a split launch, whose epilogue is
+// the reduction pass; 12.8 for the 128 x 128 tile, 5.5 where two workgroups per CU overlap; 16.5 for the 64 x 128 one).
+// Four stages: launches of one round only (one workgroup per CU); its step grows from 0.38 us with 64 CUs busy to
+// 0.53 us with all of them.  The reduction pass of a split takes 2.5 us + 3.6 us per slab and 16 MB of fp32 output, at
+// least 4.5 us.
+double dma_cost(int tile, int64_t T, int64_t tiles, int nk, int c, size_t out_bytes) {
+    const int64_t wgs = tiles * c, rounds = (wgs + 255) / 256;
+    const double reduce = c > 1 ? std::max(4.5, 2.5 + 3.6 * c * (double)out_bytes / (16 << 20)) : 0.0;
+    switch (tile) {
+        case TILE_L: return (double)rounds * (nk / c + (c > 1 ? 4.3 : 10.0)) * 1.75 + reduce;
+        case TILE_S: return (double)rounds * (nk / c + (rounds > 1 ? 5.5 : 12.8)) * 0.573 + reduce;
+        case TILE_S4: return rounds > 1 ? 1e30 : (nk / c + 22.0) * (0.34 + 0.19 * (double)wgs / 256) + reduce;
+        default: return T > 64 ? 1e30 : (double)rounds * (nk / c + 16.5) * 0.327 + reduce;
+    }
 }
 
 // the K split (1..8, whole k-tiles, at least 8 per split, slabs within ws_bytes) of least cost
-int dma_split(int64_t tiles, int nk, bool small_tile, size_t out_bytes, size_t ws_bytes, double *cost = nullptr) {
+int dma_split(int tile, int64_t T, int64_t tiles, int nk, size_t out_bytes, size_t ws_bytes, double *cost = nullptr) {
     int best = 1;
     double best_cost = 1e30;
     for (int c = 1; c <= 8; ++c) {
         if (nk % c || (c > 1 && nk / c < 8) || (c > 1 && c * out_bytes > ws_bytes)) continue;
-        const double k = dma_cost(tiles, nk, c, small_tile, out_bytes);
+        const double k = dma_cost(tile, T, tiles, nk, c, out_bytes);
         if (k < best_cost) { best_cost = k; best = c; }
     }
     if (cost) *cost = best_cost;
     return best;
 }
 
-// gemm_dma_kernel.  Fewer than 192 tiles (narrow outputs): the contraction is split over workgroups of the same
-// tile until about one workgroup per CU is in flight; slabs and the second pass as in launch_cfg.
-template <bool W_U8, int TM, int TN, int NW = 8, int NSTG = 0>
-int launch_dma(int64_t T, int64_t N, int64_t M, const rwkv_half *A, int64_t lda, const void *W, int64_t ldw, void *Y,
+// the tile of least cost for products of M_i outputs (n of them, one launch); ks: its K split
+int dma_tile(int64_t T, int nk, int n, const int64_t *M, size_t ws_bytes, int *ks) {
+    int best = TILE_S;
+    double best_cost = 1e30;
+    int64_t outs = 0;
+    for (int i = 0; i < n; ++i) outs += M[i];
+    for (int tile = 0; tile < TILES; ++tile) {
+        const TileDim d = tile_dim[tile];
+        int64_t tiles = 0;
+        for (int i = 0; i < n; ++i) tiles += ((T + d.tm - 1) / d.tm) * ((M[i] + d.tn - 1) / d.tn);
+        double c;
+        const int k = dma_split(tile, T, tiles, nk, (size_t)(T * outs) * sizeof(float), ws_bytes, &c);
+        if (c < best_cost) { best_cost = c; best = tile; *ks = k; }
+    }
+    return best;
+}
+
+// gemm_dma_kernel with K split ks ways (slabs and the second pass as in launch_cfg).
+template <bool W_U8, int TM, int TN, int NW, int NSTG>
+int launch_dma(int ks, int64_t T, int64_t N, int64_t M, const rwkv_half *A, int64_t lda, const void *W, int64_t ldw, void *Y,
                int64_t ldy, const GemmEpi &ep, hipStream_t st) {
     constexpr size_t lds = DmaCfg<W_U8, TM, TN, NW, NSTG>::LDS;
     static PerDeviceOnce once;
@@ -1238,8 +1267,6 @@ int launch_dma(int64_t T, int64_t N, int64_t M, const rwkv_half *A, int64_t lda,
     if (!dma_ok(W_U8, N, M, A, lda, W, ldw, Y, ldy, ep)) return RWKV_E_LAYOUT;
     const int64_t tiles = ((T + TM - 1) / TM) * ((M + TN - 1) / TN);
     const int nk = (int)(N / BK);
-    int ks = 1;
-    if (ep.splitk_ws && (M & 3) == 0) ks = dma_split(tiles, nk, TM < 256, (size_t)T * M * sizeof(float), ep.splitk_bytes);
     if (ks > 1) {
         hipLaunchKernelGGL((gemm_dma_kernel<W_U8, true, TM, TN, NW, NSTG>), dim3((unsigned)tiles, (unsigned)ks), dim3(64 * NW), lds, st, (int)T, (int)N,
                            (int)M, (const h16 *)A, lda, W, ldw, Y, ldy, ep, nk / ks, ep.splitk_ws);
@@ -1254,39 +1281,40 @@ int launch_dma(int64_t T, int64_t N, int64_t M, const rwkv_half *A, int64_t lda,
     return RWKV_OK;
 }
 
+constexpr int CFG_DMA = 16;   // + TILE_*
 template <bool W_U8>
-int launch_pick(int cfg, int64_t T, int64_t N, int64_t M, const rwkv_half *A, int64_t lda, const void *W, int64_t ldw,
+int launch_pick(int cfg, int ks, int64_t T, int64_t N, int64_t M, const rwkv_half *A, int64_t lda, const void *W, int64_t ldw,
                 void *Y, int64_t ldy, const GemmEpi &ep, hipStream_t st) {
     switch (cfg) {
         case 3: return launch_cfg<W_U8, 128, 128, 2, 2, 4>(T, N, M, A, lda, W, ldw, Y, ldy, ep, st);
         case 9:
             if constexpr (W_U8) return launch_cfg<true, 256, 256, 4, 4, 2>(T, N, M, A, lda, W, ldw, Y, ldy, ep, st);
             return RWKV_E_DTYPE;
-        case 14: return launch_dma<W_U8, 256, 256>(T, N, M, A, lda, W, ldw, Y, ldy, ep, st);
-        case 15: return launch_dma<W_U8, 128, 128>(T, N, M, A, lda, W, ldw, Y, ldy, ep, st);
+        case CFG_DMA + TILE_L: return launch_dma<W_U8, 256, 256, 8, 0>(ks, T, N, M, A, lda, W, ldw, Y, ldy, ep, st);
+        case CFG_DMA + TILE_S: return launch_dma<W_U8, 128, 128, 8, 0>(ks, T, N, M, A, lda, W, ldw, Y, ldy, ep, st);
+        case CFG_DMA + TILE_S4: return launch_dma<W_U8, 128, 128, 8, 4>(ks, T, N, M, A, lda, W, ldw, Y, ldy, ep, st);
+        case CFG_DMA + TILE_N: return launch_dma<W_U8, 64, 128, 4, 4>(ks, T, N, M, A, lda, W, ldw, Y, ldy, ep, st);
         default: return RWKV_E_DTYPE;
     }
 }
 
-// Tile choice (RWKV_GEMM_CFG overrides it for tuning sweeps).
-//   14 / 15  operands laid out for 16-byte loads: the direct-to-LDS kernel with 256 x 256 or 128 x 128 tiles,
-//            whichever the cost model puts first (large tiles where they fill the chip, small ones at full depth
-//            where the large ones would have to split K; small ones when another product runs beside this one)
-//    9       uint8 weights otherwise, where 256 x 256 tiles of the register-staged kernel fill the chip: one per CU
-//            and round, the last round at least 70 % full
-//    3       everything else: 128 x 128 tiles, 4 k-tiles of prefetch
-int pick_cfg(int64_t T, int64_t N, int64_t M, bool w_u8, bool alone, bool dma, size_t split_bytes) {
-    const char *e = getenv("RWKV_GEMM_CFG");  // tuning override
-    if (e && *e) return atoi(e);
-    if (!alone) return dma ? 15 : 3;   // a 256 x 256 tile's LDS leaves no room beside it on the CU, two small ones fit
-    if (dma) {
-        const int nk = (int)(N / BK);
-        const size_t out_bytes = (size_t)T * M * sizeof(float), ws = !(M & 3) ? split_bytes : 0;
-        double c14, c15;
-        dma_split(((T + 255) / 256) * ((M + 255) / 256), nk, false, out_bytes, ws, &c14);
-        dma_split(((T + 127) / 128) * ((M + 127) / 128), nk, true, out_bytes, ws, &c15);
-        return c14 <= c15 ? 14 : 15;
+// Tile choice.
+//   CFG_DMA +  operands laid out for 16-byte loads: the direct-to-LDS kernel with the tile and K split that the cost
+//              model puts first (128 x 128 tiles at full depth when another product runs beside this one: a 256 x 256
+//              tile's LDS leaves no room beside it on the CU, two small ones fit)
+//   9          uint8 weights otherwise, where 256 x 256 tiles of the register-staged kernel fill the chip: one per CU
+//              and round, the last round at least 70 % full
+//   3          everything else: 128 x 128 tiles, 4 k-tiles of prefetch
+int pick_cfg(int64_t T, int64_t N, int64_t M, bool w_u8, bool alone, bool dma, size_t split_bytes, int *ks) {
+    *ks = 1;
+    const size_t ws = !(M & 3) ? split_bytes : 0;
+    if (dma && !alone) {
+        const int64_t tiles = ((T + 127) / 128) * ((M + 127) / 128);
+        *ks = dma_split(TILE_S, T, tiles, (int)(N / BK), (size_t)(T * M) * sizeof(float), ws);
+        return CFG_DMA + TILE_S;
     }
+    if (dma) return CFG_DMA + dma_tile(T, (int)(N / BK), 1, &M, ws, ks);
+    if (!alone) return 3;
     const int64_t big = ((T + 255) / 256) * ((M + 255) / 256), rounds = (big + 255) / 256;
     return w_u8 && big * 10 >= rounds * 256 * 7 ? 9 : 3;   // fp16 weight tiles are twice the bytes: the large tile spills
 }
@@ -1296,14 +1324,11 @@ int pick_cfg(int64_t T, int64_t N, int64_t M, bool w_u8, bool alone, bool dma, s
 GemmPlan gemm_plan(bool w_u8, int64_t T, int64_t N, int64_t M, const rwkv_half *A, int64_t lda, const void *W,
                    int64_t ldw, const void *Y, int64_t ldy, const GemmEpi &ep) {
     if (skinny_ok(w_u8, T, N, A, lda, W, ldw, ep)) return GemmPlan{0, 0, 0, 1};
+    int ks;
     const int cfg = pick_cfg(T, N, M, w_u8, !ep.small_tiles, dma_ok(w_u8, N, M, A, lda, W, ldw, Y, ldy, ep),
-                             ep.splitk_ws ? ep.splitk_bytes : 0);
-    if (cfg != 14 && cfg != 15) return GemmPlan{1, 0, 0, 1};
-    const int tile = cfg == 14 ? 256 : 128;
-    const int64_t tiles = ((T + tile - 1) / tile) * ((M + tile - 1) / tile);
-    int ks = 1;   // as launch_dma decides it
-    if (ep.splitk_ws && (M & 3) == 0) ks = dma_split(tiles, (int)(N / BK), tile < 256, (size_t)T * M * sizeof(float), ep.splitk_bytes);
-    return GemmPlan{2, tile, tile, ks};
+                             ep.splitk_ws ? ep.splitk_bytes : 0, &ks);
+    if (cfg < CFG_DMA) return GemmPlan{1, 0, 0, 1};
+    return GemmPlan{2, tile_dim[cfg - CFG_DMA].tm, tile_dim[cfg - CFG_DMA].tn, ks};
 }
 
 int gemm_launch(bool w_u8, int64_t T, int64_t N, int64_t M, const rwkv_half *A, int64_t lda, const void *W,
@@ -1319,10 +1344,11 @@ int gemm_launch(bool w_u8, int64_t T, int64_t N, int64_t M, const rwkv_half *A, 
         RWKV_LAUNCH_CHECK();
         return RWKV_OK;
     }
+    int ks;
     const int cfg = pick_cfg(T, N, M, w_u8, !ep.small_tiles, dma_ok(w_u8, N, M, A, lda, W, ldw, Y, ldy, ep),
-                             ep.splitk_ws ? ep.splitk_bytes : 0);
-    return w_u8 ? launch_pick<true>(cfg, T, N, M, A, lda, W, ldw, Y, ldy, ep, st)
-                : launch_pick<false>(cfg, T, N, M, A, lda, W, ldw, Y, ldy, ep, st);
+                             ep.splitk_ws ? ep.splitk_bytes : 0, &ks);
+    return w_u8 ? launch_pick<true>(cfg, ks, T, N, M, A, lda, W, ldw, Y, ldy, ep, st)
+                : launch_pick<false>(cfg, ks, T, N, M, A, lda, W, ldw, Y, ldy, ep, st);
 }
 
 int mm8_prepare_launch(int64_t T, int64_t N, const rwkv_half *x, int64_t ldx, const rwkv_half *ry,
@@ -1369,7 +1395,7 @@ int gemm_group_launch(bool w_u8, int n, int64_t T, int64_t N, const rwkv_half *c
         }
         hipLaunchKernelGGL(mm8_prepare_group_kernel, dim3((unsigned)((T + 3) / 4), (unsigned)n), dim3(256), 0, st, (int)T, (int)N, p);
     }
-    int64_t tiles = 0, tiles_big = 0, total_big = 0, total_small = 0, out_elems = 0, max_out = 0;
+    int64_t tiles = 0, max_out = 0;   // tiles: register-staged fallback
     bool dma = true, m4 = true;
     for (int i = 0; i < n; ++i) {
         if (mats[i]->N != N) return RWKV_E_SHAPE;
@@ -1379,12 +1405,7 @@ int gemm_group_launch(bool w_u8, int n, int64_t T, int64_t N, const rwkv_half *c
         g.ep[i].ldres = g.ep[i].ldgate = mats[i]->M;
         if (w_u8) { g.ep[i].mx = mats[i]->mx; g.ep[i].rx = mats[i]->rx; g.ep[i].s0 = sums[i]; g.ep[i].s2 = sums[i] + T; }
         if (parts > 1) { g.ep[i].parts = parts; g.ep[i].p0 = sums[i] + 2 * T; g.ep[i].p2 = sums[i] + 2 * T + (size_t)T * parts; }
-        const int64_t ts = ((T + 127) / 128) * ((mats[i]->M + 127) / 128), tb = ((T + DT - 1) / DT) * ((mats[i]->M + DM - 1) / DM);
-        tiles = std::max(tiles, ts);
-        tiles_big = std::max(tiles_big, tb);
-        total_small += ts;
-        total_big += tb;
-        out_elems += T * mats[i]->M;
+        tiles = std::max<int64_t>(tiles, ((T + 127) / 128) * ((mats[i]->M + 127) / 128));
         max_out = std::max<int64_t>(max_out, T * mats[i]->M);
         m4 = m4 && !(mats[i]->M & 3);
         dma = dma && dma_ok(w_u8, N, mats[i]->M, g.A[i], N, g.W[i], g.ldw[i], g.Y[i], mats[i]->M, g.ep[i]);
@@ -1404,22 +1425,27 @@ int gemm_group_launch(bool w_u8, int n, int64_t T, int64_t N, const rwkv_half *c
         }
     }
     if (dma) {
-        // tile size and K split of least cost, as for a single product
+        // tile and K split of least cost, as for a single product
         const int nk = (int)(N / BK);
-        const size_t out_bytes = (size_t)out_elems * sizeof(float), ws = splitk_ws && m4 ? RWKV_SPLITK_WS_BYTES : 0;
-        double c_big, c_small;
-        const int ks_big = dma_split(total_big, nk, false, out_bytes, ws, &c_big);
-        const int ks_small = dma_split(total_small, nk, true, out_bytes, ws, &c_small);
-        const bool big = c_big <= c_small;
-        const int ks = big ? ks_big : ks_small;
+        int64_t outs[4];
+        for (int i = 0; i < n; ++i) outs[i] = mats[i]->M;
+        int ks = 1;
+        const int tile = dma_tile(T, nk, n, outs, splitk_ws && m4 ? RWKV_SPLITK_WS_BYTES : 0, &ks);
+        int64_t grid_x = 0;
+        for (int i = 0; i < n; ++i)
+            grid_x = std::max<int64_t>(grid_x, ((T + tile_dim[tile].tm - 1) / tile_dim[tile].tm) * ((outs[i] + tile_dim[tile].tn - 1) / tile_dim[tile].tn));
         g.nk_split = nk / ks;
         if (ks > 1) {
             float *p = splitk_ws;
             for (int i = 0; i < n; ++i) { g.part[i] = p; p += (size_t)ks * T * mats[i]->M; }
         }
         int rc;
-        if (big) rc = w_u8 ? launch_dma_group<true, DT, DM>(g, n, T, N, tiles_big, ks, st) : launch_dma_group<false, DT, DM>(g, n, T, N, tiles_big, ks, st);
-        else rc = w_u8 ? launch_dma_group<true, 128, 128>(g, n, T, N, tiles, ks, st) : launch_dma_group<false, 128, 128>(g, n, T, N, tiles, ks, st);
+        switch (tile) {
+            case TILE_L: rc = w_u8 ? launch_dma_group<true, 256, 256, 8, 0>(g, n, T, N, grid_x, ks, st) : launch_dma_group<false, 256, 256, 8, 0>(g, n, T, N, grid_x, ks, st); break;
+            case TILE_S: rc = w_u8 ? launch_dma_group<true, 128, 128, 8, 0>(g, n, T, N, grid_x, ks, st) : launch_dma_group<false, 128, 128, 8, 0>(g, n, T, N, grid_x, ks, st); break;
+            case TILE_S4: rc = w_u8 ? launch_dma_group<true, 128, 128, 8, 4>(g, n, T, N, grid_x, ks, st) : launch_dma_group<false, 128, 128, 8, 4>(g, n, T, N, grid_x, ks, st); break;
+            default: rc = w_u8 ? launch_dma_group<true, 64, 128, 4, 4>(g, n, T, N, grid_x, ks, st) : launch_dma_group<false, 64, 128, 4, 4>(g, n, T, N, grid_x, ks, st); break;
+        }
         if (rc) return rc;
         if (ks > 1) {
             const unsigned blocks = (unsigned)std::min<int64_t>((max_out + 2047) / 2048, 16384);

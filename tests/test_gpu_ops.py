@@ -119,6 +119,18 @@ def test_mm8_seq(N, M, B):
     assert np.abs(y1.cpu().numpy().astype(np.float64) - y[B - 1].cpu().numpy()).max() <= np.abs(ref).max() * 2 ** -9
 
 
+@pytest.mark.parametrize("N,M,B", [(64, 128, 33), (128, 8, 20), (1024, 1000, 17), (1024, 136, 63), (2048, 264, 64), (4096, 4096, 40),
+                                   (4096, 2056, 65), (4096, 4096, 129), (1024, 8192, 192), (16384, 512, 256)])
+def test_mm8_seq_tile_edges(N, M, B):
+    """The 64 x 128 tile (17 .. 64 rows) and the four-stage 128 x 128 tile: fewer k-tiles than stages, ragged rows and
+    columns, full depth and K split; bounds as in test_mm8_seq."""
+    ops = _ops()
+    x, ref, (q, mx, rx, my, ry) = _mm8_case(N, M, B, N + M + B)
+    y = ops.cuda_mm8_seq(B, N, M, torch.from_numpy(x).to(DEV), q, mx, rx, my, ry)
+    d = np.abs(y.cpu().numpy().astype(np.float64) - ref)
+    assert d.max() <= 1e-3 * np.sqrt(np.mean(ref ** 2)) + np.abs(ref).max() * 2 ** -10, d.max()
+
+
 @pytest.mark.parametrize("N,M", [(5120, 20480), (20480, 5120), (5120, 5120)])
 def test_mm8_seq_14b_call_length(N, M):
     """The launches of the 14B configuration at its own call length (1024 rows): 320 large
