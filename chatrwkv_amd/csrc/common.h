@@ -110,4 +110,13 @@ DEV h16x2 u8pair_hi_1024(uint32_t v) {
     return __builtin_bit_cast(h16x2, __builtin_amdgcn_perm(0x64646464u, v, 0x07030602u));
 }
 
+// exp(x) within 2 ulp for x <= 88: 2^(x log2 e) with the rounding error of the product put back (six instructions;
+// results below the smallest normal number become 0)
+DEV float exp_acc(float x) {
+    const float L = 1.44269504f, Llo = 1.92596299e-8f;   // log2 e = L + Llo
+    const float hi = x * L, lo = __builtin_fmaf(x, Llo, __builtin_fmaf(x, L, -hi));
+    const float r = __builtin_amdgcn_exp2f(hi);
+    return __builtin_fmaf(r, lo * 0.693147181f, r);
+}
+
 DEV float sigmoidf_(float x) { return 1.f / (1.f + __expf(-x)); }

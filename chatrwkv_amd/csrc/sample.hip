@@ -85,15 +85,6 @@ DEV float wave_scan(float v) {
     return v;
 }
 
-// exp(x) for x <= 0: 2^(x log2 e) with the rounding error of the product put back (within 2 ulp; results below the
-// smallest normal number become 0)
-DEV float exp_neg(float x) {
-    const float L = 1.44269504f, Llo = 1.92596299e-8f;   // log2 e = L + Llo
-    const float hi = x * L, lo = __builtin_fmaf(x, Llo, __builtin_fmaf(x, L, -hi));
-    const float r = __builtin_amdgcn_exp2f(hi);
-    return __builtin_fmaf(r, lo * 0.693147181f, r);
-}
-
 // POW: temperature other than 1 (its 64 copies stay out of the code of the usual case)
 // SROWS: group rows, at least V / 4096.  Rows past the end hold zeros and are worked on like the others: with a test
 // of V around each row the compiler made a copy of what follows for every number of rows.
@@ -178,7 +169,7 @@ __global__ __launch_bounds__(STHREADS) void sample_kernel(SampleArgs a) {
     mx = block_max(mx, red, turn);
     float s = 0.f;
 #pragma unroll
-    for (int e = 0; e < EMAX; ++e) { p[e] = (p[e] == -INFINITY) ? 0.f : exp_neg(p[e] - mx); s += p[e]; }
+    for (int e = 0; e < EMAX; ++e) { p[e] = (p[e] == -INFINITY) ? 0.f : exp_acc(p[e] - mx); s += p[e]; }
     const float inv = 1.f / block_total(s, 0.f, red, turn).s;
     float pmax = 0.f, total = 0.f;
 #pragma unroll

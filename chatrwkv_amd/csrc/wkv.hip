@@ -339,7 +339,7 @@ extern "C" int rwkv_wkv4_forward(int64_t B, int64_t T, int64_t C, const float *w
 
 // fused variant used by the model path: k, v (fp16 or fp32) and fp16 r in; y = fp16(r * fp16(wkv)).
 // ---------------------------------------------------------------------------------------
-// RWKV-5 / RWKV-6 over a sequence, model path.  A head's 64 value columns never interact (y_i and the
+// RWKV-5 / RWKV-6 over a short sequence (32 tokens to WKV_CHUNKED - 1), model path.  A head's 64 value columns never interact (y_i and the
 // column S[:, i] depend on v_i only), so a head is split over four workgroups of 16 value columns: 4 H
 // workgroups instead of H.  Thread (value i, key group g): lane & 15 = g owns keys 4g..4g+3 of column i,
 // lane >> 4 and the wave index give i.  The sum over the 16 key groups of a value is a DPP row sum in
@@ -456,6 +456,193 @@ __global__ __launch_bounds__(256) void wkv56_split_kernel(Wkv56Args a) {
     for (int e = 0; e < 4; ++e) S[(4 * g + e) * HS + i] = s[e];
 }
 
+// ---------------------------------------------------------------------------------------
+// RWKV-5 / RWKV-6 over a sequence, model path, in chunks of 16 tokens.  With A_t the product of the decays of the
+// chunk's tokens before t, and S the state (keys x values) the chunk starts from,
+//     y_t = (r_t . A_t) S + sum_{s <= t} P_ts v_s,      P_ts = sum_j r_tj k_sj prod_{s < m < t} w_mj   (P_tt: u_j for the product)
+//     S'  = A_16 S + sum_s (k_s . prod_{s < m} w_m) v_s^T
+// so all that stays sequential is one 16-token step of matrix products.  The recurrence token by token took 245 - 300
+// cycles a token, a latency chain on one wave per SIMD.
+//   wkv56_chunk_kernel   one workgroup per (head, chunk), all of them independent: r . A, P, the decayed keys, A_16.
+//                        Thread (s, key group g) carries k_s times the running product over t, the factors in the
+//                        order the recurrence applies them (no logarithms, no quotients: any decay in [0, 1]).
+//   wkv56_apply_kernel   workgroup (head, 16 values), wave jb = keys 16 jb .. + 15, one 16 x 16 block of S in MFMA
+//                        accumulators for the whole call, v_mfma_f32_16x16x4_f32 throughout (fp32 operands and sums).
+//                        An accumulator register of S is the second operand of r . A times S as it stands: key
+//                        16 jb + 4 q + e in lane group q is inner index q of step e.  The four waves' shares of y
+//                        meet in LDS, one barrier per chunk, off the state's chain.  The first kernel leaves every
+//                        operand in fragment order (five loads per wave and chunk) and pads the chunks to whole
+//                        groups of PD, so that PD chunks are in flight with no load, store or wait under a branch.
+// Raw y goes to an fp32 [T, C] scratch; GroupNorm and the gate need the whole head and follow in wkv56_gn_kernel.
+// Calls longer than WKV_SEG tokens run in segments, which bounds the scratch between the two kernels.
+// Measured per layer, 64 heads, RWKV-6 (recurrence token by token -> chunks, both without GroupNorm): 1024 tokens 111 ->
+// 47 us, 256 tokens 29.6 -> 18.4; RWKV-5, 32 heads, 333 tokens 29.3 -> 17.9.  At 64 tokens the second launch costs what
+// the chunks save (11.1 -> 12.9 us), at 96 it does not (14.4 -> 13.0): WKV_CHUNKED.
+//   WMODE 0: w[C] fp32 constant decay (RWKV-5);  WMODE 2: fp16 LoRA output [T, C] + t_decay (RWKV-6)
+// ---------------------------------------------------------------------------------------
+constexpr int CL = 16;                                // tokens per chunk
+constexpr int WKV_SEG = 2048;                         // tokens per segment
+constexpr int WKV_CHUNKED = 80;                       // calls of at least so many tokens run in chunks
+constexpr int PD = 8;                                 // chunks in flight; calls are padded to whole groups of PD chunks
+// one chunk's operands, in floats: r . A and decayed keys as [key block][lane][4], P as [key block][lane], A_16 [64], and
+// the values (fp16) as [value block][lane][4]
+constexpr int CH_R = 0, CH_K = CL * HS, CH_P = 2 * CL * HS, CH_A = CH_P + CL * CL, CH_V = CH_A + HS, CH_FLOATS = CH_V + CL * HS / 2;
+int wkv_chunks(int64_t tokens) { return (int)((tokens + CL * PD - 1) / (CL * PD)) * PD; }
+
+template <int WMODE>
+__global__ __launch_bounds__(256) void wkv56_chunk_kernel(Wkv56Args a, int H, int t_begin, float *__restrict__ scratch) {
+    __shared__ __align__(16) float sr[CL][HS], sw[CL][HS];   // sr: later the keys in fragment order
+    __shared__ __align__(16) h16 vf[CL * HS];
+    const int T = a.T, C = a.C;
+    const int h = blockIdx.x % H, c = blockIdx.x / H;
+    const int s = threadIdx.x >> 4, g = threadIdx.x & 15;   // token of the chunk, keys 4 g .. 4 g + 3
+    float *out = scratch + (size_t)blockIdx.x * CH_FLOATS;
+    const int t = t_begin + c * CL + s;
+    const bool live = t < T;                                // past the end: r = k = 0, w = 1
+    const size_t o = (size_t)min(t, T - 1) * C + h * HS + 4 * g;
+    const h16x4 r8 = *(const h16x4 *)((const rwkv_half *)a.r + o), k8 = *(const h16x4 *)((const rwkv_half *)a.k + o);
+    const h16x4 v8 = *(const h16x4 *)((const rwkv_half *)a.v + o);
+    h16x4 x8 = {};
+    if (WMODE == 2) x8 = *(const h16x4 *)((const rwkv_half *)a.w + o);
+    f32x4 r4, k4, w4, u4;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const int j = h * HS + 4 * g + e;
+        u4[e] = a.u[j];
+        w4[e] = WMODE == 2 ? exp_acc(-exp_acc(fminf(a.t_decay[j] + (float)x8[e], 88.f))) : ((const float *)a.w)[j];
+        r4[e] = live ? (float)r8[e] : 0.f;
+        k4[e] = live ? (float)k8[e] : 0.f;
+        w4[e] = live ? w4[e] : 1.f;
+    }
+    *(f32x4 *)&sr[s][4 * g] = r4;
+    *(f32x4 *)&sw[s][4 * g] = w4;
+    __syncthreads();
+    // x: the product of the decays before token s while m < s, then k_s times the decays after it; a wave holds the
+    // tokens 4 wave .. + 3, so what a step needs is decided per wave except at those four
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    f32x4 before = {1.f, 1.f, 1.f, 1.f}, x = before;
+    float mine = 0.f;
+#pragma unroll
+    for (int m = 0; m < CL; ++m) {
+        const f32x4 wm = *(const f32x4 *)&sw[m][4 * g];
+        if (m < 4 * wave) {
+            x *= wm;
+        } else {
+            const f32x4 rm = *(const f32x4 *)&sr[m][4 * g];
+            const bool own = m == s, mixed = m < 4 * wave + 4;
+            if (mixed) {
+                before = own ? x : before;
+                x = own ? k4 * u4 : x;
+            }
+            const float p = row16_sum((rm[0] * x[0] + rm[1] * x[1]) + (rm[2] * x[2] + rm[3] * x[3]));
+            if (g == m) mine = s <= m ? p : 0.f;            // P[m][s]
+            x = mixed && own ? k4 : x * wm;
+        }
+    }
+    // fragment order: token or key in the lower lane bits, the inner index q above them, the step e innermost
+    *(f32x4 *)(out + CH_R + 256 * (g >> 2) + 4 * (s + 16 * (g & 3))) = r4 * before;
+    out[CH_P + 64 * (s >> 2) + g + 16 * (s & 3)] = mine;
+    if (s == CL - 1) *(f32x4 *)(out + CH_A + 4 * g) = before * w4;
+    __syncthreads();
+    float *kf = &sr[0][0];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const int f = 256 * (g >> 2) + 4 * (4 * (g & 3) + e + 16 * (s & 3)) + (s >> 2);
+        kf[f] = x[e];
+        vf[f] = live ? v8[e] : (h16)0.f;
+    }
+    __syncthreads();
+    *(f32x4 *)(out + CH_K + 4 * threadIdx.x) = *(const f32x4 *)(kf + 4 * threadIdx.x);
+    *(h16x4 *)((h16 *)(out + CH_V) + 4 * threadIdx.x) = *(const h16x4 *)(vf + 4 * threadIdx.x);
+}
+
+__global__ __launch_bounds__(256, 2) void wkv56_apply_kernel(Wkv56Args a, int H, int t_begin, int nchunk, const float *scratch) {
+    constexpr int GC = 4;   // chunks per exchange of y: one barrier each, and the sums of a group are read during the next
+    __shared__ f32x4 red[2][GC][4][64];
+    const int C = a.C;
+    const int h = blockIdx.x % H, ib = blockIdx.x / H;
+    const int lane = threadIdx.x & 63, jb = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int n16 = lane & 15, q = lane >> 4;
+    const int i = 16 * ib + n16;                            // value column of the accumulators
+    float *S = a.state + (size_t)h * HS * HS;               // [key][value]
+    f32x4 st;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) st[e] = S[(16 * jb + 4 * q + e) * HS + i];
+    struct Ops { f32x4 r, k, al; float p; h16x4 v; };
+    auto load = [&](Ops &x, int c) {
+        const float *in = scratch + ((size_t)min(c, nchunk - 1) * H + h) * CH_FLOATS;
+        x.r = *(const f32x4 *)(in + CH_R + 256 * jb + 4 * lane);
+        x.k = *(const f32x4 *)(in + CH_K + 256 * jb + 4 * lane);
+        x.al = *(const f32x4 *)(in + CH_A + 16 * jb + 4 * q);
+        x.p = in[CH_P + 64 * jb + lane];
+        x.v = *(const h16x4 *)((const h16 *)(in + CH_V) + 256 * ib + 4 * lane);
+    };
+    float *yo = a.y + (size_t)(t_begin + 4 * q + jb) * C + h * HS + i;   // register jb of a lane's y: token 4 q + jb
+    auto step = [&](const Ops &x, int buf, int u) {
+        float v[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = (float)x.v[e];
+        const float v01 = jb == 0 ? v[0] : v[1], v23 = jb == 2 ? v[2] : v[3];
+        f32x4 y = {0.f, 0.f, 0.f, 0.f};
+        y = __builtin_amdgcn_mfma_f32_16x16x4f32(x.p, jb < 2 ? v01 : v23, y, 0, 0, 0);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) y = __builtin_amdgcn_mfma_f32_16x16x4f32(x.r[e], st[e], y, 0, 0, 0);
+        st *= x.al;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) st = __builtin_amdgcn_mfma_f32_16x16x4f32(x.k[e], v[e], st, 0, 0, 0);
+        red[buf][u][jb][lane] = y;
+    };
+    float part[GC][4];
+    auto exchange = [&](int buf) {
+        __builtin_amdgcn_s_waitcnt(0xC07F);   // LDS only: __syncthreads() would also wait for the loads in flight
+        __builtin_amdgcn_s_barrier();
+#pragma unroll
+        for (int u = 0; u < GC; ++u)
+#pragma unroll
+            for (int w = 0; w < 4; ++w) part[u][w] = ((const float *)&red[buf][u][w][lane])[jb];
+    };
+    auto store = [&]() {
+#pragma unroll
+        for (int u = 0; u < GC; ++u) {
+            *yo = (part[u][0] + part[u][1]) + (part[u][2] + part[u][3]);
+            yo += (size_t)CL * C;
+        }
+    };
+    // The order of the loads is the order of their use, which the fences keep: the compiler counts its waits over both
+    // ways into the loop, and a later chunk's load ahead of an earlier one's would make it wait for both.
+    auto fence = [] {
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    Ops ops[PD];
+#pragma unroll
+    for (int u = 0; u < PD; ++u) {
+        load(ops[u], u);
+        fence();
+    }
+    static_assert(PD == 2 * GC, "two groups per turn of the loop");
+    for (int c0 = 0; c0 < nchunk; c0 += PD) {
+#pragma unroll
+        for (int u = 0; u < PD; ++u) {
+            step(ops[u], u / GC, u % GC);
+            fence();
+            load(ops[u], c0 + u + PD);
+            fence();
+            if (u == GC - 1) {
+                if (c0) store();                  // the second group of the turn before
+                exchange(0);
+                fence();
+            }
+        }
+        store();
+        exchange(1);
+        fence();
+    }
+    store();
+#pragma unroll
+    for (int e = 0; e < 4; ++e) S[(16 * jb + 4 * q + e) * HS + i] = st[e];
+}
+
 // GroupNorm over each head's 64 outputs (eps 64e-5), affine, fp16 rounding, gate.  Four adjacent channels per lane
 // (16-byte loads of y and of the affine vectors, 8-byte accesses to the gate and the output): a row of 16 lanes owns
 // one head of one token, its two sums are DPP row sums; grid-stride over the T * C / 4 chunks.
@@ -490,6 +677,11 @@ __global__ __launch_bounds__(256) void wkv56_gn_kernel(int T, int C, const float
     }
 }
 
+
+size_t wkv56_scratch_bytes(int64_t T, int64_t C) {
+    if (T < 32) return 256;
+    return ((size_t)wkv_chunks(T) * CL * C + (size_t)wkv_chunks(std::min<int64_t>(T, WKV_SEG)) * (C / HS) * CH_FLOATS) * sizeof(float);
+}
 
 size_t wkv4_scratch_bytes(int64_t T, int64_t C) {
     if (T < 64) return 256;
@@ -552,10 +744,20 @@ int wkv56_fused_launch(bool v6, int T, int C, int H, float *state, const rwkv_ha
     a.r = r; a.k = k; a.v = v; a.w = w; a.u = u; a.t_decay = t_decay;
     a.lnx_w = lnx_w; a.lnx_b = lnx_b; a.gate = gate; a.out = out; a.dw2 = dw2; a.ld = ld;
     if (T >= 32 && y32) {
-        // long call: four workgroups per head, raw y to the fp32 scratch, GroupNorm + gate in a second launch
+        // raw y to the fp32 scratch, then GroupNorm + gate
         a.y = y32;
-        if (v6) hipLaunchKernelGGL((wkv56_split_kernel<2>), dim3((unsigned)(4 * H)), dim3(256), 0, st, a);
-        else hipLaunchKernelGGL((wkv56_split_kernel<0>), dim3((unsigned)(4 * H)), dim3(256), 0, st, a);
+        if (T < WKV_CHUNKED) {
+            if (v6) hipLaunchKernelGGL((wkv56_split_kernel<2>), dim3((unsigned)(4 * H)), dim3(256), 0, st, a);
+            else hipLaunchKernelGGL((wkv56_split_kernel<0>), dim3((unsigned)(4 * H)), dim3(256), 0, st, a);
+        }
+        float *chunks = y32 + (size_t)wkv_chunks(T) * CL * C;   // y has a row for every padded token
+        for (int t0 = 0; t0 < T && T >= WKV_CHUNKED; t0 += WKV_SEG) {
+            const int nchunk = wkv_chunks(std::min(T - t0, WKV_SEG));
+            const dim3 grid((unsigned)(H * nchunk));
+            if (v6) hipLaunchKernelGGL((wkv56_chunk_kernel<2>), grid, dim3(256), 0, st, a, H, t0, chunks);
+            else hipLaunchKernelGGL((wkv56_chunk_kernel<0>), grid, dim3(256), 0, st, a, H, t0, chunks);
+            hipLaunchKernelGGL(wkv56_apply_kernel, dim3((unsigned)(4 * H)), dim3(256), 0, st, a, H, t0, nchunk, chunks);
+        }
         hipLaunchKernelGGL(wkv56_gn_kernel, dim3((unsigned)std::min<int64_t>(((int64_t)T * C / 4 + 255) / 256, 65535)), dim3(256), 0, st,
                            T, C, y32, lnx_w, lnx_b, gate, out);
     } else if (v6 && dw2) {

@@ -399,6 +399,34 @@ def test_v56_long_prompt(ver, tag, strat):
     assert d <= LOGIT_TOL, d
 
 
+@pytest.mark.parametrize("ver", [5.2, 6])
+@pytest.mark.parametrize("T", [80, 81, 127, 129, 2049, 2177])
+def test_v56_chunked_recurrence(ver, T):
+    """The recurrence in chunks of 16 tokens (calls of 80 tokens on; ragged last chunk and group of chunks, more than one
+    segment of 2048) against the token-by-token kernels (the same prompt in calls of 64), with decays from 0.9975 down to
+    0 in fp32.  In the first layer r, k, v differ by at most one fp16 rounding, 2^-11, where the products sum in another
+    order, so its state, a sum of products of two, by less than 2^-10 in the 2-norm; behind two more roundings of
+    every activation (time mix and channel mix) the second layer's state and the logits stay within 2^-8."""
+    from chatrwkv_amd import synth
+    from chatrwkv_amd.model import RWKV
+    ck = synth.make_checkpoint(version=ver, n_layer=2, n_embd=256, n_ffn=896, vocab=211, seed=5, affine=True)
+    for i in range(2):
+        d = ck[f"blocks.{i}.att.time_decay"]
+        d.copy_(torch.linspace(-6.0, 5.5, d.numel())[torch.randperm(d.numel(), generator=torch.Generator().manual_seed(1))].reshape(d.shape))
+    m = RWKV(ck, "cuda fp16", verbose=False)
+    toks = synth.random_tokens(T, 211, seed=T)
+    out, st = m.forward(toks, None, full_output=True)
+    parts, ref = [], None
+    for i in range(0, T, 64):
+        o, ref = m.forward(toks[i:i + 64], ref, full_output=True)
+        parts.append(o.reshape(-1, 211).clone())
+    want = torch.cat(parts)
+    rel = lambda a, b: float((a.double() - b.double()).norm() / b.double().norm())
+    assert torch.isfinite(out).all() and torch.isfinite(st[1]).all() and torch.isfinite(st[4]).all()
+    assert rel(st[1], ref[1]) <= 2.0 ** -10, rel(st[1], ref[1])
+    assert rel(st[4], ref[4]) <= 2.0 ** -8 and rel(out, want) <= 2.0 ** -8, (rel(st[4], ref[4]), rel(out, want))
+
+
 @pytest.mark.parametrize("ver,tag", [(4, "v4"), (5, "v5_0"), (5.1, "v5_1"), (5.2, "v5_2"), (6, "v6_0")])
 def test_fp16_strategy_against_reference_half_run(ver, tag):
     """'cuda fp16' on the GPU against the logits and states the reference itself produced under 'cpu fp16'
