@@ -119,4 +119,12 @@ DEV float exp_acc(float x) {
     return __builtin_fmaf(r, lo * 0.693147181f, r);
 }
 
+// n / d within 1 ulp for normal d and quotient: a reciprocal estimate and one correction (the compiler's own division
+// also covers denormals and infinities, at twice the instructions)
+DEV float div_acc(float n, float d) {
+    const float r = __builtin_amdgcn_rcpf(d), q = n * r;
+    return __builtin_fmaf(__builtin_fmaf(-d, q, n), r, q);
+}
+DEV float sigmoid_acc(float x) { return div_acc(1.f, 1.f + __expf(fminf(-x, 80.f))); }
+
 DEV float sigmoidf_(float x) { return 1.f / (1.f + __expf(-x)); }

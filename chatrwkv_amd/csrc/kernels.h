@@ -65,6 +65,10 @@ int wkv56_fused_launch(bool v6, int T, int C, int H, float *state, const rwkv_ha
                        const rwkv_half *dw2 = nullptr, int ld = 0,  // dw2: v6 with w = tanh(. @ D1), product with D2 in-kernel
                        float *y32 = nullptr);  // scratch (wkv56_scratch_bytes): calls of >= 32 tokens run in chunks
 size_t wkv56_scratch_bytes(int64_t T, int64_t C);
+// The chunked recurrences (wkv.hip, v7.hip): tokens per chunk, chunks in flight, and the chunks of a call, padded to
+// whole groups of those in flight.
+constexpr int CL = 16, PD = 8;
+inline int wkv_chunks(int64_t tokens) { return (int)((tokens + CL * PD - 1) / (CL * PD)) * PD; }
 // Row-wise LayerNorm + token shift + mixes for up to 6 consumers over a [T, C] activation (seq_v4.hip).
 struct SeqMixArgs {
     int T, C;

@@ -294,6 +294,284 @@ __global__ __launch_bounds__(256) void wkv7_kernel(Wkv7Args a) {
     *(f32x4 *)S = s;
 }
 
+// ---- the recurrence over a long sequence, model path, in chunks of 16 tokens -----------------------------------
+// With A_t the product of the decays of the chunk's tokens up to and including t, S (keys x values) the state the chunk
+// starts from and u_t = the row sa of token t,
+//     u_t = (a_t . A_{t-1}) S + sum_{s<t} (AK_ts v_s + AB_ts u_s),    y_t = (r_t . A_t) S + sum_{s<=t} (QK_ts v_s + QB_ts u_s)
+//     S'  = A_16 S + sum_s (k_s . A_16/A_s) v_s^T + (b_s . A_16/A_s) u_s^T
+// (AK_ts = sum_j a_tj k_sj A_{t-1,j}/A_sj, QK with r_t and A_t, AB and QB with b_s.)  u is a unit lower triangular system,
+// so with Z = (I - AB)^-1 everything that needs no S can be formed for all chunks at once:
+//     u = TA S + TK v,   TA = Z (a . A),  TK = Z AK;      y = Y1 S + Y2 v,   Y1 = r . A + QB TA,  Y2 = QK + QB TK.
+// The decays of this model lie in (0.545, 1) (exp(-e^-0.5 sigmoid)), so A_16 >= 6e-5 and the quotients by A_s are safe
+// in fp32 and as exact as the products they replace.
+//   wkv7_chunk_kernel  one workgroup per (head, chunk): the preparation of prep7_kernel for its 16 tokens, then Y1, TA,
+//                      Y2, TK and the decayed k and b.  The four matrices and the products with Z and QB are
+//                      v_mfma_f32_16x16x4_f32 (fp32 operands and sums).
+//   wkv7_apply_kernel  workgroup (head, 16 values), wave jb = keys 16 jb .. + 15: one 16 x 16 block of S in MFMA
+//                      accumulators for the whole call.  Operands arrive in fragment order, PD chunks in flight; the
+//                      four waves' shares of u and y meet in LDS, one barrier per chunk.
+// Bound by the operands between the two (20 KB per head and chunk, fp32).  Measured per layer at 64 heads, preparation
+// and recurrence: 1024 tokens 152 -> 94 us, 777 tokens 116 -> 80, 256 tokens 42 -> 29, 100 tokens 21 -> 19; at 64 tokens
+// the two launches take as long as prep7_kernel and wkv7_kernel: CHUNKED7.
+constexpr int SEG7 = 1024;        // tokens per pair of launches: bounds the scratch between them
+constexpr int CHUNKED7 = 96;      // calls of at least so many tokens run in chunks
+// one chunk's operands, in floats: Y1, TA, decayed k, decayed b as [key block][lane][4]; (Y2, TK) as [key block][lane][2];
+// A_16 [64]; the values (fp16) as [value block][lane][4].  Lane = token or key or value, + 16 q; inner index 4 q + e.
+constexpr int C7_Y1 = 0, C7_TA = 1024, C7_K = 2048, C7_B = 3072, C7_2 = 4096, C7_A = C7_2 + 512, C7_V = C7_A + 64, C7_FLOATS = C7_V + 512;
+constexpr int LR7 = 68;           // LDS row of 64 floats, padded: 16 rows hit 16 different bank groups
+constexpr int LM7 = 20;           // LDS row of 16 floats, padded
+
+__global__ __launch_bounds__(256) void wkv7_chunk_kernel(Prep7Args a, int t_begin, float *__restrict__ scratch) {
+    __shared__ __align__(16) float la[CL][LR7], lr[CL][LR7], lk[CL][LR7], lb[CL][LR7];   // a . A, r . A, k / A, b / A
+    __shared__ __align__(16) float lw[CL][HS7], lall[HS7];          // decays; A_16
+    __shared__ __align__(16) float mat[4][CL][LM7], lz[CL][LM7];   // AK, AB, QK, QB; Z
+    __shared__ __align__(16) h16 lv[CL * HS7];
+    const int H = a.H, C = a.C, T = a.T;
+    const int h = blockIdx.x % H, c = blockIdx.x / H;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int s = tid >> 4, g = tid & 15;                 // token of the chunk, channels 4 g .. + 3 of the head
+    float *out = scratch + (size_t)blockIdx.x * C7_FLOATS;
+    const int t = t_begin + c * CL + s;
+    const bool live = t < T;                              // past the end: r = k = a = b = v = 0, w = 1
+    const int ch = h * HS7 + 4 * g;
+    const size_t o = (size_t)min(t, T - 1) * C + ch;
+    // ---- preparation, rounding by rounding as in prep7_kernel
+    const h16x4 r4 = *(const h16x4 *)(a.r + o), k4 = *(const h16x4 *)(a.k + o), v4 = *(const h16x4 *)(a.v + o);
+    const h16x4 ar4 = *(const h16x4 *)(a.a_raw + o), wr4 = *(const h16x4 *)(a.w_raw + o);
+    h16x4 vg4 = {}, vf4 = {};
+    if (a.vg_raw) { vg4 = *(const h16x4 *)(a.vg_raw + o); vf4 = *(const h16x4 *)(a.v_first + o); }
+    float kku[4], av[4], k2[4], ss = 0.f, rks = 0.f;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const float k = (float)k4[e];
+        av[e] = round_h(sigmoid_acc(round_h(h2f(a.a0[ch + e]) + (float)ar4[e])));
+        kku[e] = round_h(k * h2f(a.k_k[ch + e]));
+        ss += kku[e] * kku[e];
+        k2[e] = round_h(k * round_h(1.f + round_h(round_h(av[e] - 1.f) * h2f(a.k_a[ch + e]))));
+        rks += round_h(round_h((float)r4[e] * k2[e]) * h2f(a.r_k[ch + e]));
+    }
+    const float nrm = fmaxf(round_h(sqrtf(row16_sum(ss))), 1e-12f);
+    rks = row16_sum(rks);
+    f32x4 w, rr, kk2, aa, bb;
+    h16x4 vo = v4;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const float kk = round_h(div_acc(kku[e], nrm));
+        if (a.vg_raw) {
+            const float v = (float)v4[e];
+            const float sg = round_h(sigmoid_acc(round_h(h2f(a.v0[ch + e]) + (float)vg4[e])));
+            vo[e] = (h16)(v + round_h(round_h((float)vf4[e] - v) * sg));
+        }
+        w[e] = live ? __expf(-0.606531f * sigmoid_acc(round_h(h2f(a.w0[ch + e]) + (float)wr4[e]))) : 1.f;
+        rr[e] = live ? (float)r4[e] : 0.f;
+        kk2[e] = live ? k2[e] : 0.f;
+        aa[e] = live ? -kk : 0.f;
+        bb[e] = live ? round_h(kk * av[e]) : 0.f;
+    }
+    if (live) {
+        if (a.vg_raw) *(h16x4 *)(a.v + o) = vo;
+        if (g == 0) a.rk[(size_t)t * H + h] = round_h(rks);
+    }
+    *(f32x4 *)&lw[s][4 * g] = w;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) lv[256 * (g >> 2) + 4 * (4 * (g & 3) + e + 16 * (s >> 2)) + (s & 3)] = live ? vo[e] : (h16)0.f;
+    __syncthreads();
+    // ---- decays: before = A_{s-1}; a wave holds the tokens 4 wave .. + 3
+    f32x4 before = {1.f, 1.f, 1.f, 1.f};
+#pragma unroll
+    for (int m = 0; m < CL - 1; ++m) {
+        if (m >= 4 * wave + 3) continue;
+        const f32x4 wm = *(const f32x4 *)&lw[m][4 * g];
+        before = m < 4 * wave || m < s ? before * wm : before;
+    }
+    const f32x4 upto = before * w;
+    f32x4 inv;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) inv[e] = div_acc(1.f, upto[e]);
+    *(f32x4 *)&la[s][4 * g] = aa * before;
+    *(f32x4 *)&lr[s][4 * g] = rr * upto;
+    *(f32x4 *)&lk[s][4 * g] = kk2 * inv;
+    *(f32x4 *)&lb[s][4 * g] = bb * inv;
+    if (s == CL - 1) {
+        *(f32x4 *)(out + C7_A + 4 * g) = upto;
+        *(f32x4 *)&lall[4 * g] = upto;
+    }
+    *(h16x4 *)((h16 *)(out + C7_V) + 4 * tid) = *(const h16x4 *)(lv + 4 * tid);
+    __syncthreads();
+    // ---- wave 0: AK, 1: AB, 2: QK, 3: QB.  Row t in the first operand's lanes, s in the second's; D: column s = lane & 15,
+    // rows t = 4 q + e
+    const int n16 = lane & 15, q = lane >> 4;
+    {
+        const float (*left)[LR7] = wave < 2 ? la : lr, (*right)[LR7] = wave & 1 ? lb : lk;
+        f32x4 d = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int b = 0; b < 4; ++b) {
+            const f32x4 x = *(const f32x4 *)&left[n16][16 * b + 4 * q], y = *(const f32x4 *)&right[n16][16 * b + 4 * q];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) d = __builtin_amdgcn_mfma_f32_16x16x4f32(x[e], y[e], d, 0, 0, 0);
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int row = 4 * q + e;
+            mat[wave][row][n16] = (wave < 2 ? n16 < row : n16 <= row) ? d[e] : 0.f;
+        }
+    }
+    __syncthreads();
+    // ---- Z = (I - AB)^-1 by forward substitution, a column per lane (the four lane groups of wave 0 do the same)
+    if (wave == 0) {
+        float z[CL];
+#pragma unroll
+        for (int row = 0; row < CL; ++row) {
+            float p[2] = {row == n16 ? 1.f : 0.f, 0.f};
+#pragma unroll
+            for (int m4 = 0; m4 < row; m4 += 4) {
+                const f32x4 x = *(const f32x4 *)&mat[1][row][m4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (m4 + e < row) p[e & 1] = __builtin_fmaf(x[e], z[m4 + e], p[e & 1]);
+            }
+            z[row] = p[0] + p[1];
+            if (q == 0) lz[row][n16] = z[row];
+        }
+    }
+    __syncthreads();
+    // ---- wave b: columns 16 b .. of TA = Z (a . A) and Y1 = r . A + QB TA (a D register is the next product's second
+    // operand); wave 1 also TK = Z AK and Y2 = QK + QB TK
+    const f32x4 zf = *(const f32x4 *)&lz[n16][4 * q], qb = *(const f32x4 *)&mat[3][n16][4 * q];
+    f32x4 ta = {0.f, 0.f, 0.f, 0.f}, y1;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        ta = __builtin_amdgcn_mfma_f32_16x16x4f32(zf[e], la[4 * q + e][16 * wave + n16], ta, 0, 0, 0);
+        y1[e] = lr[4 * q + e][16 * wave + n16];
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) y1 = __builtin_amdgcn_mfma_f32_16x16x4f32(qb[e], ta[e], y1, 0, 0, 0);
+    f32x4 tk = {0.f, 0.f, 0.f, 0.f}, y2;
+    if (wave == 1) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            tk = __builtin_amdgcn_mfma_f32_16x16x4f32(zf[e], mat[0][4 * q + e][n16], tk, 0, 0, 0);
+            y2[e] = mat[2][4 * q + e][n16];
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) y2 = __builtin_amdgcn_mfma_f32_16x16x4f32(qb[e], tk[e], y2, 0, 0, 0);
+    }
+    __syncthreads();
+    // ---- to fragment order through LDS
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        la[4 * q + e][16 * wave + n16] = ta[e];
+        lr[4 * q + e][16 * wave + n16] = y1[e];
+        if (wave == 1) { mat[0][4 * q + e][n16] = tk[e]; mat[2][4 * q + e][n16] = y2[e]; }
+    }
+    const f32x4 rest = *(const f32x4 *)&lall[4 * g] * inv;                         // A_16 / A_s
+    *(f32x4 *)&lk[s][4 * g] = kk2 * rest;
+    *(f32x4 *)&lb[s][4 * g] = bb * rest;
+    __syncthreads();
+    *(f32x4 *)(out + C7_Y1 + 4 * tid) = *(const f32x4 *)&lr[n16][16 * wave + 4 * q];
+    *(f32x4 *)(out + C7_TA + 4 * tid) = *(const f32x4 *)&la[n16][16 * wave + 4 * q];
+    f32x4 kf, bf;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) { kf[e] = lk[4 * q + e][16 * wave + n16]; bf[e] = lb[4 * q + e][16 * wave + n16]; }
+    *(f32x4 *)(out + C7_K + 4 * tid) = kf;
+    *(f32x4 *)(out + C7_B + 4 * tid) = bf;
+    // wave jb of the second kernel takes the inner indices 4 q + jb of Y2 and TK
+    typedef float f32x2 __attribute__((ext_vector_type(2)));
+    *(f32x2 *)(out + C7_2 + 2 * tid) = f32x2{mat[2][n16][4 * q + wave], mat[0][n16][4 * q + wave]};
+}
+
+__global__ __launch_bounds__(256, 2) void wkv7_apply_kernel(int H, int C, float *state, float *y32, int t_begin, int nchunk, const float *scratch) {
+    __shared__ f32x4 redu[2][4][64], redy[2][4][64];
+    const int h = blockIdx.x % H, ib = blockIdx.x / H;
+    const int lane = threadIdx.x & 63, jb = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int n16 = lane & 15, q = lane >> 4;
+    const int i = 16 * ib + n16;                            // value column of the accumulators
+    float *S = state + (size_t)h * HS7 * HS7 + (size_t)i * HS7 + 16 * jb + 4 * q;   // [value][key]
+    f32x4 st = *(const f32x4 *)S;
+    typedef float f32x2 __attribute__((ext_vector_type(2)));
+    struct Ops { f32x4 ta, y1, k, b, al; f32x2 two; h16x4 v; };
+    const uint32_t o16 = (256 * jb + 4 * lane) * 4, o2 = (C7_2 + 128 * jb + 2 * lane) * 4, oa = (C7_A + 16 * jb + 4 * q) * 4,
+                   ov = C7_V * 4 + (256 * ib + 4 * lane) * 2;
+    auto load = [&](Ops &x, int c) {     // the base is the same for the whole wave, the offsets never change
+        const char *in = (const char *)(scratch + ((size_t)min(c, nchunk - 1) * H + h) * C7_FLOATS);
+        x.ta = *(const f32x4 *)(in + C7_TA * 4 + o16);
+        x.two = *(const f32x2 *)(in + o2);
+        x.v = *(const h16x4 *)(in + ov);
+        x.y1 = *(const f32x4 *)(in + C7_Y1 * 4 + o16);
+        x.al = *(const f32x4 *)(in + oa);
+        x.k = *(const f32x4 *)(in + C7_K * 4 + o16);
+        x.b = *(const f32x4 *)(in + C7_B * 4 + o16);
+    };
+    // register jb of a lane's y: token 4 q + jb; stored one chunk late, the first (empty) store to the 16 rows ahead of token 0
+    float *yo = y32 + (size_t)(4 * q + jb) * C + h * HS7 + i, *ynext = yo + (size_t)(CL + t_begin) * C;
+    // u first (the next state waits for it), the keys' update while its shares are on their way to LDS, y while they come
+    // back; y's shares are exchanged with the next chunk's u
+    f32x4 yp = {0.f, 0.f, 0.f, 0.f};
+    auto step = [&](const Ops &x, int buf) {
+        float v[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = (float)x.v[e];
+        const float v01 = jb == 0 ? v[0] : v[1], v23 = jb == 2 ? v[2] : v[3], vj = jb < 2 ? v01 : v23;
+        const f32x4 zero = {0.f, 0.f, 0.f, 0.f}, old = st;
+        f32x4 u = __builtin_amdgcn_mfma_f32_16x16x4f32(x.two[1], vj, zero, 0, 0, 0);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) u = __builtin_amdgcn_mfma_f32_16x16x4f32(x.ta[e], old[e], u, 0, 0, 0);
+        redy[buf][jb][lane] = yp;
+        st = old * x.al;
+        __builtin_amdgcn_sched_barrier(0);
+        st = __builtin_amdgcn_mfma_f32_16x16x4f32(x.k[0], v[0], st, 0, 0, 0);
+        st = __builtin_amdgcn_mfma_f32_16x16x4f32(x.k[1], v[1], st, 0, 0, 0);
+        redu[buf][jb][lane] = u;
+        __builtin_amdgcn_sched_barrier(0);
+        st = __builtin_amdgcn_mfma_f32_16x16x4f32(x.k[2], v[2], st, 0, 0, 0);
+        st = __builtin_amdgcn_mfma_f32_16x16x4f32(x.k[3], v[3], st, 0, 0, 0);
+        __builtin_amdgcn_s_waitcnt(0xC07F);   // LDS only: __syncthreads() would also wait for the loads in flight
+        __builtin_amdgcn_s_barrier();
+        const f32x4 u0 = redu[buf][0][lane], u1 = redu[buf][1][lane], u2 = redu[buf][2][lane], u3 = redu[buf][3][lane];
+        float part[4];
+#pragma unroll
+        for (int w = 0; w < 4; ++w) part[w] = ((const float *)&redy[buf][w][lane])[jb];
+        __builtin_amdgcn_sched_barrier(0);
+        yp = __builtin_amdgcn_mfma_f32_16x16x4f32(x.two[0], vj, zero, 0, 0, 0);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) yp = __builtin_amdgcn_mfma_f32_16x16x4f32(x.y1[e], old[e], yp, 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        u = (u0 + u1) + (u2 + u3);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) st = __builtin_amdgcn_mfma_f32_16x16x4f32(x.b[e], u[e], st, 0, 0, 0);
+        *yo = (part[0] + part[1]) + (part[2] + part[3]);   // the chunk before
+        yo = ynext;
+        ynext += (size_t)CL * C;
+    };
+    // The order of the loads is the order of their use, which the fences keep: the compiler counts its waits over both
+    // ways into the loop, and a later chunk's load ahead of an earlier one's would make it wait for both.
+    auto fence = [] {
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    Ops ops[PD];
+#pragma unroll
+    for (int u = 0; u < PD; ++u) {
+        load(ops[u], u);
+        fence();
+    }
+    for (int c0 = 0; c0 < nchunk; c0 += PD) {
+#pragma unroll
+        for (int u = 0; u < PD; ++u) {
+            step(ops[u], u & 1);
+            fence();
+            load(ops[u], c0 + u + PD);
+            fence();
+        }
+    }
+    __syncthreads();
+    redy[0][jb][lane] = yp;
+    __syncthreads();
+    const float *p = (const float *)&redy[0][0][lane] + jb;
+    *yo = (p[0] + p[256]) + (p[512] + p[768]);
+    *(f32x4 *)S = st;
+}
+
 // GroupNorm over each head's 64 outputs (eps 64e-5) on the fp16-rounded read-out, + bonus * v, * g.  Four adjacent
 // channels per lane (16-byte loads of y, 8-byte accesses to v, g and the output): a row of 16 lanes owns one head
 // of one token, its two sums are DPP row sums; grid-stride over the T * C / 4 chunks.
@@ -575,7 +853,7 @@ int de_gate_launch(const rwkv_v7_layer &l, int64_t T, int C, int F, int vocab, c
 struct Ws7 {
     rwkv_half *x, *mix[6], *l1, *lw, *la, *lv, *lg, *w_raw, *a_raw, *vg_raw, *g, *r, *k, *v, *v_first, *an, *b, *att, *vx,
         *xx_att, *xx_ffn, *de_ss;
-    float *dec, *rk, *y32, *splitk;
+    float *dec, *rk, *y32, *splitk, *chunks;
     size_t total;
 };
 
@@ -598,7 +876,8 @@ Ws7 carve7(void *base, int64_t T, const rwkv_v7_model *m) {
     w.de_ss = take((size_t)T * 32 * 2);
     w.dec = (float *)take((size_t)T * C * 4);
     w.rk = (float *)take((size_t)T * m->n_head * 4);
-    w.y32 = (float *)take((size_t)T * C * 4);
+    w.y32 = (float *)take((size_t)(T < CHUNKED7 ? T : (wkv_chunks(T) + 1) * CL) * C * 4);   // a row for every padded token, and 16 in front
+    w.chunks = (float *)take(T < CHUNKED7 ? 256 : (size_t)wkv_chunks(std::min<int64_t>(T, SEG7)) * m->n_head * C7_FLOATS * 4);
     w.splitk = (float *)take(RWKV_SPLITK_WS_BYTES);
     w.total = (size_t)(p - (unsigned char *)base);
     return w;
@@ -839,14 +1118,20 @@ extern "C" int rwkv_v7_forward(const rwkv_v7_model *m, const rwkv_v56_layer_stat
             a.vg_raw = i > 0 ? ws.vg_raw : nullptr; a.v_first = i > 0 ? ws.v_first : nullptr;
             a.w0 = l.w0; a.a0 = l.a0; a.v0 = l.v0; a.k_k = l.k_k; a.k_a = l.k_a; a.r_k = l.r_k;
             a.an = ws.an; a.b = ws.b; a.dec = ws.dec; a.rk = ws.rk;
-            const int64_t blocks = ((int64_t)T * C / 8 + 255) / 256;
-            hipLaunchKernelGGL(prep7_kernel, dim3((unsigned)std::min<int64_t>(blocks, 65535)), dim3(256), 0, st, a);
+            if (T >= CHUNKED7) {
+                for (int64_t t0 = 0; t0 < T; t0 += SEG7) {
+                    const int nchunk = wkv_chunks(std::min<int64_t>(T - t0, SEG7));
+                    hipLaunchKernelGGL(wkv7_chunk_kernel, dim3((unsigned)(H * nchunk)), dim3(256), 0, st, a, (int)t0, ws.chunks);
+                    hipLaunchKernelGGL(wkv7_apply_kernel, dim3((unsigned)(4 * H)), dim3(256), 0, st, H, C, s.att_kv, ws.y32, (int)t0, nchunk, ws.chunks);
+                }
+            } else {
+                const int64_t blocks = ((int64_t)T * C / 8 + 255) / 256;
+                hipLaunchKernelGGL(prep7_kernel, dim3((unsigned)std::min<int64_t>(blocks, 65535)), dim3(256), 0, st, a);
+                Wkv7Args q{(int)T, C, s.att_kv, ws.r, ws.dec, ws.k, v, ws.an, ws.b, ws.y32};
+                hipLaunchKernelGGL((wkv7_kernel<RWKV_DT_F16, true>), dim3((unsigned)(4 * H)), dim3(256), 0, st, q);
+            }
         }
-        {
-            Wkv7Args q{(int)T, C, s.att_kv, ws.r, ws.dec, ws.k, v, ws.an, ws.b, ws.y32};
-            hipLaunchKernelGGL((wkv7_kernel<RWKV_DT_F16, true>), dim3((unsigned)(4 * H)), dim3(256), 0, st, q);
-        }
-        hipLaunchKernelGGL(gn7_kernel, dim3((unsigned)std::min<int64_t>(((int64_t)T * C / 4 + 255) / 256, 65535)), dim3(256), 0, st, (int)T, C, ws.y32, l.lnx_w, l.lnx_b, ws.rk, v,
+        hipLaunchKernelGGL(gn7_kernel, dim3((unsigned)std::min<int64_t>(((int64_t)T * C / 4 + 255) / 256, 65535)), dim3(256), 0, st, (int)T, C, ws.y32 + (T >= CHUNKED7 ? (size_t)CL * C : 0), l.lnx_w, l.lnx_b, ws.rk, v,
                            ws.g, ws.att);
         if ((rc = mm(c, l.att_output, false, ws.att, ACT_RESIDUAL, ws.x, nullptr, 1.f, ws.x))) return rc;
         // ---- channel mix

@@ -480,14 +480,11 @@ __global__ __launch_bounds__(256) void wkv56_split_kernel(Wkv56Args a) {
 // the chunks save (11.1 -> 12.9 us), at 96 it does not (14.4 -> 13.0): WKV_CHUNKED.
 //   WMODE 0: w[C] fp32 constant decay (RWKV-5);  WMODE 2: fp16 LoRA output [T, C] + t_decay (RWKV-6)
 // ---------------------------------------------------------------------------------------
-constexpr int CL = 16;                                // tokens per chunk
 constexpr int WKV_SEG = 2048;                         // tokens per segment
 constexpr int WKV_CHUNKED = 80;                       // calls of at least so many tokens run in chunks
-constexpr int PD = 8;                                 // chunks in flight; calls are padded to whole groups of PD chunks
 // one chunk's operands, in floats: r . A and decayed keys as [key block][lane][4], P as [key block][lane], A_16 [64], and
 // the values (fp16) as [value block][lane][4]
 constexpr int CH_R = 0, CH_K = CL * HS, CH_P = 2 * CL * HS, CH_A = CH_P + CL * CL, CH_V = CH_A + HS, CH_FLOATS = CH_V + CL * HS / 2;
-int wkv_chunks(int64_t tokens) { return (int)((tokens + CL * PD - 1) / (CL * PD)) * PD; }
 
 template <int WMODE>
 __global__ __launch_bounds__(256) void wkv56_chunk_kernel(Wkv56Args a, int H, int t_begin, float *__restrict__ scratch) {

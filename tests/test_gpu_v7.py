@@ -240,6 +240,31 @@ def test_v7_long_prompt_and_odd_lora_ranks():
         assert np.abs(_np(s) - ref.astype(np.float32)).max() <= 1e-2 * scale, i
 
 
+@pytest.mark.parametrize("T", [96, 97, 127, 129, 1025, 1041, 2100])
+def test_v7_chunked_recurrence(T):
+    """The recurrence in chunks of 16 tokens (calls of 96 tokens on; ragged last chunk and group of chunks, more than one
+    segment of 1024) against the token-by-token kernel (the same prompt in calls of 64), decays over their whole range.
+    What differs between the two are fp16 roundings (2^-11) of activations whose products sum in another order; a state is
+    a sum of products of two of them and of its own read-outs, so 2^-9 in the 2-norm for the first layer, and 2^-7 behind
+    the two further layers' roundings."""
+    cfg = dict(n_layer=3, n_embd=256, n_ffn=1024, vocab=300, lora=(32, 96, 32, 160))
+    ck = synth.make_checkpoint_v7(seed=75, **cfg)
+    for i in range(3):
+        w0 = ck[f"blocks.{i}.att.w0"]
+        w0.copy_(torch.linspace(-9.0, 9.0, 256)[torch.randperm(256, generator=torch.Generator().manual_seed(i))].reshape(w0.shape))
+    m = _x070()(ck, "cuda fp16")
+    toks = synth.random_tokens(T, cfg["vocab"], seed=T)
+    out, st = m.forward(toks, None, full_output=True)
+    parts, ref = [], None
+    for i in range(0, T, 64):
+        o, ref = m.forward(toks[i:i + 64], ref, full_output=True)
+        parts.append(o.reshape(-1, cfg["vocab"]).clone())
+    rel = lambda a, b: float((a.double() - b.double()).norm() / b.double().norm())
+    assert torch.isfinite(out).all()
+    assert rel(st[1], ref[1]) <= 2.0 ** -9, rel(st[1], ref[1])
+    assert rel(st[7], ref[7]) <= 2.0 ** -7 and rel(out, torch.cat(parts)) <= 2.0 ** -7, (rel(st[7], ref[7]), rel(out, torch.cat(parts)))
+
+
 def test_v7_short_call_lengths():
     """Calls of 2, 3, 9 and 16 tokens: every product of such a call goes through the 2..16-row streaming kernel
     (fp16 weights, LoRA products of odd ranks included)."""
