@@ -82,6 +82,49 @@ DEV void gemm_epilogue(float v, int t, int m, float rxm, float mxm, const GemmEp
         ((rwkv_half *)Y)[(size_t)t * ldy + m] = f2h(o);
 }
 
+// Eight consecutive outputs of one row, operands laid out for 16-byte accesses (dma_ok).
+DEV void affine8(float (&v)[8], int col, float s0t, float s2t, const GemmEpi &ep) {
+    const h16x8 rx8 = *(const h16x8 *)(ep.rx + col), mx8 = *(const h16x8 *)(ep.mx + col);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = epi_affine(v[e], (float)rx8[e], (float)mx8[e], s0t, s2t);
+}
+// activation / residual and store; a0 / a2: these outputs' share of the emitted row sums
+DEV void finish_row8(const float (&v)[8], int t, int col, const GemmEpi &ep, void *Y, int64_t ldy, float &a0, float &a2) {
+    if (ep.raw_f32) {
+        float *yo = (float *)Y + (size_t)t * ldy + col;
+        *(f32x4 *)yo = f32x4{v[0], v[1], v[2], v[3]};
+        *(f32x4 *)(yo + 4) = f32x4{v[4], v[5], v[6], v[7]};
+        return;
+    }
+    h16x8 res8 = {}, gate8 = {};
+    if (ep.act == ACT_RESIDUAL || ep.act == ACT_GATED_RESIDUAL) res8 = *(const h16x8 *)(ep.res + (size_t)t * ep.ldres + col);
+    if (ep.act == ACT_GATED_RESIDUAL) gate8 = *(const h16x8 *)(ep.gate + (size_t)t * ep.ldgate + col);
+    float o[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) o[e] = epi_act(v[e], (float)res8[e], (float)gate8[e], ep);
+    h16x8 y8;
+    if (ep.emit_ry) {
+        // what the scaling pass of the next product would make of the fp16 output: fp16(y * ry), sum y, sum y * my
+        const h16x8 ery8 = *(const h16x8 *)(ep.emit_ry + col), emy8 = *(const h16x8 *)(ep.emit_my + col);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const float yf = (float)(h16)o[e];
+            y8[e] = (h16)(yf * (float)ery8[e]);
+            a0 += yf;
+            a2 += yf * (float)emy8[e];
+        }
+    } else if (ep.out_dtype == RWKV_DT_F32) {
+        float *yo = (float *)Y + (size_t)t * ldy + col;
+        *(f32x4 *)yo = f32x4{round_h(o[0]), round_h(o[1]), round_h(o[2]), round_h(o[3])};
+        *(f32x4 *)(yo + 4) = f32x4{round_h(o[4]), round_h(o[5]), round_h(o[6]), round_h(o[7])};
+        return;
+    } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) y8[e] = (h16)o[e];
+    }
+    *(h16x8 *)((rwkv_half *)Y + (size_t)t * ldy + col) = y8;
+}
+
 // Split-K second pass: sums the KS partial slabs [KS][T][M] in slab order (deterministic) and runs the epilogue.
 // Four consecutive outputs per thread (M % 4 == 0).
 __global__ __launch_bounds__(256) void splitk_epilogue_kernel(int T, int M, int KS, const float *__restrict__ part, void *Y,
@@ -128,34 +171,9 @@ DEV void splitk_rows8(int T, int M, int ks_rt, const float *__restrict__ part, v
             }
         }
         float v[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-        if (ep.rx) {
-            const h16x8 rx8 = *(const h16x8 *)(ep.rx + col), mx8 = *(const h16x8 *)(ep.mx + col);
-            const float s0t = ep.s0[t], s2t = ep.s2[t];
-#pragma unroll
-            for (int e = 0; e < 8; ++e) v[e] = epi_affine(v[e], (float)rx8[e], (float)mx8[e], s0t, s2t);
-        }
-        if (ep.raw_f32) {
-            float *yo = (float *)Y + (size_t)t * ldy + col;
-            *(f32x4 *)yo = f32x4{v[0], v[1], v[2], v[3]};
-            *(f32x4 *)(yo + 4) = f32x4{v[4], v[5], v[6], v[7]};
-            continue;
-        }
-        h16x8 res8 = {}, gate8 = {};
-        if (ep.act == ACT_RESIDUAL || ep.act == ACT_GATED_RESIDUAL) res8 = *(const h16x8 *)(ep.res + (size_t)t * ep.ldres + col);
-        if (ep.act == ACT_GATED_RESIDUAL) gate8 = *(const h16x8 *)(ep.gate + (size_t)t * ep.ldgate + col);
-        float o[8];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) o[e] = epi_act(v[e], (float)res8[e], (float)gate8[e], ep);
-        if (ep.out_dtype == RWKV_DT_F32) {
-            float *yo = (float *)Y + (size_t)t * ldy + col;
-            *(f32x4 *)yo = f32x4{round_h(o[0]), round_h(o[1]), round_h(o[2]), round_h(o[3])};
-            *(f32x4 *)(yo + 4) = f32x4{round_h(o[4]), round_h(o[5]), round_h(o[6]), round_h(o[7])};
-        } else {
-            h16x8 y8;
-#pragma unroll
-            for (int e = 0; e < 8; ++e) y8[e] = (h16)o[e];
-            *(h16x8 *)((rwkv_half *)Y + (size_t)t * ldy + col) = y8;
-        }
+        if (ep.rx) affine8(v, col, ep.s0[t], ep.s2[t], ep);
+        float a0 = 0.f, a2 = 0.f;
+        finish_row8(v, t, col, ep, Y, ldy, a0, a2);
     }
 }
 
@@ -382,14 +400,21 @@ template <bool W_U8, int TM, int TN, int NW = 8, int NSTG = 0> struct DmaCfg {
     static constexpr size_t BODY = (size_t)NST * STAGE > (size_t)128 * STG_STRIDE * 4 ? (size_t)NST * STAGE : (size_t)128 * STG_STRIDE * 4;
     static constexpr size_t LDS = BODY + (W_U8 ? 2 * TM * 4 : 0);   // past the stages: the tile rows' sums s0, s2 (GemmEpi::parts)
 };
+// This workgroup's tile: the hardware deals consecutive workgroup ids round-robin to the 8 XCDs; undone here, so that
+// each XCD gets a contiguous range of tiles (those walk the T direction first, and share weight tiles in its L2).
+DEV int xcd_tile() {
+    const int bid = blockIdx.x;
+    return (gridDim.x & 7) == 0 ? (bid & 7) * (gridDim.x >> 3) + (bid >> 3) : bid;
+}
 // s_waitcnt immediates: vmcnt(n) alone, vmcnt(n) with lgkmcnt(0), lgkmcnt(n) alone
 constexpr int vm_only(int n) { return 0x0F70 | (n & 15) | ((n >> 4) << 14); }
 constexpr int vm_lgkm0(int n) { return 0x0070 | (n & 15) | ((n >> 4) << 14); }
 constexpr int lgkm_only(int n) { return 0xC07F | (n << 8); }
 
 template <bool W_U8, bool SPLIT, int TM, int TN, int NW = 8, int NSTG = 0>
-DEV void gemm_dma_body(int T, int N, int M, const h16 *__restrict__ A, int64_t lda, const void *__restrict__ Wv, int64_t ldw,
-                       void *__restrict__ Y, int64_t ldy, const GemmEpi &ep, int nk_split, float *__restrict__ part, int split) {
+DEV void gemm_dma_body(int bid, int T, int N, int M, const h16 *__restrict__ A, int64_t lda, const void *__restrict__ Wv,
+                       int64_t ldw, void *__restrict__ Y, int64_t ldy, const GemmEpi &ep, int nk_split,
+                       float *__restrict__ part, int split) {
     using Cfg = DmaCfg<W_U8, TM, TN, NW, NSTG>;
     constexpr int D_A = Cfg::A, D_STAGE = Cfg::STAGE, D_NST = Cfg::NST, AL = Cfg::AL, WL = Cfg::WL, MI = Cfg::MI, NI = Cfg::NI;
     static_assert((TM == 256 || TM == 128 || TM == 64) && (TN == 256 || TN == 128), "tile");
@@ -398,10 +423,7 @@ DEV void gemm_dma_body(int T, int N, int M, const h16 *__restrict__ A, int64_t l
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wr = wave / Cfg::WC, wc = wave % Cfg::WC;
     const int tiles_t = (T + TM - 1) / TM;
-    int bid = blockIdx.x;
-    if ((gridDim.x & 7) == 0) bid = (bid & 7) * (gridDim.x >> 3) + (bid >> 3);
     const int t0 = (bid % tiles_t) * TM, m0 = (bid / tiles_t) * TN;
-    if (m0 >= M) return;   // grouped launches size the grid for their widest member
     const int kbase = SPLIT ? split * nk_split : 0, nk = SPLIT ? nk_split : N / BK;
 
     // load sources; rows past the end re-read the last row (never stored)
@@ -784,18 +806,22 @@ template <bool W_U8, bool SPLIT, int TM, int TN, int NW, int NSTG>
 __global__ __launch_bounds__(64 * NW) void gemm_dma_kernel(int T, int N, int M, const h16 *__restrict__ A, int64_t lda,
                                                            const void *__restrict__ W, int64_t ldw, void *__restrict__ Y,
                                                            int64_t ldy, GemmEpi ep, int nk_split, float *__restrict__ part) {
-    gemm_dma_body<W_U8, SPLIT, TM, TN, NW, NSTG>(T, N, M, A, lda, W, ldw, Y, ldy, ep, nk_split, part, SPLIT ? blockIdx.y : 0);
+    gemm_dma_body<W_U8, SPLIT, TM, TN, NW, NSTG>(xcd_tile(), T, N, M, A, lda, W, ldw, Y, ldy, ep, nk_split, part, SPLIT ? blockIdx.y : 0);
 }
 
-// Up to four contractions [T, N] x [N, M_i] in one launch (blockIdx.y picks the operands), at full depth: short
-// calls, where each of them alone would split K and need a reduction pass.
+// Up to four contractions [T, N] x [N, M_i] in one launch: short calls, where each of them alone would split K and need
+// a reduction pass.  Register-staged tiles: blockIdx.y picks the member, the grid is as wide as the widest one.
+// Direct-to-LDS tiles: blockIdx.x runs over the tiles of all members, first[i] being member i's first.  (With a grid
+// for the widest member the tiles of the narrow ones all fell on the first XCDs: four first LoRA stages of 128, 128,
+// 128 and 512 outputs took two rounds on two XCDs with the others idle, 41 us instead of 23 with the 64 x 64 tile.)
 struct GemmGroup {
     const h16 *A[4];
     const void *W[4];
     void *Y[4];
-    int64_t lda, ldw[4];
+    int64_t lda, ldw[4], ldy[4];
     int M[4];
     float *part[4];   // split-K slabs of member i, [splits][T][M_i] (direct-to-LDS group only)
+    int first[4];     // members that are not there: INT_MAX
     int nk_split;
     GemmEpi ep[4];
 };
@@ -807,16 +833,32 @@ __global__ __launch_bounds__(64 * WT * WM) void gemm_group_kernel(int T, int N, 
                                                nullptr);
 }
 
-// the same through the direct-to-LDS kernel; blockIdx.z is the k split when the group has too few tiles for the chip
+DEV int group_member(const GemmGroup &g, int &tile) {
+    const int gi = (tile >= g.first[1]) + (tile >= g.first[2]) + (tile >= g.first[3]);
+    tile -= g.first[gi];
+    return gi;
+}
+// fills `first` for tiles of tm x tn; returns the tiles of the launch
+int64_t group_tiles(GemmGroup &g, int n, int64_t T, int tm, int tn) {
+    int64_t tiles = 0;
+    for (int i = 0; i < 4; ++i) {
+        g.first[i] = i < n ? (int)tiles : 0x7fffffff;
+        if (i < n) tiles += ((T + tm - 1) / tm) * ((g.M[i] + tn - 1) / tn);
+    }
+    return tiles;
+}
+
+// the same through the direct-to-LDS kernel; blockIdx.y is the k split when the group has too few tiles for the chip
 template <bool W_U8, bool SPLIT, int TM, int TN, int NW, int NSTG>
 __global__ __launch_bounds__(64 * NW) void gemm_dma_group_kernel(int T, int N, GemmGroup g) {
-    const int gi = blockIdx.y, M = g.M[gi];
-    gemm_dma_body<W_U8, SPLIT, TM, TN, NW, NSTG>(T, N, M, g.A[gi], g.lda, g.W[gi], g.ldw[gi], g.Y[gi], M, g.ep[gi], SPLIT ? g.nk_split : N / BK,
-                                       g.part[gi], SPLIT ? blockIdx.z : 0);
+    int tile = xcd_tile();
+    const int gi = group_member(g, tile), M = g.M[gi];
+    gemm_dma_body<W_U8, SPLIT, TM, TN, NW, NSTG>(tile, T, N, M, g.A[gi], g.lda, g.W[gi], g.ldw[gi], g.Y[gi], M, g.ep[gi],
+                                                 SPLIT ? g.nk_split : N / BK, g.part[gi], SPLIT ? blockIdx.y : 0);
 }
 
 template <bool W_U8, int TM, int TN, int NW, int NSTG>
-int launch_dma_group(const GemmGroup &g, int n, int64_t T, int64_t N, int64_t grid_x, int ks, hipStream_t st) {
+int launch_dma_group(GemmGroup &g, int n, int64_t T, int64_t N, int ks, hipStream_t st) {
     constexpr size_t lds = DmaCfg<W_U8, TM, TN, NW, NSTG>::LDS;
     static PerDeviceOnce once;
     bool *attr_done = once.slot();
@@ -829,12 +871,268 @@ int launch_dma_group(const GemmGroup &g, int n, int64_t T, int64_t N, int64_t gr
         if (e != hipSuccess) return (int)e;
         if (attr_done) *attr_done = true;
     }
-    const dim3 grid((unsigned)grid_x, (unsigned)n, (unsigned)ks);
+    const dim3 grid((unsigned)group_tiles(g, n, T, TM, TN), (unsigned)ks);
     if (ks > 1) hipLaunchKernelGGL((gemm_dma_group_kernel<W_U8, true, TM, TN, NW, NSTG>), grid, dim3(64 * NW), lds, st, (int)T, (int)N, g);
     else hipLaunchKernelGGL((gemm_dma_group_kernel<W_U8, false, TM, TN, NW, NSTG>), grid, dim3(64 * NW), lds, st, (int)T, (int)N, g);
     return RWKV_OK;
 }
 
+// ---- K over the waves of a workgroup: products whose large tiles would leave the chip idle --------------------
+// [T, 768..4096] x [.., 768..4096] products of a few hundred rows have 12 to 100 tiles of 128 x 128: most CUs idle, or a
+// K split whose fp32 slabs need a second launch.  Here the tile is 64 x 64 and K is split over the four waves of the
+// workgroup: wave w computes the WHOLE tile over the k-tiles w, w + 4, ... and the four partial tiles are added in wave
+// order through LDS (deterministic).  A 64 x 64 wave tile reads as few fragment bytes per MFMA as the tile allows
+// (32 x 32 wave tiles of the same workgroup tile: twice as many), and as a wave only ever reads what it has
+// loaded itself there is no barrier in the loop: each wave has its own stages (three of 12 KB for uint8 weights, two of
+// 16 KB for fp16), waits for its own direct-to-LDS loads and refills a stage as soon as its last fragment is back.
+// Fragments: half a k-tile at a time, the next half's reads in flight while one multiplies; a lane of half h takes
+// k 32 h + 8 s .. + 7 in step s for both operands, so uint8 fragments are 16-byte reads (two steps' worth each).
+// LDS swizzles as in gemm_dma_body.  Bound by how fast operand tiles reach the CU: 0.235 us per k-tile of 12-16 KB with
+// weights from HBM (0.15 from L2), whatever the number of workgroups, + 6 us of launch, first tiles and epilogue.
+// Measured, weights from HBM, us: fp16 [513 x 768] x [768 x 768] 11.9 -> 8.9, [333 x 2048] x [2048 x 2048] 19.3 (K split in
+// four, with its second pass) -> 13.5; uint8 with the scaling pass [256 x 768] x [768 x 768] 14.7 -> 10.9, [384 x 2048] x
+// [2048 x 2048] 22.0 -> 16.4, [256 x 4096] x [4096 x 4096] 26.1 -> 24.6; slower from the second round on ([513 x 4096] x
+// [4096 x 4096] 39.9 -> 52.4: one workgroup per CU, every round pays its first tiles) and for long K on few rows.
+// The same split with operands loaded straight into MFMA registers (no LDS; 16 rows x 64 bytes per load instruction)
+// took 2.5 times as long: the lanes of a quad then lie in four rows and nothing coalesces.
+template <bool W_U8> struct KwCfg {
+    static constexpr int A = 64 * BK * 2, W = W_U8 ? 64 * BK : 64 * BK * 2, STAGE = A + W;
+    static constexpr int NST = W_U8 ? 3 : 2, AL = A / 1024, WL = W / 1024, LOADS = AL + WL;
+    static constexpr int SW = 68;   // row stride (floats) of the partial tiles
+    static constexpr size_t REGION = (size_t)NST * STAGE, LDS = 4 * REGION + 2 * 64 * 4;
+    static_assert((size_t)64 * SW * 4 <= REGION, "partial tile");
+};
+template <bool W_U8>
+DEV void gemm_kw_body(int bid, int T, int N, int M, const h16 *__restrict__ A, int64_t lda, const void *__restrict__ Wv, int64_t ldw,
+                      void *__restrict__ Y, int64_t ldy, const GemmEpi &ep) {
+    using Cfg = KwCfg<W_U8>;
+    constexpr int NST = Cfg::NST, STAGE = Cfg::STAGE, AL = Cfg::AL, WL = Cfg::WL, SW = Cfg::SW;
+    extern __shared__ __align__(1024) unsigned char smem[];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int tiles_t = (T + 63) / 64;
+    const int t0 = (bid % tiles_t) * 64, m0 = (bid / tiles_t) * 64;
+    const int nk = N / BK, mine = (nk - wave + 3) / 4;   // k-tiles of this wave
+
+    unsigned char *base = smem + wave * Cfg::REGION;
+    const h16 *ga[AL];
+#pragma unroll
+    for (int i = 0; i < AL; ++i) {
+        const int r = i * 8 + (lane >> 3), c = (lane & 7) ^ ((r >> 1) & 7);
+        ga[i] = A + (size_t)min(t0 + r, T - 1) * lda + c * 8;
+    }
+    const unsigned char *gw[WL];
+#pragma unroll
+    for (int i = 0; i < WL; ++i) {
+        if (W_U8) {
+            const int r = i * 16 + (lane >> 2), c = (lane & 3) ^ ((r >> 2) & 3);
+            gw[i] = (const unsigned char *)Wv + (size_t)min(m0 + r, M - 1) * ldw + c * 16;
+        } else {
+            const int r = i * 8 + (lane >> 3), c = (lane & 7) ^ ((r >> 1) & 7);
+            gw[i] = (const unsigned char *)((const h16 *)Wv + (size_t)min(m0 + r, M - 1) * ldw + c * 8);
+        }
+    }
+    typedef __attribute__((address_space(1))) const void *gptr;
+    typedef __attribute__((address_space(3))) void *lptr;
+    // my i-th k-tile into stage byte offset so; past the end the last k-tile again (never multiplied)
+    auto issue = [&](int i, int so) {
+        const int kt = min(wave + 4 * i, nk - 1);
+#pragma unroll
+        for (int j = 0; j < AL; ++j)
+            __builtin_amdgcn_global_load_lds((gptr)(ga[j] + kt * BK), (lptr)(base + so + j * 1024), 16, 0, 0);
+#pragma unroll
+        for (int j = 0; j < WL; ++j)
+            __builtin_amdgcn_global_load_lds((gptr)(gw[j] + kt * BK * (W_U8 ? 1 : 2)), (lptr)(base + so + Cfg::A + j * 1024), 16, 0, 0);
+    };
+    f32x16 acc[2][2];   // [weight block][token block]
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int a = 0; a < 2; ++a)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[b][a][e] = 0.f;
+    // fragments: lane (row, h) takes k 32 h + 8 s .. + 7 in step s, for both operands
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)base;
+    const int row = lane & 31, h = lane >> 5;
+    uint32_t vA[4], vB[W_U8 ? 2 : 4];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) vA[s] = lds0 + row * 128 + (((4 * h + s) ^ ((row >> 1) & 7)) << 4);
+#pragma unroll
+    for (int s = 0; s < (W_U8 ? 2 : 4); ++s)
+        vB[s] = W_U8 ? lds0 + Cfg::A + row * 64 + (((2 * h + s) ^ ((row >> 2) & 3)) << 4)
+                     : lds0 + Cfg::A + row * 128 + (((4 * h + s) ^ ((row >> 1) & 7)) << 4);
+    constexpr int BN = W_U8 ? 1 : 2;
+    h16x8 fa[2][2][2];     // [set][step of the half][token block]
+    u32x4 fw[2][BN][2];    // [set][read][weight block]
+    auto ldhalf = [&](int set, int so, int p) {
+#pragma unroll
+        for (int j = 0; j < BN; ++j) {
+            const uint32_t pb = vB[W_U8 ? p : 2 * p + j] + so;
+            if constexpr (W_U8) {
+                asm volatile("ds_read_b128 %0, %1" : "=v"(fw[set][j][0]) : "v"(pb));
+                asm volatile("ds_read_b128 %0, %1 offset:2048" : "=v"(fw[set][j][1]) : "v"(pb));
+            } else {
+                asm volatile("ds_read_b128 %0, %1" : "=v"(fw[set][j][0]) : "v"(pb));
+                asm volatile("ds_read_b128 %0, %1 offset:4096" : "=v"(fw[set][j][1]) : "v"(pb));
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const uint32_t pa = vA[2 * p + j] + so;
+            asm volatile("ds_read_b128 %0, %1" : "=v"(fa[set][j][0]) : "v"(pa));
+            asm volatile("ds_read_b128 %0, %1 offset:4096" : "=v"(fa[set][j][1]) : "v"(pa));
+        }
+    };
+    const h16x2 off = {(h16)1023.5f, (h16)1023.5f};
+    auto mulhalf = [&](int set) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            h16x8 wf[2];
+#pragma unroll
+            for (int b = 0; b < 2; ++b) {
+                if constexpr (W_U8) {
+                    const uint32_t b0 = j ? fw[set][0][b].z : fw[set][0][b].x, b1 = j ? fw[set][0][b].w : fw[set][0][b].y;
+                    const h16x2 q0 = u8pair_lo_1024(b0) - off, q1 = u8pair_hi_1024(b0) - off;
+                    const h16x2 q2 = u8pair_lo_1024(b1) - off, q3 = u8pair_hi_1024(b1) - off;
+                    wf[b] = h16x8{q0.x, q0.y, q1.x, q1.y, q2.x, q2.y, q3.x, q3.y};
+                } else {
+                    wf[b] = __builtin_bit_cast(h16x8, fw[set][j][b]);
+                }
+            }
+#pragma unroll
+            for (int b = 0; b < 2; ++b)
+#pragma unroll
+                for (int a = 0; a < 2; ++a) acc[b][a] = __builtin_amdgcn_mfma_f32_32x32x16_f16(wf[b], fa[set][j][a], acc[b][a], 0, 0, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto reads_done = [&]() {
+        __builtin_amdgcn_s_waitcnt(lgkm_only(0));
+        __builtin_amdgcn_sched_barrier(0);
+    };
+#pragma unroll
+    for (int i = 0; i < NST; ++i) issue(i, i * STAGE);
+    bool lds_sums = false;
+    float *lsum = (float *)(smem + 4 * Cfg::REGION);
+    if constexpr (W_U8) {
+        if (ep.parts > 1) {
+            lds_sums = true;
+            if (tid < 128) {
+                const int r = tid & 63, which = tid >> 6, t = min(t0 + r, T - 1);
+                const float *p = (which ? ep.p2 : ep.p0) + (size_t)t * ep.parts;
+                float tot = 0.f;
+                for (int j = 0; j < ep.parts; j += 64) {
+                    f32x4 v[16];
+#pragma unroll
+                    for (int u = 0; u < 16; ++u) v[u] = j + 4 * u < ep.parts ? *(const f32x4 *)(p + j + 4 * u) : f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                    for (int u = 0; u < 16; ++u) tot = (((tot + v[u][0]) + v[u][1]) + v[u][2]) + v[u][3];
+                }
+                lsum[tid] = tot;
+            }
+        }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_waitcnt(vm_lgkm0((NST - 1) * Cfg::LOADS));
+    __builtin_amdgcn_sched_barrier(0);
+    ldhalf(0, 0, 0);
+    reads_done();
+    int so = 0;
+    for (int i = 0; i < mine; ++i) {
+        const int sn = so + STAGE >= NST * STAGE ? 0 : so + STAGE;
+        ldhalf(1, so, 1);
+        __builtin_amdgcn_sched_barrier(0);
+        mulhalf(0);
+        reads_done();                      // all my reads of this stage are back
+        issue(i + NST, so);
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_waitcnt(vm_only((NST - 1) * Cfg::LOADS));   // my next k-tile has landed
+        __builtin_amdgcn_sched_barrier(0);
+        ldhalf(0, sn, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        mulhalf(1);
+        reads_done();
+        so = sn;
+    }
+    // nothing may land in LDS or in a fragment register after this point (see gemm_dma_body)
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_waitcnt(0x0070);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int set = 0; set < 2; ++set) {
+#pragma unroll
+        for (int j = 0; j < BN; ++j)
+#pragma unroll
+            for (int b = 0; b < 2; ++b) asm volatile("" ::"v"(fw[set][j][b]));
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int a = 0; a < 2; ++a) asm volatile("" ::"v"(fa[set][j][a]));
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    float *mypart = (float *)base;
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int a = 0; a < 2; ++a)
+#pragma unroll
+            for (int g = 0; g < 4; ++g)
+                *(f32x4 *)(mypart + (a * 32 + row) * SW + b * 32 + 8 * g + 4 * h) =
+                    f32x4{acc[b][a][4 * g], acc[b][a][4 * g + 1], acc[b][a][4 * g + 2], acc[b][a][4 * g + 3]};
+    __syncthreads();
+    const bool emit = ep.emit_ry != nullptr;
+#pragma unroll 1
+    for (int i = tid; i < 64 * 8; i += 256) {
+        const int r = i >> 3, cq = i & 7, t = t0 + r, col = m0 + cq * 8;
+        const bool valid = t < T && col < M;
+        float a0 = 0.f, a2 = 0.f;
+        if (valid) {
+            const float *p = (const float *)smem + r * SW + cq * 8;
+            f32x4 lo = *(const f32x4 *)p, hi = *(const f32x4 *)(p + 4);
+#pragma unroll
+            for (int k = 1; k < 4; ++k) {
+                lo += *(const f32x4 *)(p + k * (Cfg::REGION / 4));
+                hi += *(const f32x4 *)(p + k * (Cfg::REGION / 4) + 4);
+            }
+            float v[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+            if constexpr (W_U8) {
+                const float s0t = lds_sums ? lsum[r] : ep.s0[t], s2t = lds_sums ? lsum[64 + r] : ep.s2[t];
+                affine8(v, col, s0t, s2t, ep);
+            }
+            finish_row8(v, t, col, ep, Y, ldy, a0, a2);
+        }
+        if (emit) {   // the eight threads of a row are neighbours in one wave; every lane takes part
+#pragma unroll
+            for (int o = 1; o < 8; o <<= 1) { a0 += __shfl_xor(a0, o, WAVE); a2 += __shfl_xor(a2, o, WAVE); }
+            if (valid && cq == 0) {
+                const size_t pi = (size_t)t * ((M + 63) / 64) + m0 / 64;
+                ep.emit_s0[pi] = a0;
+                ep.emit_s2[pi] = a2;
+            }
+        }
+    }
+}
+
+template <bool W_U8>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void gemm_kw_kernel(int T, int N, GemmGroup g) {
+    int tile = xcd_tile();
+    const int gi = group_member(g, tile), M = g.M[gi];
+    gemm_kw_body<W_U8>(tile, T, N, M, g.A[gi], g.lda, g.W[gi], g.ldw[gi], g.Y[gi], g.ldy[gi], g.ep[gi]);
+}
+
+template <bool W_U8>
+int launch_kw(GemmGroup &g, int n, int64_t T, int64_t N, hipStream_t st) {
+    constexpr size_t lds = KwCfg<W_U8>::LDS;
+    static PerDeviceOnce once;
+    bool *attr_done = once.slot();
+    if (!attr_done || !*attr_done) {
+        const hipError_t e = hipFuncSetAttribute((const void *)gemm_kw_kernel<W_U8>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        if (e != hipSuccess) return (int)e;
+        if (attr_done) *attr_done = true;
+    }
+    hipLaunchKernelGGL((gemm_kw_kernel<W_U8>), dim3((unsigned)group_tiles(g, n, T, 64, 64)), dim3(256), lds, st, (int)T, (int)N, g);
+    RWKV_LAUNCH_CHECK();
+    return RWKV_OK;
+}
 // second pass of a split group launch: member blockIdx.y, as splitk_epilogue8_kernel
 __global__ __launch_bounds__(256) void splitk_group_epilogue8_kernel(int T, int KS, GemmGroup g) {
     const int gi = blockIdx.y;
@@ -1196,10 +1494,10 @@ bool dma_ok(bool w_u8, int64_t N, int64_t M, const void *A, int64_t lda, const v
     return true;
 }
 
-// The direct-to-LDS tiles: rows and columns.  TILE_S4 is TILE_S with four stages.
-enum { TILE_L, TILE_S, TILE_S4, TILE_N, TILES };
+// The direct-to-LDS tiles: rows and columns.  TILE_S4 is TILE_S with four stages, TILE_K gemm_kw_kernel.
+enum { TILE_L, TILE_S, TILE_S4, TILE_N, TILE_K, TILES };
 struct TileDim { int tm, tn; };
-constexpr TileDim tile_dim[TILES] = {{256, 256}, {128, 128}, {128, 128}, {64, 128}};
+constexpr TileDim tile_dim[TILES] = {{256, 256}, {128, 128}, {128, 128}, {64, 128}, {64, 64}};
 
 // Cost model of a direct-to-LDS launch in microseconds, fitted to launches of the 7B shapes (20 to 4096 rows):
 // `tiles` tiles of nk k-tiles split c ways run in whole rounds over the 256 CUs; a k-tile step takes 1.75 us with
@@ -1208,7 +1506,8 @@ constexpr TileDim tile_dim[TILES] = {{256, 256}, {128, 128}, {128, 128}, {64, 12
 // the reduction pass; 12.8 for the 128 x 128 tile, 5.5 where two workgroups per CU overlap; 16.5 for the 64 x 128 one).
 // Four stages: launches of one round only (one workgroup per CU); its step grows from 0.38 us with 64 CUs busy to
 // 0.53 us with all of them.  The reduction pass of a split takes 2.5 us + 3.6 us per slab and 16 MB of fp32 output, at
-// least 4.5 us.
+// least 4.5 us.  The 64 x 64 tile with K over the waves: 0.245 us per k-tile, 4 us per round and 2.5 us per launch, never
+// split over workgroups.
 double dma_cost(int tile, int64_t T, int64_t tiles, int nk, int c, size_t out_bytes) {
     const int64_t wgs = tiles * c, rounds = (wgs + 255) / 256;
     const double reduce = c > 1 ? std::max(4.5, 2.5 + 3.6 * c * (double)out_bytes / (16 << 20)) : 0.0;
@@ -1216,7 +1515,8 @@ double dma_cost(int tile, int64_t T, int64_t tiles, int nk, int c, size_t out_by
         case TILE_L: return (double)rounds * (nk / c + (c > 1 ? 4.3 : 10.0)) * 1.75 + reduce;
         case TILE_S: return (double)rounds * (nk / c + (rounds > 1 ? 5.5 : 12.8)) * 0.573 + reduce;
         case TILE_S4: return rounds > 1 ? 1e30 : (nk / c + 22.0) * (0.34 + 0.19 * (double)wgs / 256) + reduce;
-        default: return T > 64 ? 1e30 : (double)rounds * (nk / c + 16.5) * 0.327 + reduce;
+        case TILE_N: return T > 64 ? 1e30 : (double)rounds * (nk / c + 16.5) * 0.327 + reduce;
+        default: return c > 1 ? 1e30 : (double)rounds * (nk * 0.245 + 4.0) + 2.5;
     }
 }
 
@@ -1294,6 +1594,11 @@ int launch_pick(int cfg, int ks, int64_t T, int64_t N, int64_t M, const rwkv_hal
         case CFG_DMA + TILE_S: return launch_dma<W_U8, 128, 128, 8, 0>(ks, T, N, M, A, lda, W, ldw, Y, ldy, ep, st);
         case CFG_DMA + TILE_S4: return launch_dma<W_U8, 128, 128, 8, 4>(ks, T, N, M, A, lda, W, ldw, Y, ldy, ep, st);
         case CFG_DMA + TILE_N: return launch_dma<W_U8, 64, 128, 4, 4>(ks, T, N, M, A, lda, W, ldw, Y, ldy, ep, st);
+        case CFG_DMA + TILE_K: {
+            GemmGroup g{};
+            g.A[0] = (const h16 *)A; g.W[0] = W; g.Y[0] = Y; g.lda = lda; g.ldw[0] = ldw; g.ldy[0] = ldy; g.M[0] = (int)M; g.ep[0] = ep;
+            return launch_kw<W_U8>(g, 1, T, N, st);
+        }
         default: return RWKV_E_DTYPE;
     }
 }
@@ -1400,7 +1705,7 @@ int gemm_group_launch(bool w_u8, int n, int64_t T, int64_t N, const rwkv_half *c
     for (int i = 0; i < n; ++i) {
         if (mats[i]->N != N) return RWKV_E_SHAPE;
         g.A[i] = (const h16 *)(prep ? xs[i] : x[i]);
-        g.W[i] = mats[i]->w; g.ldw[i] = mats[i]->ld; g.Y[i] = Y[i]; g.M[i] = (int)mats[i]->M;
+        g.W[i] = mats[i]->w; g.ldw[i] = mats[i]->ld; g.Y[i] = Y[i]; g.ldy[i] = mats[i]->M; g.M[i] = (int)mats[i]->M;
         g.ep[i] = eps[i];
         g.ep[i].ldres = g.ep[i].ldgate = mats[i]->M;
         if (w_u8) { g.ep[i].mx = mats[i]->mx; g.ep[i].rx = mats[i]->rx; g.ep[i].s0 = sums[i]; g.ep[i].s2 = sums[i] + T; }
@@ -1431,9 +1736,6 @@ int gemm_group_launch(bool w_u8, int n, int64_t T, int64_t N, const rwkv_half *c
         for (int i = 0; i < n; ++i) outs[i] = mats[i]->M;
         int ks = 1;
         const int tile = dma_tile(T, nk, n, outs, splitk_ws && m4 ? RWKV_SPLITK_WS_BYTES : 0, &ks);
-        int64_t grid_x = 0;
-        for (int i = 0; i < n; ++i)
-            grid_x = std::max<int64_t>(grid_x, ((T + tile_dim[tile].tm - 1) / tile_dim[tile].tm) * ((outs[i] + tile_dim[tile].tn - 1) / tile_dim[tile].tn));
         g.nk_split = nk / ks;
         if (ks > 1) {
             float *p = splitk_ws;
@@ -1441,10 +1743,11 @@ int gemm_group_launch(bool w_u8, int n, int64_t T, int64_t N, const rwkv_half *c
         }
         int rc;
         switch (tile) {
-            case TILE_L: rc = w_u8 ? launch_dma_group<true, 256, 256, 8, 0>(g, n, T, N, grid_x, ks, st) : launch_dma_group<false, 256, 256, 8, 0>(g, n, T, N, grid_x, ks, st); break;
-            case TILE_S: rc = w_u8 ? launch_dma_group<true, 128, 128, 8, 0>(g, n, T, N, grid_x, ks, st) : launch_dma_group<false, 128, 128, 8, 0>(g, n, T, N, grid_x, ks, st); break;
-            case TILE_S4: rc = w_u8 ? launch_dma_group<true, 128, 128, 8, 4>(g, n, T, N, grid_x, ks, st) : launch_dma_group<false, 128, 128, 8, 4>(g, n, T, N, grid_x, ks, st); break;
-            default: rc = w_u8 ? launch_dma_group<true, 64, 128, 4, 4>(g, n, T, N, grid_x, ks, st) : launch_dma_group<false, 64, 128, 4, 4>(g, n, T, N, grid_x, ks, st); break;
+            case TILE_L: rc = w_u8 ? launch_dma_group<true, 256, 256, 8, 0>(g, n, T, N, ks, st) : launch_dma_group<false, 256, 256, 8, 0>(g, n, T, N, ks, st); break;
+            case TILE_S: rc = w_u8 ? launch_dma_group<true, 128, 128, 8, 0>(g, n, T, N, ks, st) : launch_dma_group<false, 128, 128, 8, 0>(g, n, T, N, ks, st); break;
+            case TILE_S4: rc = w_u8 ? launch_dma_group<true, 128, 128, 8, 4>(g, n, T, N, ks, st) : launch_dma_group<false, 128, 128, 8, 4>(g, n, T, N, ks, st); break;
+            case TILE_K: rc = w_u8 ? launch_kw<true>(g, n, T, N, st) : launch_kw<false>(g, n, T, N, st); break;
+            default: rc = w_u8 ? launch_dma_group<true, 64, 128, 4, 4>(g, n, T, N, ks, st) : launch_dma_group<false, 64, 128, 4, 4>(g, n, T, N, ks, st); break;
         }
         if (rc) return rc;
         if (ks > 1) {

@@ -352,8 +352,8 @@ struct SeqWs {
     size_t total;
 };
 
-// most partial sums a row can have: one per 128 columns of the channel-mix key product, one per 64 channels of WKV
-int64_t parts_max(int64_t C, int64_t F) { return std::max((F + 127) / 128, (C + 63) / 64); }
+// most partial sums a row can have: one per 64 columns of the channel-mix key product
+int64_t parts_max(int64_t F) { return (F + 63) / 64; }
 
 SeqWs carve(void *base, int64_t T, int64_t C, int64_t F) {
     SeqWs w;
@@ -371,7 +371,7 @@ SeqWs carve(void *base, int64_t T, int64_t C, int64_t F) {
     w.xx_att = (rwkv_half *)take((size_t)C * 2);
     w.xx_ffn = (rwkv_half *)take((size_t)C * 2);
     w.sums = (float *)take((size_t)T * 8 * sizeof(float));
-    w.parts = (float *)take((size_t)T * 2 * parts_max(C, F) * sizeof(float));
+    w.parts = (float *)take((size_t)T * 2 * parts_max(F) * sizeof(float));
     w.splitk = (float *)take(RWKV_SPLITK_WS_BYTES);
     w.wkv = (float *)take(wkv4_scratch_bytes(T, C));
     w.total = (size_t)(p - (unsigned char *)base);

@@ -131,6 +131,22 @@ def test_mm8_seq_tile_edges(N, M, B):
     assert d.max() <= 1e-3 * np.sqrt(np.mean(ref ** 2)) + np.abs(ref).max() * 2 ** -10, d.max()
 
 
+@pytest.mark.parametrize("N,M,B", [(64, 64, 65), (128, 8, 100), (320, 72, 129), (768, 768, 513), (1024, 1000, 70), (2048, 2048, 333),
+                                   (4096, 1032, 256)])
+def test_64x64_tile_edges(N, M, B):
+    """The 64 x 64 tile with K over its four waves, both weight types: fewer k-tiles than waves, k-tiles that do not divide
+    by four, ragged rows and columns; bounds as in test_mm8_seq and test_gemm_f16."""
+    ops = _ops()
+    x, ref, (q, mx, rx, my, ry) = _mm8_case(N, M, B, N + M + B)
+    xt = torch.from_numpy(x).to(DEV)
+    d = np.abs(ops.cuda_mm8_seq(B, N, M, xt, q, mx, rx, my, ry).cpu().numpy().astype(np.float64) - ref)
+    assert d.max() <= 1e-3 * np.sqrt(np.mean(ref ** 2)) + np.abs(ref).max() * 2 ** -10, d.max()
+    w = (_rng(N + M).standard_normal((N, M)) * 0.02).astype(np.float16)
+    ref = x.astype(np.float64) @ w.astype(np.float64)
+    y = ops.matmul_float(xt, _to_dev_ic(w), output_dtype=torch.float32)
+    assert np.abs(y.cpu().numpy() - ref).max() <= 1e-4 * np.sqrt(np.mean(ref ** 2))
+
+
 @pytest.mark.parametrize("N,M", [(5120, 20480), (20480, 5120), (5120, 5120)])
 def test_mm8_seq_14b_call_length(N, M):
     """The launches of the 14B configuration at its own call length (1024 rows): 320 large
