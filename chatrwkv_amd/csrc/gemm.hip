@@ -82,20 +82,61 @@ DEV void gemm_epilogue(float v, int t, int m, float rxm, float mxm, const GemmEp
         ((rwkv_half *)Y)[(size_t)t * ldy + m] = f2h(o);
 }
 
-// Eight consecutive outputs of one row, operands laid out for 16-byte accesses (dma_ok).
-DEV void affine8(float (&v)[8], int col, float s0t, float s2t, const GemmEpi &ep) {
-    const h16x8 rx8 = *(const h16x8 *)(ep.rx + col), mx8 = *(const h16x8 *)(ep.mx + col);
+// Epilogue of a few consecutive outputs of one row, operands laid out as dma_ok asks.
+// n (< 4 or 8 in the last group of a width that is no multiple of it): values that are there
+template <class V, int K>
+DEV V load_n(const rwkv_half *p, int n) {
+    if (n >= K) return *(const V *)p;
+    V v = {};
+#pragma unroll
+    for (int e = 0; e < K; ++e)
+        if (e < n) v[e] = __builtin_bit_cast(h16, p[e]);
+    return v;
+}
+// May these outputs be stored 16 bytes at a time?  (An output width of 50277 has rows that start anywhere.)
+DEV bool wide_rows(int M, int64_t ldy, const void *Y) { return (((M | (int)ldy) & 7) | (int)((uintptr_t)Y & 15)) == 0; }
+typedef float f32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
+
+// Four outputs: fp32 results, and widths or strides that allow no aligned 16-byte stores of fp16 (no residual, gate or
+// emitted sums there).  Fp32 leaves 16 bytes at a time on whatever 4-byte boundary the row has.
+DEV void affine4(f32x4 &v, int col, int M, float s0t, float s2t, const GemmEpi &ep) {
+    const h16x4 rx4 = load_n<h16x4, 4>(ep.rx + col, M - col), mx4 = load_n<h16x4, 4>(ep.mx + col, M - col);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = epi_affine(v[e], (float)rx4[e], (float)mx4[e], s0t, s2t);
+}
+DEV void finish_row4(f32x4 v, int t, int col, int M, const GemmEpi &ep, void *Y, int64_t ldy) {
+    const int n = M - col;
+    const bool f32 = ep.raw_f32 || ep.out_dtype == RWKV_DT_F32;
+    const size_t at = (size_t)t * ldy + col;
+    if (!ep.raw_f32) {
+        h16x4 res4 = {}, gate4 = {};
+        if (ep.act == ACT_RESIDUAL || ep.act == ACT_GATED_RESIDUAL) res4 = *(const h16x4 *)(ep.res + (size_t)t * ep.ldres + col);
+        if (ep.act == ACT_GATED_RESIDUAL) gate4 = *(const h16x4 *)(ep.gate + (size_t)t * ep.ldgate + col);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = round_h(epi_act(v[e], (float)res4[e], (float)gate4[e], ep));
+    }
+    if (f32 && n >= 4) {
+        *(f32x4_a4 *)((float *)Y + at) = f32x4_a4{v[0], v[1], v[2], v[3]};
+        return;
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+        if (e < n) {
+            if (f32) ((float *)Y)[at + e] = v[e];
+            else ((rwkv_half *)Y)[at + e] = f2h(v[e]);
+        }
+}
+// Eight outputs.
+DEV void affine8(float (&v)[8], int col, int M, float s0t, float s2t, const GemmEpi &ep) {
+    const h16x8 rx8 = load_n<h16x8, 8>(ep.rx + col, M - col), mx8 = load_n<h16x8, 8>(ep.mx + col, M - col);
 #pragma unroll
     for (int e = 0; e < 8; ++e) v[e] = epi_affine(v[e], (float)rx8[e], (float)mx8[e], s0t, s2t);
 }
-// activation / residual and store; a0 / a2: these outputs' share of the emitted row sums
+DEV bool by_four(int M, int64_t ldy, const void *Y, const GemmEpi &ep) {
+    return ep.raw_f32 || ep.out_dtype == RWKV_DT_F32 || !wide_rows(M, ldy, Y);
+}
+// activation / residual and 16-byte store of fp16 outputs; a0 / a2: these outputs' share of the emitted row sums
 DEV void finish_row8(const float (&v)[8], int t, int col, const GemmEpi &ep, void *Y, int64_t ldy, float &a0, float &a2) {
-    if (ep.raw_f32) {
-        float *yo = (float *)Y + (size_t)t * ldy + col;
-        *(f32x4 *)yo = f32x4{v[0], v[1], v[2], v[3]};
-        *(f32x4 *)(yo + 4) = f32x4{v[4], v[5], v[6], v[7]};
-        return;
-    }
     h16x8 res8 = {}, gate8 = {};
     if (ep.act == ACT_RESIDUAL || ep.act == ACT_GATED_RESIDUAL) res8 = *(const h16x8 *)(ep.res + (size_t)t * ep.ldres + col);
     if (ep.act == ACT_GATED_RESIDUAL) gate8 = *(const h16x8 *)(ep.gate + (size_t)t * ep.ldgate + col);
@@ -113,18 +154,12 @@ DEV void finish_row8(const float (&v)[8], int t, int col, const GemmEpi &ep, voi
             a0 += yf;
             a2 += yf * (float)emy8[e];
         }
-    } else if (ep.out_dtype == RWKV_DT_F32) {
-        float *yo = (float *)Y + (size_t)t * ldy + col;
-        *(f32x4 *)yo = f32x4{round_h(o[0]), round_h(o[1]), round_h(o[2]), round_h(o[3])};
-        *(f32x4 *)(yo + 4) = f32x4{round_h(o[4]), round_h(o[5]), round_h(o[6]), round_h(o[7])};
-        return;
     } else {
 #pragma unroll
         for (int e = 0; e < 8; ++e) y8[e] = (h16)o[e];
     }
     *(h16x8 *)((rwkv_half *)Y + (size_t)t * ldy + col) = y8;
 }
-
 // Split-K second pass: sums the KS partial slabs [KS][T][M] in slab order (deterministic) and runs the epilogue.
 // Four consecutive outputs per thread (M % 4 == 0).
 __global__ __launch_bounds__(256) void splitk_epilogue_kernel(int T, int M, int KS, const float *__restrict__ part, void *Y,
@@ -171,7 +206,12 @@ DEV void splitk_rows8(int T, int M, int ks_rt, const float *__restrict__ part, v
             }
         }
         float v[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-        if (ep.rx) affine8(v, col, ep.s0[t], ep.s2[t], ep);
+        if (ep.rx) affine8(v, col, M, ep.s0[t], ep.s2[t], ep);
+        if (by_four(M, ldy, Y, ep)) {
+            finish_row4(f32x4{v[0], v[1], v[2], v[3]}, t, col, M, ep, Y, ldy);
+            finish_row4(f32x4{v[4], v[5], v[6], v[7]}, t, col + 4, M, ep, Y, ldy);
+            continue;
+        }
         float a0 = 0.f, a2 = 0.f;
         finish_row8(v, t, col, ep, Y, ldy, a0, a2);
     }
@@ -695,9 +735,9 @@ DEV void gemm_dma_body(int bid, int T, int N, int M, const h16 *__restrict__ A, 
     // does not).
     constexpr int CPR = TN / 8, RPI = 64 * NW / CPR;   // 8-wide chunks per tile row; rows one pass of the workgroup covers
     const int cq = tid % CPR, col = m0 + cq * 8;
-    const bool col_ok = col < M;   // M % 8 == 0
+    const bool col_ok = col < M;
     h16x8 rx8, mx8, ery8 = {}, emy8 = {};
-    if (W_U8 && col_ok) { rx8 = *(const h16x8 *)(ep.rx + col); mx8 = *(const h16x8 *)(ep.mx + col); }
+    if (W_U8 && col_ok) { rx8 = load_n<h16x8, 8>(ep.rx + col, M - col); mx8 = load_n<h16x8, 8>(ep.mx + col, M - col); }
     const bool emit = ep.emit_ry != nullptr;
     if (emit && col_ok) { ery8 = *(const h16x8 *)(ep.emit_ry + col); emy8 = *(const h16x8 *)(ep.emit_my + col); }
     const float *lsum = (const float *)(smem + Cfg::BODY);
@@ -707,12 +747,6 @@ DEV void gemm_dma_body(int bid, int T, int N, int M, const h16 *__restrict__ A, 
             const float s0t = lds_sums ? lsum[trow] : ep.s0[t], s2t = lds_sums ? lsum[TM + trow] : ep.s2[t];
 #pragma unroll
             for (int e = 0; e < 8; ++e) v[e] = epi_affine(v[e], (float)rx8[e], (float)mx8[e], s0t, s2t);
-        }
-        if (ep.raw_f32) {
-            float *yo = (float *)Y + (size_t)t * ldy + col;
-            *(f32x4 *)yo = f32x4{v[0], v[1], v[2], v[3]};
-            *(f32x4 *)(yo + 4) = f32x4{v[4], v[5], v[6], v[7]};
-            return;
         }
         h16x8 res8 = {}, gate8 = {};
         if (ep.act == ACT_RESIDUAL || ep.act == ACT_GATED_RESIDUAL) res8 = *(const h16x8 *)(ep.res + (size_t)t * ep.ldres + col);
@@ -731,10 +765,6 @@ DEV void gemm_dma_body(int bid, int T, int N, int M, const h16 *__restrict__ A, 
                 a2 += yf * (float)emy8[e];
             }
             *(h16x8 *)((rwkv_half *)Y + (size_t)t * ldy + col) = y8;
-        } else if (ep.out_dtype == RWKV_DT_F32) {
-            float *yo = (float *)Y + (size_t)t * ldy + col;
-            *(f32x4 *)yo = f32x4{round_h(o[0]), round_h(o[1]), round_h(o[2]), round_h(o[3])};
-            *(f32x4 *)(yo + 4) = f32x4{round_h(o[4]), round_h(o[5]), round_h(o[6]), round_h(o[7])};
         } else {
             h16x8 y8;
 #pragma unroll
@@ -762,6 +792,10 @@ DEV void gemm_dma_body(int bid, int T, int N, int M, const h16 *__restrict__ A, 
         constexpr int SW = Cfg::STG_STRIDE;   // row stride in floats: 4 rows apart = 32 banks apart for the two half-waves
         constexpr int WROWS = 32 * MI;        // tile rows of one wave row
         float *stg = (float *)smem;
+        // fp32 outputs, and rows that start on no 16-byte boundary, leave four at a time.  A 50277-wide head is such a
+        // product (through the register-staged kernel before): fp32 out [513 x 768] 109 -> 92 us, [1024 x 4096] 580 -> 542,
+        // uint8 weights, fp16 out 133 -> 87 and 706 -> 487.
+        const bool four = by_four(M, ldy, Y, ep);
         __syncthreads();   // every wave has read its last fragments
 #pragma unroll 1
         for (int h = 0; h < (TM + 127) / 128; ++h) {
@@ -781,6 +815,21 @@ DEV void gemm_dma_body(int bid, int T, int N, int M, const h16 *__restrict__ A, 
                 const int row = it * RPI + tid / CPR, t = t0 + h * 128 + row;
                 const bool valid = t < T && col_ok;
                 float a0 = 0.f, a2 = 0.f;
+                if (four) {
+                    if (t >= T) continue;
+#pragma unroll
+                    for (int g = 0; g < 2; ++g) {
+                        const int c = g * (TN / 2) + cq * 4;
+                        if (m0 + c >= M) continue;
+                        f32x4 v = *(const f32x4 *)(stg + row * SW + c);
+                        if constexpr (W_U8) {
+                            const int tr = h * 128 + row;
+                            affine4(v, m0 + c, M, lds_sums ? lsum[tr] : ep.s0[t], lds_sums ? lsum[TM + tr] : ep.s2[t], ep);
+                        }
+                        finish_row4(v, t, m0 + c, M, ep, Y, ldy);
+                    }
+                    continue;
+                }
                 if (valid) {
                     const f32x4 v0 = *(const f32x4 *)(stg + row * SW + cq * 8), v1 = *(const f32x4 *)(stg + row * SW + cq * 8 + 4);
                     float v[8] = {v0[0], v0[1], v0[2], v0[3], v1[0], v1[1], v1[2], v1[3]};
@@ -1079,12 +1128,27 @@ DEV void gemm_kw_body(int bid, int T, int N, int M, const h16 *__restrict__ A, i
                 *(f32x4 *)(mypart + (a * 32 + row) * SW + b * 32 + 8 * g + 4 * h) =
                     f32x4{acc[b][a][4 * g], acc[b][a][4 * g + 1], acc[b][a][4 * g + 2], acc[b][a][4 * g + 3]};
     __syncthreads();
-    const bool emit = ep.emit_ry != nullptr;
+    const bool emit = ep.emit_ry != nullptr, four = by_four(M, ldy, Y, ep);
 #pragma unroll 1
     for (int i = tid; i < 64 * 8; i += 256) {
         const int r = i >> 3, cq = i & 7, t = t0 + r, col = m0 + cq * 8;
         const bool valid = t < T && col < M;
         float a0 = 0.f, a2 = 0.f;
+        if (four) {
+            if (t >= T) continue;
+#pragma unroll
+            for (int g = 0; g < 2; ++g) {
+                const int c = g * 32 + cq * 4;
+                if (m0 + c >= M) continue;
+                const float *p = (const float *)smem + r * SW + c;
+                f32x4 v = *(const f32x4 *)p;
+#pragma unroll
+                for (int k = 1; k < 4; ++k) v += *(const f32x4 *)(p + k * (Cfg::REGION / 4));
+                if constexpr (W_U8) affine4(v, m0 + c, M, lds_sums ? lsum[r] : ep.s0[t], lds_sums ? lsum[64 + r] : ep.s2[t], ep);
+                finish_row4(v, t, m0 + c, M, ep, Y, ldy);
+            }
+            continue;
+        }
         if (valid) {
             const float *p = (const float *)smem + r * SW + cq * 8;
             f32x4 lo = *(const f32x4 *)p, hi = *(const f32x4 *)(p + 4);
@@ -1096,7 +1160,7 @@ DEV void gemm_kw_body(int bid, int T, int N, int M, const h16 *__restrict__ A, i
             float v[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
             if constexpr (W_U8) {
                 const float s0t = lds_sums ? lsum[r] : ep.s0[t], s2t = lds_sums ? lsum[64 + r] : ep.s2[t];
-                affine8(v, col, s0t, s2t, ep);
+                affine8(v, col, M, s0t, s2t, ep);
             }
             finish_row8(v, t, col, ep, Y, ldy, a0, a2);
         }
@@ -1479,12 +1543,16 @@ int launch_cfg(int64_t T, int64_t N, int64_t M, const rwkv_half *A, int64_t lda,
     return RWKV_OK;
 }
 
-// what gemm_dma_kernel assumes: whole k-tiles, 16-byte rows and row starts for its loads and its eight-wide epilogue
+// what the direct-to-LDS kernels assume: whole k-tiles, 16-byte rows and row starts for their loads, and for the eight-wide
+// epilogue unless the outputs are stored plainly (four at a time then, any width, stride and boundary)
 bool dma_ok(bool w_u8, int64_t N, int64_t M, const void *A, int64_t lda, const void *W, int64_t ldw, const void *Y, int64_t ldy,
             const GemmEpi &ep) {
     auto a16 = [](const void *p) { return (((uintptr_t)p) & 15) == 0; };
-    if ((N % BK) || (M & 7) || (lda & 7) || (ldw & (w_u8 ? 15 : 7)) || (ldy & 7)) return false;
-    if (!a16(A) || !a16(W) || !a16(Y)) return false;
+    if ((N % BK) || (lda & 7) || (ldw & (w_u8 ? 15 : 7))) return false;
+    // output rows that are not made of aligned 16-byte pieces: plain stores only
+    const bool wide = !(M & 7) && !(ldy & 7) && a16(Y);
+    if (!wide && (ep.act == ACT_RESIDUAL || ep.act == ACT_GATED_RESIDUAL || ep.emit_ry)) return false;
+    if (!a16(A) || !a16(W)) return false;
     if (w_u8 && (!ep.rx || !ep.mx || !ep.s0 || !ep.s2 || !a16(ep.rx) || !a16(ep.mx))) return false;
     if (!w_u8 && ep.rx) return false;
     if (ep.act == ACT_RESIDUAL || ep.act == ACT_GATED_RESIDUAL)
@@ -1612,7 +1680,7 @@ int launch_pick(int cfg, int ks, int64_t T, int64_t N, int64_t M, const rwkv_hal
 //   3          everything else: 128 x 128 tiles, 4 k-tiles of prefetch
 int pick_cfg(int64_t T, int64_t N, int64_t M, bool w_u8, bool alone, bool dma, size_t split_bytes, int *ks) {
     *ks = 1;
-    const size_t ws = !(M & 3) ? split_bytes : 0;
+    const size_t ws = !(M & 7) ? split_bytes : 0;   // the slabs and the reduction pass are eight outputs wide
     if (dma && !alone) {
         const int64_t tiles = ((T + 127) / 128) * ((M + 127) / 128);
         *ks = dma_split(TILE_S, T, tiles, (int)(N / BK), (size_t)(T * M) * sizeof(float), ws);
@@ -1701,7 +1769,7 @@ int gemm_group_launch(bool w_u8, int n, int64_t T, int64_t N, const rwkv_half *c
         hipLaunchKernelGGL(mm8_prepare_group_kernel, dim3((unsigned)((T + 3) / 4), (unsigned)n), dim3(256), 0, st, (int)T, (int)N, p);
     }
     int64_t tiles = 0, max_out = 0;   // tiles: register-staged fallback
-    bool dma = true, m4 = true;
+    bool dma = true, m8 = true;
     for (int i = 0; i < n; ++i) {
         if (mats[i]->N != N) return RWKV_E_SHAPE;
         g.A[i] = (const h16 *)(prep ? xs[i] : x[i]);
@@ -1712,7 +1780,7 @@ int gemm_group_launch(bool w_u8, int n, int64_t T, int64_t N, const rwkv_half *c
         if (parts > 1) { g.ep[i].parts = parts; g.ep[i].p0 = sums[i] + 2 * T; g.ep[i].p2 = sums[i] + 2 * T + (size_t)T * parts; }
         tiles = std::max<int64_t>(tiles, ((T + 127) / 128) * ((mats[i]->M + 127) / 128));
         max_out = std::max<int64_t>(max_out, T * mats[i]->M);
-        m4 = m4 && !(mats[i]->M & 3);
+        m8 = m8 && !(mats[i]->M & 7);
         dma = dma && dma_ok(w_u8, N, mats[i]->M, g.A[i], N, g.W[i], g.ldw[i], g.Y[i], mats[i]->M, g.ep[i]);
     }
     {
@@ -1735,7 +1803,7 @@ int gemm_group_launch(bool w_u8, int n, int64_t T, int64_t N, const rwkv_half *c
         int64_t outs[4];
         for (int i = 0; i < n; ++i) outs[i] = mats[i]->M;
         int ks = 1;
-        const int tile = dma_tile(T, nk, n, outs, splitk_ws && m4 ? RWKV_SPLITK_WS_BYTES : 0, &ks);
+        const int tile = dma_tile(T, nk, n, outs, splitk_ws && m8 ? RWKV_SPLITK_WS_BYTES : 0, &ks);
         g.nk_split = nk / ks;
         if (ks > 1) {
             float *p = splitk_ws;

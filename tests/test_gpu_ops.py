@@ -147,6 +147,23 @@ def test_64x64_tile_edges(N, M, B):
     assert np.abs(y.cpu().numpy() - ref).max() <= 1e-4 * np.sqrt(np.mean(ref ** 2))
 
 
+@pytest.mark.parametrize("N,M,B", [(64, 33, 40), (128, 203, 70), (192, 1001, 300), (2048, 257, 129), (768, 50277, 130), (256, 4099, 1025)])
+def test_odd_output_widths(N, M, B):
+    """Output rows that start on no 16-byte boundary and end inside a group of eight, both weight types and output types, in
+    calls of every tile; bounds as in test_mm8_seq and test_gemm_f16."""
+    ops = _ops()
+    x, ref, (q, mx, rx, my, ry) = _mm8_case(N, M, B, N + M + B)
+    xt = torch.from_numpy(x).to(DEV)
+    d = np.abs(ops.cuda_mm8_seq(B, N, M, xt, q, mx, rx, my, ry).cpu().numpy().astype(np.float64) - ref)
+    assert d.max() <= 1e-3 * np.sqrt(np.mean(ref ** 2)) + np.abs(ref).max() * 2 ** -10, d.max()
+    w = (_rng(N + M).standard_normal((N, M)) * 0.02).astype(np.float16)
+    ref = x.astype(np.float64) @ w.astype(np.float64)
+    wt = _to_dev_ic(w)
+    for dt, tol in ((torch.float32, 0.0), (torch.float16, np.abs(ref).max() * 2 ** -10)):
+        y = ops.matmul_float(xt, wt, output_dtype=dt).cpu().numpy().astype(np.float64)
+        assert np.abs(y - ref).max() <= 1e-4 * np.sqrt(np.mean(ref ** 2)) + tol
+
+
 @pytest.mark.parametrize("N,M", [(5120, 20480), (20480, 5120), (5120, 5120)])
 def test_mm8_seq_14b_call_length(N, M):
     """The launches of the 14B configuration at its own call length (1024 rows): 320 large
