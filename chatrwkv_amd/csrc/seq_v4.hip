@@ -157,9 +157,9 @@ __global__ __launch_bounds__(256) void ln_f32_f16_kernel(int C, const float *__r
 // operations in the same order as in lnmix_seq_kernel, so the two agree bit for bit.
 // PRE: the mix / scale vectors too are requested at the top (3 NJ CH more registers per thread: shorter chain, fewer
 // workgroups per CU -- for short calls, where a CU has one or two rows anyway).
-template <int NJ, int CH, bool PRE>
-__global__ __launch_bounds__(256) void lnmix_seq_fast_kernel(SeqMixArgs a) {
-    __shared__ float red[4 * 2 * NJ > 12 ? 4 * 2 * NJ : 12];
+template <int NJ, int CH, bool PRE, int NT>
+__global__ __launch_bounds__(NT) void lnmix_seq_fast_kernel(SeqMixArgs a) {
+    __shared__ float red[NT / 64 * (2 * NJ > 3 ? 2 * NJ : 3)];
     const int t = blockIdx.x, C = a.C, nch = C >> 3;
     const rwkv_half *x = a.x + (size_t)t * C;
     const bool shift = a.sx != nullptr, prev_row = shift && t > 0;
@@ -170,7 +170,7 @@ __global__ __launch_bounds__(256) void lnmix_seq_fast_kernel(SeqMixArgs a) {
     h16x8 xv[CH], pxv[CH], lv[CH], wv[CH], bv[CH], mv[PRE ? NJ : 1][CH], rv[PRE ? NJ : 1][CH], yv[PRE ? NJ : 1][CH];
 #pragma unroll
     for (int c = 0; c < CH; ++c) {
-        const int j8 = min((int)threadIdx.x + c * 256, nch - 1);   // chunks past the end repeat the last one (unused)
+        const int j8 = min((int)threadIdx.x + c * NT, nch - 1);   // chunks past the end repeat the last one (unused)
         xv[c] = *(const h16x8 *)(x + 8 * j8);
         pxv[c] = *(const h16x8 *)(xp + 8 * j8);
         lv[c] = *(const h16x8 *)(xl + 8 * j8);
@@ -187,7 +187,7 @@ __global__ __launch_bounds__(256) void lnmix_seq_fast_kernel(SeqMixArgs a) {
     float st[3] = {0.f, 0.f, 0.f};
 #pragma unroll
     for (int c = 0; c < CH; ++c)
-        if ((int)threadIdx.x + c * 256 < nch) {
+        if ((int)threadIdx.x + c * NT < nch) {
 #pragma unroll
             for (int e = 0; e < 8; ++e) { st[0] += (float)xv[c][e]; st[1] += (float)pxv[c][e]; }
             if (commit)   // the last row's statistics: only the workgroup that writes the new state needs them
@@ -199,7 +199,7 @@ __global__ __launch_bounds__(256) void lnmix_seq_fast_kernel(SeqMixArgs a) {
     st[0] = st[1] = st[2] = 0.f;
 #pragma unroll
     for (int c = 0; c < CH; ++c)
-        if ((int)threadIdx.x + c * 256 < nch) {
+        if ((int)threadIdx.x + c * NT < nch) {
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
                 const float d = (float)xv[c][e] - mean, pd = (float)pxv[c][e] - pmean;
@@ -220,7 +220,7 @@ __global__ __launch_bounds__(256) void lnmix_seq_fast_kernel(SeqMixArgs a) {
     for (int i = 0; i < 2 * NJ; ++i) acc[i] = 0.f;
 #pragma unroll
     for (int c = 0; c < CH; ++c) {
-        const int j8 = threadIdx.x + c * 256;
+        const int j8 = threadIdx.x + c * NT;
         if (j8 >= nch) break;
         h16x8 xx, pv;
 #pragma unroll
@@ -287,28 +287,33 @@ __global__ __launch_bounds__(256) void lnmix_seq_fast_kernel(SeqMixArgs a) {
 
 }  // namespace
 
-template <int CH, bool PRE>
+template <int CH, bool PRE, int NT = 256>
 static bool lnmix_seq_fast_launch(const SeqMixArgs &a, int nj, hipStream_t st) {
-    const dim3 grid((unsigned)a.T), block(256);
+    const dim3 grid((unsigned)a.T), block(NT);
     switch (nj) {
-        case 1: hipLaunchKernelGGL((lnmix_seq_fast_kernel<1, CH, PRE>), grid, block, 0, st, a); break;
-        case 2: hipLaunchKernelGGL((lnmix_seq_fast_kernel<2, CH, PRE>), grid, block, 0, st, a); break;
-        case 3: hipLaunchKernelGGL((lnmix_seq_fast_kernel<3, CH, PRE>), grid, block, 0, st, a); break;
-        case 4: hipLaunchKernelGGL((lnmix_seq_fast_kernel<4, CH, PRE && CH <= 2>), grid, block, 0, st, a); break;
-        case 6: hipLaunchKernelGGL((lnmix_seq_fast_kernel<6, CH, PRE && CH <= 1>), grid, block, 0, st, a); break;
+        case 1: hipLaunchKernelGGL((lnmix_seq_fast_kernel<1, CH, PRE, NT>), grid, block, 0, st, a); break;
+        case 2: hipLaunchKernelGGL((lnmix_seq_fast_kernel<2, CH, PRE, NT>), grid, block, 0, st, a); break;
+        case 3: hipLaunchKernelGGL((lnmix_seq_fast_kernel<3, CH, PRE, NT>), grid, block, 0, st, a); break;
+        case 4: hipLaunchKernelGGL((lnmix_seq_fast_kernel<4, CH, PRE && CH <= 2, NT>), grid, block, 0, st, a); break;
+        case 6: hipLaunchKernelGGL((lnmix_seq_fast_kernel<6, CH, PRE && CH <= 1 && NT == 256, NT>), grid, block, 0, st, a); break;
         default: return false;
     }
     return true;
 }
 
 int lnmix_seq_launch(const SeqMixArgs &a, int nj, hipStream_t st) {
-    // rows of up to 8192 channels: the register-resident kernel (1, 2 or 4 chunks of 8 channels per thread); calls of
-    // up to 512 rows also hold the mix and scale vectors in registers
+    // Rows of up to 8192 channels: the register-resident kernel (1, 2 or 4 chunks of 8 channels per thread).  Calls of up
+    // to 512 rows have one or two rows per CU: there a row's own chain of conversions and mixes is the time, so rows of
+    // more than 2048 channels get 512 threads instead of 256 (4096 channels, us: three mixes 45 rows 10.8 -> 8.2, two mixes
+    // 256 rows 10.0 -> 8.0, six mixes without scaling 40 rows 13.2 -> 8.8, 400 rows 17.2 -> 12.2; 1024 rows 20.7 / 21.0,
+    // bound by instruction issue either way), and up to 4096 the mix and scale vectors are requested at the top too, except
+    // for six mixes.  Several rows per workgroup, sharing vectors and the previous row's statistics: slower at every length
+    // (1024 rows 21.8 with two, 33 with four).
     if (a.C <= 8192 && (nj == 1 || nj == 2 || nj == 3 || nj == 4 || nj == 6)) {
         const bool pre = a.T <= 512;
         if (a.C <= 2048) pre ? lnmix_seq_fast_launch<1, true>(a, nj, st) : lnmix_seq_fast_launch<1, false>(a, nj, st);
-        else if (a.C <= 4096) pre ? lnmix_seq_fast_launch<2, true>(a, nj, st) : lnmix_seq_fast_launch<2, false>(a, nj, st);
-        else lnmix_seq_fast_launch<4, false>(a, nj, st);
+        else if (a.C <= 4096) pre ? lnmix_seq_fast_launch<1, true, 512>(a, nj, st) : lnmix_seq_fast_launch<2, false>(a, nj, st);
+        else pre ? lnmix_seq_fast_launch<2, false, 512>(a, nj, st) : lnmix_seq_fast_launch<4, false>(a, nj, st);
         RWKV_LAUNCH_CHECK();
         return RWKV_OK;
     }

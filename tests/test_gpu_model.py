@@ -746,6 +746,21 @@ def test_handover_against_scaling_pass(shape, monkeypatch):
             assert float((a.float() - b.float()).abs().max()) <= 2e-3 * s, (T, i)
 
 
+@pytest.mark.parametrize("C,T", [(2112, 37), (4096, 512), (5120, 33)])
+def test_short_calls_of_wide_rows(C, T):
+    """Rows of more than 2048 channels in calls of up to 512 tokens (512 threads per row in the LayerNorm-and-mix kernel):
+    one that ends inside a thread's last chunk, the widest with one chunk per thread, and one with two."""
+    ck = synth.make_checkpoint(version=4, n_layer=1, n_embd=C, n_ffn=512, vocab=300, seed=C)
+    m, o = _rwkv()(ck, "cuda fp16i8", verbose=False), OracleRWKV(ck, "cuda fp16i8")
+    toks = synth.random_tokens(T, 300, seed=T)
+    out, st = m.forward(toks, None)
+    ref, ost = o.forward(toks, None)
+    assert np.abs(_np(out) - ref).max() <= LOGIT_TOL
+    for a, b in zip(st, ost):
+        b = np.asarray(b, dtype=np.float32)
+        assert np.abs(_np(a).reshape(b.shape) - b).max() <= 1e-2 * max(float(np.abs(b).max()), 1.0)
+
+
 @pytest.mark.parametrize("L", [8, 32])
 def test_depth_oracle_parity(L, capsys):
     """Eight layers, and all 32 layers, of the 7B RWKV-4 shape under 'cuda fp16i8' against the oracle (short vocabulary;
