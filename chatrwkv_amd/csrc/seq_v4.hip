@@ -309,11 +309,16 @@ int lnmix_seq_launch(const SeqMixArgs &a, int nj, hipStream_t st) {
     // bound by instruction issue either way), and up to 4096 the mix and scale vectors are requested at the top too, except
     // for six mixes.  Several rows per workgroup, sharing vectors and the previous row's statistics: slower at every length
     // (1024 rows 21.8 with two, 33 with four).
+    // Calls of up to 16 rows keep 256 threads: they are bound by streaming the weights, and they are where a conversation
+    // starts.  RWKV-7 normalises read-outs of a nearly empty state there, which blows up the last bit of a LayerNorm sum:
+    // after 15 tokens of the 7B shape the two thread counts' states differ by 2 % of their norm, 0.6 rms at most (after
+    // 777 tokens 0.5 %, 0.06).
     if (a.C <= 8192 && (nj == 1 || nj == 2 || nj == 3 || nj == 4 || nj == 6)) {
-        const bool pre = a.T <= 512;
+        const bool pre = a.T <= 512, wide = pre && a.T > 16;
         if (a.C <= 2048) pre ? lnmix_seq_fast_launch<1, true>(a, nj, st) : lnmix_seq_fast_launch<1, false>(a, nj, st);
-        else if (a.C <= 4096) pre ? lnmix_seq_fast_launch<1, true, 512>(a, nj, st) : lnmix_seq_fast_launch<2, false>(a, nj, st);
-        else pre ? lnmix_seq_fast_launch<2, false, 512>(a, nj, st) : lnmix_seq_fast_launch<4, false>(a, nj, st);
+        else if (a.C <= 4096) wide ? lnmix_seq_fast_launch<1, true, 512>(a, nj, st)
+                                   : pre ? lnmix_seq_fast_launch<2, true>(a, nj, st) : lnmix_seq_fast_launch<2, false>(a, nj, st);
+        else wide ? lnmix_seq_fast_launch<2, false, 512>(a, nj, st) : lnmix_seq_fast_launch<4, false>(a, nj, st);
         RWKV_LAUNCH_CHECK();
         return RWKV_OK;
     }

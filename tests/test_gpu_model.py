@@ -746,10 +746,10 @@ def test_handover_against_scaling_pass(shape, monkeypatch):
             assert float((a.float() - b.float()).abs().max()) <= 2e-3 * s, (T, i)
 
 
-@pytest.mark.parametrize("C,T", [(2112, 37), (4096, 512), (5120, 33)])
+@pytest.mark.parametrize("C,T", [(2112, 37), (4096, 512), (5120, 33), (4096, 16), (4096, 17), (5120, 16)])
 def test_short_calls_of_wide_rows(C, T):
-    """Rows of more than 2048 channels in calls of up to 512 tokens (512 threads per row in the LayerNorm-and-mix kernel):
-    one that ends inside a thread's last chunk, the widest with one chunk per thread, and one with two."""
+    """Rows of more than 2048 channels in calls of 17 to 512 tokens (512 threads per row in the LayerNorm-and-mix kernel; 256
+    up to 16): one that ends inside a thread's last chunk, the widest with one chunk per thread, and one with two."""
     ck = synth.make_checkpoint(version=4, n_layer=1, n_embd=C, n_ffn=512, vocab=300, seed=C)
     m, o = _rwkv()(ck, "cuda fp16i8", verbose=False), OracleRWKV(ck, "cuda fp16i8")
     toks = synth.random_tokens(T, 300, seed=T)
