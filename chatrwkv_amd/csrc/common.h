@@ -125,6 +125,7 @@ DEV float div_acc(float n, float d) {
     const float r = __builtin_amdgcn_rcpf(d), q = n * r;
     return __builtin_fmaf(__builtin_fmaf(-d, q, n), r, q);
 }
-DEV float sigmoid_acc(float x) { return div_acc(1.f, 1.f + __expf(fminf(-x, 80.f))); }
+DEV float at_most(float x, float m) { return x > m ? m : x; }   // fminf would turn a NaN into m
+DEV float sigmoid_acc(float x) { return div_acc(1.f, 1.f + __expf(at_most(-x, 80.f))); }
 
 DEV float sigmoidf_(float x) { return 1.f / (1.f + __expf(-x)); }

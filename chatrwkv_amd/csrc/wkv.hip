@@ -474,6 +474,8 @@ __global__ __launch_bounds__(256) void wkv56_split_kernel(Wkv56Args a) {
 //                        operand in fragment order (five loads per wave and chunk) and pads the chunks to whole
 //                        groups of PD, so that PD chunks are in flight with no load, store or wait under a branch.
 // Raw y goes to an fp32 [T, C] scratch; GroupNorm and the gate need the whole head and follow in wkv56_gn_kernel.
+// A value that overflowed to infinity makes NaN of its column in the whole chunk, the up to 15 tokens before it included (a
+// matrix product multiplies it by their zeros of P); the tokens after it and the state are lost either way.
 // Calls longer than WKV_SEG tokens run in segments, which bounds the scratch between the two kernels.
 // Measured per layer, 64 heads, RWKV-6 (recurrence token by token -> chunks, both without GroupNorm): 1024 tokens 111 ->
 // 47 us, 256 tokens 29.6 -> 18.4; RWKV-5, 32 heads, 333 tokens 29.3 -> 17.9.  At 64 tokens the second launch costs what
@@ -506,7 +508,7 @@ __global__ __launch_bounds__(256) void wkv56_chunk_kernel(Wkv56Args a, int H, in
     for (int e = 0; e < 4; ++e) {
         const int j = h * HS + 4 * g + e;
         u4[e] = a.u[j];
-        w4[e] = WMODE == 2 ? exp_acc(-exp_acc(fminf(a.t_decay[j] + (float)x8[e], 88.f))) : ((const float *)a.w)[j];
+        w4[e] = WMODE == 2 ? exp_acc(-exp_acc(at_most(a.t_decay[j] + (float)x8[e], 88.f))) : ((const float *)a.w)[j];
         r4[e] = live ? (float)r8[e] : 0.f;
         k4[e] = live ? (float)k8[e] : 0.f;
         w4[e] = live ? w4[e] : 1.f;

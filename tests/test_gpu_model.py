@@ -427,6 +427,21 @@ def test_v56_chunked_recurrence(ver, T):
     assert rel(st[4], ref[4]) <= 2.0 ** -8 and rel(out, want) <= 2.0 ** -8, (rel(st[4], ref[4]), rel(out, want))
 
 
+def test_v6_chunked_recurrence_keeps_nan():
+    """A decay that is no number stays one in the chunked recurrence (80 tokens on), as in the token-by-token kernels."""
+    from chatrwkv_amd import synth
+    from chatrwkv_amd.model import RWKV
+    ck = synth.make_checkpoint(version=6, n_layer=1, n_embd=128, n_ffn=448, vocab=211, seed=5, affine=True)
+    ck["blocks.0.att.time_decay"].view(-1)[70] = float("nan")
+    m = RWKV(ck, "cuda fp16", verbose=False)
+    toks = synth.random_tokens(81, 211, seed=3)
+    for n in (64, 81):
+        out, st = m.forward(toks[:n], None)
+        bad = torch.isnan(st[1].reshape(2, 64, 64))
+        assert torch.isnan(out).all() and not bad[0].any(), n
+        assert bad[1, 6].all() and int(bad.sum()) == 64, (n, int(bad.sum()))   # key 70 - 64 of head 1, all its values
+
+
 @pytest.mark.parametrize("ver,tag", [(4, "v4"), (5, "v5_0"), (5.1, "v5_1"), (5.2, "v5_2"), (6, "v6_0")])
 def test_fp16_strategy_against_reference_half_run(ver, tag):
     """'cuda fp16' on the GPU against the logits and states the reference itself produced under 'cpu fp16'

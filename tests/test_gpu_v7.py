@@ -265,6 +265,20 @@ def test_v7_chunked_recurrence(T):
     assert rel(st[7], ref[7]) <= 2.0 ** -7 and rel(out, torch.cat(parts)) <= 2.0 ** -7, (rel(st[7], ref[7]), rel(out, torch.cat(parts)))
 
 
+@pytest.mark.parametrize("name", ["w0", "a0", "v0"])
+def test_v7_chunked_recurrence_keeps_nan(name):
+    """A gate that is no number stays one in the chunked recurrence (96 tokens on), as in the token-by-token kernels."""
+    ck = synth.make_checkpoint_v7(n_layer=2, n_embd=128, n_ffn=512, vocab=300, seed=75)
+    ck[f"blocks.1.att.{name}"].view(-1)[70] = float("nan")
+    m = _x070()(ck, "cuda fp16")
+    toks = synth.random_tokens(97, 300, seed=3)
+    for n in (64, 97):
+        out, st = m.forward(toks[:n], None)
+        assert torch.isnan(out).all() and torch.isfinite(st[1]).all(), n
+        bad = torch.isnan(st[4].reshape(2, 64, 64))
+        assert not bad[0].any() and bad[1].any(), n
+
+
 def test_v7_short_call_lengths():
     """Calls of 2, 3, 9 and 16 tokens: every product of such a call goes through the 2..16-row streaming kernel
     (fp16 weights, LoRA products of odd ranks included)."""
