@@ -527,6 +527,7 @@ __global__ __launch_bounds__(256, 2) void wkv7_apply_kernel(int H, int C, float 
         st = __builtin_amdgcn_mfma_f32_16x16x4f32(x.k[3], v[3], st, 0, 0, 0);
         __builtin_amdgcn_s_waitcnt(0xC07F);   // LDS only: __syncthreads() would also wait for the loads in flight
         __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");        // no read of the exchange ahead of the barrier
         const f32x4 u0 = redu[buf][0][lane], u1 = redu[buf][1][lane], u2 = redu[buf][2][lane], u3 = redu[buf][3][lane];
         float part[4];
 #pragma unroll

@@ -595,6 +595,7 @@ __global__ __launch_bounds__(256, 2) void wkv56_apply_kernel(Wkv56Args a, int H,
     auto exchange = [&](int buf) {
         __builtin_amdgcn_s_waitcnt(0xC07F);   // LDS only: __syncthreads() would also wait for the loads in flight
         __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");        // no read of the exchange ahead of the barrier
 #pragma unroll
         for (int u = 0; u < GC; ++u)
 #pragma unroll
