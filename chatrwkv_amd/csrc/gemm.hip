@@ -54,23 +54,45 @@ DEV float epi_affine(float v, float rxm, float mxm, float s0, float s2) {
     asm("" : "+v"(r));
     return r;
 }
-// v: the contraction after epi_affine; res / gate: the residual and gate inputs where ep.act uses them
-DEV float epi_act(float v, float res, float gate, const GemmEpi &ep) {
-    float o = round_h(v);
+// Activation, residual and output scale of K outputs.  v: the contraction after epi_affine; res / gate: the residual and
+// gate inputs where ep.act uses them.  The branch on the activation (the same for a whole launch) stands outside the loops
+// over the elements: inside them every element stepped over the code of the other activations, and a launch fetched its
+// epilogue from 12 KB of instructions.
+template <int K, class V>
+DEV void epi_act(float (&v)[K], V res, V gate, const GemmEpi &ep) {
+#pragma unroll
+    for (int e = 0; e < K; ++e) v[e] = round_h(v[e]);
     switch (ep.act) {
-        case ACT_SIGMOID: o = sigmoidf_(o); break;
-        case ACT_RELU_SQ: o = fmaxf(o, 0.f); o = o * o; break;
-        case ACT_SILU: o = o * sigmoidf_(o); break;
-        case ACT_TANH: o = tanhf(o); break;
-        case ACT_RESIDUAL: o = res + o; break;
+        case ACT_SIGMOID:
+#pragma unroll
+            for (int e = 0; e < K; ++e) v[e] = sigmoidf_(v[e]);
+            break;
+        case ACT_RELU_SQ:
+#pragma unroll
+            for (int e = 0; e < K; ++e) { v[e] = fmaxf(v[e], 0.f); v[e] = v[e] * v[e]; }
+            break;
+        case ACT_SILU:
+#pragma unroll
+            for (int e = 0; e < K; ++e) v[e] = v[e] * sigmoidf_(v[e]);
+            break;
+        case ACT_TANH:
+#pragma unroll
+            for (int e = 0; e < K; ++e) v[e] = tanhf(v[e]);
+            break;
         case ACT_GATED_RESIDUAL:
-            o = round_h(gate * o);
-            o = res + o;
+#pragma unroll
+            for (int e = 0; e < K; ++e) v[e] = round_h((float)gate[e] * v[e]);
+            [[fallthrough]];
+        case ACT_RESIDUAL:
+#pragma unroll
+            for (int e = 0; e < K; ++e) v[e] = (float)res[e] + v[e];
             break;
         default: break;
     }
-    if (ep.out_scale != 1.f) o = round_h(o) * ep.out_scale;
-    return o;
+    if (ep.out_scale != 1.f) {
+#pragma unroll
+        for (int e = 0; e < K; ++e) v[e] = round_h(v[e]) * ep.out_scale;
+    }
 }
 DEV void gemm_epilogue(float v, int t, int m, float rxm, float mxm, const GemmEpi &ep, void *Y, int64_t ldy) {
     if (ep.rx) v = epi_affine(v, rxm, mxm, ep.s0[t], ep.s2[t]);
@@ -78,14 +100,15 @@ DEV void gemm_epilogue(float v, int t, int m, float rxm, float mxm, const GemmEp
         ((float *)Y)[(size_t)t * ldy + m] = v;
         return;
     }
-    float res = 0.f, gate = 0.f;
-    if (ep.act == ACT_RESIDUAL || ep.act == ACT_GATED_RESIDUAL) res = h2f(ep.res[(size_t)t * ep.ldres + m]);
-    if (ep.act == ACT_GATED_RESIDUAL) gate = h2f(ep.gate[(size_t)t * ep.ldgate + m]);
-    const float o = epi_act(v, res, gate, ep);
+    h16 res[1] = {}, gate[1] = {};
+    if (ep.act == ACT_RESIDUAL || ep.act == ACT_GATED_RESIDUAL) res[0] = __builtin_bit_cast(h16, ep.res[(size_t)t * ep.ldres + m]);
+    if (ep.act == ACT_GATED_RESIDUAL) gate[0] = __builtin_bit_cast(h16, ep.gate[(size_t)t * ep.ldgate + m]);
+    float o[1] = {v};
+    epi_act<1, const h16 *>(o, res, gate, ep);
     if (ep.out_dtype == RWKV_DT_F32)
-        ((float *)Y)[(size_t)t * ldy + m] = round_h(o);
+        ((float *)Y)[(size_t)t * ldy + m] = round_h(o[0]);
     else
-        ((rwkv_half *)Y)[(size_t)t * ldy + m] = f2h(o);
+        ((rwkv_half *)Y)[(size_t)t * ldy + m] = f2h(o[0]);
 }
 
 // Epilogue of a few consecutive outputs of one row, operands laid out as dma_ok asks.
@@ -118,8 +141,10 @@ DEV void finish_row4(f32x4 v, int t, int col, int M, const GemmEpi &ep, void *Y,
         h16x4 res4 = {}, gate4 = {};
         if (ep.act == ACT_RESIDUAL || ep.act == ACT_GATED_RESIDUAL) res4 = *(const h16x4 *)(ep.res + (size_t)t * ep.ldres + col);
         if (ep.act == ACT_GATED_RESIDUAL) gate4 = *(const h16x4 *)(ep.gate + (size_t)t * ep.ldgate + col);
+        float o[4] = {v[0], v[1], v[2], v[3]};
+        epi_act(o, res4, gate4, ep);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = round_h(epi_act(v[e], (float)res4[e], (float)gate4[e], ep));
+        for (int e = 0; e < 4; ++e) v[e] = round_h(o[e]);
     }
     if (f32 && n >= 4) {
         *(f32x4_a4 *)((float *)Y + at) = f32x4_a4{v[0], v[1], v[2], v[3]};
@@ -146,29 +171,36 @@ DEV Emit8 emit8(const GemmEpi &ep, int col, bool ok) {
 DEV bool by_four(int M, int64_t ldy, const void *Y, const GemmEpi &ep) {
     return ep.raw_f32 || ep.out_dtype == RWKV_DT_F32 || !wide_rows(M, ldy, Y);
 }
+// What eight outputs of row t read besides the contraction: the residual and gate, and (uint8 weights) the row's sums.
+// Requested for all rows of a thread before the first one is finished: with the loads inside the loop over the rows every
+// row waited for its own, 4 to 16 times 0.5 - 1 us at the end of a launch.
+struct EpiIn { h16x8 res, gate; float s0, s2; };
+DEV EpiIn epi_in(const GemmEpi &ep, int t, int col, bool ok, bool sums) {
+    EpiIn in = {};
+    if (!ok) return in;
+    if (ep.act == ACT_RESIDUAL || ep.act == ACT_GATED_RESIDUAL) in.res = *(const h16x8 *)(ep.res + (size_t)t * ep.ldres + col);
+    if (ep.act == ACT_GATED_RESIDUAL) in.gate = *(const h16x8 *)(ep.gate + (size_t)t * ep.ldgate + col);
+    if (sums) { in.s0 = ep.s0[t]; in.s2 = ep.s2[t]; }
+    return in;
+}
 // activation / residual and 16-byte store of fp16 outputs; a0 / a2: these outputs' share of the emitted row sums (EMIT:
 // products that may emit them)
 template <bool EMIT>
-DEV void finish_row8(const float (&v)[8], int t, int col, const GemmEpi &ep, void *Y, int64_t ldy, const Emit8 &em, float &a0, float &a2) {
-    h16x8 res8 = {}, gate8 = {};
-    if (ep.act == ACT_RESIDUAL || ep.act == ACT_GATED_RESIDUAL) res8 = *(const h16x8 *)(ep.res + (size_t)t * ep.ldres + col);
-    if (ep.act == ACT_GATED_RESIDUAL) gate8 = *(const h16x8 *)(ep.gate + (size_t)t * ep.ldgate + col);
-    float o[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) o[e] = epi_act(v[e], (float)res8[e], (float)gate8[e], ep);
+DEV void finish_row8(float (&v)[8], const EpiIn &in, int t, int col, const GemmEpi &ep, void *Y, int64_t ldy, const Emit8 &em, float &a0, float &a2) {
+    epi_act(v, in.res, in.gate, ep);
     h16x8 y8;
     if (EMIT && ep.emit_ry) {
         // what the scaling pass of the next product would make of the fp16 output: fp16(y * ry), sum y, sum y * my
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
-            const float yf = (float)(h16)o[e];
+            const float yf = (float)(h16)v[e];
             y8[e] = (h16)(yf * (float)em.ry[e]);
             a0 += yf;
             a2 += yf * (float)em.my[e];
         }
     } else {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) y8[e] = (h16)o[e];
+        for (int e = 0; e < 8; ++e) y8[e] = (h16)v[e];
     }
     *(h16x8 *)((rwkv_half *)Y + (size_t)t * ldy + col) = y8;
 }
@@ -195,53 +227,63 @@ __global__ __launch_bounds__(256) void splitk_epilogue_kernel(int T, int M, int 
 // eight consecutive outputs per thread, all slab loads of a thread in flight together, 16-byte loads of the
 // residual / gate rows and 16-byte stores.  Same slab order and the same arithmetic per element as above.
 template <int KS>
-DEV void splitk_rows8(int T, int M, int ks_rt, const float *__restrict__ part, void *Y, int64_t ldy, const GemmEpi &ep,
+DEV void slab_sum8(int ks, size_t n, const float *__restrict__ p, f32x4 &lo, f32x4 &hi) {
+    lo = *(const f32x4 *)p;
+    hi = *(const f32x4 *)(p + 4);
+    if constexpr (KS > 0) {
+        f32x4 pl[KS], ph[KS];
+#pragma unroll
+        for (int k = 1; k < KS; ++k) {
+            pl[k] = *(const f32x4 *)(p + k * n);
+            ph[k] = *(const f32x4 *)(p + k * n + 4);
+        }
+#pragma unroll
+        for (int k = 1; k < KS; ++k) { lo += pl[k]; hi += ph[k]; }
+    } else {
+        for (int k = 1; k < ks; ++k) {
+            lo += *(const f32x4 *)(p + k * n);
+            hi += *(const f32x4 *)(p + k * n + 4);
+        }
+    }
+}
+DEV void splitk_rows8(int T, int M, int ks, const float *__restrict__ part, void *Y, int64_t ldy, const GemmEpi &ep,
                       int64_t first, int64_t stride) {
     const int64_t n8 = (int64_t)T * M / 8, n = (int64_t)T * M;
-    const int m8 = M / 8, ks = KS ? KS : ks_rt;
+    const int m8 = M / 8;
+    const bool four = by_four(M, ldy, Y, ep);
     for (int64_t i = first; i < n8; i += stride) {
         const int t = (int)(i / m8), col = (int)(i - (int64_t)t * m8) * 8;
-        f32x4 lo = *(const f32x4 *)(part + 8 * i), hi = *(const f32x4 *)(part + 8 * i + 4);
-        if constexpr (KS > 0) {
-            f32x4 pl[KS], ph[KS];
-#pragma unroll
-            for (int k = 1; k < KS; ++k) {
-                pl[k] = *(const f32x4 *)(part + (size_t)k * n + 8 * i);
-                ph[k] = *(const f32x4 *)(part + (size_t)k * n + 8 * i + 4);
-            }
-#pragma unroll
-            for (int k = 1; k < KS; ++k) { lo += pl[k]; hi += ph[k]; }
-        } else {
-            for (int k = 1; k < ks; ++k) {
-                lo += *(const f32x4 *)(part + (size_t)k * n + 8 * i);
-                hi += *(const f32x4 *)(part + (size_t)k * n + 8 * i + 4);
-            }
+        EpiIn in = {};
+        h16x8 rx8 = {}, mx8 = {};
+        if (!four) in = epi_in(ep, t, col, true, false);
+        if (ep.rx) {   // M % 8 == 0
+            rx8 = *(const h16x8 *)(ep.rx + col);
+            mx8 = *(const h16x8 *)(ep.mx + col);
+            in.s0 = ep.s0[t];
+            in.s2 = ep.s2[t];
+        }
+        f32x4 lo, hi;
+        switch (ks) {
+            case 2: slab_sum8<2>(ks, n, part + 8 * i, lo, hi); break;
+            case 4: slab_sum8<4>(ks, n, part + 8 * i, lo, hi); break;
+            case 8: slab_sum8<8>(ks, n, part + 8 * i, lo, hi); break;
+            default: slab_sum8<0>(ks, n, part + 8 * i, lo, hi); break;
         }
         float v[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-        if (ep.rx) affine8(v, *(const h16x8 *)(ep.rx + col), *(const h16x8 *)(ep.mx + col), ep.s0[t], ep.s2[t]);   // M % 8 == 0
-        if (by_four(M, ldy, Y, ep)) {
-            finish_row4(f32x4{v[0], v[1], v[2], v[3]}, t, col, M, ep, Y, ldy);
-            finish_row4(f32x4{v[4], v[5], v[6], v[7]}, t, col + 4, M, ep, Y, ldy);
+        if (ep.rx) affine8(v, rx8, mx8, in.s0, in.s2);
+        if (four) {
+#pragma unroll 1
+            for (int g = 0; g < 2; ++g) finish_row4(g ? f32x4{v[4], v[5], v[6], v[7]} : f32x4{v[0], v[1], v[2], v[3]}, t, col + 4 * g, M, ep, Y, ldy);
             continue;
         }
         float a0 = 0.f, a2 = 0.f;   // a product that emits row sums does not split K
-        finish_row8<false>(v, t, col, ep, Y, ldy, Emit8{}, a0, a2);
-    }
-}
-
-DEV void splitk_rows8_any(int T, int M, int KS, const float *__restrict__ part, void *Y, int64_t ldy, const GemmEpi &ep,
-                          int64_t first, int64_t stride) {
-    switch (KS) {
-        case 2: splitk_rows8<2>(T, M, KS, part, Y, ldy, ep, first, stride); break;
-        case 4: splitk_rows8<4>(T, M, KS, part, Y, ldy, ep, first, stride); break;
-        case 8: splitk_rows8<8>(T, M, KS, part, Y, ldy, ep, first, stride); break;
-        default: splitk_rows8<0>(T, M, KS, part, Y, ldy, ep, first, stride); break;
+        finish_row8<false>(v, in, t, col, ep, Y, ldy, Emit8{}, a0, a2);
     }
 }
 
 __global__ __launch_bounds__(256) void splitk_epilogue8_kernel(int T, int M, int KS, const float *__restrict__ part, void *Y,
                                                                int64_t ldy, GemmEpi ep) {
-    splitk_rows8_any(T, M, KS, part, Y, ldy, ep, (int64_t)blockIdx.x * 256 + threadIdx.x, (int64_t)gridDim.x * 256);
+    splitk_rows8(T, M, KS, part, Y, ldy, ep, (int64_t)blockIdx.x * 256 + threadIdx.x, (int64_t)gridDim.x * 256);
 }
 
 template <bool W_U8, int BT, int BM, int WT, int WM, int PF, bool SPLIT>
@@ -790,15 +832,26 @@ DEV void gemm_dma_body(int bid, int T, int N, int M, const h16 *__restrict__ A, 
                             stg[(wr * WROWS - h * 128 + a * 32 + 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3)) * SW + wc * 32 * NI + b * 32 + (lane & 31)] =
                                 acc[a][b][e];
             }
-            __syncthreads();
+            constexpr int ITS = (TM < 128 ? TM : 128) / RPI, AHEAD_ROWS = TM == 256 ? 2 : 4;   // rows of a thread; rows requested together
+            EpiIn in[AHEAD_ROWS];
 #pragma unroll 1
-            for (int it = 0; it < (TM < 128 ? TM : 128) / RPI; ++it) {
+            for (int it = 0; it < ITS; ++it) {
                 const int row = it * RPI + tid / CPR, t = t0 + h * 128 + row;
                 const bool valid = t < T && col_ok;
+                if (it % AHEAD_ROWS == 0) {
+                    if (!four) {
+#pragma unroll
+                        for (int i = 0; i < AHEAD_ROWS; ++i) in[i] = epi_in(ep, t + i * RPI, col, t + i * RPI < T && col_ok, W_U8 && !lds_sums);
+                    }
+                    if (it == 0) __syncthreads();   // the accumulators are in LDS
+                }
+                const EpiIn cur = in[0];
+#pragma unroll
+                for (int i = 0; i + 1 < AHEAD_ROWS; ++i) in[i] = in[i + 1];   // a loop that is not unrolled has no other index
                 float a0 = 0.f, a2 = 0.f;
                 if (four) {
                     if (t >= T) continue;
-#pragma unroll
+#pragma unroll 1
                     for (int g = 0; g < 2; ++g) {
                         const int c = g * (TN / 2) + cq * 4;
                         if (m0 + c >= M) continue;
@@ -816,9 +869,9 @@ DEV void gemm_dma_body(int bid, int T, int N, int M, const h16 *__restrict__ A, 
                     float v[8] = {v0[0], v0[1], v0[2], v0[3], v1[0], v1[1], v1[2], v1[3]};
                     if constexpr (W_U8) {
                         const int tr = h * 128 + row;
-                        affine8(v, rx8, mx8, lds_sums ? lsum[tr] : ep.s0[t], lds_sums ? lsum[TM + tr] : ep.s2[t]);
+                        affine8(v, rx8, mx8, lds_sums ? lsum[tr] : cur.s0, lds_sums ? lsum[TM + tr] : cur.s2);
                     }
-                    finish_row8<true>(v, t, col, ep, Y, ldy, em, a0, a2);
+                    finish_row8<true>(v, cur, t, col, ep, Y, ldy, em, a0, a2);
                 }
                 if (emit) {   // the CPR threads of a row are neighbours in one wave; every lane takes part
                     a0 = row16_sum(a0);
@@ -1111,16 +1164,28 @@ DEV void gemm_kw_body(int bid, int T, int N, int M, const h16 *__restrict__ A, i
             for (int g = 0; g < 4; ++g)
                 *(f32x4 *)(mypart + (a * 32 + row) * SW + b * 32 + 8 * g + 4 * h) =
                     f32x4{acc[b][a][4 * g], acc[b][a][4 * g + 1], acc[b][a][4 * g + 2], acc[b][a][4 * g + 3]};
-    __syncthreads();
     const bool emit = ep.emit_ry != nullptr, four = by_four(M, ldy, Y, ep);
+    const int cq = tid & 7, col = m0 + cq * 8;   // this thread's columns; its rows: tid / 8 and 32 further
+    const bool col_ok = col < M;
+    EpiIn in0 = {}, in1 = {};
+    h16x8 rx8 = {}, mx8 = {};
+    Emit8 em = {};
+    if (!four) {
+        const int t = t0 + (tid >> 3);
+        in0 = epi_in(ep, t, col, t < T && col_ok, W_U8 && !lds_sums);
+        in1 = epi_in(ep, t + 32, col, t + 32 < T && col_ok, W_U8 && !lds_sums);
+        if (W_U8 && col_ok) { rx8 = load_n<h16x8, 8>(ep.rx + col, M - col); mx8 = load_n<h16x8, 8>(ep.mx + col, M - col); }
+        em = emit8(ep, col, col_ok);
+    }
+    __syncthreads();
 #pragma unroll 1
-    for (int i = tid; i < 64 * 8; i += 256) {
-        const int r = i >> 3, cq = i & 7, t = t0 + r, col = m0 + cq * 8;
-        const bool valid = t < T && col < M;
+    for (int i = 0; i < 2; ++i) {
+        const int r = (tid >> 3) + 32 * i, t = t0 + r;
+        const bool valid = t < T && col_ok;
         float a0 = 0.f, a2 = 0.f;
         if (four) {
             if (t >= T) continue;
-#pragma unroll
+#pragma unroll 1
             for (int g = 0; g < 2; ++g) {
                 const int c = g * 32 + cq * 4;
                 if (m0 + c >= M) continue;
@@ -1142,11 +1207,9 @@ DEV void gemm_kw_body(int bid, int T, int N, int M, const h16 *__restrict__ A, i
                 hi += *(const f32x4 *)(p + k * (Cfg::REGION / 4) + 4);
             }
             float v[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-            if constexpr (W_U8) {
-                const float s0t = lds_sums ? lsum[r] : ep.s0[t], s2t = lds_sums ? lsum[64 + r] : ep.s2[t];
-                affine8(v, load_n<h16x8, 8>(ep.rx + col, M - col), load_n<h16x8, 8>(ep.mx + col, M - col), s0t, s2t);
-            }
-            finish_row8<true>(v, t, col, ep, Y, ldy, emit8(ep, col, true), a0, a2);
+            const EpiIn in = i ? in1 : in0;
+            if constexpr (W_U8) affine8(v, rx8, mx8, lds_sums ? lsum[r] : in.s0, lds_sums ? lsum[64 + r] : in.s2);
+            finish_row8<true>(v, in, t, col, ep, Y, ldy, em, a0, a2);
         }
         if (emit) {   // the eight threads of a row are neighbours in one wave; every lane takes part
 #pragma unroll
@@ -1184,7 +1247,7 @@ int launch_kw(GemmGroup &g, int n, int64_t T, int64_t N, hipStream_t st) {
 // second pass of a split group launch: member blockIdx.y, as splitk_epilogue8_kernel
 __global__ __launch_bounds__(256) void splitk_group_epilogue8_kernel(int T, int KS, GemmGroup g) {
     const int gi = blockIdx.y;
-    splitk_rows8_any(T, g.M[gi], KS, g.part[gi], g.Y[gi], g.M[gi], g.ep[gi], (int64_t)blockIdx.x * 256 + threadIdx.x,
+    splitk_rows8(T, g.M[gi], KS, g.part[gi], g.Y[gi], g.M[gi], g.ep[gi], (int64_t)blockIdx.x * 256 + threadIdx.x,
                      (int64_t)gridDim.x * 256);
 }
 
@@ -1457,9 +1520,11 @@ __global__ __launch_bounds__(512) void narrow_kernel(int T, int N, int M, const 
         for (int w = 1; w < 8; ++w) v += red[w][lane];
         const int t = t0 + sub, m = m0 + 4 * q;
         if (t < T && m < M) {   // M % 4 == 0
+            float r[4] = {v[0], v[1], v[2], v[3]};
+            epi_act(r, h16x4{}, h16x4{}, ep);
             h16x4 o;
 #pragma unroll
-            for (int e = 0; e < 4; ++e) o[e] = (h16)epi_act(v[e], 0.f, 0.f, ep);
+            for (int e = 0; e < 4; ++e) o[e] = (h16)r[e];
             *(h16x4 *)((h16 *)Y + (size_t)t * ldy + m) = o;
         }
     }
