@@ -18,6 +18,7 @@
 // Workgroup ids are remapped so that the workgroups which share a weight tile (same m0,
 // different t0) run on the same XCD and the tile is fetched into that XCD's L2 once.
 #include <algorithm>
+#include <type_traits>
 #include "kernels.h"
 #include "../../include/rwkv_hip_bench.h"
 #include <cstdlib>
@@ -963,71 +964,93 @@ int launch_dma_group(GemmGroup &g, int n, int64_t T, int64_t N, int ks, hipStrea
     return RWKV_OK;
 }
 
-// ---- K over the waves of a workgroup: products whose large tiles would leave the chip idle --------------------
+// ---- K over wave groups: products whose large tiles would leave the chip idle ---------------------------------
 // [T, 768..4096] x [.., 768..4096] products of a few hundred rows have 12 to 100 tiles of 128 x 128: most CUs idle, or a
-// K split whose fp32 slabs need a second launch.  Here the tile is 64 x 64 and K is split over the four waves of the
-// workgroup: wave w computes the WHOLE tile over the k-tiles w, w + 4, ... and the four partial tiles are added in wave
-// order through LDS (deterministic).  A 64 x 64 wave tile reads as few fragment bytes per MFMA as the tile allows
-// (32 x 32 wave tiles of the same workgroup tile: twice as many), and as a wave only ever reads what it has
-// loaded itself there is no barrier in the loop: each wave has its own stages (three of 12 KB for uint8 weights, two of
-// 16 KB for fp16), waits for its own direct-to-LDS loads and refills a stage as soon as its last fragment is back.
-// Fragments: half a k-tile at a time, the next half's reads in flight while one multiplies; a lane of half h takes
-// k 32 h + 8 s .. + 7 in step s for both operands, so uint8 fragments are 16-byte reads (two steps' worth each).
-// LDS swizzles as in gemm_dma_body.  Bound by how fast operand tiles reach the CU: 0.235 us per k-tile of 12-16 KB with
-// weights from HBM (0.15 from L2), whatever the number of workgroups, + 6 us of launch, first tiles and epilogue.
-// Measured, weights from HBM, us: fp16 [513 x 768] x [768 x 768] 11.9 -> 8.9, [333 x 2048] x [2048 x 2048] 19.3 (K split in
-// four, with its second pass) -> 13.5; uint8 with the scaling pass [256 x 768] x [768 x 768] 14.7 -> 10.9, [384 x 2048] x
-// [2048 x 2048] 22.0 -> 16.4, [256 x 4096] x [4096 x 4096] 26.1 -> 24.6; slower from the second round on ([513 x 4096] x
-// [4096 x 4096] 39.9 -> 52.4: one workgroup per CU, every round pays its first tiles) and for long K on few rows.
-// The same split with operands loaded straight into MFMA registers (no LDS; 16 rows x 64 bytes per load instruction)
-// took 2.5 times as long: the lanes of a quad then lie in four rows and nothing coalesces.
-template <bool W_U8> struct KwCfg {
-    static constexpr int A = 64 * BK * 2, W = W_U8 ? 64 * BK : 64 * BK * 2, STAGE = A + W;
-    static constexpr int NST = W_U8 ? 3 : 2, AL = A / 1024, WL = W / 1024, LOADS = AL + WL;
-    static constexpr int SW = 68;   // row stride (floats) of the partial tiles
-    static constexpr size_t REGION = (size_t)NST * STAGE, LDS = 4 * REGION + 2 * 64 * 4;
-    static_assert((size_t)64 * SW * 4 <= REGION, "partial tile");
+// K split whose fp32 slabs need a second launch; and calls of up to 128 rows are bound by how fast the weights arrive.
+// Here the tile is 64 x 64 or 64 x 128 and a workgroup's eight waves are KG = 8 or 4 groups that share K: every wave
+// computes a 64 x 64 block (the fewest fragment bytes per MFMA that eight waves allow) over its part of each stage, and the
+// partial blocks are added in group order through LDS (deterministic).  A stage holds 128 or 256 k's, so that a uint8 weight
+// row is one or two whole 128-byte lines: with 64 k's per stage half a line per request, at the same cost per request.
+// Lane half h of a group takes 8 consecutive k's per MFMA step from KW / 2 h on, for both operands, so uint8 fragments are
+// 16-byte reads of two steps' worth; a stage's first fragments are read while the stage before multiplies.
+// What bounds it, loops taken apart: from about 190 workgroups on the weights (uint8 [45 x 4096] x [4096 x 12288] 4.1 TB/s in
+// the loop, fp16 4.8), otherwise the requests that a CU has in flight (0.14 - 0.2 us per 64 k's of a 64 x 64 tile); + 5 - 7 us
+// of launch, first stages and epilogue.  Rows past T are not worth skipping (buffer loads with bounds: 2 - 4 % slower).
+// Measured, weights from HBM, us, against the same with K over four waves that each had stages of their own, and the
+// 128 x 128 tiles: uint8 [256 x 4096] x [4096 x 4096] 17.3 -> 16.6, [45 x 4096] x [4096 x 12288] 20.3 (two K splits of 64 x 128
+// tiles 19.4) -> 17.7, [128 x 4096] x [4096 x 12288] 31.8 (two splits 24.4) -> 25.3, [100 x 16384] x [16384 x 2048] 32.3 -> 20.6;
+// fp16 [513 x 768] x [768 x 768] 7.8 -> 7.2, [333 x 2048] x [2048 x 2048] 10.4 -> 10.1, [128 x 4096] x [4096 x 768] 12.8 -> 10.5.
+// 128 x 128 (KG = 2) and 128 x 256 (1) tiles of this form: 42.0 and 55.8 against 38.8 us on [1024 x 4096] x [4096 x 4096],
+// not built.
+template <bool W_U8, int TM, int TN> struct KgCfg {
+    static constexpr int RA = TM / 64, RB = TN / 64, KG = 8 / (RA * RB);   // 64 x 64 blocks of the tile; groups that share K
+    static constexpr int BKS = W_U8 && KG == 8 ? 256 : 128;                // k's of a stage
+    static constexpr int KW = BKS / KG, US = KW / 16;                                  // k's and MFMA steps of a wave and stage
+    static constexpr int ABYTES = BKS * 2, WBYTES = W_U8 ? BKS : BKS * 2;              // bytes of a row
+    static constexpr int A = TM * ABYTES, W = TN * WBYTES, STAGE = A + W;
+    static constexpr int AL = A / 8192, WL = W / 8192, LOADS = AL + WL;                // 1 KB loads per wave and stage
+    static constexpr int SW = 68, REGION = 64 * SW * 4;                                // partial tile of a wave: row stride (floats), bytes
+    static constexpr int NST = (160 * 1024 - 2 * TM * 4) / STAGE < 4 ? (160 * 1024 - 2 * TM * 4) / STAGE : 4;
+    static constexpr size_t BODY = NST * STAGE > 8 * REGION ? NST * STAGE : 8 * REGION, LDS = BODY + (W_U8 ? 2 * TM * 4 : 0);
+    static_assert((KG == 8 || KG == 4) && (US == 1 || US == 2) && NST >= 2 && LDS <= 160 * 1024 && (NST - 1) * LOADS < 64, "tile");
 };
-template <bool W_U8>
-DEV void gemm_kw_body(int bid, int T, int N, int M, const h16 *__restrict__ A, int64_t lda, const void *__restrict__ Wv, int64_t ldw,
-                      void *__restrict__ Y, int64_t ldy, const GemmEpi &ep) {
-    using Cfg = KwCfg<W_U8>;
-    constexpr int NST = Cfg::NST, STAGE = Cfg::STAGE, AL = Cfg::AL, WL = Cfg::WL, SW = Cfg::SW;
+// slot of a 16-byte chunk in a row of RBYTES: conflict-free for 16 rows x one chunk (64 banks of 4 bytes)
+template <int RBYTES> DEV int kg_key(int row) {
+    constexpr int RPB = RBYTES < 256 ? 256 / RBYTES : 1, CH = RBYTES / 16 < 16 ? RBYTES / 16 : 16;
+    return (row / RPB) & (CH - 1);
+}
+template <bool W_U8, bool SPLIT, int TM, int TN>
+DEV void gemm_kg_body(int bid, int T, int N, int M, const h16 *__restrict__ A, int64_t lda, const void *__restrict__ Wv, int64_t ldw,
+                      void *__restrict__ Y, int64_t ldy, const GemmEpi &ep, int nk_split, float *__restrict__ part, int split) {
+    using Cfg = KgCfg<W_U8, TM, TN>;
+    constexpr int NST = Cfg::NST, STAGE = Cfg::STAGE, AL = Cfg::AL, WL = Cfg::WL, BKS = Cfg::BKS, KW = Cfg::KW, US = Cfg::US;
+    constexpr int AB = Cfg::ABYTES, WB = Cfg::WBYTES, RA = Cfg::RA, RB = Cfg::RB, SW = Cfg::SW;
     extern __shared__ __align__(1024) unsigned char smem[];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int tiles_t = (T + 63) / 64;
-    const int t0 = (bid % tiles_t) * 64, m0 = (bid / tiles_t) * 64;
-    const int nk = N / BK, mine = (nk - wave + 3) / 4;   // k-tiles of this wave
+    const int blk = wave % (RA * RB), grp = wave / (RA * RB), wr = blk / RB, wc = blk % RB;
+    const int tiles_t = (T + TM - 1) / TM;
+    const int t0 = (bid % tiles_t) * TM, m0 = (bid / tiles_t) * TN;
+    const int kbase = SPLIT ? split * nk_split * BK : 0, K = SPLIT ? nk_split * BK : N;   // this workgroup's k's (a multiple of 64)
+    const int nk = (K + BKS - 1) / BKS;
 
-    unsigned char *base = smem + wave * Cfg::REGION;
-    const h16 *ga[AL];
+    // load sources; rows past the end re-read the last row (never stored).  Load i of a wave fills 1 KB: the rows
+    // (wave AL + i) 1024 / AB and up; the lane that fills slot p of row r fetches chunk p ^ key(r).
+    constexpr int ALR = AB / 16, WLR = WB / 16;   // lanes per row
+    auto a_row = [&](int i) { return (wave * AL + i) * (64 / ALR) + lane / ALR; };
+    auto w_row = [&](int i) { return (wave * WL + i) * (64 / WLR) + lane / WLR; };
+    auto a_k = [&](int i) { return ((lane % ALR) ^ kg_key<AB>(a_row(i))) * 8; };
+    auto w_k = [&](int i) { return ((lane % WLR) ^ kg_key<WB>(w_row(i))) * (W_U8 ? 16 : 8); };
+    const unsigned char *ga[AL], *gw[WL];
 #pragma unroll
-    for (int i = 0; i < AL; ++i) {
-        const int r = i * 8 + (lane >> 3), c = (lane & 7) ^ ((r >> 1) & 7);
-        ga[i] = A + (size_t)min(t0 + r, T - 1) * lda + c * 8;
-    }
-    const unsigned char *gw[WL];
+    for (int i = 0; i < AL; ++i) ga[i] = (const unsigned char *)(A + (size_t)min(t0 + a_row(i), T - 1) * lda + kbase + a_k(i));
 #pragma unroll
-    for (int i = 0; i < WL; ++i) {
-        if (W_U8) {
-            const int r = i * 16 + (lane >> 2), c = (lane & 3) ^ ((r >> 2) & 3);
-            gw[i] = (const unsigned char *)Wv + (size_t)min(m0 + r, M - 1) * ldw + c * 16;
-        } else {
-            const int r = i * 8 + (lane >> 3), c = (lane & 7) ^ ((r >> 1) & 7);
-            gw[i] = (const unsigned char *)((const h16 *)Wv + (size_t)min(m0 + r, M - 1) * ldw + c * 8);
-        }
-    }
+    for (int i = 0; i < WL; ++i)
+        gw[i] = (const unsigned char *)Wv + ((size_t)min(m0 + w_row(i), M - 1) * ldw + kbase + w_k(i)) * (W_U8 ? 1 : 2);
     typedef __attribute__((address_space(1))) const void *gptr;
     typedef __attribute__((address_space(3))) void *lptr;
-    // my i-th k-tile into stage byte offset so; past the end the last k-tile again (never multiplied)
-    auto issue = [&](int i, int so) {
-        const int kt = min(wave + 4 * i, nk - 1);
+    auto issue = [&](int kt, int so) {   // a whole stage
+        unsigned char *base = smem + so;
 #pragma unroll
-        for (int j = 0; j < AL; ++j)
-            __builtin_amdgcn_global_load_lds((gptr)(ga[j] + kt * BK), (lptr)(base + so + j * 1024), 16, 0, 0);
+        for (int i = 0; i < AL; ++i) __builtin_amdgcn_global_load_lds((gptr)(ga[i] + kt * AB), (lptr)(base + (wave * AL + i) * 1024), 16, 0, 0);
 #pragma unroll
-        for (int j = 0; j < WL; ++j)
-            __builtin_amdgcn_global_load_lds((gptr)(gw[j] + kt * BK * (W_U8 ? 1 : 2)), (lptr)(base + so + Cfg::A + j * 1024), 16, 0, 0);
+        for (int i = 0; i < WL; ++i) __builtin_amdgcn_global_load_lds((gptr)(gw[i] + kt * WB), (lptr)(base + Cfg::A + (wave * WL + i) * 1024), 16, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto issue_any = [&](int kt, int so) {
+        if (kt * BKS + BKS <= K) { issue(kt, so); return; }
+        // the last stage of a K that is no multiple of BKS: chunks past the end fetch k 0 .. 63 (never multiplied)
+        unsigned char *base = smem + so;
+#pragma unroll
+        for (int i = 0; i < AL; ++i) {
+            const int k = a_k(i), d = kt * BKS + k < K ? kt * BKS : (k & 63) - k;
+            __builtin_amdgcn_global_load_lds((gptr)(ga[i] + d * 2), (lptr)(base + (wave * AL + i) * 1024), 16, 0, 0);
+        }
+#pragma unroll
+        for (int i = 0; i < WL; ++i) {
+            const int k = w_k(i), d = kt * BKS + k < K ? kt * BKS : (k & 63) - k;
+            __builtin_amdgcn_global_load_lds((gptr)(gw[i] + d * (W_U8 ? 1 : 2)), (lptr)(base + Cfg::A + (wave * WL + i) * 1024), 16, 0, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
     };
     f32x16 acc[2][2];   // [weight block][token block]
 #pragma unroll
@@ -1036,59 +1059,51 @@ DEV void gemm_kw_body(int bid, int T, int N, int M, const h16 *__restrict__ A, i
         for (int a = 0; a < 2; ++a)
 #pragma unroll
             for (int e = 0; e < 16; ++e) acc[b][a][e] = 0.f;
-    // fragments: lane (row, h) takes k 32 h + 8 s .. + 7 in step s, for both operands
-    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)base;
-    const int row = lane & 31, h = lane >> 5;
-    uint32_t vA[4], vB[W_U8 ? 2 : 4];
+
+    // fragments: lane (row, h) of group g takes k g KW + h KW / 2 + 8 s .. + 7 of the stage in step s, for both operands
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)smem;
+    const int row = lane & 31, h = lane >> 5, k0 = grp * KW + h * (KW / 2);
+    constexpr int WN = W_U8 ? 1 : US;   // weight reads per stage and block
+    uint32_t vA[US], vW[WN];
 #pragma unroll
-    for (int s = 0; s < 4; ++s) vA[s] = lds0 + row * 128 + (((4 * h + s) ^ ((row >> 1) & 7)) << 4);
+    for (int j = 0; j < US; ++j) vA[j] = lds0 + (wr * 64 + row) * AB + (((k0 / 8 + j) ^ kg_key<AB>(row)) << 4);
 #pragma unroll
-    for (int s = 0; s < (W_U8 ? 2 : 4); ++s)
-        vB[s] = W_U8 ? lds0 + Cfg::A + row * 64 + (((2 * h + s) ^ ((row >> 2) & 3)) << 4)
-                     : lds0 + Cfg::A + row * 128 + (((4 * h + s) ^ ((row >> 1) & 7)) << 4);
-    constexpr int BN = W_U8 ? 1 : 2;
-    h16x8 fa[2][2][2];     // [set][step of the half][token block]
-    u32x4 fw[2][BN][2];    // [set][read][weight block]
-    auto ldhalf = [&](int set, int so, int p) {
+    for (int j = 0; j < WN; ++j) vW[j] = lds0 + Cfg::A + (wc * 64 + row) * WB + (((W_U8 ? k0 / 16 : k0 / 8 + j) ^ kg_key<WB>(row)) << 4);
+    h16x8 fa[2][US][2];    // [set][step][token block]
+    u32x4 fw[2][WN][2];    // [set][read][weight block]
+    auto ldstage = [&](int set, int so) {
 #pragma unroll
-        for (int j = 0; j < BN; ++j) {
-            const uint32_t pb = vB[W_U8 ? p : 2 * p + j] + so;
-            if constexpr (W_U8) {
-                asm volatile("ds_read_b128 %0, %1" : "=v"(fw[set][j][0]) : "v"(pb));
-                asm volatile("ds_read_b128 %0, %1 offset:2048" : "=v"(fw[set][j][1]) : "v"(pb));
-            } else {
-                asm volatile("ds_read_b128 %0, %1" : "=v"(fw[set][j][0]) : "v"(pb));
-                asm volatile("ds_read_b128 %0, %1 offset:4096" : "=v"(fw[set][j][1]) : "v"(pb));
-            }
+        for (int j = 0; j < WN; ++j) {
+            const uint32_t p = vW[j] + so;
+            asm volatile("ds_read_b128 %0, %1" : "=v"(fw[set][j][0]) : "v"(p));
+            asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(fw[set][j][1]) : "v"(p), "n"(32 * WB));
         }
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const uint32_t pa = vA[2 * p + j] + so;
-            asm volatile("ds_read_b128 %0, %1" : "=v"(fa[set][j][0]) : "v"(pa));
-            asm volatile("ds_read_b128 %0, %1 offset:4096" : "=v"(fa[set][j][1]) : "v"(pa));
+        for (int j = 0; j < US; ++j) {
+            const uint32_t p = vA[j] + so;
+            asm volatile("ds_read_b128 %0, %1" : "=v"(fa[set][j][0]) : "v"(p));
+            asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(fa[set][j][1]) : "v"(p), "n"(32 * AB));
         }
+        __builtin_amdgcn_sched_barrier(0);
     };
     const h16x2 off = {(h16)1023.5f, (h16)1023.5f};
-    auto mulhalf = [&](int set) {
+    auto mul = [&](int set, int j) {
+        h16x8 wf[2];
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            h16x8 wf[2];
-#pragma unroll
-            for (int b = 0; b < 2; ++b) {
-                if constexpr (W_U8) {
-                    const uint32_t b0 = j ? fw[set][0][b].z : fw[set][0][b].x, b1 = j ? fw[set][0][b].w : fw[set][0][b].y;
-                    const h16x2 q0 = u8pair_lo_1024(b0) - off, q1 = u8pair_hi_1024(b0) - off;
-                    const h16x2 q2 = u8pair_lo_1024(b1) - off, q3 = u8pair_hi_1024(b1) - off;
-                    wf[b] = h16x8{q0.x, q0.y, q1.x, q1.y, q2.x, q2.y, q3.x, q3.y};
-                } else {
-                    wf[b] = __builtin_bit_cast(h16x8, fw[set][j][b]);
-                }
+        for (int b = 0; b < 2; ++b) {
+            if constexpr (W_U8) {
+                const uint32_t b0 = j ? fw[set][0][b].z : fw[set][0][b].x, b1 = j ? fw[set][0][b].w : fw[set][0][b].y;
+                const h16x2 q0 = u8pair_lo_1024(b0) - off, q1 = u8pair_hi_1024(b0) - off;
+                const h16x2 q2 = u8pair_lo_1024(b1) - off, q3 = u8pair_hi_1024(b1) - off;
+                wf[b] = h16x8{q0.x, q0.y, q1.x, q1.y, q2.x, q2.y, q3.x, q3.y};
+            } else {
+                wf[b] = __builtin_bit_cast(h16x8, fw[set][j][b]);
             }
-#pragma unroll
-            for (int b = 0; b < 2; ++b)
-#pragma unroll
-                for (int a = 0; a < 2; ++a) acc[b][a] = __builtin_amdgcn_mfma_f32_32x32x16_f16(wf[b], fa[set][j][a], acc[b][a], 0, 0, 0);
         }
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+            for (int a = 0; a < 2; ++a) acc[b][a] = __builtin_amdgcn_mfma_f32_32x32x16_f16(wf[b], fa[set][j][a], acc[b][a], 0, 0, 0);
         __builtin_amdgcn_sched_barrier(0);
     };
     auto reads_done = [&]() {
@@ -1096,48 +1111,72 @@ DEV void gemm_kw_body(int bid, int T, int N, int M, const h16 *__restrict__ A, i
         __builtin_amdgcn_sched_barrier(0);
     };
 #pragma unroll
-    for (int i = 0; i < NST; ++i) issue(i, i * STAGE);
+    for (int s = 0; s < NST; ++s)
+        if (s < nk) issue_any(s, s * STAGE);
     bool lds_sums = false;
-    float *lsum = (float *)(smem + 4 * Cfg::REGION);
+    float *lsum = (float *)(smem + Cfg::BODY);
     if constexpr (W_U8) {
-        if (ep.parts > 1) {
-            lds_sums = true;
-            if (tid < 128) {
-                const int r = tid & 63, which = tid >> 6, t = min(t0 + r, T - 1);
+        if (ep.parts > 1 && (!SPLIT || (m0 == 0 && split == 0))) {
+            lds_sums = !SPLIT;
+            if (tid < 2 * TM) {
+                const int r = tid & (TM - 1), which = tid / TM, t = min(t0 + r, T - 1);
                 const float *p = (which ? ep.p2 : ep.p0) + (size_t)t * ep.parts;
                 float tot = 0.f;
                 for (int j = 0; j < ep.parts; j += 64) {
                     f32x4 v[16];
 #pragma unroll
-                    for (int u = 0; u < 16; ++u) v[u] = j + 4 * u < ep.parts ? *(const f32x4 *)(p + j + 4 * u) : f32x4{0.f, 0.f, 0.f, 0.f};
+                    for (int q = 0; q < 16; ++q) v[q] = j + 4 * q < ep.parts ? *(const f32x4 *)(p + j + 4 * q) : f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                    for (int u = 0; u < 16; ++u) tot = (((tot + v[u][0]) + v[u][1]) + v[u][2]) + v[u][3];
+                    for (int q = 0; q < 16; ++q) tot = (((tot + v[q][0]) + v[q][1]) + v[q][2]) + v[q][3];
                 }
-                lsum[tid] = tot;
+                if constexpr (SPLIT) {
+                    if (t0 + r < T) (which ? (float *)ep.s2 : (float *)ep.s0)[t] = tot;
+                } else {
+                    lsum[tid] = tot;
+                }
             }
         }
     }
     __builtin_amdgcn_sched_barrier(0);
-    __builtin_amdgcn_s_waitcnt(vm_lgkm0((NST - 1) * Cfg::LOADS));
+    if (nk >= NST) __builtin_amdgcn_s_waitcnt(vm_lgkm0((NST - 1) * Cfg::LOADS));   // my part of stage 0 has landed
+    else __builtin_amdgcn_s_waitcnt(vm_lgkm0(0));
+    __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
-    ldhalf(0, 0, 0);
-    reads_done();
     int so = 0;
-    for (int i = 0; i < mine; ++i) {
+    ldstage(0, 0);
+    reads_done();
+    // One stage.  Past its barrier stage kt + 1 has landed for every wave and nobody reads stage kt any more, so stage kt + NST
+    // goes where it was.  STEADY: that one is there and whole; the last stages take the form with the branches (four of them
+    // per stage left the matrix cores idle for 170 clocks, as both waves of a SIMD stand at the same barrier).  With two
+    // steps per stage the first one's products go ahead of the loads and reads, which then issue while the matrix cores work.
+    auto stage = [&](auto steady, int kt, int set) {
+        constexpr bool STEADY = decltype(steady)::value;
+        const bool mine = STEADY || kt * BKS + grp * KW < K;   // the wave's k's of the last stage may be past the end
         const int sn = so + STAGE >= NST * STAGE ? 0 : so + STAGE;
-        ldhalf(1, so, 1);
+        if (STEADY || kt + NST <= nk) __builtin_amdgcn_s_waitcnt(vm_only((NST - 2) * Cfg::LOADS));
+        else __builtin_amdgcn_s_waitcnt(vm_only(0));
+        __builtin_amdgcn_s_barrier();
         __builtin_amdgcn_sched_barrier(0);
-        mulhalf(0);
-        reads_done();                      // all my reads of this stage are back
-        issue(i + NST, so);
-        __builtin_amdgcn_sched_barrier(0);
-        __builtin_amdgcn_s_waitcnt(vm_only((NST - 1) * Cfg::LOADS));   // my next k-tile has landed
-        __builtin_amdgcn_sched_barrier(0);
-        ldhalf(0, sn, 0);
-        __builtin_amdgcn_sched_barrier(0);
-        mulhalf(1);
+        if (US == 1) ldstage(set ^ 1, sn);
+        if (mine) mul(set, 0);
+        if constexpr (STEADY) issue(kt + NST, so);
+        else if (kt + NST < nk) issue_any(kt + NST, so);
+        if (US > 1) {
+            ldstage(set ^ 1, sn);
+            if (mine) mul(set, US - 1);
+        }
         reads_done();
         so = sn;
+    };
+    int kt = 0;
+    const int steady = max(K / BKS - NST, 0) & ~1;   // stage kt + NST is whole for kt < K / BKS - NST
+    for (; kt < steady; kt += 2) {
+        stage(std::true_type{}, kt, 0);
+        stage(std::true_type{}, kt + 1, 1);
+    }
+    for (; kt < nk; kt += 2) {   // an odd number of stages ends with one in which nobody multiplies
+        stage(std::false_type{}, kt, 0);
+        stage(std::false_type{}, kt + 1, 1);
     }
     // nothing may land in LDS or in a fragment register after this point (see gemm_dma_body)
     __builtin_amdgcn_sched_barrier(0);
@@ -1146,104 +1185,130 @@ DEV void gemm_kw_body(int bid, int T, int N, int M, const h16 *__restrict__ A, i
 #pragma unroll
     for (int set = 0; set < 2; ++set) {
 #pragma unroll
-        for (int j = 0; j < BN; ++j)
+        for (int j = 0; j < WN; ++j)
 #pragma unroll
             for (int b = 0; b < 2; ++b) asm volatile("" ::"v"(fw[set][j][b]));
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
+        for (int j = 0; j < US; ++j)
 #pragma unroll
             for (int a = 0; a < 2; ++a) asm volatile("" ::"v"(fa[set][j][a]));
     }
     __builtin_amdgcn_sched_barrier(0);
-    float *mypart = (float *)base;
+    float *mypart = (float *)(smem + wave * Cfg::REGION);
 #pragma unroll
     for (int b = 0; b < 2; ++b)
 #pragma unroll
         for (int a = 0; a < 2; ++a)
 #pragma unroll
-            for (int g = 0; g < 4; ++g)
-                *(f32x4 *)(mypart + (a * 32 + row) * SW + b * 32 + 8 * g + 4 * h) =
-                    f32x4{acc[b][a][4 * g], acc[b][a][4 * g + 1], acc[b][a][4 * g + 2], acc[b][a][4 * g + 3]};
-    const bool emit = ep.emit_ry != nullptr, four = by_four(M, ldy, Y, ep);
-    const int cq = tid & 7, col = m0 + cq * 8;   // this thread's columns; its rows: tid / 8 and 32 further
+            for (int q = 0; q < 4; ++q)
+                *(f32x4 *)(mypart + (a * 32 + row) * SW + b * 32 + 8 * q + 4 * h) =
+                    f32x4{acc[b][a][4 * q], acc[b][a][4 * q + 1], acc[b][a][4 * q + 2], acc[b][a][4 * q + 3]};
+    // eight consecutive outputs of a row per thread and pass: the partial tiles of the groups are added in group order
+    constexpr int CPR = TN / 8, RPI = 512 / CPR, ITS = TM / RPI, AHEAD_ROWS = ITS < 4 ? ITS : 4;
+    auto tile_sum = [&](int r, int c, f32x4 &lo) {   // four values at tile row r, column c
+        const float *p = (const float *)(smem + ((r >> 6) * RB + (c >> 6)) * Cfg::REGION) + (r & 63) * SW + (c & 63);
+        lo = *(const f32x4 *)p;
+#pragma unroll
+        for (int k = 1; k < Cfg::KG; ++k) lo += *(const f32x4 *)(p + k * (RA * RB * Cfg::REGION / 4));
+    };
+    const int cq = tid % CPR, col = m0 + cq * 8;
     const bool col_ok = col < M;
-    EpiIn in0 = {}, in1 = {};
-    h16x8 rx8 = {}, mx8 = {};
-    Emit8 em = {};
-    if (!four) {
-        const int t = t0 + (tid >> 3);
-        in0 = epi_in(ep, t, col, t < T && col_ok, W_U8 && !lds_sums);
-        in1 = epi_in(ep, t + 32, col, t + 32 < T && col_ok, W_U8 && !lds_sums);
-        if (W_U8 && col_ok) { rx8 = load_n<h16x8, 8>(ep.rx + col, M - col); mx8 = load_n<h16x8, 8>(ep.mx + col, M - col); }
-        em = emit8(ep, col, col_ok);
-    }
-    __syncthreads();
-#pragma unroll 1
-    for (int i = 0; i < 2; ++i) {
-        const int r = (tid >> 3) + 32 * i, t = t0 + r;
-        const bool valid = t < T && col_ok;
-        float a0 = 0.f, a2 = 0.f;
-        if (four) {
-            if (t >= T) continue;
-#pragma unroll 1
-            for (int g = 0; g < 2; ++g) {
-                const int c = g * 32 + cq * 4;
-                if (m0 + c >= M) continue;
-                const float *p = (const float *)smem + r * SW + c;
-                f32x4 v = *(const f32x4 *)p;
+    if constexpr (SPLIT) {
+        __syncthreads();
+        float *slab = part + (size_t)split * T * M;
 #pragma unroll
-                for (int k = 1; k < 4; ++k) v += *(const f32x4 *)(p + k * (Cfg::REGION / 4));
-                if constexpr (W_U8) affine4(v, m0 + c, M, lds_sums ? lsum[r] : ep.s0[t], lds_sums ? lsum[64 + r] : ep.s2[t], ep);
-                finish_row4(v, t, m0 + c, M, ep, Y, ldy);
-            }
-            continue;
+        for (int it = 0; it < ITS; ++it) {
+            const int r = it * RPI + tid / CPR, t = t0 + r;
+            f32x4 lo, hi;
+            tile_sum(r, cq * 8, lo);
+            tile_sum(r, cq * 8 + 4, hi);
+            if (t < T && col < M) *(f32x4 *)(slab + (size_t)t * M + col) = lo;           // M % 4 == 0
+            if (t < T && col + 4 < M) *(f32x4 *)(slab + (size_t)t * M + col + 4) = hi;
         }
-        if (valid) {
-            const float *p = (const float *)smem + r * SW + cq * 8;
-            f32x4 lo = *(const f32x4 *)p, hi = *(const f32x4 *)(p + 4);
-#pragma unroll
-            for (int k = 1; k < 4; ++k) {
-                lo += *(const f32x4 *)(p + k * (Cfg::REGION / 4));
-                hi += *(const f32x4 *)(p + k * (Cfg::REGION / 4) + 4);
-            }
-            float v[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-            const EpiIn in = i ? in1 : in0;
-            if constexpr (W_U8) affine8(v, rx8, mx8, lds_sums ? lsum[r] : in.s0, lds_sums ? lsum[64 + r] : in.s2);
-            finish_row8<true>(v, in, t, col, ep, Y, ldy, em, a0, a2);
+    } else {
+        const bool emit = ep.emit_ry != nullptr, four = by_four(M, ldy, Y, ep);
+        h16x8 rx8 = {}, mx8 = {};
+        Emit8 em = {};
+        EpiIn in[AHEAD_ROWS] = {};
+        if (!four) {
+            if (W_U8 && col_ok) { rx8 = load_n<h16x8, 8>(ep.rx + col, M - col); mx8 = load_n<h16x8, 8>(ep.mx + col, M - col); }
+            em = emit8(ep, col, col_ok);
         }
-        if (emit) {   // the eight threads of a row are neighbours in one wave; every lane takes part
+#pragma unroll 1
+        for (int it = 0; it < ITS; ++it) {
+            const int r = it * RPI + tid / CPR, t = t0 + r;
+            if (it % AHEAD_ROWS == 0) {
+                if (!four) {
 #pragma unroll
-            for (int o = 1; o < 8; o <<= 1) { a0 += __shfl_xor(a0, o, WAVE); a2 += __shfl_xor(a2, o, WAVE); }
-            if (valid && cq == 0) {
-                const size_t pi = (size_t)t * ((M + 63) / 64) + m0 / 64;
-                ep.emit_s0[pi] = a0;
-                ep.emit_s2[pi] = a2;
+                    for (int i = 0; i < AHEAD_ROWS; ++i) in[i] = epi_in(ep, t + i * RPI, col, t + i * RPI < T && col_ok, W_U8 && !lds_sums);
+                }
+                if (it == 0) __syncthreads();   // the partial tiles are in LDS
+            }
+            const EpiIn cur = in[0];
+#pragma unroll
+            for (int i = 0; i + 1 < AHEAD_ROWS; ++i) in[i] = in[i + 1];
+            const bool valid = t < T && col_ok;
+            float a0 = 0.f, a2 = 0.f;
+            if (four) {
+                if (t >= T) continue;
+#pragma unroll 1
+                for (int g = 0; g < 2; ++g) {
+                    const int c = g * (TN / 2) + cq * 4;
+                    if (m0 + c >= M) continue;
+                    f32x4 v;
+                    tile_sum(r, c, v);
+                    if constexpr (W_U8) affine4(v, m0 + c, M, lds_sums ? lsum[r] : ep.s0[t], lds_sums ? lsum[TM + r] : ep.s2[t], ep);
+                    finish_row4(v, t, m0 + c, M, ep, Y, ldy);
+                }
+                continue;
+            }
+            if (valid) {
+                f32x4 lo, hi;
+                tile_sum(r, cq * 8, lo);
+                tile_sum(r, cq * 8 + 4, hi);
+                float v[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+                if constexpr (W_U8) affine8(v, rx8, mx8, lds_sums ? lsum[r] : cur.s0, lds_sums ? lsum[TM + r] : cur.s2);
+                finish_row8<true>(v, cur, t, col, ep, Y, ldy, em, a0, a2);
+            }
+            if (emit) {   // the CPR threads of a row are neighbours in one wave; every lane takes part
+#pragma unroll
+                for (int o = 1; o < CPR; o <<= 1) { a0 += __shfl_xor(a0, o, WAVE); a2 += __shfl_xor(a2, o, WAVE); }
+                if (valid && cq == 0) {
+                    const size_t pi = (size_t)t * ((M + TN - 1) / TN) + m0 / TN;
+                    ep.emit_s0[pi] = a0;
+                    ep.emit_s2[pi] = a2;
+                }
             }
         }
     }
 }
 
-template <bool W_U8>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void gemm_kw_kernel(int T, int N, GemmGroup g) {
+template <bool W_U8, bool SPLIT, int TM, int TN>
+__global__ __launch_bounds__(512) void gemm_kg_kernel(int T, int N, GemmGroup g) {
     int tile = xcd_tile();
     const int gi = group_member(g, tile), M = g.M[gi];
-    gemm_kw_body<W_U8>(tile, T, N, M, g.A[gi], g.lda, g.W[gi], g.ldw[gi], g.Y[gi], g.ldy[gi], g.ep[gi]);
+    gemm_kg_body<W_U8, SPLIT, TM, TN>(tile, T, N, M, g.A[gi], g.lda, g.W[gi], g.ldw[gi], g.Y[gi], g.ldy[gi], g.ep[gi],
+                                      SPLIT ? g.nk_split : N / BK, g.part[gi], SPLIT ? blockIdx.y : 0);
 }
 
-template <bool W_U8>
-int launch_kw(GemmGroup &g, int n, int64_t T, int64_t N, hipStream_t st) {
-    constexpr size_t lds = KwCfg<W_U8>::LDS;
+template <bool W_U8, int TM, int TN>
+int launch_kg(GemmGroup &g, int n, int64_t T, int64_t N, int ks, hipStream_t st) {
+    constexpr size_t lds = KgCfg<W_U8, TM, TN>::LDS;
     static PerDeviceOnce once;
     bool *attr_done = once.slot();
     if (!attr_done || !*attr_done) {
-        const hipError_t e = hipFuncSetAttribute((const void *)gemm_kw_kernel<W_U8>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        hipError_t e = hipFuncSetAttribute((const void *)gemm_kg_kernel<W_U8, false, TM, TN>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        if (e == hipSuccess) e = hipFuncSetAttribute((const void *)gemm_kg_kernel<W_U8, true, TM, TN>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) return (int)e;
         if (attr_done) *attr_done = true;
     }
-    hipLaunchKernelGGL((gemm_kw_kernel<W_U8>), dim3((unsigned)group_tiles(g, n, T, 64, 64)), dim3(256), lds, st, (int)T, (int)N, g);
+    const dim3 grid((unsigned)group_tiles(g, n, T, TM, TN), (unsigned)ks);
+    if (ks > 1) hipLaunchKernelGGL((gemm_kg_kernel<W_U8, true, TM, TN>), grid, dim3(512), lds, st, (int)T, (int)N, g);
+    else hipLaunchKernelGGL((gemm_kg_kernel<W_U8, false, TM, TN>), grid, dim3(512), lds, st, (int)T, (int)N, g);
     RWKV_LAUNCH_CHECK();
     return RWKV_OK;
 }
+
 // second pass of a split group launch: member blockIdx.y, as splitk_epilogue8_kernel
 __global__ __launch_bounds__(256) void splitk_group_epilogue8_kernel(int T, int KS, GemmGroup g) {
     const int gi = blockIdx.y;
@@ -1611,10 +1676,11 @@ bool dma_ok(bool w_u8, int64_t N, int64_t M, const void *A, int64_t lda, const v
     return true;
 }
 
-// The direct-to-LDS tiles: rows and columns.  TILE_S4 is TILE_S with four stages, TILE_K gemm_kw_kernel.
-enum { TILE_L, TILE_S, TILE_S4, TILE_N, TILE_K, TILES };
+// The direct-to-LDS tiles: rows and columns.  TILE_S4 is TILE_S with four stages, TILE_K8 and TILE_K4 gemm_kg_kernel with
+// eight and four groups.
+enum { TILE_L, TILE_S, TILE_S4, TILE_N, TILE_K8, TILE_K4, TILES };
 struct TileDim { int tm, tn; };
-constexpr TileDim tile_dim[TILES] = {{256, 256}, {128, 128}, {128, 128}, {64, 128}, {64, 64}};
+constexpr TileDim tile_dim[TILES] = {{256, 256}, {128, 128}, {128, 128}, {64, 128}, {64, 64}, {64, 128}};
 
 // Cost model of a direct-to-LDS launch in microseconds, fitted to launches of the 7B shapes (20 to 4096 rows):
 // `tiles` tiles of nk k-tiles split c ways run in whole rounds over the 256 CUs; a k-tile step takes 1.75 us with
@@ -1632,8 +1698,13 @@ constexpr TileDim tile_dim[TILES] = {{256, 256}, {128, 128}, {128, 128}, {64, 12
 // n_embd 1280, 777 tokens 938 -> 979 us with uint8 weights, 994 -> 1028 with fp16).  And fp16 weights, whose tiles are twice
 // the bytes, over long K: 0.50 us a step with 160 CUs busy where the last row of tiles is full, 0.42 where it is not (640 x
 // 14336 x 4096 130 us against 102 in four splits of the 256 x 256 tile, 513 rows 102 against 100).
-// The reduction pass of a split takes 2.5 us + 3.6 us per slab and 16 MB of fp32 output, at least 4.5 us.  The 64 x 64 tile
-// with K over the waves: 0.245 us per k-tile, 4 us per round and 2.5 us per launch, never split over workgroups.
+// The reduction pass of a split takes 2.5 us + 3.6 us per slab and 16 MB of fp32 output, at least 4.5 us.
+// A round of 256 x 256 tiles that leaves CUs idle runs at a higher clock: 1.17 - 1.28 us a step up to 128 workgroups, 1.38 at
+// 192, 1.70 at 256.  Priced as a full round, the receptance / key / value group of 1024 rows and 4096 channels (192 tiles) went
+// to three rounds of 128 x 128 ones: 114 us against 103 with uint8 weights, 127 against 110 with fp16.
+// gemm_kg_kernel: per launch, per round (split launches leave the epilogue to the second pass) and per k-tile by the CUs busy,
+// fitted to 1640 products (21 lengths, 8 widths) with the other tiles' prices as they stand: the tile it picks is 1.5 % slower
+// than the best of all on average, 4.2 % with the four tiles and prices before; 3.3 % less time.
 // slow_epi: see slow_epilogue.
 struct CostOf { bool w_u8, slow_epi; };
 bool slow_epilogue(const GemmEpi &ep) { return ep.act == ACT_RESIDUAL || ep.act == ACT_GATED_RESIDUAL || ep.act == ACT_SIGMOID; }
@@ -1641,7 +1712,11 @@ double dma_cost(CostOf of, int tile, int64_t T, int64_t tiles, int nk, int c, si
     const int64_t wgs = tiles * c, rounds = (wgs + 255) / 256;
     const double reduce = c > 1 ? std::max(4.5, 2.5 + 3.6 * c * (double)out_bytes / (16 << 20)) : 0.0;
     switch (tile) {
-        case TILE_L: return (double)rounds * (nk / c + (c > 1 ? 4.3 : 10.0)) * 1.75 + reduce;
+        case TILE_L: {
+            const int64_t last = wgs % 256;
+            const double step = 1.28 + 0.47 * std::max<double>((double)(last - 128) / 128, 0.0);
+            return (nk / c + (c > 1 ? 4.3 : 10.0)) * ((double)(wgs / 256) * 1.75 + (last ? step : 0.0)) + reduce;
+        }
         case TILE_S: return (double)rounds * (nk / c + (rounds > 1 ? 5.5 : 12.8)) * 0.573 + reduce;
         case TILE_S4:
             if (rounds > 1) return 1e30;
@@ -1649,7 +1724,16 @@ double dma_cost(CostOf of, int tile, int64_t T, int64_t tiles, int nk, int c, si
                 return (nk / c + 17.0) * (0.42 + 0.12 * (double)wgs / 256) * (0.55 + 0.45 * T / (double)((T + 127) / 128 * 128)) + reduce;
             return (nk / c + 22.0) * std::min(0.50, 0.34 + 0.19 * (double)wgs / 256) + reduce + (c == 1 && of.slow_epi && nk < 32 ? 2.0 : 0.0);
         case TILE_N: return T > 64 ? 1e30 : (double)rounds * (nk / c + std::max(16.5, 13.0 + T / 10.0)) * 0.327 + reduce;
-        default: return c > 1 ? 1e30 : (double)rounds * (nk * 0.245 + 4.0) + 2.5;
+        default: {
+            // [uint8][groups 8, 4]
+            constexpr struct { double launch, round, split_round, step_0, step_1; } kg[2][2] = {
+                {{3.0, 2.6, 3.6, 0.195, 0.212}, {2.8, 3.6, 4.8, 0.170, 0.420}}, {{2.1, 3.0, 2.5, 0.140, 0.186}, {2.9, 4.2, 3.8, 0.212, 0.320}}};
+            const auto &k = kg[of.w_u8][tile == TILE_K4];
+            const int64_t last = wgs % 256;
+            const double round = c > 1 ? k.split_round : k.round, n = nk / c;
+            return k.launch + (double)(wgs / 256) * (round + n * k.step_1) +
+                   (last ? round + n * (k.step_0 + (k.step_1 - k.step_0) * (double)last / 256) : 0.0) + reduce;
+        }
     }
 }
 
@@ -1683,7 +1767,18 @@ int dma_tile(CostOf of, int64_t T, int nk, int n, const int64_t *M, size_t ws_by
     return best;
 }
 
-// gemm_dma_kernel with K split ks ways (slabs as in launch_cfg; the second pass eight outputs wide where M is a multiple).
+// The second pass of a direct-to-LDS launch with K split ks ways: eight outputs wide where M is a multiple.
+int launch_splitk_epilogue(int ks, int64_t T, int64_t M, void *Y, int64_t ldy, const GemmEpi &ep, hipStream_t st) {
+    const int64_t n = T * M;
+    const int per_block = M & 7 ? 1024 : 2048;
+    const unsigned blocks = (unsigned)std::min<int64_t>((n + per_block - 1) / per_block, 16384);
+    if (M & 7) hipLaunchKernelGGL(splitk_epilogue_kernel, dim3(blocks), dim3(256), 0, st, (int)T, (int)M, ks, ep.splitk_ws, Y, ldy, ep);
+    else hipLaunchKernelGGL(splitk_epilogue8_kernel, dim3(blocks), dim3(256), 0, st, (int)T, (int)M, ks, ep.splitk_ws, Y, ldy, ep);
+    RWKV_LAUNCH_CHECK();
+    return RWKV_OK;
+}
+
+// gemm_dma_kernel with K split ks ways (slabs as in launch_cfg).
 template <bool W_U8, int TM, int TN, int NW, int NSTG>
 int launch_dma(int ks, int64_t T, int64_t N, int64_t M, const rwkv_half *A, int64_t lda, const void *W, int64_t ldw, void *Y,
                int64_t ldy, const GemmEpi &ep, hipStream_t st) {
@@ -1703,11 +1798,7 @@ int launch_dma(int ks, int64_t T, int64_t N, int64_t M, const rwkv_half *A, int6
     if (ks > 1) {
         hipLaunchKernelGGL((gemm_dma_kernel<W_U8, true, TM, TN, NW, NSTG>), dim3((unsigned)tiles, (unsigned)ks), dim3(64 * NW), lds, st, (int)T, (int)N,
                            (int)M, (const h16 *)A, lda, W, ldw, Y, ldy, ep, nk / ks, ep.splitk_ws);
-        const int64_t n = T * M;
-        const int per_block = M & 7 ? 1024 : 2048;
-        const unsigned blocks = (unsigned)std::min<int64_t>((n + per_block - 1) / per_block, 16384);
-        if (M & 7) hipLaunchKernelGGL(splitk_epilogue_kernel, dim3(blocks), dim3(256), 0, st, (int)T, (int)M, ks, ep.splitk_ws, Y, ldy, ep);
-        else hipLaunchKernelGGL(splitk_epilogue8_kernel, dim3(blocks), dim3(256), 0, st, (int)T, (int)M, ks, ep.splitk_ws, Y, ldy, ep);
+        return launch_splitk_epilogue(ks, T, M, Y, ldy, ep, st);
     } else {
         hipLaunchKernelGGL((gemm_dma_kernel<W_U8, false, TM, TN, NW, NSTG>), dim3((unsigned)tiles), dim3(64 * NW), lds, st, (int)T, (int)N, (int)M,
                            (const h16 *)A, lda, W, ldw, Y, ldy, ep, nk, (float *)nullptr);
@@ -1729,17 +1820,23 @@ int launch_pick(int cfg, int ks, int64_t T, int64_t N, int64_t M, const rwkv_hal
         case CFG_DMA + TILE_S: return launch_dma<W_U8, 128, 128, 8, 0>(ks, T, N, M, A, lda, W, ldw, Y, ldy, ep, st);
         case CFG_DMA + TILE_S4: return launch_dma<W_U8, 128, 128, 8, 4>(ks, T, N, M, A, lda, W, ldw, Y, ldy, ep, st);
         case CFG_DMA + TILE_N: return launch_dma<W_U8, 64, 128, 4, 4>(ks, T, N, M, A, lda, W, ldw, Y, ldy, ep, st);
-        case CFG_DMA + TILE_K: {
+        case CFG_DMA + TILE_K8:
+        case CFG_DMA + TILE_K4: {
             GemmGroup g{};
             g.A[0] = (const h16 *)A; g.W[0] = W; g.Y[0] = Y; g.lda = lda; g.ldw[0] = ldw; g.ldy[0] = ldy; g.M[0] = (int)M; g.ep[0] = ep;
-            return launch_kw<W_U8>(g, 1, T, N, st);
+            g.nk_split = (int)(N / BK) / ks;
+            g.part[0] = ep.splitk_ws;
+            const int rc = cfg == CFG_DMA + TILE_K8 ? launch_kg<W_U8, 64, 64>(g, 1, T, N, ks, st) : launch_kg<W_U8, 64, 128>(g, 1, T, N, ks, st);
+            if (rc || ks == 1) return rc;
+            return launch_splitk_epilogue(ks, T, M, Y, ldy, ep, st);
         }
         default: return RWKV_E_DTYPE;
     }
 }
 
-// Tile choice (RWKV_GEMM_CFG = 3, 9, 14 or 15 overrides it for tuning sweeps: the register-staged tiles by their number
-// here, the direct-to-LDS 256 x 256 and 128 x 128 tiles with the K split of least cost).
+// Tile choice (RWKV_GEMM_CFG = 3, 9, 14, 15, 20 or 21 overrides it for tuning sweeps: the register-staged tiles by their
+// number here, the direct-to-LDS 256 x 256 and 128 x 128 tiles and gemm_kg_kernel's 64 x 64 and 64 x 128 ones with the K split
+// of least cost).
 //   CFG_DMA +  operands laid out for 16-byte loads: the direct-to-LDS kernel with the tile and K split that the cost
 //              model puts first (128 x 128 tiles at full depth when another product runs beside this one: a 256 x 256
 //              tile's LDS leaves no room beside it on the CU, two small ones fit)
@@ -1761,7 +1858,8 @@ int pick_cfg(int64_t T, int64_t N, int64_t M, bool w_u8, const GemmEpi &ep, bool
     const char *e = getenv("RWKV_GEMM_CFG");
     if (e && *e) {
         const int cfg = atoi(e);
-        return cfg == 14 ? with_split(TILE_L) : cfg == 15 ? with_split(TILE_S) : cfg < CFG_DMA ? cfg : -1;
+        return cfg == 14 ? with_split(TILE_L) : cfg == 15 ? with_split(TILE_S) : cfg == CFG_DMA + TILE_K8 ? with_split(TILE_K8)
+             : cfg == CFG_DMA + TILE_K4 ? with_split(TILE_K4) : cfg < CFG_DMA ? cfg : -1;
     }
     if (dma && !alone) return with_split(TILE_S);
     if (dma) return CFG_DMA + dma_tile(of, T, (int)(N / BK), 1, &M, ws, ks);
@@ -1890,7 +1988,8 @@ int gemm_group_launch(bool w_u8, int n, int64_t T, int64_t N, const rwkv_half *c
             case TILE_L: rc = w_u8 ? launch_dma_group<true, 256, 256, 8, 0>(g, n, T, N, ks, st) : launch_dma_group<false, 256, 256, 8, 0>(g, n, T, N, ks, st); break;
             case TILE_S: rc = w_u8 ? launch_dma_group<true, 128, 128, 8, 0>(g, n, T, N, ks, st) : launch_dma_group<false, 128, 128, 8, 0>(g, n, T, N, ks, st); break;
             case TILE_S4: rc = w_u8 ? launch_dma_group<true, 128, 128, 8, 4>(g, n, T, N, ks, st) : launch_dma_group<false, 128, 128, 8, 4>(g, n, T, N, ks, st); break;
-            case TILE_K: rc = w_u8 ? launch_kw<true>(g, n, T, N, st) : launch_kw<false>(g, n, T, N, st); break;
+            case TILE_K8: rc = w_u8 ? launch_kg<true, 64, 64>(g, n, T, N, ks, st) : launch_kg<false, 64, 64>(g, n, T, N, ks, st); break;
+            case TILE_K4: rc = w_u8 ? launch_kg<true, 64, 128>(g, n, T, N, ks, st) : launch_kg<false, 64, 128>(g, n, T, N, ks, st); break;
             default: rc = w_u8 ? launch_dma_group<true, 64, 128, 4, 4>(g, n, T, N, ks, st) : launch_dma_group<false, 64, 128, 4, 4>(g, n, T, N, ks, st); break;
         }
         if (rc) return rc;

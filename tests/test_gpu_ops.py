@@ -134,8 +134,8 @@ def test_mm8_seq_tile_edges(N, M, B):
 @pytest.mark.parametrize("N,M,B", [(64, 64, 65), (128, 8, 100), (320, 72, 129), (768, 768, 513), (1024, 1000, 70), (2048, 2048, 333),
                                    (4096, 1032, 256)])
 def test_64x64_tile_edges(N, M, B):
-    """The 64 x 64 tile with K over its four waves, both weight types: fewer k-tiles than waves, k-tiles that do not divide
-    by four, ragged rows and columns; bounds as in test_mm8_seq and test_gemm_f16."""
+    """Products of a few tiles, both weight types: few k-tiles, ragged rows and columns; bounds as in test_mm8_seq and
+    test_gemm_f16."""
     ops = _ops()
     x, ref, (q, mx, rx, my, ry) = _mm8_case(N, M, B, N + M + B)
     xt = torch.from_numpy(x).to(DEV)
@@ -180,6 +180,24 @@ def test_mm8_epilogue_rounding(N, M, B):
         assert (want != at_once).any()                            # the two ways of rounding can be told apart here
     y = _ops().cuda_mm8_seq(B, N, M, torch.from_numpy(x).to(DEV), _to_dev_ic(q), *(torch.from_numpy(a).to(DEV) for a in (mx, rx, my, ry)))
     assert np.array_equal(y.cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("cfg", ["20", "21"])
+@pytest.mark.parametrize("N,M,B", [(64, 64, 17), (128, 8, 100), (192, 136, 45), (320, 1000, 64), (448, 520, 65), (1088, 264, 130),
+                                   (4096, 768, 100), (4160, 260, 33), (16384, 1004, 100)])
+def test_wave_group_tiles(N, M, B, cfg, monkeypatch):
+    """The 64 x 64 and 64 x 128 tiles whose wave groups share K, both weight types: K shorter than a stage, a last stage that
+    is there in part, an odd number of stages, ragged rows and columns, K splits (the last three).  The sums are exact, so
+    the results are equal bit for bit."""
+    ops = _ops()
+    x, (q, mx, rx, my, ry), want, _ = _affine_case(N, M, B, N + M + B)
+    xt = torch.from_numpy(x).to(DEV)
+    monkeypatch.setenv("RWKV_GEMM_CFG", cfg)
+    y = ops.cuda_mm8_seq(B, N, M, xt, _to_dev_ic(q), *(torch.from_numpy(a).to(DEV) for a in (mx, rx, my, ry)))
+    assert np.array_equal(y.cpu().numpy(), want)
+    w = (_rng(N).integers(-64, 65, (N, M)) / 64).astype(np.float16)
+    y = ops.matmul_float(xt, _to_dev_ic(w), output_dtype=torch.float32)
+    assert np.array_equal(y.cpu().numpy(), x.astype(np.float64) @ w.astype(np.float64))
 
 
 @pytest.mark.parametrize("N,M,B", [(4096, 4096, 100), (768, 3072, 513)])
