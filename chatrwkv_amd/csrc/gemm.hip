@@ -501,6 +501,17 @@ DEV int xcd_tile() {
     const int bid = blockIdx.x;
     return (gridDim.x & 7) == 0 ? (bid & 7) * (gridDim.x >> 3) + (bid >> 3) : bid;
 }
+// Its place.  The walk goes along T, so that an XCD reads all activations and its own part of the weights, unless the activations
+// are the larger operand and more than its 4 MB of L2 hold: then along M.  us, uint8, T -> M: 64 x 64 tile, [2048 x 4096] x [4096 x
+// 1024] 49.0 -> 29.1, [777 x 4096] x [4096 x 512] 16.1 -> 14.7; [2048 x 3072] x [3072 x 768] 64 x 128 tile 18.9 -> 17.6, 128 x 128
+// in two splits 21.8 -> 20.9; activations that fit: [2048 x 768] x [768 x 768] 10.7 -> 11.2, [1400 x 1024] x [1024 x 1024] 11.7 -> 12.3.
+bool walks_m(bool w_u8, int64_t T, int64_t N, int64_t M) { return T * 2 > M * (w_u8 ? 1 : 2) && T * N > (2 << 20); }
+struct TileAt { int t0, m0; };
+template <int TM, int TN>
+DEV TileAt tile_at(int bid, int T, int M, int walk_m) {
+    const int n = walk_m ? (M + TN - 1) / TN : (T + TM - 1) / TM, q = bid / n, r = bid - q * n;
+    return {(walk_m ? q : r) * TM, (walk_m ? r : q) * TN};
+}
 // s_waitcnt immediates: vmcnt(n) alone, vmcnt(n) with lgkmcnt(0), lgkmcnt(n) alone
 constexpr int vm_only(int n) { return 0x0F70 | (n & 15) | ((n >> 4) << 14); }
 constexpr int vm_lgkm0(int n) { return 0x0070 | (n & 15) | ((n >> 4) << 14); }
@@ -517,8 +528,8 @@ DEV void gemm_dma_body(int bid, int T, int N, int M, const h16 *__restrict__ A, 
     extern __shared__ __align__(1024) unsigned char smem[];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wr = wave / Cfg::WC, wc = wave % Cfg::WC;
-    const int tiles_t = (T + TM - 1) / TM;
-    const int t0 = (bid % tiles_t) * TM, m0 = (bid / tiles_t) * TN;
+    const TileAt at = tile_at<TM, TN>(bid, T, M, ep.walk_m);
+    const int t0 = at.t0, m0 = at.m0;
     const int kbase = SPLIT ? split * nk_split : 0, nk = SPLIT ? nk_split : N / BK;
 
     // load sources; rows past the end re-read the last row (never stored)
@@ -925,9 +936,10 @@ DEV int group_member(const GemmGroup &g, int &tile) {
     tile -= g.first[gi];
     return gi;
 }
-// fills `first` for tiles of tm x tn; returns the tiles of the launch
-int64_t group_tiles(GemmGroup &g, int n, int64_t T, int tm, int tn) {
+// fills `first` and the walks for tiles of tm x tn; returns the tiles of the launch
+int64_t group_tiles(bool w_u8, GemmGroup &g, int n, int64_t T, int64_t N, int tm, int tn) {
     int64_t tiles = 0;
+    for (int i = 0; i < n; ++i) g.ep[i].walk_m = walks_m(w_u8, T, N, g.M[i]);
     for (int i = 0; i < 4; ++i) {
         g.first[i] = i < n ? (int)tiles : 0x7fffffff;
         if (i < n) tiles += ((T + tm - 1) / tm) * ((g.M[i] + tn - 1) / tn);
@@ -958,7 +970,7 @@ int launch_dma_group(GemmGroup &g, int n, int64_t T, int64_t N, int ks, hipStrea
         if (e != hipSuccess) return (int)e;
         if (attr_done) *attr_done = true;
     }
-    const dim3 grid((unsigned)group_tiles(g, n, T, TM, TN), (unsigned)ks);
+    const dim3 grid((unsigned)group_tiles(W_U8, g, n, T, N, TM, TN), (unsigned)ks);
     if (ks > 1) hipLaunchKernelGGL((gemm_dma_group_kernel<W_U8, true, TM, TN, NW, NSTG>), grid, dim3(64 * NW), lds, st, (int)T, (int)N, g);
     else hipLaunchKernelGGL((gemm_dma_group_kernel<W_U8, false, TM, TN, NW, NSTG>), grid, dim3(64 * NW), lds, st, (int)T, (int)N, g);
     return RWKV_OK;
@@ -1008,8 +1020,8 @@ DEV void gemm_kg_body(int bid, int T, int N, int M, const h16 *__restrict__ A, i
     extern __shared__ __align__(1024) unsigned char smem[];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int blk = wave % (RA * RB), grp = wave / (RA * RB), wr = blk / RB, wc = blk % RB;
-    const int tiles_t = (T + TM - 1) / TM;
-    const int t0 = (bid % tiles_t) * TM, m0 = (bid / tiles_t) * TN;
+    const TileAt at = tile_at<TM, TN>(bid, T, M, ep.walk_m);
+    const int t0 = at.t0, m0 = at.m0;
     const int kbase = SPLIT ? split * nk_split * BK : 0, K = SPLIT ? nk_split * BK : N;   // this workgroup's k's (a multiple of 64)
     const int nk = (K + BKS - 1) / BKS;
 
@@ -1302,7 +1314,7 @@ int launch_kg(GemmGroup &g, int n, int64_t T, int64_t N, int ks, hipStream_t st)
         if (e != hipSuccess) return (int)e;
         if (attr_done) *attr_done = true;
     }
-    const dim3 grid((unsigned)group_tiles(g, n, T, TM, TN), (unsigned)ks);
+    const dim3 grid((unsigned)group_tiles(W_U8, g, n, T, N, TM, TN), (unsigned)ks);
     if (ks > 1) hipLaunchKernelGGL((gemm_kg_kernel<W_U8, true, TM, TN>), grid, dim3(512), lds, st, (int)T, (int)N, g);
     else hipLaunchKernelGGL((gemm_kg_kernel<W_U8, false, TM, TN>), grid, dim3(512), lds, st, (int)T, (int)N, g);
     RWKV_LAUNCH_CHECK();
@@ -1781,7 +1793,7 @@ int launch_splitk_epilogue(int ks, int64_t T, int64_t M, void *Y, int64_t ldy, c
 // gemm_dma_kernel with K split ks ways (slabs as in launch_cfg).
 template <bool W_U8, int TM, int TN, int NW, int NSTG>
 int launch_dma(int ks, int64_t T, int64_t N, int64_t M, const rwkv_half *A, int64_t lda, const void *W, int64_t ldw, void *Y,
-               int64_t ldy, const GemmEpi &ep, hipStream_t st) {
+               int64_t ldy, GemmEpi ep, hipStream_t st) {
     constexpr size_t lds = DmaCfg<W_U8, TM, TN, NW, NSTG>::LDS;
     static PerDeviceOnce once;
     bool *attr_done = once.slot();
@@ -1793,6 +1805,7 @@ int launch_dma(int ks, int64_t T, int64_t N, int64_t M, const rwkv_half *A, int6
         if (attr_done) *attr_done = true;
     }
     if (!dma_ok(W_U8, N, M, A, lda, W, ldw, Y, ldy, ep)) return RWKV_E_LAYOUT;
+    ep.walk_m = walks_m(W_U8, T, N, M);
     const int64_t tiles = ((T + TM - 1) / TM) * ((M + TN - 1) / TN);
     const int nk = (int)(N / BK);
     if (ks > 1) {

@@ -29,6 +29,7 @@ struct GemmEpi {
     float *emit_s0, *emit_s2;
     int parts;
     const float *p0, *p2;
+    int walk_m;                    // set by the launch: consecutive tiles walk along M first (direct-to-LDS launches)
 };
 
 // How gemm_launch would run a product: kind 0 = the 2..16-row kernel, 1 = register-staged tiles, 2 = direct-to-LDS
