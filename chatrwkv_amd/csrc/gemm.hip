@@ -24,17 +24,6 @@
 #include <cstdlib>
 #include <mutex>
 
-// Set-up that must run once per device (function attributes belong to the current device's copy of a kernel).
-struct PerDeviceOnce {
-    bool done[64] = {};
-    // the slot of the current device, or nullptr when the device cannot be read (the caller then repeats the set-up)
-    bool *slot() {
-        int dev = 0;
-        if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return nullptr;
-        return &done[dev];
-    }
-};
-
 namespace {
 
 constexpr int BK = 64;  // halves per LDS row

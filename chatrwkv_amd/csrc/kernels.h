@@ -2,6 +2,17 @@
 #pragma once
 #include "common.h"
 
+// Set-up that must run once per device (function attributes belong to the current device's copy of a kernel).
+struct PerDeviceOnce {
+    bool done[64] = {};
+    // the slot of the current device, or nullptr when the device cannot be read (the caller then repeats the set-up)
+    bool *slot() {
+        int dev = 0;
+        if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return nullptr;
+        return &done[dev];
+    }
+};
+
 enum { ACT_NONE = 0, ACT_SIGMOID = 1, ACT_RELU_SQ = 2, ACT_RESIDUAL = 3, ACT_GATED_RESIDUAL = 4, ACT_SILU = 5, ACT_TANH = 6 };
 
 // Epilogue of the MFMA contraction (gemm.hip).

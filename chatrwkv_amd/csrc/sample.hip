@@ -85,11 +85,89 @@ DEV float wave_scan(float v) {
     return v;
 }
 
+// Does a bound hold whose entries add up to t?  The nucleus cut asks for a sum, the k-th largest value (top_k >= 0) for a count.
+DEV bool enough(SumCount t, float top_p, int top_k) { return top_k >= 0 ? t.n >= (float)top_k : t.s >= top_p; }
+
+// The largest bit pattern c in [lo, hi) that holds, from the n <= LIST_MAX entries of [lo, hi) in LDS: it holds at lo (the
+// entries from there on: at_lo) and not at hi (at_hi).
+DEV unsigned search_list(const float *list, int n, unsigned lo, unsigned hi, SumCount at_lo, SumCount at_hi, float top_p, int top_k,
+                         float *tail, f32x4 (&red)[2][SWAVES / 2], int &turn) {
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const SumCount past_hi = at_hi;
+            float left = (float)n;   // entries still between the bounds
+            while (hi - lo > 1 && left > 64.f) {
+                const unsigned step = (hi - lo) / (SWAVES + 1) + 1;
+                const unsigned c = lo + step * (wave + 1);
+                SumCount t = at_hi;      // the totals at hi and past it
+                if (c < hi) {
+                    const float fc = __uint_as_float(c);
+                    float sc = 0.f, k = 0.f;
+                    for (int i = lane; i < n; i += 64) {
+                        const float v = list[i];
+                        if (v >= fc) { sc += v; k += 1.f; }
+                    }
+                    t.s = past_hi.s + wave_sum(sc);
+                    t.n = past_hi.n + wave_sum(k);
+                }
+                f32x4 *buf = red[turn];
+                turn ^= 1;
+                if (lane == 0) {
+                    ((float *)buf)[2 * wave] = t.s;
+                    ((float *)buf)[2 * wave + 1] = t.n;
+                }
+                __syncthreads();
+                int good = 0;            // the bounds that hold are a leading run up to rounding: take the largest
+                SumCount above_good = at_hi;
+    #pragma unroll
+                for (int w = SWAVES - 1; w >= 0; --w) {
+                    const SumCount q = {((float *)buf)[2 * w], ((float *)buf)[2 * w + 1]};
+                    if (good == 0) {
+                        if (lo + step * (w + 1) < hi && enough(q, top_p, top_k)) { good = w + 1; at_lo = q; }
+                        else above_good = q;
+                    }
+                }
+                hi = min(hi, lo + step * (good + 1));
+                lo = lo + step * good;
+                at_hi = above_good;
+                left = at_lo.n - at_hi.n;
+            }
+            if (hi - lo <= 1) return lo;
+            // at most 64 are left: one to a lane, in list order; the largest of them at which the condition holds is the answer
+            {
+                const float l1 = __uint_as_float(max(lo, 1u)), h1 = __uint_as_float(hi);
+                if (wave == 0) {
+                    int at64 = 0;
+                    for (int i0 = 0; i0 < n; i0 += 64) {
+                        const float v = i0 + lane < n ? list[i0 + lane] : 0.f;
+                        const bool in = v >= l1 && v < h1;
+                        const unsigned long long m = __ballot(in);
+                        if (in) tail[min(at64 + (int)__popcll(m & ((1ull << lane) - 1)), 63)] = v;
+                        at64 += (int)__popcll(m);
+                    }
+                    if (lane >= at64) tail[lane] = 0.f;
+                }
+                __syncthreads();
+                const float mine64 = tail[lane];
+                SumCount t = at_hi;
+    #pragma unroll 2
+                for (int i = 0; i < 64; i += 4) {
+                    const f32x4 v = *(const f32x4 *)&tail[i];
+    #pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        if (v[e] >= mine64) { t.s += v[e]; t.n += v[e] > 0.f ? 1.f : 0.f; }
+                }
+                const float best = wave_max(mine64 > 0.f && enough(t, top_p, top_k) ? mine64 : 0.f);
+                __syncthreads();         // the lists may be written again
+                if (best > 0.f) lo = __float_as_uint(best);
+            }
+    return lo;
+}
+
 // POW: temperature other than 1 (its 64 copies stay out of the code of the usual case)
 // SROWS: group rows, at least V / 4096.  Rows past the end hold zeros and are worked on like the others: with a test
 // of V around each row the compiler made a copy of what follows for every number of rows.
 template <int SROWS, bool POW>
-__global__ __launch_bounds__(STHREADS) void sample_kernel(SampleArgs a) {
+DEV void sample_one_workgroup(const SampleArgs &a) {
     __shared__ f32x4 red[2][SWAVES / 2];
     __shared__ float list[LIST_MAX];
     __shared__ __align__(16) float tail[64];
@@ -193,17 +271,15 @@ __global__ __launch_bounds__(STHREADS) void sample_kernel(SampleArgs a) {
     // The largest bit pattern c in [lo, hi) for which enough({sum, count} of the entries >= c) holds: it holds at lo
     // and not at hi.  `guess` is the first bound tried.  at_lo / at_hi: the totals there.
     auto search = [&](unsigned lo, unsigned hi, unsigned guess, SumCount at_lo, bool counts) {
-        auto enough = [&](SumCount t) { return counts ? t.n >= (float)a.top_k : t.s >= top_p; };
         SumCount at_hi = {0.f, 0.f};   // hi lies past the largest entry
         unsigned cand = guess;
         while (hi - lo > 1 && at_lo.n - at_hi.n > (float)LIST_MAX) {
             if (cand <= lo || cand >= hi) cand = lo + ((hi - lo) >> 1);
             const SumCount t = above(__uint_as_float(cand));
-            if (enough(t)) { lo = cand; at_lo = t; } else { hi = cand; at_hi = t; }
+            if (enough(t, top_p, counts ? a.top_k : -1)) { lo = cand; at_lo = t; } else { hi = cand; at_hi = t; }
             cand = 0;
         }
         if (hi - lo <= 1) return lo;
-        const SumCount past_hi = at_hi;
         // the entries in [lo, hi) to LDS, in thread order (zeros, padding among them, decide nothing and stay out)
         const float flo = __uint_as_float(max(lo, 1u)), fhi = __uint_as_float(hi);
         int mine = 0;
@@ -233,73 +309,7 @@ __global__ __launch_bounds__(STHREADS) void sample_kernel(SampleArgs a) {
         for (int e = 0; e < EMAX; ++e)
             if (p[e] >= flo2 && p[e] < fhi2) list[min(at++, LIST_MAX - 1)] = p[e];
         __syncthreads();
-        float left = (float)n;   // entries still between the bounds
-        while (hi - lo > 1 && left > 64.f) {
-            const unsigned step = (hi - lo) / (SWAVES + 1) + 1;
-            const unsigned c = lo + step * (wave + 1);
-            SumCount t = at_hi;      // the totals at hi and past it
-            if (c < hi) {
-                const float fc = __uint_as_float(c);
-                float sc = 0.f, k = 0.f;
-                for (int i = lane; i < n; i += 64) {
-                    const float v = list[i];
-                    if (v >= fc) { sc += v; k += 1.f; }
-                }
-                t.s = past_hi.s + wave_sum(sc);
-                t.n = past_hi.n + wave_sum(k);
-            }
-            f32x4 *buf = red[turn];
-            turn ^= 1;
-            if (lane == 0) {
-                ((float *)buf)[2 * wave] = t.s;
-                ((float *)buf)[2 * wave + 1] = t.n;
-            }
-            __syncthreads();
-            int good = 0;            // the bounds that hold are a leading run up to rounding: take the largest
-            SumCount above_good = at_hi;
-#pragma unroll
-            for (int w = SWAVES - 1; w >= 0; --w) {
-                const SumCount q = {((float *)buf)[2 * w], ((float *)buf)[2 * w + 1]};
-                if (good == 0) {
-                    if (lo + step * (w + 1) < hi && enough(q)) { good = w + 1; at_lo = q; }
-                    else above_good = q;
-                }
-            }
-            hi = min(hi, lo + step * (good + 1));
-            lo = lo + step * good;
-            at_hi = above_good;
-            left = at_lo.n - at_hi.n;
-        }
-        if (hi - lo <= 1) return lo;
-        // at most 64 are left: one to a lane, in list order; the largest of them at which the condition holds is the answer
-        {
-            const float l1 = __uint_as_float(max(lo, 1u)), h1 = __uint_as_float(hi);
-            if (wave == 0) {
-                int at64 = 0;
-                for (int i0 = 0; i0 < n; i0 += 64) {
-                    const float v = i0 + lane < n ? list[i0 + lane] : 0.f;
-                    const bool in = v >= l1 && v < h1;
-                    const unsigned long long m = __ballot(in);
-                    if (in) tail[min(at64 + (int)__popcll(m & ((1ull << lane) - 1)), 63)] = v;
-                    at64 += (int)__popcll(m);
-                }
-                if (lane >= at64) tail[lane] = 0.f;
-            }
-            __syncthreads();
-            const float mine64 = tail[lane];
-            SumCount t = at_hi;
-#pragma unroll 2
-            for (int i = 0; i < 64; i += 4) {
-                const f32x4 v = *(const f32x4 *)&tail[i];
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    if (v[e] >= mine64) { t.s += v[e]; t.n += v[e] > 0.f ? 1.f : 0.f; }
-            }
-            const float best = wave_max(mine64 > 0.f && enough(t) ? mine64 : 0.f);
-            __syncthreads();         // the lists may be written again
-            if (best > 0.f) lo = __float_as_uint(best);
-        }
-        return lo;
+        return search_list(list, n, lo, hi, at_lo, at_hi, top_p, counts ? a.top_k : -1, tail, red, turn);
     };
 
     // ---- nucleus cut (utils.py:55-58, 66-69): temperature 0 means top_p 0
@@ -425,6 +435,307 @@ __global__ __launch_bounds__(STHREADS) void sample_kernel(SampleArgs a) {
     }
 }
 
+template <int SROWS, bool POW>
+__global__ __launch_bounds__(STHREADS) void sample_kernel(SampleArgs a) { sample_one_workgroup<SROWS, POW>(a); }
+
+// ---- the same draw over the chip -------------------------------------------------------------------------------
+// One workgroup issues every instruction of a pass over 65536 entries 256 times per SIMD, half a microsecond each, and the
+// exponential alone takes twenty.  With scratch from the caller the passes over the vocabulary run on one workgroup per
+// SEG entries, in three launches:
+//   adjust: bans and penalties, the segment's largest logit and sum of exponentials;
+//   probs:  the probabilities (every workgroup forms the total), for BOUNDS bounds half an octave apart below the largest
+//           one the segment's sum and count of the entries that reach it, and the list, in index order, of the entries that
+//           the nucleus can need: those below (1 - top_p) / 2 V cannot add up to what may be left out;
+//   draw:   every workgroup finds the cut for itself -- the bounds leave half an octave, whose entries are searched as in
+//           the kernel above -- and draws; it writes the filtered probabilities and the occurrence counts of its segment.
+// Sums are added in a fixed order throughout.  Where the lists are too long for LDS, or the total is no positive number, the
+// last launch's first workgroup does the whole draw as the kernel above.
+// Bound by the latency of the three launches.  Measured as above, V = 65536: @@ us a draw, 39 with one workgroup.
+constexpr int SEG = 1024, SEGS_MAX = 64, BOUNDS = 32, CAND_MAX = 32768;
+constexpr int PART = 2 * BOUNDS + 2;          // per segment: sums and counts at the bounds, sum of all, length of the list
+
+struct SampleWs {
+    float *p;          // [segments][SEG] adjusted logits, then probabilities
+    float *list;       // [segments][SEG] candidates in index order
+    uint16_t *idx;     // [segments][SEG] their places in the segment
+    float *soft;       // [segments][2] largest logit, sum of exponentials
+    float *part;       // [segments][PART]
+};
+
+__global__ __launch_bounds__(256) void sample_adjust_kernel(SampleArgs a, SampleWs ws) {
+    __shared__ float red[8];
+    const int V = a.V, i0 = blockIdx.x * SEG + 4 * threadIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    f32x4 x;
+    uint32_t flag = 0;
+    if (i0 + 3 < V && (((uintptr_t)a.logits) & 15) == 0 && (((uintptr_t)a.seen) & 3) == 0) {
+        x = *(const f32x4 *)(a.logits + i0);
+        if (a.seen) flag = *(const uint32_t *)(a.seen + i0);
+    } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            x[e] = i0 + e < V ? a.logits[i0 + e] : -INFINITY;
+            if (a.seen && i0 + e < V) flag |= (uint32_t)a.seen[i0 + e] << (8 * e);
+        }
+    }
+    if (flag) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            if ((flag >> (8 * e)) & 0xff) x[e] -= a.presence + a.occ[i0 + e] * a.frequency;
+    }
+    for (int b = 0; b < a.n_ban; ++b) {
+        const int k = a.ban[b] - i0;
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            if (e == k) x[e] = -INFINITY;
+    }
+    *(f32x4 *)(ws.p + i0) = x;
+    float m = wave_max(fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3])));
+    if (lane == 0) red[wave] = m;
+    __syncthreads();
+    m = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+    float s = 0.f;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) s += x[e] == -INFINITY ? 0.f : expf(x[e] - m);
+    s = wave_sum(s);
+    if (lane == 0) red[4 + wave] = s;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        ws.soft[2 * blockIdx.x] = m;
+        ws.soft[2 * blockIdx.x + 1] = (red[4] + red[5]) + (red[6] + red[7]);
+    }
+}
+
+// The largest logit and the sum of the exponentials from the segments'; every lane gets both.
+struct Soft { float mx, sum; };
+DEV Soft soft_total(const float *soft, int segs) {
+    const int lane = threadIdx.x & 63;
+    const float m = lane < segs ? soft[2 * lane] : -INFINITY, s = lane < segs ? soft[2 * lane + 1] : 0.f;
+    const float mx = wave_max(m);
+    return {mx, wave_sum(m == -INFINITY ? 0.f : s * expf(m - mx))};
+}
+DEV float bound_at(float pmax, int k) { return __uint_as_float(__float_as_uint(pmax) - ((unsigned)(k + 1) << 22)); }
+
+__global__ __launch_bounds__(256) void sample_probs_kernel(SampleArgs a, SampleWs ws) {
+    __shared__ float red[4][PART];
+    const int i0 = blockIdx.x * SEG + 4 * threadIdx.x, lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    f32x4 p = *(const f32x4 *)(ws.p + i0);
+    const Soft st = soft_total(ws.soft, gridDim.x);
+    const float inv = 1.f / st.sum;   // of the largest entry: its exponential is 1
+#pragma unroll
+    for (int e = 0; e < 4; ++e) p[e] = p[e] == -INFINITY ? 0.f : expf(p[e] - st.mx) * inv;
+    *(f32x4 *)(ws.p + i0) = p;
+    const float top_p = a.temperature == 0.f ? 0.f : a.top_p;
+    const float floor_ = top_p > 0.f ? 0.5f * (1.f - top_p) / (float)a.V : inv;
+    // sums and counts at the bounds: lane k keeps those of bound k
+    float mine_s = 0.f, mine_n = 0.f;
+#pragma unroll 4
+    for (int k = 0; k < BOUNDS; ++k) {
+        const float b = bound_at(inv, k);
+        float s = 0.f, n = 0.f;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const bool in = p[e] >= b;
+            s += in ? p[e] : 0.f;
+            n += (float)__popcll(__ballot(in));
+        }
+        s = wave_sum(s);
+        if (lane == k) { mine_s = s; mine_n = n; }
+    }
+    const float total = wave_sum((p[0] + p[1]) + (p[2] + p[3]));
+    unsigned long long in[4];
+    int before = 0, n_wave = 0;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        in[e] = __ballot(p[e] >= floor_);
+        before += (int)__popcll(in[e] & ((1ull << lane) - 1));
+        n_wave += (int)__popcll(in[e]);
+    }
+    if (lane < BOUNDS) { red[wave][lane] = mine_s; red[wave][BOUNDS + lane] = mine_n; }
+    if (lane == 0) { red[wave][2 * BOUNDS] = total; red[wave][2 * BOUNDS + 1] = (float)n_wave; }
+    __syncthreads();
+    int at = blockIdx.x * SEG + before;
+#pragma unroll
+    for (int w = 0; w < 3; ++w)
+        if (w < wave) at += (int)red[w][2 * BOUNDS + 1];
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+        if ((in[e] >> lane) & 1) {
+            ws.list[at] = p[e];
+            ws.idx[at++] = (uint16_t)(4 * threadIdx.x + e);
+        }
+    if (threadIdx.x < PART)
+        ws.part[blockIdx.x * PART + threadIdx.x] =
+            (red[0][threadIdx.x] + red[1][threadIdx.x]) + (red[2][threadIdx.x] + red[3][threadIdx.x]);
+}
+
+template <int SROWS, bool POW>
+__global__ __launch_bounds__(STHREADS) void sample_draw_kernel(SampleArgs a, SampleWs ws) {
+    extern __shared__ __align__(16) float cand[];          // the candidates of all segments, in index order
+    __shared__ f32x4 red[2][SWAVES / 2];
+    __shared__ float list[LIST_MAX], tail[64], cols[SWAVES][2 * BOUNDS], seg_sum[SEGS_MAX];
+    __shared__ int first[SEGS_MAX + 1], pick;
+    const int V = a.V, tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), segs = gridDim.x;
+    const int own = blockIdx.x * SEG + tid;                 // this thread's entry
+    const float p_own = ws.p[own];
+    const uint8_t seen_own = a.seen && own < V ? a.seen[own] : 0;
+    const float target_u = *a.u;
+    const float top_p = a.temperature == 0.f ? 0.f : a.top_p;
+    // ---- totals of the segments
+    {
+        float c = 0.f;
+#pragma unroll
+        for (int j = 0; j < SEGS_MAX / SWAVES; ++j) {
+            const int sg = wave * (SEGS_MAX / SWAVES) + j;
+            if (sg < segs) c += ws.part[sg * PART + lane];
+        }
+        cols[wave][lane] = c;
+    }
+    const Soft st = soft_total(ws.soft, segs);
+    const float pmax = 1.f / st.sum;
+    const float all = wave_sum(lane < segs ? ws.part[lane * PART + 2 * BOUNDS] : 0.f);
+    const float len = lane < segs ? ws.part[lane * PART + 2 * BOUNDS + 1] : 0.f, incl = wave_scan(len);
+    const int n = (int)__shfl(incl, 63, WAVE);
+    if (wave == 0) {
+        first[lane] = (int)(incl - len);
+        if (lane == 63) first[SEGS_MAX] = n;
+    }
+    __syncthreads();
+    if (!(st.sum > 0.f && st.sum < INFINITY) || n > CAND_MAX || (top_p > 0.f && !(all >= 0.5f + 0.5f * top_p))) {
+        if (blockIdx.x == 0) sample_one_workgroup<SROWS, POW>(a);
+        return;
+    }
+    // ---- the candidates to LDS: 16 threads a segment
+    const int sg = tid >> 4, r = tid & 15, at0 = first[sg], n_seg = first[sg + 1] - at0;
+    for (int i = 4 * r; i < n_seg; i += 64) {
+        const f32x4 v = *(const f32x4 *)(ws.list + sg * SEG + i);
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            if (i + e < n_seg) cand[at0 + i + e] = v[e];
+    }
+    // ---- which half octave holds the cut: lane k has the sum and the count at bound k
+    SumCount at_k = {0.f, 0.f};
+#pragma unroll
+    for (int w = 0; w < SWAVES; ++w) {
+        at_k.s += cols[w][lane & (BOUNDS - 1)];
+        at_k.n += cols[w][BOUNDS + (lane & (BOUNDS - 1))];
+    }
+    __syncthreads();
+    int turn = 0;
+    auto above = [&](float c) {
+        float sc = 0.f, k = 0.f;
+        for (int i = tid; i < n; i += STHREADS) {
+            const float v = cand[i];
+            if (v >= c) { sc += v; k += 1.f; }
+        }
+        return block_total(sc, k, red, turn);
+    };
+    float cut = pmax;   // as in the kernel above
+#pragma unroll 1
+    for (int counts = 0; counts < 2; ++counts) {
+        const int want = counts ? a.top_k : -1;
+        unsigned lo, hi = __float_as_uint(pmax) + 1;
+        SumCount at_lo, at_hi = {0.f, 0.f};
+        if (!counts) {
+            if (!(top_p > 0.f && all >= top_p)) continue;
+            lo = 0u;
+            at_lo = {all, (float)n};
+        } else {
+            if (!(a.top_k > 0 && a.top_k < V)) continue;
+            at_lo = above(cut);
+            if (!(at_lo.n > (float)a.top_k)) continue;
+            lo = __float_as_uint(cut);
+        }
+        const unsigned long long holds = __ballot(lane < BOUNDS && enough(at_k, top_p, want));
+        const int k = holds ? __builtin_ctzll(holds) : BOUNDS;
+        if (k < BOUNDS && __float_as_uint(bound_at(pmax, k)) > lo) {
+            lo = __float_as_uint(bound_at(pmax, k));
+            at_lo = {__shfl(at_k.s, k, WAVE), __shfl(at_k.n, k, WAVE)};
+        }
+        if (k > 0) {
+            hi = __float_as_uint(bound_at(pmax, k - 1));
+            at_hi = {__shfl(at_k.s, k - 1, WAVE), __shfl(at_k.n, k - 1, WAVE)};
+        }
+        while (hi - lo > 1 && at_lo.n - at_hi.n > (float)LIST_MAX) {
+            const unsigned c = lo + ((hi - lo) >> 1);
+            const SumCount t = above(__uint_as_float(c));
+            if (enough(t, top_p, want)) { lo = c; at_lo = t; } else { hi = c; at_hi = t; }
+        }
+        if (hi - lo > 1) {
+            // the entries of [lo, hi), in thread order
+            const float flo = __uint_as_float(max(lo, 1u)), fhi = __uint_as_float(hi);
+            int mine = 0;
+            for (int i = tid; i < n; i += STHREADS) mine += (cand[i] >= flo && cand[i] < fhi) ? 1 : 0;
+            const float upto = wave_scan((float)mine);
+            f32x4 *buf = red[turn];
+            turn ^= 1;
+            if (lane == 63) ((float *)buf)[wave] = upto;
+            __syncthreads();
+            float before = 0.f, sum = 0.f;
+#pragma unroll
+            for (int w = 0; w < SWAVES; ++w) {
+                const float v = ((float *)buf)[w];
+                before += w < wave ? v : 0.f;
+                sum += v;
+            }
+            int at = (int)(before + upto) - mine;
+            for (int i = tid; i < n; i += STHREADS) {
+                const float v = cand[i];
+                if (v >= flo && v < fhi) list[min(at++, LIST_MAX - 1)] = v;
+            }
+            __syncthreads();
+            lo = search_list(list, (int)sum, lo, hi, at_lo, at_hi, top_p, want, tail, red, turn);
+        }
+        cut = __uint_as_float(lo);
+    }
+    // ---- filter, temperature, sums of the segments
+    const float invt = 1.f / a.temperature;
+    auto kept = [&](float v) {
+        v = v >= cut && v > 0.f ? v : 0.f;
+        if (POW && v > 0.f) v = powf(v, invt);
+        return v;
+    };
+    {
+        float sum = 0.f;
+        for (int i = r; i < n_seg; i += 16) sum += kept(cand[at0 + i]);
+        sum = row16_sum(sum);
+        if (r == 0) seg_sum[sg] = sum;
+    }
+    if (a.probs && own < V) a.probs[own] = kept(p_own);
+    __syncthreads();
+    // ---- draw: first index whose running sum exceeds u * total; the last kept entry where rounding leaves none
+    if (wave == 0) {
+        const float mine = seg_sum[lane], upto = wave_scan(mine), target = target_u * __shfl(upto, 63, WAVE);
+        const unsigned long long hit = __ballot(mine > 0.f && upto > target), some = __ballot(mine > 0.f);
+        const int from = hit ? __builtin_ctzll(hit) : (some ? 63 - __builtin_clzll(some) : 0);
+        float run = __shfl(upto - mine, from, WAVE);
+        const int begin = first[from], end = first[from + 1];
+        int found = -1, last = 0;
+        for (int i0 = begin; i0 < end && found < 0; i0 += 64) {
+            const float v = i0 + lane < end ? kept(cand[i0 + lane]) : 0.f, up = run + wave_scan(v);
+            const unsigned long long over = __ballot(v > 0.f && up > target), any = __ballot(v > 0.f);
+            if (hit && over) found = i0 - begin + __builtin_ctzll(over);
+            if (any) last = i0 - begin + 63 - __builtin_clzll(any);
+            run = __shfl(up, 63, WAVE);
+        }
+        if (lane == 0) pick = some ? from * SEG + (int)ws.idx[from * SEG + (found >= 0 ? found : last)] : 0;
+    }
+    __syncthreads();
+    const int tok = pick;
+    if (blockIdx.x == 0 && tid == 0) *a.token = tok;
+    // ---- occurrence table: decay, then add the drawn token's weight
+    if (a.seen && own < V && (seen_own || own == tok)) {
+        const float w = own == tok ? (a.weight ? a.weight[tok] : 1.f) : 0.f;
+        float o = w;
+        if (seen_own) {
+            o = a.occ[own] * a.decay;
+            if (own == tok) o += w;
+        } else {
+            a.seen[own] = 1;
+        }
+        a.occ[own] = o;
+    }
+}
+
 }  // namespace
 
 // The temperature-0 draw without penalties or bans: the index of the largest logit, the lowest such index on
@@ -473,16 +784,26 @@ extern "C" int rwkv_greedy_token(const void *logits, int dtype, int64_t V, int32
     return RWKV_OK;
 }
 
-extern "C" int rwkv_sample_logits(const float *logits, int64_t V, float temperature, float top_p, int32_t top_k,
-                                  const int32_t *token_ban, int32_t n_ban, uint8_t *seen, float *occurrence,
-                                  const float *token_weight, float alpha_presence, float alpha_frequency,
-                                  float alpha_decay, const float *u, float *probs, int32_t *token, void *stream) {
+static int sample_args(SampleArgs &a, const float *logits, int64_t V, float temperature, float top_p, int32_t top_k,
+                       const int32_t *token_ban, int32_t n_ban, uint8_t *seen, float *occurrence, const float *token_weight,
+                       float alpha_presence, float alpha_frequency, float alpha_decay, const float *u, float *probs, int32_t *token) {
     if (!logits || !u || !token) return RWKV_E_NULL;
     if (V <= 0 || V > (int64_t)STHREADS * 4 * ROWS_MAX || n_ban < 0 || (n_ban > 0 && !token_ban)) return RWKV_E_SHAPE;
     if ((seen == nullptr) != (occurrence == nullptr)) return RWKV_E_NULL;
     if (!(temperature >= 0.f) || top_k < 0) return RWKV_E_SHAPE;
-    SampleArgs a{logits, (int)V, temperature, top_p, top_k, token_ban, n_ban, seen, occurrence, token_weight,
-                 alpha_presence, alpha_frequency, alpha_decay, u, probs, token};
+    a = SampleArgs{logits, (int)V, temperature, top_p, top_k, token_ban, n_ban, seen, occurrence, token_weight,
+                   alpha_presence, alpha_frequency, alpha_decay, u, probs, token};
+    return RWKV_OK;
+}
+
+extern "C" int rwkv_sample_logits(const float *logits, int64_t V, float temperature, float top_p, int32_t top_k,
+                                  const int32_t *token_ban, int32_t n_ban, uint8_t *seen, float *occurrence,
+                                  const float *token_weight, float alpha_presence, float alpha_frequency,
+                                  float alpha_decay, const float *u, float *probs, int32_t *token, void *stream) {
+    SampleArgs a;
+    const int rc = sample_args(a, logits, V, temperature, top_p, top_k, token_ban, n_ban, seen, occurrence, token_weight,
+                               alpha_presence, alpha_frequency, alpha_decay, u, probs, token);
+    if (rc) return rc;
     // group rows: 4 (small vocabularies), 13 (the 50277-entry ones) or 16
     const bool pow = temperature != 0.f && temperature != 1.f;
 #define RWKV_SAMPLE(ROWS)                                                                                                      \
@@ -494,6 +815,66 @@ extern "C" int rwkv_sample_logits(const float *logits, int64_t V, float temperat
     else if (V <= 13 * 4 * STHREADS) RWKV_SAMPLE(13);
     else RWKV_SAMPLE(16);
 #undef RWKV_SAMPLE
+    RWKV_LAUNCH_CHECK();
+    return RWKV_OK;
+}
+
+static size_t sample_ws(SampleWs &ws, void *base, int64_t V) {
+    const size_t segs = (size_t)((V + SEG - 1) / SEG), n = segs * SEG;
+    ws.p = (float *)base;
+    ws.list = ws.p + n;
+    ws.part = ws.list + n;
+    ws.soft = ws.part + segs * PART;
+    ws.idx = (uint16_t *)(ws.soft + 2 * segs);
+    return (2 * n + segs * (PART + 2)) * sizeof(float) + n * sizeof(uint16_t);
+}
+
+extern "C" size_t rwkv_sample_workspace(int64_t V) {
+    SampleWs ws;
+    return V > 0 && V <= SEG * SEGS_MAX ? sample_ws(ws, nullptr, V) : 0;
+}
+
+extern "C" int rwkv_sample_logits_ws(const float *logits, int64_t V, float temperature, float top_p, int32_t top_k,
+                                     const int32_t *token_ban, int32_t n_ban, uint8_t *seen, float *occurrence,
+                                     const float *token_weight, float alpha_presence, float alpha_frequency, float alpha_decay,
+                                     const float *u, float *probs, int32_t *token, void *workspace, size_t workspace_bytes,
+                                     void *stream) {
+    SampleArgs a;
+    const int rc = sample_args(a, logits, V, temperature, top_p, top_k, token_ban, n_ban, seen, occurrence, token_weight,
+                               alpha_presence, alpha_frequency, alpha_decay, u, probs, token);
+    if (rc) return rc;
+    if (!workspace) return RWKV_E_NULL;
+    if (workspace_bytes < rwkv_sample_workspace(V) || !aligned16(workspace)) return RWKV_E_WORKSPACE;
+    // One workgroup: vocabularies that are four entries a thread there, and cuts that leave (almost) everything.
+    if (V <= 4 * 4 * STHREADS || (temperature != 0.f && !(top_p <= 0.999f)))
+        return rwkv_sample_logits(logits, V, temperature, top_p, top_k, token_ban, n_ban, seen, occurrence, token_weight, alpha_presence,
+                                  alpha_frequency, alpha_decay, u, probs, token, stream);
+    hipStream_t st = (hipStream_t)stream;
+    SampleWs ws;
+    sample_ws(ws, workspace, V);
+    const dim3 grid((unsigned)((V + SEG - 1) / SEG));
+    constexpr size_t lds = CAND_MAX * sizeof(float);
+    const bool pow = temperature != 0.f && temperature != 1.f;
+    static PerDeviceOnce once;
+    bool *attr_done = once.slot();
+    if (!attr_done || !*attr_done) {
+        for (const void *k : {(const void *)sample_draw_kernel<13, true>, (const void *)sample_draw_kernel<13, false>,
+                              (const void *)sample_draw_kernel<16, true>, (const void *)sample_draw_kernel<16, false>}) {
+            const hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+            if (e != hipSuccess) return (int)e;
+        }
+        if (attr_done) *attr_done = true;
+    }
+    hipLaunchKernelGGL(sample_adjust_kernel, grid, dim3(256), 0, st, a, ws);
+    hipLaunchKernelGGL(sample_probs_kernel, grid, dim3(256), 0, st, a, ws);
+#define RWKV_DRAW(ROWS)                                                                                            \
+    do {                                                                                                           \
+        if (pow) hipLaunchKernelGGL((sample_draw_kernel<ROWS, true>), grid, dim3(STHREADS), lds, st, a, ws);       \
+        else hipLaunchKernelGGL((sample_draw_kernel<ROWS, false>), grid, dim3(STHREADS), lds, st, a, ws);          \
+    } while (0)
+    if (V <= 13 * 4 * STHREADS) RWKV_DRAW(13);
+    else RWKV_DRAW(16);
+#undef RWKV_DRAW
     RWKV_LAUNCH_CHECK();
     return RWKV_OK;
 }

@@ -51,6 +51,8 @@ class Sampler:
         self.probs = torch.empty(self.V, dtype=torch.float32, device=self.device)
         self.token = torch.zeros(1, dtype=torch.int32, device=self.device)
         self.u = torch.zeros(1, dtype=torch.float32, device=self.device)
+        # 0 bytes for a vocabulary the kernels do not take: sample() refuses it
+        self.ws = torch.empty(self.L.rwkv_sample_workspace(self.V), dtype=torch.uint8, device=self.device)
         self.gen = torch.Generator(device=self.device)
         if seed is not None:
             self.gen.manual_seed(int(seed))
@@ -79,13 +81,13 @@ class Sampler:
             self.u.fill_(float(u))
         seen = self.seen.data_ptr() if penalties else None
         occ = self.occurrence.data_ptr() if penalties else None
-        rc = self.L.rwkv_sample_logits(
+        rc = self.L.rwkv_sample_logits_ws(
             logits.data_ptr(), self.V, float(temperature), float(top_p), int(top_k),
             self.ban.data_ptr() if self.ban is not None else None, 0 if self.ban is None else self.ban.numel(),
             seen, occ, self.weight.data_ptr() if (self.weight is not None and penalties) else None,
             float(alpha_presence), float(alpha_frequency), float(alpha_decay),
-            unif.data_ptr(), self.probs.data_ptr(), self.token.data_ptr(), _stream())
-        _lib.check(rc, "rwkv_sample_logits")
+            unif.data_ptr(), self.probs.data_ptr(), self.token.data_ptr(), self.ws.data_ptr(), self.ws.numel(), _stream())
+        _lib.check(rc, "rwkv_sample_logits_ws")
         return self.token
 
 

@@ -187,6 +187,13 @@ int rwkv_sample_logits(const float *logits, int64_t V, float temperature, float 
                        const int32_t *token_ban, int32_t n_ban, uint8_t *seen, float *occurrence,
                        const float *token_weight, float alpha_presence, float alpha_frequency, float alpha_decay,
                        const float *u, float *probs, int32_t *token, void *stream);
+/* The same draw with scratch of rwkv_sample_workspace(V) bytes (16-byte aligned, the caller's until the launches have
+   run): the passes over the vocabulary on many workgroups. */
+size_t rwkv_sample_workspace(int64_t V);
+int rwkv_sample_logits_ws(const float *logits, int64_t V, float temperature, float top_p, int32_t top_k,
+                          const int32_t *token_ban, int32_t n_ban, uint8_t *seen, float *occurrence,
+                          const float *token_weight, float alpha_presence, float alpha_frequency, float alpha_decay,
+                          const float *u, float *probs, int32_t *token, void *workspace, size_t workspace_bytes, void *stream);
 
 /* The temperature-0 case of the same step without bans or penalties (rwkv/utils.py:56-58: top_p = 0 keeps the
  * largest probability alone; what a greedy caller writes as logits.argmax()): token <- the index of the

@@ -263,3 +263,55 @@ def test_uniform_number_from_a_device_tensor():
         for u in (grid[i, j], grid[i:i + 1, j:j + 1], grid[i, j].double(), grid[i, j].cpu()):
             assert draws(u) == want, (i, j, u)
     assert len({draws(v) for v in grid.flatten()}) > 5 and torch.equal(grid, before)
+
+
+@pytest.mark.parametrize("V", [16388, 20001, 50277, 65536])
+@pytest.mark.parametrize("scale", [0.3, 3.0, 30.0])
+def test_draw_over_the_chip_against_one_workgroup(V, scale):
+    """Vocabularies of more than 16384 entries: the three launches against the one-workgroup kernel on the same operands --
+    ragged segments, flat logits (lists too long for LDS), peaked ones (every bound above the cut), masks of -inf and of the
+    type's lowest value, bans, penalties, ties, cuts by sum and by count, temperatures.  The probabilities differ by the
+    order of the sum they are divided by and two roundings (2^-23 each; a power by up to 1 / T times that), the rest is equal
+    where no running sum lies within that of the cut or of the drawn number."""
+    from chatrwkv_amd import lib
+    from chatrwkv_amd.sampling import Sampler
+    L = lib.load()
+    rng = np.random.Generator(np.random.PCG64([V, int(10 * scale)]))
+    x = (rng.standard_normal(V) * scale).astype(np.float32)
+    x[rng.integers(0, V, 50)] = -np.inf
+    x[rng.integers(0, V, 50)] = np.finfo(np.float32).min
+    x[rng.integers(0, V, 200)] = np.float32(x.max() - 1)          # ties
+    xt = torch.from_numpy(x).to(DEV)
+    for top_p, top_k, temp in [(0.7, 0, 1.0), (0.05, 0, 1.0), (0.95, 0, 0.7), (0.999, 0, 1.0), (0.9, 40, 1.0), (0.95, 2000, 1.3),
+                               (0.85, 1, 1.0), (0.85, 0, 0.0), (0.0, 3, 1.0), (1.0, 100, 1.0), (0.5, 150, 1.0)]:
+        s = Sampler(V, device=DEV, token_ban=[0, V - 1, 777])
+        seen = rng.integers(0, V, 40)
+        s.seen[torch.from_numpy(seen).to(DEV)] = 1
+        s.occurrence[torch.from_numpy(seen).to(DEV)] = 2.5
+        probs, token = torch.empty_like(s.probs), torch.zeros_like(s.token)
+        tables = s.seen.clone(), s.occurrence.clone()
+        u = torch.tensor([float(rng.random())], device=DEV)
+        s.sample(xt, temp, top_p, top_k, 0.2, 0.3, 0.996, u=u)
+        lib.check(L.rwkv_sample_logits(xt.data_ptr(), V, temp, top_p, top_k, s.ban.data_ptr(), 3, tables[0].data_ptr(), tables[1].data_ptr(),
+                                       None, 0.2, 0.3, 0.996, u.data_ptr(), probs.data_ptr(), token.data_ptr(),
+                                       torch.cuda.current_stream().cuda_stream), "rwkv_sample_logits")
+        got, ref = s.probs.cpu().numpy().astype(np.float64), probs.cpu().numpy().astype(np.float64)
+        assert abs(int((got > 0).sum()) - int((ref > 0).sum())) <= (0 if top_k or top_p in (0.0, 1.0) else 1), (top_p, top_k, temp)
+        both = (got > 0) & (ref > 0)
+        np.testing.assert_allclose(got[both], ref[both], rtol=4e-6, atol=1e-30)
+        cdf = np.cumsum(ref)
+        near = np.abs(cdf / cdf[-1] - float(u)).min()
+        if near > 1e-5 and np.array_equal(got > 0, ref > 0):
+            assert int(s.token) == int(token), (top_p, top_k, temp)
+            assert torch.equal(s.seen, tables[0]) and torch.equal(s.occurrence, tables[1])
+
+
+def test_draw_without_a_finite_total():
+    """Logits that are NaN, infinite or all masked: the three launches leave these to the one-workgroup kernel."""
+    from chatrwkv_amd.sampling import Sampler
+    V = 50277
+    for fill in (float("nan"), float("inf"), float("-inf")):
+        x = torch.zeros(V, device=DEV) if fill != float("-inf") else torch.full((V,), fill, device=DEV)
+        x[5] = fill
+        s = Sampler(V, device=DEV)
+        assert 0 <= int(s.sample(x, 1.0, 0.7, 0, 0.2, 0.2, 0.996, u=0.5)) < V
