@@ -74,16 +74,21 @@ DEV float block_max(float v, f32x4 (&red)[2][SWAVES / 2], int &turn) {
     return m;
 }
 
-// inclusive sum over the lanes of a wave
+// inclusive sum over the lanes of a wave: four steps within the rows of 16 lanes, the last lanes of the rows before (DPP)
+template <int CTRL, int ROWS>
+DEV float dpp_rows(float v) {   // 0 in the rows that are not written
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, ROWS, 0xf, true));
+}
 DEV float wave_scan(float v) {
-    const int lane = threadIdx.x & 63;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        const float up = __shfl_up(v, o, WAVE);
-        if (lane >= o) v += up;
-    }
+    v += dpp_rows<0x111, 0xf>(v);   // row_shr 1, 2, 4, 8
+    v += dpp_rows<0x112, 0xf>(v);
+    v += dpp_rows<0x114, 0xf>(v);
+    v += dpp_rows<0x118, 0xf>(v);
+    v += dpp_rows<0x142, 0xa>(v);   // row_bcast 15 into rows 1 and 3
+    v += dpp_rows<0x143, 0xc>(v);   // row_bcast 31 into rows 2 and 3
     return v;
 }
+DEV float last_lane(float v) { return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 63)); }
 
 // Does a bound hold whose entries add up to t?  The nucleus cut asks for a sum, the k-th largest value (top_k >= 0) for a count.
 DEV bool enough(SumCount t, float top_p, int top_k) { return top_k >= 0 ? t.n >= (float)top_k : t.s >= top_p; }
@@ -448,10 +453,12 @@ __global__ __launch_bounds__(STHREADS) void sample_kernel(SampleArgs a) { sample
 //           the nucleus can need: those below (1 - top_p) / 2 V cannot add up to what may be left out;
 //   draw:   every workgroup finds the cut for itself -- the bounds leave half an octave, whose entries are searched as in
 //           the kernel above -- and draws; it writes the filtered probabilities and the occurrence counts of its segment.
-// Sums are added in a fixed order throughout.  Where the lists are too long for LDS, or the total is no positive number, the
-// last launch's first workgroup does the whole draw as the kernel above.
-// Bound by the latency of the three launches.  Measured as above, V = 65536: @@ us a draw, 39 with one workgroup.
-constexpr int SEG = 1024, SEGS_MAX = 64, BOUNDS = 32, CAND_MAX = 32768;
+// Sums are added in a fixed order throughout.  Where the total is no positive number the last launch's first workgroup does
+// the whole draw as the kernel above.
+// Bound by the latency of the three launches.  Measured as above, V = 65536: 21.5 us a draw (2.7 + 4.3 + 12.7 and the gaps), 39 with one
+// workgroup; with the lists in LDS and the bracket searched by search_list 25.8, 5 us of it in the search.
+constexpr int SEG = 1024, SEGS_MAX = 64, BOUNDS = 32;
+constexpr int FEW = 256;                      // entries of a bracket that are compared with each other at once
 constexpr int PART = 2 * BOUNDS + 2;          // per segment: sums and counts at the bounds, sum of all, length of the list
 
 struct SampleWs {
@@ -516,7 +523,10 @@ DEV Soft soft_total(const float *soft, int segs) {
 DEV float bound_at(float pmax, int k) { return __uint_as_float(__float_as_uint(pmax) - ((unsigned)(k + 1) << 22)); }
 
 __global__ __launch_bounds__(256) void sample_probs_kernel(SampleArgs a, SampleWs ws) {
-    __shared__ float red[4][PART];
+    __shared__ unsigned long long bin_s[BOUNDS];   // sums times 2^40: the same in any order
+    __shared__ unsigned bin_n[BOUNDS];
+    __shared__ float red[4][2];
+    if (threadIdx.x < BOUNDS) { bin_s[threadIdx.x] = 0; bin_n[threadIdx.x] = 0; }
     const int i0 = blockIdx.x * SEG + 4 * threadIdx.x, lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     f32x4 p = *(const f32x4 *)(ws.p + i0);
     const Soft st = soft_total(ws.soft, gridDim.x);
@@ -526,20 +536,15 @@ __global__ __launch_bounds__(256) void sample_probs_kernel(SampleArgs a, SampleW
     *(f32x4 *)(ws.p + i0) = p;
     const float top_p = a.temperature == 0.f ? 0.f : a.top_p;
     const float floor_ = top_p > 0.f ? 0.5f * (1.f - top_p) / (float)a.V : inv;
-    // sums and counts at the bounds: lane k keeps those of bound k
-    float mine_s = 0.f, mine_n = 0.f;
-#pragma unroll 4
-    for (int k = 0; k < BOUNDS; ++k) {
-        const float b = bound_at(inv, k);
-        float s = 0.f, n = 0.f;
+    __syncthreads();
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const bool in = p[e] >= b;
-            s += in ? p[e] : 0.f;
-            n += (float)__popcll(__ballot(in));
+    for (int e = 0; e < 4; ++e) {
+        const unsigned k = (__float_as_uint(inv) - __float_as_uint(p[e])) >> 22;   // the first bound that the entry reaches is k or k - 1
+        const unsigned bin = k < BOUNDS + 1 ? (k > 0 && p[e] >= bound_at(inv, k - 1) ? k - 1 : k) : BOUNDS;
+        if (bin < BOUNDS) {
+            atomicAdd(&bin_s[bin], (unsigned long long)(p[e] * 1099511627776.f));
+            atomicAdd(&bin_n[bin], 1u);
         }
-        s = wave_sum(s);
-        if (lane == k) { mine_s = s; mine_n = n; }
     }
     const float total = wave_sum((p[0] + p[1]) + (p[2] + p[3]));
     unsigned long long in[4];
@@ -550,36 +555,53 @@ __global__ __launch_bounds__(256) void sample_probs_kernel(SampleArgs a, SampleW
         before += (int)__popcll(in[e] & ((1ull << lane) - 1));
         n_wave += (int)__popcll(in[e]);
     }
-    if (lane < BOUNDS) { red[wave][lane] = mine_s; red[wave][BOUNDS + lane] = mine_n; }
-    if (lane == 0) { red[wave][2 * BOUNDS] = total; red[wave][2 * BOUNDS + 1] = (float)n_wave; }
+    if (lane == 0) { red[wave][0] = total; red[wave][1] = (float)n_wave; }
     __syncthreads();
     int at = blockIdx.x * SEG + before;
 #pragma unroll
     for (int w = 0; w < 3; ++w)
-        if (w < wave) at += (int)red[w][2 * BOUNDS + 1];
+        if (w < wave) at += (int)red[w][1];
 #pragma unroll
     for (int e = 0; e < 4; ++e)
         if ((in[e] >> lane) & 1) {
             ws.list[at] = p[e];
             ws.idx[at++] = (uint16_t)(4 * threadIdx.x + e);
         }
-    if (threadIdx.x < PART)
-        ws.part[blockIdx.x * PART + threadIdx.x] =
-            (red[0][threadIdx.x] + red[1][threadIdx.x]) + (red[2][threadIdx.x] + red[3][threadIdx.x]);
+    float *part = ws.part + blockIdx.x * PART;
+    if (threadIdx.x < 2) part[2 * BOUNDS + threadIdx.x] = (red[0][threadIdx.x] + red[1][threadIdx.x]) + (red[2][threadIdx.x] + red[3][threadIdx.x]);
+    if (wave == 1 && lane < BOUNDS) {   // an entry of bin k reaches the bounds from k on
+        unsigned long long sum = 0;
+        unsigned n = 0;
+#pragma unroll
+        for (int k = 0; k < BOUNDS; ++k) {
+            sum += k <= lane ? bin_s[k] : 0;
+            n += k <= lane ? bin_n[k] : 0;
+        }
+        part[lane] = (float)sum * 0x1p-40f;
+        part[BOUNDS + lane] = (float)n;
+    }
 }
 
 template <int SROWS, bool POW>
 __global__ __launch_bounds__(STHREADS) void sample_draw_kernel(SampleArgs a, SampleWs ws) {
-    extern __shared__ __align__(16) float cand[];          // the candidates of all segments, in index order
     __shared__ f32x4 red[2][SWAVES / 2];
-    __shared__ float list[LIST_MAX], tail[64], cols[SWAVES][2 * BOUNDS], seg_sum[SEGS_MAX];
-    __shared__ int first[SEGS_MAX + 1], pick;
+    __shared__ float list[LIST_MAX], tail[64], seg_sum[SEGS_MAX];
+    __shared__ __align__(16) float cols[2 * BOUNDS][SWAVES + 4], few[FEW], sorted[FEW];
+    __shared__ int pick, n_few[2];
     const int V = a.V, tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), segs = gridDim.x;
     const int own = blockIdx.x * SEG + tid;                 // this thread's entry
     const float p_own = ws.p[own];
     const uint8_t seen_own = a.seen && own < V ? a.seen[own] : 0;
     const float target_u = *a.u;
     const float top_p = a.temperature == 0.f ? 0.f : a.top_p;
+    // 16 threads a segment hold its list: thread r the entries 64 j + 4 r .. + 3.  The first rounds are requested before the
+    // lengths are known
+    constexpr int EARLY = 4;
+    const int sg = tid >> 4, r = tid & 15;
+    f32x4 v[SEG / 64];
+#pragma unroll
+    for (int j = 0; j < EARLY; ++j) v[j] = *(const f32x4 *)(ws.list + min(sg, segs - 1) * SEG + 64 * j + 4 * r);
+    if (tid < 2) n_few[tid] = 0;
     // ---- totals of the segments
     {
         float c = 0.f;
@@ -588,46 +610,55 @@ __global__ __launch_bounds__(STHREADS) void sample_draw_kernel(SampleArgs a, Sam
             const int sg = wave * (SEGS_MAX / SWAVES) + j;
             if (sg < segs) c += ws.part[sg * PART + lane];
         }
-        cols[wave][lane] = c;
+        cols[lane][wave] = c;
     }
     const Soft st = soft_total(ws.soft, segs);
     const float pmax = 1.f / st.sum;
     const float all = wave_sum(lane < segs ? ws.part[lane * PART + 2 * BOUNDS] : 0.f);
-    const float len = lane < segs ? ws.part[lane * PART + 2 * BOUNDS + 1] : 0.f, incl = wave_scan(len);
-    const int n = (int)__shfl(incl, 63, WAVE);
-    if (wave == 0) {
-        first[lane] = (int)(incl - len);
-        if (lane == 63) first[SEGS_MAX] = n;
-    }
-    __syncthreads();
-    if (!(st.sum > 0.f && st.sum < INFINITY) || n > CAND_MAX || (top_p > 0.f && !(all >= 0.5f + 0.5f * top_p))) {
+    if (!(st.sum > 0.f && st.sum < INFINITY) || (top_p > 0.f && !(all >= 0.5f + 0.5f * top_p))) {
         if (blockIdx.x == 0) sample_one_workgroup<SROWS, POW>(a);
         return;
     }
-    // ---- the candidates to LDS: 16 threads a segment
-    const int sg = tid >> 4, r = tid & 15, at0 = first[sg], n_seg = first[sg + 1] - at0;
-    for (int i = 4 * r; i < n_seg; i += 64) {
-        const f32x4 v = *(const f32x4 *)(ws.list + sg * SEG + i);
+    const float len = lane < segs ? ws.part[lane * PART + 2 * BOUNDS + 1] : 0.f;
+    const float n = wave_sum(len);                          // candidates
+    const int n_seg = (int)__shfl(len, sg, WAVE), rounds = ((int)wave_max(len) + 63) >> 6;   // rounds: those that any segment has
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
-            if (i + e < n_seg) cand[at0 + i + e] = v[e];
-    }
+    for (int j = EARLY; j < SEG / 64; ++j)
+        if (j < rounds) v[j] = *(const f32x4 *)(ws.list + min(sg, segs - 1) * SEG + 64 * j + 4 * r);
+#pragma unroll
+    for (int j = 0; j < SEG / 64; ++j)
+        if (j < rounds) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[j][e] = 64 * j + 4 * r + e < n_seg ? v[j][e] : 0.f;
+        }
+    __syncthreads();
+    // calls f for every candidate that this thread holds (zeros fill the last round)
+    auto each = [&](auto f) {
+#pragma unroll
+        for (int j = 0; j < SEG / 64; ++j)
+            if (j < rounds) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) f(v[j][e]);
+            }
+    };
     // ---- which half octave holds the cut: lane k has the sum and the count at bound k
     SumCount at_k = {0.f, 0.f};
 #pragma unroll
-    for (int w = 0; w < SWAVES; ++w) {
-        at_k.s += cols[w][lane & (BOUNDS - 1)];
-        at_k.n += cols[w][BOUNDS + (lane & (BOUNDS - 1))];
+    for (int w = 0; w < SWAVES; w += 4) {
+        const f32x4 x = *(const f32x4 *)&cols[lane & (BOUNDS - 1)][w], y = *(const f32x4 *)&cols[BOUNDS + (lane & (BOUNDS - 1))][w];
+        at_k.s += (x[0] + x[1]) + (x[2] + x[3]);
+        at_k.n += (y[0] + y[1]) + (y[2] + y[3]);
     }
-    __syncthreads();
     int turn = 0;
-    auto above = [&](float c) {
-        float sc = 0.f, k = 0.f;
-        for (int i = tid; i < n; i += STHREADS) {
-            const float v = cand[i];
-            if (v >= c) { sc += v; k += 1.f; }
-        }
-        return block_total(sc, k, red, turn);
+    auto above = [&](float c) {   // c > 0
+        float sc = 0.f;
+        unsigned k = 0;
+        each([&](float x) {
+            const bool in = x >= c;
+            sc += in ? x : 0.f;
+            k += in ? 1u : 0u;
+        });
+        return block_total(sc, (float)k, red, turn);
     };
     float cut = pmax;   // as in the kernel above
 #pragma unroll 1
@@ -638,7 +669,7 @@ __global__ __launch_bounds__(STHREADS) void sample_draw_kernel(SampleArgs a, Sam
         if (!counts) {
             if (!(top_p > 0.f && all >= top_p)) continue;
             lo = 0u;
-            at_lo = {all, (float)n};
+            at_lo = {all, n};
         } else {
             if (!(a.top_k > 0 && a.top_k < V)) continue;
             at_lo = above(cut);
@@ -660,11 +691,47 @@ __global__ __launch_bounds__(STHREADS) void sample_draw_kernel(SampleArgs a, Sam
             const SumCount t = above(__uint_as_float(c));
             if (enough(t, top_p, want)) { lo = c; at_lo = t; } else { hi = c; at_hi = t; }
         }
-        if (hi - lo > 1) {
-            // the entries of [lo, hi), in thread order
-            const float flo = __uint_as_float(max(lo, 1u)), fhi = __uint_as_float(hi);
+        const float flo = __uint_as_float(max(lo, 1u)), fhi = __uint_as_float(hi);
+        if (hi - lo > 1 && at_lo.n - at_hi.n <= (float)FEW) {
+            // in any order at first
+            each([&](float x) {
+                if (x >= flo && x < fhi) few[min(atomicAdd(&n_few[counts], 1), FEW - 1)] = x;
+            });
+            __syncthreads();
+            // sorted by counting the larger ones (four threads an entry), then added from the largest down
+            const int m = min(n_few[counts], FEW), own_few = tid >> 2, q4 = tid & 3;
+            if (16 * wave < m) {
+                const float x = few[own_few];
+                int rank = 0;
+                for (int i = 4 * q4; i < m; i += 16) {
+                    const f32x4 y = *(const f32x4 *)&few[i];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) rank += (i + e < m && (y[e] > x || (y[e] == x && i + e < own_few))) ? 1 : 0;
+                }
+                rank += __builtin_amdgcn_update_dpp(0, rank, 0xB1, 0xf, 0xf, true);
+                rank += __builtin_amdgcn_update_dpp(0, rank, 0x4E, 0xf, 0xf, true);
+                if (q4 == 0 && own_few < m) sorted[rank] = x;
+            }
+            __syncthreads();
+            const f32x4 y = *(const f32x4 *)&sorted[4 * lane];
+            float in4[4], four = 0.f;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                in4[e] = 4 * lane + e < m ? y[e] : 0.f;
+                four += in4[e];
+            }
+            float sum = at_hi.s + (wave_scan(four) - four), at = -1.f;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                sum += in4[e];
+                if (at < 0.f && in4[e] > 0.f && enough(SumCount{sum, at_hi.n + (float)(4 * lane + e + 1)}, top_p, want)) at = in4[e];
+            }
+            const unsigned long long good = __ballot(at > 0.f);
+            if (good) lo = (unsigned)__builtin_amdgcn_readlane(__builtin_bit_cast(int, at), __builtin_ctzll(good));
+        } else if (hi - lo > 1) {
+            // in thread order
             int mine = 0;
-            for (int i = tid; i < n; i += STHREADS) mine += (cand[i] >= flo && cand[i] < fhi) ? 1 : 0;
+            each([&](float x) { mine += (x >= flo && x < fhi) ? 1 : 0; });
             const float upto = wave_scan((float)mine);
             f32x4 *buf = red[turn];
             turn ^= 1;
@@ -678,10 +745,10 @@ __global__ __launch_bounds__(STHREADS) void sample_draw_kernel(SampleArgs a, Sam
                 sum += v;
             }
             int at = (int)(before + upto) - mine;
-            for (int i = tid; i < n; i += STHREADS) {
-                const float v = cand[i];
-                if (v >= flo && v < fhi) list[min(at++, LIST_MAX - 1)] = v;
-            }
+            if (__ballot(mine > 0))
+                each([&](float x) {
+                    if (x >= flo && x < fhi) list[min(at++, LIST_MAX - 1)] = x;
+                });
             __syncthreads();
             lo = search_list(list, (int)sum, lo, hi, at_lo, at_hi, top_p, want, tail, red, turn);
         }
@@ -696,7 +763,7 @@ __global__ __launch_bounds__(STHREADS) void sample_draw_kernel(SampleArgs a, Sam
     };
     {
         float sum = 0.f;
-        for (int i = r; i < n_seg; i += 16) sum += kept(cand[at0 + i]);
+        each([&](float x) { sum += kept(x); });
         sum = row16_sum(sum);
         if (r == 0) seg_sum[sg] = sum;
     }
@@ -704,20 +771,36 @@ __global__ __launch_bounds__(STHREADS) void sample_draw_kernel(SampleArgs a, Sam
     __syncthreads();
     // ---- draw: first index whose running sum exceeds u * total; the last kept entry where rounding leaves none
     if (wave == 0) {
-        const float mine = seg_sum[lane], upto = wave_scan(mine), target = target_u * __shfl(upto, 63, WAVE);
+        const float mine = seg_sum[lane], upto = wave_scan(mine), target = target_u * last_lane(upto);
         const unsigned long long hit = __ballot(mine > 0.f && upto > target), some = __ballot(mine > 0.f);
         const int from = hit ? __builtin_ctzll(hit) : (some ? 63 - __builtin_clzll(some) : 0);
         float run = __shfl(upto - mine, from, WAVE);
-        const int begin = first[from], end = first[from + 1];
-        int found = -1, last = 0;
-        for (int i0 = begin; i0 < end && found < 0; i0 += 64) {
-            const float v = i0 + lane < end ? kept(cand[i0 + lane]) : 0.f, up = run + wave_scan(v);
-            const unsigned long long over = __ballot(v > 0.f && up > target), any = __ballot(v > 0.f);
-            if (hit && over) found = i0 - begin + __builtin_ctzll(over);
-            if (any) last = i0 - begin + 63 - __builtin_clzll(any);
-            run = __shfl(up, 63, WAVE);
+        const int end = (int)__shfl(len, from, WAVE);
+        int found = -1, last = 0;                 // places in the segment
+        for (int i0 = 0; i0 < end && found < 0; i0 += 256) {   // four entries a lane
+            const int i = i0 + 4 * lane;
+            f32x4 q = *(const f32x4 *)(ws.list + from * SEG + i);
+            const uint2 id = *(const uint2 *)(ws.idx + from * SEG + i);
+            const int ids[4] = {(int)(id.x & 0xffff), (int)(id.x >> 16), (int)(id.y & 0xffff), (int)(id.y >> 16)};
+#pragma unroll
+            for (int e = 0; e < 4; ++e) q[e] = i + e < end ? kept(q[e]) : 0.f;
+            const float mine4 = (q[0] + q[1]) + (q[2] + q[3]), up = wave_scan(mine4);
+            float at = run + (up - mine4);
+            int f = -1, l = -1;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                at += q[e];
+                if (q[e] > 0.f) {
+                    l = ids[e];
+                    if (f < 0 && at > target) f = ids[e];
+                }
+            }
+            const unsigned long long over = __ballot(f >= 0), any = __ballot(l >= 0);
+            if (hit && over) found = __shfl(f, __builtin_ctzll(over), WAVE);
+            if (any) last = __shfl(l, 63 - __builtin_clzll(any), WAVE);
+            run += last_lane(up);
         }
-        if (lane == 0) pick = some ? from * SEG + (int)ws.idx[from * SEG + (found >= 0 ? found : last)] : 0;
+        if (lane == 0) pick = some ? from * SEG + (found >= 0 ? found : last) : 0;
     }
     __syncthreads();
     const int tok = pick;
@@ -853,24 +936,13 @@ extern "C" int rwkv_sample_logits_ws(const float *logits, int64_t V, float tempe
     SampleWs ws;
     sample_ws(ws, workspace, V);
     const dim3 grid((unsigned)((V + SEG - 1) / SEG));
-    constexpr size_t lds = CAND_MAX * sizeof(float);
     const bool pow = temperature != 0.f && temperature != 1.f;
-    static PerDeviceOnce once;
-    bool *attr_done = once.slot();
-    if (!attr_done || !*attr_done) {
-        for (const void *k : {(const void *)sample_draw_kernel<13, true>, (const void *)sample_draw_kernel<13, false>,
-                              (const void *)sample_draw_kernel<16, true>, (const void *)sample_draw_kernel<16, false>}) {
-            const hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-            if (e != hipSuccess) return (int)e;
-        }
-        if (attr_done) *attr_done = true;
-    }
     hipLaunchKernelGGL(sample_adjust_kernel, grid, dim3(256), 0, st, a, ws);
     hipLaunchKernelGGL(sample_probs_kernel, grid, dim3(256), 0, st, a, ws);
 #define RWKV_DRAW(ROWS)                                                                                            \
     do {                                                                                                           \
-        if (pow) hipLaunchKernelGGL((sample_draw_kernel<ROWS, true>), grid, dim3(STHREADS), lds, st, a, ws);       \
-        else hipLaunchKernelGGL((sample_draw_kernel<ROWS, false>), grid, dim3(STHREADS), lds, st, a, ws);          \
+        if (pow) hipLaunchKernelGGL((sample_draw_kernel<ROWS, true>), grid, dim3(STHREADS), 0, st, a, ws);       \
+        else hipLaunchKernelGGL((sample_draw_kernel<ROWS, false>), grid, dim3(STHREADS), 0, st, a, ws);          \
     } while (0)
     if (V <= 13 * 4 * STHREADS) RWKV_DRAW(13);
     else RWKV_DRAW(16);

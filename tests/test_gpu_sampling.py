@@ -296,7 +296,10 @@ def test_draw_over_the_chip_against_one_workgroup(V, scale):
                                        None, 0.2, 0.3, 0.996, u.data_ptr(), probs.data_ptr(), token.data_ptr(),
                                        torch.cuda.current_stream().cuda_stream), "rwkv_sample_logits")
         got, ref = s.probs.cpu().numpy().astype(np.float64), probs.cpu().numpy().astype(np.float64)
-        assert abs(int((got > 0).sum()) - int((ref > 0).sum())) <= (0 if top_k or top_p in (0.0, 1.0) else 1), (top_p, top_k, temp)
+        # a running sum near 1 over up to 16 terms in turn and 16 levels of pairs is within 32 * 2^-24 = 2e-6 of the exact one in
+        # either order: entries at the cut that add up to twice that may fall to either side
+        least = min(v[v > 0].min() ** temp if temp else 1.0 for v in (got, ref))
+        assert abs(int((got > 0).sum()) - int((ref > 0).sum())) <= (0 if top_k or top_p in (0.0, 1.0) else 1 + 4e-6 / least), (top_p, top_k, temp)
         both = (got > 0) & (ref > 0)
         np.testing.assert_allclose(got[both], ref[both], rtol=4e-6, atol=1e-30)
         cdf = np.cumsum(ref)
