@@ -51,40 +51,58 @@ DEV void wkv4_step(float kk, float vv, float u, float w, float &aa, float &bb, f
     pp = p;
 }
 
+// The tokens [t0, t1) of channel c in turn, step(k, v, r, place).  Two batches of eight tokens: one is in flight while the
+// other goes through the chain.  Every load is issued (past the end the last token again): with the loads of a batch in front
+// of its own steps, and those of the last T % 8 tokens in front of each, the chain waited for memory once per batch and token.
+// Measured, us: 45 tokens, 4096 channels 9.6 -> 8.0; chunked, 1024 tokens, 4096 channels 6.7 + 17.2 -> 7.1 + 13.6, 513 tokens, 768
+// channels 4.1 + 11.0 -> 4.6 + 8.1 (the second launch also folds its chunk's predecessors eight at a time, not one).
+template <bool R, int MODE, class Step>
+DEV void wkv4_tokens(const Wkv4IO<MODE> &io, size_t base, int C, int t0, int t1, Step step) {
+    constexpr int UNR = 8;
+    struct Batch { float k[UNR], v[UNR], r[UNR]; } b0, b1;
+    auto load = [&](Batch &b, int t) {
+#pragma unroll
+        for (int i = 0; i < UNR; ++i) {
+            const size_t o = base + (size_t)min(t + i, t1 - 1) * C;
+            b.k[i] = io.ldk(o);
+            b.v[i] = io.ldv(o);
+            b.r[i] = R ? io.ldr(o) : 0.f;
+        }
+    };
+    auto run = [&](const Batch &b, int t) {
+        if (t + UNR <= t1) {   // no branch between the tokens: the division of one runs beside the chain of the next
+#pragma unroll
+            for (int i = 0; i < UNR; ++i) step(b.k[i], b.v[i], b.r[i], base + (size_t)(t + i) * C);
+        } else {
+#pragma unroll
+            for (int i = 0; i < UNR - 1; ++i)
+                if (t + i < t1) step(b.k[i], b.v[i], b.r[i], base + (size_t)(t + i) * C);
+        }
+    };
+    load(b0, t0);
+    for (int t = t0; t < t1; t += 2 * UNR) {
+        load(b1, t + UNR);
+        run(b0, t);
+        load(b0, t + 2 * UNR);
+        run(b1, t + UNR);
+    }
+}
+
 template <int MODE>
 __global__ __launch_bounds__(64) void wkv4_kernel(int T, int C, const float *__restrict__ w_, const float *__restrict__ u_,
                                                   Wkv4IO<MODE> io, float *__restrict__ aa_, float *__restrict__ bb_,
                                                   float *__restrict__ pp_) {
-    constexpr int UNR = 8;
     const int c = blockIdx.x * 64 + threadIdx.x;
     const int b = blockIdx.y;
     if (c >= C) return;
-    const size_t base = (size_t)b * T * C + c;
     const int so = b * C + c;
     const float u = u_[c], w = w_[c];
     float aa = aa_[so], bb = bb_[so], pp = pp_[so];
-    int t = 0;
-    for (; t + UNR <= T; t += UNR) {
-        float kk[UNR], vv[UNR], rr[UNR];
-#pragma unroll
-        for (int i = 0; i < UNR; ++i) {
-            const size_t o = base + (size_t)(t + i) * C;
-            kk[i] = io.ldk(o); vv[i] = io.ldv(o); rr[i] = io.ldr(o);
-        }
-#pragma unroll
-        for (int i = 0; i < UNR; ++i) {
-            float out;
-            wkv4_step(kk[i], vv[i], u, w, aa, bb, pp, out);
-            io.st(base + (size_t)(t + i) * C, out, rr[i]);
-        }
-    }
-    for (; t < T; ++t) {
-        const size_t o = base + (size_t)t * C;
+    wkv4_tokens<true>(io, (size_t)b * T * C + c, C, 0, T, [&](float kk, float vv, float rr, size_t o) {
         float out;
-        const float rr = io.ldr(o);
-        wkv4_step(io.ldk(o), io.ldv(o), u, w, aa, bb, pp, out);
+        wkv4_step(kk, vv, u, w, aa, bb, pp, out);
         io.st(o, out, rr);
-    }
+    });
     aa_[so] = aa; bb_[so] = bb; pp_[so] = pp;
 }
 
@@ -113,35 +131,21 @@ __global__ __launch_bounds__(64) void wkv4_chunk_summary_kernel(int T, int C, in
                                                                 Wkv4IO<MODE> io, const float *__restrict__ aa_,
                                                                 const float *__restrict__ bb_, const float *__restrict__ pp_,
                                                                 float *__restrict__ scratch) {
-    constexpr int UNR = 8;
     const int c = blockIdx.x * 64 + threadIdx.x, j = blockIdx.y;
     if (c >= C) return;
     if (j == 0) {
         scratch[c] = aa_[c]; scratch[C + c] = bb_[c]; scratch[2 * C + c] = pp_[c];
     }
     const float w = w_[c];
-    const int t0 = j * L, t1 = min(T, t0 + L);
     float aa = 0.f, bb = 0.f, pp = -1e38f;
-    auto step = [&](float kk, float vv) {
+    wkv4_tokens<false>(io, c, C, j * L, min(T, (j + 1) * L), [&](float kk, float vv, float, size_t) {
         const float ww = w + pp;
         const float p = fmaxf(ww, kk);
         const float e1 = __expf(ww - p), e2 = __expf(kk - p);
         aa = e1 * aa + e2 * vv;
         bb = e1 * bb + e2;
         pp = p;
-    };
-    int t = t0;
-    for (; t + UNR <= t1; t += UNR) {
-        float kk[UNR], vv[UNR];
-#pragma unroll
-        for (int i = 0; i < UNR; ++i) {
-            const size_t o = (size_t)(t + i) * C + c;
-            kk[i] = io.ldk(o); vv[i] = io.ldv(o);
-        }
-#pragma unroll
-        for (int i = 0; i < UNR; ++i) step(kk[i], vv[i]);
-    }
-    for (; t < t1; ++t) step(io.ldk((size_t)t * C + c), io.ldv((size_t)t * C + c));
+    });
     float *o = scratch + (size_t)(j + 1) * 3 * C;
     o[c] = aa; o[C + c] = bb; o[2 * C + c] = pp;
 }
@@ -151,40 +155,32 @@ __global__ __launch_bounds__(64) void wkv4_chunk_apply_kernel(int T, int C, int 
                                                               const float *__restrict__ u_, Wkv4IO<MODE> io,
                                                               float *__restrict__ aa_, float *__restrict__ bb_,
                                                               float *__restrict__ pp_, const float *__restrict__ scratch) {
-    constexpr int UNR = 8;
     const int c = blockIdx.x * 64 + threadIdx.x, j = blockIdx.y;
     if (c >= C) return;
     const float u = u_[c], w = w_[c];
     const int t0 = j * L, t1 = min(T, t0 + L);
     float aa = scratch[c], bb = scratch[C + c], pp = scratch[2 * C + c];
     const float wl = w * (float)L;
-    for (int i = 0; i < j; ++i) {
-        const float *sm = scratch + (size_t)(i + 1) * 3 * C;
-        pp += wl;
-        wkv4_merge(aa, bb, pp, sm[c], sm[C + c], sm[2 * C + c]);
-    }
-    int t = t0;
-    for (; t + UNR <= t1; t += UNR) {
-        float kk[UNR], vv[UNR], rr[UNR];
+    constexpr int FOLD = 8;
+    for (int i0 = 0; i0 < j; i0 += FOLD) {
+        float a2[FOLD], b2[FOLD], p2[FOLD];
 #pragma unroll
-        for (int i = 0; i < UNR; ++i) {
-            const size_t o = (size_t)(t + i) * C + c;
-            kk[i] = io.ldk(o); vv[i] = io.ldv(o); rr[i] = io.ldr(o);
+        for (int i = 0; i < FOLD; ++i) {
+            const float *sm = scratch + (size_t)(min(i0 + i, j - 1) + 1) * 3 * C;
+            a2[i] = sm[c]; b2[i] = sm[C + c]; p2[i] = sm[2 * C + c];
         }
 #pragma unroll
-        for (int i = 0; i < UNR; ++i) {
-            float out;
-            wkv4_step(kk[i], vv[i], u, w, aa, bb, pp, out);
-            io.st((size_t)(t + i) * C + c, out, rr[i]);
-        }
+        for (int i = 0; i < FOLD; ++i)
+            if (i0 + i < j) {
+                pp += wl;
+                wkv4_merge(aa, bb, pp, a2[i], b2[i], p2[i]);
+            }
     }
-    for (; t < t1; ++t) {
-        const size_t o = (size_t)t * C + c;
+    wkv4_tokens<true>(io, c, C, t0, t1, [&](float kk, float vv, float rr, size_t o) {
         float out;
-        const float rr = io.ldr(o);
-        wkv4_step(io.ldk(o), io.ldv(o), u, w, aa, bb, pp, out);
+        wkv4_step(kk, vv, u, w, aa, bb, pp, out);
         io.st(o, out, rr);
-    }
+    });
     if (t1 == T) { aa_[c] = aa; bb_[c] = bb; pp_[c] = pp; }
 }
 
