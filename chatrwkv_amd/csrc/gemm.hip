@@ -18,6 +18,7 @@
 // Workgroup ids are remapped so that the workgroups which share a weight tile (same m0,
 // different t0) run on the same XCD and the tile is fetched into that XCD's L2 once.
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 #include "kernels.h"
 #include "../../include/rwkv_hip_bench.h"
@@ -1700,9 +1701,10 @@ constexpr TileDim tile_dim[TILES] = {{256, 256}, {128, 128}, {128, 128}, {64, 12
 // the bytes, over long K: 0.50 us a step with 160 CUs busy where the last row of tiles is full, 0.42 where it is not (640 x
 // 14336 x 4096 130 us against 102 in four splits of the 256 x 256 tile, 513 rows 102 against 100).
 // The reduction pass of a split takes 2.5 us + 3.6 us per slab and 16 MB of fp32 output, at least 4.5 us.
-// A round of 256 x 256 tiles that leaves CUs idle runs at a higher clock: 1.17 - 1.28 us a step up to 128 workgroups, 1.38 at
-// 192, 1.70 at 256.  Priced as a full round, the receptance / key / value group of 1024 rows and 4096 channels (192 tiles) went
-// to three rounds of 128 x 128 ones: 114 us against 103 with uint8 weights, 127 against 110 with fp16.
+// A round of 256 x 256 tiles that leaves CUs idle runs at a higher clock: in short bursts 1.17 - 1.28 us a step up to 128
+// workgroups, 1.38 at 192, 1.70 at 256; within a call, whose launches keep the chip at its power limit, 1.63 at 192.  Priced as
+// a full round, the receptance / key / value group of 4096 channels (192 tiles) of a 777-row RWKV-7 call went to 2.6 rounds of
+// 128 x 128 ones, 120 us against 116 with fp16 weights; with uint8 weights and 1024 rows it belongs there (118.5 against 120.5).
 // gemm_kg_kernel: per launch, per round (split launches leave the epilogue to the second pass) and per k-tile by the CUs busy,
 // fitted to 1640 products (21 lengths, 8 widths) with the other tiles' prices as they stand: the tile it picks is 1.5 % slower
 // than the best of all on average, 4.2 % with the four tiles and prices before; 3.3 % less time.
@@ -1715,10 +1717,10 @@ double dma_cost(CostOf of, int tile, int64_t T, int64_t tiles, int nk, int c, si
     switch (tile) {
         case TILE_L: {
             const int64_t last = wgs % 256;
-            const double step = 1.28 + 0.47 * std::max<double>((double)(last - 128) / 128, 0.0);
+            const double step = 1.28 + 0.47 * std::sqrt(std::max<double>((double)(last - 64) / 192, 0.0));
             return (nk / c + (c > 1 ? 4.3 : 10.0)) * ((double)(wgs / 256) * 1.75 + (last ? step : 0.0)) + reduce;
         }
-        case TILE_S: return (double)rounds * (nk / c + (rounds > 1 ? 5.5 : 12.8)) * 0.573 + reduce;
+        case TILE_S: return (double)rounds * (nk / c + (rounds > 1 ? 5.5 : 12.8)) * (rounds > 1 && !of.w_u8 ? 0.60 : 0.573) + reduce;
         case TILE_S4:
             if (rounds > 1) return 1e30;
             if (!of.w_u8 && nk / c >= 128)
