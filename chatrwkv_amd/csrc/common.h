@@ -56,6 +56,14 @@ DEV float wave_sum(float v) {
     const float r3 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(b, 48));
     return (r0 + r1) + (r2 + r3);
 }
+// Sum over the wave that only the last lane needs: the row butterfly, then the row totals travel up through
+// two DPP row broadcasts, (r3 + r2) + (r1 + r0) -- the value wave_sum forms, in 6 instructions instead of 11.
+DEV float wave_sum_lane63(float v) {
+    v = row16_sum(v);
+    v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x142, 0xa, 0xf, false));  // row_bcast:15
+    v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x143, 0xc, 0xf, false));  // row_bcast:31
+    return v;
+}
 DEV float wave_max(float v) {
     v = fmaxf(v, dpp_mov<0xB1>(v));
     v = fmaxf(v, dpp_mov<0x4E>(v));

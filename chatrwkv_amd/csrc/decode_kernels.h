@@ -36,14 +36,6 @@ struct MatDev {
     const rwkv_half *mx, *rx, *my, *ry;
 };
 
-// Sum over the wave that only the last lane needs: the row butterfly, then the row totals travel up through
-// two DPP row broadcasts, (r3 + r2) + (r1 + r0) -- the value wave_sum forms, in 6 instructions instead of 11.
-DEV float wave_sum_lane63(float v) {
-    v = row16_sum(v);
-    v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x142, 0xa, 0xf, false));  // row_bcast:15
-    v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x143, 0xc, 0xf, false));  // row_bcast:31
-    return v;
-}
 // Sums of K values over the first `npw` waves of the workgroup (the waves that run a prologue), in two
 // halves with a synchronisation between them, which the caller places: `put` by each of those waves
 // before it, `get` by any wave after it.  `red` (K * DWAVES floats) must not be in use by an

@@ -100,7 +100,7 @@ struct SeqMixArgs {
     const rwkv_half *ry[6], *my[6];  // NULL ry = no scaling / sums (fp16 weights)
     rwkv_half *xs[6];          // [T, C] outputs
     float *s0[6], *s2[6];      // [T] outputs
-    int maa_form;              // RWKV-6 / RWKV-7 mixing kx = xx + (prev - xx) * m, rounded after every step
+    int maa_form;              // RWKV-6 / RWKV-7 mixing kx = xx + (prev - xx) * m: the difference rounded to fp16, then one rounding
 };
 
 int lnmix_seq_launch(const SeqMixArgs &a, int nj, hipStream_t st);

@@ -30,24 +30,87 @@ __global__ __launch_bounds__(256) void copy16_kernel(int n16, const u32x4 *__res
     if (i < n16) dst[i] = src[i];
 }
 
+// ---- LayerNorm and mix, eight channels at a time ----------------------------------------------------------------
+// Long calls are bound by vector-instruction issue, so each step is the fewest instructions that form the same value:
+// sums take two channels per v_dot2_f32_f16 (exact products with 1, fp32 accumulation, subnormals kept), x - mean reads
+// its fp16 operand in place (v_fma_mix_f32 with 1.0: one rounding, as the conversion and subtraction), the affine and the
+// mixes end in v_fma_mix{lo,hi}_f16.  The compiler takes three to four instructions for each of these.
+DEV h16x2 pair(h16x8 v, int p) { return h16x2{v[2 * p], v[2 * p + 1]}; }
+DEV float dot8(h16x8 v, h16x8 w, float a) {
+#pragma unroll
+    for (int p = 0; p < 4; ++p) a = __builtin_amdgcn_fdot2(pair(v, p), pair(w, p), a, false);
+    return a;
+}
+DEV float sum8(h16x8 v, float a) {
+    const h16 one = (h16)1.f;
+    return dot8(v, h16x8{one, one, one, one, one, one, one, one}, a);
+}
+DEV void less_mean8(h16x8 v, float mean, float (&d)[8]) {
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+        asm("v_fma_mix_f32 %0, %1, 1.0, -%2 op_sel_hi:[1,0,0]" : "=v"(d[2 * p]) : "v"(pair(v, p)), "v"(mean));
+        asm("v_fma_mix_f32 %0, %1, 1.0, -%2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(d[2 * p + 1]) : "v"(pair(v, p)), "v"(mean));
+    }
+}
+DEV float squares8(const float (&d)[8], float a) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) a = __builtin_fmaf(d[e], d[e], a);
+    return a;
+}
+// fp16(fma(t, w, b)) of two channels
+DEV h16x2 fma_pair(float t0, float t1, h16x2 w, h16x2 b) {
+    h16x2 r;
+    asm("v_fma_mixlo_f16 %0, %1, %3, %4 op_sel_hi:[0,1,1]\n\tv_fma_mixhi_f16 %0, %2, %3, %4 op_sel:[0,1,1] op_sel_hi:[0,1,1]"
+        : "=&v"(r) : "v"(t0), "v"(t1), "v"(w), "v"(b));
+    return r;
+}
+DEV h16x8 join8(const h16x2 (&q)[4]) { return h16x8{q[0].x, q[0].y, q[1].x, q[1].y, q[2].x, q[2].y, q[3].x, q[3].y}; }
+DEV h16x8 norm8(const float (&d)[8], float rstd, h16x8 w, h16x8 b) {
+    h16x2 q[4];
+#pragma unroll
+    for (int p = 0; p < 4; ++p) q[p] = fma_pair(d[2 * p] * rstd, d[2 * p + 1] * rstd, pair(w, p), pair(b, p));
+    return join8(q);
+}
+// What all mixes of a token share: xx - prev in fp32 (RWKV-4, 5), or prev - xx in fp16 (RWKV-6, 7: maa_form).
+struct Shift8 { float d[8]; h16x8 d16; };
+DEV Shift8 shift8(h16x8 xx, h16x8 prev, bool maa_form) {
+    Shift8 s = {};
+    if (maa_form) s.d16 = prev - xx;
+    else
+#pragma unroll
+        for (int p = 0; p < 4; ++p) {
+            asm("v_fma_mix_f32 %0, %1, 1.0, -%2 op_sel_hi:[1,0,1]" : "=v"(s.d[2 * p]) : "v"(pair(xx, p)), "v"(pair(prev, p)));
+            asm("v_fma_mix_f32 %0, %1, 1.0, -%2 op_sel:[1,0,1] op_sel_hi:[1,0,1]" : "=v"(s.d[2 * p + 1]) : "v"(pair(xx, p)), "v"(pair(prev, p)));
+        }
+    return s;
+}
+// xx m + prev (1 - m) as fp16(prev + (xx - prev) m): one rounding after the difference, which is exact but for the last bits
+// of operands that differ by more than 2^13.  maa_form: xx + (prev - xx) m, the difference rounded to fp16.
+DEV h16x8 mix8(h16x8 xx, h16x8 prev, const Shift8 &s, h16x8 m, bool maa_form) {
+    if (maa_form) return __builtin_elementwise_fma(s.d16, m, xx);
+    h16x2 q[4];
+#pragma unroll
+    for (int p = 0; p < 4; ++p) q[p] = fma_pair(s.d[2 * p], s.d[2 * p + 1], pair(m, p), pair(prev, p));
+    return join8(q);
+}
+DEV float row_mean(float sum, int C) { return sum / C; }
+DEV float row_rstd(float squares, int C) { return rsqrtf(squares / C + LN_EPS); }
+
 DEV void row_stats(const rwkv_half *x, int C, float *red, float &mean, float &rstd) {
     float s = 0.f;
+    for (int j8 = threadIdx.x; j8 < (C >> 3); j8 += blockDim.x) s = sum8(*(const h16x8 *)(x + 8 * j8), s);
+    mean = row_mean(block_sum(s, red), C);
+    float q = 0.f, d[8];
     for (int j8 = threadIdx.x; j8 < (C >> 3); j8 += blockDim.x) {
-        const h16x8 v = *(const h16x8 *)(x + 8 * j8);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) s += (float)v[e];
+        less_mean8(*(const h16x8 *)(x + 8 * j8), mean, d);
+        q = squares8(d, q);
     }
-    mean = block_sum(s, red) / C;
-    float q = 0.f;
-    for (int j8 = threadIdx.x; j8 < (C >> 3); j8 += blockDim.x) {
-        const h16x8 v = *(const h16x8 *)(x + 8 * j8);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            const float d = (float)v[e] - mean;
-            q += d * d;
-        }
-    }
-    rstd = rsqrtf(block_sum(q, red) / C + LN_EPS);
+    rstd = row_rstd(block_sum(q, red), C);
+}
+DEV h16x8 row_norm8(const rwkv_half *x, float mean, float rstd, h16x8 w, h16x8 b) {
+    float d[8];
+    less_mean8(*(const h16x8 *)x, mean, d);
+    return norm8(d, rstd, w, b);
 }
 
 // One workgroup per token row.  Row t needs LN(x[t-1]) for the token shift: it is recomputed here
@@ -67,47 +130,20 @@ __global__ __launch_bounds__(256) void lnmix_seq_kernel(SeqMixArgs a) {
 #pragma unroll
     for (int i = 0; i < 2 * NJ; ++i) acc[i] = 0.f;
     for (int j8 = threadIdx.x; j8 < (C >> 3); j8 += blockDim.x) {
-        const h16x8 xv = *(const h16x8 *)(x + 8 * j8);
-        const h16x8 wv = *(const h16x8 *)(a.ln_w + 8 * j8);
-        const h16x8 bv = *(const h16x8 *)(a.ln_b + 8 * j8);
-        h16x8 xx, pv;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) xx[e] = (h16)(((float)xv[e] - mean) * rstd * (float)wv[e] + (float)bv[e]);
-        pv = xx;
-        if (shift) {
-            if (t > 0) {
-                const h16x8 pxv = *(const h16x8 *)(xp + 8 * j8);
-#pragma unroll
-                for (int e = 0; e < 8; ++e)
-                    pv[e] = (h16)(((float)pxv[e] - pmean) * prstd * (float)wv[e] + (float)bv[e]);
-            } else {
-                pv = *(const h16x8 *)(a.sx + 8 * j8);
-            }
-        }
+        const h16x8 wv = *(const h16x8 *)(a.ln_w + 8 * j8), bv = *(const h16x8 *)(a.ln_b + 8 * j8);
+        const h16x8 xx = row_norm8(x + 8 * j8, mean, rstd, wv, bv);
+        h16x8 pv = xx;
+        if (shift) pv = t > 0 ? row_norm8(xp + 8 * j8, pmean, prstd, wv, bv) : *(const h16x8 *)(a.sx + 8 * j8);
         if (a.xx_last && t == a.T - 1) *(h16x8 *)(a.xx_last + 8 * j8) = xx;
+        const Shift8 sh = shift8(xx, pv, a.maa_form);
 #pragma unroll
         for (int j = 0; j < NJ; ++j) {
-            h16x8 kx = xx;
-            if (a.mix[j]) {
-                const h16x8 mv = *(const h16x8 *)(a.mix[j] + 8 * j8);
-#pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    const float m = (float)mv[e];
-                    kx[e] = a.maa_form ? (h16)((float)xx[e] + (float)(h16)((float)(h16)((float)pv[e] - (float)xx[e]) * m))
-                                       : (h16)((float)xx[e] * m + (float)pv[e] * (1.f - m));
-                }
-            }
+            const h16x8 kx = a.mix[j] ? mix8(xx, pv, sh, *(const h16x8 *)(a.mix[j] + 8 * j8), a.maa_form) : xx;
             h16x8 o = kx;
             if (a.ry[j]) {
-                const h16x8 rv = *(const h16x8 *)(a.ry[j] + 8 * j8);
-                const h16x8 yv = *(const h16x8 *)(a.my[j] + 8 * j8);
-#pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    const float k = (float)kx[e];
-                    o[e] = (h16)(k * (float)rv[e]);
-                    acc[2 * j] += k;
-                    acc[2 * j + 1] += k * (float)yv[e];
-                }
+                o = kx * *(const h16x8 *)(a.ry[j] + 8 * j8);
+                acc[2 * j] = sum8(kx, acc[2 * j]);
+                acc[2 * j + 1] = dot8(kx, *(const h16x8 *)(a.my[j] + 8 * j8), acc[2 * j + 1]);
             }
             *(h16x8 *)(a.xs[j] + (size_t)t * C + 8 * j8) = o;
         }
@@ -123,15 +159,9 @@ __global__ __launch_bounds__(256) void lnmix_seq_kernel(SeqMixArgs a) {
     if (a.state_out && t == 0) {
         const rwkv_half *xl = a.x + (size_t)(a.T - 1) * C;
         if (a.T > 1) row_stats(xl, C, red, mean, rstd);
-        for (int j8 = threadIdx.x; j8 < (C >> 3); j8 += blockDim.x) {
-            const h16x8 xv = *(const h16x8 *)(xl + 8 * j8);
-            const h16x8 wv = *(const h16x8 *)(a.ln_w + 8 * j8);
-            const h16x8 bv = *(const h16x8 *)(a.ln_b + 8 * j8);
-            h16x8 xx;
-#pragma unroll
-            for (int e = 0; e < 8; ++e) xx[e] = (h16)(((float)xv[e] - mean) * rstd * (float)wv[e] + (float)bv[e]);
-            *(h16x8 *)(a.state_out + 8 * j8) = xx;
-        }
+        for (int j8 = threadIdx.x; j8 < (C >> 3); j8 += blockDim.x)
+            *(h16x8 *)(a.state_out + 8 * j8) =
+                row_norm8(xl + 8 * j8, mean, rstd, *(const h16x8 *)(a.ln_w + 8 * j8), *(const h16x8 *)(a.ln_b + 8 * j8));
     }
 }
 
@@ -152,37 +182,37 @@ __global__ __launch_bounds__(256) void ln_f32_f16_kernel(int C, const float *__r
 // K sums over a row whose 8-wide chunks are dealt to 256 threads, chunk v, v + 256, ... to thread v, each thread adding up
 // its own in that order: add(v) adds this thread's chunks to v.  With 512 threads the second 256 hold the later half of
 // those chunks and go on, through LDS, from where the first left off: the same additions in the same order, so the
-// totals are the same bits with either number of threads.  v starts at zero; hop: K * 256 floats (512 threads only).
+// totals are the same bits with either number of threads.  v starts at zero; red: 4 K floats of these sums' own, 16-byte
+// aligned; hop: K * 256 floats (512 threads only).
 template <int K, int NT, class Add>
 DEV void row_sums(float (&v)[K], float *red, float *hop, Add add) {
-    if constexpr (NT == 256) {
-        add(v);
-        block_sum_n<K>(v, red);
-    } else {
-        static_assert(NT == 512, "two threads per chain");
-        const int chain = threadIdx.x & 255, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    static_assert(NT == 256 || NT == 512, "two threads per chain at most");
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if constexpr (NT == 512) {
+        const int chain = threadIdx.x & 255;
         if (wave < 4) {
             add(v);
 #pragma unroll
             for (int k = 0; k < K; ++k) hop[k * 256 + chain] = v[k];
         }
-        __syncthreads();              // also: the totals of the sums before have been read
-        if (wave >= 4) {
+        __syncthreads();
+        if (wave >= 4)
 #pragma unroll
             for (int k = 0; k < K; ++k) v[k] = hop[k * 256 + chain];
-            add(v);
+    }
+    if (NT == 256 || wave >= 4) {
+        add(v);
 #pragma unroll
-            for (int k = 0; k < K; ++k) v[k] = wave_sum(v[k]);
-            if ((threadIdx.x & 63) == 0)
+        for (int k = 0; k < K; ++k) v[k] = wave_sum_lane63(v[k]);
+        if ((threadIdx.x & 63) == 63)
 #pragma unroll
-                for (int k = 0; k < K; ++k) red[k * 4 + wave - 4] = v[k];
-        }
-        __syncthreads();
+            for (int k = 0; k < K; ++k) red[k * 4 + (wave & 3)] = v[k];
+    }
+    __syncthreads();
 #pragma unroll
-        for (int k = 0; k < K; ++k) {  // as block_sum_n adds up four waves
-            v[k] = 0.f;
-            for (int i = 0; i < 4; ++i) v[k] += red[k * 4 + i];
-        }
+    for (int k = 0; k < K; ++k) {
+        const f32x4 r = *(const f32x4 *)(red + 4 * k);
+        v[k] = ((r[0] + r[1]) + r[2]) + r[3];
     }
 }
 
@@ -197,7 +227,8 @@ DEV void row_sums(float (&v)[K], float *red, float *hop, Add add) {
 template <int NJ, int CH, bool PRE, int NT>
 __global__ __launch_bounds__(NT) void lnmix_seq_fast_kernel(SeqMixArgs a) {
     constexpr int NSUM = 2 * NJ > 3 ? 2 * NJ : 3;
-    __shared__ float red[4 * NSUM], hop[NT == 512 ? 256 * NSUM : 1];
+    __shared__ __align__(16) float red[24 + 8 * NJ];
+    __shared__ float hop[NT == 512 ? 256 * NSUM : 1];
     const int t = blockIdx.x, C = a.C, nch = C >> 3;
     // this thread's chunk c: tid + 256 c, or with 512 threads the first CH and the last CH of a chain's 2 CH
     const int j8_0 = NT == 256 ? (int)threadIdx.x : (int)(threadIdx.x & 255) + 256 * CH * (int)(threadIdx.x >> 8);
@@ -219,7 +250,7 @@ __global__ __launch_bounds__(NT) void lnmix_seq_fast_kernel(SeqMixArgs a) {
         if constexpr (PRE) {
 #pragma unroll
             for (int j = 0; j < NJ; ++j) {
-                if (a.mix[j]) mv[j][c] = *(const h16x8 *)(a.mix[j] + 8 * j8);
+                mv[j][c] = *(const h16x8 *)((a.mix[j] ? a.mix[j] : a.ln_w) + 8 * j8);
                 if (a.ry[j]) { rv[j][c] = *(const h16x8 *)(a.ry[j] + 8 * j8); yv[j][c] = *(const h16x8 *)(a.my[j] + 8 * j8); }
             }
         }
@@ -229,85 +260,69 @@ __global__ __launch_bounds__(NT) void lnmix_seq_fast_kernel(SeqMixArgs a) {
 #pragma unroll
         for (int c = 0; c < CH; ++c)
             if (j8_0 + c * 256 < nch) {
-#pragma unroll
-                for (int e = 0; e < 8; ++e) { v[0] += (float)xv[c][e]; v[1] += (float)pxv[c][e]; }
-                if (commit)   // the last row's statistics: only the workgroup that writes the new state needs them
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) v[2] += (float)lv[c][e];
+                v[0] = sum8(xv[c], v[0]);
+                v[1] = sum8(pxv[c], v[1]);
+                v[2] = sum8(lv[c], v[2]);
             }
     });
-    const float mean = st[0] / C, pmean = st[1] / C, lmean = st[2] / C;
+    const float mean = row_mean(st[0], C), pmean = row_mean(st[1], C), lmean = row_mean(st[2], C);
+    float dx[CH][8], dp[CH][8];
     st[0] = st[1] = st[2] = 0.f;
-    row_sums<3, NT>(st, red, hop, [&](float (&v)[3]) {
+    row_sums<3, NT>(st, red + 12, hop, [&](float (&v)[3]) {
 #pragma unroll
-        for (int c = 0; c < CH; ++c)
+        for (int c = 0; c < CH; ++c) {
+            less_mean8(xv[c], mean, dx[c]);
+            less_mean8(pxv[c], pmean, dp[c]);
             if (j8_0 + c * 256 < nch) {
-#pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    const float d = (float)xv[c][e] - mean, pd = (float)pxv[c][e] - pmean;
-                    v[0] += d * d;
-                    v[1] += pd * pd;
+                v[0] = squares8(dx[c], v[0]);
+                v[1] = squares8(dp[c], v[1]);
+                if (commit) {   // the last row's statistics: only the workgroup that writes the new state needs them
+                    float dl[8];
+                    less_mean8(lv[c], lmean, dl);
+                    v[2] = squares8(dl, v[2]);
                 }
-                if (commit)
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) {
-                        const float ld = (float)lv[c][e] - lmean;
-                        v[2] += ld * ld;
-                    }
             }
+        }
     });
-    const float rstd = rsqrtf(st[0] / C + LN_EPS), prstd = rsqrtf(st[1] / C + LN_EPS), lrstd = rsqrtf(st[2] / C + LN_EPS);
+    const float rstd = row_rstd(st[0], C), prstd = row_rstd(st[1], C), lrstd = row_rstd(st[2], C);
     float acc[2 * NJ];
 #pragma unroll
     for (int i = 0; i < 2 * NJ; ++i) acc[i] = 0.f;
-    // Two products at a time, explicitly: the compiler makes v_dot2 of neighbouring fused multiply-adds in some places and
-    // not in others, and the two round differently.
     auto add_mix = [](float (&v)[2 * NJ], int j, h16x8 kx, h16x8 y8) {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) v[2 * j] += (float)kx[e];
-#pragma unroll
-        for (int e = 0; e < 8; e += 2)
-            v[2 * j + 1] = __builtin_amdgcn_fdot2(h16x2{kx[e], kx[e + 1]}, h16x2{y8[e], y8[e + 1]}, v[2 * j + 1], false);
+        v[2 * j] = sum8(kx, v[2 * j]);
+        v[2 * j + 1] = dot8(kx, y8, v[2 * j + 1]);
     };
     h16x8 kv[CH][NJ], sv[CH][NJ];   // 512 threads: the mixes and their my, added up when the first half's sums are there
 #pragma unroll
     for (int c = 0; c < CH; ++c) {
         const int j8 = j8_0 + c * 256;
         if (j8 >= nch) break;
-        h16x8 xx, pv;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) xx[e] = (h16)(((float)xv[c][e] - mean) * rstd * (float)wv[c][e] + (float)bv[c][e]);
-        pv = xx;
+        if (NT == 512) {   // a thread of one half has skipped the other half's sums
+            less_mean8(xv[c], mean, dx[c]);
+            less_mean8(pxv[c], pmean, dp[c]);
+        }
+        const h16x8 xx = norm8(dx[c], rstd, wv[c], bv[c]);
+        h16x8 pv = xx;
         if (shift) {
-            if (t > 0) {
-#pragma unroll
-                for (int e = 0; e < 8; ++e)
-                    pv[e] = (h16)(((float)pxv[c][e] - pmean) * prstd * (float)wv[c][e] + (float)bv[c][e]);
-            } else {
-                pv = *(const h16x8 *)(a.sx + 8 * j8);
-            }
+            if (t > 0) pv = norm8(dp[c], prstd, wv[c], bv[c]);
+            else pv = *(const h16x8 *)(a.sx + 8 * j8);
         }
         if (a.xx_last && t == a.T - 1) *(h16x8 *)(a.xx_last + 8 * j8) = xx;
+        const Shift8 sh = shift8(xx, pv, a.maa_form);
 #pragma unroll
         for (int j = 0; j < NJ; ++j) {
             h16x8 kx = xx;
             if (a.mix[j]) {
                 h16x8 m8;
                 if constexpr (PRE) m8 = mv[j][c]; else m8 = *(const h16x8 *)(a.mix[j] + 8 * j8);
-#pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    const float m = (float)m8[e];
-                    kx[e] = a.maa_form ? (h16)((float)xx[e] + (float)(h16)((float)(h16)((float)pv[e] - (float)xx[e]) * m))
-                                       : (h16)((float)xx[e] * m + (float)pv[e] * (1.f - m));
-                }
+                kx = mix8(xx, pv, sh, m8, a.maa_form);
             }
             h16x8 o = kx;
             if (a.ry[j]) {
                 h16x8 r8, y8;
                 if constexpr (PRE) { r8 = rv[j][c]; y8 = yv[j][c]; }
                 else { r8 = *(const h16x8 *)(a.ry[j] + 8 * j8); y8 = *(const h16x8 *)(a.my[j] + 8 * j8); }
-#pragma unroll
-                for (int e = 0; e < 8; ++e) o[e] = (h16)((float)kx[e] * (float)r8[e]);
+                o = kx * r8;
                 if constexpr (NT == 256) add_mix(acc, j, kx, y8);
                 else { kv[c][j] = kx; sv[c][j] = y8; }
             }
@@ -316,17 +331,16 @@ __global__ __launch_bounds__(NT) void lnmix_seq_fast_kernel(SeqMixArgs a) {
         // Only row 0 reads the old state, so row 0's workgroup writes the new one, each thread exactly the chunk it
         // has just read: no second launch.
         if (commit) {
-            h16x8 ls;
-#pragma unroll
-            for (int e = 0; e < 8; ++e) ls[e] = (h16)(((float)lv[c][e] - lmean) * lrstd * (float)wv[c][e] + (float)bv[c][e]);
-            *(h16x8 *)(a.state_out + 8 * j8) = ls;
+            float dl[8];
+            less_mean8(lv[c], lmean, dl);
+            *(h16x8 *)(a.state_out + 8 * j8) = norm8(dl, lrstd, wv[c], bv[c]);
         }
     }
     bool any = false;
 #pragma unroll
     for (int j = 0; j < NJ; ++j) any = any || a.ry[j];
     if (any) {
-        row_sums<2 * NJ, NT>(acc, red, hop, [&](float (&v)[2 * NJ]) {
+        row_sums<2 * NJ, NT>(acc, red + 24, hop, [&](float (&v)[2 * NJ]) {
             if constexpr (NT > 256)
 #pragma unroll
                 for (int c = 0; c < CH; ++c)
@@ -360,15 +374,18 @@ static bool lnmix_seq_fast_launch(const SeqMixArgs &a, int nj, hipStream_t st) {
 
 int lnmix_seq_launch(const SeqMixArgs &a, int nj, hipStream_t st) {
     // Rows of up to 8192 channels: the register-resident kernel (1, 2 or 4 chunks of 8 channels per chain of additions).
-    // Calls of up to 512 rows have one or two rows per CU: there a row's own sequence of conversions and mixes is the time,
+    // Calls of up to 512 rows have one or two rows per CU: there a row's own chain of barriers and instructions is the time,
     // so rows of more than 2048 channels get 512 threads instead of 256, with the same sums (row_sums).  4096 channels, us,
-    // 256 -> 512 threads at 4 / 16 / 45 / 256 / 512 rows: one mix 6.2 -> 4.2, 6.1 -> 4.7, 7.0 -> 5.1, 7.1 -> 5.4, 8.0 -> 6.8;
-    // three mixes with scaling 10.5 -> 7.0, 10.3 -> 7.1, 10.9 -> 7.4, 12.4 -> 8.7, 13.8 -> 11.5; six mixes without 11.9 -> 7.6,
-    // 11.6 -> 7.6, 14.0 -> 8.6, 16.7 -> 10.7, 18.2 -> 12.7.  Longer calls are bound by instruction issue (5120 channels, three
-    // mixes: 512 rows 21.8 -> 16.4, 600 rows 22.0 -> 22.7, one mix 600 rows 10.2 -> 11.2; 4096 channels, 1024 rows 20.7 -> 21.0).
+    // 256 -> 512 threads at 45 / 256 / 512 / 600 / 1024 rows: one mix 4.2 -> 3.4, 4.4 -> 3.6, 4.7 -> 4.8, 5.4 -> 5.7, 6.6 -> 7.1;
+    // three mixes with scaling 6.7 -> 5.4, 7.4 -> 6.1, 8.4 -> 7.9, 9.4 -> 10.4, 11.7 -> 12.6; six mixes without 6.7 -> 5.5, 8.0 ->
+    // 6.8, 9.1 -> 8.5, 10.0 -> 11.7, 12.8 -> 14.5 (5120 channels, three mixes: 512 rows 10.6 -> 10.2, 600 rows 11.8 -> 14.6).
     // Up to 4096 channels the mix and scale vectors of these calls are requested at the top too, except for six mixes.
-    // Several rows per workgroup, sharing vectors and the previous row's statistics: slower at every length (1024 rows 21.8
-    // with two, 33 with four).
+    // us before the element code above was written out (three to four instructions per step, sums over loops of unknown length):
+    // three scaled mixes of 4096 channels at 45 / 1024 rows 6.6 / 16.4, now 5.4 / 11.7; six at 777 rows 14.9, now 11.0; four of 2048
+    // channels at 333 rows 7.1, now 5.1; three of 768 at 513 rows 7.4, now 4.5.  An empty launch is 3.2; at 1024 rows it is the 130 KB
+    // per row through a CU's L1 and the 24 MB of stores.
+    // Several rows per workgroup, sharing vectors and the previous row's statistics, measured with the element code before: slower
+    // at every length (1024 rows 21.8 with two, 33 with four, 20.7 with one).
     if (a.C <= 8192 && (nj == 1 || nj == 2 || nj == 3 || nj == 4 || nj == 6)) {
         const bool few = a.T <= 512;
         if (a.C <= 2048) few ? lnmix_seq_fast_launch<1, true, 256>(a, nj, st) : lnmix_seq_fast_launch<1, false, 256>(a, nj, st);
