@@ -1754,7 +1754,7 @@ int dma_split(CostOf of, int tile, int64_t T, int64_t tiles, int nk, size_t out_
 }
 
 // the tile of least cost for products of M_i outputs (n of them, one launch); ks: its K split
-int dma_tile(CostOf of, int64_t T, int nk, int n, const int64_t *M, size_t ws_bytes, int *ks) {
+int dma_tile(CostOf of, int64_t T, int nk, int n, const int64_t *M, size_t ws_bytes, int *ks, double *cost = nullptr) {
     int best = TILE_S;
     double best_cost = 1e30;
     int64_t outs = 0;
@@ -1767,6 +1767,7 @@ int dma_tile(CostOf of, int64_t T, int nk, int n, const int64_t *M, size_t ws_by
         const int k = dma_split(of, tile, T, tiles, nk, (size_t)(T * outs) * sizeof(float), ws_bytes, &c);
         if (c < best_cost) { best_cost = c; best = tile; *ks = k; }
     }
+    if (cost) *cost = best_cost;
     return best;
 }
 
@@ -1876,11 +1877,14 @@ int pick_cfg(int64_t T, int64_t N, int64_t M, bool w_u8, const GemmEpi &ep, bool
 
 GemmPlan gemm_plan(bool w_u8, int64_t T, int64_t N, int64_t M, const rwkv_half *A, int64_t lda, const void *W,
                    int64_t ldw, const void *Y, int64_t ldy, const GemmEpi &ep) {
-    if (skinny_ok(w_u8, T, N, A, lda, W, ldw, ep)) return GemmPlan{0, 0, 0, 1};
+    if (skinny_ok(w_u8, T, N, A, lda, W, ldw, ep)) return GemmPlan{0, 0, 0, 1, 0.0};
     int ks;
     const int cfg = pick_cfg(T, N, M, w_u8, ep, dma_ok(w_u8, N, M, A, lda, W, ldw, Y, ldy, ep), &ks);
-    if (cfg < CFG_DMA) return GemmPlan{1, 0, 0, 1};
-    return GemmPlan{2, tile_dim[cfg - CFG_DMA].tm, tile_dim[cfg - CFG_DMA].tn, ks};
+    if (cfg < CFG_DMA) return GemmPlan{1, 0, 0, 1, 0.0};
+    const TileDim d = tile_dim[cfg - CFG_DMA];
+    const int64_t tiles = ((T + d.tm - 1) / d.tm) * ((M + d.tn - 1) / d.tn);
+    return GemmPlan{2, d.tm, d.tn, ks,
+                    dma_cost({w_u8, slow_epilogue(ep)}, cfg - CFG_DMA, T, tiles, (int)(N / BK), ks, (size_t)(T * M) * sizeof(float))};
 }
 
 int gemm_launch(bool w_u8, int64_t T, int64_t N, int64_t M, const rwkv_half *A, int64_t lda, const void *W,
@@ -1913,22 +1917,54 @@ int mm8_prepare_launch(int64_t T, int64_t N, const rwkv_half *x, int64_t ldx, co
 // n (2..4) products [T, N] x [N, M_i] of uint8 or fp16 weights with their own inputs, outputs and epilogues in one
 // launch.  uint8 with xs != NULL: x[i] is the unscaled activation and xs[i] / sums[i] (2 T floats) are scratch;
 // uint8 with xs == NULL: x[i] is already scaled by ry and sums[i] holds its row sums -- as 2 T totals, or with
-// parts > 1 (a multiple of four; direct-to-LDS launches only, see gemm_group_takes_parts) as 2 T floats of scratch
+// parts > 1 (a multiple of four; direct-to-LDS launches only, see gemm_group_plan) as 2 T floats of scratch
 // followed by [T][parts] partial sums of x and [T][parts] of x * my, which the launch adds up in index order.
 // Operands laid out for 16-byte loads: the direct-to-LDS kernel, tile size and K split (over splitk_ws,
 // RWKV_SPLITK_WS_BYTES of scratch, or NULL) from the cost model; otherwise register-staged 128 x 128 tiles at full depth.
-bool gemm_group_takes_parts(bool w_u8, int n, int64_t T, int64_t N, const rwkv_half *const *x, const rwkv_mat *const *mats,
-                            void *const *Y) {
-    if (!w_u8 || n < 2 || n > 4 || (N % BK)) return false;
+static int group_tile(bool w_u8, int n, int64_t T, int64_t N, const rwkv_mat *const *mats, bool may_split, int *ks, double *us = nullptr) {
+    int64_t outs[4];
+    bool m8 = true;
+    for (int i = 0; i < n; ++i) {
+        outs[i] = mats[i]->M;
+        m8 = m8 && !(mats[i]->M & 7);
+    }
+    return dma_tile({w_u8, false}, T, (int)(N / BK), n, outs, may_split && m8 ? RWKV_SPLITK_WS_BYTES : 0, ks, us);
+}
+GemmPlan gemm_group_plan(bool w_u8, int n, int64_t T, int64_t N, const rwkv_half *const *x, const rwkv_mat *const *mats,
+                         void *const *Y, bool may_split) {
+    GemmPlan p{1, 0, 0, 1, 0.0};
+    if (n < 2 || n > 4 || (N % BK)) return p;
     const float one = 0.f;
     bool skinny = true;
     for (int i = 0; i < n; ++i) {
         GemmEpi e{};
-        e.mx = mats[i]->mx; e.rx = mats[i]->rx; e.s0 = &one; e.s2 = &one; e.out_dtype = RWKV_DT_F16;
-        if (mats[i]->N != N || !dma_ok(true, N, mats[i]->M, x[i], N, mats[i]->w, mats[i]->ld, Y[i], mats[i]->M, e)) return false;
-        skinny = skinny && skinny_ok(true, T, N, x[i], N, mats[i]->w, mats[i]->ld, e);
+        if (w_u8) { e.mx = mats[i]->mx; e.rx = mats[i]->rx; e.s0 = &one; e.s2 = &one; }
+        e.out_dtype = RWKV_DT_F16;
+        if (mats[i]->N != N || !dma_ok(w_u8, N, mats[i]->M, x[i], N, mats[i]->w, mats[i]->ld, Y[i], mats[i]->M, e)) return p;
+        skinny = skinny && skinny_ok(w_u8, T, N, x[i], N, mats[i]->w, mats[i]->ld, e);
     }
-    return !skinny;
+    if (skinny) { p.kind = 0; return p; }
+    const int tile = group_tile(w_u8, n, T, N, mats, may_split, &p.ks, &p.us);
+    p.kind = 2;
+    p.tm = tile_dim[tile].tm;
+    p.tn = tile_dim[tile].tn;
+    return p;
+}
+bool gemm_group_pays(bool w_u8, int n, int64_t T, int64_t N, const rwkv_half *const *x, const rwkv_mat *const *mats,
+                     void *const *Y, const GemmEpi *eps, float *splitk_ws) {
+    const GemmPlan g = gemm_group_plan(w_u8, n, T, N, x, mats, Y, splitk_ws != nullptr);
+    if (g.kind != 2) return false;
+    const float one = 0.f;
+    double us = 0.0;
+    for (int i = 0; i < n; ++i) {
+        GemmEpi e = eps[i];
+        e.splitk_ws = splitk_ws; e.splitk_bytes = RWKV_SPLITK_WS_BYTES;
+        if (w_u8) { e.mx = mats[i]->mx; e.rx = mats[i]->rx; e.s0 = &one; e.s2 = &one; }
+        const GemmPlan p = gemm_plan(w_u8, T, N, mats[i]->M, x[i], N, mats[i]->w, mats[i]->ld, Y[i], mats[i]->M, e);
+        if (p.kind != 2) return false;
+        us += p.us;
+    }
+    return g.us < us;
 }
 
 int gemm_group_launch(bool w_u8, int n, int64_t T, int64_t N, const rwkv_half *const *x, const rwkv_mat *const *mats,
@@ -1947,7 +1983,7 @@ int gemm_group_launch(bool w_u8, int n, int64_t T, int64_t N, const rwkv_half *c
         hipLaunchKernelGGL(mm8_prepare_group_kernel, dim3((unsigned)((T + 3) / 4), (unsigned)n), dim3(256), 0, st, (int)T, (int)N, p);
     }
     int64_t tiles = 0, max_out = 0;   // tiles: register-staged fallback
-    bool dma = true, m8 = true;
+    bool dma = true;
     for (int i = 0; i < n; ++i) {
         if (mats[i]->N != N) return RWKV_E_SHAPE;
         g.A[i] = (const h16 *)(prep ? xs[i] : x[i]);
@@ -1958,7 +1994,6 @@ int gemm_group_launch(bool w_u8, int n, int64_t T, int64_t N, const rwkv_half *c
         if (parts > 1) { g.ep[i].parts = parts; g.ep[i].p0 = sums[i] + 2 * T; g.ep[i].p2 = sums[i] + 2 * T + (size_t)T * parts; }
         tiles = std::max<int64_t>(tiles, ((T + 127) / 128) * ((mats[i]->M + 127) / 128));
         max_out = std::max<int64_t>(max_out, T * mats[i]->M);
-        m8 = m8 && !(mats[i]->M & 7);
         dma = dma && dma_ok(w_u8, N, mats[i]->M, g.A[i], N, g.W[i], g.ldw[i], g.Y[i], mats[i]->M, g.ep[i]);
     }
     {
@@ -1978,10 +2013,8 @@ int gemm_group_launch(bool w_u8, int n, int64_t T, int64_t N, const rwkv_half *c
     if (dma) {
         // tile and K split of least cost, as for a single product
         const int nk = (int)(N / BK);
-        int64_t outs[4];
-        for (int i = 0; i < n; ++i) outs[i] = mats[i]->M;
         int ks = 1;
-        const int tile = dma_tile({w_u8, false}, T, nk, n, outs, splitk_ws && m8 ? RWKV_SPLITK_WS_BYTES : 0, &ks);
+        const int tile = group_tile(w_u8, n, T, N, mats, splitk_ws != nullptr, &ks);
         g.nk_split = nk / ks;
         if (ks > 1) {
             float *p = splitk_ws;

@@ -44,8 +44,8 @@ struct GemmEpi {
 };
 
 // How gemm_launch would run a product: kind 0 = the 2..16-row kernel, 1 = register-staged tiles, 2 = direct-to-LDS
-// tiles of tm x tn with K split ks ways.
-struct GemmPlan { int kind, tm, tn, ks; };
+// tiles of tm x tn with K split ks ways; us: what the cost model says of the latter.
+struct GemmPlan { int kind, tm, tn, ks; double us; };
 GemmPlan gemm_plan(bool w_u8, int64_t T, int64_t N, int64_t M, const rwkv_half *A, int64_t lda, const void *W,
                    int64_t ldw, const void *Y, int64_t ldy, const GemmEpi &ep);
 
@@ -58,10 +58,13 @@ int gemm_launch(bool w_u8, int64_t T, int64_t N, int64_t M, const rwkv_half *A, 
 int gemm_group_launch(bool w_u8, int n, int64_t T, int64_t N, const rwkv_half *const *x, const rwkv_mat *const *mats,
                       void *const *Y, const GemmEpi *eps, rwkv_half *const *xs, float *const *sums, float *splitk_ws,
                       hipStream_t st, int parts = 0);
-// true where that launch would go through the direct-to-LDS kernel, which can take the row sums of already scaled
-// inputs as `parts` partial sums per row (GemmEpi::parts)
-bool gemm_group_takes_parts(bool w_u8, int n, int64_t T, int64_t N, const rwkv_half *const *x, const rwkv_mat *const *mats,
-                            void *const *Y);
+// How that launch would run (fp16 outputs, inputs already scaled).  kind 2: it can take the row sums of its inputs as `parts`
+// partial sums per row and, where ks is 1, emit those of its outputs (GemmEpi).
+GemmPlan gemm_group_plan(bool w_u8, int n, int64_t T, int64_t N, const rwkv_half *const *x, const rwkv_mat *const *mats,
+                         void *const *Y, bool may_split);
+// Is that launch the better one, against one launch for each of them?
+bool gemm_group_pays(bool w_u8, int n, int64_t T, int64_t N, const rwkv_half *const *x, const rwkv_mat *const *mats,
+                     void *const *Y, const GemmEpi *eps, float *splitk_ws);
 int mm8_prepare_launch(int64_t T, int64_t N, const rwkv_half *x, int64_t ldx, const rwkv_half *ry,
                        const rwkv_half *my, rwkv_half *xs, float *s0, float *s2, hipStream_t st);
 int gemv_f16_launch(int64_t N, int64_t M, const rwkv_half *x, const rwkv_half *w, int64_t ldw, void *y,

@@ -680,22 +680,42 @@ extern "C" int rwkv_v4_forward_seq(const rwkv_v4_model *m, const rwkv_v4_layer_s
         e = GemmEpi{};
         e.out_scale = 1.f; e.out_dtype = RWKV_DT_F16;
         e.act = ACT_SIGMOID;
+        int vparts = 0;   // > 0: the key product hands the value product its input with this many partial sums per row
+        // the partial sums that a key launch of this plan hands over, 0: the value product's input has a scaling pass
+        auto handed_over = [&](const GemmPlan &pk) {
+            if (!handover_enabled() || pk.kind != 2 || pk.ks != 1) return 0;
+            GemmEpi ev{};
+            ev.out_scale = 1.f; ev.out_dtype = RWKV_DT_F16;
+            ev.act = ACT_GATED_RESIDUAL; ev.gate = ws.r; ev.ldgate = C; ev.res = ws.x; ev.ldres = C;
+            const GemmPlan pv = plan_gemm(l.ffn_value, true, T, ws.xsv, s0v, s2v, ws.x, C, ev, ws.splitk);
+            const int np = (F + pk.tn - 1) / pk.tn;
+            return pv.kind == 2 && np > 1 && !(np & 3) ? np : 0;
+        };
+        auto emit = [&](GemmEpi &k, int np) {
+            if (!np) return;
+            k.emit_ry = l.ffn_value.ry; k.emit_my = l.ffn_value.my;
+            k.emit_s0 = ws.parts; k.emit_s2 = ws.parts + (size_t)T * np;
+        };
+        const rwkv_half *xrk[2] = {ws.xs[0], ws.xs[1]};
+        const rwkv_mat *mrk[2] = {&l.ffn_receptance, &l.ffn_key};
+        void *ork[2] = {ws.r, u8 ? ws.xsv : ws.vx};
+        GemmEpi erk[2] = {e, e};
+        erk[1].act = ACT_RELU_SQ;
+        if ((T <= 128 && !(C & 127) && !(F & 127)) || gemm_group_pays(u8, 2, T, C, xrk, mrk, ork, erk, ws.splitk)) {
+            // Receptance and key in one grouped launch: short calls, and where the cost model puts it first.  8 layers, us, by
+            // the limit of 128 tokens before -> by cost: n_embd 768, fp16, 200 tokens 516 -> 455, 513 635 -> 609; 2048, uint8, 140
+            // tokens 807 -> 726, 513 1388 -> 1305; 4096, uint8, 700 tokens 3814 -> 3396, 256 and 1000 tokens, which stay two launches,
+            // 1647 and 4131 against 1686 and 4334 as one.  The key launch of a group hands over like one of its own (20 to 45 tokens
+            // of 4096 channels, uint8: 957 -> 915).
+            if (u8) vparts = handed_over(gemm_group_plan(true, 2, T, C, xrk, mrk, ork, true));
+            emit(erk[1], vparts);
+            if (!vparts) ork[1] = ws.vx;
+            if ((rc = gemm_group_launch(u8, 2, T, C, xrk, mrk, ork, erk, nullptr, s0, ws.splitk, st))) return rc;
+        } else {
         // the receptance product beside the key product: where neither would split K, and in calls of three row tiles
         // (257 .. 384 tokens: +4 % at n_embd 4096; slower at 256 and from 385 on)
         ForkScope par2(ss, st, 1, !dma_seq && ((T / 128) * (C / 128) > 128 || ((T + 127) / 128 == 3 && C == 4096)));
         float *sk2 = par2 ? nullptr : ws.splitk;
-        int vparts = 0;   // > 0: the key product hands the value product its input with this many partial sums per row
-        if (T <= 128 && !(C & 127) && !(F & 127)) {
-            // Short calls: receptance and key in one grouped launch.  16 layers of n_embd 4096, uint8, ms, one after the other ->
-            // grouped: 160 tokens 3.34 -> 3.28, 200 3.44 -> 3.37, 256 3.52 -> 3.53; fp16 160 tokens 3.42 -> 3.44, 256 3.77 ->
-            // 3.85.  Narrow models would gain beyond the limit (n_embd 768, 256 tokens 1.25 -> 1.12): it is set by the wide ones.
-            const rwkv_half *xin[2] = {ws.xs[0], ws.xs[1]};
-            const rwkv_mat *mats[2] = {&l.ffn_receptance, &l.ffn_key};
-            void *outs[2] = {ws.r, ws.vx};
-            GemmEpi ep[2] = {e, e};
-            ep[1].act = ACT_RELU_SQ;
-            if ((rc = gemm_group_launch(u8, 2, T, C, xin, mats, outs, ep, nullptr, s0, ws.splitk, st))) return rc;
-        } else {
         // uint8: the three-stage tile for both, so that one of each fits a CU (2 x 73 KB; the four-stage tile that the
         // receptance product gets by itself takes 97: 4.89 ms against 4.82 for 16 layers of n_embd 4096 at 257 tokens, 5.15
         // against 5.07 at 384).  Two fp16 tiles fit no CU with either: 4.85 four-stage, 4.91 three-stage at 257.
@@ -706,19 +726,8 @@ extern "C" int rwkv_v4_forward_seq(const rwkv_v4_model *m, const rwkv_v4_layer_s
         // Where the key product runs at full depth through the direct-to-LDS kernel and the value product through that
         // kernel too, the key product's epilogue writes relu(k)^2 already scaled for the value product, with the row
         // sums as one partial sum per column tile: no scaling pass, and the unscaled [T, F] activation is never stored.
-        if (u8 && handover_enabled()) {
-            const GemmPlan pk = plan_gemm(l.ffn_key, true, T, ws.xs[1], s0[1], s2[1], ws.xsv, F, e, sk2);
-            GemmEpi ev{};
-            ev.out_scale = 1.f; ev.out_dtype = RWKV_DT_F16;
-            ev.act = ACT_GATED_RESIDUAL; ev.gate = ws.r; ev.ldgate = C; ev.res = ws.x; ev.ldres = C;
-            const GemmPlan pv = plan_gemm(l.ffn_value, true, T, ws.xsv, s0v, s2v, ws.x, C, ev, ws.splitk);
-            const int np = pk.kind == 2 ? (F + pk.tn - 1) / pk.tn : 0;
-            if (pk.kind == 2 && pk.ks == 1 && pv.kind == 2 && np > 1 && !(np & 3)) {
-                vparts = np;
-                e.emit_ry = l.ffn_value.ry; e.emit_my = l.ffn_value.my;
-                e.emit_s0 = ws.parts; e.emit_s2 = ws.parts + (size_t)T * np;
-            }
-        }
+        if (u8) vparts = handed_over(plan_gemm(l.ffn_key, true, T, ws.xs[1], s0[1], s2[1], ws.xsv, F, e, sk2));
+        emit(e, vparts);
         if ((rc = run_gemm(l.ffn_key, u8, T, ws.xs[1], s0[1], s2[1], vparts ? ws.xsv : ws.vx, F, e, st, sk2))) return rc;
         e.small_tiles = 0;
         e.emit_ry = e.emit_my = nullptr; e.emit_s0 = e.emit_s2 = nullptr;

@@ -390,7 +390,7 @@ extern "C" int rwkv_v56_forward(const rwkv_v56_model *m, const rwkv_v56_layer_st
                 const rwkv_half *xin[4] = {ws.mix[3], ws.mix[1], ws.mix[2], ws.mix[4]};
                 const rwkv_mat *mats[4] = {&l.att_receptance, &l.att_key, &l.att_value, &l.att_gate};
                 void *outs[4] = {ws.r, ws.k, ws.v, ws.g};
-                if (gemm_group_takes_parts(true, 4, T, C, xin, mats, outs)) {
+                if (gemm_group_plan(true, 4, T, C, xin, mats, outs, true).kind == 2) {
                     att_np = mix_parts(C);
                     const rwkv_mat *mj[5] = {nullptr, &l.att_key, &l.att_value, &l.att_receptance, &l.att_gate};
                     b.npart = att_np;
@@ -520,18 +520,30 @@ extern "C" int rwkv_v56_forward(const rwkv_v56_model *m, const rwkv_v56_layer_st
             }
             if ((rc = lnmix_seq_launch(a, 2, st))) return rc;
         }
-        if (T <= 128 && !(C & 127) && !(F & 127)) {
-            // Short calls: receptance and key in one grouped launch.  16 layers, ms, one after the other -> grouped: RWKV-6,
-            // n_embd 4096, uint8, 160 tokens 4.12 -> 4.16, 256 4.41 -> 4.44, 320 6.09 -> 5.73, 511 6.97 -> 7.03.  Narrow models
-            // would gain up to 333 (n_embd 2048, fp16, 256 tokens 2.17 -> 2.01, 448 2.56 -> 2.68): the limit is set by the wide ones.
-            const rwkv_half *xin[2] = {fx[0], fx[1]};
-            const rwkv_mat *mats[2] = {&l.ffn_receptance, &l.ffn_key};
-            void *outs[2] = {ws.r, ws.vx};
-            GemmEpi ep[2] = {};
-            ep[0].act = ACT_SIGMOID; ep[1].act = ACT_RELU_SQ;
-            for (int j = 0; j < 2; ++j) { ep[j].out_scale = 1.f; ep[j].out_dtype = RWKV_DT_F16; }
-            if ((rc = gemm_group_launch(u8, 2, T, C, xin, mats, outs, ep, nullptr, fs, ws.splitk, st))) return rc;
-            if ((rc = mm(c, l.ffn_value, u8, ws.vx, ACT_GATED_RESIDUAL, ws.x, ws.r, scale, ws.x))) return rc;
+        const rwkv_half *xrk[2] = {fx[0], fx[1]};
+        const rwkv_mat *mrk[2] = {&l.ffn_receptance, &l.ffn_key};
+        void *ork[2] = {ws.r, u8 ? ws.xs : ws.vx};
+        GemmEpi erk[2] = {};
+        erk[0].act = ACT_SIGMOID; erk[1].act = ACT_RELU_SQ;
+        for (int j = 0; j < 2; ++j) { erk[j].out_scale = 1.f; erk[j].out_dtype = RWKV_DT_F16; }
+        if ((T <= 128 && !(C & 127) && !(F & 127)) || gemm_group_pays(u8, 2, T, C, xrk, mrk, ork, erk, ws.splitk)) {
+            // Receptance and key in one grouped launch: short calls, and where the cost model puts it first.  The key product
+            // hands the value product its input scaled where it can.  8 layers, us, by the limit of 128 tokens before -> by
+            // cost: RWKV-5.2, n_embd 2048, fp16, 140 tokens 891 -> 813, 333 1070 -> 1012; RWKV-6, 4096, uint8, 333 tokens 2929 ->
+            // 2757, 200 and 1000 tokens, which stay two launches, 1951 and 5100 against 2032 and 5330 as one.
+            int np = 0;
+            if (u8)
+                np = mm_pair_parts(gemm_group_plan(true, 2, T, C, xrk, mrk, ork, true), c, l.ffn_key, l.ffn_value, true, ACT_GATED_RESIDUAL,
+                                   ws.x, ws.r, ws.x, ws.parts);
+            if (np) {
+                erk[1].emit_ry = l.ffn_value.ry; erk[1].emit_my = l.ffn_value.my;
+                erk[1].emit_s0 = ws.parts; erk[1].emit_s2 = ws.parts + (size_t)T * np;
+            } else {
+                ork[1] = ws.vx;
+            }
+            if ((rc = gemm_group_launch(u8, 2, T, C, xrk, mrk, ork, erk, nullptr, fs, ws.splitk, st))) return rc;
+            if ((rc = mm_pair_second(c, l.ffn_key, l.ffn_value, u8, ws.vx, ACT_GATED_RESIDUAL, ws.x, ws.r, scale, ws.x, ws.parts, np)))
+                return rc;
         } else {
             // channel-mix receptance beside the key product (one after the other in long calls); the key product
             // hands the value product its input already scaled where both run through the direct-to-LDS kernel
