@@ -18,6 +18,8 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 #define DEV __device__ __forceinline__
 
+constexpr float LN_EPS = 1e-5f;   // LayerNorm
+
 // ---- launch bookkeeping -------------------------------------------------------------------
 #define RWKV_LAUNCH_CHECK()                         \
     do {                                            \

@@ -16,7 +16,6 @@ namespace {
 
 constexpr int DTHREADS = 1024;
 constexpr int DWAVES = DTHREADS / 64;
-constexpr float LN_EPS = 1e-5f;
 constexpr int VP = 4;  // most 8-element groups per thread the vector prologue keeps in registers (N <= 32768)
 
 // x for this step: the embedding row of the token (first layer) or the running activation.  The id comes

@@ -10,10 +10,9 @@
 #include <cstdlib>
 #include <mutex>
 #include "kernels.h"
+#include "rows.h"
 
 namespace {
-
-constexpr float LN_EPS = 1e-5f;
 
 // ids outside [0, vocab) are clamped to the nearest valid row: a bad id never becomes an out-of-bounds read
 __global__ __launch_bounds__(256) void gather_emb_kernel(int T, int C, int vocab, const int32_t *__restrict__ tokens,
@@ -30,72 +29,6 @@ __global__ __launch_bounds__(256) void copy16_kernel(int n16, const u32x4 *__res
     if (i < n16) dst[i] = src[i];
 }
 
-// ---- LayerNorm and mix, eight channels at a time ----------------------------------------------------------------
-// Long calls are bound by vector-instruction issue, so each step is the fewest instructions that form the same value:
-// sums take two channels per v_dot2_f32_f16 (exact products with 1, fp32 accumulation, subnormals kept), x - mean reads
-// its fp16 operand in place (v_fma_mix_f32 with 1.0: one rounding, as the conversion and subtraction), the affine and the
-// mixes end in v_fma_mix{lo,hi}_f16.  The compiler takes three to four instructions for each of these.
-DEV h16x2 pair(h16x8 v, int p) { return h16x2{v[2 * p], v[2 * p + 1]}; }
-DEV float dot8(h16x8 v, h16x8 w, float a) {
-#pragma unroll
-    for (int p = 0; p < 4; ++p) a = __builtin_amdgcn_fdot2(pair(v, p), pair(w, p), a, false);
-    return a;
-}
-DEV float sum8(h16x8 v, float a) {
-    const h16 one = (h16)1.f;
-    return dot8(v, h16x8{one, one, one, one, one, one, one, one}, a);
-}
-DEV void less_mean8(h16x8 v, float mean, float (&d)[8]) {
-#pragma unroll
-    for (int p = 0; p < 4; ++p) {
-        asm("v_fma_mix_f32 %0, %1, 1.0, -%2 op_sel_hi:[1,0,0]" : "=v"(d[2 * p]) : "v"(pair(v, p)), "v"(mean));
-        asm("v_fma_mix_f32 %0, %1, 1.0, -%2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(d[2 * p + 1]) : "v"(pair(v, p)), "v"(mean));
-    }
-}
-DEV float squares8(const float (&d)[8], float a) {
-#pragma unroll
-    for (int e = 0; e < 8; ++e) a = __builtin_fmaf(d[e], d[e], a);
-    return a;
-}
-// fp16(fma(t, w, b)) of two channels
-DEV h16x2 fma_pair(float t0, float t1, h16x2 w, h16x2 b) {
-    h16x2 r;
-    asm("v_fma_mixlo_f16 %0, %1, %3, %4 op_sel_hi:[0,1,1]\n\tv_fma_mixhi_f16 %0, %2, %3, %4 op_sel:[0,1,1] op_sel_hi:[0,1,1]"
-        : "=&v"(r) : "v"(t0), "v"(t1), "v"(w), "v"(b));
-    return r;
-}
-DEV h16x8 join8(const h16x2 (&q)[4]) { return h16x8{q[0].x, q[0].y, q[1].x, q[1].y, q[2].x, q[2].y, q[3].x, q[3].y}; }
-DEV h16x8 norm8(const float (&d)[8], float rstd, h16x8 w, h16x8 b) {
-    h16x2 q[4];
-#pragma unroll
-    for (int p = 0; p < 4; ++p) q[p] = fma_pair(d[2 * p] * rstd, d[2 * p + 1] * rstd, pair(w, p), pair(b, p));
-    return join8(q);
-}
-// What all mixes of a token share: xx - prev in fp32 (RWKV-4, 5), or prev - xx in fp16 (RWKV-6, 7: maa_form).
-struct Shift8 { float d[8]; h16x8 d16; };
-DEV Shift8 shift8(h16x8 xx, h16x8 prev, bool maa_form) {
-    Shift8 s = {};
-    if (maa_form) s.d16 = prev - xx;
-    else
-#pragma unroll
-        for (int p = 0; p < 4; ++p) {
-            asm("v_fma_mix_f32 %0, %1, 1.0, -%2 op_sel_hi:[1,0,1]" : "=v"(s.d[2 * p]) : "v"(pair(xx, p)), "v"(pair(prev, p)));
-            asm("v_fma_mix_f32 %0, %1, 1.0, -%2 op_sel:[1,0,1] op_sel_hi:[1,0,1]" : "=v"(s.d[2 * p + 1]) : "v"(pair(xx, p)), "v"(pair(prev, p)));
-        }
-    return s;
-}
-// xx m + prev (1 - m) as fp16(prev + (xx - prev) m): one rounding after the difference, which is exact but for the last bits
-// of operands that differ by more than 2^13.  maa_form: xx + (prev - xx) m, the difference rounded to fp16.
-DEV h16x8 mix8(h16x8 xx, h16x8 prev, const Shift8 &s, h16x8 m, bool maa_form) {
-    if (maa_form) return __builtin_elementwise_fma(s.d16, m, xx);
-    h16x2 q[4];
-#pragma unroll
-    for (int p = 0; p < 4; ++p) q[p] = fma_pair(s.d[2 * p], s.d[2 * p + 1], pair(m, p), pair(prev, p));
-    return join8(q);
-}
-DEV float row_mean(float sum, int C) { return sum / C; }
-DEV float row_rstd(float squares, int C) { return rsqrtf(squares / C + LN_EPS); }
-
 DEV void row_stats(const rwkv_half *x, int C, float *red, float &mean, float &rstd) {
     float s = 0.f;
     for (int j8 = threadIdx.x; j8 < (C >> 3); j8 += blockDim.x) s = sum8(*(const h16x8 *)(x + 8 * j8), s);
@@ -103,7 +36,7 @@ DEV void row_stats(const rwkv_half *x, int C, float *red, float &mean, float &rs
     float q = 0.f, d[8];
     for (int j8 = threadIdx.x; j8 < (C >> 3); j8 += blockDim.x) {
         less_mean8(*(const h16x8 *)(x + 8 * j8), mean, d);
-        q = squares8(d, q);
+        q = j8 < (int)blockDim.x ? squares8<true>(d, q) : squares8<false>(d, q);
     }
     rstd = row_rstd(block_sum(q, red), C);
 }
@@ -179,43 +112,6 @@ __global__ __launch_bounds__(256) void ln_f32_f16_kernel(int C, const float *__r
     for (int j = threadIdx.x; j < C; j += blockDim.x) y[j] = f2h((x[j] - mean) * rstd * w[j] + b[j]);
 }
 
-// K sums over a row whose 8-wide chunks are dealt to 256 threads, chunk v, v + 256, ... to thread v, each thread adding up
-// its own in that order: add(v) adds this thread's chunks to v.  With 512 threads the second 256 hold the later half of
-// those chunks and go on, through LDS, from where the first left off: the same additions in the same order, so the
-// totals are the same bits with either number of threads.  v starts at zero; red: 4 K floats of these sums' own, 16-byte
-// aligned; hop: K * 256 floats (512 threads only).
-template <int K, int NT, class Add>
-DEV void row_sums(float (&v)[K], float *red, float *hop, Add add) {
-    static_assert(NT == 256 || NT == 512, "two threads per chain at most");
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    if constexpr (NT == 512) {
-        const int chain = threadIdx.x & 255;
-        if (wave < 4) {
-            add(v);
-#pragma unroll
-            for (int k = 0; k < K; ++k) hop[k * 256 + chain] = v[k];
-        }
-        __syncthreads();
-        if (wave >= 4)
-#pragma unroll
-            for (int k = 0; k < K; ++k) v[k] = hop[k * 256 + chain];
-    }
-    if (NT == 256 || wave >= 4) {
-        add(v);
-#pragma unroll
-        for (int k = 0; k < K; ++k) v[k] = wave_sum_lane63(v[k]);
-        if ((threadIdx.x & 63) == 63)
-#pragma unroll
-            for (int k = 0; k < K; ++k) red[k * 4 + (wave & 3)] = v[k];
-    }
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < K; ++k) {
-        const f32x4 r = *(const f32x4 *)(red + 4 * k);
-        v[k] = ((r[0] + r[1]) + r[2]) + r[3];
-    }
-}
-
 // lnmix_seq_kernel with a short dependent chain, for C <= 8 NT CH: a thread's chunks of the row, of the previous row
 // and of the LayerNorm vectors are requested together at the top and kept in registers, the statistics of the two
 // rows share their barriers, and so do the 2 NJ sums at the end: two global round trips and three rounds of
@@ -256,7 +152,7 @@ __global__ __launch_bounds__(NT) void lnmix_seq_fast_kernel(SeqMixArgs a) {
         }
     }
     float st[3] = {0.f, 0.f, 0.f};
-    row_sums<3, NT>(st, red, hop, [&](float (&v)[3]) {
+    row_sums<3, NT>(st, red, hop, [&](float (&v)[3], auto) {
 #pragma unroll
         for (int c = 0; c < CH; ++c)
             if (j8_0 + c * 256 < nch) {
@@ -268,18 +164,19 @@ __global__ __launch_bounds__(NT) void lnmix_seq_fast_kernel(SeqMixArgs a) {
     const float mean = row_mean(st[0], C), pmean = row_mean(st[1], C), lmean = row_mean(st[2], C);
     float dx[CH][8], dp[CH][8];
     st[0] = st[1] = st[2] = 0.f;
-    row_sums<3, NT>(st, red + 12, hop, [&](float (&v)[3]) {
+    row_sums<3, NT>(st, red + 12, hop, [&](float (&v)[3], auto first) {
+        constexpr bool FIRST = decltype(first)::value;
 #pragma unroll
         for (int c = 0; c < CH; ++c) {
             less_mean8(xv[c], mean, dx[c]);
             less_mean8(pxv[c], pmean, dp[c]);
             if (j8_0 + c * 256 < nch) {
-                v[0] = squares8(dx[c], v[0]);
-                v[1] = squares8(dp[c], v[1]);
+                v[0] = FIRST && c == 0 ? squares8<true>(dx[c], v[0]) : squares8<false>(dx[c], v[0]);
+                v[1] = FIRST && c == 0 ? squares8<true>(dp[c], v[1]) : squares8<false>(dp[c], v[1]);
                 if (commit) {   // the last row's statistics: only the workgroup that writes the new state needs them
                     float dl[8];
                     less_mean8(lv[c], lmean, dl);
-                    v[2] = squares8(dl, v[2]);
+                    v[2] = FIRST && c == 0 ? squares8<true>(dl, v[2]) : squares8<false>(dl, v[2]);
                 }
             }
         }
@@ -340,7 +237,7 @@ __global__ __launch_bounds__(NT) void lnmix_seq_fast_kernel(SeqMixArgs a) {
 #pragma unroll
     for (int j = 0; j < NJ; ++j) any = any || a.ry[j];
     if (any) {
-        row_sums<2 * NJ, NT>(acc, red + 24, hop, [&](float (&v)[2 * NJ]) {
+        row_sums<2 * NJ, NT>(acc, red + 24, hop, [&](float (&v)[2 * NJ], auto) {
             if constexpr (NT > 256)
 #pragma unroll
                 for (int c = 0; c < CH; ++c)

@@ -11,10 +11,9 @@
 // mm(): T == 1 -> streaming GEMV (vec_kernel: ry scaling and the row sums in its prologue,
 // activation / residual in its epilogue); T > 1 -> mm8_prepare + MFMA GEMM with the same epilogues.
 #include "mm_dispatch.h"
+#include "rows.h"
 
 namespace {
-
-constexpr float LN_EPS56 = 1e-5f;
 
 struct Mix1Args {
     int T, C;
@@ -22,75 +21,79 @@ struct Mix1Args {
     rwkv_half *xx, *sxd, *xxx, *state_out;   // state_out: the token-shift state (may be sx)
 };
 
-// grid T x 256 threads: xx = LN1(x[t]); sxd = prev - xx; xxx = xx + sxd * maa_x.
-// Rows of up to 2048 CH channels keep a thread's chunks of the row and of the previous row in registers from one round
-// of loads, and the four sums of the two rows' statistics share one pair of barriers.
-template <int CH>
-__global__ __launch_bounds__(256) void v6_mix1_kernel(Mix1Args a) {
-    __shared__ float red[24];
+// One workgroup per row, NT threads: xx = LN1(x[t]); sxd = prev - xx; xxx = xx + sxd * maa_x (rows.h).  A thread's
+// chunks of the row and of the previous row stay in registers from one round of loads, and the four sums of the two rows'
+// statistics share their barriers.
+template <int CH, int NT>
+__global__ __launch_bounds__(NT) void v6_mix1_kernel(Mix1Args a) {
+    __shared__ __align__(16) float red[24];
+    __shared__ float hop[NT == 512 ? 256 * 6 : 1];
     const int t = blockIdx.x, C = a.C, nch = C >> 3;
+    const int j8_0 = NT == 256 ? (int)threadIdx.x : (int)(threadIdx.x & 255) + 256 * CH * (int)(threadIdx.x >> 8);
     const rwkv_half *x = a.x + (size_t)t * C;
     const rwkv_half *xp = t > 0 ? x - C : x;
     // row 0's workgroup also forms the new token-shift state LN1(x[T-1]); its statistics ride in the same barriers
     const bool commit = t == 0;
     const rwkv_half *xl = commit ? a.x + (size_t)(a.T - 1) * C : x;
-    h16x8 xr[CH], pr[CH], lr[CH];
+    h16x8 xv[CH], pxv[CH], lv[CH], wv[CH], bv[CH], mv[CH];
 #pragma unroll
     for (int c = 0; c < CH; ++c) {
-        const int j8 = min((int)threadIdx.x + c * 256, nch - 1);   // chunks past the end repeat the last one (unused)
-        xr[c] = *(const h16x8 *)(x + 8 * j8);
-        pr[c] = *(const h16x8 *)(xp + 8 * j8);
-        lr[c] = *(const h16x8 *)(xl + 8 * j8);
+        const int j8 = min(j8_0 + c * 256, nch - 1);   // chunks past the end repeat the last one (unused)
+        xv[c] = *(const h16x8 *)(x + 8 * j8);
+        pxv[c] = *(const h16x8 *)(xp + 8 * j8);
+        lv[c] = *(const h16x8 *)(xl + 8 * j8);
+        wv[c] = *(const h16x8 *)(a.ln_w + 8 * j8);
+        bv[c] = *(const h16x8 *)(a.ln_b + 8 * j8);
+        mv[c] = *(const h16x8 *)(a.maa_x + 8 * j8);
     }
     float sq[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};   // sum and sum of squares of the row, the previous row, the last row
+    row_sums<6, NT>(sq, red, hop, [&](float (&v)[6], auto) {
 #pragma unroll
-    for (int c = 0; c < CH; ++c)
-        if ((int)threadIdx.x + c * 256 < nch) {
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const float f = (float)xr[c][e], g = (float)pr[c][e], h = (float)lr[c][e];
-                sq[0] += f; sq[1] += f * f; sq[2] += g; sq[3] += g * g; sq[4] += h; sq[5] += h * h;
+        for (int c = 0; c < CH; ++c)
+            if (j8_0 + c * 256 < nch) {
+                sum_and_squares8(xv[c], v[0], v[1]);
+                sum_and_squares8(pxv[c], v[2], v[3]);
+                if (commit) sum_and_squares8(lv[c], v[4], v[5]);
             }
-        }
-    block_sum_n<6>(sq, red);
-    const float mean = sq[0] / C, rstd = rsqrtf(fmaxf(sq[1] / C - mean * mean, 0.f) + LN_EPS56);
-    const float pmean = sq[2] / C, prstd = rsqrtf(fmaxf(sq[3] / C - pmean * pmean, 0.f) + LN_EPS56);
-    const float lmean = sq[4] / C, lrstd = rsqrtf(fmaxf(sq[5] / C - lmean * lmean, 0.f) + LN_EPS56);
+    });
+    const float mean = sq[0] / C, rstd = rsqrtf(fmaxf(sq[1] / C - mean * mean, 0.f) + LN_EPS);
+    const float pmean = sq[2] / C, prstd = rsqrtf(fmaxf(sq[3] / C - pmean * pmean, 0.f) + LN_EPS);
+    const float lmean = sq[4] / C, lrstd = rsqrtf(fmaxf(sq[5] / C - lmean * lmean, 0.f) + LN_EPS);
+    float d[8];
 #pragma unroll
     for (int c = 0; c < CH; ++c) {
-        const int j8 = threadIdx.x + c * 256;
+        const int j8 = j8_0 + c * 256;
         if (j8 >= nch) break;
-        const h16x8 xv = xr[c];
-        const h16x8 wv = *(const h16x8 *)(a.ln_w + 8 * j8), bv = *(const h16x8 *)(a.ln_b + 8 * j8);
-        const h16x8 mv = *(const h16x8 *)(a.maa_x + 8 * j8);
-        h16x8 xx, pv, sd, xo;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) xx[e] = (h16)(((float)xv[e] - mean) * rstd * (float)wv[e] + (float)bv[e]);
+        less_mean8(xv[c], mean, d);
+        const h16x8 xx = norm8(d, rstd, wv[c], bv[c]);
+        h16x8 pv;
         if (t > 0) {
-            const h16x8 pxv = pr[c];
-#pragma unroll
-            for (int e = 0; e < 8; ++e) pv[e] = (h16)(((float)pxv[e] - pmean) * prstd * (float)wv[e] + (float)bv[e]);
+            less_mean8(pxv[c], pmean, d);
+            pv = norm8(d, prstd, wv[c], bv[c]);
         } else {
             pv = *(const h16x8 *)(a.sx + 8 * j8);
         }
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            sd[e] = (h16)((float)pv[e] - (float)xx[e]);
-            xo[e] = (h16)((float)xx[e] + (float)(h16)((float)sd[e] * (float)mv[e]));
-        }
+        const Shift8 sh = shift8(xx, pv, true);
         const size_t o = (size_t)t * C + 8 * j8;
         *(h16x8 *)(a.xx + o) = xx;
-        *(h16x8 *)(a.sxd + o) = sd;
-        *(h16x8 *)(a.xxx + o) = xo;
+        *(h16x8 *)(a.sxd + o) = sh.d16;
+        *(h16x8 *)(a.xxx + o) = mix8(xx, pv, sh, mv[c], true);
         // the new token-shift state: written by row 0's workgroup, the only one that reads the old state, each thread
         // exactly the chunk it has just read
         if (commit) {
-            h16x8 ls;
-#pragma unroll
-            for (int e = 0; e < 8; ++e) ls[e] = (h16)(((float)lr[c][e] - lmean) * lrstd * (float)wv[e] + (float)bv[e]);
-            *(h16x8 *)(a.state_out + 8 * j8) = ls;
+            less_mean8(lv[c], lmean, d);
+            *(h16x8 *)(a.state_out + 8 * j8) = norm8(d, lrstd, wv[c], bv[c]);
         }
     }
+}
+// 256 or 512 threads per row as in lnmix_seq_launch.  us, 256 rows of 4096 channels: 7.2 -> 5.4 with
+// the element code of rows.h.
+void v6_mix1_launch(const Mix1Args &a, hipStream_t st) {
+    const bool few = a.T <= 512;
+    const auto kernel = a.C <= 2048   ? v6_mix1_kernel<1, 256>
+                        : a.C <= 4096 ? (few ? v6_mix1_kernel<1, 512> : v6_mix1_kernel<2, 256>)
+                                      : (few ? v6_mix1_kernel<2, 512> : v6_mix1_kernel<4, 256>);
+    hipLaunchKernelGGL(kernel, dim3((unsigned)a.T), dim3(few && a.C > 2048 ? 512 : 256), 0, st, a);
 }
 
 struct Mix2Args {
@@ -101,16 +104,16 @@ struct Mix2Args {
     const rwkv_half *prev;           // [C] token-shift state
     const rwkv_half *maa[5];         // w, k, v, r, g
     rwkv_half *out[5];               // [T, C] each
-    // v6_mix2x4_kernel, uint8 matrices: ry[j] != NULL: out[j] is stored as fp16(mix * ry[j]), the input of matrix j's
-    // product, and the sums of mix and mix * my[j] over each block of 1024 channels go to p0[j] / p2[j] [T][npart]
+    // v6_mix2_mfma_kernel, uint8 matrices: ry[j] != NULL: out[j] is stored as fp16(mix * ry[j]), the input of matrix j's
+    // product, and the sums of mix and mix * my[j] over each block of 256 channels go to p0[j] / p2[j] [T][npart]
     // (npart = the number of blocks rounded up to a multiple of four, the padding entries zero)
     const rwkv_half *ry[5], *my[5];
     float *p0[5], *p2[5];
     int npart;
 };
 
-// grid (ceil(T / 16), C/256, 5): m_j[c] = sum_i t1[t, jR + i] * w2[j][i][c]; out_j = xx + sxd * (maa_j + m_j).
-// One (channel, mix) per thread for a tile of MIX2_TT tokens (16, or 1 for a one-token call): the R coefficients of the channel are loaded once
+// grid (ceil(T / MIX2_TT), C/256, 5): m_j[c] = sum_i t1[t, jR + i] * w2[j][i][c]; out_j = xx + sxd * (maa_j + m_j).
+// One (channel, mix) per thread for a tile of MIX2_TT tokens (4, or 1 for a one-token call): the R coefficients of the channel are loaded once
 // and reused for every token of the tile; the sum runs in index order.
 template <int MIX2_TT>
 __global__ __launch_bounds__(256) void v6_mix2_kernel(Mix2Args a) {
@@ -151,86 +154,110 @@ __global__ __launch_bounds__(256) void v6_mix2_kernel(Mix2Args a) {
     }
 }
 
-// The same sums for sequence calls with four adjacent channels per thread: grid (ceil(T / TT), ceil(C / 1024), 5), TT
-// tokens per workgroup (16, or 4 in short calls, which would otherwise have too few workgroups for the chip).  The
-// coefficient, xx, sxd and output accesses are 8 bytes per lane instead of 2, and one LDS read of four tokens' t1
-// serves four channels; every channel's sum still runs in index order, so the results equal v6_mix2_kernel's.
-template <int TT>
-__global__ __launch_bounds__(256) void v6_mix2x4_kernel(Mix2Args a) {
-    __shared__ __align__(16) float st1[64][TT];
-    const int t0 = blockIdx.x * TT, c = (blockIdx.y * 256 + threadIdx.x) * 4, j = blockIdx.z, R = a.R, C = a.C;
-    const int nt = min(TT, a.T - t0);
-    for (int i = threadIdx.x; i < TT * R; i += 256) {
-        const int tt = i / R, r = i - tt * R;
-        st1[r][tt] = tt < nt ? h2f(a.t1[(size_t)(t0 + tt) * 5 * R + j * R + r]) : 0.f;
+// The same for sequence calls, on the matrix cores: 16 tokens x 64 channels per wave, four waves side by side, the R (8 to 64)
+// coefficients of a mix as one or two v_mfma_f32_16x16x32_f16 per 16 channels (fp16 operands, fp32 sums; k's past R are zero in
+// both).  w2 is [R][C], so a block's coefficients pass through LDS, two k's of a channel to a word (rows of 16 KS + 2 words: two
+// lanes to a bank when written, none when read).  Row r of the MFMA of block b is channel 16 (r / 4) + 4 b + r % 4 of the wave's
+// 64, so that a lane ends with 16 adjacent channels of one token and four lanes cover a 128-byte line.  All of a workgroup's
+// loads are requested at the top.  grid (ceil(T / 16), ceil(C / 256), 5): all five mixes in one workgroup, which reads xx and sxd
+// once, is 0.5 % of a call faster at 1000 tokens and 3 % slower up to 45.
+// The form before multiplied on the vector units, 4 or 16 tokens x 4 channels per thread, and was bound by their issue.  us, 4096
+// channels, rank 32, uint8 (scaled, with sums), 256 tokens: 15.9 -> 11.1; 6 % of a call of 513 tokens.
+template <int KS>
+__global__ __launch_bounds__(256) void v6_mix2_mfma_kernel(Mix2Args a) {
+    constexpr int ROW = 32 * KS + 4;                                     // halves of a channel's row
+    __shared__ __align__(16) h16 sw[256 * ROW];
+    __shared__ float red[2][4][16];
+    const int C = a.C, R = a.R, t0 = blockIdx.x * 16, j = blockIdx.z;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), n = lane & 15, q = lane >> 4;
+    const int cb = blockIdx.y * 256;                                     // C % 64 == 0: a wave's channels are all there or none
+    const bool live = cb + 64 * wave < C, scaled = a.ry[j] != nullptr;   // scaled: the same for the whole workgroup
+    const int c = live ? cb + 64 * wave + 16 * q : 0;                    // this lane's first channel
+    const int t = min(t0 + n, a.T - 1);
+    const size_t o = (size_t)t * C + c;
+    // coefficients: thread (pair kp of k's, group g of 8 channels) of this workgroup's 256
+    const int kp = threadIdx.x & 7, g = threadIdx.x >> 3, cg = min(cb + 8 * g, C - 8);
+    h16x8 wr[2 * KS][2], tf[KS], mv[2], rv[2] = {}, yv[2] = {}, xx[2], sd[2];
+#pragma unroll
+    for (int i = 0; i < 2 * KS; ++i)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const int k = 2 * (kp + 8 * i) + h;                          // rows past R: loaded from row 0, zeroed below
+            wr[i][h] = *(const h16x8 *)(a.w2 + ((size_t)j * R + (k < R ? k : 0)) * C + cg);
+        }
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+        const int k = 32 * s + 8 * q;
+        tf[s] = *(const h16x8 *)(a.t1 + (size_t)t * 5 * R + j * R + (k < R ? k : 0));
+    }
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+        xx[p] = *(const h16x8 *)(a.xx + o + 8 * p);
+        sd[p] = *(const h16x8 *)(a.sxd + o + 8 * p);
+        mv[p] = *(const h16x8 *)(a.maa[j] + c + 8 * p);
+        if (scaled) { rv[p] = *(const h16x8 *)(a.ry[j] + c + 8 * p); yv[p] = *(const h16x8 *)(a.my[j] + c + 8 * p); }
+    }
+#pragma unroll
+    for (int i = 0; i < 2 * KS; ++i) {
+        const bool in = 2 * (kp + 8 * i) < R;                            // R % 8 == 0
+#pragma unroll
+        for (int e = 0; e < 8; ++e) *(h16x2 *)(sw + (8 * g + e) * ROW + 2 * (kp + 8 * i)) = in ? h16x2{wr[i][0][e], wr[i][1][e]} : h16x2{};
     }
     __syncthreads();
-    const bool scaled = a.ry[j] != nullptr;   // the same for the whole workgroup
-    if (c >= C && !scaled) return;
-    const bool live = c < C;
-    const int cl = live ? c : 0;              // channels past the end take part in the sums with zeros
-    const h16x4 maa = *(const h16x4 *)(a.maa[j] + cl);
-    const rwkv_half *w = a.w2 + (size_t)j * R * C + cl;
-    f32x4 m[TT];
+    f32x4 acc[4];
 #pragma unroll
-    for (int tt = 0; tt < TT; ++tt) m[tt] = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (int i0 = 0; i0 < R; i0 += 8) {
-        h16x4 wv[8];
+    for (int b = 0; b < 4; ++b) {
+        acc[b] = f32x4{0.f, 0.f, 0.f, 0.f};
+        const h16 *row = sw + (64 * wave + 16 * (n >> 2) + 4 * b + (n & 3)) * ROW + 8 * q;
 #pragma unroll
-        for (int i = 0; i < 8; ++i) wv[i] = *(const h16x4 *)(w + (size_t)(i0 + i) * C);   // R is a multiple of 8
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const f32x4 wf = {(float)wv[i][0], (float)wv[i][1], (float)wv[i][2], (float)wv[i][3]};
-#pragma unroll
-            for (int q = 0; q < TT / 4; ++q) {
-                const f32x4 s4 = *(const f32x4 *)&st1[i0 + i][4 * q];
-                m[4 * q + 0] += s4[0] * wf;
-                m[4 * q + 1] += s4[1] * wf;
-                m[4 * q + 2] += s4[2] * wf;
-                m[4 * q + 3] += s4[3] * wf;
-            }
+        for (int s = 0; s < KS; ++s) {
+            const h16x4 lo = *(const h16x4 *)(row + 32 * s), hi = *(const h16x4 *)(row + 32 * s + 4);
+            acc[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(h16x8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]},
+                                                           32 * s + 8 * q < R ? tf[s] : h16x8{}, acc[b], 0, 0, 0);
         }
     }
-    h16x4 ry4 = {}, my4 = {};
-    if (scaled) { ry4 = *(const h16x4 *)(a.ry[j] + cl); my4 = *(const h16x4 *)(a.my[j] + cl); }
-    float sums[2 * TT];
+    float a0 = 0.f, a2 = 0.f;
 #pragma unroll
-    for (int tt = 0; tt < TT; ++tt) {
-        const size_t o = (size_t)(t0 + min(tt, nt - 1)) * C + cl;
-        const h16x4 xx4 = *(const h16x4 *)(a.xx + o), sd4 = *(const h16x4 *)(a.sxd + o);
-        h16x4 out4;
-        float a0 = 0.f, a2 = 0.f;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const float xx = (float)xx4[e];
-            const float mm = round_h((float)maa[e] + round_h(m[tt][e]));
-            out4[e] = (h16)(xx + round_h((float)sd4[e] * mm));
-            if (scaled) {
-                const float kf = (float)out4[e];
-                out4[e] = (h16)(kf * (float)ry4[e]);
-                a0 += kf;
-                a2 += kf * (float)my4[e];
-            }
+    for (int p = 0; p < 2; ++p) {
+        const f32x4 u = acc[2 * p], v = acc[2 * p + 1];
+        const h16x8 m = {(h16)u[0], (h16)u[1], (h16)u[2], (h16)u[3], (h16)v[0], (h16)v[1], (h16)v[2], (h16)v[3]};
+        h16x8 k = __builtin_elementwise_fma(sd[p], mv[p] + m, xx[p]);
+        if (scaled) {
+            a0 = sum8(k, a0);
+            a2 = dot8(k, yv[p], a2);
+            k = k * rv[p];
         }
-        sums[2 * tt] = live ? a0 : 0.f;
-        sums[2 * tt + 1] = live ? a2 : 0.f;
-        if (tt < nt && live) *(h16x4 *)(a.out[j] + o) = out4;
+        if (t0 + n < a.T && live) *(h16x8 *)(a.out[j] + o + 8 * p) = k;
     }
-    if (scaled) {
-        __shared__ float red[2 * TT * 4];
-        block_sum_n<2 * TT>(sums, red);
-        if (threadIdx.x < nt) {
-            const size_t pi = (size_t)(t0 + threadIdx.x) * a.npart;
-            float s0 = 0.f, s2 = 0.f;
-#pragma unroll
-            for (int tt = 0; tt < TT; ++tt)
-                if (tt == (int)threadIdx.x) { s0 = sums[2 * tt]; s2 = sums[2 * tt + 1]; }
-            a.p0[j][pi + blockIdx.y] = s0;
-            a.p2[j][pi + blockIdx.y] = s2;
-            if (blockIdx.y == 0)
-                for (int q = gridDim.y; q < a.npart; ++q) { a.p0[j][pi + q] = 0.f; a.p2[j][pi + q] = 0.f; }
-        }
+    if (!scaled) return;
+    a0 += __shfl_xor(a0, 16, WAVE);
+    a2 += __shfl_xor(a2, 16, WAVE);
+    a0 += __shfl_xor(a0, 32, WAVE);
+    a2 += __shfl_xor(a2, 32, WAVE);
+    if (lane < 16) { red[0][wave][lane] = live ? a0 : 0.f; red[1][wave][lane] = live ? a2 : 0.f; }
+    __syncthreads();
+    const int tok = threadIdx.x & 15, which = threadIdx.x >> 4;
+    if (which < 2 && t0 + tok < a.T) {
+        float *p = (which ? a.p2[j] : a.p0[j]) + (size_t)(t0 + tok) * a.npart;
+        const float(&r)[4][16] = red[which];
+        p[blockIdx.y] = ((r[0][tok] + r[1][tok]) + r[2][tok]) + r[3][tok];
+        if (blockIdx.y == 0)
+            for (int i = gridDim.y; i < a.npart; ++i) p[i] = 0.f;
     }
+}
+// what its 16-byte loads assume beyond the layer's own checks: C ABI callers may put these on any boundary
+bool mix2_mfma_ok(const rwkv_v56_layer &l) {
+    for (int j = 1; j < 6; ++j)
+        if (!aligned16(l.att_mix[j])) return false;
+    return aligned16(l.tm_w2);
+}
+// Calls of up to 16 tokens keep the sums in index order, so that a conversation's first tokens come out as they did: a deep
+// model whose state is nearly empty makes percents of its logits from the last bit of a mix.  The matrix cores gain 2 % of a
+// call there.
+void v6_mix2_launch(const Mix2Args &a, bool mfma, hipStream_t st) {
+    const auto kernel = !mfma ? v6_mix2_kernel<4> : a.R <= 32 ? v6_mix2_mfma_kernel<1> : v6_mix2_mfma_kernel<2>;
+    const int tt = mfma ? 16 : 4;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)((a.T + tt - 1) / tt), (unsigned)((a.C + 255) / 256), 5), dim3(256), 0, st, a);
 }
 
 struct Ws56 {
@@ -243,8 +270,8 @@ struct Ws56 {
     size_t total;
 };
 
-// partial sums per row that v6_mix2x4_kernel writes: one per block of 1024 channels, rounded up to a multiple of four
-int mix_parts(int64_t C) { return (int)((((C + 1023) / 1024) + 3) & ~(int64_t)3); }
+// partial sums per row that v6_mix2_mfma_kernel writes: one per block of 256 channels, rounded up to a multiple of four
+int mix_parts(int64_t C) { return (int)((((C + 255) / 256) + 3) & ~(int64_t)3); }
 
 Ws56 carve56(void *base, int64_t T, int64_t C, int64_t F, int64_t lm, int64_t ld) {
     Ws56 w;
@@ -376,9 +403,7 @@ extern "C" int rwkv_v56_forward(const rwkv_v56_model *m, const rwkv_v56_layer_st
                 b.xx = ws.xx_att; b.sxd = nullptr; b.prev = s.att_xx;
             } else {
                 Mix1Args a{(int)T, C, ws.x, l.ln1_w, l.ln1_b, s.att_xx, l.att_mix[0], ws.xx, ws.sxd, ws.xxx, s.att_xx};
-                if (C <= 2048) hipLaunchKernelGGL(v6_mix1_kernel<1>, dim3((unsigned)T), dim3(256), 0, st, a);
-                else if (C <= 4096) hipLaunchKernelGGL(v6_mix1_kernel<2>, dim3((unsigned)T), dim3(256), 0, st, a);
-                else hipLaunchKernelGGL(v6_mix1_kernel<4>, dim3((unsigned)T), dim3(256), 0, st, a);
+                v6_mix1_launch(a, st);
                 if ((rc = mm(c, lora_mat(l.tm_w1, C, 5 * lm), false, ws.xxx, ACT_TANH, nullptr, nullptr, 1.f, ws.t1))) return rc;
                 b.xx = ws.xx; b.sxd = ws.sxd; b.prev = nullptr;
             }
@@ -386,7 +411,8 @@ extern "C" int rwkv_v56_forward(const rwkv_v56_model *m, const rwkv_v56_layer_st
             for (int j = 0; j < 5; ++j) { b.maa[j] = l.att_mix[1 + j]; b.out[j] = ws.mix[j]; }
             // uint8 matrices, the four products as one grouped direct-to-LDS launch: the mixing kernel writes their
             // inputs already scaled, with partial row sums that the grouped launch adds up -- no scaling pass
-            if (T > 1 && u8 && grouped && !(C & 3) && lm <= 64 && handover_enabled()) {
+            const bool mfma = T > 16 && mix2_mfma_ok(l);
+            if (mfma && u8 && grouped && handover_enabled()) {
                 const rwkv_half *xin[4] = {ws.mix[3], ws.mix[1], ws.mix[2], ws.mix[4]};
                 const rwkv_mat *mats[4] = {&l.att_receptance, &l.att_key, &l.att_value, &l.att_gate};
                 void *outs[4] = {ws.r, ws.k, ws.v, ws.g};
@@ -401,11 +427,7 @@ extern "C" int rwkv_v56_forward(const rwkv_v56_model *m, const rwkv_v56_layer_st
                 }
             }
             if (T == 1) hipLaunchKernelGGL(v6_mix2_kernel<1>, dim3(1, (unsigned)((C + 255) / 256), 5), dim3(256), 0, st, b);
-            else if (!(C & 3) && lm <= 64) {
-                if (T <= 512) hipLaunchKernelGGL(v6_mix2x4_kernel<4>, dim3((unsigned)((T + 3) / 4), (unsigned)((C + 1023) / 1024), 5), dim3(256), 0, st, b);
-                else hipLaunchKernelGGL(v6_mix2x4_kernel<16>, dim3((unsigned)((T + 15) / 16), (unsigned)((C + 1023) / 1024), 5), dim3(256), 0, st, b);
-            }
-            else hipLaunchKernelGGL(v6_mix2_kernel<16>, dim3((unsigned)((T + 15) / 16), (unsigned)((C + 255) / 256), 5), dim3(256), 0, st, b);
+            else v6_mix2_launch(b, mfma, st);
             wx = ws.mix[0]; kx = ws.mix[1]; vx = ws.mix[2]; rx = ws.mix[3]; gx = ws.mix[4];
             // one token: the first decay-LoRA stage rides at the end of the receptance / key / value / gate launch
             fuse_d1 = T == 1 && C <= 8 * 512;
