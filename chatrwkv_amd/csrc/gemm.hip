@@ -1389,14 +1389,23 @@ __global__ __launch_bounds__(256) void mm8_prepare_group_kernel(int T, int N, Pr
 // ---- calls of 2 .. 16 rows: every weight row streamed once ---------------------------------------------------
 // A ragged last prompt chunk (rwkv/utils.py:98-101) or a short chat turn has a handful of tokens: with 128-row
 // tiles the contraction kernels spend their time on empty rows and a call costs several one-token steps.  Here
-// a workgroup of 16 waves takes 16 output rows at a time and splits K over its waves: wave w owns the k-chunks
-// w, w + 16, ... (64 wide for uint8 rows, 32 for fp16 rows); per chunk a lane loads 16 bytes of one weight row
-// (lane = row + 16 q: the four lanes of a row cover 64 contiguous bytes) and the matching 16 / 8 activation values
-// of one token (lane = token + 16 q, rows past T repeat the last one), widens uint8 to the exact fp16 value b + 1/2
-// and issues v_mfma_f32_16x16x32_f16 with the weights as the first and the activations as the second operand, so
-// that lane (token j, q) ends with rows 4 q .. 4 q + 3 of token j.  The 16 partial 16 x 16 blocks are added in wave
-// order through LDS (deterministic), and 256 threads run the same epilogue as the large kernels.  Activations come
-// from L2 (T x N values, re-read per row group); weights from HBM, each byte once.
+// a workgroup of 16 waves, one per CU, takes a consecutive share of the launch's row groups (16 output rows each, the
+// groups of all members in one order) and splits K over its waves: wave w owns the 64-wide units w, w + 16, ...; per
+// unit a lane loads 16 (uint8) or 2 x 16 bytes (fp16) of one weight row (lane = row + 16 q) and multiplies them, uint8
+// widened to the exact fp16 value b + 1/2, with its token's values (lane = token + 16 q, rows past T repeat the last
+// one) by v_mfma_f32_16x16x32_f16, weights first, so that lane (token j, q) ends with rows 4 q .. 4 q + 3 of token j.
+// The 16 partial blocks are added in wave order through LDS (deterministic) by four of the waves, which round and store.
+// Bound by HBM: the next step's weights, of the next row group where this one's end, are requested before a step is
+// multiplied, and the barrier of an exchange waits for LDS only, so a wave always has a step in flight.  (A workgroup
+// per row group, two to a CU, had its start, its activations and its end between any two requests.)
+//   NU > 0   rows of up to 16 NU units: a wave holds its share of the activations in registers for all row groups.
+//   NU == 0  longer rows: the activations come from L2 with the weights.  Fragment order asks for 16 rows per 16 lanes,
+//            which the CU takes at 16 bytes a clock (9 TB/s over the chip from L2, 15.5 where four lanes ask for 64
+//            consecutive bytes): they are read eight lanes to a row and change order in LDS of the wave's own.
+// us a launch, 8 rows, against a workgroup per row group with fragment-order loads throughout: uint8, 4096 wide, three members
+// of 4096 outputs 18.7 -> 16.8, [8 x 16384] x [16384 x 4096] 22.9 -> 21.4, three of 5120 at 5120 wide 45.3 -> 28.9,
+// [8 x 20480] x [20480 x 5120] 51.9 -> 46.6 (320 row groups on 256 CUs); fp16, 4096 wide, three of 4096 25.5 -> 23.1,
+// [8 x 16384] x [16384 x 4096] 38.3 -> 33.6 (4.0 TB/s).
 struct SkinnyGroup {
     const h16 *A[4];
     const void *W[4];
@@ -1406,102 +1415,187 @@ struct SkinnyGroup {
     GemmEpi ep[4];
 };
 
-// NCI > 0: a wave owns at most NCI chunks and keeps their activation values in registers for all its row groups
-// (rows of up to 16 * NCI chunks: the loop then issues weight loads only); NCI == 0: any row length, activations
-// re-read from L2 for every row group.
-template <bool W_U8, int NCI>
-__global__ __launch_bounds__(1024) void skinny_kernel(int T, int N, SkinnyGroup g) {
-    __shared__ float red[16][64][4];
-    const int gi = blockIdx.y, M = g.M[gi];
-    const h16 *__restrict__ A = g.A[gi];
-    const unsigned char *__restrict__ W = (const unsigned char *)g.W[gi];
-    const int64_t lda = g.lda, ldw = g.ldw[gi];
+template <bool W_U8, int NU>
+__global__ __launch_bounds__(1024) void skinny_kernel(int T, int N, int n, int total, SkinnyGroup g) {
+    constexpr bool HELD = NU > 0;
+    constexpr int WL = W_U8 ? 1 : 2;                            // weight loads per unit
+    constexpr int UB = NU == 1 ? 1 : NU == 4 && W_U8 ? 4 : 2;   // units of a step
+    constexpr int NS = HELD ? NU / UB : 2;                      // steps of a row group; NU == 0: of a pass of its loop
+    constexpr int NB = HELD ? 2 : 1;                            // exchange buffers: with two, one barrier per row group
+    constexpr int RQ = 80;                                      // floats per q of a block: the readers' banks differ
+    __shared__ __align__(16) float red[NB][16][4 * RQ];
+    __shared__ __align__(16) h16 sx[HELD ? 1 : 16][HELD ? 8 : 16 * 64];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int sub = lane & 15, q = lane >> 4;
-    constexpr int CK = W_U8 ? 64 : 32;               // k values per chunk
-    const int nchunks = N / CK;
-    const int ngroups = (M + 15) >> 4;
-    const h16 *arow = A + (size_t)min(sub, T - 1) * lda;   // this lane's token
+    const int nunits = N / 64;
     const h16x2 off = {(h16)1023.5f, (h16)1023.5f};
-    constexpr int NB = NCI > 0 ? NCI : 4;            // chunks loaded before any is multiplied
-    auto load_x = [&](int c, h16x8 &x0, h16x8 &x1) {
-        if (W_U8) {
-            x0 = *(const h16x8 *)(arow + (size_t)c * 64 + 16 * q);
-            x1 = *(const h16x8 *)(arow + (size_t)c * 64 + 16 * q + 8);
-        } else {
-            x0 = *(const h16x8 *)(arow + (size_t)c * 32 + 8 * q);
-            x1 = x0;
-        }
+    const int b0 = (int)((int64_t)total * blockIdx.x / gridDim.x), b1 = (int)((int64_t)total * (blockIdx.x + 1) / gridDim.x);
+    // the k's of a unit that a lane multiplies: two pieces of eight
+    const int p0 = W_U8 ? 2 * q : q, p1 = W_U8 ? 2 * q + 1 : 4 + q;
+    auto fence = [] {                                           // loads are used in the order of their issue (v7.hip)
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
     };
-    auto load_w = [&](const unsigned char *wrow, int c) {
-        if (W_U8) return __builtin_nontemporal_load((const u32x4 *)(wrow + (size_t)c * 64 + 16 * q));
-        return __builtin_nontemporal_load((const u32x4 *)(wrow + ((size_t)c * 32 + 8 * q) * 2));
-    };
-    auto multiply = [&](u32x4 wv, h16x8 x0, h16x8 x1, f32x4 &acc) {
-        if (W_U8) {
+    auto multiply = [&](const u32x4 (&w)[WL], h16x8 x0, h16x8 x1, f32x4 &acc) {
+        if constexpr (W_U8) {
+            const u32x4 wv = w[0];
             const h16x2 a0 = u8pair_lo_1024(wv.x) - off, a1 = u8pair_hi_1024(wv.x) - off;
             const h16x2 a2 = u8pair_lo_1024(wv.y) - off, a3 = u8pair_hi_1024(wv.y) - off;
-            const h16x2 b0 = u8pair_lo_1024(wv.z) - off, b1 = u8pair_hi_1024(wv.z) - off;
-            const h16x2 b2 = u8pair_lo_1024(wv.w) - off, b3 = u8pair_hi_1024(wv.w) - off;
+            const h16x2 c0 = u8pair_lo_1024(wv.z) - off, c1 = u8pair_hi_1024(wv.z) - off;
+            const h16x2 c2 = u8pair_lo_1024(wv.w) - off, c3 = u8pair_hi_1024(wv.w) - off;
             const h16x8 wa = {a0.x, a0.y, a1.x, a1.y, a2.x, a2.y, a3.x, a3.y};
-            const h16x8 wb = {b0.x, b0.y, b1.x, b1.y, b2.x, b2.y, b3.x, b3.y};
+            const h16x8 wb = {c0.x, c0.y, c1.x, c1.y, c2.x, c2.y, c3.x, c3.y};
             acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(wa, x0, acc, 0, 0, 0);
             acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(wb, x1, acc, 0, 0, 0);
         } else {
-            acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h16x8, wv), x0, acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h16x8, w[0]), x0, acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h16x8, w[1]), x1, acc, 0, 0, 0);
         }
     };
-    // chunks past the end of the row repeat the last one and multiply zeros: no branch sits between the loads and
-    // their use (loads would be sunk behind it, one chunk in flight at a time)
-    h16x8 rx0[NB], rx1[NB];
-    if (NCI > 0) {
+    int base = 0, count = 0;                                    // row groups of the members before; done by this workgroup
+    for (int gi = 0; gi < n; ++gi) {
+        const int M = g.M[gi], groups = (M + 15) >> 4;
+        const int lo = max(b0, base) - base, hi = min(b1, base + groups) - base;
+        base += groups;
+        if (lo >= hi) continue;
+        const GemmEpi &ep = g.ep[gi];
+        const h16 *A = g.A[gi];
+        const unsigned char *W = (const unsigned char *)g.W[gi];
+        const int64_t ldw = g.ldw[gi] * (W_U8 ? 1 : 2);
+        // In place of a unit past the end of the row, and of every unit past the share's last row group, all lanes load the
+        // first bytes of the matrix, which nothing uses: a branch around a load would make the waits for those before it longer.
+        struct Step { u32x4 w[UB][WL]; h16x8 x[HELD ? 1 : UB][2]; };
+        auto load_w = [&](Step &s, int grp, int i0) {
+            const bool there = grp < hi;
+            const size_t row = (size_t)min(16 * grp + sub, M - 1) * ldw + 16 * q;
 #pragma unroll
-        for (int i = 0; i < NB; ++i) {
-            load_x(min(wave + 16 * i, nchunks - 1), rx0[i], rx1[i]);
-            if (wave + 16 * i >= nchunks) { rx0[i] = h16x8{}; rx1[i] = h16x8{}; }
-        }
-    }
-    for (int grp = blockIdx.x; grp < ngroups; grp += gridDim.x) {
-        const int m0 = grp << 4;
-        const unsigned char *wrow = W + (size_t)min(m0 + sub, M - 1) * ldw * (W_U8 ? 1 : 2);
-        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-        if (NCI > 0) {
-            u32x4 wv[NB];
+            for (int i = 0; i < UB; ++i) {
+                const int u = wave + 16 * (i0 + i);
+                const bool ok = there && u < nunits;
+                const size_t at = ok ? row + (size_t)u * (64 * WL) : 0;
 #pragma unroll
-            for (int i = 0; i < NB; ++i) wv[i] = load_w(wrow, min(wave + 16 * i, nchunks - 1));
+                for (int e = 0; e < WL; ++e) s.w[i][e] = __builtin_nontemporal_load((const u32x4 *)(W + at + (ok ? 64 * e : 0)));
+            }
+        };
+        struct Ops { rwkv_half rx, mx, res, gate; float s0, s2; };
+        const int ft = (threadIdx.x & 255) >> 4, fm = threadIdx.x & 15;   // the output that a thread of the four waves finishes
+        const bool has_res = ep.act == ACT_RESIDUAL || ep.act == ACT_GATED_RESIDUAL, has_gate = ep.act == ACT_GATED_RESIDUAL;
+        auto load_ops = [&](int grp) {
+            Ops o = {};
+            const int t = min(ft, T - 1), m = min(16 * grp + fm, M - 1);
+            if constexpr (W_U8) { o.rx = ep.rx[m]; o.mx = ep.mx[m]; o.s0 = ep.s0[t]; o.s2 = ep.s2[t]; }
+            o.res = *(has_res ? ep.res + (size_t)t * ep.ldres + m : (const rwkv_half *)A);
+            o.gate = *(has_gate ? ep.gate + (size_t)t * ep.ldgate + m : (const rwkv_half *)A);
+            return o;
+        };
+        auto finish = [&](int grp, const f32x4 &acc, const Ops &o) {
+            const int buf = count & (NB - 1);
+            if (NB == 1 && count) {                              // the sums of the row group before have been read
+                __builtin_amdgcn_s_barrier();
+                asm volatile("" ::: "memory");
+            }
+            *(f32x4 *)&red[buf][wave][RQ * q + 4 * sub] = acc;
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_s_waitcnt(0xC07F);                  // LDS only: __syncthreads() would also wait for the loads in flight
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+            if ((wave >> 2) == (count & 3)) {
+                float v = 0.f;
 #pragma unroll
-            for (int i = 0; i < NB; ++i) multiply(wv[i], rx0[i], rx1[i], acc);
-        } else {
-            for (int c0 = wave; c0 < nchunks; c0 += 16 * NB) {
-                u32x4 wv[NB];
-                h16x8 x0[NB], x1[NB];
-#pragma unroll
-                for (int i = 0; i < NB; ++i) {
-                    const int c = min(c0 + 16 * i, nchunks - 1);
-                    wv[i] = load_w(wrow, c);
-                    load_x(c, x0[i], x1[i]);
+                for (int w = 0; w < 16; ++w) v += red[buf][w][RQ * (fm >> 2) + 4 * ft + (fm & 3)];
+                const int m = 16 * grp + fm;
+                if (m < M && ft < T) {
+                    const size_t at = (size_t)ft * g.ldy[gi] + m;
+                    if constexpr (W_U8) v = epi_affine(v, h2f(o.rx), h2f(o.mx), o.s0, o.s2);
+                    if (ep.raw_f32) {
+                        ((float *)g.Y[gi])[at] = v;
+                    } else {
+                        float r[1] = {v};
+                        h16 res[1] = {__builtin_bit_cast(h16, o.res)}, gate[1] = {__builtin_bit_cast(h16, o.gate)};
+                        epi_act<1, const h16 *>(r, res, gate, ep);
+                        if (ep.out_dtype == RWKV_DT_F32) ((float *)g.Y[gi])[at] = round_h(r[0]);
+                        else ((rwkv_half *)g.Y[gi])[at] = f2h(r[0]);
+                    }
                 }
+                if (NB == 1) __builtin_amdgcn_s_waitcnt(0xC07F);
+            }
+            ++count;
+        };
+        Step st[2];
+        if constexpr (HELD) {
+            const h16 *arow = A + (size_t)min(sub, T - 1) * g.lda;
+            h16x8 rx[NU][2];
 #pragma unroll
-                for (int i = 0; i < NB; ++i) {
-                    if (c0 + 16 * i >= nchunks) { x0[i] = h16x8{}; x1[i] = h16x8{}; }
-                    multiply(wv[i], x0[i], x1[i], acc);
+            for (int i = 0; i < NU; ++i) {
+                const int u = wave + 16 * i;
+                const h16 *p = arow + (size_t)min(u, nunits - 1) * 64;
+                rx[i][0] = *(const h16x8 *)(p + 8 * p0);
+                rx[i][1] = *(const h16x8 *)(p + 8 * p1);
+            }
+            fence();
+            load_w(st[0], lo, 0);
+            fence();
+            constexpr int PASS = NS == 1 ? 2 : 1;                // row groups per pass: the two steps' registers alternate
+            for (int grp = lo; grp < hi; grp += PASS) {
+#pragma unroll
+                for (int p = 0; p < PASS; ++p) {
+                    if (grp + p >= hi) break;
+                    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+                    const Ops o = load_ops(grp + p);
+                    fence();
+#pragma unroll
+                    for (int k = 0; k < NS; ++k) {
+                        const int j = p * NS + k;
+                        load_w(st[(j + 1) & 1], k + 1 < NS ? grp + p : grp + p + 1, k + 1 < NS ? (k + 1) * UB : 0);
+                        fence();
+#pragma unroll
+                        for (int i = 0; i < UB; ++i)
+                            if (wave + 16 * (k * UB + i) < nunits) multiply(st[j & 1].w[i], rx[k * UB + i][0], rx[k * UB + i][1], acc);
+                        fence();
+                    }
+                    finish(grp + p, acc, o);
                 }
             }
-        }
-        __syncthreads();                                          // the previous group's sums have been read
-        *(f32x4 *)&red[wave][lane][0] = acc;
-        __syncthreads();
-        if (threadIdx.x < 256) {
-            const int l = threadIdx.x & 63, r = threadIdx.x >> 6;
-            float v = 0.f;
+        } else {
+            const int r8 = lane >> 3, seg = lane & 7;
+            const size_t xa = (size_t)min(r8, T - 1) * g.lda + 8 * seg, xb = (size_t)min(r8 + 8, T - 1) * g.lda + 8 * seg;
+            h16 *slot = sx[wave];
+            h16 *wr = slot + 64 * r8 + 8 * (seg ^ r8);           // (r8 + 8) & 7 == r8
+            const h16 *rd0 = slot + 64 * sub + 8 * (p0 ^ (sub & 7)), *rd1 = slot + 64 * sub + 8 * (p1 ^ (sub & 7));
+            auto load = [&](Step &s, int grp, int i0) {
 #pragma unroll
-            for (int w = 0; w < 16; ++w) v += red[w][l][r];
-            const int m = m0 + 4 * (l >> 4) + r, t = l & 15;
-            if (m < M && t < T) {
-                const GemmEpi &ep = g.ep[gi];
-                float rxm = 1.f, mxm = 0.f;
-                if (ep.rx) { rxm = h2f(ep.rx[m]); mxm = h2f(ep.mx[m]); }
-                gemm_epilogue(v, t, m, rxm, mxm, ep, g.Y[gi], g.ldy[gi]);
+                for (int i = 0; i < UB; ++i) {
+                    const int u = wave + 16 * (i0 + i);
+                    const bool ok = grp < hi && u < nunits;
+                    s.x[i][0] = *(const h16x8 *)(A + (ok ? xa + (size_t)u * 64 : 0));
+                    s.x[i][1] = *(const h16x8 *)(A + (ok ? xb + (size_t)u * 64 : 0));
+                }
+                load_w(s, grp, i0);
+            };
+            // units per wave, whole passes
+            const int span = ((nunits + 15) / 16 + NS * UB - 1) / (NS * UB) * (NS * UB);
+            load(st[0], lo, 0);
+            fence();
+            for (int grp = lo; grp < hi; ++grp) {
+                f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+                for (int i0 = 0; i0 < span; i0 += NS * UB) {
+#pragma unroll
+                    for (int k = 0; k < NS; ++k) {
+                        const int next = i0 + (k + 1) * UB;
+                        load(st[(k + 1) & 1], next < span ? grp : grp + 1, next < span ? next : 0);
+                        fence();
+#pragma unroll
+                        for (int i = 0; i < UB; ++i) {
+                            if (wave + 16 * (i0 + k * UB + i) >= nunits) continue;
+                            *(h16x8 *)wr = st[k & 1].x[i][0];
+                            *(h16x8 *)(wr + 8 * 64) = st[k & 1].x[i][1];
+                            const h16x8 x0 = *(const h16x8 *)rd0, x1 = *(const h16x8 *)rd1;
+                            multiply(st[k & 1].w[i], x0, x1, acc);
+                        }
+                        fence();
+                    }
+                }
+                finish(grp, acc, load_ops(grp));
             }
         }
     }
@@ -1509,7 +1603,7 @@ __global__ __launch_bounds__(1024) void skinny_kernel(int T, int N, SkinnyGroup 
 
 constexpr int SKINNY_MAX_ROWS = 16;
 
-// what skinny_kernel assumes of one product: whole chunks, 16-byte aligned rows for its 16-byte loads
+// what skinny_kernel assumes of one product: whole units, 16-byte aligned rows for its 16-byte loads
 bool skinny_ok(bool w_u8, int64_t T, int64_t N, const void *A, int64_t lda, const void *W, int64_t ldw, const GemmEpi &ep) {
     auto a16 = [](const void *p) { return (((uintptr_t)p) & 15) == 0; };
     if (T < 2 || T > SKINNY_MAX_ROWS || N < 64 || (N % 64)) return false;
@@ -1521,14 +1615,14 @@ bool skinny_ok(bool w_u8, int64_t T, int64_t N, const void *A, int64_t lda, cons
 }
 
 int skinny_launch(bool w_u8, int n, int64_t T, int64_t N, const SkinnyGroup &g, hipStream_t st) {
-    int maxg = 1;
-    for (int i = 0; i < n; ++i) maxg = std::max(maxg, (g.M[i] + 15) / 16);
-    const dim3 grid((unsigned)std::min(maxg, 2 * num_cu()), (unsigned)n);
-    const int64_t per_wave = (N / (w_u8 ? 64 : 32) + 15) / 16;    // chunks a wave owns
-#define RWKV_SKINNY(NCI)                                                                                         \
-    do {                                                                                                         \
-        if (w_u8) hipLaunchKernelGGL((skinny_kernel<true, NCI>), grid, dim3(1024), 0, st, (int)T, (int)N, g);   \
-        else hipLaunchKernelGGL((skinny_kernel<false, NCI>), grid, dim3(1024), 0, st, (int)T, (int)N, g);       \
+    int total = 0;
+    for (int i = 0; i < n; ++i) total += (g.M[i] + 15) / 16;
+    const dim3 grid((unsigned)std::min(total, num_cu()));
+    const int64_t per_wave = (N / 64 + 15) / 16;                  // units a wave owns
+#define RWKV_SKINNY(NU)                                                                                                  \
+    do {                                                                                                                 \
+        if (w_u8) hipLaunchKernelGGL((skinny_kernel<true, NU>), grid, dim3(1024), 0, st, (int)T, (int)N, n, total, g);   \
+        else hipLaunchKernelGGL((skinny_kernel<false, NU>), grid, dim3(1024), 0, st, (int)T, (int)N, n, total, g);       \
     } while (0)
     if (per_wave <= 1) RWKV_SKINNY(1);
     else if (per_wave <= 2) RWKV_SKINNY(2);

@@ -119,6 +119,29 @@ def test_mm8_seq(N, M, B):
     assert np.abs(y1.cpu().numpy().astype(np.float64) - y[B - 1].cpu().numpy()).max() <= np.abs(ref).max() * 2 ** -9
 
 
+@pytest.mark.parametrize("N,M,B", [(64, 4100, 16), (1088, 12304, 2), (2048, 24, 9), (3136, 8200, 8), (4096, 12304, 15), (5120, 8208, 9),
+                                   (8192, 4112, 3), (8256, 200, 16), (8320, 4128, 5), (16384, 4112, 13)])
+def test_products_of_short_calls(N, M, B):
+    """2 .. 16 rows: every number of units a wave holds and the form for longer rows, units that only some waves have, more
+    row groups than CUs and fewer, a last one of 4 or 8 rows.  fp16 weights: sums of small whole numbers, so exact, with one
+    infinite weight, which stays in its own output.  uint8: bounds as in test_mm8_seq."""
+    ops = _ops()
+    r = _rng(N + M + B)
+    x = r.integers(-2, 3, (B, N)).astype(np.float16)
+    w = r.integers(-3, 4, (N, M)).astype(np.float16)
+    ref = (x.astype(np.float32) @ w.astype(np.float32)).astype(np.float16)
+    wt, xt = _to_dev_ic(w), torch.from_numpy(x).to(DEV)
+    y = ops.matmul_float(xt, wt, output_dtype=torch.float16)
+    assert np.array_equal(y.cpu().numpy(), ref)
+    wt[0, 0] = float("inf")
+    y = ops.matmul_float(xt, wt, output_dtype=torch.float32).cpu().numpy()
+    assert np.array_equal(y[:, 1:], ref[:, 1:].astype(np.float32)) and not np.isfinite(y[:, 0]).any()
+    x, ref, (q, mx, rx, my, ry) = _mm8_case(N, M, B, N + M + B)
+    y = ops.cuda_mm8_seq(B, N, M, torch.from_numpy(x).to(DEV), q, mx, rx, my, ry)
+    d = np.abs(y.cpu().numpy().astype(np.float64) - ref)
+    assert d.max() <= 1e-3 * np.sqrt(np.mean(ref ** 2)) + np.abs(ref).max() * 2 ** -10, d.max()
+
+
 @pytest.mark.parametrize("N,M,B", [(64, 128, 33), (128, 8, 20), (1024, 1000, 17), (1024, 136, 63), (2048, 264, 64), (4096, 4096, 40),
                                    (4096, 2056, 65), (4096, 4096, 129), (1024, 8192, 192), (16384, 512, 256)])
 def test_mm8_seq_tile_edges(N, M, B):
