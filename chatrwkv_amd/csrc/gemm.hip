@@ -1638,23 +1638,29 @@ int skinny_launch(bool w_u8, int n, int64_t T, int64_t N, const SkinnyGroup &g, 
 // The first stage of a low-rank product (RWKV-6 mixing and decay LoRA, RWKV-7's four) has thousands of input columns
 // and a few dozen to a few hundred outputs: a handful of 128 x 128 tiles, which the tile kernels can only spread
 // over the chip by splitting K and adding the slabs in a second launch.  Here a workgroup of eight waves takes a
-// 16 x 16 block of the output and splits K over its waves: wave w owns the 32-wide k-chunks w, w + 8, ...; per
-// chunk a lane loads 16 bytes of one weight row and of one activation row (lane = row + 16 q: the four lanes of a
-// row cover 64 contiguous bytes), sixteen chunks in flight, and issues v_mfma_f32_16x16x32_f16 with the weights as
-// the first operand, so that lane (token j, q) ends with outputs 4 q .. 4 q + 3 of token j.  The eight partial
-// blocks are added in wave order through LDS (deterministic) and 64 threads round, apply the activation and store
-// 8 bytes each.  Operands come from L2: the weights are read once per 16 rows of the call, the activation once per
-// 16 outputs, so the kernel serves calls of up to NARROW_MAX_T rows ([256 x 4096] x [4096 x 160]: 9 us against
-// 14 us for the K-split tiles and their second pass; at 1024 rows the tiles win, 23 against 14 us).
+// 16 x 16 block of the output and splits K over its waves: wave w owns the 32-wide k-chunks w, w + 8, ...; it loads
+// 16 bytes a lane of the weight rows and of the activation rows, sixteen chunks in flight (one round at 4096), and issues
+// v_mfma_f32_16x16x32_f16 with the weights as the first operand, so that lane (token j, q) ends with outputs 4 q .. 4 q + 3
+// of token j.  The eight partial blocks are added in wave order through LDS (deterministic) and 64 threads round, apply the
+// activation and store 8 bytes each.  Operands come from L2: the weights once per 16 rows of the call, the activation once
+// per 16 outputs, 256 KB a workgroup at 4096, at the rate its CU takes them: 16 bytes a clock in the order of the fragments
+// (16 rows for 16 lanes), 64 where four neighbouring lanes ask for 64 bytes of a row.  So they are loaded that way and change
+// order in 2 KB of LDS per wave.  [256 x 4096] x [4096 x 160]: 9.9 us in fragment order with the ten loads in flight that the
+// compiler left, 6.8 now; K-split tiles and their second pass 21.
 __global__ __launch_bounds__(512) void narrow_kernel(int T, int N, int M, const h16 *__restrict__ A, int64_t lda,
                                                      const h16 *__restrict__ W, int64_t ldw, rwkv_half *__restrict__ Y,
                                                      int64_t ldy, GemmEpi ep) {
     __shared__ f32x4 red[8][64];
+    __shared__ __align__(16) h16 order[8][2][16 * 32];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int sub = lane & 15, q = lane >> 4;
     const int t0 = blockIdx.x * 16, m0 = blockIdx.y * 16;
-    const h16 *arow = A + (size_t)min(t0 + sub, T - 1) * lda + 8 * q;
-    const h16 *wrow = W + (size_t)min(m0 + sub, M - 1) * ldw + 8 * q;
+    // loaded: row lane / 4, piece lane & 3 of eight k's; multiplied: row sub, piece q.  Piece p of row r lies at p ^ (r / 4)
+    const int lr = lane >> 2, lp = lane & 3;
+    const h16 *arow = A + (size_t)min(t0 + lr, T - 1) * lda + 8 * lp;
+    const h16 *wrow = W + (size_t)min(m0 + lr, M - 1) * ldw + 8 * lp;
+    h16 *const in = &order[wave][0][32 * lr + 8 * (lp ^ (lr >> 2))];
+    const h16 *const frag = &order[wave][0][32 * sub + 8 * (q ^ (sub >> 2))];
     const int nchunks = N / 32;
     constexpr int NB = 16;   // chunks in flight per wave: a 4096-wide row is one round
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
@@ -1667,10 +1673,14 @@ __global__ __launch_bounds__(512) void narrow_kernel(int T, int N, int M, const 
             wv[i] = *(const h16x8 *)(wrow + (size_t)c * 32);
             xv[i] = *(const h16x8 *)(arow + (size_t)c * 32);
         }
+        __builtin_amdgcn_sched_barrier(0);   // all of them before the first use
 #pragma unroll
         for (int i = 0; i < NB; ++i) {
             if (c0 + 8 * i >= nchunks) xv[i] = h16x8{};
-            acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(wv[i], xv[i], acc, 0, 0, 0);
+            *(h16x8 *)in = wv[i];
+            *(h16x8 *)(in + 16 * 32) = xv[i];
+            const h16x8 wf = *(const h16x8 *)frag, xf = *(const h16x8 *)(frag + 16 * 32);
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(wf, xf, acc, 0, 0, 0);
         }
     }
     red[wave][lane] = acc;
@@ -1692,13 +1702,17 @@ __global__ __launch_bounds__(512) void narrow_kernel(int T, int N, int M, const 
 }
 
 // narrow_kernel's operands: fp16 weights, at most NARROW_MAX_M outputs, rows of whole 32-wide chunks laid out for
-// 16-byte loads, an epilogue without residual or gate, fp16 out.  RWKV_NO_NARROW=1 sends these through the tile
-// kernels (tuning).
-constexpr int NARROW_MAX_M = 192, NARROW_MAX_T = 512;
+// 16-byte loads, an epilogue without residual or gate, fp16 out; as many workgroups as CUs, or twice that where the rows are
+// long.  us a product, this kernel and the tiles: one round, [400 x 512] x [512 x 64] 5.3 / 5.9, [256 x 768] x [768 x 160]
+// 5.4 / 6.4, [1024 x 4096] x [4096 x 64] 6.6 / 15.7; two rounds, [777 x 4096] x [4096 x 160] 15.1 / 15.8, [512 x 2560] x
+// [2560 x 160] 10.4 / 12.8, [777 x 2048] x [2048 x 160] 11.1 / 10.8, [512 x 1024] x [1024 x 160] 8.6 / 8.0; three, [1024 x
+// 2560] x [2560 x 160] 14.0 / 12.5.  RWKV_NO_NARROW=1 sends these through the tile kernels (tuning).
+constexpr int NARROW_MAX_M = 192;
 bool narrow_ok(bool w_u8, int64_t T, int64_t N, int64_t M, const void *A, int64_t lda, const void *W, int64_t ldw, const void *Y,
                int64_t ldy, const GemmEpi &ep) {
     auto a16 = [](const void *p) { return (((uintptr_t)p) & 15) == 0; };
-    if (w_u8 || ep.rx || T <= SKINNY_MAX_ROWS || T > NARROW_MAX_T || M > NARROW_MAX_M || (M & 3) || N < 1024 || (N % 32)) return false;
+    if (w_u8 || ep.rx || T <= SKINNY_MAX_ROWS || M > NARROW_MAX_M || (M & 3) || N < 512 || (N % 32)) return false;
+    if (((T + 15) / 16) * ((M + 15) / 16) > (N < 2560 ? 1 : 2) * num_cu()) return false;
     if ((lda & 7) || (ldw & 7) || (ldy & 3) || !a16(A) || !a16(W) || (((uintptr_t)Y) & 7)) return false;
     if (ep.act == ACT_RESIDUAL || ep.act == ACT_GATED_RESIDUAL || ep.raw_f32 || ep.out_dtype != RWKV_DT_F16) return false;
     const char *e = getenv("RWKV_NO_NARROW");

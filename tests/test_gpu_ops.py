@@ -142,6 +142,17 @@ def test_products_of_short_calls(N, M, B):
     assert d.max() <= 1e-3 * np.sqrt(np.mean(ref ** 2)) + np.abs(ref).max() * 2 ** -10, d.max()
 
 
+@pytest.mark.parametrize("N,M,B", [(512, 4, 700), (544, 20, 17), (1056, 100, 300), (2592, 64, 1024), (4096, 192, 651), (8192, 36, 45)])
+def test_narrow_outputs(N, M, B):
+    """Products of few outputs that one or two rounds of 16 x 16 blocks cover: a last chunk that only some waves have, rows
+    that take two rounds of chunks, ragged blocks in both directions.  Sums of small whole numbers, so exact."""
+    r = _rng(N + M + B)
+    x = r.integers(-2, 3, (B, N)).astype(np.float16)
+    w = r.integers(-3, 4, (N, M)).astype(np.float16)
+    y = _ops().matmul_float(torch.from_numpy(x).to(DEV), _to_dev_ic(w), output_dtype=torch.float16)
+    assert np.array_equal(y.cpu().numpy(), (x.astype(np.float32) @ w.astype(np.float32)).astype(np.float16))
+
+
 @pytest.mark.parametrize("N,M,B", [(64, 128, 33), (128, 8, 20), (1024, 1000, 17), (1024, 136, 63), (2048, 264, 64), (4096, 4096, 40),
                                    (4096, 2056, 65), (4096, 4096, 129), (1024, 8192, 192), (16384, 512, 256)])
 def test_mm8_seq_tile_edges(N, M, B):
