@@ -80,8 +80,8 @@ int wkv56_fused_launch(bool v6, int T, int C, int H, float *state, const rwkv_ha
                        const rwkv_half *dw2 = nullptr, int ld = 0,  // dw2: v6 with w = tanh(. @ D1), product with D2 in-kernel
                        float *y32 = nullptr);  // scratch (wkv56_scratch_bytes) of calls of >= 32 tokens
 size_t wkv56_scratch_bytes(int64_t T, int64_t C);
-// The chunked recurrences (wkv.hip, v7.hip): tokens per chunk, chunks in flight, and the chunks of a call, padded to
-// whole groups of those in flight.
+// The chunked recurrences (wkv.hip, v7.hip): tokens per chunk, chunks in flight, and the chunks that the scratch of a call
+// has room for (it runs fewer: each recurrence ends with its last chunk or group of them).
 constexpr int CL = 16, PD = 8;
 inline int wkv_chunks(int64_t tokens) { return (int)((tokens + CL * PD - 1) / (CL * PD)) * PD; }
 // Is it true in any thread of a workgroup of four waves?  flags: four ints of LDS that nothing else uses meanwhile.

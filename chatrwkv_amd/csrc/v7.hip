@@ -313,8 +313,10 @@ __global__ __launch_bounds__(256) void wkv7_kernel(Wkv7Args a) {
 // Values that are not finite count as 0 in TK v and Y2 v, as in the chunks of RWKV-5/6 (wkv.hip); other operands that are
 // not finite are kept from the tokens before them where the first kernel forms its products.
 // 20 KB of fp32 operands pass from one to the other per head and chunk.  The first kernel moves them at 3.0 TB/s of a
-// copy's 4.8 (1024 tokens, 64 heads: 49.5 us): its six barriers and the forward substitution of one wave beside three that
-// wait are the rest.  The second is a chain of one exchange per chunk (39.9 us, 0.62 a chunk).  Per layer at 64 heads,
+// copy's 4.8: about 1000 vector instructions a wave, a third of them the five exact divisions per element, six barriers and
+// the forward substitution of one wave beside three that wait.  Seven workgroups a CU against the five of 30 KB of LDS, and no
+// chunks past the last: 777 tokens 39.3 -> 37 us.  The second is a chain of one exchange per chunk (35 us, 0.72 a chunk).  A
+// 4096-wide layer, both together: 260 tokens 321 -> 314.5 us, 777 561.5 -> 557, 1024 the same.  Per layer at 64 heads,
 // preparation and recurrence, token by token -> chunks: 1024 tokens 152 -> 89 us, 777 tokens 116 -> 75, 256 tokens 42 -> 31,
 // 100 tokens 21 -> 19; at 64 tokens the two launches take as long as prep7_kernel and wkv7_kernel: CHUNKED7.
 constexpr int SEG7 = 1024;        // tokens per pair of launches: bounds the scratch between them
@@ -327,9 +329,14 @@ constexpr int LM7 = 20;           // LDS row of 16 floats, padded
 
 __global__ __launch_bounds__(256) void wkv7_chunk_kernel(Prep7Args a, int t_begin, float *__restrict__ scratch) {
     __shared__ __align__(16) float la[CL][LR7], lr[CL][LR7], lk[CL][LR7], lb[CL][LR7];   // a . A, r . A, k / A, b / A
-    __shared__ __align__(16) float lw[CL][HS7], lall[HS7];          // decays; A_16
-    __shared__ __align__(16) float mat[4][CL][LM7], lz[CL][LM7];   // AK, AB, QK, QB; Z
-    __shared__ __align__(16) h16 lv[CL * HS7];
+    // 22 KB in all, so that seven workgroups share a CU: A_16 in the pads of la, piece g in row g; the decays where the
+    // matrices come, Z over the rows of AB that it has used, the values at last over Z and QB
+    __shared__ __align__(16) float mat[4][CL][LM7];
+    constexpr int AK = 0, QK = 1, AB = 2, QB = 3;
+    float (*const lw)[HS7] = (float (*)[HS7])&mat[0][0][0];
+    float (*const lz)[LM7] = mat[AB];
+    h16 *const lv = (h16 *)&mat[AB][0][0];
+    static_assert(CL * HS7 <= 4 * CL * LM7 && CL * HS7 * sizeof(h16) <= 2 * CL * LM7 * sizeof(float) && LR7 == HS7 + 4, "");
     const int H = a.H, C = a.C, T = a.T;
     const int h = blockIdx.x % H, c = blockIdx.x / H;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -377,8 +384,6 @@ __global__ __launch_bounds__(256) void wkv7_chunk_kernel(Prep7Args a, int t_begi
         if (g == 0) a.rk[(size_t)t * H + h] = round_h(rks);
     }
     *(f32x4 *)&lw[s][4 * g] = w;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) lv[256 * (g >> 2) + 4 * (4 * (g & 3) + e + 16 * (s >> 2)) + (s & 3)] = live ? vo[e] : (h16)0.f;
     __syncthreads();
     // ---- decays: before = A_{s-1}; a wave holds the tokens 4 wave .. + 3
     f32x4 before = {1.f, 1.f, 1.f, 1.f};
@@ -398,9 +403,8 @@ __global__ __launch_bounds__(256) void wkv7_chunk_kernel(Prep7Args a, int t_begi
     *(f32x4 *)&lb[s][4 * g] = bb * inv;
     if (s == CL - 1) {
         *(f32x4 *)(out + C7_A + 4 * g) = upto;
-        *(f32x4 *)&lall[4 * g] = upto;
+        *(f32x4 *)&la[g][HS7] = upto;
     }
-    *(h16x4 *)((h16 *)(out + C7_V) + 4 * tid) = *(const h16x4 *)(lv + 4 * tid);
     __syncthreads();
     // ---- wave 0: AK, 1: AB, 2: QK, 3: QB.  Row t in the first operand's lanes, s in the second's; D: column s = lane & 15,
     // rows t = 4 q + e
@@ -417,7 +421,7 @@ __global__ __launch_bounds__(256) void wkv7_chunk_kernel(Prep7Args a, int t_begi
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             const int row = 4 * q + e;
-            mat[wave][row][n16] = (wave < 2 ? n16 < row : n16 <= row) ? d[e] : 0.f;
+            mat[wave >> 1 | (wave & 1) << 1][row][n16] = (wave < 2 ? n16 < row : n16 <= row) ? d[e] : 0.f;
         }
     }
     __syncthreads();
@@ -429,7 +433,7 @@ __global__ __launch_bounds__(256) void wkv7_chunk_kernel(Prep7Args a, int t_begi
             float p[2] = {row == n16 ? 1.f : 0.f, 0.f};
 #pragma unroll
             for (int m4 = 0; m4 < row; m4 += 4) {
-                const f32x4 x = *(const f32x4 *)&mat[1][row][m4];
+                const f32x4 x = *(const f32x4 *)&mat[AB][row][m4];
 #pragma unroll
                 for (int e = 0; e < 4; ++e)
                     if (m4 + e < row) p[e & 1] = __builtin_fmaf(x[e], z[m4 + e], p[e & 1]);
@@ -441,7 +445,7 @@ __global__ __launch_bounds__(256) void wkv7_chunk_kernel(Prep7Args a, int t_begi
     __syncthreads();
     // ---- wave b: columns 16 b .. of TA = Z (a . A) and Y1 = r . A + QB TA (a D register is the next product's second
     // operand); wave 1 also TK = Z AK and Y2 = QK + QB TK
-    const f32x4 zf = *(const f32x4 *)&lz[n16][4 * q], qb = *(const f32x4 *)&mat[3][n16][4 * q];
+    const f32x4 zf = *(const f32x4 *)&lz[n16][4 * q], qb = *(const f32x4 *)&mat[QB][n16][4 * q];
     f32x4 ta = {0.f, 0.f, 0.f, 0.f}, y1;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
@@ -454,8 +458,8 @@ __global__ __launch_bounds__(256) void wkv7_chunk_kernel(Prep7Args a, int t_begi
     if (wave == 1) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            tk = __builtin_amdgcn_mfma_f32_16x16x4f32(zf[e], mat[0][4 * q + e][n16], tk, 0, 0, 0);
-            y2[e] = mat[2][4 * q + e][n16];
+            tk = __builtin_amdgcn_mfma_f32_16x16x4f32(zf[e], mat[AK][4 * q + e][n16], tk, 0, 0, 0);
+            y2[e] = mat[QK][4 * q + e][n16];
         }
 #pragma unroll
         for (int e = 0; e < 4; ++e) y2 = __builtin_amdgcn_mfma_f32_16x16x4f32(qb[e], tk[e], y2, 0, 0, 0);
@@ -480,12 +484,12 @@ __global__ __launch_bounds__(256) void wkv7_chunk_kernel(Prep7Args a, int t_begi
 #pragma unroll
         for (int e = 0; e < 4; ++e) { x[e] = la[4 * q + e][16 * wave + n16]; y[e] = lr[4 * q + e][16 * wave + n16]; }
         ta = add(zero, lz, x);
-        y1 = add(y, mat[3], ta);
+        y1 = add(y, mat[QB], ta);
         if (wave == 1) {
 #pragma unroll
-            for (int e = 0; e < 4; ++e) { x[e] = mat[0][4 * q + e][n16]; y[e] = mat[2][4 * q + e][n16]; }
+            for (int e = 0; e < 4; ++e) { x[e] = mat[AK][4 * q + e][n16]; y[e] = mat[QK][4 * q + e][n16]; }
             tk = add(zero, lz, x);
-            y2 = add(y, mat[3], tk);
+            y2 = add(y, mat[QB], tk);
         }
     }
     __syncthreads();
@@ -494,9 +498,10 @@ __global__ __launch_bounds__(256) void wkv7_chunk_kernel(Prep7Args a, int t_begi
     for (int e = 0; e < 4; ++e) {
         la[4 * q + e][16 * wave + n16] = ta[e];
         lr[4 * q + e][16 * wave + n16] = y1[e];
-        if (wave == 1) { mat[0][4 * q + e][n16] = tk[e]; mat[2][4 * q + e][n16] = y2[e]; }
+        if (wave == 1) { mat[AK][4 * q + e][n16] = tk[e]; mat[QK][4 * q + e][n16] = y2[e]; }
+        lv[256 * (g >> 2) + 4 * (4 * (g & 3) + e + 16 * (s >> 2)) + (s & 3)] = live ? vo[e] : (h16)0.f;
     }
-    const f32x4 rest = *(const f32x4 *)&lall[4 * g] * inv;                         // A_16 / A_s
+    const f32x4 rest = *(const f32x4 *)&la[g][HS7] * inv;                          // A_16 / A_s
     *(f32x4 *)&lk[s][4 * g] = kk2 * rest;
     *(f32x4 *)&lb[s][4 * g] = bb * rest;
     __syncthreads();
@@ -509,7 +514,8 @@ __global__ __launch_bounds__(256) void wkv7_chunk_kernel(Prep7Args a, int t_begi
     *(f32x4 *)(out + C7_B + 4 * tid) = bf;
     // wave jb of the second kernel takes the inner indices 4 q + jb of Y2 and TK
     typedef float f32x2 __attribute__((ext_vector_type(2)));
-    *(f32x2 *)(out + C7_2 + 2 * tid) = f32x2{mat[2][n16][4 * q + wave], mat[0][n16][4 * q + wave]};
+    *(f32x2 *)(out + C7_2 + 2 * tid) = f32x2{mat[QK][n16][4 * q + wave], mat[AK][n16][4 * q + wave]};
+    *(h16x4 *)((h16 *)(out + C7_V) + 4 * tid) = *(const h16x4 *)(lv + 4 * tid);
 }
 
 __global__ __launch_bounds__(256, 2) void wkv7_apply_kernel(int H, int C, float *state, float *y32, int t_begin, int nchunk, const float *scratch) {
@@ -596,6 +602,7 @@ __global__ __launch_bounds__(256, 2) void wkv7_apply_kernel(int H, int C, float 
     for (int c0 = 0; c0 < nchunk; c0 += PD) {
 #pragma unroll
         for (int u = 0; u < PD; ++u) {
+            if (c0 + u >= nchunk) break;
             step(ops[u], u & 1);
             fence();
             load(ops[u], c0 + u + PD);
@@ -1174,7 +1181,7 @@ extern "C" int rwkv_v7_forward(const rwkv_v7_model *m, const rwkv_v56_layer_stat
             a.an = ws.an; a.b = ws.b; a.dec = ws.dec; a.rk = ws.rk;
             if (T >= CHUNKED7) {
                 for (int64_t t0 = 0; t0 < T; t0 += SEG7) {
-                    const int nchunk = wkv_chunks(std::min<int64_t>(T - t0, SEG7));
+                    const int nchunk = (int)((std::min<int64_t>(T - t0, SEG7) + CL - 1) / CL);
                     hipLaunchKernelGGL(wkv7_chunk_kernel, dim3((unsigned)(H * nchunk)), dim3(256), 0, st, a, (int)t0, ws.chunks);
                     hipLaunchKernelGGL(wkv7_apply_kernel, dim3((unsigned)(4 * H)), dim3(256), 0, st, H, C, s.att_kv, ws.y32, (int)t0, nchunk, ws.chunks);
                 }

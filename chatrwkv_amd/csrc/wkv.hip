@@ -553,8 +553,9 @@ __global__ __launch_bounds__(256) void wkv56_chunk_kernel(Wkv56Args a, int H, in
     *(h16x4 *)((h16 *)(out + CH_V) + 4 * threadIdx.x) = *(const h16x4 *)(vf + 4 * threadIdx.x);
 }
 
+constexpr int GC = 4;   // chunks per exchange of y: one barrier each, and the sums of a group are read during the next
+static int wkv56_chunks(int tokens) { return (tokens + CL * GC - 1) / (CL * GC) * GC; }   // whole groups
 __global__ __launch_bounds__(256, 2) void wkv56_apply_kernel(Wkv56Args a, int H, int t_begin, int nchunk, const float *scratch) {
-    constexpr int GC = 4;   // chunks per exchange of y: one barrier each, and the sums of a group are read during the next
     __shared__ f32x4 red[2][GC][4][64];
     const int C = a.C;
     const int h = blockIdx.x % H, ib = blockIdx.x / H;
@@ -633,8 +634,10 @@ __global__ __launch_bounds__(256, 2) void wkv56_apply_kernel(Wkv56Args a, int H,
                 if (c0) store();                  // the second group of the turn before
                 exchange(0);
                 fence();
+                if (c0 + GC >= nchunk) break;
             }
         }
+        if (c0 + GC >= nchunk) break;
         store();
         exchange(1);
         fence();
@@ -642,7 +645,7 @@ __global__ __launch_bounds__(256, 2) void wkv56_apply_kernel(Wkv56Args a, int H,
     store();
 #pragma unroll
     for (int e = 0; e < 4; ++e) S[(16 * jb + 4 * q + e) * HS + i] = st[e];
-    if (any_wave(broken, (int *)red[0])) {                  // red[0]: read before the last barrier
+    if (any_wave(broken, (int *)red[nchunk / GC & 1])) {    // the buffer that was read before the last barrier
         yo -= (size_t)nchunk * CL * C;                      // the same thread stored these
         for (int c = 0; c < nchunk; ++c, yo += (size_t)CL * C) {
             Ops x;
@@ -768,7 +771,7 @@ int wkv56_fused_launch(bool v6, int T, int C, int H, float *state, const rwkv_ha
         }
         float *chunks = y32 + (size_t)wkv_chunks(T) * CL * C;   // y has a row for every padded token
         for (int t0 = 0; t0 < T && T >= WKV_CHUNKED; t0 += WKV_SEG) {
-            const int nchunk = wkv_chunks(std::min(T - t0, WKV_SEG));
+            const int nchunk = wkv56_chunks(std::min(T - t0, WKV_SEG));
             const dim3 grid((unsigned)(H * nchunk));
             if (v6) hipLaunchKernelGGL((wkv56_chunk_kernel<2>), grid, dim3(256), 0, st, a, H, t0, chunks);
             else hipLaunchKernelGGL((wkv56_chunk_kernel<0>), grid, dim3(256), 0, st, a, H, t0, chunks);
