@@ -1389,11 +1389,11 @@ __global__ __launch_bounds__(256) void mm8_prepare_group_kernel(int T, int N, Pr
 // ---- calls of 2 .. 16 rows: every weight row streamed once ---------------------------------------------------
 // A ragged last prompt chunk (rwkv/utils.py:98-101) or a short chat turn has a handful of tokens: with 128-row
 // tiles the contraction kernels spend their time on empty rows and a call costs several one-token steps.  Here
-// a workgroup of 16 waves, one per CU, takes a consecutive share of the launch's row groups (16 output rows each, the
+// (uint8) a workgroup of 16 waves, one per CU, takes a consecutive share of the launch's row groups (16 output rows each, the
 // groups of all members in one order) and splits K over its waves: wave w owns the 64-wide units w, w + 16, ...; per
-// unit a lane loads 16 (uint8) or 2 x 16 bytes (fp16) of one weight row (lane = row + 16 q) and multiplies them, uint8
-// widened to the exact fp16 value b + 1/2, with its token's values (lane = token + 16 q, rows past T repeat the last
-// one) by v_mfma_f32_16x16x32_f16, weights first, so that lane (token j, q) ends with rows 4 q .. 4 q + 3 of token j.
+// unit a lane loads 16 bytes of one weight row (lane = row + 16 q), widens them to the exact fp16 value b + 1/2 and
+// multiplies them with its token's values (lane = token + 16 q, rows past T repeat the last one) by
+// v_mfma_f32_16x16x32_f16, weights first, so that lane (token j, q) ends with rows 4 q .. 4 q + 3 of token j.
 // The 16 partial blocks are added in wave order through LDS (deterministic) by four of the waves, which round and store.
 // Bound by HBM: the next step's weights, of the next row group where this one's end, are requested before a step is
 // multiplied, and the barrier of an exchange waits for LDS only, so a wave always has a step in flight.  (A workgroup
@@ -1402,10 +1402,9 @@ __global__ __launch_bounds__(256) void mm8_prepare_group_kernel(int T, int N, Pr
 //   NU == 0  longer rows: the activations come from L2 with the weights.  Fragment order asks for 16 rows per 16 lanes,
 //            which the CU takes at 16 bytes a clock (9 TB/s over the chip from L2, 15.5 where four lanes ask for 64
 //            consecutive bytes): they are read eight lanes to a row and change order in LDS of the wave's own.
-// us a launch, 8 rows, against a workgroup per row group with fragment-order loads throughout: uint8, 4096 wide, three members
-// of 4096 outputs 18.7 -> 16.8, [8 x 16384] x [16384 x 4096] 22.9 -> 21.4, three of 5120 at 5120 wide 45.3 -> 28.9,
-// [8 x 20480] x [20480 x 5120] 51.9 -> 46.6 (320 row groups on 256 CUs); fp16, 4096 wide, three of 4096 25.5 -> 23.1,
-// [8 x 16384] x [16384 x 4096] 38.3 -> 33.6 (4.0 TB/s).
+// us a launch, 8 rows, against a workgroup per row group with fragment-order loads throughout: 4096 wide, three members of 4096
+// outputs 18.7 -> 16.8, [8 x 16384] x [16384 x 4096] 22.9 -> 21.4, three of 5120 at 5120 wide 45.3 -> 28.9, [8 x 20480] x
+// [20480 x 5120] 51.9 -> 46.6 (320 row groups on 256 CUs).  The same sums in the same order.
 struct SkinnyGroup {
     const h16 *A[4];
     const void *W[4];
@@ -1415,11 +1414,10 @@ struct SkinnyGroup {
     GemmEpi ep[4];
 };
 
-template <bool W_U8, int NU>
-__global__ __launch_bounds__(1024) void skinny_kernel(int T, int N, int n, int total, SkinnyGroup g) {
+template <int NU>
+__global__ __launch_bounds__(1024) void skinny_u8_kernel(int T, int N, int n, int total, SkinnyGroup g) {
     constexpr bool HELD = NU > 0;
-    constexpr int WL = W_U8 ? 1 : 2;                            // weight loads per unit
-    constexpr int UB = NU == 1 ? 1 : NU == 4 && W_U8 ? 4 : 2;   // units of a step
+    constexpr int UB = NU == 1 ? 1 : NU == 4 ? 4 : 2;           // units of a step
     constexpr int NS = HELD ? NU / UB : 2;                      // steps of a row group; NU == 0: of a pass of its loop
     constexpr int NB = HELD ? 2 : 1;                            // exchange buffers: with two, one barrier per row group
     constexpr int RQ = 80;                                      // floats per q of a block: the readers' banks differ
@@ -1430,27 +1428,19 @@ __global__ __launch_bounds__(1024) void skinny_kernel(int T, int N, int n, int t
     const int nunits = N / 64;
     const h16x2 off = {(h16)1023.5f, (h16)1023.5f};
     const int b0 = (int)((int64_t)total * blockIdx.x / gridDim.x), b1 = (int)((int64_t)total * (blockIdx.x + 1) / gridDim.x);
-    // the k's of a unit that a lane multiplies: two pieces of eight
-    const int p0 = W_U8 ? 2 * q : q, p1 = W_U8 ? 2 * q + 1 : 4 + q;
     auto fence = [] {                                           // loads are used in the order of their issue (v7.hip)
         asm volatile("" ::: "memory");
         __builtin_amdgcn_sched_barrier(0);
     };
-    auto multiply = [&](const u32x4 (&w)[WL], h16x8 x0, h16x8 x1, f32x4 &acc) {
-        if constexpr (W_U8) {
-            const u32x4 wv = w[0];
-            const h16x2 a0 = u8pair_lo_1024(wv.x) - off, a1 = u8pair_hi_1024(wv.x) - off;
-            const h16x2 a2 = u8pair_lo_1024(wv.y) - off, a3 = u8pair_hi_1024(wv.y) - off;
-            const h16x2 c0 = u8pair_lo_1024(wv.z) - off, c1 = u8pair_hi_1024(wv.z) - off;
-            const h16x2 c2 = u8pair_lo_1024(wv.w) - off, c3 = u8pair_hi_1024(wv.w) - off;
-            const h16x8 wa = {a0.x, a0.y, a1.x, a1.y, a2.x, a2.y, a3.x, a3.y};
-            const h16x8 wb = {c0.x, c0.y, c1.x, c1.y, c2.x, c2.y, c3.x, c3.y};
-            acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(wa, x0, acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(wb, x1, acc, 0, 0, 0);
-        } else {
-            acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h16x8, w[0]), x0, acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h16x8, w[1]), x1, acc, 0, 0, 0);
-        }
+    auto multiply = [&](u32x4 wv, h16x8 x0, h16x8 x1, f32x4 &acc) {
+        const h16x2 a0 = u8pair_lo_1024(wv.x) - off, a1 = u8pair_hi_1024(wv.x) - off;
+        const h16x2 a2 = u8pair_lo_1024(wv.y) - off, a3 = u8pair_hi_1024(wv.y) - off;
+        const h16x2 c0 = u8pair_lo_1024(wv.z) - off, c1 = u8pair_hi_1024(wv.z) - off;
+        const h16x2 c2 = u8pair_lo_1024(wv.w) - off, c3 = u8pair_hi_1024(wv.w) - off;
+        const h16x8 wa = {a0.x, a0.y, a1.x, a1.y, a2.x, a2.y, a3.x, a3.y};
+        const h16x8 wb = {c0.x, c0.y, c1.x, c1.y, c2.x, c2.y, c3.x, c3.y};
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(wa, x0, acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(wb, x1, acc, 0, 0, 0);
     };
     int base = 0, count = 0;                                    // row groups of the members before; done by this workgroup
     for (int gi = 0; gi < n; ++gi) {
@@ -1461,20 +1451,17 @@ __global__ __launch_bounds__(1024) void skinny_kernel(int T, int N, int n, int t
         const GemmEpi &ep = g.ep[gi];
         const h16 *A = g.A[gi];
         const unsigned char *W = (const unsigned char *)g.W[gi];
-        const int64_t ldw = g.ldw[gi] * (W_U8 ? 1 : 2);
+        const int64_t ldw = g.ldw[gi];
         // In place of a unit past the end of the row, and of every unit past the share's last row group, all lanes load the
         // first bytes of the matrix, which nothing uses: a branch around a load would make the waits for those before it longer.
-        struct Step { u32x4 w[UB][WL]; h16x8 x[HELD ? 1 : UB][2]; };
+        struct Step { u32x4 w[UB]; h16x8 x[HELD ? 1 : UB][2]; };
         auto load_w = [&](Step &s, int grp, int i0) {
             const bool there = grp < hi;
             const size_t row = (size_t)min(16 * grp + sub, M - 1) * ldw + 16 * q;
 #pragma unroll
             for (int i = 0; i < UB; ++i) {
                 const int u = wave + 16 * (i0 + i);
-                const bool ok = there && u < nunits;
-                const size_t at = ok ? row + (size_t)u * (64 * WL) : 0;
-#pragma unroll
-                for (int e = 0; e < WL; ++e) s.w[i][e] = __builtin_nontemporal_load((const u32x4 *)(W + at + (ok ? 64 * e : 0)));
+                s.w[i] = __builtin_nontemporal_load((const u32x4 *)(W + (there && u < nunits ? row + (size_t)u * 64 : 0)));
             }
         };
         struct Ops { rwkv_half rx, mx, res, gate; float s0, s2; };
@@ -1483,7 +1470,7 @@ __global__ __launch_bounds__(1024) void skinny_kernel(int T, int N, int n, int t
         auto load_ops = [&](int grp) {
             Ops o = {};
             const int t = min(ft, T - 1), m = min(16 * grp + fm, M - 1);
-            if constexpr (W_U8) { o.rx = ep.rx[m]; o.mx = ep.mx[m]; o.s0 = ep.s0[t]; o.s2 = ep.s2[t]; }
+            o.rx = ep.rx[m]; o.mx = ep.mx[m]; o.s0 = ep.s0[t]; o.s2 = ep.s2[t];
             o.res = *(has_res ? ep.res + (size_t)t * ep.ldres + m : (const rwkv_half *)A);
             o.gate = *(has_gate ? ep.gate + (size_t)t * ep.ldgate + m : (const rwkv_half *)A);
             return o;
@@ -1506,7 +1493,7 @@ __global__ __launch_bounds__(1024) void skinny_kernel(int T, int N, int n, int t
                 const int m = 16 * grp + fm;
                 if (m < M && ft < T) {
                     const size_t at = (size_t)ft * g.ldy[gi] + m;
-                    if constexpr (W_U8) v = epi_affine(v, h2f(o.rx), h2f(o.mx), o.s0, o.s2);
+                    v = epi_affine(v, h2f(o.rx), h2f(o.mx), o.s0, o.s2);
                     if (ep.raw_f32) {
                         ((float *)g.Y[gi])[at] = v;
                     } else {
@@ -1529,8 +1516,8 @@ __global__ __launch_bounds__(1024) void skinny_kernel(int T, int N, int n, int t
             for (int i = 0; i < NU; ++i) {
                 const int u = wave + 16 * i;
                 const h16 *p = arow + (size_t)min(u, nunits - 1) * 64;
-                rx[i][0] = *(const h16x8 *)(p + 8 * p0);
-                rx[i][1] = *(const h16x8 *)(p + 8 * p1);
+                rx[i][0] = *(const h16x8 *)(p + 16 * q);
+                rx[i][1] = *(const h16x8 *)(p + 16 * q + 8);
             }
             fence();
             load_w(st[0], lo, 0);
@@ -1561,7 +1548,7 @@ __global__ __launch_bounds__(1024) void skinny_kernel(int T, int N, int n, int t
             const size_t xa = (size_t)min(r8, T - 1) * g.lda + 8 * seg, xb = (size_t)min(r8 + 8, T - 1) * g.lda + 8 * seg;
             h16 *slot = sx[wave];
             h16 *wr = slot + 64 * r8 + 8 * (seg ^ r8);           // (r8 + 8) & 7 == r8
-            const h16 *rd0 = slot + 64 * sub + 8 * (p0 ^ (sub & 7)), *rd1 = slot + 64 * sub + 8 * (p1 ^ (sub & 7));
+            const h16 *rd0 = slot + 64 * sub + 8 * (2 * q ^ (sub & 7)), *rd1 = slot + 64 * sub + 8 * ((2 * q + 1) ^ (sub & 7));
             auto load = [&](Step &s, int grp, int i0) {
 #pragma unroll
                 for (int i = 0; i < UB; ++i) {
@@ -1601,9 +1588,86 @@ __global__ __launch_bounds__(1024) void skinny_kernel(int T, int N, int n, int t
     }
 }
 
+// fp16 weights: a workgroup per 16 output rows (two to a CU), the same split of K over its waves: wave w owns the 32-wide
+// chunks w, w + 16, ...  NCI > 0: a wave owns at most NCI chunks and keeps their activation values in registers; NCI == 0: any
+// row length, activations re-read from L2 for every row group.  The uint8 form above with units of two neighbouring chunks, a
+// whole line of a row, is 5 to 15 % faster per call, but adds in another order, and a deep RWKV-7 model at the start of a
+// conversation makes 8 % of that (2-norm of its state); with these chunks, half a line to a request, it is up to 4 % slower in
+// calls of 2 tokens (RWKV-7, 4096 wide, us a layer: 142.9 / 148.6).
+template <int NCI>
+__global__ __launch_bounds__(1024) void skinny_f16_kernel(int T, int N, SkinnyGroup g) {
+    __shared__ float red[16][64][4];
+    const int gi = blockIdx.y, M = g.M[gi];
+    const h16 *__restrict__ A = g.A[gi];
+    const unsigned char *__restrict__ W = (const unsigned char *)g.W[gi];
+    const int64_t lda = g.lda, ldw = g.ldw[gi];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int sub = lane & 15, q = lane >> 4;
+    const int nchunks = N / 32;
+    const int ngroups = (M + 15) >> 4;
+    const h16 *arow = A + (size_t)min(sub, T - 1) * lda;   // this lane's token
+    constexpr int NB = NCI > 0 ? NCI : 4;            // chunks loaded before any is multiplied
+    auto load_x = [&](int c) { return *(const h16x8 *)(arow + (size_t)c * 32 + 8 * q); };
+    auto load_w = [&](const unsigned char *wrow, int c) {
+        return __builtin_nontemporal_load((const u32x4 *)(wrow + ((size_t)c * 32 + 8 * q) * 2));
+    };
+    auto multiply = [&](u32x4 wv, h16x8 x, f32x4 &acc) {
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h16x8, wv), x, acc, 0, 0, 0);
+    };
+    // chunks past the end of the row repeat the last one and multiply zeros: no branch sits between the loads and
+    // their use (loads would be sunk behind it, one chunk in flight at a time)
+    h16x8 rx[NB];
+    if (NCI > 0) {
+#pragma unroll
+        for (int i = 0; i < NB; ++i) {
+            rx[i] = load_x(min(wave + 16 * i, nchunks - 1));
+            if (wave + 16 * i >= nchunks) rx[i] = h16x8{};
+        }
+    }
+    for (int grp = blockIdx.x; grp < ngroups; grp += gridDim.x) {
+        const int m0 = grp << 4;
+        const unsigned char *wrow = W + (size_t)min(m0 + sub, M - 1) * ldw * 2;
+        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+        if (NCI > 0) {
+            u32x4 wv[NB];
+#pragma unroll
+            for (int i = 0; i < NB; ++i) wv[i] = load_w(wrow, min(wave + 16 * i, nchunks - 1));
+#pragma unroll
+            for (int i = 0; i < NB; ++i) multiply(wv[i], rx[i], acc);
+        } else {
+            for (int c0 = wave; c0 < nchunks; c0 += 16 * NB) {
+                u32x4 wv[NB];
+                h16x8 x[NB];
+#pragma unroll
+                for (int i = 0; i < NB; ++i) {
+                    const int c = min(c0 + 16 * i, nchunks - 1);
+                    wv[i] = load_w(wrow, c);
+                    x[i] = load_x(c);
+                }
+#pragma unroll
+                for (int i = 0; i < NB; ++i) {
+                    if (c0 + 16 * i >= nchunks) x[i] = h16x8{};
+                    multiply(wv[i], x[i], acc);
+                }
+            }
+        }
+        __syncthreads();                                          // the previous group's sums have been read
+        *(f32x4 *)&red[wave][lane][0] = acc;
+        __syncthreads();
+        if (threadIdx.x < 256) {
+            const int l = threadIdx.x & 63, r = threadIdx.x >> 6;
+            float v = 0.f;
+#pragma unroll
+            for (int w = 0; w < 16; ++w) v += red[w][l][r];
+            const int m = m0 + 4 * (l >> 4) + r, t = l & 15;
+            if (m < M && t < T) gemm_epilogue(v, t, m, 1.f, 0.f, g.ep[gi], g.Y[gi], g.ldy[gi]);
+        }
+    }
+}
+
 constexpr int SKINNY_MAX_ROWS = 16;
 
-// what skinny_kernel assumes of one product: whole units, 16-byte aligned rows for its 16-byte loads
+// what these kernels assume of one product: whole units or chunks, 16-byte aligned rows for its 16-byte loads
 bool skinny_ok(bool w_u8, int64_t T, int64_t N, const void *A, int64_t lda, const void *W, int64_t ldw, const GemmEpi &ep) {
     auto a16 = [](const void *p) { return (((uintptr_t)p) & 15) == 0; };
     if (T < 2 || T > SKINNY_MAX_ROWS || N < 64 || (N % 64)) return false;
@@ -1615,14 +1679,18 @@ bool skinny_ok(bool w_u8, int64_t T, int64_t N, const void *A, int64_t lda, cons
 }
 
 int skinny_launch(bool w_u8, int n, int64_t T, int64_t N, const SkinnyGroup &g, hipStream_t st) {
-    int total = 0;
-    for (int i = 0; i < n; ++i) total += (g.M[i] + 15) / 16;
-    const dim3 grid((unsigned)std::min(total, num_cu()));
-    const int64_t per_wave = (N / 64 + 15) / 16;                  // units a wave owns
-#define RWKV_SKINNY(NU)                                                                                                  \
-    do {                                                                                                                 \
-        if (w_u8) hipLaunchKernelGGL((skinny_kernel<true, NU>), grid, dim3(1024), 0, st, (int)T, (int)N, n, total, g);   \
-        else hipLaunchKernelGGL((skinny_kernel<false, NU>), grid, dim3(1024), 0, st, (int)T, (int)N, n, total, g);       \
+    int total = 0, maxg = 1;
+    for (int i = 0; i < n; ++i) {
+        total += (g.M[i] + 15) / 16;
+        maxg = std::max(maxg, (g.M[i] + 15) / 16);
+    }
+    const int64_t per_wave = (N / (w_u8 ? 64 : 32) + 15) / 16;    // chunks a wave owns
+#define RWKV_SKINNY(NC)                                                                                                              \
+    do {                                                                                                                             \
+        if (w_u8) hipLaunchKernelGGL((skinny_u8_kernel<NC>), dim3((unsigned)std::min(total, num_cu())), dim3(1024), 0, st, (int)T,   \
+                                     (int)N, n, total, g);                                                                           \
+        else hipLaunchKernelGGL((skinny_f16_kernel<NC>), dim3((unsigned)std::min(maxg, 2 * num_cu()), (unsigned)n), dim3(1024), 0,   \
+                                st, (int)T, (int)N, g);                                                                              \
     } while (0)
     if (per_wave <= 1) RWKV_SKINNY(1);
     else if (per_wave <= 2) RWKV_SKINNY(2);
