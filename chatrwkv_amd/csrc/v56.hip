@@ -450,7 +450,7 @@ extern "C" int rwkv_v56_forward(const rwkv_v56_model *m, const rwkv_v56_layer_st
             if ((rc = lnmix_seq_launch(a, nj, st))) return rc;
             kx = ws.mix[0]; vx = ws.mix[1]; rx = ws.mix[2]; gx = gated ? ws.mix[3] : nullptr;
         }
-        // the first matrix call also commits the new token-shift state (all readers of the old one are done)
+        // one token: the first matrix call also commits the new token-shift state (all readers of the old one are done)
         if (T == 1 && C <= 8 * 512) {
             // one launch for the receptance, key, value (and gate) rows
             MultiVecArgs a{};
@@ -497,7 +497,7 @@ extern "C" int rwkv_v56_forward(const rwkv_v56_model *m, const rwkv_v56_layer_st
             ForkScope par(ss, st, 2, !dma_seq);
             Ctx cr = c;
             if (par) cr.splitk = nullptr;
-            if ((rc = mm(cr, l.att_receptance, u8, rx, ACT_NONE, nullptr, nullptr, 1.f, ws.r))) return rc;
+            if ((rc = mm(cr, l.att_receptance, u8, rx, ACT_NONE, nullptr, nullptr, 1.f, ws.r, ws.xx_att, T == 1 ? s.att_xx : nullptr, C))) return rc;
             if ((rc = mm(par ? cs[0] : c, l.att_key, u8, kx, ACT_NONE, nullptr, nullptr, 1.f, ws.k))) return rc;
             if ((rc = mm(par ? cs[1] : c, l.att_value, u8, vx, ACT_NONE, nullptr, nullptr, 1.f, ws.v))) return rc;
             if (gated && (rc = mm(c, l.att_gate, u8, gx, ACT_SILU, nullptr, nullptr, 1.f, ws.g))) return rc;
