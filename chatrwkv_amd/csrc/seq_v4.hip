@@ -68,10 +68,9 @@ __global__ __launch_bounds__(256) void lnmix_seq_kernel(SeqMixArgs a) {
         h16x8 pv = xx;
         if (shift) pv = t > 0 ? row_norm8(xp + 8 * j8, pmean, prstd, wv, bv) : *(const h16x8 *)(a.sx + 8 * j8);
         if (a.xx_last && t == a.T - 1) *(h16x8 *)(a.xx_last + 8 * j8) = xx;
-        const Shift8 sh = shift8(xx, pv, a.maa_form);
 #pragma unroll
         for (int j = 0; j < NJ; ++j) {
-            const h16x8 kx = a.mix[j] ? mix8(xx, pv, sh, *(const h16x8 *)(a.mix[j] + 8 * j8), a.maa_form) : xx;
+            const h16x8 kx = a.mix[j] ? mix8(xx, pv, *(const h16x8 *)(a.mix[j] + 8 * j8), a.maa_form) : xx;
             h16x8 o = kx;
             if (a.ry[j]) {
                 o = kx * *(const h16x8 *)(a.ry[j] + 8 * j8);
@@ -205,14 +204,13 @@ __global__ __launch_bounds__(NT) void lnmix_seq_fast_kernel(SeqMixArgs a) {
             else pv = *(const h16x8 *)(a.sx + 8 * j8);
         }
         if (a.xx_last && t == a.T - 1) *(h16x8 *)(a.xx_last + 8 * j8) = xx;
-        const Shift8 sh = shift8(xx, pv, a.maa_form);
 #pragma unroll
         for (int j = 0; j < NJ; ++j) {
             h16x8 kx = xx;
             if (a.mix[j]) {
                 h16x8 m8;
                 if constexpr (PRE) m8 = mv[j][c]; else m8 = *(const h16x8 *)(a.mix[j] + 8 * j8);
-                kx = mix8(xx, pv, sh, m8, a.maa_form);
+                kx = mix8(xx, pv, m8, a.maa_form);
             }
             h16x8 o = kx;
             if (a.ry[j]) {

@@ -73,11 +73,10 @@ __global__ __launch_bounds__(NT) void v6_mix1_kernel(Mix1Args a) {
         } else {
             pv = *(const h16x8 *)(a.sx + 8 * j8);
         }
-        const Shift8 sh = shift8(xx, pv, true);
         const size_t o = (size_t)t * C + 8 * j8;
         *(h16x8 *)(a.xx + o) = xx;
-        *(h16x8 *)(a.sxd + o) = sh.d16;
-        *(h16x8 *)(a.xxx + o) = mix8(xx, pv, sh, mv[c], true);
+        *(h16x8 *)(a.sxd + o) = pv - xx;
+        *(h16x8 *)(a.xxx + o) = mix8(xx, pv, mv[c], true);
         // the new token-shift state: written by row 0's workgroup, the only one that reads the old state, each thread
         // exactly the chunk it has just read
         if (commit) {
