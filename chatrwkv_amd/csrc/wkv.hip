@@ -37,17 +37,20 @@ template <> struct Wkv4IO<2> {
     DEV void st(size_t i, float wkv, float rr) const { y[i] = f2h(rr * round_h(wkv)); }
 };
 
+// Sums of two products as one product that is rounded and one that is not, spelled out: left to the compiler, which of the two
+// that is depended on a token's place in its batch of eight, and with it the last bit of the state.
+DEV float wkv4_sum(float e1, float a, float e2, float v) { return __builtin_fmaf(e1, a, e2 * v); }
 DEV void wkv4_step(float kk, float vv, float u, float w, float &aa, float &bb, float &pp, float &out) {
     float ww = u + kk;
     float p = fmaxf(pp, ww);
     float e1 = __expf(pp - p), e2 = __expf(ww - p);
-    out = (e1 * aa + e2 * vv) / (e1 * bb + e2);
+    out = wkv4_sum(e1, aa, e2, vv) / __builtin_fmaf(e1, bb, e2);
     ww = w + pp;
     p = fmaxf(ww, kk);
     e1 = __expf(ww - p);
     e2 = __expf(kk - p);
-    aa = e1 * aa + e2 * vv;
-    bb = e1 * bb + e2;
+    aa = wkv4_sum(e1, aa, e2, vv);
+    bb = __builtin_fmaf(e1, bb, e2);
     pp = p;
 }
 
@@ -121,8 +124,8 @@ __global__ __launch_bounds__(64) void wkv4_kernel(int T, int C, const float *__r
 DEV void wkv4_merge(float &a, float &b, float &p, float a2, float b2, float p2) {
     const float q = fmaxf(p, p2);
     const float e1 = __expf(p - q), e2 = __expf(p2 - q);
-    a = e1 * a + e2 * a2;
-    b = e1 * b + e2 * b2;
+    a = wkv4_sum(e1, a, e2, a2);
+    b = wkv4_sum(e1, b, e2, b2);
     p = q;
 }
 
@@ -142,8 +145,8 @@ __global__ __launch_bounds__(64) void wkv4_chunk_summary_kernel(int T, int C, in
         const float ww = w + pp;
         const float p = fmaxf(ww, kk);
         const float e1 = __expf(ww - p), e2 = __expf(kk - p);
-        aa = e1 * aa + e2 * vv;
-        bb = e1 * bb + e2;
+        aa = wkv4_sum(e1, aa, e2, vv);
+        bb = __builtin_fmaf(e1, bb, e2);
         pp = p;
     });
     float *o = scratch + (size_t)(j + 1) * 3 * C;

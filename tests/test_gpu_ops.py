@@ -542,6 +542,24 @@ def test_wkv4(T, C):
         np.testing.assert_allclose(tp.cpu().numpy(), p_ref, rtol=1e-5, atol=1e-5)
 
 
+@pytest.mark.parametrize("T", [2, 8, 37, 63])
+def test_wkv4_bits_do_not_depend_on_a_tokens_place(T):
+    """One call, and the same tokens one call each: the recurrence of a call that is not cut into chunks rounds every token
+    alike, wherever in the kernel's batches of eight it stands, so outputs and state agree bit for bit."""
+    ops = _ops()
+    C = 768
+    r = _rng(T)
+    k, v = (torch.from_numpy(r.standard_normal((T, C)).astype(np.float32)).to(DEV) for _ in range(2))
+    w = torch.from_numpy(-np.exp(r.uniform(-6, -1, C)).astype(np.float32)).to(DEV)
+    u = torch.from_numpy(r.uniform(-1, 1, C).astype(np.float32)).to(DEV)
+    one, each = ([torch.zeros(C, device=DEV), torch.zeros(C, device=DEV), torch.full((C,), -1e30, device=DEV)] for _ in range(2))
+    y = ops.cuda_wkv(T, C, w, u, k, v, *one)[0]
+    for t in range(T):
+        yt = ops.cuda_wkv(1, C, w, u, k[t:t + 1].contiguous(), v[t:t + 1].contiguous(), *each)[0]
+        assert torch.equal(yt[0], y[t]), t
+    assert all(torch.equal(a, b) for a, b in zip(one, each))
+
+
 @pytest.mark.parametrize("T,H", [(1, 2), (5, 3), (16, 2), (17, 2), (50, 4), (256, 64)])
 @pytest.mark.parametrize("v6", [False, True])
 @pytest.mark.parametrize("layout", [0, 1])
