@@ -2003,6 +2003,7 @@ int launch_pick(int cfg, int ks, int64_t T, int64_t N, int64_t M, const rwkv_hal
         case CFG_DMA + TILE_N: return launch_dma<W_U8, 64, 128, 4, 4>(ks, T, N, M, A, lda, W, ldw, Y, ldy, ep, st);
         case CFG_DMA + TILE_K8:
         case CFG_DMA + TILE_K4: {
+            if (!dma_ok(W_U8, N, M, A, lda, W, ldw, Y, ldy, ep)) return RWKV_E_LAYOUT;
             GemmGroup g{};
             g.A[0] = (const h16 *)A; g.W[0] = W; g.Y[0] = Y; g.lda = lda; g.ldw[0] = ldw; g.ldy[0] = ldy; g.M[0] = (int)M; g.ep[0] = ep;
             g.nk_split = (int)(N / BK) / ks;

@@ -252,6 +252,22 @@ def test_forced_tile_configurations(N, M, B, monkeypatch):
             call()
 
 
+@pytest.mark.parametrize("cfg", ["14", "15", "20", "21"])
+def test_forced_direct_to_lds_tiles_refuse_other_layouts(cfg, monkeypatch):
+    """RWKV_GEMM_CFG (tuning): operands that the direct-to-LDS kernels do not take -- here mx on no 16-byte boundary -- are
+    refused by every one of their tiles, before anything is launched on them."""
+    from chatrwkv_amd import lib
+    N, M, B = 128, 72, 40
+    x, (q, mx, rx, my, ry), want, _ = _affine_case(N, M, B, 7)
+    odd = torch.empty(M + 1, dtype=torch.float16, device=DEV)[1:]
+    odd.copy_(torch.from_numpy(mx))
+    args = (torch.from_numpy(x).to(DEV), _to_dev_ic(q), odd, *(torch.from_numpy(a).to(DEV) for a in (rx, my, ry)))
+    assert np.array_equal(_ops().cuda_mm8_seq(B, N, M, *args).cpu().numpy(), want)
+    monkeypatch.setenv("RWKV_GEMM_CFG", cfg)
+    with pytest.raises(lib.RwkvHipError):
+        _ops().cuda_mm8_seq(B, N, M, *args)
+
+
 @pytest.mark.parametrize("N,M,B", [(4096, 4096, 100), (768, 3072, 513), (64, 130, 17), (1024, 16384, 1024)])
 @pytest.mark.parametrize("which", ["mx", "rx"])
 def test_mm8_scales_on_any_boundary(N, M, B, which):
