@@ -96,75 +96,75 @@ DEV bool enough(SumCount t, float top_p, int top_k) { return top_k >= 0 ? t.n >=
 // The largest bit pattern c in [lo, hi) that holds, from the n <= LIST_MAX entries of [lo, hi) in LDS: it holds at lo (the
 // entries from there on: at_lo) and not at hi (at_hi).
 DEV unsigned search_list(const float *list, int n, unsigned lo, unsigned hi, SumCount at_lo, SumCount at_hi, float top_p, int top_k,
-                         float *tail, f32x4 (&red)[2][SWAVES / 2], int &turn) {
+                         f32x4 (&tail)[16], f32x4 (&red)[2][SWAVES / 2], int &turn) {
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const SumCount past_hi = at_hi;
-            float left = (float)n;   // entries still between the bounds
-            while (hi - lo > 1 && left > 64.f) {
-                const unsigned step = (hi - lo) / (SWAVES + 1) + 1;
-                const unsigned c = lo + step * (wave + 1);
-                SumCount t = at_hi;      // the totals at hi and past it
-                if (c < hi) {
-                    const float fc = __uint_as_float(c);
-                    float sc = 0.f, k = 0.f;
-                    for (int i = lane; i < n; i += 64) {
-                        const float v = list[i];
-                        if (v >= fc) { sc += v; k += 1.f; }
-                    }
-                    t.s = past_hi.s + wave_sum(sc);
-                    t.n = past_hi.n + wave_sum(k);
-                }
-                f32x4 *buf = red[turn];
-                turn ^= 1;
-                if (lane == 0) {
-                    ((float *)buf)[2 * wave] = t.s;
-                    ((float *)buf)[2 * wave + 1] = t.n;
-                }
-                __syncthreads();
-                int good = 0;            // the bounds that hold are a leading run up to rounding: take the largest
-                SumCount above_good = at_hi;
-    #pragma unroll
-                for (int w = SWAVES - 1; w >= 0; --w) {
-                    const SumCount q = {((float *)buf)[2 * w], ((float *)buf)[2 * w + 1]};
-                    if (good == 0) {
-                        if (lo + step * (w + 1) < hi && enough(q, top_p, top_k)) { good = w + 1; at_lo = q; }
-                        else above_good = q;
-                    }
-                }
-                hi = min(hi, lo + step * (good + 1));
-                lo = lo + step * good;
-                at_hi = above_good;
-                left = at_lo.n - at_hi.n;
+    float left = (float)n;   // entries still between the bounds
+    while (hi - lo > 1 && left > 64.f) {
+        const unsigned step = (hi - lo) / (SWAVES + 1) + 1;
+        const unsigned c = lo + step * (wave + 1);
+        SumCount t = at_hi;      // the totals at hi and past it
+        if (c < hi) {
+            const float fc = __uint_as_float(c);
+            float sc = 0.f, k = 0.f;
+            for (int i = lane; i < n; i += 64) {
+                const float v = list[i];
+                if (v >= fc) { sc += v; k += 1.f; }
             }
-            if (hi - lo <= 1) return lo;
-            // at most 64 are left: one to a lane, in list order; the largest of them at which the condition holds is the answer
-            {
-                const float l1 = __uint_as_float(max(lo, 1u)), h1 = __uint_as_float(hi);
-                if (wave == 0) {
-                    int at64 = 0;
-                    for (int i0 = 0; i0 < n; i0 += 64) {
-                        const float v = i0 + lane < n ? list[i0 + lane] : 0.f;
-                        const bool in = v >= l1 && v < h1;
-                        const unsigned long long m = __ballot(in);
-                        if (in) tail[min(at64 + (int)__popcll(m & ((1ull << lane) - 1)), 63)] = v;
-                        at64 += (int)__popcll(m);
-                    }
-                    if (lane >= at64) tail[lane] = 0.f;
-                }
-                __syncthreads();
-                const float mine64 = tail[lane];
-                SumCount t = at_hi;
-    #pragma unroll 2
-                for (int i = 0; i < 64; i += 4) {
-                    const f32x4 v = *(const f32x4 *)&tail[i];
-    #pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        if (v[e] >= mine64) { t.s += v[e]; t.n += v[e] > 0.f ? 1.f : 0.f; }
-                }
-                const float best = wave_max(mine64 > 0.f && enough(t, top_p, top_k) ? mine64 : 0.f);
-                __syncthreads();         // the lists may be written again
-                if (best > 0.f) lo = __float_as_uint(best);
+            t.s = past_hi.s + wave_sum(sc);
+            t.n = past_hi.n + wave_sum(k);
+        }
+        f32x4 *buf = red[turn];
+        turn ^= 1;
+        if (lane == 0) {
+            ((float *)buf)[2 * wave] = t.s;
+            ((float *)buf)[2 * wave + 1] = t.n;
+        }
+        __syncthreads();
+        int good = 0;            // the bounds that hold are a leading run up to rounding: take the largest
+        SumCount above_good = at_hi;
+#pragma unroll
+        for (int w = SWAVES - 1; w >= 0; --w) {
+            const SumCount q = {((float *)buf)[2 * w], ((float *)buf)[2 * w + 1]};
+            if (good == 0) {
+                if (lo + step * (w + 1) < hi && enough(q, top_p, top_k)) { good = w + 1; at_lo = q; }
+                else above_good = q;
             }
+        }
+        hi = min(hi, lo + step * (good + 1));
+        lo = lo + step * good;
+        at_hi = above_good;
+        left = at_lo.n - at_hi.n;
+    }
+    if (hi - lo <= 1) return lo;
+    // at most 64 are left: one to a lane, in list order; the largest of them at which the condition holds is the answer
+    {
+        const float l1 = __uint_as_float(max(lo, 1u)), h1 = __uint_as_float(hi);
+        if (wave == 0) {
+            int at64 = 0;
+            for (int i0 = 0; i0 < n; i0 += 64) {
+                const float v = i0 + lane < n ? list[i0 + lane] : 0.f;
+                const bool in = v >= l1 && v < h1;
+                const unsigned long long m = __ballot(in);
+                if (in) ((float *)tail)[min(at64 + (int)__popcll(m & ((1ull << lane) - 1)), 63)] = v;
+                at64 += (int)__popcll(m);
+            }
+            if (lane >= at64) ((float *)tail)[lane] = 0.f;
+        }
+        __syncthreads();
+        const float mine64 = ((float *)tail)[lane];
+        SumCount t = at_hi;
+#pragma unroll 2
+        for (int i = 0; i < 16; ++i) {
+            const f32x4 v = tail[i];
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                if (v[e] >= mine64) { t.s += v[e]; t.n += v[e] > 0.f ? 1.f : 0.f; }
+        }
+        const float best = wave_max(mine64 > 0.f && enough(t, top_p, top_k) ? mine64 : 0.f);
+        __syncthreads();         // the lists may be written again
+        if (best > 0.f) lo = __float_as_uint(best);
+    }
     return lo;
 }
 
@@ -175,7 +175,7 @@ template <int SROWS, bool POW>
 DEV void sample_one_workgroup(const SampleArgs &a) {
     __shared__ f32x4 red[2][SWAVES / 2];
     __shared__ float list[LIST_MAX];
-    __shared__ __align__(16) float tail[64];
+    __shared__ f32x4 tail[16];
     __shared__ __align__(16) float seg[ROWS_MAX * SWAVES];   // sums of the runs of 256 entries, in index order
     __shared__ int pick_seg, pick_tok;
     __shared__ float pick_before, pick_target;
@@ -585,7 +585,8 @@ __global__ __launch_bounds__(256) void sample_probs_kernel(SampleArgs a, SampleW
 template <int SROWS, bool POW>
 __global__ __launch_bounds__(STHREADS) void sample_draw_kernel(SampleArgs a, SampleWs ws) {
     __shared__ f32x4 red[2][SWAVES / 2];
-    __shared__ float list[LIST_MAX], tail[64], seg_sum[SEGS_MAX];
+    __shared__ f32x4 tail[16];
+    __shared__ float list[LIST_MAX], seg_sum[SEGS_MAX];
     __shared__ __align__(16) float cols[2 * BOUNDS][SWAVES + 4], few[FEW], sorted[FEW];
     __shared__ int pick, n_few[2];
     const int V = a.V, tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), segs = gridDim.x;
