@@ -172,7 +172,7 @@ DEV unsigned search_list(const float *list, int n, unsigned lo, unsigned hi, Sum
 // SROWS: group rows, at least V / 4096.  Rows past the end hold zeros and are worked on like the others: with a test
 // of V around each row the compiler made a copy of what follows for every number of rows.
 template <int SROWS, bool POW>
-DEV void sample_one_workgroup(const SampleArgs &a) {
+__global__ __launch_bounds__(STHREADS) void sample_kernel(SampleArgs a) {
     __shared__ f32x4 red[2][SWAVES / 2];
     __shared__ float list[LIST_MAX];
     __shared__ f32x4 tail[16];
@@ -440,9 +440,6 @@ DEV void sample_one_workgroup(const SampleArgs &a) {
     }
 }
 
-template <int SROWS, bool POW>
-__global__ __launch_bounds__(STHREADS) void sample_kernel(SampleArgs a) { sample_one_workgroup<SROWS, POW>(a); }
-
 // ---- the same draw over the chip -------------------------------------------------------------------------------
 // One workgroup issues every instruction of a pass over 65536 entries 256 times per SIMD, half a microsecond each, and the
 // exponential alone takes twenty.  With scratch from the caller the passes over the vocabulary run on one workgroup per
@@ -453,8 +450,8 @@ __global__ __launch_bounds__(STHREADS) void sample_kernel(SampleArgs a) { sample
 //           the nucleus can need: those below (1 - top_p) / 2 V cannot add up to what may be left out;
 //   draw:   every workgroup finds the cut for itself -- the bounds leave half an octave, whose entries are searched as in
 //           the kernel above -- and draws; it writes the filtered probabilities and the occurrence counts of its segment.
-// Sums are added in a fixed order throughout.  Where the total is no positive number the last launch's first workgroup does
-// the whole draw as the kernel above.
+// Sums are added in a fixed order throughout.  Where the total is no positive number (a NaN, an infinity or nothing but masks
+// among the logits) nothing is kept and id 0 is drawn, which is what the kernel above makes of such logits.
 // Bound by the latency of the three launches.  Measured as above, V = 65536: 21.5 us a draw (2.7 + 4.3 + 12.7 and the gaps), 39 with one
 // workgroup; with the lists in LDS and the bracket searched by search_list 25.8, 5 us of it in the search.
 constexpr int SEG = 1024, SEGS_MAX = 64, BOUNDS = 32;
@@ -582,7 +579,7 @@ __global__ __launch_bounds__(256) void sample_probs_kernel(SampleArgs a, SampleW
     }
 }
 
-template <int SROWS, bool POW>
+template <bool POW>
 __global__ __launch_bounds__(STHREADS) void sample_draw_kernel(SampleArgs a, SampleWs ws) {
     __shared__ f32x4 red[2][SWAVES / 2];
     __shared__ f32x4 tail[16];
@@ -616,8 +613,25 @@ __global__ __launch_bounds__(STHREADS) void sample_draw_kernel(SampleArgs a, Sam
     const Soft st = soft_total(ws.soft, segs);
     const float pmax = 1.f / st.sum;
     const float all = wave_sum(lane < segs ? ws.part[lane * PART + 2 * BOUNDS] : 0.f);
-    if (!(st.sum > 0.f && st.sum < INFINITY) || (top_p > 0.f && !(all >= 0.5f + 0.5f * top_p))) {
-        if (blockIdx.x == 0) sample_one_workgroup<SROWS, POW>(a);
+    // token, and the occurrence table: decay, then add the drawn token's weight
+    auto store = [&](int tok) {
+        if (blockIdx.x == 0 && tid == 0) *a.token = tok;
+        if (a.seen && own < V && (seen_own || own == tok)) {
+            const float w = own == tok ? (a.weight ? a.weight[tok] : 1.f) : 0.f;
+            float o = w;
+            if (seen_own) {
+                o = a.occ[own] * a.decay;
+                if (own == tok) o += w;
+            } else {
+                a.seen[own] = 1;
+            }
+            a.occ[own] = o;
+        }
+    };
+    // all: NaN where soft_total left out the NaN of a segment that is masked otherwise
+    if (!(st.sum > 0.f && st.sum < INFINITY && all > 0.f)) {
+        if (a.probs && own < V) a.probs[own] = 0.f;
+        store(0);
         return;
     }
     const float len = lane < segs ? ws.part[lane * PART + 2 * BOUNDS + 1] : 0.f;
@@ -804,20 +818,7 @@ __global__ __launch_bounds__(STHREADS) void sample_draw_kernel(SampleArgs a, Sam
         if (lane == 0) pick = some ? from * SEG + (found >= 0 ? found : last) : 0;
     }
     __syncthreads();
-    const int tok = pick;
-    if (blockIdx.x == 0 && tid == 0) *a.token = tok;
-    // ---- occurrence table: decay, then add the drawn token's weight
-    if (a.seen && own < V && (seen_own || own == tok)) {
-        const float w = own == tok ? (a.weight ? a.weight[tok] : 1.f) : 0.f;
-        float o = w;
-        if (seen_own) {
-            o = a.occ[own] * a.decay;
-            if (own == tok) o += w;
-        } else {
-            a.seen[own] = 1;
-        }
-        a.occ[own] = o;
-    }
+    store(pick);
 }
 
 }  // namespace
@@ -940,14 +941,8 @@ extern "C" int rwkv_sample_logits_ws(const float *logits, int64_t V, float tempe
     const bool pow = temperature != 0.f && temperature != 1.f;
     hipLaunchKernelGGL(sample_adjust_kernel, grid, dim3(256), 0, st, a, ws);
     hipLaunchKernelGGL(sample_probs_kernel, grid, dim3(256), 0, st, a, ws);
-#define RWKV_DRAW(ROWS)                                                                                            \
-    do {                                                                                                           \
-        if (pow) hipLaunchKernelGGL((sample_draw_kernel<ROWS, true>), grid, dim3(STHREADS), 0, st, a, ws);       \
-        else hipLaunchKernelGGL((sample_draw_kernel<ROWS, false>), grid, dim3(STHREADS), 0, st, a, ws);          \
-    } while (0)
-    if (V <= 13 * 4 * STHREADS) RWKV_DRAW(13);
-    else RWKV_DRAW(16);
-#undef RWKV_DRAW
+    if (pow) hipLaunchKernelGGL(sample_draw_kernel<true>, grid, dim3(STHREADS), 0, st, a, ws);
+    else hipLaunchKernelGGL(sample_draw_kernel<false>, grid, dim3(STHREADS), 0, st, a, ws);
     RWKV_LAUNCH_CHECK();
     return RWKV_OK;
 }

@@ -318,3 +318,40 @@ def test_draw_without_a_finite_total():
         x[5] = fill
         s = Sampler(V, device=DEV)
         assert 0 <= int(s.sample(x, 1.0, 0.7, 0, 0.2, 0.2, 0.996, u=0.5)) < V
+
+
+@pytest.mark.parametrize("V", [16388, 50277, 65536])
+@pytest.mark.parametrize("temp", [1.0, 0.7, 0.0])
+@pytest.mark.parametrize("kind", ["nan", "inf", "masked", "nan among masks"])
+def test_draw_without_a_total_as_one_workgroup_makes_it(V, temp, kind):
+    """Logits whose exponentials have no positive finite sum: token, probabilities and both tables as the one-workgroup kernel
+    leaves them, bit for bit, from buffers that held something else."""
+    from chatrwkv_amd import lib
+    from chatrwkv_amd.sampling import Sampler
+    L = lib.load()
+    rng = np.random.Generator(np.random.PCG64([V, 7]))
+    x = torch.from_numpy((rng.standard_normal(V) * 3).astype(np.float32)).to(DEV)
+    if kind == "nan":
+        x[V // 2] = float("nan")
+    elif kind == "inf":
+        x[V // 2] = float("inf")
+    elif kind == "masked":
+        x[:] = float("-inf")
+    else:                                   # the 1024 entries around the one that is no number are masked
+        x[8192:9216] = float("-inf")
+        x[8200] = float("nan")
+    s = Sampler(V, device=DEV, token_ban=[3])
+    seen = torch.from_numpy(rng.integers(0, V, 40)).to(DEV)
+    s.seen[seen] = 1
+    s.occurrence[seen] = 2.5
+    tables = s.seen.clone(), s.occurrence.clone()
+    s.token.fill_(-1)
+    s.probs.fill_(7.0)
+    probs, token = s.probs.clone(), s.token.clone()
+    u = torch.tensor([0.4], device=DEV)
+    s.sample(x, temp, 0.7, 0, 0.2, 0.3, 0.996, u=u)
+    lib.check(L.rwkv_sample_logits(x.data_ptr(), V, temp, 0.7, 0, s.ban.data_ptr(), 1, tables[0].data_ptr(), tables[1].data_ptr(),
+                                   None, 0.2, 0.3, 0.996, u.data_ptr(), probs.data_ptr(), token.data_ptr(),
+                                   torch.cuda.current_stream().cuda_stream), "rwkv_sample_logits")
+    assert int(s.token) == int(token) and torch.equal(s.seen, tables[0]) and torch.equal(s.occurrence, tables[1])
+    np.testing.assert_array_equal(s.probs.cpu().numpy(), probs.cpu().numpy())
