@@ -355,3 +355,53 @@ def test_draw_without_a_total_as_one_workgroup_makes_it(V, temp, kind):
                                    torch.cuda.current_stream().cuda_stream), "rwkv_sample_logits")
     assert int(s.token) == int(token) and torch.equal(s.seen, tables[0]) and torch.equal(s.occurrence, tables[1])
     np.testing.assert_array_equal(s.probs.cpu().numpy(), probs.cpu().numpy())
+
+
+def _wide(kind, V, rng):
+    """Logits of which thousands lie in half an octave: equal ones, two levels, a slope, all with a few outliers and masks"""
+    if kind == "equal":
+        x = np.zeros(V)
+    elif kind == "levels":
+        x = np.where(rng.random(V) < 0.4, 0.0, -0.25)
+    elif kind == "slope":
+        x = rng.permutation(V) * (0.3 / V)
+    else:
+        x = rng.standard_normal(V) * 3
+    x = x.astype(np.float32)
+    if kind != "equal":
+        x[rng.integers(0, V, 3)] += 2
+    x[rng.integers(0, V, 20)] = -np.inf
+    return torch.from_numpy(x).to(DEV)
+
+
+def _one_workgroup(L, x, temp, top_p, top_k, u, probs, token):
+    from chatrwkv_amd import lib
+    lib.check(L.rwkv_sample_logits(x.data_ptr(), x.numel(), temp, top_p, top_k, None, 0, None, None, None, 0.0, 0.0, 1.0, u.data_ptr(),
+                                   probs.data_ptr(), token.data_ptr(), torch.cuda.current_stream().cuda_stream), "rwkv_sample_logits")
+
+
+@pytest.mark.parametrize("V", [16388, 50277, 65536])
+@pytest.mark.parametrize("kind", ["equal", "levels", "slope", "normal"])
+def test_draw_from_logits_close_to_each_other(V, kind):
+    """Thousands of entries around the cut, ties among them: kept sets and probabilities as the one-workgroup kernel has them;
+    bounds as in test_draw_over_the_chip_against_one_workgroup (equal entries stand or fall together)."""
+    from chatrwkv_amd import lib
+    from chatrwkv_amd.sampling import Sampler
+    L = lib.load()
+    rng = np.random.Generator(np.random.PCG64([V, 11]))
+    x = _wide(kind, V, rng)
+    s = Sampler(V, device=DEV)
+    for top_p, top_k, temp in [(0.3, 0, 1.0), (0.7, 0, 1.0), (0.97, 0, 0.8), (0.999, 0, 1.0), (0.9, 50, 1.0), (0.9, 7000, 1.0), (0.8, 3, 1.2)]:
+        u = torch.tensor([float(rng.random())], device=DEV)
+        probs, token = torch.empty_like(s.probs), torch.full_like(s.token, -1)
+        s.sample(x, temp, top_p, top_k, u=u)
+        _one_workgroup(L, x, temp, top_p, top_k, u, probs, token)
+        got, ref = s.probs.cpu().numpy().astype(np.float64), probs.cpu().numpy().astype(np.float64)
+        least = min(v[v > 0].min() ** temp for v in (got, ref))
+        loose = 0 if top_k or kind in ("equal", "levels") else 1 + 4e-6 / least
+        assert abs(int((got > 0).sum()) - int((ref > 0).sum())) <= loose, (top_p, top_k, temp)
+        both = (got > 0) & (ref > 0)
+        np.testing.assert_allclose(got[both], ref[both], rtol=4e-6, atol=1e-30)
+        cdf = np.cumsum(ref)
+        if np.abs(cdf / cdf[-1] - float(u)).min() > 1e-5 and np.array_equal(got > 0, ref > 0):
+            assert int(s.token) == int(token), (top_p, top_k, temp)
