@@ -445,7 +445,7 @@ __global__ __launch_bounds__(STHREADS) void sample_kernel(SampleArgs a) {
 // exponential alone takes twenty.  With scratch from the caller the passes over the vocabulary run on one workgroup per
 // SEG entries, in three launches:
 //   adjust: bans and penalties, the segment's largest logit and sum of exponentials;
-//   probs:  the probabilities (every workgroup forms the total), for BOUNDS bounds half an octave apart below the largest
+//   probs:  the probabilities (every workgroup forms the total) and their powers, for BOUNDS bounds half an octave apart below the largest
 //           one the segment's sum and count of the entries that reach it, and the list, in index order, of the entries that
 //           the nucleus can need: those below (1 - top_p) / 2 V cannot add up to what may be left out;
 //   draw:   every workgroup finds the cut for itself -- the bounds leave half an octave, which goes to its 64th part that
@@ -453,7 +453,7 @@ __global__ __launch_bounds__(STHREADS) void sample_kernel(SampleArgs a) {
 //           probabilities and the occurrence counts of its segment.
 // Sums are added in a fixed order throughout.  Where the total is no positive number (a NaN, an infinity or nothing but masks
 // among the logits) nothing is kept and id 0 is drawn, which is what the kernel above makes of such logits.
-// Bound by the latency of the three launches.  Measured as above, V = 65536: 21.5 us a draw (2.7 + 4.3 + 12.7 and the gaps), 39 with one
+// Bound by the latency of the three launches.  Measured as above, V = 65536: 19.8 us a draw (2.9 + 4.3 + 10.8 and the gaps), 38 with one
 // workgroup; with the lists in LDS and the bracket searched by search_list 25.8, 5 us of it in the search.
 constexpr int SEG = 1024, SEGS_MAX = 64, BOUNDS = 32;
 constexpr int FEW = 256;                      // entries of a bracket that are compared with each other at once
@@ -462,6 +462,7 @@ constexpr int PART = 2 * BOUNDS + 2;          // per segment: sums and counts at
 struct SampleWs {
     float *p;          // [segments][SEG] adjusted logits, then probabilities
     float *list;       // [segments][SEG] candidates in index order
+    float *pow;        // [segments][SEG] the same to the power 1 / temperature, at temperatures other than 0 and 1
     uint16_t *idx;     // [segments][SEG] their places in the segment
     float *soft;       // [segments][2] largest logit, sum of exponentials
     float *part;       // [segments][PART]
@@ -521,6 +522,10 @@ DEV Soft soft_total(const float *soft, int segs) {
 DEV float list_floor(float top_p, int V) { return 0.5f * (1.f - top_p) / (float)V; }   // of the candidates
 DEV float bound_at(float pmax, int k) { return __uint_as_float(__float_as_uint(pmax) - ((unsigned)(k + 1) << 22)); }
 
+// POW: the candidates' powers are formed here, four entries a thread over the chip.  In sample_draw_kernel each of the up to 64
+// workgroups formed those of all candidates, 64 a thread, half of a draw from flat logits.  us a draw, 50277 entries, top_p 0.85,
+// temperature 0.8, one workgroup / powers there / here: N(0, 0.3) 81 / 95 / 45, N(0, 3) 68 / 38 / 24.
+template <bool POW>
 __global__ __launch_bounds__(256) void sample_probs_kernel(SampleArgs a, SampleWs ws) {
     __shared__ unsigned long long bin_s[BOUNDS];   // sums times 2^40: the same in any order
     __shared__ unsigned bin_n[BOUNDS];
@@ -564,6 +569,7 @@ __global__ __launch_bounds__(256) void sample_probs_kernel(SampleArgs a, SampleW
     for (int e = 0; e < 4; ++e)
         if ((in[e] >> lane) & 1) {
             ws.list[at] = p[e];
+            if (POW) ws.pow[at] = powf(p[e], 1.f / a.temperature);
             ws.idx[at++] = (uint16_t)(4 * threadIdx.x + e);
         }
     float *part = ws.part + blockIdx.x * PART;
@@ -707,7 +713,7 @@ __global__ __launch_bounds__(STHREADS) void sample_draw_kernel(SampleArgs a, Sam
         while (hi - lo > 1 && at_lo.n - at_hi.n > (float)FEW) {
             // Sums and counts of up to 64 equal parts of the interval.  Sums in whole units of 2^-40 of the power of two past fhi, so
             // they are the same in any order and lose less than 2^-23 of fhi.  us a draw, one workgroup / bisection down to 1024
-            // entries and a list of these / this: 65536 equal logits, top_p 0.7 67 / 68 / 29, 50277 of them 58 / 67 / 27; 50277
+            // entries and a list of these / this: 65536 equal logits, top_p 0.7 67 / 68 / 34, 50277 of them 58 / 67 / 33; 50277
             // from N(0, 3), top_p 0.999 40.6 / 49.3 / 41.1 (58.5 from 0 up instead of list_floor: three parts take all additions).
             const int shift = max(26 - __builtin_clz(hi - lo - 1), 0), octave = (int)((hi - 1) >> 23) - 127;
             const float unit = __uint_as_float((unsigned)(39 - octave + 127) << 23), inv_unit = __uint_as_float((unsigned)(octave - 39 + 127) << 23);
@@ -780,19 +786,21 @@ __global__ __launch_bounds__(STHREADS) void sample_draw_kernel(SampleArgs a, Sam
         cut = __uint_as_float(lo);
     }
     // ---- filter, temperature, sums of the segments
-    const float invt = 1.f / a.temperature;
-    auto kept = [&](float v) {
-        v = v >= cut && v > 0.f ? v : 0.f;
-        if (POW && v > 0.f) v = powf(v, invt);
-        return v;
-    };
+    auto keep = [&](float x) { return x >= cut && x > 0.f; };
     {
         float sum = 0.f;
-        each([&](float x) { sum += kept(x); });
+#pragma unroll
+        for (int j = 0; j < SEG / 64; ++j)
+            if (j < rounds) {
+                f32x4 q = v[j];
+                if (POW) q = *(const f32x4 *)(ws.pow + min(sg, segs - 1) * SEG + 64 * j + 4 * r);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) sum += keep(v[j][e]) ? q[e] : 0.f;
+            }
         sum = row16_sum(sum);
         if (r == 0) seg_sum[sg] = sum;
     }
-    if (a.probs && own < V) a.probs[own] = kept(p_own);
+    if (!POW && a.probs && own < V) a.probs[own] = keep(p_own) ? p_own : 0.f;
     __syncthreads();
     // ---- draw: first index whose running sum exceeds u * total; the last kept entry where rounding leaves none
     if (wave == 0) {
@@ -804,11 +812,12 @@ __global__ __launch_bounds__(STHREADS) void sample_draw_kernel(SampleArgs a, Sam
         int found = -1, last = 0;                 // places in the segment
         for (int i0 = 0; i0 < end && found < 0; i0 += 256) {   // four entries a lane
             const int i = i0 + 4 * lane;
-            f32x4 q = *(const f32x4 *)(ws.list + from * SEG + i);
+            f32x4 q = *(const f32x4 *)(ws.list + from * SEG + i), w = q;
+            if (POW) w = *(const f32x4 *)(ws.pow + from * SEG + i);
             const uint2 id = *(const uint2 *)(ws.idx + from * SEG + i);
             const int ids[4] = {(int)(id.x & 0xffff), (int)(id.x >> 16), (int)(id.y & 0xffff), (int)(id.y >> 16)};
 #pragma unroll
-            for (int e = 0; e < 4; ++e) q[e] = i + e < end ? kept(q[e]) : 0.f;
+            for (int e = 0; e < 4; ++e) q[e] = i + e < end && keep(q[e]) ? w[e] : 0.f;
             const float mine4 = (q[0] + q[1]) + (q[2] + q[3]), up = wave_scan(mine4);
             float at = run + (up - mine4);
             int f = -1, l = -1;
@@ -829,6 +838,7 @@ __global__ __launch_bounds__(STHREADS) void sample_draw_kernel(SampleArgs a, Sam
     }
     __syncthreads();
     store(pick);
+    if (POW && a.probs && own < V) a.probs[own] = keep(p_own) ? powf(p_own, 1.f / a.temperature) : 0.f;
 }
 
 }  // namespace
@@ -918,10 +928,11 @@ static size_t sample_ws(SampleWs &ws, void *base, int64_t V) {
     const size_t segs = (size_t)((V + SEG - 1) / SEG), n = segs * SEG;
     ws.p = (float *)base;
     ws.list = ws.p + n;
-    ws.part = ws.list + n;
+    ws.pow = ws.list + n;
+    ws.part = ws.pow + n;
     ws.soft = ws.part + segs * PART;
     ws.idx = (uint16_t *)(ws.soft + 2 * segs);
-    return (2 * n + segs * (PART + 2)) * sizeof(float) + n * sizeof(uint16_t);
+    return (3 * n + segs * (PART + 2)) * sizeof(float) + n * sizeof(uint16_t);
 }
 
 extern "C" size_t rwkv_sample_workspace(int64_t V) {
@@ -950,9 +961,13 @@ extern "C" int rwkv_sample_logits_ws(const float *logits, int64_t V, float tempe
     const dim3 grid((unsigned)((V + SEG - 1) / SEG));
     const bool pow = temperature != 0.f && temperature != 1.f;
     hipLaunchKernelGGL(sample_adjust_kernel, grid, dim3(256), 0, st, a, ws);
-    hipLaunchKernelGGL(sample_probs_kernel, grid, dim3(256), 0, st, a, ws);
-    if (pow) hipLaunchKernelGGL(sample_draw_kernel<true>, grid, dim3(STHREADS), 0, st, a, ws);
-    else hipLaunchKernelGGL(sample_draw_kernel<false>, grid, dim3(STHREADS), 0, st, a, ws);
+    if (pow) {
+        hipLaunchKernelGGL(sample_probs_kernel<true>, grid, dim3(256), 0, st, a, ws);
+        hipLaunchKernelGGL(sample_draw_kernel<true>, grid, dim3(STHREADS), 0, st, a, ws);
+    } else {
+        hipLaunchKernelGGL(sample_probs_kernel<false>, grid, dim3(256), 0, st, a, ws);
+        hipLaunchKernelGGL(sample_draw_kernel<false>, grid, dim3(STHREADS), 0, st, a, ws);
+    }
     RWKV_LAUNCH_CHECK();
     return RWKV_OK;
 }

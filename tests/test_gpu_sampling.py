@@ -405,3 +405,35 @@ def test_draw_from_logits_close_to_each_other(V, kind):
         cdf = np.cumsum(ref)
         if np.abs(cdf / cdf[-1] - float(u)).min() > 1e-5 and np.array_equal(got > 0, ref > 0):
             assert int(s.token) == int(token), (top_p, top_k, temp)
+
+
+@pytest.mark.parametrize("V", [16388, 50277, 65536])
+@pytest.mark.parametrize("kind,top_p,temp", [("equal", 0.7, 1.0), ("slope", 0.85, 0.8), ("normal", 0.999, 1.0), ("normal", 0.999, 0.8)])
+def test_draws_over_the_chip_are_not_slower(V, kind, top_p, temp):
+    """Draws that keep or search thousands of entries: the three launches take no longer than the one-workgroup kernel on the
+    same operands, by the best of several runs (a tenth is left for the clock)."""
+    from chatrwkv_amd import lib
+    from chatrwkv_amd.sampling import Sampler
+    L = lib.load()
+    x = _wide(kind, V, np.random.Generator(np.random.PCG64([V, 11])))
+    s = Sampler(V, device=DEV)
+    u = torch.tensor([0.4], device=DEV)
+    token, probs = torch.zeros_like(s.token), torch.empty_like(s.probs)
+
+    def best(draw):
+        ms = []
+        for _ in range(8):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            for _ in range(50):
+                draw()
+            b.record()
+            torch.cuda.synchronize()
+            ms.append(a.elapsed_time(b))
+        return min(ms)
+
+    stream = torch.cuda.current_stream().cuda_stream
+    chip = best(lambda: lib.check(L.rwkv_sample_logits_ws(x.data_ptr(), V, temp, top_p, 0, None, 0, None, None, None, 0.0, 0.0, 1.0, u.data_ptr(),
+                                                          probs.data_ptr(), token.data_ptr(), s.ws.data_ptr(), s.ws.numel(), stream), "ws"))
+    one = best(lambda: _one_workgroup(L, x, temp, top_p, 0, u, probs, token))
+    assert chip <= 1.1 * one, (chip, one)
