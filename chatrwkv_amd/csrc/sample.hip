@@ -522,12 +522,17 @@ DEV Soft soft_total(const float *soft, int segs) {
 DEV float list_floor(float top_p, int V) { return 0.5f * (1.f - top_p) / (float)V; }   // of the candidates
 DEV float bound_at(float pmax, int k) { return __uint_as_float(__float_as_uint(pmax) - ((unsigned)(k + 1) << 22)); }
 
+// Probabilities in units of 2^-62.  Those from 2^-39 on are whole numbers of them (a bound is at least 2^-32, a candidate 2^-27),
+// and all together are about 1: their sums are exact, so the same in any order, and rounded once.
+DEV unsigned long long fixed(float p) { return (unsigned long long)(p * 0x1p62f); }
+DEV float from_fixed(unsigned long long s) { return (float)s * 0x1p-62f; }
+
 // POW: the candidates' powers are formed here, four entries a thread over the chip.  In sample_draw_kernel each of the up to 64
 // workgroups formed those of all candidates, 64 a thread, half of a draw from flat logits.  us a draw, 50277 entries, top_p 0.85,
 // temperature 0.8, one workgroup / powers there / here: N(0, 0.3) 81 / 95 / 45, N(0, 3) 68 / 38 / 24.
 template <bool POW>
 __global__ __launch_bounds__(256) void sample_probs_kernel(SampleArgs a, SampleWs ws) {
-    __shared__ unsigned long long bin_s[BOUNDS];   // sums times 2^40: the same in any order
+    __shared__ unsigned long long bin_s[BOUNDS];   // sums in fixed point
     __shared__ unsigned bin_n[BOUNDS];
     __shared__ float red[4][2];
     if (threadIdx.x < BOUNDS) { bin_s[threadIdx.x] = 0; bin_n[threadIdx.x] = 0; }
@@ -546,7 +551,7 @@ __global__ __launch_bounds__(256) void sample_probs_kernel(SampleArgs a, SampleW
         const unsigned k = (__float_as_uint(inv) - __float_as_uint(p[e])) >> 22;   // the first bound that the entry reaches is k or k - 1
         const unsigned bin = k < BOUNDS + 1 ? (k > 0 && p[e] >= bound_at(inv, k - 1) ? k - 1 : k) : BOUNDS;
         if (bin < BOUNDS) {
-            atomicAdd(&bin_s[bin], (unsigned long long)(p[e] * 1099511627776.f));
+            atomicAdd(&bin_s[bin], fixed(p[e]));
             atomicAdd(&bin_n[bin], 1u);
         }
     }
@@ -582,7 +587,7 @@ __global__ __launch_bounds__(256) void sample_probs_kernel(SampleArgs a, SampleW
             sum += k <= lane ? bin_s[k] : 0;
             n += k <= lane ? bin_n[k] : 0;
         }
-        part[lane] = (float)sum * 0x1p-40f;
+        part[lane] = from_fixed(sum);
         part[BOUNDS + lane] = (float)n;
     }
 }
@@ -711,12 +716,10 @@ __global__ __launch_bounds__(STHREADS) void sample_draw_kernel(SampleArgs a, Sam
             at_hi = {__shfl(at_k.s, k - 1, WAVE), __shfl(at_k.n, k - 1, WAVE)};
         }
         while (hi - lo > 1 && at_lo.n - at_hi.n > (float)FEW) {
-            // Sums and counts of up to 64 equal parts of the interval.  Sums in whole units of 2^-40 of the power of two past fhi, so
-            // they are the same in any order and lose less than 2^-23 of fhi.  us a draw, one workgroup / bisection down to 1024
-            // entries and a list of these / this: 65536 equal logits, top_p 0.7 67 / 68 / 34, 50277 of them 58 / 67 / 33; 50277
-            // from N(0, 3), top_p 0.999 40.6 / 49.3 / 41.1 (58.5 from 0 up instead of list_floor: three parts take all additions).
-            const int shift = max(26 - __builtin_clz(hi - lo - 1), 0), octave = (int)((hi - 1) >> 23) - 127;
-            const float unit = __uint_as_float((unsigned)(39 - octave + 127) << 23), inv_unit = __uint_as_float((unsigned)(octave - 39 + 127) << 23);
+            // Sums and counts of up to 64 equal parts of the interval.  us a draw, one workgroup / bisection down to 1024 entries and a
+            // list of these / this: 65536 equal logits, top_p 0.7 67 / 68 / 34, 50277 of them 58 / 67 / 33; 50277 from N(0, 3),
+            // top_p 0.999 40.6 / 49.3 / 41.1 (58.5 from 0 up instead of list_floor: three parts take all additions).
+            const int shift = max(26 - __builtin_clz(hi - lo - 1), 0);
             const float flo = __uint_as_float(max(lo, 1u)), fhi = __uint_as_float(hi);
             if (tid < 64) { part_s[tid] = 0; part_n[tid] = 0; }
             __syncthreads();
@@ -730,13 +733,13 @@ __global__ __launch_bounds__(STHREADS) void sample_draw_kernel(SampleArgs a, Sam
                 if (ties ? lane == 0 : in) {
                     const float y = ties ? __uint_as_float(first) : x;
                     const unsigned part = (__float_as_uint(y) - lo) >> shift;
-                    atomicAdd(&part_s[part], (unsigned long long)n * (unsigned long long)(y * unit));
+                    atomicAdd(&part_s[part], (unsigned long long)n * fixed(y));
                     atomicAdd(&part_n[part], (unsigned)n);
                 }
             });
             __syncthreads();
             // lane i: the part i from above, and the sum and the count from its lower end on
-            const SumCount t = {at_hi.s + wave_scan((float)part_s[63 - lane] * inv_unit), at_hi.n + wave_scan((float)part_n[63 - lane])};
+            const SumCount t = {at_hi.s + wave_scan(from_fixed(part_s[63 - lane])), at_hi.n + wave_scan((float)part_n[63 - lane])};
             const unsigned long long good = __ballot(enough(t, top_p, want));
             const int i = good ? __builtin_ctzll(good) : 63;
             if (good) at_lo = {__shfl(t.s, i, WAVE), __shfl(t.n, i, WAVE)};
