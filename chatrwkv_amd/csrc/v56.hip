@@ -162,6 +162,8 @@ __global__ __launch_bounds__(256) void v6_mix2_kernel(Mix2Args a) {
 // once, is 0.5 % of a call faster at 1000 tokens and 3 % slower up to 45.
 // The form before multiplied on the vector units, 4 or 16 tokens x 4 channels per thread, and was bound by their issue.  us, 4096
 // channels, rank 32, uint8 (scaled, with sums), 256 tokens: 15.9 -> 11.1; 6 % of a call of 513 tokens.
+// C callers may put w2 and the maa vectors on any boundary: their loads are of a type that is aligned to its elements.
+typedef h16x8 h16x8_a2 __attribute__((aligned(2)));
 template <int KS>
 __global__ __launch_bounds__(256) void v6_mix2_mfma_kernel(Mix2Args a) {
     constexpr int ROW = 32 * KS + 4;                                     // halves of a channel's row
@@ -182,7 +184,7 @@ __global__ __launch_bounds__(256) void v6_mix2_mfma_kernel(Mix2Args a) {
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             const int k = 2 * (kp + 8 * i) + h;                          // rows past R: loaded from row 0, zeroed below
-            wr[i][h] = *(const h16x8 *)(a.w2 + ((size_t)j * R + (k < R ? k : 0)) * C + cg);
+            wr[i][h] = *(const h16x8_a2 *)(a.w2 + ((size_t)j * R + (k < R ? k : 0)) * C + cg);
         }
 #pragma unroll
     for (int s = 0; s < KS; ++s) {
@@ -193,7 +195,7 @@ __global__ __launch_bounds__(256) void v6_mix2_mfma_kernel(Mix2Args a) {
     for (int p = 0; p < 2; ++p) {
         xx[p] = *(const h16x8 *)(a.xx + o + 8 * p);
         sd[p] = *(const h16x8 *)(a.sxd + o + 8 * p);
-        mv[p] = *(const h16x8 *)(a.maa[j] + c + 8 * p);
+        mv[p] = *(const h16x8_a2 *)(a.maa[j] + c + 8 * p);
         if (scaled) { rv[p] = *(const h16x8 *)(a.ry[j] + c + 8 * p); yv[p] = *(const h16x8 *)(a.my[j] + c + 8 * p); }
     }
 #pragma unroll
@@ -243,12 +245,6 @@ __global__ __launch_bounds__(256) void v6_mix2_mfma_kernel(Mix2Args a) {
         if (blockIdx.y == 0)
             for (int i = gridDim.y; i < a.npart; ++i) p[i] = 0.f;
     }
-}
-// what its 16-byte loads assume beyond the layer's own checks: C ABI callers may put these on any boundary
-bool mix2_mfma_ok(const rwkv_v56_layer &l) {
-    for (int j = 1; j < 6; ++j)
-        if (!aligned16(l.att_mix[j])) return false;
-    return aligned16(l.tm_w2);
 }
 // Calls of up to 16 tokens keep the sums in index order, so that a conversation's first tokens come out as they did: a deep
 // model whose state is nearly empty makes percents of its logits from the last bit of a mix.  The matrix cores gain 2 % of a
@@ -410,7 +406,7 @@ extern "C" int rwkv_v56_forward(const rwkv_v56_model *m, const rwkv_v56_layer_st
             for (int j = 0; j < 5; ++j) { b.maa[j] = l.att_mix[1 + j]; b.out[j] = ws.mix[j]; }
             // uint8 matrices, the four products as one grouped direct-to-LDS launch: the mixing kernel writes their
             // inputs already scaled, with partial row sums that the grouped launch adds up -- no scaling pass
-            const bool mfma = T > 16 && mix2_mfma_ok(l);
+            const bool mfma = T > 16;
             if (mfma && u8 && grouped && handover_enabled()) {
                 const rwkv_half *xin[4] = {ws.mix[3], ws.mix[1], ws.mix[2], ws.mix[4]};
                 const rwkv_mat *mats[4] = {&l.att_receptance, &l.att_key, &l.att_value, &l.att_gate};
