@@ -252,6 +252,23 @@ def test_forced_tile_configurations(N, M, B, monkeypatch):
             call()
 
 
+@pytest.mark.parametrize("cfg", ["", "14", "15", "20", "21"])
+@pytest.mark.parametrize("N,M,B", [(1088, 1000, 2176), (8192, 200, 520), (8192, 516, 600)])
+def test_tiles_that_walk_along_the_outputs(N, M, B, cfg, monkeypatch):
+    """More activations than weights and more than an XCD's L2 holds: consecutive tiles go along the outputs.  Several columns
+    of tiles, the last one ragged, at full depth (the first) and in K splits (the others), every tile size, both weight types;
+    the sums are exact, so the results are equal bit for bit."""
+    ops = _ops()
+    x, (q, mx, rx, my, ry), want, _ = _affine_case(N, M, B, N + M + B)
+    xt = torch.from_numpy(x).to(DEV)
+    monkeypatch.setenv("RWKV_GEMM_CFG", cfg)
+    y = ops.cuda_mm8_seq(B, N, M, xt, _to_dev_ic(q), *(torch.from_numpy(a).to(DEV) for a in (mx, rx, my, ry)))
+    assert np.array_equal(y.cpu().numpy(), want)
+    w = (_rng(N).integers(-64, 65, (N, M)) / 64).astype(np.float16)
+    y = ops.matmul_float(xt, _to_dev_ic(w), output_dtype=torch.float32)
+    assert np.array_equal(y.cpu().numpy(), x.astype(np.float64) @ w.astype(np.float64))
+
+
 @pytest.mark.parametrize("cfg", ["14", "15", "20", "21"])
 def test_forced_direct_to_lds_tiles_refuse_other_layouts(cfg, monkeypatch):
     """RWKV_GEMM_CFG (tuning): operands that the direct-to-LDS kernels do not take -- here mx on no 16-byte boundary -- are
