@@ -314,10 +314,10 @@ __global__ __launch_bounds__(256) void wkv7_kernel(Wkv7Args a) {
 // not finite are kept from the tokens before them where the first kernel forms its products.
 // 20 KB of fp32 operands pass from one to the other per head and chunk.  The first kernel moves them at 3.0 TB/s of a
 // copy's 4.8: about 1000 vector instructions a wave, a third of them the five exact divisions per element, six barriers and
-// the forward substitution of one wave beside three that wait.  Seven workgroups a CU against the five of 30 KB of LDS, and no
-// chunks past the last: 777 tokens 39.3 -> 37 us.  The second is a chain of one exchange per chunk (35 us, 0.72 a chunk).  A
+// the forward substitution of one wave beside three that wait.  Six workgroups a CU, by its 78 registers, against five by 30 KB
+// of LDS, and no chunks past the last: 777 tokens 39.3 -> 37 us.  The second is a chain of one exchange per chunk (35 us, 0.72 a chunk).  A
 // 4096-wide layer, both together: 260 tokens 321 -> 314.5 us, 777 561.5 -> 557, 1024 the same.  Per layer at 64 heads,
-// preparation and recurrence, token by token -> chunks: 1024 tokens 152 -> 89 us, 777 tokens 116 -> 75, 256 tokens 42 -> 31,
+// preparation and recurrence, token by token -> chunks: 1024 tokens 152 -> 89 us, 777 tokens 116 -> 72, 256 tokens 42 -> 31,
 // 100 tokens 21 -> 19; at 64 tokens the two launches take as long as prep7_kernel and wkv7_kernel: CHUNKED7.
 constexpr int SEG7 = 1024;        // tokens per pair of launches: bounds the scratch between them
 constexpr int CHUNKED7 = 96;      // calls of at least so many tokens run in chunks
@@ -329,7 +329,7 @@ constexpr int LM7 = 20;           // LDS row of 16 floats, padded
 
 __global__ __launch_bounds__(256) void wkv7_chunk_kernel(Prep7Args a, int t_begin, float *__restrict__ scratch) {
     __shared__ __align__(16) float la[CL][LR7], lr[CL][LR7], lk[CL][LR7], lb[CL][LR7];   // a . A, r . A, k / A, b / A
-    // 22 KB in all, so that seven workgroups share a CU: A_16 in the pads of la, piece g in row g; the decays where the
+    // 22 KB in all, room for seven workgroups a CU (the registers leave six): A_16 in the pads of la, piece g in row g; the decays where the
     // matrices come, Z over the rows of AB that it has used, the values at last over Z and QB
     __shared__ __align__(16) float mat[4][CL][LM7];
     constexpr int AK = 0, QK = 1, AB = 2, QB = 3;
