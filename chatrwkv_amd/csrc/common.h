@@ -78,12 +78,6 @@ DEV float wave_max(float v) {
     const float r3 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(b, 48));
     return fmaxf(fmaxf(r0, r1), fmaxf(r2, r3));
 }
-DEV float wave_min(float v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = fminf(v, __shfl_xor(v, o, WAVE));
-    return v;
-}
-
 // Sum over the whole workgroup; every thread gets the result.  `red` is LDS scratch of at
 // least (blockDim.x / 64) floats; safe to call repeatedly with the same scratch.
 DEV float block_sum(float v, float *red) {
@@ -95,26 +89,6 @@ DEV float block_sum(float v, float *red) {
     float t = 0.f;
     for (int i = 0; i < nw; ++i) t += red[i];
     return t;
-}
-
-// Sum K values over the workgroup at once (one pair of barriers); every thread gets all K totals, each formed
-// exactly as block_sum forms it.  `red` is LDS scratch of at least K * (blockDim.x / 64) floats.
-template <int K>
-DEV void block_sum_n(float (&v)[K], float *red) {
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, nw = (blockDim.x + 63) >> 6;
-#pragma unroll
-    for (int k = 0; k < K; ++k) v[k] = wave_sum(v[k]);
-    __syncthreads();
-    if (lane == 0)
-#pragma unroll
-        for (int k = 0; k < K; ++k) red[k * nw + wid] = v[k];
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < K; ++k) {
-        float t = 0.f;
-        for (int i = 0; i < nw; ++i) t += red[k * nw + i];
-        v[k] = t;
-    }
 }
 
 // ---- uint8 -> fp16 pairs -------------------------------------------------------------------

@@ -29,74 +29,6 @@ __global__ __launch_bounds__(256) void copy16_kernel(int n16, const u32x4 *__res
     if (i < n16) dst[i] = src[i];
 }
 
-DEV void row_stats(const rwkv_half *x, int C, float *red, float &mean, float &rstd) {
-    float s = 0.f;
-    for (int j8 = threadIdx.x; j8 < (C >> 3); j8 += blockDim.x) s = sum8(*(const h16x8 *)(x + 8 * j8), s);
-    mean = row_mean(block_sum(s, red), C);
-    float q = 0.f, d[8];
-    for (int j8 = threadIdx.x; j8 < (C >> 3); j8 += blockDim.x) {
-        less_mean8(*(const h16x8 *)(x + 8 * j8), mean, d);
-        q = j8 < (int)blockDim.x ? squares8<true>(d, q) : squares8<false>(d, q);
-    }
-    rstd = row_rstd(block_sum(q, red), C);
-}
-DEV h16x8 row_norm8(const rwkv_half *x, float mean, float rstd, h16x8 w, h16x8 b) {
-    float d[8];
-    less_mean8(*(const h16x8 *)x, mean, d);
-    return norm8(d, rstd, w, b);
-}
-
-// One workgroup per token row.  Row t needs LN(x[t-1]) for the token shift: it is recomputed here
-// from x[t-1] (same code, same data => same bits as row t-1 computes for itself), which keeps all
-// rows independent.
-template <int NJ>
-__global__ __launch_bounds__(256) void lnmix_seq_kernel(SeqMixArgs a) {
-    __shared__ float red[32];
-    const int t = blockIdx.x, C = a.C;
-    const rwkv_half *x = a.x + (size_t)t * C;
-    float mean, rstd, pmean = 0.f, prstd = 0.f;
-    row_stats(x, C, red, mean, rstd);
-    const bool shift = a.sx != nullptr;
-    const rwkv_half *xp = x - C;
-    if (shift && t > 0) row_stats(xp, C, red, pmean, prstd);
-    float acc[2 * NJ];
-#pragma unroll
-    for (int i = 0; i < 2 * NJ; ++i) acc[i] = 0.f;
-    for (int j8 = threadIdx.x; j8 < (C >> 3); j8 += blockDim.x) {
-        const h16x8 wv = *(const h16x8 *)(a.ln_w + 8 * j8), bv = *(const h16x8 *)(a.ln_b + 8 * j8);
-        const h16x8 xx = row_norm8(x + 8 * j8, mean, rstd, wv, bv);
-        h16x8 pv = xx;
-        if (shift) pv = t > 0 ? row_norm8(xp + 8 * j8, pmean, prstd, wv, bv) : *(const h16x8 *)(a.sx + 8 * j8);
-        if (a.xx_last && t == a.T - 1) *(h16x8 *)(a.xx_last + 8 * j8) = xx;
-#pragma unroll
-        for (int j = 0; j < NJ; ++j) {
-            const h16x8 kx = a.mix[j] ? mix8(xx, pv, *(const h16x8 *)(a.mix[j] + 8 * j8), a.maa_form) : xx;
-            h16x8 o = kx;
-            if (a.ry[j]) {
-                o = kx * *(const h16x8 *)(a.ry[j] + 8 * j8);
-                acc[2 * j] = sum8(kx, acc[2 * j]);
-                acc[2 * j + 1] = dot8(kx, *(const h16x8 *)(a.my[j] + 8 * j8), acc[2 * j + 1]);
-            }
-            *(h16x8 *)(a.xs[j] + (size_t)t * C + 8 * j8) = o;
-        }
-    }
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) {
-        if (!a.ry[j]) continue;
-        const float v0 = block_sum(acc[2 * j], red), v2 = block_sum(acc[2 * j + 1], red);
-        if (threadIdx.x == 0) { a.s0[j][t] = v0; a.s2[j][t] = v2; }
-    }
-    // The new token-shift state is LN(x[T-1]).  Only row 0 reads the old one, so row 0's workgroup writes the new
-    // one once its own reads are done (each thread overwrites exactly the chunks it has read): no second launch.
-    if (a.state_out && t == 0) {
-        const rwkv_half *xl = a.x + (size_t)(a.T - 1) * C;
-        if (a.T > 1) row_stats(xl, C, red, mean, rstd);
-        for (int j8 = threadIdx.x; j8 < (C >> 3); j8 += blockDim.x)
-            *(h16x8 *)(a.state_out + 8 * j8) =
-                row_norm8(xl + 8 * j8, mean, rstd, *(const h16x8 *)(a.ln_w + 8 * j8), *(const h16x8 *)(a.ln_b + 8 * j8));
-    }
-}
-
 __global__ __launch_bounds__(256) void ln_f32_f16_kernel(int C, const float *__restrict__ x_, const float *__restrict__ w,
                                                          const float *__restrict__ b, rwkv_half *__restrict__ y_) {
     __shared__ float red[4];
@@ -111,12 +43,12 @@ __global__ __launch_bounds__(256) void ln_f32_f16_kernel(int C, const float *__r
     for (int j = threadIdx.x; j < C; j += blockDim.x) y[j] = f2h((x[j] - mean) * rstd * w[j] + b[j]);
 }
 
-// lnmix_seq_kernel with a short dependent chain, for C <= 8 NT CH: a thread's chunks of the row, of the previous row
-// and of the LayerNorm vectors are requested together at the top and kept in registers, the statistics of the two
-// rows share their barriers, and so do the 2 NJ sums at the end: two global round trips and three rounds of
-// barriers per workgroup instead of five and ten (and no longer chain in row 0's workgroup, which forms the new
-// token-shift state).  Every value is formed with the same operations in the same order as in lnmix_seq_kernel, with
-// 256 threads per row and with 512 (row_sums), so all agree bit for bit.
+// LayerNorm, token shift and mixes of a row of C <= 8 NT CH channels, one workgroup per row.  Row t needs LN(x[t-1]) for the token
+// shift: it is recomputed here from x[t-1] (same code, same data => same bits as row t-1 computes for itself), which keeps all
+// rows independent.  A thread's chunks of the row, of the previous row and of the LayerNorm vectors are requested together at the
+// top and kept in registers, the statistics of the two rows share their barriers, and so do the 2 NJ sums at the end: two global
+// round trips and three rounds of barriers.  256 threads per row and 512 form every value with the same operations in the same
+// order (row_sums), so both agree bit for bit.
 // PRE: the mix / scale vectors too are requested at the top (3 NJ CH more registers per thread: shorter chain, fewer
 // workgroups per CU -- for short calls, where a CU has one or two rows anyway).
 template <int NJ, int CH, bool PRE, int NT>
@@ -268,7 +200,7 @@ static bool lnmix_seq_fast_launch(const SeqMixArgs &a, int nj, hipStream_t st) {
 }
 
 int lnmix_seq_launch(const SeqMixArgs &a, int nj, hipStream_t st) {
-    // Rows of up to 8192 channels: the register-resident kernel (1, 2 or 4 chunks of 8 channels per chain of additions).
+    // A chain of additions has 1, 2 or 4 chunks of 8 channels (every model has at most 8192).
     // Calls of up to 512 rows have one or two rows per CU: there a row's own chain of barriers and instructions is the time,
     // so rows of more than 2048 channels get 512 threads instead of 256, with the same sums (row_sums).  4096 channels, us,
     // 256 -> 512 threads at 45 / 256 / 512 / 600 / 1024 rows: one mix 4.2 -> 3.4, 4.4 -> 3.6, 4.7 -> 4.8, 5.4 -> 5.7, 6.6 -> 7.1;
@@ -281,23 +213,13 @@ int lnmix_seq_launch(const SeqMixArgs &a, int nj, hipStream_t st) {
     // per row through a CU's L1 and the 24 MB of stores.
     // Several rows per workgroup, sharing vectors and the previous row's statistics, measured with the element code before: slower
     // at every length (1024 rows 21.8 with two, 33 with four, 20.7 with one).
-    if (a.C <= 8192 && (nj == 1 || nj == 2 || nj == 3 || nj == 4 || nj == 6)) {
-        const bool few = a.T <= 512;
-        if (a.C <= 2048) few ? lnmix_seq_fast_launch<1, true, 256>(a, nj, st) : lnmix_seq_fast_launch<1, false, 256>(a, nj, st);
-        else if (a.C <= 4096) few ? lnmix_seq_fast_launch<1, true, 512>(a, nj, st) : lnmix_seq_fast_launch<2, false, 256>(a, nj, st);
-        else few ? lnmix_seq_fast_launch<2, false, 512>(a, nj, st) : lnmix_seq_fast_launch<4, false, 256>(a, nj, st);
-        RWKV_LAUNCH_CHECK();
-        return RWKV_OK;
-    }
-    const dim3 grid((unsigned)a.T), block(256);
-    switch (nj) {
-        case 1: hipLaunchKernelGGL(lnmix_seq_kernel<1>, grid, block, 0, st, a); break;
-        case 2: hipLaunchKernelGGL(lnmix_seq_kernel<2>, grid, block, 0, st, a); break;
-        case 3: hipLaunchKernelGGL(lnmix_seq_kernel<3>, grid, block, 0, st, a); break;
-        case 4: hipLaunchKernelGGL(lnmix_seq_kernel<4>, grid, block, 0, st, a); break;
-        case 6: hipLaunchKernelGGL(lnmix_seq_kernel<6>, grid, block, 0, st, a); break;
-        default: return RWKV_E_DTYPE;
-    }
+    if (a.C > 8192) return RWKV_E_SHAPE;
+    const bool few = a.T <= 512;
+    bool known;
+    if (a.C <= 2048) known = few ? lnmix_seq_fast_launch<1, true, 256>(a, nj, st) : lnmix_seq_fast_launch<1, false, 256>(a, nj, st);
+    else if (a.C <= 4096) known = few ? lnmix_seq_fast_launch<1, true, 512>(a, nj, st) : lnmix_seq_fast_launch<2, false, 256>(a, nj, st);
+    else known = few ? lnmix_seq_fast_launch<2, false, 512>(a, nj, st) : lnmix_seq_fast_launch<4, false, 256>(a, nj, st);
+    if (!known) return RWKV_E_SHAPE;
     RWKV_LAUNCH_CHECK();
     return RWKV_OK;
 }
@@ -525,13 +447,7 @@ extern "C" int rwkv_v4_forward_seq(const rwkv_v4_model *m, const rwkv_v4_layer_s
         e.out_scale = 1.f;
         // k, v: uint8 weights return fp16 (widened by the consumer); fp16 weights return fp32 directly
         e.act = ACT_NONE; e.out_dtype = u8 ? RWKV_DT_F16 : RWKV_DT_F32; e.raw_f32 = u8 ? 0 : 1;
-        // side by side when none of them would split K (the split-K scratch is shared)
-        // long calls: every product through the direct-to-LDS kernel, one after the other (its tiles take a whole
-        // CU, so products side by side on several streams gain nothing); k, v, r as one group
-        const bool dma_seq = T >= 512;
-        const bool group_kvr = true;       // k, v, r as one grouped launch at every length (tile size and K split by cost)
-        ForkScope par(ss, st, 2, !group_kvr && (T / 128) * (C / 128) > 128);
-        if (group_kvr) {
+        {   // k, v, r as one grouped launch at every length (tile size and K split by cost)
             const rwkv_half *xin[3] = {ws.xs[0], ws.xs[1], ws.xs[2]};
             const rwkv_mat *mats[3] = {&l.att_key, &l.att_value, &l.att_receptance};
             void *outs[3] = {ws.k, ws.v, ws.r};
@@ -539,14 +455,6 @@ extern "C" int rwkv_v4_forward_seq(const rwkv_v4_model *m, const rwkv_v4_layer_s
             e.act = ACT_SIGMOID; e.out_dtype = RWKV_DT_F16; e.raw_f32 = 0;   // receptance, and every product after it
             ep[2] = e;
             if ((rc = gemm_group_launch(u8, 3, T, C, xin, mats, outs, ep, nullptr, s0, ws.splitk, st))) return rc;
-        } else {
-        hipStream_t sv = par ? ss->s[0] : st, sr = par ? ss->s[1] : st;
-        float *sk = par ? nullptr : ws.splitk;   // products that run side by side do not split K
-        if ((rc = run_gemm(l.att_key, u8, T, ws.xs[0], s0[0], s2[0], ws.k, C, e, st, sk))) return rc;
-        if ((rc = run_gemm(l.att_value, u8, T, ws.xs[1], s0[1], s2[1], ws.v, C, e, sv, sk))) return rc;
-        e.act = ACT_SIGMOID; e.out_dtype = RWKV_DT_F16; e.raw_f32 = 0;
-        if ((rc = run_gemm(l.att_receptance, u8, T, ws.xs[2], s0[2], s2[2], ws.r, C, e, sr, sk))) return rc;
-        if (!par.join()) return (int)hipErrorUnknown;
         }
         if ((rc = wkv4_fused_launch((int)T, C, l.time_decay, l.time_first, ws.k, ws.v, u8 ? 0 : 1, ws.r, ws.rwkv, s.aa,
                                     s.bb, s.pp, st, ws.wkv)))
@@ -607,9 +515,9 @@ extern "C" int rwkv_v4_forward_seq(const rwkv_v4_model *m, const rwkv_v4_layer_s
             if (!vparts) ork[1] = ws.vx;
             if ((rc = gemm_group_launch(u8, 2, T, C, xrk, mrk, ork, erk, nullptr, s0, ws.splitk, st))) return rc;
         } else {
-        // the receptance product beside the key product: where neither would split K, and in calls of three row tiles
-        // (257 .. 384 tokens: +4 % at n_embd 4096; slower at 256 and from 385 on)
-        ForkScope par2(ss, st, 1, !dma_seq && ((T / 128) * (C / 128) > 128 || ((T + 127) / 128 == 3 && C == 4096)));
+        // The receptance product beside the key product where neither would split K.  From 512 tokens on one after the other: the
+        // direct-to-LDS tiles take a whole CU, so products side by side gain nothing.
+        ForkScope par2(ss, st, 1, T < 512 && (T / 128) * (C / 128) > 128);
         float *sk2 = par2 ? nullptr : ws.splitk;
         // uint8: the three-stage tile for both, so that one of each fits a CU (2 x 73 KB; the four-stage tile that the
         // receptance product gets by itself takes 97: 4.89 ms against 4.82 for 16 layers of n_embd 4096 at 257 tokens, 5.15
