@@ -207,10 +207,11 @@ int lnmix_seq_launch(const SeqMixArgs &a, int nj, hipStream_t st) {
     // three mixes with scaling 6.7 -> 5.4, 7.4 -> 6.1, 8.4 -> 7.9, 9.4 -> 10.4, 11.7 -> 12.6; six mixes without 6.7 -> 5.5, 8.0 ->
     // 6.8, 9.1 -> 8.5, 10.0 -> 11.7, 12.8 -> 14.5 (5120 channels, three mixes: 512 rows 10.6 -> 10.2, 600 rows 11.8 -> 14.6).
     // Up to 4096 channels the mix and scale vectors of these calls are requested at the top too, except for six mixes.
-    // us before the element code above was written out (three to four instructions per step, sums over loops of unknown length):
-    // three scaled mixes of 4096 channels at 45 / 1024 rows 6.6 / 16.4, now 5.4 / 11.7; six at 777 rows 14.9, now 11.0; four of 2048
-    // channels at 333 rows 7.1, now 5.1; three of 768 at 513 rows 7.4, now 4.5.  An empty launch is 3.2; at 1024 rows it is the 130 KB
-    // per row through a CU's L1 and the 24 MB of stores.
+    // These are launches one after the other on the same rows.  Within a call, whose products have used the caches since, us
+    // before the element code of rows.h was written out (three to four instructions per step) and now: three scaled mixes of 4096
+    // channels at 45 / 1024 rows 7.3 / 20.5 -> 5.9 / 16.1, two 6.3 / 16.5 -> 5.6 / 12.7; at 777 rows six 20.3 -> 16.7, one 9.5 ->
+    // 7.0; four of 2048 channels at 333 rows 7.1 -> 5.3; three of 768 at 513 rows 6.7 -> 4.9.  An empty launch is 3.2; at 1024 rows
+    // it is the 130 KB per row through a CU's L1 and the 24 MB of stores.
     // Several rows per workgroup, sharing vectors and the previous row's statistics, measured with the element code before: slower
     // at every length (1024 rows 21.8 with two, 33 with four, 20.7 with one).
     if (a.C > 8192) return RWKV_E_SHAPE;
