@@ -1883,7 +1883,10 @@ constexpr TileDim tile_dim[TILES] = {{256, 256}, {128, 128}, {128, 128}, {64, 12
 // 128 x 128 ones, 120 us against 116 with fp16 weights; with uint8 weights and 1024 rows it belongs there (118.5 against 120.5).
 // gemm_kg_kernel: per launch, per round (split launches leave the epilogue to the second pass) and per k-tile by the CUs busy,
 // fitted to 1640 products (21 lengths, 8 widths) with the other tiles' prices as they stand: the tile it picks is 1.5 % slower
-// than the best of all on average, 4.2 % with the four tiles and prices before; 3.3 % less time.
+// than the best of all on average, 4.2 % with the four tiles and prices before; 3.3 % less time.  fp16, 64 x 128 tile: the line
+// of that fit is far too low below 150 CUs, where such launches would have few and long tiles and split K: a CU then takes 24 KB a
+// k-tile in 0.32 to 0.37 us whatever the others do.  Callers without scratch for a split got it all the same: [48 x 16384] x
+// [16384 x 1000] 94 us, 61 with the 64 x 64 tile, [64 x 4096] x [4096 x 512] 29.7 and 21.4.
 // slow_epi: see slow_epilogue.
 struct CostOf { bool w_u8, slow_epi; };
 bool slow_epilogue(const GemmEpi &ep) { return ep.act == ACT_RESIDUAL || ep.act == ACT_GATED_RESIDUAL || ep.act == ACT_SIGMOID; }
@@ -1910,8 +1913,9 @@ double dma_cost(CostOf of, int tile, int64_t T, int64_t tiles, int nk, int c, si
             const auto &k = kg[of.w_u8][tile == TILE_K4];
             const int64_t last = wgs % 256;
             const double round = c > 1 ? k.split_round : k.round, n = nk / c;
-            return k.launch + (double)(wgs / 256) * (round + n * k.step_1) +
-                   (last ? round + n * (k.step_0 + (k.step_1 - k.step_0) * (double)last / 256) : 0.0) + reduce;
+            double step = k.step_0 + (k.step_1 - k.step_0) * (double)last / 256;
+            if (!of.w_u8 && tile == TILE_K4) step = std::max(step, 0.32);
+            return k.launch + (double)(wgs / 256) * (round + n * k.step_1) + (last ? round + n * step : 0.0) + reduce;
         }
     }
 }
