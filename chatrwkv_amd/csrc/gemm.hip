@@ -835,25 +835,13 @@ DEV void gemm_dma_body(int bid, int T, int N, int M, const h16 *__restrict__ A, 
                                 acc[a][b][e];
             }
             constexpr int ITS = (TM < 128 ? TM : 128) / RPI, AHEAD_ROWS = TM == 256 ? 2 : 4;   // rows of a thread; rows requested together
-            EpiIn in[AHEAD_ROWS];
+            if (four) {   // a loop of its own: nothing of the other one's rows in flight is carried along
+                __syncthreads();
 #pragma unroll 1
-            for (int it = 0; it < ITS; ++it) {
-                const int row = it * RPI + tid / CPR, t = t0 + h * 128 + row;
-                const bool valid = t < T && col_ok;
-                if (it % AHEAD_ROWS == 0) {
-                    if (!four) {
+                for (int it = 0; it < ITS; ++it) {
+                    const int row = it * RPI + tid / CPR, t = t0 + h * 128 + row;
+                    if (t >= T) break;
 #pragma unroll
-                        for (int i = 0; i < AHEAD_ROWS; ++i) in[i] = epi_in(ep, t + i * RPI, col, t + i * RPI < T && col_ok, W_U8 && !lds_sums);
-                    }
-                    if (it == 0) __syncthreads();   // the accumulators are in LDS
-                }
-                const EpiIn cur = in[0];
-#pragma unroll
-                for (int i = 0; i + 1 < AHEAD_ROWS; ++i) in[i] = in[i + 1];   // a loop that is not unrolled has no other index
-                float a0 = 0.f, a2 = 0.f;
-                if (four) {
-                    if (t >= T) continue;
-#pragma unroll 1
                     for (int g = 0; g < 2; ++g) {
                         const int c = g * (TN / 2) + cq * 4;
                         if (m0 + c >= M) continue;
@@ -864,8 +852,24 @@ DEV void gemm_dma_body(int bid, int T, int N, int M, const h16 *__restrict__ A, 
                         }
                         finish_row4(v, t, m0 + c, M, ep, Y, ldy);
                     }
-                    continue;
                 }
+                __syncthreads();
+                continue;
+            }
+            EpiIn in[AHEAD_ROWS];
+#pragma unroll 1
+            for (int it = 0; it < ITS; ++it) {
+                const int row = it * RPI + tid / CPR, t = t0 + h * 128 + row;
+                const bool valid = t < T && col_ok;
+                if (it % AHEAD_ROWS == 0) {
+#pragma unroll
+                    for (int i = 0; i < AHEAD_ROWS; ++i) in[i] = epi_in(ep, t + i * RPI, col, t + i * RPI < T && col_ok, W_U8 && !lds_sums);
+                    if (it == 0) __syncthreads();   // the accumulators are in LDS
+                }
+                const EpiIn cur = in[0];
+#pragma unroll
+                for (int i = 0; i + 1 < AHEAD_ROWS; ++i) in[i] = in[i + 1];   // a loop that is not unrolled has no other index
+                float a0 = 0.f, a2 = 0.f;
                 if (valid) {
                     const f32x4 v0 = *(const f32x4 *)(stg + row * SW + cq * 8), v1 = *(const f32x4 *)(stg + row * SW + cq * 8 + 4);
                     float v[8] = {v0[0], v0[1], v0[2], v0[3], v1[0], v1[1], v1[2], v1[3]};
@@ -1228,32 +1232,13 @@ DEV void gemm_kg_body(int bid, int T, int N, int M, const h16 *__restrict__ A, i
             if (t < T && col + 4 < M) *(f32x4 *)(slab + (size_t)t * M + col + 4) = hi;
         }
     } else {
-        const bool emit = ep.emit_ry != nullptr, four = by_four(M, ldy, Y, ep);
-        h16x8 rx8 = {}, mx8 = {};
-        Emit8 em = {};
-        EpiIn in[AHEAD_ROWS] = {};
-        if (!four) {
-            if (W_U8 && col_ok) { rx8 = load_n<h16x8, 8>(ep.rx + col, M - col); mx8 = load_n<h16x8, 8>(ep.mx + col, M - col); }
-            em = emit8(ep, col, col_ok);
-        }
+        if (by_four(M, ldy, Y, ep)) {   // a loop of its own, as in gemm_dma_body
+            __syncthreads();
 #pragma unroll 1
-        for (int it = 0; it < ITS; ++it) {
-            const int r = it * RPI + tid / CPR, t = t0 + r;
-            if (it % AHEAD_ROWS == 0) {
-                if (!four) {
+            for (int it = 0; it < ITS; ++it) {
+                const int r = it * RPI + tid / CPR, t = t0 + r;
+                if (t >= T) break;
 #pragma unroll
-                    for (int i = 0; i < AHEAD_ROWS; ++i) in[i] = epi_in(ep, t + i * RPI, col, t + i * RPI < T && col_ok, W_U8 && !lds_sums);
-                }
-                if (it == 0) __syncthreads();   // the partial tiles are in LDS
-            }
-            const EpiIn cur = in[0];
-#pragma unroll
-            for (int i = 0; i + 1 < AHEAD_ROWS; ++i) in[i] = in[i + 1];
-            const bool valid = t < T && col_ok;
-            float a0 = 0.f, a2 = 0.f;
-            if (four) {
-                if (t >= T) continue;
-#pragma unroll 1
                 for (int g = 0; g < 2; ++g) {
                     const int c = g * (TN / 2) + cq * 4;
                     if (m0 + c >= M) continue;
@@ -1262,8 +1247,27 @@ DEV void gemm_kg_body(int bid, int T, int N, int M, const h16 *__restrict__ A, i
                     if constexpr (W_U8) affine4(v, m0 + c, M, lds_sums ? lsum[r] : ep.s0[t], lds_sums ? lsum[TM + r] : ep.s2[t], ep);
                     finish_row4(v, t, m0 + c, M, ep, Y, ldy);
                 }
-                continue;
             }
+            return;
+        }
+        const bool emit = ep.emit_ry != nullptr;
+        h16x8 rx8 = {}, mx8 = {};
+        EpiIn in[AHEAD_ROWS] = {};
+        if (W_U8 && col_ok) { rx8 = load_n<h16x8, 8>(ep.rx + col, M - col); mx8 = load_n<h16x8, 8>(ep.mx + col, M - col); }
+        const Emit8 em = emit8(ep, col, col_ok);
+#pragma unroll 1
+        for (int it = 0; it < ITS; ++it) {
+            const int r = it * RPI + tid / CPR, t = t0 + r;
+            if (it % AHEAD_ROWS == 0) {
+#pragma unroll
+                for (int i = 0; i < AHEAD_ROWS; ++i) in[i] = epi_in(ep, t + i * RPI, col, t + i * RPI < T && col_ok, W_U8 && !lds_sums);
+                if (it == 0) __syncthreads();   // the partial tiles are in LDS
+            }
+            const EpiIn cur = in[0];
+#pragma unroll
+            for (int i = 0; i + 1 < AHEAD_ROWS; ++i) in[i] = in[i + 1];
+            const bool valid = t < T && col_ok;
+            float a0 = 0.f, a2 = 0.f;
             if (valid) {
                 f32x4 lo, hi;
                 tile_sum(r, cq * 8, lo);
