@@ -1873,7 +1873,8 @@ constexpr TileDim tile_dim[TILES] = {{256, 256}, {128, 128}, {128, 128}, {64, 12
 // 64 rows ran through it instead of the 64 x 64 tile, 5 % of such a model's call).
 // Four stages: launches of one round only (one workgroup per CU); its step grows from 0.38 us with 64 CUs busy to
 // 0.50 us with 216 and does not grow further: with 0.53 us for all of them launches of exactly 256 workgroups took the
-// three-stage tile, which is 5 to 9 % slower there (512 x 4096 x 8192 49.7 / 46.7, 1024 x 4096 x 4096 51.2 / 48.5).
+// three-stage tile, which is 5 to 9 % slower there (512 x 4096 x 8192 49.7 / 46.7, 1024 x 4096 x 4096 51.2 / 48.5).  fp16 weights:
+// from 0.30 us, 20 steps of fill, drain and epilogue.
 // Two of its launches cost more.  An epilogue that reads a residual or takes an exponential ends a tile by itself where a
 // split leaves it to the whole chip in the second pass: 2 us, below 32 k-tiles.  Without them the square products of models
 // of 1152 to 1792 channels ran through it at full depth instead of in two splits of the three-stage tile (6 layers, RWKV-4,
@@ -1887,10 +1888,15 @@ constexpr TileDim tile_dim[TILES] = {{256, 256}, {128, 128}, {128, 128}, {64, 12
 // 128 x 128 ones, 120 us against 116 with fp16 weights; with uint8 weights and 1024 rows it belongs there (118.5 against 120.5).
 // gemm_kg_kernel: per launch, per round (split launches leave the epilogue to the second pass) and per k-tile by the CUs busy,
 // fitted to 1640 products (21 lengths, 8 widths) with the other tiles' prices as they stand: the tile it picks is 1.5 % slower
-// than the best of all on average, 4.2 % with the four tiles and prices before; 3.3 % less time.  fp16, 64 x 128 tile: the line
-// of that fit is far too low below 150 CUs, where such launches would have few and long tiles and split K: a CU then takes 24 KB a
-// k-tile in 0.32 to 0.37 us whatever the others do.  Callers without scratch for a split got it all the same: [48 x 16384] x
-// [16384 x 1000] 94 us, 61 with the 64 x 64 tile, [64 x 4096] x [4096 x 512] 29.7 and 21.4.
+// than the best of all on average, 4.2 % with the four tiles and prices before; 3.3 % less time.  fp16, 64 x 128 tile: the line of
+// that fit, 0.17 us a k-tile and up, was far too low: a CU takes its 24 KB in 0.32 to 0.5 us whatever the others do.  Callers
+// without scratch for a split got it for long rows and few tiles, [48 x 16384] x [16384 x 1000] 94 us, 61 with the 64 x 64 tile,
+// [64 x 4096] x [4096 x 512] 29.7 and 21.4, and those with scratch beside four stages, whose price for fp16 was too high:
+// [256 x 5120] x [5120 x 5120] 39.7 us, 35.7 with four stages, [513 x 3904] x [3904 x 2880] 35.5 and 30.4 (336 products of 24 widths: 15
+// change, all for the better).  Both tiles: 0.08 us more per k-tile
+// of what exceeds one round, of which that fit had little.  uint8, that tile and the one it is now: [1922 x 3904] x [3904 x
+// 2880] 83.7 and 67.8 us, [663 x 3584] x [3584 x 7042] 76.2 and 66.4, [45 x 2048] x [2048 x 65536] 42.7 and 37.7 (672 products
+// of 24 widths: eight change, 3 to 19 % faster each).
 // slow_epi: see slow_epilogue.
 struct CostOf { bool w_u8, slow_epi; };
 bool slow_epilogue(const GemmEpi &ep) { return ep.act == ACT_RESIDUAL || ep.act == ACT_GATED_RESIDUAL || ep.act == ACT_SIGMOID; }
@@ -1908,18 +1914,19 @@ double dma_cost(CostOf of, int tile, int64_t T, int64_t tiles, int nk, int c, si
             if (rounds > 1) return 1e30;
             if (!of.w_u8 && nk / c >= 128)
                 return (nk / c + 17.0) * (0.42 + 0.12 * (double)wgs / 256) * (0.55 + 0.45 * T / (double)((T + 127) / 128 * 128)) + reduce;
-            return (nk / c + 22.0) * std::min(0.50, 0.34 + 0.19 * (double)wgs / 256) + reduce + (c == 1 && of.slow_epi && nk < 32 ? 2.0 : 0.0);
+            return (nk / c + (of.w_u8 ? 22.0 : 20.0)) * std::min(0.50, (of.w_u8 ? 0.34 : 0.30) + 0.19 * (double)wgs / 256) + reduce +
+                   (c == 1 && of.slow_epi && nk < 32 ? 2.0 : 0.0);
         case TILE_N: return T > 64 ? 1e30 : (double)rounds * (nk / c + std::max(16.5, 13.0 + T / 10.0)) * 0.327 + reduce;
         default: {
             // [uint8][groups 8, 4]
             constexpr struct { double launch, round, split_round, step_0, step_1; } kg[2][2] = {
-                {{3.0, 2.6, 3.6, 0.195, 0.212}, {2.8, 3.6, 4.8, 0.170, 0.420}}, {{2.1, 3.0, 2.5, 0.140, 0.186}, {2.9, 4.2, 3.8, 0.212, 0.320}}};
+                {{3.0, 2.6, 3.6, 0.195, 0.212}, {2.8, 3.6, 4.8, 0.36, 0.37}}, {{2.1, 3.0, 2.5, 0.140, 0.186}, {2.9, 4.2, 3.8, 0.212, 0.320}}};
             const auto &k = kg[of.w_u8][tile == TILE_K4];
             const int64_t last = wgs % 256;
             const double round = c > 1 ? k.split_round : k.round, n = nk / c;
-            double step = k.step_0 + (k.step_1 - k.step_0) * (double)last / 256;
-            if (!of.w_u8 && tile == TILE_K4) step = std::max(step, 0.32);
-            return k.launch + (double)(wgs / 256) * (round + n * k.step_1) + (last ? round + n * step : 0.0) + reduce;
+            return k.launch + (double)(wgs / 256) * (round + n * k.step_1) +
+                   (last ? round + n * (k.step_0 + (k.step_1 - k.step_0) * (double)last / 256) : 0.0) +
+                   0.08 * n * std::max((double)wgs / 256 - 1.0, 0.0) + reduce;
         }
     }
 }
