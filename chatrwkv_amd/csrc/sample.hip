@@ -453,11 +453,11 @@ __global__ __launch_bounds__(STHREADS) void sample_kernel(SampleArgs a) {
 //           probabilities and the occurrence counts of its segment.
 // Sums are added in a fixed order throughout.  Where the total is no positive number (a NaN, an infinity or nothing but masks
 // among the logits) nothing is kept and id 0 is drawn, which is what the kernel above makes of such logits.
-// Bound by the latency of the three launches.  Measured as above, V = 65536: 19.8 us a draw (2.9 + 4.3 + 10.8 and the gaps), 38 with one
+// Bound by the latency of the three launches.  Measured as above, V = 65536: 20 us a draw (2.9 + 4.3 + 10.8 and the gaps), 38 with one
 // workgroup; with the lists in LDS and the bracket searched by search_list 25.8, 5 us of it in the search.
 constexpr int SEG = 1024, SEGS_MAX = 64, BOUNDS = 32;
 constexpr int FEW = 256;                      // entries of a bracket that are compared with each other at once
-constexpr int PART = 2 * BOUNDS + 2;          // per segment: sums and counts at the bounds, sum of all, length of the list
+constexpr int PART = 2 * BOUNDS + 3;          // per segment: sums and counts at the bounds, sum of all, length of the list, its smallest entry
 
 struct SampleWs {
     float *p;          // [segments][SEG] adjusted logits, then probabilities
@@ -527,6 +527,25 @@ DEV float bound_at(float pmax, int k) { return __uint_as_float(__float_as_uint(p
 DEV unsigned long long fixed(float p) { return (unsigned long long)(p * 0x1p62f); }
 DEV float from_fixed(unsigned long long s) { return (float)s * 0x1p-62f; }
 
+// Sums over the 16 lanes of a row, in every one of them.
+constexpr int COPIES = 16;
+template <int CTRL> DEV unsigned dpp_u32(unsigned v) { return (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xf, 0xf, true); }
+template <int CTRL> DEV unsigned long long dpp_u64(unsigned long long v) {
+    return (unsigned long long)dpp_u32<CTRL>((unsigned)(v >> 32)) << 32 | dpp_u32<CTRL>((unsigned)v);
+}
+DEV unsigned row16_total(unsigned v) {
+    v += dpp_u32<0xB1>(v);    // quad_perm: neighbours, then pairs
+    v += dpp_u32<0x4E>(v);
+    v += dpp_u32<0x141>(v);   // row_half_mirror
+    return v + dpp_u32<0x140>(v);   // row_mirror
+}
+DEV unsigned long long row16_total(unsigned long long v) {
+    v += dpp_u64<0xB1>(v);
+    v += dpp_u64<0x4E>(v);
+    v += dpp_u64<0x141>(v);
+    return v + dpp_u64<0x140>(v);
+}
+
 // POW: the candidates' powers are formed here, four entries a thread over the chip.  In sample_draw_kernel each of the up to 64
 // workgroups formed those of all candidates, 64 a thread, half of a draw from flat logits.  us a draw, 50277 entries, top_p 0.85,
 // temperature 0.8, one workgroup / powers there / here: N(0, 0.3) 81 / 95 / 45, N(0, 3) 68 / 38 / 24.
@@ -534,7 +553,7 @@ template <bool POW>
 __global__ __launch_bounds__(256) void sample_probs_kernel(SampleArgs a, SampleWs ws) {
     __shared__ unsigned long long bin_s[BOUNDS];   // sums in fixed point
     __shared__ unsigned bin_n[BOUNDS];
-    __shared__ float red[4][2];
+    __shared__ float red[4][2], least[4];
     if (threadIdx.x < BOUNDS) { bin_s[threadIdx.x] = 0; bin_n[threadIdx.x] = 0; }
     const int i0 = blockIdx.x * SEG + 4 * threadIdx.x, lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     f32x4 p = *(const f32x4 *)(ws.p + i0);
@@ -558,13 +577,16 @@ __global__ __launch_bounds__(256) void sample_probs_kernel(SampleArgs a, SampleW
     const float total = wave_sum((p[0] + p[1]) + (p[2] + p[3]));
     unsigned long long in[4];
     int before = 0, n_wave = 0;
+    float small = INFINITY;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
         in[e] = __ballot(p[e] >= floor_);
+        small = p[e] >= floor_ ? fminf(small, p[e]) : small;
         before += (int)__popcll(in[e] & ((1ull << lane) - 1));
         n_wave += (int)__popcll(in[e]);
     }
-    if (lane == 0) { red[wave][0] = total; red[wave][1] = (float)n_wave; }
+    small = -wave_max(-small);
+    if (lane == 0) { red[wave][0] = total; red[wave][1] = (float)n_wave; least[wave] = small; }
     __syncthreads();
     int at = blockIdx.x * SEG + before;
 #pragma unroll
@@ -578,6 +600,7 @@ __global__ __launch_bounds__(256) void sample_probs_kernel(SampleArgs a, SampleW
             ws.idx[at++] = (uint16_t)(4 * threadIdx.x + e);
         }
     float *part = ws.part + blockIdx.x * PART;
+    if (threadIdx.x == 2) part[2 * BOUNDS + 2] = fminf(fminf(least[0], least[1]), fminf(least[2], least[3]));
     if (threadIdx.x < 2) part[2 * BOUNDS + threadIdx.x] = (red[0][threadIdx.x] + red[1][threadIdx.x]) + (red[2][threadIdx.x] + red[3][threadIdx.x]);
     if (wave == 1 && lane < BOUNDS) {   // an entry of bin k reaches the bounds from k on
         unsigned long long sum = 0;
@@ -596,8 +619,8 @@ template <bool POW>
 __global__ __launch_bounds__(STHREADS) void sample_draw_kernel(SampleArgs a, SampleWs ws) {
     __shared__ f32x4 red[2][SWAVES / 2];
     __shared__ float seg_sum[SEGS_MAX];
-    __shared__ unsigned long long part_s[64];
-    __shared__ unsigned part_n[64];
+    __shared__ unsigned long long part_s[64 * COPIES], total_s[64];
+    __shared__ unsigned part_n[64 * COPIES], total_n[64];
     __shared__ __align__(16) float cols[2 * BOUNDS][SWAVES + 4], few[FEW], sorted[FEW];
     __shared__ int pick, n_few[2];
     const int V = a.V, tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), segs = gridDim.x;
@@ -715,13 +738,21 @@ __global__ __launch_bounds__(STHREADS) void sample_draw_kernel(SampleArgs a, Sam
             hi = __float_as_uint(bound_at(pmax, k - 1));
             at_hi = {__shfl(at_k.s, k - 1, WAVE), __shfl(at_k.n, k - 1, WAVE)};
         }
+        if (!counts && at_lo.n == n && n - at_hi.n > (float)FEW)   // all candidates reach lo: begin at the smallest of them
+            lo = max(lo, __float_as_uint(-wave_max(lane < segs ? -ws.part[lane * PART + 2 * BOUNDS + 2] : -INFINITY)));
         while (hi - lo > 1 && at_lo.n - at_hi.n > (float)FEW) {
             // Sums and counts of up to 64 equal parts of the interval.  us a draw, one workgroup / bisection down to 1024 entries and a
             // list of these / this: 65536 equal logits, top_p 0.7 67 / 68 / 34, 50277 of them 58 / 67 / 33; 50277 from N(0, 3),
-            // top_p 0.999 40.6 / 49.3 / 41.1 (58.5 from 0 up instead of list_floor: three parts take all additions).
+            // top_p 0.999 40.6 / 49.3 / 41.1 (58.5 from 0 up instead of list_floor: three parts take all additions).  Logits closer to
+            // each other than that fell into two or three parts, whose additions wait for each other: so the interval begins at the
+            // smallest candidate, and a part has COPIES sums, each for four lanes of a wave.  50277 from N(0, 0.003), top_p 0.7, one workgroup /
+            // neither / the former / both 51 / 117 / 57.5 / 50.7, N(0, 0.03) 46.4 / 61.7 / 54.9 / 49.7, N(0, 0.3) 42.0 / 42.0 / 42.3 /
+            // 43.5, equal ones 58 / 33 / 19 / 19, N(0, 3) 32.0 / 16.2 / 16.3 / 16.4.
             const int shift = max(26 - __builtin_clz(hi - lo - 1), 0);
             const float flo = __uint_as_float(max(lo, 1u)), fhi = __uint_as_float(hi);
-            if (tid < 64) { part_s[tid] = 0; part_n[tid] = 0; }
+            static_assert(64 * COPIES == STHREADS, "a thread clears and adds up a copy");
+            part_s[tid] = 0;
+            part_n[tid] = 0;
             __syncthreads();
             each([&](float x) {
                 const bool in = x >= flo && x < fhi;
@@ -732,14 +763,20 @@ __global__ __launch_bounds__(STHREADS) void sample_draw_kernel(SampleArgs a, Sam
                 const int n = ties ? (int)__popcll(m) : 1;
                 if (ties ? lane == 0 : in) {
                     const float y = ties ? __uint_as_float(first) : x;
-                    const unsigned part = (__float_as_uint(y) - lo) >> shift;
+                    const unsigned part = ((__float_as_uint(y) - lo) >> shift) * COPIES + (lane & (COPIES - 1));
                     atomicAdd(&part_s[part], (unsigned long long)n * fixed(y));
                     atomicAdd(&part_n[part], (unsigned)n);
                 }
             });
             __syncthreads();
+            {
+                const unsigned long long s = row16_total(part_s[tid]);
+                const unsigned n = row16_total(part_n[tid]);
+                if ((tid & (COPIES - 1)) == 0) { total_s[tid / COPIES] = s; total_n[tid / COPIES] = n; }
+            }
+            __syncthreads();
             // lane i: the part i from above, and the sum and the count from its lower end on
-            const SumCount t = {at_hi.s + wave_scan(from_fixed(part_s[63 - lane])), at_hi.n + wave_scan((float)part_n[63 - lane])};
+            const SumCount t = {at_hi.s + wave_scan(from_fixed(total_s[63 - lane])), at_hi.n + wave_scan((float)total_n[63 - lane])};
             const unsigned long long good = __ballot(enough(t, top_p, want));
             const int i = good ? __builtin_ctzll(good) : 63;
             if (good) at_lo = {__shfl(t.s, i, WAVE), __shfl(t.n, i, WAVE)};

@@ -358,17 +358,20 @@ def test_draw_without_a_total_as_one_workgroup_makes_it(V, temp, kind):
 
 
 def _wide(kind, V, rng):
-    """Logits of which thousands lie in half an octave: equal ones, two levels, a slope, all with a few outliers and masks"""
+    """Logits of which thousands lie in half an octave: equal ones, two levels, a slope, close ones (an untrained model's), all
+    with masks and all but equal and close ones with a few outliers"""
     if kind == "equal":
         x = np.zeros(V)
     elif kind == "levels":
         x = np.where(rng.random(V) < 0.4, 0.0, -0.25)
     elif kind == "slope":
         x = rng.permutation(V) * (0.3 / V)
+    elif kind == "close":
+        x = rng.standard_normal(V) * 0.003
     else:
         x = rng.standard_normal(V) * 3
     x = x.astype(np.float32)
-    if kind != "equal":
+    if kind not in ("equal", "close"):
         x[rng.integers(0, V, 3)] += 2
     x[rng.integers(0, V, 20)] = -np.inf
     return torch.from_numpy(x).to(DEV)
@@ -381,7 +384,7 @@ def _one_workgroup(L, x, temp, top_p, top_k, u, probs, token):
 
 
 @pytest.mark.parametrize("V", [16388, 50277, 65536])
-@pytest.mark.parametrize("kind", ["equal", "levels", "slope", "normal"])
+@pytest.mark.parametrize("kind", ["equal", "levels", "slope", "close", "normal"])
 def test_draw_from_logits_close_to_each_other(V, kind):
     """Thousands of entries around the cut, ties among them: kept sets and probabilities as the one-workgroup kernel has them;
     bounds as in test_draw_over_the_chip_against_one_workgroup (equal entries stand or fall together)."""
@@ -408,7 +411,7 @@ def test_draw_from_logits_close_to_each_other(V, kind):
 
 
 @pytest.mark.parametrize("V", [16388, 50277, 65536])
-@pytest.mark.parametrize("kind,top_p,temp", [("equal", 0.7, 1.0), ("slope", 0.85, 0.8), ("normal", 0.999, 1.0), ("normal", 0.999, 0.8)])
+@pytest.mark.parametrize("kind,top_p,temp", [("equal", 0.7, 1.0), ("close", 0.7, 1.0), ("slope", 0.85, 0.8), ("normal", 0.999, 1.0), ("normal", 0.999, 0.8)])
 def test_draws_over_the_chip_are_not_slower(V, kind, top_p, temp):
     """Draws that keep or search thousands of entries: the three launches take no longer than the one-workgroup kernel on the
     same operands, by the best of several runs (a tenth is left for the clock)."""
