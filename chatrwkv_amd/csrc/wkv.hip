@@ -1,5 +1,6 @@
 // WKV recurrences: RWKV-4 (per channel, running-maximum form) and RWKV-5/6 (per-head 64x64 state).
 #include <algorithm>
+#include <type_traits>
 #include "gemv_core.h"
 #include "kernels.h"
 
@@ -14,27 +15,27 @@ namespace {
 //   MODE 1: k, v fp16; y = fp16(r * fp16(wkv)) with r fp16 (already sigmoid'ed), fp16 out
 //   MODE 2: as MODE 1 with k, v fp32
 // ---------------------------------------------------------------------------------------
-template <int MODE> struct Wkv4IO;
-template <> struct Wkv4IO<0> {
-    const float *k, *v; float *y; const rwkv_half *r;
-    DEV float ldk(size_t i) const { return k[i]; }
-    DEV float ldv(size_t i) const { return v[i]; }
-    DEV float ldr(size_t) const { return 1.f; }
-    DEV void st(size_t i, float wkv, float) const { y[i] = wkv; }
+// Rows of a tensor from one that the whole wave shares on: element c of row t by buffer instructions, whose address is a scalar
+// base, a scalar offset t C and the lane's own, so that a token costs a few scalar instructions.  One wave per SIMD is bound by
+// how many instructions it issues.
+template <class E> struct Rows {
+    __amdgpu_buffer_rsrc_t p;
+    DEV Rows(const E *base) : p(__builtin_amdgcn_make_buffer_rsrc((void *)base, 0, -1, 0x00027000)) {}
+    DEV float ld(int row, int c) const {
+        if constexpr (sizeof(E) == 4) return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(p, 4 * c, 4 * row, 0));
+        else return h2f(__builtin_amdgcn_raw_buffer_load_b16(p, 2 * c, 2 * row, 0));
+    }
+    DEV void st(int row, int c, float v) const {
+        if constexpr (sizeof(E) == 4) __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), p, 4 * c, 4 * row, 0);
+        else __builtin_amdgcn_raw_buffer_store_b16(f2h(v), p, 2 * c, 2 * row, 0);
+    }
 };
-template <> struct Wkv4IO<1> {
-    const rwkv_half *k, *v; rwkv_half *y; const rwkv_half *r;
-    DEV float ldk(size_t i) const { return h2f(k[i]); }
-    DEV float ldv(size_t i) const { return h2f(v[i]); }
-    DEV float ldr(size_t i) const { return h2f(r[i]); }
-    DEV void st(size_t i, float wkv, float rr) const { y[i] = f2h(rr * round_h(wkv)); }
-};
-template <> struct Wkv4IO<2> {
-    const float *k, *v; rwkv_half *y; const rwkv_half *r;
-    DEV float ldk(size_t i) const { return k[i]; }
-    DEV float ldv(size_t i) const { return v[i]; }
-    DEV float ldr(size_t i) const { return h2f(r[i]); }
-    DEV void st(size_t i, float wkv, float rr) const { y[i] = f2h(rr * round_h(wkv)); }
+template <int MODE> struct Wkv4IO {
+    using KV = std::conditional_t<MODE == 1, rwkv_half, float>;
+    using Y = std::conditional_t<MODE == 0, float, rwkv_half>;
+    const KV *k, *v;
+    Y *y;
+    const rwkv_half *r;
 };
 
 // Sums of two products as one product that is rounded and one that is not, spelled out: left to the compiler, which of the two
@@ -54,40 +55,53 @@ DEV void wkv4_step(float kk, float vv, float u, float w, float &aa, float &bb, f
     pp = p;
 }
 
-// The tokens [t0, t1) of channel c in turn, step(k, v, r, place).  Two batches of eight tokens: one is in flight while the
+// The tokens [t0, t1) of channel c of the rows from `base` on, in turn: step(k, v, out), and out stored where OUT.  Two batches of eight tokens: one is in flight while the
 // other goes through the chain.  Every load is issued (past the end the last token again): with the loads of a batch in front
 // of its own steps, and those of the last T % 8 tokens in front of each, the chain waited for memory once per batch and token.
-// Measured, us: 45 tokens, 4096 channels 9.6 -> 8.0; chunked, 1024 tokens, 4096 channels 6.7 + 17.2 -> 7.1 + 13.6, 513 tokens, 768
-// channels 4.1 + 11.0 -> 4.6 + 8.1 (the second launch also folds its chunk's predecessors eight at a time, not one).
-template <bool R, int MODE, class Step>
-DEV void wkv4_tokens(const Wkv4IO<MODE> &io, size_t base, int C, int t0, int t1, Step step) {
+// Measured within a call, us, eight tokens' loads in front of their steps / two batches with 64-bit addresses per lane / now: 45
+// tokens, 4096 channels 9.3 / 7.7 / 7.3; chunked, 1024 tokens, 4096 channels 6.3 + 17.3 / 7.2 + 13.9 / 6.4 + 13.9, 513 tokens, 768
+// channels 4.7 + 10.5 / 4.4 + 8.1 / 4.0 + 7.8 (the second launch also folds its chunk's predecessors eight at a time, not one).
+// Operands in the caches, 1024 tokens, 768 channels 96.6 / 106 / 101.
+template <bool OUT, int MODE, class Step>
+DEV void wkv4_tokens(const Wkv4IO<MODE> &io, size_t base, int c, int C, int t0, int t1, Step step) {
     constexpr int UNR = 8;
+    constexpr bool R = OUT && MODE != 0;
     struct Batch { float k[UNR], v[UNR], r[UNR]; } b0, b1;
-    auto load = [&](Batch &b, int t) {
+    size_t row = base + (size_t)t0 * C;
+    int left = t1 - t0;       // tokens from `row` on
+    auto load = [&](Batch &b, int at) {
+        const Rows<typename Wkv4IO<MODE>::KV> k(io.k + row), v(io.v + row);
+        const Rows<rwkv_half> r(io.r + row);
 #pragma unroll
         for (int i = 0; i < UNR; ++i) {
-            const size_t o = base + (size_t)min(t + i, t1 - 1) * C;
-            b.k[i] = io.ldk(o);
-            b.v[i] = io.ldv(o);
-            b.r[i] = R ? io.ldr(o) : 0.f;
+            const int o = min(at + i, left - 1) * C;
+            b.k[i] = k.ld(o, c);
+            b.v[i] = v.ld(o, c);
+            b.r[i] = R ? r.ld(o, c) : 0.f;
         }
     };
-    auto run = [&](const Batch &b, int t) {
-        if (t + UNR <= t1) {   // no branch between the tokens: the division of one runs beside the chain of the next
+    load(b0, 0);
+    for (; left > 0; left -= 2 * UNR, row += 2 * UNR * (size_t)C) {
+        const Rows<typename Wkv4IO<MODE>::Y> y(io.y + row);
+        auto one = [&](const Batch &b, int at, int i) {
+            float out = 0.f;
+            step(b.k[i], b.v[i], out);
+            if (OUT) y.st((at + i) * C, c, MODE == 0 ? out : b.r[i] * round_h(out));
+        };
+        auto run = [&](const Batch &b, int at) {
+            if (at + UNR <= left) {   // no branch between the tokens: the division of one runs beside the chain of the next
 #pragma unroll
-            for (int i = 0; i < UNR; ++i) step(b.k[i], b.v[i], b.r[i], base + (size_t)(t + i) * C);
-        } else {
+                for (int i = 0; i < UNR; ++i) one(b, at, i);
+            } else {
 #pragma unroll
-            for (int i = 0; i < UNR - 1; ++i)
-                if (t + i < t1) step(b.k[i], b.v[i], b.r[i], base + (size_t)(t + i) * C);
-        }
-    };
-    load(b0, t0);
-    for (int t = t0; t < t1; t += 2 * UNR) {
-        load(b1, t + UNR);
-        run(b0, t);
-        load(b0, t + 2 * UNR);
-        run(b1, t + UNR);
+                for (int i = 0; i < UNR - 1; ++i)
+                    if (at + i < left) one(b, at, i);
+            }
+        };
+        load(b1, UNR);
+        run(b0, 0);
+        load(b0, 2 * UNR);
+        run(b1, UNR);
     }
 }
 
@@ -101,11 +115,7 @@ __global__ __launch_bounds__(64) void wkv4_kernel(int T, int C, const float *__r
     const int so = b * C + c;
     const float u = u_[c], w = w_[c];
     float aa = aa_[so], bb = bb_[so], pp = pp_[so];
-    wkv4_tokens<true>(io, (size_t)b * T * C + c, C, 0, T, [&](float kk, float vv, float rr, size_t o) {
-        float out;
-        wkv4_step(kk, vv, u, w, aa, bb, pp, out);
-        io.st(o, out, rr);
-    });
+    wkv4_tokens<true>(io, (size_t)b * T * C, c, C, 0, T, [&](float kk, float vv, float &out) { wkv4_step(kk, vv, u, w, aa, bb, pp, out); });
     aa_[so] = aa; bb_[so] = bb; pp_[so] = pp;
 }
 
@@ -141,7 +151,7 @@ __global__ __launch_bounds__(64) void wkv4_chunk_summary_kernel(int T, int C, in
     }
     const float w = w_[c];
     float aa = 0.f, bb = 0.f, pp = -1e38f;
-    wkv4_tokens<false>(io, c, C, j * L, min(T, (j + 1) * L), [&](float kk, float vv, float, size_t) {
+    wkv4_tokens<false>(io, 0, c, C, j * L, min(T, (j + 1) * L), [&](float kk, float vv, float &) {
         const float ww = w + pp;
         const float p = fmaxf(ww, kk);
         const float e1 = __expf(ww - p), e2 = __expf(kk - p);
@@ -179,11 +189,7 @@ __global__ __launch_bounds__(64) void wkv4_chunk_apply_kernel(int T, int C, int 
                 wkv4_merge(aa, bb, pp, a2[i], b2[i], p2[i]);
             }
     }
-    wkv4_tokens<true>(io, c, C, t0, t1, [&](float kk, float vv, float rr, size_t o) {
-        float out;
-        wkv4_step(kk, vv, u, w, aa, bb, pp, out);
-        io.st(o, out, rr);
-    });
+    wkv4_tokens<true>(io, 0, c, C, t0, t1, [&](float kk, float vv, float &out) { wkv4_step(kk, vv, u, w, aa, bb, pp, out); });
     if (t1 == T) { aa_[c] = aa; bb_[c] = bb; pp_[c] = pp; }
 }
 
