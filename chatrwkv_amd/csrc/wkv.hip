@@ -17,7 +17,8 @@ namespace {
 // ---------------------------------------------------------------------------------------
 // Rows of a tensor from one that the whole wave shares on: element c of row t by buffer instructions, whose address is a scalar
 // base, a scalar offset t C and the lane's own, so that a token costs a few scalar instructions.  One wave per SIMD is bound by
-// how many instructions it issues.
+// how many instructions it issues.  Offsets are 32 bits: up to 24 rows of WKV4_C values.
+constexpr int64_t WKV4_C = 1 << 24;
 template <class E> struct Rows {
     __amdgpu_buffer_rsrc_t p;
     DEV Rows(const E *base) : p(__builtin_amdgcn_make_buffer_rsrc((void *)base, 0, -1, 0x00027000)) {}
@@ -55,9 +56,10 @@ DEV void wkv4_step(float kk, float vv, float u, float w, float &aa, float &bb, f
     pp = p;
 }
 
-// The tokens [t0, t1) of channel c of the rows from `base` on, in turn: step(k, v, out), and out stored where OUT.  Two batches of eight tokens: one is in flight while the
-// other goes through the chain.  Every load is issued (past the end the last token again): with the loads of a batch in front
-// of its own steps, and those of the last T % 8 tokens in front of each, the chain waited for memory once per batch and token.
+// The tokens [t0, t1) of channel c of the rows from `base` on, in turn: step(k, v, out), and out stored where OUT.  Two batches of
+// eight tokens: one is in flight while the other goes through the chain.  Every load is issued (past the end the last token
+// again): with the loads of a batch in front of its own steps, and those of the last T % 8 tokens in front of each, the chain
+// waited for memory once per batch and token.
 // Measured within a call, us, eight tokens' loads in front of their steps / two batches with 64-bit addresses per lane / now: 45
 // tokens, 4096 channels 9.3 / 7.7 / 7.3; chunked, 1024 tokens, 4096 channels 6.3 + 17.3 / 7.2 + 13.9 / 6.4 + 13.9, 513 tokens, 768
 // channels 4.7 + 10.5 / 4.4 + 8.1 / 4.0 + 7.8 (the second launch also folds its chunk's predecessors eight at a time, not one).
@@ -115,7 +117,7 @@ __global__ __launch_bounds__(64) void wkv4_kernel(int T, int C, const float *__r
     const int so = b * C + c;
     const float u = u_[c], w = w_[c];
     float aa = aa_[so], bb = bb_[so], pp = pp_[so];
-    wkv4_tokens<true>(io, (size_t)b * T * C, c, C, 0, T, [&](float kk, float vv, float &out) { wkv4_step(kk, vv, u, w, aa, bb, pp, out); });
+    wkv4_tokens<true>(io, (size_t)b * T * C + blockIdx.x * 64, threadIdx.x, C, 0, T, [&](float kk, float vv, float &out) { wkv4_step(kk, vv, u, w, aa, bb, pp, out); });
     aa_[so] = aa; bb_[so] = bb; pp_[so] = pp;
 }
 
@@ -334,7 +336,15 @@ extern "C" int rwkv_wkv4_forward(int64_t B, int64_t T, int64_t C, const float *w
     dim3 grid((unsigned)((C + 63) / 64), (unsigned)B);
     if (kv_dtype == RWKV_DT_F32) {
         Wkv4IO<0> io{(const float *)k, (const float *)v, (float *)y, nullptr};
-        hipLaunchKernelGGL(wkv4_kernel<0>, grid, dim3(64), 0, (hipStream_t)stream, (int)T, (int)C, w, u, io, aa, bb, pp);
+        if (C <= WKV4_C) {
+            hipLaunchKernelGGL(wkv4_kernel<0>, grid, dim3(64), 0, (hipStream_t)stream, (int)T, (int)C, w, u, io, aa, bb, pp);
+        } else {   // a row at a time: no offsets between rows
+            for (int64_t r = 0; r < B * T; ++r) {
+                const int64_t at = r * C, s = r / T * C;
+                hipLaunchKernelGGL(wkv4_kernel<0>, dim3(grid.x), dim3(64), 0, (hipStream_t)stream, 1, (int)C, w, u,
+                                   (Wkv4IO<0>{io.k + at, io.v + at, io.y + at, nullptr}), aa + s, bb + s, pp + s);
+            }
+        }
     } else {
         return RWKV_E_DTYPE;
     }

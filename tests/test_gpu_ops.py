@@ -625,6 +625,22 @@ def test_wkv4_bits_do_not_depend_on_a_tokens_place(T):
     assert all(torch.equal(a, b) for a, b in zip(one, each))
 
 
+@pytest.mark.parametrize("C", [1 << 24, (1 << 24) + 5])
+def test_wkv4_rows_on_both_sides_of_the_offsets_range(C):
+    """Rows as long as 32-bit offsets allow, and longer ones, which go one at a time: the channels at both ends come out as in calls
+    of their own."""
+    ops = _ops()
+    T = 3
+    k, v = (torch.randn(T, C, device=DEV) for _ in range(2))
+    w, u = -torch.rand(C, device=DEV), torch.randn(C, device=DEV)
+    st = [torch.zeros(C, device=DEV), torch.zeros(C, device=DEV), torch.full((C,), -1e30, device=DEV)]
+    y = ops.cuda_wkv(T, C, w, u, k, v, *st)[0]
+    for part in (slice(0, 100), slice(C - 100, C)):
+        own = [torch.zeros(100, device=DEV), torch.zeros(100, device=DEV), torch.full((100,), -1e30, device=DEV)]
+        want = ops.cuda_wkv(T, 100, w[part], u[part], k[:, part], v[:, part], *own)[0]
+        assert torch.equal(y[:, part], want) and all(torch.equal(a[part], b) for a, b in zip(st, own))
+
+
 @pytest.mark.parametrize("T,H", [(1, 2), (5, 3), (16, 2), (17, 2), (50, 4), (256, 64)])
 @pytest.mark.parametrize("v6", [False, True])
 @pytest.mark.parametrize("layout", [0, 1])
