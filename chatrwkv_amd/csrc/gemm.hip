@@ -114,7 +114,7 @@ DEV V load_n(const rwkv_half *p, int n) {
     return v;
 }
 // May these outputs be stored 16 bytes at a time?  (An output width of 50277 has rows that start anywhere.)
-DEV bool wide_rows(int M, int64_t ldy, const void *Y) { return (((M | (int)ldy) & 7) | (int)((uintptr_t)Y & 15)) == 0; }
+__host__ DEV bool wide_rows(int M, int64_t ldy, const void *Y) { return (((M | (int)ldy) & 7) | (int)((uintptr_t)Y & 15)) == 0; }
 typedef float f32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
 
 // Four outputs: fp32 results, and widths or strides that allow no aligned 16-byte stores of fp16 (no residual, gate or
@@ -159,7 +159,7 @@ DEV Emit8 emit8(const GemmEpi &ep, int col, bool ok) {
     if (ep.emit_ry && ok) { e.ry = *(const h16x8 *)(ep.emit_ry + col); e.my = *(const h16x8 *)(ep.emit_my + col); }
     return e;
 }
-DEV bool by_four(int M, int64_t ldy, const void *Y, const GemmEpi &ep) {
+__host__ DEV bool by_four(int M, int64_t ldy, const void *Y, const GemmEpi &ep) {
     return ep.raw_f32 || ep.out_dtype == RWKV_DT_F32 || !wide_rows(M, ldy, Y);
 }
 // What eight outputs of row t read besides the contraction: the residual and gate, and (uint8 weights) the row's sums.
@@ -507,7 +507,8 @@ constexpr int vm_only(int n) { return 0x0F70 | (n & 15) | ((n >> 4) << 14); }
 constexpr int vm_lgkm0(int n) { return 0x0070 | (n & 15) | ((n >> 4) << 14); }
 constexpr int lgkm_only(int n) { return 0xC07F | (n << 8); }
 
-template <bool W_U8, bool SPLIT, int TM, int TN, int NW = 8, int NSTG = 0>
+// FOURS: outputs leave four at a time (1), eight (0), or as by_four says (-1)
+template <bool W_U8, bool SPLIT, int TM, int TN, int NW, int NSTG, int FOURS>
 DEV void gemm_dma_body(int bid, int T, int N, int M, const h16 *__restrict__ A, int64_t lda, const void *__restrict__ Wv,
                        int64_t ldw, void *__restrict__ Y, int64_t ldy, const GemmEpi &ep, int nk_split,
                        float *__restrict__ part, int split) {
@@ -820,7 +821,8 @@ DEV void gemm_dma_body(int bid, int T, int N, int M, const h16 *__restrict__ A, 
         // fp32 outputs, and rows that start on no 16-byte boundary, leave four at a time.  A 50277-wide head is such a
         // product (through the register-staged kernel before): fp32 out [513 x 768] 109 -> 92 us, [1024 x 4096] 580 -> 542,
         // uint8 weights, fp16 out 133 -> 87 and 706 -> 487.
-        const bool four = by_four(M, ldy, Y, ep);
+        const bool four = FOURS < 0 ? by_four(M, ldy, Y, ep) : FOURS == 1;
+        constexpr bool OWN_LOOP = TM < 256 || FOURS == 1;
         __syncthreads();   // every wave has read its last fragments
 #pragma unroll 1
         for (int h = 0; h < (TM + 127) / 128; ++h) {
@@ -835,23 +837,30 @@ DEV void gemm_dma_body(int bid, int T, int N, int M, const h16 *__restrict__ A, 
                                 acc[a][b][e];
             }
             constexpr int ITS = (TM < 128 ? TM : 128) / RPI, AHEAD_ROWS = TM == 256 ? 2 : 4;   // rows of a thread; rows requested together
-            if (four) {   // a loop of its own: nothing of the other one's rows in flight is carried along
+            auto fours = [&](int row, int t) {
+#pragma unroll OWN_LOOP ? 2 : 1
+                for (int g = 0; g < 2; ++g) {
+                    const int c = g * (TN / 2) + cq * 4;
+                    if (m0 + c >= M) continue;
+                    f32x4 v = *(const f32x4 *)(stg + row * SW + c);
+                    if constexpr (W_U8) {
+                        const int tr = h * 128 + row;
+                        affine4(v, m0 + c, M, lds_sums ? lsum[tr] : ep.s0[t], lds_sums ? lsum[TM + tr] : ep.s2[t], ep);
+                    }
+                    finish_row4(v, t, m0 + c, M, ep, Y, ldy);
+                }
+            };
+            // A loop of their own: nothing of the other one's rows in flight is carried along.  The 256 x 256 tile has no registers
+            // for two loops (34 spilled ones: [1024 x 4096] x [4096 x 16384] 131.1 us instead of 128.6), so its single products have
+            // a kernel for either: fp32 out [256 x 1024] x [1024 x 50277] 44.8 -> 41.1 us, uint8 [1024 x 4096] x [4096 x 50277]
+            // 523 -> 501 (489 with both loops' code before rows were requested ahead).
+            if (OWN_LOOP && four) {
                 __syncthreads();
 #pragma unroll 1
                 for (int it = 0; it < ITS; ++it) {
                     const int row = it * RPI + tid / CPR, t = t0 + h * 128 + row;
                     if (t >= T) break;
-#pragma unroll
-                    for (int g = 0; g < 2; ++g) {
-                        const int c = g * (TN / 2) + cq * 4;
-                        if (m0 + c >= M) continue;
-                        f32x4 v = *(const f32x4 *)(stg + row * SW + c);
-                        if constexpr (W_U8) {
-                            const int tr = h * 128 + row;
-                            affine4(v, m0 + c, M, lds_sums ? lsum[tr] : ep.s0[t], lds_sums ? lsum[TM + tr] : ep.s2[t], ep);
-                        }
-                        finish_row4(v, t, m0 + c, M, ep, Y, ldy);
-                    }
+                    fours(row, t);
                 }
                 __syncthreads();
                 continue;
@@ -862,14 +871,20 @@ DEV void gemm_dma_body(int bid, int T, int N, int M, const h16 *__restrict__ A, 
                 const int row = it * RPI + tid / CPR, t = t0 + h * 128 + row;
                 const bool valid = t < T && col_ok;
                 if (it % AHEAD_ROWS == 0) {
+                    if (OWN_LOOP || !four) {
 #pragma unroll
-                    for (int i = 0; i < AHEAD_ROWS; ++i) in[i] = epi_in(ep, t + i * RPI, col, t + i * RPI < T && col_ok, W_U8 && !lds_sums);
+                        for (int i = 0; i < AHEAD_ROWS; ++i) in[i] = epi_in(ep, t + i * RPI, col, t + i * RPI < T && col_ok, W_U8 && !lds_sums);
+                    }
                     if (it == 0) __syncthreads();   // the accumulators are in LDS
                 }
                 const EpiIn cur = in[0];
 #pragma unroll
                 for (int i = 0; i + 1 < AHEAD_ROWS; ++i) in[i] = in[i + 1];   // a loop that is not unrolled has no other index
                 float a0 = 0.f, a2 = 0.f;
+                if (!OWN_LOOP && four) {
+                    if (t < T) fours(row, t);
+                    continue;
+                }
                 if (valid) {
                     const f32x4 v0 = *(const f32x4 *)(stg + row * SW + cq * 8), v1 = *(const f32x4 *)(stg + row * SW + cq * 8 + 4);
                     float v[8] = {v0[0], v0[1], v0[2], v0[3], v1[0], v1[1], v1[2], v1[3]};
@@ -895,11 +910,11 @@ DEV void gemm_dma_body(int bid, int T, int N, int M, const h16 *__restrict__ A, 
     }
 }
 
-template <bool W_U8, bool SPLIT, int TM, int TN, int NW, int NSTG>
+template <bool W_U8, bool SPLIT, int TM, int TN, int NW, int NSTG, int FOURS>
 __global__ __launch_bounds__(64 * NW) void gemm_dma_kernel(int T, int N, int M, const h16 *__restrict__ A, int64_t lda,
                                                            const void *__restrict__ W, int64_t ldw, void *__restrict__ Y,
                                                            int64_t ldy, GemmEpi ep, int nk_split, float *__restrict__ part) {
-    gemm_dma_body<W_U8, SPLIT, TM, TN, NW, NSTG>(xcd_tile(), T, N, M, A, lda, W, ldw, Y, ldy, ep, nk_split, part, SPLIT ? blockIdx.y : 0);
+    gemm_dma_body<W_U8, SPLIT, TM, TN, NW, NSTG, FOURS>(xcd_tile(), T, N, M, A, lda, W, ldw, Y, ldy, ep, nk_split, part, SPLIT ? blockIdx.y : 0);
 }
 
 // Up to four contractions [T, N] x [N, M_i] in one launch: short calls, where each of them alone would split K and need
@@ -946,7 +961,7 @@ template <bool W_U8, bool SPLIT, int TM, int TN, int NW, int NSTG>
 __global__ __launch_bounds__(64 * NW) void gemm_dma_group_kernel(int T, int N, GemmGroup g) {
     int tile = xcd_tile();
     const int gi = group_member(g, tile), M = g.M[gi];
-    gemm_dma_body<W_U8, SPLIT, TM, TN, NW, NSTG>(tile, T, N, M, g.A[gi], g.lda, g.W[gi], g.ldw[gi], g.Y[gi], M, g.ep[gi],
+    gemm_dma_body<W_U8, SPLIT, TM, TN, NW, NSTG, -1>(tile, T, N, M, g.A[gi], g.lda, g.W[gi], g.ldw[gi], g.Y[gi], M, g.ep[gi],
                                                  SPLIT ? g.nk_split : N / BK, g.part[gi], SPLIT ? blockIdx.y : 0);
 }
 
@@ -1978,12 +1993,15 @@ template <bool W_U8, int TM, int TN, int NW, int NSTG>
 int launch_dma(int ks, int64_t T, int64_t N, int64_t M, const rwkv_half *A, int64_t lda, const void *W, int64_t ldw, void *Y,
                int64_t ldy, GemmEpi ep, hipStream_t st) {
     constexpr size_t lds = DmaCfg<W_U8, TM, TN, NW, NSTG>::LDS;
+    constexpr int FOURS = TM == 256 ? 1 : -1, EIGHTS = TM == 256 ? 0 : -1;
     static PerDeviceOnce once;
     bool *attr_done = once.slot();
     if (!attr_done || !*attr_done) {
-        hipError_t e = hipFuncSetAttribute((const void *)gemm_dma_kernel<W_U8, false, TM, TN, NW, NSTG>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        hipError_t e = hipFuncSetAttribute((const void *)gemm_dma_kernel<W_U8, false, TM, TN, NW, NSTG, EIGHTS>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e == hipSuccess)
-            e = hipFuncSetAttribute((const void *)gemm_dma_kernel<W_U8, true, TM, TN, NW, NSTG>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+            e = hipFuncSetAttribute((const void *)gemm_dma_kernel<W_U8, false, TM, TN, NW, NSTG, FOURS>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        if (e == hipSuccess)
+            e = hipFuncSetAttribute((const void *)gemm_dma_kernel<W_U8, true, TM, TN, NW, NSTG, -1>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) return (int)e;
         if (attr_done) *attr_done = true;
     }
@@ -1992,12 +2010,14 @@ int launch_dma(int ks, int64_t T, int64_t N, int64_t M, const rwkv_half *A, int6
     const int64_t tiles = ((T + TM - 1) / TM) * ((M + TN - 1) / TN);
     const int nk = (int)(N / BK);
     if (ks > 1) {
-        hipLaunchKernelGGL((gemm_dma_kernel<W_U8, true, TM, TN, NW, NSTG>), dim3((unsigned)tiles, (unsigned)ks), dim3(64 * NW), lds, st, (int)T, (int)N,
+        hipLaunchKernelGGL((gemm_dma_kernel<W_U8, true, TM, TN, NW, NSTG, -1>), dim3((unsigned)tiles, (unsigned)ks), dim3(64 * NW), lds, st, (int)T, (int)N,
                            (int)M, (const h16 *)A, lda, W, ldw, Y, ldy, ep, nk / ks, ep.splitk_ws);
         return launch_splitk_epilogue(ks, T, M, Y, ldy, ep, st);
     } else {
-        hipLaunchKernelGGL((gemm_dma_kernel<W_U8, false, TM, TN, NW, NSTG>), dim3((unsigned)tiles), dim3(64 * NW), lds, st, (int)T, (int)N, (int)M,
-                           (const h16 *)A, lda, W, ldw, Y, ldy, ep, nk, (float *)nullptr);
+        const auto kernel = by_four((int)M, ldy, Y, ep) ? gemm_dma_kernel<W_U8, false, TM, TN, NW, NSTG, FOURS>
+                                                       : gemm_dma_kernel<W_U8, false, TM, TN, NW, NSTG, EIGHTS>;
+        hipLaunchKernelGGL(kernel, dim3((unsigned)tiles), dim3(64 * NW), lds, st, (int)T, (int)N, (int)M, (const h16 *)A, lda, W, ldw,
+                           Y, ldy, ep, nk, (float *)nullptr);
     }
     RWKV_LAUNCH_CHECK();
     return RWKV_OK;
