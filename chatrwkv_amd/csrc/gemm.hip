@@ -1,4 +1,4 @@
-// Prefill contraction y[T, M] = xs[T, N] @ W on fp16 MFMA (v_mfma_f32_32x32x16_f16).
+// Prefill contraction y[T, M] = xs[T, N] @ W on fp16 MFMA.
 //
 // W is read in the input-contiguous layout (row m = N consecutive uint8 or fp16).  For
 // uint8 weights each 16-byte global load is widened in registers to the exact fp16 values
@@ -218,24 +218,17 @@ __global__ __launch_bounds__(256) void splitk_epilogue_kernel(int T, int M, int 
 // eight consecutive outputs per thread, all slab loads of a thread in flight together, 16-byte loads of the
 // residual / gate rows and 16-byte stores.  Same slab order and the same arithmetic per element as above.
 template <int KS>
-DEV void slab_sum8(int ks, size_t n, const float *__restrict__ p, f32x4 &lo, f32x4 &hi) {
+DEV void slab_sum8(size_t n, const float *__restrict__ p, f32x4 &lo, f32x4 &hi) {
     lo = *(const f32x4 *)p;
     hi = *(const f32x4 *)(p + 4);
-    if constexpr (KS > 0) {
-        f32x4 pl[KS], ph[KS];
+    f32x4 pl[KS], ph[KS];
 #pragma unroll
-        for (int k = 1; k < KS; ++k) {
-            pl[k] = *(const f32x4 *)(p + k * n);
-            ph[k] = *(const f32x4 *)(p + k * n + 4);
-        }
-#pragma unroll
-        for (int k = 1; k < KS; ++k) { lo += pl[k]; hi += ph[k]; }
-    } else {
-        for (int k = 1; k < ks; ++k) {
-            lo += *(const f32x4 *)(p + k * n);
-            hi += *(const f32x4 *)(p + k * n + 4);
-        }
+    for (int k = 1; k < KS; ++k) {
+        pl[k] = *(const f32x4 *)(p + k * n);
+        ph[k] = *(const f32x4 *)(p + k * n + 4);
     }
+#pragma unroll
+    for (int k = 1; k < KS; ++k) { lo += pl[k]; hi += ph[k]; }
 }
 DEV void splitk_rows8(int T, int M, int ks, const float *__restrict__ part, void *Y, int64_t ldy, const GemmEpi &ep,
                       int64_t first, int64_t stride) {
@@ -255,10 +248,13 @@ DEV void splitk_rows8(int T, int M, int ks, const float *__restrict__ part, void
         }
         f32x4 lo, hi;
         switch (ks) {
-            case 2: slab_sum8<2>(ks, n, part + 8 * i, lo, hi); break;
-            case 4: slab_sum8<4>(ks, n, part + 8 * i, lo, hi); break;
-            case 8: slab_sum8<8>(ks, n, part + 8 * i, lo, hi); break;
-            default: slab_sum8<0>(ks, n, part + 8 * i, lo, hi); break;
+            case 2: slab_sum8<2>(n, part + 8 * i, lo, hi); break;
+            case 3: slab_sum8<3>(n, part + 8 * i, lo, hi); break;
+            case 4: slab_sum8<4>(n, part + 8 * i, lo, hi); break;
+            case 5: slab_sum8<5>(n, part + 8 * i, lo, hi); break;
+            case 6: slab_sum8<6>(n, part + 8 * i, lo, hi); break;
+            case 7: slab_sum8<7>(n, part + 8 * i, lo, hi); break;
+            default: slab_sum8<8>(n, part + 8 * i, lo, hi); break;   // dma_split: at most eight
         }
         float v[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
         if (ep.rx) affine8(v, rx8, mx8, in.s0, in.s2);
@@ -449,42 +445,62 @@ __global__ __launch_bounds__(64 * WT * WM) void gemm_kernel(int T, int N, int M,
     gemm_body<W_U8, BT, BM, WT, WM, PF, SPLIT>(T, N, M, A, lda, Wv, ldw, Y, ldy, ep, nk_split, part);
 }
 
-// ---- uint8 weights, large products: operands go from global memory straight into LDS ------------------------
-// 256 x 256 tile, 8 waves (2 x 4, each 128 x 64), three LDS stages of one 64-deep k-tile each.  The loads are
-// global_load_lds_dwordx4: one wave instruction copies 64 x 16 B into 1 KB of LDS without passing through
-// registers, so no wave spends issue slots on ds_write or on holding prefetched tiles.  The weight tile stays
-// uint8 in LDS (half the bytes of fp16) and becomes fp16 in the B fragments on the way to the matrix cores.
-// LDS layout of a stage: A tile [256 rows][8 chunks of 16 B], chunk c of row r at slot c ^ ((r >> 1) & 7);
-// W tile [256 rows][4 chunks of 16 B], chunk c of row r at slot c ^ ((r >> 2) & 3): both make the fragment reads
-// (32 rows x one chunk per half-wave) hit every bank once.  The swizzle is applied on the global side: the lane
-// that fills slot p of row r loads chunk p ^ key(r).
-// Schedule of one k-tile: fragments of step ks + 1 are read while step ks multiplies (registers double-buffered);
-// after the third of four steps every wave waits for its own loads of the next tile and meets the others at the
-// one barrier, then issues the loads of tile kt + 3 into the stage it has just finished and reads the first
-// fragments of tile kt + 1 while the fourth step multiplies.  LDS reads are inline asm with hand-placed
-// s_waitcnt: the compiler waits for lgkmcnt(0) wherever older and newer reads are both outstanding.
-// fp16 weights (W_U8 = false): the weight tile is laid out like the A tile (32 KB), a stage is 64 KB and two fit, so
-// one tile is in flight while one multiplies.
-// Tile TM x TN is 256 x 256 (wave tile 128 x 64: the long, wide products), 128 x 128 (wave tile 64 x 32, a stage of
-// 24 KB: products with too few 256 x 256 tiles for the chip run at full depth with these instead of splitting K) or
-// 64 x 128 (four waves of 64 x 32, a stage of 16 KB: calls of up to 64 rows, which are HBM bound -- with 128 rows two
-// thirds of the bytes in flight were copies of the last row).  NSTG: stages, 0 = the default above.
-// Measured (uint8, us, scaling pass included): four stages instead of three on the 128 x 128 tile [256 x 4096] x
-// [4096 x 12288] 46.0 -> 40.2, [256 x 4096] x [4096 x 4096] at full depth 45.6 -> 37.4, with one tile for every CU [1024 x
-// 4096] x [4096 x 4096] 51.2 -> 48.5 and [256 x 4096] x [4096 x 16384] 51.2 -> 46.7; 5 % slower where the tiles take several rounds, as only one workgroup then fits a CU.  64 x 128 tile at
-// 64 rows: [4096 x 12288] 29.5 -> 24.4, [4096 x 20480] 44.1 -> 35.3, [16384 x 4096] 34.6 -> 29.1, [4096 x 4096] 19.1 -> 17.5.
-// Not faster on the 128 x 128 tile: four waves of 64 x 64 (45.0 against 41.7 us on [1024 x 4096] x [4096 x 4096]), and
-// eight waves of 64 x 64 that halve K between them (40 % fewer fragment reads: 48.1 against 50.0, several rounds slower).
+// ---- operands straight from global memory into LDS ------------------------------------------------------------
+// Tiles of 64 to 256 rows and 128 to 256 columns, eight waves (2 x 4; the 64-row tile four, 1 x 4), stages of one 64-deep k-tile.
+// The loads are global_load_lds_dwordx4: one wave instruction copies 64 x 16 B into 1 KB of LDS without passing through
+// registers, so no wave spends issue slots on ds_write or on holding prefetched tiles.  A uint8 weight tile stays
+// uint8 in LDS (half the bytes of fp16) and becomes fp16 in the fragments on the way to the matrix cores.
+// The MFMA is v_mfma_f32_16x16x32_f16.  A chip full of large tiles is bound by its clock under load, and this one does more for
+// the power: loops of nothing but MFMAs on random operands sustain 1870 TFLOP/s with it and 1600 with v_mfma_f32_32x32x16_f16
+// (whose accumulator it reads and writes half as often per product).  [1024 x 4096] x [4096 x 16384] 126 -> 115 us (uint8), 133 ->
+// 119 (fp16).  It also makes sides that are any multiple of 32, see tile_price.
+// LDS layout of a stage: 128-byte rows [row][8 chunks of 16 B], chunk c of row r at slot c ^ ((r >> 1) & 7); uint8 weight rows
+// [row][4 chunks of 16 B], chunk c of row r at slot c ^ ((r >> 2) & 3): the fragment reads (16 rows x one chunk per 16 lanes) hit every
+// bank once.  The swizzle is applied on the global side: the lane that fills slot p of row r loads chunk p ^ key(r).
+// LDS reads are inline asm with hand-placed s_waitcnt: the compiler waits for lgkmcnt(0) wherever older and newer reads are
+// both outstanding.
+// Schedules of a k-tile, two MFMA steps of 32 k's; its one barrier stands where the reads of the tile are back and the next tile has
+// landed:
+//   HS = 2     (more than 64 rows a wave) each step in two halves of the row blocks.  A half's activation fragments are read two halves
+//              ahead, the uint8 fragments of a step widened behind the MFMAs of the one before; the barrier follows the second half,
+//              and with three stages the loads of tile kt + 2 are issued in three parts between the halves.
+//   HS = 1     (64 rows a wave) a step's fragments are read while the other step multiplies; the barrier follows the first step, and
+//              the loads of the tile NST ahead go into the stage that has just been read.
+//   KG = 2     (128 x 128 with four stages, one workgroup to a CU) the waves are two groups of 2 x 2, group g takes step g: 64 x 64 a
+//              wave instead of 64 x 32, two fifths fewer fragment bytes; all fragments of a tile are read while the one before
+//              multiplies.  us, one step after the other / two groups / as HS = 1: uint8 [256 x 4096] x [4096 x 12288] 38.8 / 37.5 /
+//              40.4, [1024 x 4096] x [4096 x 4096] 40.7 / 39.5 / 41.8; fp16 [333 x 2048] x [2048 x 8192] 21.6 / 21.5 / 23.5.
+// What a launch of one 256 x 256 tile per CU spends outside its k-tiles, by time stamps (us, uint8, 1024 rows, 115 in all): 4 until the
+// first wave and after the last, 2.5 until the first tile is there, 3 until the outputs are in LDS, 7 until they have left (32 MB at once).
+// Four stages instead of three on the 128 x 128 tile [256 x 4096] x [4096 x 12288] 46.0 -> 40.2 us; slower where the tiles take
+// several rounds, as only one workgroup then fits a CU.
 template <bool W_U8, int TM, int TN, int NW = 8, int NSTG = 0> struct DmaCfg {
     static constexpr int A = TM * BK * 2, W = W_U8 ? TN * BK : TN * BK * 2, STAGE = A + W;
-    static constexpr int NST = NSTG ? NSTG : (W_U8 || TM < 256) ? 3 : 2;
-    static constexpr int AL = A / 1024 / NW, WL = W / 1024 / NW, LOADS = AL + WL;   // 1 KB loads per wave and tile
-    static constexpr int WR = TM >= 128 ? 2 : 1, WC = NW / WR;           // waves: 2 rows x 4 columns; 64-row tile: 1 x 4
-    static constexpr int MI = TM / (32 * WR), NI = TN / (32 * WC);       // 32 x 32 blocks per wave
-    static constexpr int STG_STRIDE = TN + 8;   // epilogue staging: 128 rows of TN floats, padded (see the epilogue)
-    static constexpr size_t BODY = (size_t)NST * STAGE > (size_t)128 * STG_STRIDE * 4 ? (size_t)NST * STAGE : (size_t)128 * STG_STRIDE * 4;
-    static constexpr size_t LDS = BODY + (W_U8 ? 2 * TM * 4 : 0);   // past the stages: the tile rows' sums s0, s2 (GemmEpi::parts)
+    static constexpr int NST = NSTG ? NSTG : 3 * STAGE + (W_U8 ? 2 * TM * 4 + 2 * TN * 2 : 0) <= 160 * 1024 ? 3 : 2;
+    static constexpr int AP = A / 1024, WP = W / 1024;                                        // 1 KB loads of a stage
+    static constexpr int AL = (AP + NW - 1) / NW, WL = (WP + NW - 1) / NW, LOADS = AL + WL;   // per wave; past the end the last one again
+    static constexpr int KG = TM == 128 && NST == 4 ? 2 : 1;                                  // groups of waves that share K
+    static constexpr int WR = TM >= 128 ? 2 : 1, WC = NW / WR / KG;                           // waves: 2 rows x 4 columns; 64-row tile: 1 x 4
+    static constexpr int MI = TM / (16 * WR), NI = TN / (16 * WC);                            // 16 x 16 blocks per wave
+    static constexpr int HS = MI > 4 ? 2 : 1, H0 = HS == 2 ? (MI + 1) / 2 : MI;               // row blocks in one or two halves
+    static constexpr int STG_STRIDE = TN + 4;   // epilogue staging, floats: 16 bytes apart, so 16 rows fill all banks
+    static constexpr int HSTRIDE = TN + 8;      // the same for fp16 outputs
+    static constexpr int FROWS = TM > 128 ? TM / 2 : TM;                                      // rows of a pass of the former
+    static constexpr int CPR = TN == 192 ? 32 : TN / 8;                                       // threads that finish a row, eight outputs each
+    static constexpr size_t max3(size_t a, size_t b, size_t c) { return a > b ? (a > c ? a : c) : (b > c ? b : c); }
+    static constexpr size_t BODY = max3((size_t)NST * STAGE, (size_t)KG * FROWS * STG_STRIDE * 4, (size_t)TM * HSTRIDE * 2);
+    static constexpr size_t LDS = BODY + (W_U8 ? 2 * TM * 4 + 2 * TN * 2 : 0);   // uint8: past the stages the rows' sums s0, s2 and the columns' rx, mx
+    static_assert(TM % (16 * WR) == 0 && TN % (16 * WC) == 0 && MI <= 8 && NI <= 4 && H0 <= 4 && 2 * TM <= 64 * NW, "waves");
+    static_assert((NST - 1) * LOADS < 64 && LDS <= 160 * 1024 && (TN == 64 || TN == 128 || TN == 192 || TN == 256), "tile");
 };
+DEV void emit_parts(const GemmEpi &ep, int t, int m0, int M, int TN, float a0, float a2) {
+    const int parts = emitted_parts(M, TN), i = m0 / TN;
+    float *p0 = ep.emit_s0 + (size_t)t * parts, *p2 = ep.emit_s2 + (size_t)t * parts;
+    p0[i] = a0;
+    p2[i] = a2;
+    if (m0 + TN >= M)
+        for (int j = i + 1; j < parts; ++j) p0[j] = p2[j] = 0.f;
+}
 // This workgroup's tile: the hardware deals consecutive workgroup ids round-robin to the 8 XCDs; undone here, so that
 // each XCD gets a contiguous range of tiles (those walk the T direction first, and share weight tiles in its L2).
 DEV int xcd_tile() {
@@ -507,37 +523,37 @@ constexpr int vm_only(int n) { return 0x0F70 | (n & 15) | ((n >> 4) << 14); }
 constexpr int vm_lgkm0(int n) { return 0x0070 | (n & 15) | ((n >> 4) << 14); }
 constexpr int lgkm_only(int n) { return 0xC07F | (n << 8); }
 
-// FOURS: outputs leave four at a time (1), eight (0), or as by_four says (-1)
-template <bool W_U8, bool SPLIT, int TM, int TN, int NW, int NSTG, int FOURS>
+template <bool W_U8, bool SPLIT, int TM, int TN, int NW, int NSTG>
 DEV void gemm_dma_body(int bid, int T, int N, int M, const h16 *__restrict__ A, int64_t lda, const void *__restrict__ Wv,
                        int64_t ldw, void *__restrict__ Y, int64_t ldy, const GemmEpi &ep, int nk_split,
                        float *__restrict__ part, int split) {
     using Cfg = DmaCfg<W_U8, TM, TN, NW, NSTG>;
     constexpr int D_A = Cfg::A, D_STAGE = Cfg::STAGE, D_NST = Cfg::NST, AL = Cfg::AL, WL = Cfg::WL, MI = Cfg::MI, NI = Cfg::NI;
-    static_assert((TM == 256 || TM == 128 || TM == 64) && (TN == 256 || TN == 128), "tile");
-    static_assert((NW == 8 || NW == 4) && 2 * TM <= 64 * NW && MI >= 2 && MI <= 4 && NI >= 1 && NI <= 2, "waves");
+    constexpr int HS = Cfg::HS, H0 = Cfg::H0, KG = Cfg::KG;
     extern __shared__ __align__(1024) unsigned char smem[];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wr = wave / Cfg::WC, wc = wave % Cfg::WC;
+    const int grp = wave / (Cfg::WR * Cfg::WC), wr = wave / Cfg::WC % Cfg::WR, wc = wave % Cfg::WC;
     const TileAt at = tile_at<TM, TN>(bid, T, M, ep.walk_m);
     const int t0 = at.t0, m0 = at.m0;
     const int kbase = SPLIT ? split * nk_split : 0, nk = SPLIT ? nk_split : N / BK;
 
     // load sources; rows past the end re-read the last row (never stored)
+    auto a_piece = [&](int i) { return min(wave * AL + i, Cfg::AP - 1); };
+    auto w_piece = [&](int i) { return min(wave * WL + i, Cfg::WP - 1); };
     const h16 *ga[AL];
 #pragma unroll
     for (int i = 0; i < AL; ++i) {
-        const int r = (wave * AL + i) * 8 + (lane >> 3), c = (lane & 7) ^ ((r >> 1) & 7);
+        const int r = a_piece(i) * 8 + (lane >> 3), c = (lane & 7) ^ ((r >> 1) & 7);
         ga[i] = A + (size_t)min(t0 + r, T - 1) * lda + (size_t)kbase * BK + c * 8;
     }
     const unsigned char *gw[WL];   // byte pointers
 #pragma unroll
     for (int i = 0; i < WL; ++i) {
         if (W_U8) {
-            const int r = (wave * WL + i) * 16 + (lane >> 2), c = (lane & 3) ^ ((r >> 2) & 3);
+            const int r = w_piece(i) * 16 + (lane >> 2), c = (lane & 3) ^ ((r >> 2) & 3);
             gw[i] = (const unsigned char *)Wv + (size_t)min(m0 + r, M - 1) * ldw + (size_t)kbase * BK + c * 16;
         } else {
-            const int r = (wave * WL + i) * 8 + (lane >> 3), c = (lane & 7) ^ ((r >> 1) & 7);
+            const int r = w_piece(i) * 8 + (lane >> 3), c = (lane & 7) ^ ((r >> 1) & 7);
             gw[i] = (const unsigned char *)((const h16 *)Wv + (size_t)min(m0 + r, M - 1) * ldw + (size_t)kbase * BK + c * 8);
         }
     }
@@ -549,72 +565,86 @@ DEV void gemm_dma_body(int bid, int T, int N, int M, const h16 *__restrict__ A, 
 #pragma unroll
         for (int i = 0; i < AL; ++i)
             if (part < 0 || part == (i >= (AL + 1) / 2 ? 1 : 0))
-                __builtin_amdgcn_global_load_lds((gptr)(ga[i] + kt * BK), (lptr)(base + (wave * AL + i) * 1024), 16, 0, 0);
+                __builtin_amdgcn_global_load_lds((gptr)(ga[i] + kt * BK), (lptr)(base + a_piece(i) * 1024), 16, 0, 0);
         if (part < 0 || part == 2) {
 #pragma unroll
             for (int i = 0; i < WL; ++i)
-                __builtin_amdgcn_global_load_lds((gptr)(gw[i] + kt * BK * (W_U8 ? 1 : 2)), (lptr)(base + D_A + (wave * WL + i) * 1024), 16, 0, 0);
+                __builtin_amdgcn_global_load_lds((gptr)(gw[i] + kt * BK * (W_U8 ? 1 : 2)), (lptr)(base + D_A + w_piece(i) * 1024), 16, 0, 0);
         }
     };
 
-    f32x16 acc[MI][NI];
+    f32x4 acc[MI][NI];
 #pragma unroll
     for (int a = 0; a < MI; ++a)
 #pragma unroll
-        for (int b = 0; b < NI; ++b)
-#pragma unroll
-            for (int e = 0; e < 16; ++e) acc[a][b][e] = 0.f;
+        for (int b = 0; b < NI; ++b) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-    // fragment addresses within a stage; the swizzle keys depend on the lane only
+    // Fragments: lane (row, q) takes the k's 16 q + 8 s .. + 7 of the k-tile in MFMA step s, for both operands, so that a uint8
+    // weight fragment of both steps is one 16-byte read.  Two groups: group g takes the k's 32 g + 8 q .. + 7.
+    // Addresses within a stage; the swizzle keys depend on the lane only.
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)smem;
-    uint32_t vA[4], vB[4];
+    const int row = lane & 15, q = lane >> 4;
+    constexpr int STEPS = KG == 2 ? 1 : 2, WN = W_U8 ? 1 : STEPS;
+    uint32_t vA[STEPS], vB[WN];
+    auto half_chunk = [&](int s) { return ((KG == 2 ? 4 * grp + q : 2 * q + s) ^ ((row >> 1) & 7)) << 4; };
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks) {
-        vA[ks] = lds0 + (wr * 32 * MI + (lane & 31)) * 128 + (((2 * ks + (lane >> 5)) ^ ((lane >> 1) & 7)) << 4);
-        if (W_U8) vB[ks] = lds0 + D_A + (wc * 32 * NI + (lane & 31)) * 64 + ((ks ^ ((lane >> 2) & 3)) << 4) + (lane >> 5) * 8;
-        else vB[ks] = lds0 + D_A + (wc * 32 * NI + (lane & 31)) * 128 + (((2 * ks + (lane >> 5)) ^ ((lane >> 1) & 7)) << 4);
-    }
-    h16x8 fa[2][MI], fbh[2][NI];   // fbh: B fragments of fp16 weights
-    u32x2 rawb[2][NI];             // B fragments of uint8 weights, before conversion
-    auto ldfrag = [&](int buf, int so, int ks) {
-        const uint32_t pa = vA[ks] + so, pb = vB[ks] + so;
-        if constexpr (W_U8) {
-            asm volatile("ds_read_b64 %0, %1" : "=v"(rawb[buf][0]) : "v"(pb));
-            if constexpr (NI > 1) asm volatile("ds_read_b64 %0, %1 offset:2048" : "=v"(rawb[buf][NI > 1 ? 1 : 0]) : "v"(pb));
-        } else {
-            asm volatile("ds_read_b128 %0, %1" : "=v"(fbh[buf][0]) : "v"(pb));
-            if constexpr (NI > 1) asm volatile("ds_read_b128 %0, %1 offset:4096" : "=v"(fbh[buf][NI > 1 ? 1 : 0]) : "v"(pb));
+    for (int s = 0; s < STEPS; ++s) vA[s] = lds0 + (wr * 16 * MI + row) * 128 + half_chunk(s);
+#pragma unroll
+    for (int s = 0; s < WN; ++s)
+        vB[s] = lds0 + D_A + (!W_U8 ? (wc * 16 * NI + row) * 128 + half_chunk(s)
+                              : (wc * 16 * NI + row) * 64 + (((KG == 2 ? 2 * grp + (q >> 1) : q) ^ ((row >> 2) & 3)) << 4) + (KG == 2 ? (q & 1) * 8 : 0));
+    h16x8 fa[2][H0];                             // [set][row block]
+    u32x4 rawb[NI];                              // uint8 weights, both steps of a k-tile
+    u32x2 rawg[2][NI];                           // the same with two groups: [set]
+    h16x8 fb[2][NI];                             // [step], two groups: [set]
+    auto ld_a = [&](int set, int so, int s, int half) {
+        const uint32_t p = vA[s] + so;
+#pragma unroll
+        for (int i = 0; i < H0; ++i)
+            if (half * H0 + i < MI) asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(fa[set][i]) : "v"(p), "n"((half * H0 + i) * 2048));
+    };
+    auto ld_w = [&](int so, int s) {   // uint8: both steps, whatever s is
+        const uint32_t p = vB[W_U8 ? 0 : s] + so;
+#pragma unroll
+        for (int i = 0; i < NI; ++i) {
+            if constexpr (W_U8) asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(rawb[i]) : "v"(p), "n"(i * 1024));
+            else asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(fb[s][i]) : "v"(p), "n"(i * 2048));
         }
-        asm volatile("ds_read_b128 %0, %1" : "=v"(fa[buf][0]) : "v"(pa));
-        asm volatile("ds_read_b128 %0, %1 offset:4096" : "=v"(fa[buf][1]) : "v"(pa));
-        if constexpr (MI > 2) {
-            asm volatile("ds_read_b128 %0, %1 offset:8192" : "=v"(fa[buf][MI > 2 ? 2 : 0]) : "v"(pa));
-            asm volatile("ds_read_b128 %0, %1 offset:12288" : "=v"(fa[buf][MI > 2 ? 3 : 0]) : "v"(pa));
+    };
+    auto ld_group = [&](int set, int so) {
+        const uint32_t p = vB[0] + so;
+#pragma unroll
+        for (int i = 0; i < NI; ++i) {
+            if constexpr (W_U8) asm volatile("ds_read_b64 %0, %1 offset:%2" : "=v"(rawg[set][i]) : "v"(p), "n"(i * 1024));
+            else asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(fb[set][i]) : "v"(p), "n"(i * 2048));
         }
+        ld_a(set, so, 0, 0);
     };
     const h16x2 off = {(h16)1023.5f, (h16)1023.5f};
-    // waits until only the newest fragment set (MI + NI reads) of this wave is outstanding: the one before has returned
-    auto older_reads_done = [&]() {
-        __builtin_amdgcn_s_waitcnt(lgkm_only(MI + NI));
+    auto widen8 = [&](uint32_t x, uint32_t y) {
+        const h16x2 q0 = u8pair_lo_1024(x) - off, q1 = u8pair_hi_1024(x) - off, q2 = u8pair_lo_1024(y) - off, q3 = u8pair_hi_1024(y) - off;
+        return h16x8{q0.x, q0.y, q1.x, q1.y, q2.x, q2.y, q3.x, q3.y};
+    };
+    auto widen = [&](int s) {
+        if constexpr (W_U8) {
+#pragma unroll
+            for (int i = 0; i < NI; ++i)
+                fb[s][i] = KG == 2 ? widen8(rawg[s][i].x, rawg[s][i].y) : widen8(s ? rawb[i].z : rawb[i].x, s ? rawb[i].w : rawb[i].y);
+        }
+    };
+    // weights first: a lane ends with four consecutive outputs of one row
+    auto mfmas = [&](int set, int s, int half) {
+#pragma unroll
+        for (int a = 0; a < H0; ++a)
+            if (half * H0 + a < MI) {
+#pragma unroll
+                for (int b = 0; b < NI; ++b)
+                    acc[half * H0 + a][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fb[s][b], fa[set][a], acc[half * H0 + a][b], 0, 0, 0);
+            }
         __builtin_amdgcn_sched_barrier(0);
     };
-    auto multiply = [&](int cur) {
-        h16x8 fb[NI];
-#pragma unroll
-        for (int b = 0; b < NI; ++b) {
-            if constexpr (W_U8) {
-                const u32x2 raw = rawb[cur][b];
-                const h16x2 q0 = u8pair_lo_1024(raw.x) - off, q1 = u8pair_hi_1024(raw.x) - off;
-                const h16x2 q2 = u8pair_lo_1024(raw.y) - off, q3 = u8pair_hi_1024(raw.y) - off;
-                fb[b] = h16x8{q0.x, q0.y, q1.x, q1.y, q2.x, q2.y, q3.x, q3.y};
-            } else {
-                fb[b] = fbh[cur][b];
-            }
-        }
-#pragma unroll
-        for (int a = 0; a < MI; ++a)
-#pragma unroll
-            for (int b = 0; b < NI; ++b) acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fa[cur][a], fb[b], acc[a][b], 0, 0, 0);
+    auto reads_done = [&]() {
+        __builtin_amdgcn_s_waitcnt(lgkm_only(0));
         __builtin_amdgcn_sched_barrier(0);
     };
 
@@ -624,22 +654,40 @@ DEV void gemm_dma_body(int bid, int T, int N, int M, const h16 *__restrict__ A, 
     // issued in three parts between the MFMA steps, into the stage tile kt - 1 was read from (a burst of all of
     // them right after the barrier measured 2 % slower).  Two stages: tile kt + 2 can only go where tile kt is, so
     // its loads follow the barrier in one go.
-    constexpr bool SPREAD = D_NST >= 3;
-    constexpr int PD = SPREAD ? D_NST - 1 : 2;   // tiles in flight ahead of the one being multiplied
+    constexpr bool SPREAD = HS == 2 && D_NST >= 3;
+    constexpr int PD = HS == 1 ? D_NST : SPREAD ? D_NST - 1 : 2;   // tiles in flight ahead of the one being multiplied
+    // What the epilogue reads of the uint8 format is put into LDS while the first tiles are in flight: a row's sums and a column's
+    // rx and mx, requested ahead of the tiles.
+    float *const lsum = (float *)(smem + Cfg::BODY);
+    h16 *const lcol = (h16 *)(lsum + 2 * TM);
+    const bool parts = W_U8 && ep.parts > 1;
+    float sum1 = 0.f;
+    h16x4 col4 = {};
+    if constexpr (W_U8 && !SPLIT) {
+        if (tid < TN / 2) {
+            const int c = tid % (TN / 4) * 4;
+            if (m0 + c < M) col4 = load_n<h16x4, 4>((tid < TN / 4 ? ep.rx : ep.mx) + m0 + c, M - m0 - c);
+        }
+        if (!parts && tid < 2 * TM) sum1 = (tid < TM ? ep.s0 : ep.s2)[min(t0 + tid % TM, T - 1)];
+        __builtin_amdgcn_sched_barrier(0);
+    }
     issue(0, 0, -1);
     issue(min(1, nk - 1), D_STAGE, -1);
 #pragma unroll
     for (int p = 2; p < PD; ++p) issue(min(p, nk - 1), p * D_STAGE, -1);
+    if constexpr (W_U8 && !SPLIT) {
+        __builtin_amdgcn_sched_barrier(0);
+        if (tid < TN / 2) *(h16x4 *)(lcol + tid * 4) = col4;
+        if (!parts && tid < 2 * TM) lsum[tid] = sum1;
+    }
     // The input's row sums arrive as partial sums per column tile of the launch that produced it: this tile's rows
     // are added up here, in index order, while the first two tiles are in flight (the waits for these loads cover the
     // older tile loads too, so the counted waits below still hold).  Full depth: into LDS for the epilogue;
     // K split: the first column tile's first split writes the totals out for the second pass.
-    bool lds_sums = false;
     if constexpr (W_U8) {
-        if (ep.parts > 1 && (!SPLIT || (m0 == 0 && split == 0))) {
-            lds_sums = !SPLIT;
+        if (parts && (!SPLIT || (m0 == 0 && split == 0))) {
             if (tid < 2 * TM) {
-                const int row = tid & (TM - 1), which = tid / TM, t = min(t0 + row, T - 1);
+                const int row = tid % TM, which = tid / TM, t = min(t0 + row, T - 1);
                 const float *p = (which ? ep.p2 : ep.p0) + (size_t)t * ep.parts;
                 float tot = 0.f;
                 for (int j = 0; j < ep.parts; j += 64) {   // parts % 4 == 0; up to 64 partial sums in flight per thread
@@ -652,7 +700,7 @@ DEV void gemm_dma_body(int bid, int T, int N, int M, const h16 *__restrict__ A, 
                 if constexpr (SPLIT) {
                     if (t0 + row < T) (which ? (float *)ep.s2 : (float *)ep.s0)[t] = tot;
                 } else {
-                    ((float *)(smem + Cfg::BODY))[tid] = tot;
+                    lsum[tid] = tot;
                 }
             }
         }
@@ -660,109 +708,90 @@ DEV void gemm_dma_body(int bid, int T, int N, int M, const h16 *__restrict__ A, 
     __builtin_amdgcn_s_waitcnt(vm_only((PD - 1) * Cfg::LOADS));   // tile 0 has landed
     __builtin_amdgcn_s_barrier();
     int so = 0, sp = (D_NST - 1) * D_STAGE;   // the stage being read and (three stages and more) the one read before it
-    // Second schedule (uint8 weights, and the large tile with fp16 weights; measured: [1024 x 4096] x [4096 x 4096]
-    // uint8 57 -> 50 us, the large tile 1-4 % faster, the small tile with fp16 weights 10-15 % slower):
-    // fragments are read TWO steps ahead of their MFMAs and the uint8 -> fp16 widening of step s + 1 is issued
-    // right after the MFMAs of step s, so it runs while the matrix core works instead of between a fragment's
-    // arrival and its MFMAs.  Step s uses register set s & 1 and refills it with step s + 2 once its MFMAs are
-    // issued; all reads of a tile are therefore issued by its second step, where the one barrier per tile sits:
-    // past it tile kt + 1 has landed for every wave and nobody reads tile kt's stage any more.
-    constexpr bool AHEAD = W_U8 || TM == 256;
-    if constexpr (AHEAD) {
-        h16x8 fbc[2][NI];              // widened B fragments
-        auto widen = [&](int buf) {
-#pragma unroll
-            for (int b = 0; b < NI; ++b) {
-                if constexpr (W_U8) {
-                    const u32x2 raw = rawb[buf][b];
-                    const h16x2 q0 = u8pair_lo_1024(raw.x) - off, q1 = u8pair_hi_1024(raw.x) - off;
-                    const h16x2 q2 = u8pair_lo_1024(raw.y) - off, q3 = u8pair_hi_1024(raw.y) - off;
-                    fbc[buf][b] = h16x8{q0.x, q0.y, q1.x, q1.y, q2.x, q2.y, q3.x, q3.y};
-                } else {
-                    fbc[buf][b] = fbh[buf][b];
-                }
-            }
-        };
-        auto mfmas = [&](int buf) {
-#pragma unroll
-            for (int a = 0; a < MI; ++a)
-#pragma unroll
-                for (int b = 0; b < NI; ++b) acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fa[buf][a], fbc[buf][b], acc[a][b], 0, 0, 0);
-            __builtin_amdgcn_sched_barrier(0);
-        };
-        auto reads_done = [&]() {
-            __builtin_amdgcn_s_waitcnt(lgkm_only(0));
-            __builtin_amdgcn_sched_barrier(0);
-        };
-        ldfrag(0, 0, 0);
-        ldfrag(1, 0, 1);
-        older_reads_done();
+    if constexpr (KG == 1) {
+        ld_a(0, 0, 0, 0);
+        ld_w(0, 0);
+        ld_a(1, 0, HS == 1, HS == 2);
+        if (!W_U8 && HS == 1) ld_w(0, 1);
+        reads_done();
         widen(0);
+    } else {
+        ld_group(0, 0);
+        reads_done();
+    }
+    if constexpr (KG == 2) {
+        // all fragments of a k-tile are read while the one before multiplies
+        auto tile = [&](int kt, int set) {
+            const int sn = so + D_STAGE >= D_NST * D_STAGE ? 0 : so + D_STAGE;
+            __builtin_amdgcn_s_waitcnt(vm_only((D_NST - 2) * Cfg::LOADS));   // my part of tile kt + 1 has landed
+            __builtin_amdgcn_s_barrier();
+            __builtin_amdgcn_sched_barrier(0);
+            ld_group(set ^ 1, sn);
+            issue(min(kt + PD, nk - 1), so, -1);
+            widen(set);
+            mfmas(set, set, 0);
+            reads_done();
+            so = sn;
+        };
+        int kt = 0;
+        for (; kt + 1 < nk; kt += 2) {
+            tile(kt, 0);
+            tile(kt + 1, 1);
+        }
+        if (kt < nk) tile(kt, 0);
+    } else if constexpr (HS == 2) {
         for (int kt = 0; kt < nk; ++kt) {
             const int sn = so + D_STAGE >= D_NST * D_STAGE ? 0 : so + D_STAGE;
             const int kl = min(kt + PD, nk - 1);
-            // step 0
-            mfmas(0);
+            mfmas(0, 0, 0);
             reads_done();
             widen(1);
-            ldfrag(0, so, 2);
+            ld_a(0, so, 1, 0);
+            if (!W_U8) ld_w(so, 1);
             if (SPREAD) issue(kl, sp, 0);
             __builtin_amdgcn_sched_barrier(0);
-            // step 1
-            mfmas(1);
+            mfmas(1, 0, 1);
             reads_done();
-            widen(0);
-            ldfrag(1, so, 3);
+            ld_a(1, so, 1, 1);
             if (SPREAD) issue(kl, sp, 1);
             __builtin_amdgcn_sched_barrier(0);
             // my part of tile kt + 1 has landed (newer: the A loads of tile kt + 2) and all my reads of tile kt are back
             __builtin_amdgcn_s_waitcnt(vm_lgkm0(SPREAD ? (PD - 2) * Cfg::LOADS + AL : 0));
             __builtin_amdgcn_s_barrier();
             if (!SPREAD) issue(kl, so, -1);
-            // step 2
-            mfmas(0);
-            widen(1);
-            ldfrag(0, sn, 0);
+            mfmas(0, 1, 0);
+            ld_a(0, sn, 0, 0);
+            ld_w(sn, 0);
             if (SPREAD) issue(kl, sp, 2);
             __builtin_amdgcn_sched_barrier(0);
-            // step 3
-            mfmas(1);
+            mfmas(1, 1, 1);
             reads_done();
             widen(0);
-            ldfrag(1, sn, 1);
+            ld_a(1, sn, 0, 1);
             __builtin_amdgcn_sched_barrier(0);
             sp = so;
             so = sn;
         }
     } else {
-        ldfrag(0, 0, 0);
         for (int kt = 0; kt < nk; ++kt) {
             const int sn = so + D_STAGE >= D_NST * D_STAGE ? 0 : so + D_STAGE;
             const int kl = min(kt + PD, nk - 1);
-            ldfrag(1, so, 1);
-            if (SPREAD) issue(kl, sp, 0);
-            __builtin_amdgcn_sched_barrier(0);
-            older_reads_done();
-            multiply(0);
-            ldfrag(0, so, 2);
-            if (SPREAD) issue(kl, sp, 1);
-            __builtin_amdgcn_sched_barrier(0);
-            older_reads_done();
-            multiply(1);
-            ldfrag(1, so, 3);
-            if (SPREAD) issue(kl, sp, 2);
-            __builtin_amdgcn_sched_barrier(0);
-            older_reads_done();
-            multiply(0);
-            // all my reads of this stage have returned and my part of tile kt + 1 has landed (with three stages tile
-            // kt + 2 is in flight)
-            __builtin_amdgcn_s_waitcnt(vm_lgkm0(SPREAD ? (PD - 1) * Cfg::LOADS : 0));
+            mfmas(0, 0, 0);
+            widen(1);
+            // my part of tile kt + 1 has landed and all my reads of tile kt are back
+            __builtin_amdgcn_s_waitcnt(vm_lgkm0((D_NST - 2) * Cfg::LOADS));
             __builtin_amdgcn_s_barrier();
-            if (!SPREAD) issue(kl, so, -1);
-            ldfrag(0, sn, 0);
             __builtin_amdgcn_sched_barrier(0);
-            multiply(1);
-            sp = so;
+            issue(kl, so, -1);
+            ld_a(0, sn, 0, 0);
+            ld_w(sn, 0);
+            __builtin_amdgcn_sched_barrier(0);
+            mfmas(1, 1, 0);
+            reads_done();
+            widen(0);
+            ld_a(1, sn, 1, 0);
+            if (!W_U8) ld_w(sn, 1);
+            __builtin_amdgcn_sched_barrier(0);
             so = sn;
         }
     }
@@ -776,148 +805,198 @@ DEV void gemm_dma_body(int bid, int T, int N, int M, const h16 *__restrict__ A, 
     __builtin_amdgcn_s_waitcnt(0x0070);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int buf = 0; buf < 2; ++buf) {
+    for (int set = 0; set < 2; ++set)
 #pragma unroll
-        for (int a = 0; a < MI; ++a) asm volatile("" ::"v"(fa[buf][a]));
+        for (int a = 0; a < H0; ++a)
+            if (set * H0 + a < MI || HS == 1) asm volatile("" ::"v"(fa[set][a]));
 #pragma unroll
-        for (int b = 0; b < NI; ++b) {
-            if constexpr (W_U8) asm volatile("" ::"v"(rawb[buf][b]));
-            else asm volatile("" ::"v"(fbh[buf][b]));
-        }
+    for (int b = 0; b < NI; ++b) {
+        if constexpr (W_U8 && KG == 2) asm volatile("" ::"v"(rawg[0][b]), "v"(rawg[1][b]));
+        else if constexpr (W_U8) asm volatile("" ::"v"(rawb[b]));
+        else asm volatile("" ::"v"(fb[0][b]), "v"(fb[1][b]));
     }
     __builtin_amdgcn_sched_barrier(0);
 
-    // Each thread finishes eight consecutive outputs of one row: 16-byte loads of the residual / gate rows, 16-byte
-    // stores, and a body small enough to stay in the instruction cache (per-element code for 128 accumulators
-    // does not).
-    constexpr int CPR = TN / 8, RPI = 64 * NW / CPR;   // 8-wide chunks per tile row; rows one pass of the workgroup covers
+    constexpr int CPR = Cfg::CPR, RPI = 64 * NW / CPR;   // threads per row, rows per pass of the workgroup
     const int cq = tid % CPR, col = m0 + cq * 8;
-    const bool col_ok = col < M;
-    h16x8 rx8, mx8;
-    if (W_U8 && col_ok) { rx8 = load_n<h16x8, 8>(ep.rx + col, M - col); mx8 = load_n<h16x8, 8>(ep.mx + col, M - col); }
-    const bool emit = ep.emit_ry != nullptr;
-    const Emit8 em = emit8(ep, col, col_ok);
-    const float *lsum = (const float *)(smem + Cfg::BODY);
+    const bool in_tile = cq * 8 < TN, col_ok = in_tile && col < M;
+    constexpr int SW = Cfg::STG_STRIDE;                  // row stride of fp32 in LDS, in floats
+    float *const stg = (float *)smem;
+    constexpr int ITS = TM / RPI, AHEAD_ROWS = ITS % 4 ? 2 : 4;      // rows of a thread; rows requested together
+    static_assert(ITS % AHEAD_ROWS == 0 && TM % RPI == 0 && Cfg::FROWS % RPI == 0, "rows");
+    // the sums of a row of the tile that the CPR threads finishing it hold, neighbours in one wave: every lane takes part
+    auto emit_row = [&](int t, bool valid, float a0, float a2) {
+        a0 = row16_sum(a0);
+        a2 = row16_sum(a2);
+        if constexpr (CPR == 32) { a0 += __shfl_xor(a0, 16, WAVE); a2 += __shfl_xor(a2, 16, WAVE); }
+        if (valid && cq == 0) emit_parts(ep, t, m0, M, TN, a0, a2);
+    };
+    auto request = [&](EpiIn (&in)[AHEAD_ROWS], int it) {
+#pragma unroll
+        for (int i = 0; i < AHEAD_ROWS; ++i) {
+            const int t = t0 + (it + i) * RPI + tid / CPR;
+            in[i] = epi_in(ep, t, col, t < T && col_ok, false);
+        }
+    };
 
+    if constexpr (KG == 2) {
+        // the partial tiles of both groups meet in LDS and are added in group order
+        static_assert(TM == Cfg::FROWS && TM * SW * 8 <= (int)Cfg::BODY && ITS == AHEAD_ROWS, "two groups");
+        __syncthreads();   // every wave has read its last fragments
+#pragma unroll
+        for (int a = 0; a < MI; ++a)
+#pragma unroll
+            for (int b = 0; b < NI; ++b)
+                *(f32x4 *)(stg + (grp * TM + wr * 16 * MI + a * 16 + row) * SW + wc * 16 * NI + b * 16 + 4 * q) = acc[a][b];
+        auto sum4 = [&](int r, int c) { return *(const f32x4 *)(stg + r * SW + c) + *(const f32x4 *)(stg + (TM + r) * SW + c); };
+        if constexpr (SPLIT) {
+            __syncthreads();
+            float *slab = part + (size_t)split * T * M;
+#pragma unroll
+            for (int it = 0; it < ITS; ++it) {
+                const int r = it * RPI + tid / CPR, t = t0 + r;
+                if (t < T && col < M) *(f32x4 *)(slab + (size_t)t * M + col) = sum4(r, cq * 8);           // M % 4 == 0
+                if (t < T && col + 4 < M) *(f32x4 *)(slab + (size_t)t * M + col + 4) = sum4(r, cq * 8 + 4);
+            }
+        } else if (by_four(M, ldy, Y, ep)) {
+            __syncthreads();
+#pragma unroll 1
+            for (int it = 0; it < ITS; ++it) {
+                const int r = it * RPI + tid / CPR, t = t0 + r;
+                if (t >= T) break;
+#pragma unroll
+                for (int g = 0; g < 2; ++g) {
+                    const int c = g * (TN / 2) + cq * 4;
+                    if (m0 + c >= M) continue;
+                    f32x4 v = sum4(r, c);
+                    if constexpr (W_U8) affine4(v, m0 + c, M, lsum[r], lsum[TM + r], ep);
+                    finish_row4(v, t, m0 + c, M, ep, Y, ldy);
+                }
+            }
+        } else {
+            const Emit8 em = emit8(ep, col, col_ok);
+            EpiIn in[AHEAD_ROWS];
+            request(in, 0);
+            __syncthreads();
+#pragma unroll 1
+            for (int it = 0; it < ITS; ++it) {
+                const EpiIn cur = in[0];
+#pragma unroll
+                for (int i = 0; i + 1 < AHEAD_ROWS; ++i) in[i] = in[i + 1];   // a loop that is not unrolled has no other index
+                const int r = it * RPI + tid / CPR, t = t0 + r;
+                const bool valid = t < T && col_ok;
+                float a0 = 0.f, a2 = 0.f;
+                if (valid) {
+                    const f32x4 lo = sum4(r, cq * 8), hi = sum4(r, cq * 8 + 4);
+                    float v[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+                    if constexpr (W_U8) affine8(v, *(const h16x8 *)(lcol + cq * 8), *(const h16x8 *)(lcol + TN + cq * 8), lsum[r], lsum[TM + r]);
+                    finish_row8<true>(v, cur, t, col, ep, Y, ldy, em, a0, a2);
+                }
+                if (ep.emit_ry) emit_row(t, valid, a0, a2);
+            }
+        }
+        return;
+    }
+    const int roff = wr * 16 * MI;   // this wave's first row
     if constexpr (SPLIT) {
         // partial sums go to this split's fp32 slab; splitk_epilogue8_kernel adds the slabs and finishes
         float *slab = part + (size_t)split * T * M;
 #pragma unroll
-        for (int b = 0; b < NI; ++b) {
-            const int m = m0 + wc * 32 * NI + b * 32 + (lane & 31);
+        for (int a = 0; a < MI; ++a) {
+            const int t = t0 + roff + a * 16 + row;
 #pragma unroll
-            for (int a = 0; a < MI; ++a)
-#pragma unroll
-                for (int e = 0; e < 16; ++e) {
-                    const int t = t0 + wr * 32 * MI + a * 32 + 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3);
-                    if (m < M && t < T) slab[(size_t)t * M + m] = acc[a][b][e];
-                }
+            for (int b = 0; b < NI; ++b) {
+                const int m = m0 + wc * 16 * NI + b * 16 + 4 * q;
+                if (m < M && t < T) *(f32x4 *)(slab + (size_t)t * M + m) = acc[a][b];   // M % 4 == 0
+            }
         }
     } else {
-        // The accumulators pass through LDS (free now), 128 tile rows at a time.
-        constexpr int SW = Cfg::STG_STRIDE;   // row stride in floats: 4 rows apart = 32 banks apart for the two half-waves
-        constexpr int WROWS = 32 * MI;        // tile rows of one wave row
-        float *stg = (float *)smem;
-        // fp32 outputs, and rows that start on no 16-byte boundary, leave four at a time.  A 50277-wide head is such a
-        // product (through the register-staged kernel before): fp32 out [513 x 768] 109 -> 92 us, [1024 x 4096] 580 -> 542,
-        // uint8 weights, fp16 out 133 -> 87 and 706 -> 487.
-        const bool four = FOURS < 0 ? by_four(M, ldy, Y, ep) : FOURS == 1;
-        constexpr bool OWN_LOOP = TM < 256 || FOURS == 1;
         __syncthreads();   // every wave has read its last fragments
+        if (by_four(M, ldy, Y, ep)) {
+            // fp32 outputs, and rows that start on no 16-byte boundary, leave four at a time: the accumulators pass through LDS (free
+            // now), at most 128 tile rows at a time.  A 50277-wide head is such a product.
+            constexpr int FROWS = Cfg::FROWS;
 #pragma unroll 1
-        for (int h = 0; h < (TM + 127) / 128; ++h) {
-            if ((wr * WROWS) / 128 == h) {
-#pragma unroll
-                for (int b = 0; b < NI; ++b)
+            for (int h = 0; h < TM / FROWS; ++h) {
+                if (TM == FROWS || wr == h) {
 #pragma unroll
                     for (int a = 0; a < MI; ++a)
 #pragma unroll
-                        for (int e = 0; e < 16; ++e)
-                            stg[(wr * WROWS - h * 128 + a * 32 + 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3)) * SW + wc * 32 * NI + b * 32 + (lane & 31)] =
-                                acc[a][b][e];
-            }
-            constexpr int ITS = (TM < 128 ? TM : 128) / RPI, AHEAD_ROWS = TM == 256 ? 2 : 4;   // rows of a thread; rows requested together
-            auto fours = [&](int row, int t) {
-#pragma unroll OWN_LOOP ? 2 : 1
-                for (int g = 0; g < 2; ++g) {
-                    const int c = g * (TN / 2) + cq * 4;
-                    if (m0 + c >= M) continue;
-                    f32x4 v = *(const f32x4 *)(stg + row * SW + c);
-                    if constexpr (W_U8) {
-                        const int tr = h * 128 + row;
-                        affine4(v, m0 + c, M, lds_sums ? lsum[tr] : ep.s0[t], lds_sums ? lsum[TM + tr] : ep.s2[t], ep);
-                    }
-                    finish_row4(v, t, m0 + c, M, ep, Y, ldy);
+                        for (int b = 0; b < NI; ++b)
+                            *(f32x4 *)(stg + (roff - h * FROWS + a * 16 + row) * SW + wc * 16 * NI + b * 16 + 4 * q) = acc[a][b];
                 }
-            };
-            // A loop of their own: nothing of the other one's rows in flight is carried along.  The 256 x 256 tile has no registers
-            // for two loops (34 spilled ones: [1024 x 4096] x [4096 x 16384] 131.1 us instead of 128.6), so its single products have
-            // a kernel for either: fp32 out [256 x 1024] x [1024 x 50277] 44.8 -> 41.1 us, uint8 [1024 x 4096] x [4096 x 50277]
-            // 523 -> 501 (489 with both loops' code before rows were requested ahead).
-            if (OWN_LOOP && four) {
                 __syncthreads();
 #pragma unroll 1
-                for (int it = 0; it < ITS; ++it) {
-                    const int row = it * RPI + tid / CPR, t = t0 + h * 128 + row;
+                for (int it = 0; it < FROWS / RPI; ++it) {
+                    const int r = h * FROWS + it * RPI + tid / CPR, t = t0 + r;
                     if (t >= T) break;
-                    fours(row, t);
+#pragma unroll
+                    for (int g = 0; g < 2; ++g) {
+                        const int c = g * (TN / 2) + cq * 4;
+                        if (!in_tile || m0 + c >= M) continue;
+                        f32x4 v = *(const f32x4 *)(stg + (r - h * FROWS) * SW + c);
+                        if constexpr (W_U8) affine4(v, m0 + c, M, lsum[r], lsum[TM + r], ep);
+                        finish_row4(v, t, m0 + c, M, ep, Y, ldy);
+                    }
                 }
                 __syncthreads();
-                continue;
             }
-            EpiIn in[AHEAD_ROWS];
+            return;
+        }
+        // fp16 outputs: corrected and rounded where they are, which the other steps begin with anyway, so the whole tile fits LDS as
+        // fp16; then each thread finishes eight consecutive outputs of a row, with 16-byte loads of the residual / gate rows and
+        // 16-byte stores.  The activations stay in that loop, whose body is small enough for the instruction cache (written out for
+        // 128 accumulators they were not: 28 us of a launch of 160).
+        constexpr int HW = Cfg::HSTRIDE;                   // row stride in halves: 16 rows x 8 bytes fall on different banks
+        h16 *const hstg = (h16 *)smem;
+        h16x4 rx4[NI], mx4[NI];
+        if constexpr (W_U8) {
+#pragma unroll
+            for (int b = 0; b < NI; ++b) {
+                const int c = wc * 16 * NI + b * 16 + 4 * q;
+                rx4[b] = *(const h16x4 *)(lcol + c);
+                mx4[b] = *(const h16x4 *)(lcol + TN + c);
+            }
+        }
+#pragma unroll
+        for (int a = 0; a < MI; ++a) {
+            const int r = roff + a * 16 + row;
+            const float s0 = W_U8 ? lsum[r] : 0.f, s2 = W_U8 ? lsum[TM + r] : 0.f;
+#pragma unroll
+            for (int b = 0; b < NI; ++b) {
+                h16x4 o;
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    o[e] = (h16)(W_U8 ? epi_affine(acc[a][b][e], (float)rx4[b][e], (float)mx4[b][e], s0, s2) : acc[a][b][e]);
+                *(h16x4 *)(hstg + r * HW + wc * 16 * NI + b * 16 + 4 * q) = o;
+            }
+        }
+        const Emit8 em = emit8(ep, col, col_ok);
 #pragma unroll 1
-            for (int it = 0; it < ITS; ++it) {
-                const int row = it * RPI + tid / CPR, t = t0 + h * 128 + row;
+        for (int it = 0; it < ITS; it += AHEAD_ROWS) {
+            EpiIn in[AHEAD_ROWS];
+            request(in, it);
+            if (it == 0) __syncthreads();                  // the outputs are in LDS
+            if (t0 + it * RPI >= T) break;
+#pragma unroll
+            for (int i = 0; i < AHEAD_ROWS; ++i) {
+                const int r = (it + i) * RPI + tid / CPR, t = t0 + r;
                 const bool valid = t < T && col_ok;
-                if (it % AHEAD_ROWS == 0) {
-                    if (OWN_LOOP || !four) {
-#pragma unroll
-                        for (int i = 0; i < AHEAD_ROWS; ++i) in[i] = epi_in(ep, t + i * RPI, col, t + i * RPI < T && col_ok, W_U8 && !lds_sums);
-                    }
-                    if (it == 0) __syncthreads();   // the accumulators are in LDS
-                }
-                const EpiIn cur = in[0];
-#pragma unroll
-                for (int i = 0; i + 1 < AHEAD_ROWS; ++i) in[i] = in[i + 1];   // a loop that is not unrolled has no other index
                 float a0 = 0.f, a2 = 0.f;
-                if (!OWN_LOOP && four) {
-                    if (t < T) fours(row, t);
-                    continue;
-                }
                 if (valid) {
-                    const f32x4 v0 = *(const f32x4 *)(stg + row * SW + cq * 8), v1 = *(const f32x4 *)(stg + row * SW + cq * 8 + 4);
-                    float v[8] = {v0[0], v0[1], v0[2], v0[3], v1[0], v1[1], v1[2], v1[3]};
-                    if constexpr (W_U8) {
-                        const int tr = h * 128 + row;
-                        affine8(v, rx8, mx8, lds_sums ? lsum[tr] : cur.s0, lds_sums ? lsum[TM + tr] : cur.s2);
-                    }
-                    finish_row8<true>(v, cur, t, col, ep, Y, ldy, em, a0, a2);
+                    const h16x8 y = *(const h16x8 *)(hstg + r * HW + cq * 8);
+                    float v[8];
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) v[e] = (float)y[e];
+                    finish_row8<true>(v, in[i], t, col, ep, Y, ldy, em, a0, a2);
                 }
-                if (emit) {   // the CPR threads of a row are neighbours in one wave; every lane takes part
-                    a0 = row16_sum(a0);
-                    a2 = row16_sum(a2);
-                    if constexpr (CPR == 32) { a0 += __shfl_xor(a0, 16, WAVE); a2 += __shfl_xor(a2, 16, WAVE); }
-                    if (valid && cq == 0) {
-                        const size_t pi = (size_t)t * ((M + TN - 1) / TN) + m0 / TN;
-                        ep.emit_s0[pi] = a0;
-                        ep.emit_s2[pi] = a2;
-                    }
-                }
+                if (ep.emit_ry) emit_row(t, valid, a0, a2);
             }
-            __syncthreads();
         }
     }
 }
 
-template <bool W_U8, bool SPLIT, int TM, int TN, int NW, int NSTG, int FOURS>
-__global__ __launch_bounds__(64 * NW) void gemm_dma_kernel(int T, int N, int M, const h16 *__restrict__ A, int64_t lda,
-                                                           const void *__restrict__ W, int64_t ldw, void *__restrict__ Y,
-                                                           int64_t ldy, GemmEpi ep, int nk_split, float *__restrict__ part) {
-    gemm_dma_body<W_U8, SPLIT, TM, TN, NW, NSTG, FOURS>(xcd_tile(), T, N, M, A, lda, W, ldw, Y, ldy, ep, nk_split, part, SPLIT ? blockIdx.y : 0);
-}
-
-// Up to four contractions [T, N] x [N, M_i] in one launch: short calls, where each of them alone would split K and need
+// One to four contractions [T, N] x [N, M_i] in one launch: short calls, where each of them alone would split K and need
 // a reduction pass.  Register-staged tiles: blockIdx.y picks the member, the grid is as wide as the widest one.
 // Direct-to-LDS tiles: blockIdx.x runs over the tiles of all members, first[i] being member i's first.  (With a grid
 // for the widest member the tiles of the narrow ones all fell on the first XCDs: four first LoRA stages of 128, 128,
@@ -956,32 +1035,33 @@ int64_t group_tiles(bool w_u8, GemmGroup &g, int n, int64_t T, int64_t N, int tm
     return tiles;
 }
 
-// the same through the direct-to-LDS kernel; blockIdx.y is the k split when the group has too few tiles for the chip
+// the direct-to-LDS kernel; blockIdx.y is the K split
 template <bool W_U8, bool SPLIT, int TM, int TN, int NW, int NSTG>
-__global__ __launch_bounds__(64 * NW) void gemm_dma_group_kernel(int T, int N, GemmGroup g) {
+__global__ __launch_bounds__(64 * NW) void gemm_dma_kernel(int T, int N, GemmGroup g) {
     int tile = xcd_tile();
     const int gi = group_member(g, tile), M = g.M[gi];
-    gemm_dma_body<W_U8, SPLIT, TM, TN, NW, NSTG, -1>(tile, T, N, M, g.A[gi], g.lda, g.W[gi], g.ldw[gi], g.Y[gi], M, g.ep[gi],
+    gemm_dma_body<W_U8, SPLIT, TM, TN, NW, NSTG>(tile, T, N, M, g.A[gi], g.lda, g.W[gi], g.ldw[gi], g.Y[gi], g.ldy[gi], g.ep[gi],
                                                  SPLIT ? g.nk_split : N / BK, g.part[gi], SPLIT ? blockIdx.y : 0);
 }
 
 template <bool W_U8, int TM, int TN, int NW, int NSTG>
-int launch_dma_group(GemmGroup &g, int n, int64_t T, int64_t N, int ks, hipStream_t st) {
+int launch_dma(GemmGroup &g, int n, int64_t T, int64_t N, int ks, hipStream_t st) {
     constexpr size_t lds = DmaCfg<W_U8, TM, TN, NW, NSTG>::LDS;
     static PerDeviceOnce once;
     bool *attr_done = once.slot();
     if (!attr_done || !*attr_done) {
-        hipError_t e = hipFuncSetAttribute((const void *)gemm_dma_group_kernel<W_U8, false, TM, TN, NW, NSTG>,
+        hipError_t e = hipFuncSetAttribute((const void *)gemm_dma_kernel<W_U8, false, TM, TN, NW, NSTG>,
                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e == hipSuccess)
-            e = hipFuncSetAttribute((const void *)gemm_dma_group_kernel<W_U8, true, TM, TN, NW, NSTG>, hipFuncAttributeMaxDynamicSharedMemorySize,
+            e = hipFuncSetAttribute((const void *)gemm_dma_kernel<W_U8, true, TM, TN, NW, NSTG>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                     (int)lds);
         if (e != hipSuccess) return (int)e;
         if (attr_done) *attr_done = true;
     }
     const dim3 grid((unsigned)group_tiles(W_U8, g, n, T, N, TM, TN), (unsigned)ks);
-    if (ks > 1) hipLaunchKernelGGL((gemm_dma_group_kernel<W_U8, true, TM, TN, NW, NSTG>), grid, dim3(64 * NW), lds, st, (int)T, (int)N, g);
-    else hipLaunchKernelGGL((gemm_dma_group_kernel<W_U8, false, TM, TN, NW, NSTG>), grid, dim3(64 * NW), lds, st, (int)T, (int)N, g);
+    if (ks > 1) hipLaunchKernelGGL((gemm_dma_kernel<W_U8, true, TM, TN, NW, NSTG>), grid, dim3(64 * NW), lds, st, (int)T, (int)N, g);
+    else hipLaunchKernelGGL((gemm_dma_kernel<W_U8, false, TM, TN, NW, NSTG>), grid, dim3(64 * NW), lds, st, (int)T, (int)N, g);
+    RWKV_LAUNCH_CHECK();
     return RWKV_OK;
 }
 
@@ -1294,11 +1374,7 @@ DEV void gemm_kg_body(int bid, int T, int N, int M, const h16 *__restrict__ A, i
             if (emit) {   // the CPR threads of a row are neighbours in one wave; every lane takes part
 #pragma unroll
                 for (int o = 1; o < CPR; o <<= 1) { a0 += __shfl_xor(a0, o, WAVE); a2 += __shfl_xor(a2, o, WAVE); }
-                if (valid && cq == 0) {
-                    const size_t pi = (size_t)t * ((M + TN - 1) / TN) + m0 / TN;
-                    ep.emit_s0[pi] = a0;
-                    ep.emit_s2[pi] = a2;
-                }
+                if (valid && cq == 0) emit_parts(ep, t, m0, M, TN, a0, a2);
             }
         }
     }
@@ -1873,86 +1949,82 @@ bool dma_ok(bool w_u8, int64_t N, int64_t M, const void *A, int64_t lda, const v
     return true;
 }
 
-// The direct-to-LDS tiles: rows and columns.  TILE_S4 is TILE_S with four stages, TILE_K8 and TILE_K4 gemm_kg_kernel with
-// eight and four groups.
-enum { TILE_L, TILE_S, TILE_S4, TILE_N, TILE_K8, TILE_K4, TILES };
+// The direct-to-LDS tiles: rows and columns.  TILE_S is 128 x 128 with three stages (two workgroups fit a CU), TILE_S4 with four
+// and K over two groups, TILE_N 64 x 128 with four waves, TILE_K8 and TILE_K4 gemm_kg_kernel with eight and four groups.
+enum {
+    TILE_256x256, TILE_S, TILE_S4, TILE_N, TILE_K8, TILE_K4, TILE_256x192, TILE_224x256, TILE_224x192, TILE_192x256, TILE_192x192,
+    TILE_160x256, TILE_160x192, TILE_128x256, TILE_128x192, TILES
+};
 struct TileDim { int tm, tn; };
-constexpr TileDim tile_dim[TILES] = {{256, 256}, {128, 128}, {128, 128}, {64, 128}, {64, 64}, {64, 128}};
+constexpr TileDim tile_dim[TILES] = {{256, 256}, {128, 128}, {128, 128}, {64, 128}, {64, 64}, {64, 128}, {256, 192}, {224, 256}, {224, 192},
+                                     {192, 256}, {192, 192}, {160, 256}, {160, 192}, {128, 256}, {128, 192}};
 
-// Cost model of a direct-to-LDS launch in microseconds, fitted to launches of the 7B shapes (20 to 4096 rows):
-// `tiles` tiles of nk k-tiles split c ways run in whole rounds over the 256 CUs; a k-tile step takes 1.75 us with
-// the 256 x 256 tile, 0.573 us with the 128 x 128 one (a quarter of the work in a third of the time) and 0.327 us with
-// the 64 x 128 one; every round adds its fill, drain and epilogue (10 steps; 4.3 for a split launch, whose epilogue is
-// the reduction pass; 12.8 for the 128 x 128 tile, 5.5 where two workgroups per CU overlap; 16.5 for the 64 x 128 one, up
-// to 19.4 as its 256 threads finish up to 64 rows: with 16.5 whatever T is, products of 512 and 768 input columns and 49 to
-// 64 rows ran through it instead of the 64 x 64 tile, 5 % of such a model's call).
-// Four stages: launches of one round only (one workgroup per CU); its step grows from 0.38 us with 64 CUs busy to
-// 0.50 us with 216 and does not grow further: with 0.53 us for all of them launches of exactly 256 workgroups took the
-// three-stage tile, which is 5 to 9 % slower there (512 x 4096 x 8192 49.7 / 46.7, 1024 x 4096 x 4096 51.2 / 48.5).  fp16 weights:
-// from 0.30 us, 20 steps of fill, drain and epilogue.
-// Two of its launches cost more.  An epilogue that reads a residual or takes an exponential ends a tile by itself where a
-// split leaves it to the whole chip in the second pass: 2 us, below 32 k-tiles.  Without them the square products of models
-// of 1152 to 1792 channels ran through it at full depth instead of in two splits of the three-stage tile (6 layers, RWKV-4,
-// n_embd 1280, 777 tokens 938 -> 979 us with uint8 weights, 994 -> 1028 with fp16).  And fp16 weights, whose tiles are twice
-// the bytes, over long K: 0.50 us a step with 160 CUs busy where the last row of tiles is full, 0.42 where it is not (640 x
-// 14336 x 4096 130 us against 102 in four splits of the 256 x 256 tile, 513 rows 102 against 100).
-// The reduction pass of a split takes 2.5 us + 3.6 us per slab and 16 MB of fp32 output, at least 4.5 us.
-// A round of 256 x 256 tiles that leaves CUs idle runs at a higher clock: in short bursts 1.17 - 1.28 us a step up to 128
-// workgroups, 1.38 at 192, 1.70 at 256; within a call, whose launches keep the chip at its power limit, 1.63 at 192.  Priced as
-// a full round, the receptance / key / value group of 4096 channels (192 tiles) of a 777-row RWKV-7 call went to 2.6 rounds of
-// 128 x 128 ones, 120 us against 116 with fp16 weights; with uint8 weights and 1024 rows it belongs there (118.5 against 120.5).
-// gemm_kg_kernel: per launch, per round (split launches leave the epilogue to the second pass) and per k-tile by the CUs busy,
-// fitted to 1640 products (21 lengths, 8 widths) with the other tiles' prices as they stand: the tile it picks is 1.5 % slower
-// than the best of all on average, 4.2 % with the four tiles and prices before; 3.3 % less time.  fp16, 64 x 128 tile: the line of
-// that fit, 0.17 us a k-tile and up, was far too low: a CU takes its 24 KB in 0.32 to 0.5 us whatever the others do.  Callers
-// without scratch for a split got it for long rows and few tiles, [48 x 16384] x [16384 x 1000] 94 us, 61 with the 64 x 64 tile,
-// [64 x 4096] x [4096 x 512] 29.7 and 21.4, and those with scratch beside four stages, whose price for fp16 was too high:
-// [256 x 5120] x [5120 x 5120] 39.7 us, 35.7 with four stages, [513 x 3904] x [3904 x 2880] 35.5 and 30.4 (336 products of 24 widths: 15
-// change, all for the better).  Both tiles: 0.08 us more per k-tile
-// of what exceeds one round, of which that fit had little.  uint8, that tile and the one it is now: [1922 x 3904] x [3904 x
-// 2880] 83.7 and 67.8 us, [663 x 3584] x [3584 x 7042] 76.2 and 66.4, [45 x 2048] x [2048 x 65536] 42.7 and 37.7 (672 products
-// of 24 widths: eight change, 3 to 19 % faster each).
-// slow_epi: see slow_epilogue.
-struct CostOf { bool w_u8, slow_epi; };
-bool slow_epilogue(const GemmEpi &ep) { return ep.act == ACT_RESIDUAL || ep.act == ACT_GATED_RESIDUAL || ep.act == ACT_SIGMOID; }
-double dma_cost(CostOf of, int tile, int64_t T, int64_t tiles, int nk, int c, size_t out_bytes) {
-    const int64_t wgs = tiles * c, rounds = (wgs + 255) / 256;
-    const double reduce = c > 1 ? std::max(4.5, 2.5 + 3.6 * c * (double)out_bytes / (16 << 20)) : 0.0;
-    switch (tile) {
-        case TILE_L: {
-            const int64_t last = wgs % 256;
-            const double step = 1.28 + 0.47 * std::sqrt(std::max<double>((double)(last - 64) / 192, 0.0));
-            return (nk / c + (c > 1 ? 4.3 : 10.0)) * ((double)(wgs / 256) * 1.75 + (last ? step : 0.0)) + reduce;
-        }
-        case TILE_S: return (double)rounds * (nk / c + (rounds > 1 ? 5.5 : 12.8)) * (rounds > 1 && !of.w_u8 ? 0.60 : 0.573) + reduce;
-        case TILE_S4:
-            if (rounds > 1) return 1e30;
-            if (!of.w_u8 && nk / c >= 128)
-                return (nk / c + 17.0) * (0.42 + 0.12 * (double)wgs / 256) * (0.55 + 0.45 * T / (double)((T + 127) / 128 * 128)) + reduce;
-            return (nk / c + (of.w_u8 ? 22.0 : 20.0)) * std::min(0.50, (of.w_u8 ? 0.34 : 0.30) + 0.19 * (double)wgs / 256) + reduce +
-                   (c == 1 && of.slow_epi && nk < 32 ? 2.0 : 0.0);
-        case TILE_N: return T > 64 ? 1e30 : (double)rounds * (nk / c + std::max(16.5, 13.0 + T / 10.0)) * 0.327 + reduce;
-        default: {
-            // [uint8][groups 8, 4]
-            constexpr struct { double launch, round, split_round, step_0, step_1; } kg[2][2] = {
-                {{3.0, 2.6, 3.6, 0.195, 0.212}, {2.8, 3.6, 4.8, 0.36, 0.37}}, {{2.1, 3.0, 2.5, 0.140, 0.186}, {2.9, 4.2, 3.8, 0.212, 0.320}}};
-            const auto &k = kg[of.w_u8][tile == TILE_K4];
-            const int64_t last = wgs % 256;
-            const double round = c > 1 ? k.split_round : k.round, n = nk / c;
-            return k.launch + (double)(wgs / 256) * (round + n * k.step_1) +
-                   (last ? round + n * (k.step_0 + (k.step_1 - k.step_0) * (double)last / 256) : 0.0) +
-                   0.08 * n * std::max((double)wgs / 256 - 1.0, 0.0) + reduce;
-        }
-    }
+// Cost model of a direct-to-LDS launch in microseconds.  `tiles` tiles of nk k-tiles split c ways run in rounds over the 256 CUs:
+//   launch + rounds * (round, or split_round, which leaves the epilogue to the second pass)
+//          + k-tiles * (step_1 for every full round, between step_0 and step_1 for the last one by the CUs busy,
+//                       extra for what exceeds one round)
+//          + with a split, slab per 16 MB of fp32 slabs written and read and split per slab.
+// One fit per tile and type, over launches within 1.6 times the best one of 342 products each (18 lengths from 24 to 2048 rows, 19 widths
+// from 512 to 16384; weights from HBM; the chip under load before): the tile and split it picks takes 0.5 % (uint8) and 1.2 %
+// (fp16) longer than the best of all on average, 13 and 25 % at most.  A tile per round costs between 5 and 13 us whatever K is, so
+// tiles of many sizes pay: each of these is the best one somewhere, the ones with sides of 160, 192 and 224 where 256 x 256 or 128 x
+// 128 leave CUs idle or rows empty.  us, uint8 / fp16 weights: [1024 x 4096] x [4096 x 12288] three rounds of 128 x 128 115.7 / 132.5,
+// one of 256 x 192 90 / 97; [777 x 4096] x [4096 x 16384] 256 x 256 126 / 130, 224 x 256 100 / 107; [768 x 4096] x [4096 x 12288]
+// 104 / 109, 192 x 192 71 / 80.
+struct TilePrice { float launch, round, split_round, step_0, step_1, extra, slab, split; };
+constexpr TilePrice tile_price[2][TILES] = {
+    {   // fp16 weights
+        {3.708f, 9.540f, 10.123f, 1.082f, 1.646f, -0.034f, 3.361f, 0.187f},   // 256x256
+        {3.602f, 2.757f, 3.837f, 0.442f, 0.611f, 0.008f, 5.384f, 0.127f},   // S
+        {2.318f, 4.510f, 4.717f, 0.327f, 0.562f, -0.021f, 7.471f, 0.249f},   // S4
+        {3.693f, 1.904f, 2.695f, 0.368f, 0.662f, 0.050f, 6.663f, 0.f},   // N
+        {2.217f, 2.471f, 4.018f, 0.151f, 0.255f, -0.038f, 6.035f, 0.232f},   // K8
+        {2.313f, 2.916f, 3.938f, 0.236f, 0.421f, -0.066f, 7.570f, 0.214f},   // K4
+        {2.492f, 11.106f, 9.222f, 0.863f, 1.307f, -0.029f, 3.933f, 0.054f},   // 256x192
+        {5.828f, 7.739f, 7.996f, 1.014f, 1.453f, -0.058f, 3.693f, 0.052f},   // 224x256
+        {1.500f, 9.906f, 8.848f, 0.769f, 1.229f, -0.063f, 3.795f, 0.134f},   // 224x192
+        {2.319f, 8.198f, 9.022f, 0.924f, 1.341f, -0.100f, 4.147f, 0.119f},   // 192x256
+        {1.500f, 7.879f, 8.029f, 0.677f, 1.136f, -0.093f, 4.020f, 0.115f},   // 192x192
+        {1.500f, 7.941f, 8.551f, 0.744f, 1.251f, -0.211f, 4.156f, 0.262f},   // 160x256
+        {3.484f, 4.923f, 5.617f, 0.601f, 1.136f, -0.080f, 3.797f, 0.106f},   // 160x192
+        {5.276f, 4.061f, 5.783f, 0.703f, 1.013f, 0.007f, 3.958f, 0.064f},   // 128x256
+        {3.435f, 5.320f, 4.890f, 0.556f, 0.818f, -0.009f, 6.064f, 0.088f},   // 128x192
+    }, {   // uint8
+        {5.421f, 9.020f, 8.769f, 1.060f, 1.557f, 0.035f, 3.401f, 0.f},   // 256x256
+        {6.865f, 0.f, 1.265f, 0.368f, 0.545f, -0.069f, 4.173f, 0.112f},   // S
+        {5.254f, 3.096f, 3.291f, 0.325f, 0.487f, 0.080f, 4.998f, 0.145f},   // S4
+        {5.979f, 0.f, 0.f, 0.385f, 0.448f, -0.153f, 8.262f, 0.100f},   // N
+        {2.896f, 3.047f, 4.100f, 0.118f, 0.178f, 0.011f, 5.349f, 0.166f},   // K8
+        {3.277f, 2.970f, 3.735f, 0.204f, 0.297f, 0.032f, 7.355f, 0.128f},   // K4
+        {5.830f, 10.148f, 5.253f, 0.816f, 1.178f, 0.103f, 4.239f, 0.f},   // 256x192
+        {5.115f, 10.229f, 9.416f, 0.904f, 1.400f, -0.089f, 2.933f, 0.f},   // 224x256
+        {6.133f, 8.038f, 5.055f, 0.749f, 1.082f, 0.098f, 4.030f, 0.f},   // 224x192
+        {6.073f, 6.623f, 6.623f, 0.846f, 1.216f, 0.047f, 3.270f, 0.087f},   // 192x256
+        {6.485f, 6.782f, 3.426f, 0.603f, 0.936f, 0.129f, 4.279f, 0.044f},   // 192x192
+        {6.755f, 5.550f, 5.237f, 0.764f, 1.092f, 0.061f, 3.441f, 0.023f},   // 160x256
+        {6.725f, 5.622f, 3.040f, 0.535f, 0.854f, 0.116f, 4.004f, 0.077f},   // 160x192
+        {6.404f, 4.079f, 3.566f, 0.619f, 0.886f, 0.093f, 4.419f, 0.120f},   // 128x256
+        {6.151f, 3.907f, 2.421f, 0.540f, 0.721f, 0.089f, 5.413f, 0.129f},   // 128x192
+    }};
+double dma_cost(bool w_u8, int tile, int64_t T, int64_t tiles, int nk, int c, size_t out_bytes) {
+    if (tile == TILE_N && T > 64) return 1e30;
+    const TilePrice &p = tile_price[w_u8][tile];
+    const int64_t wgs = tiles * c, full = wgs / 256;
+    const float n = (float)(nk / c), last = (float)(wgs % 256) / 256.f;
+    float us = p.launch + (float)(full + (last > 0.f)) * (c > 1 ? p.split_round : p.round) + n * p.step_1 * ((float)full + last);
+    if (last > 0.f) us += n * p.step_0 * (1.f - last);
+    if (wgs > 256) us += n * p.extra * ((float)wgs / 256.f - 1.f);
+    if (c > 1) us += (float)c * (p.split + p.slab * (float)out_bytes / (float)(16 << 20));
+    return us;
 }
 
 // the K split (1..8, whole k-tiles, at least 8 per split, slabs within ws_bytes) of least cost
-int dma_split(CostOf of, int tile, int64_t T, int64_t tiles, int nk, size_t out_bytes, size_t ws_bytes, double *cost = nullptr) {
+int dma_split(bool w_u8, int tile, int64_t T, int64_t tiles, int nk, size_t out_bytes, size_t ws_bytes, double *cost = nullptr) {
     int best = 1;
     double best_cost = 1e30;
     for (int c = 1; c <= 8; ++c) {
         if (nk % c || (c > 1 && nk / c < 8) || (c > 1 && c * out_bytes > ws_bytes)) continue;
-        const double k = dma_cost(of, tile, T, tiles, nk, c, out_bytes);
+        const double k = dma_cost(w_u8, tile, T, tiles, nk, c, out_bytes);
         if (k < best_cost) { best_cost = k; best = c; }
     }
     if (cost) *cost = best_cost;
@@ -1960,7 +2032,7 @@ int dma_split(CostOf of, int tile, int64_t T, int64_t tiles, int nk, size_t out_
 }
 
 // the tile of least cost for products of M_i outputs (n of them, one launch); ks: its K split
-int dma_tile(CostOf of, int64_t T, int nk, int n, const int64_t *M, size_t ws_bytes, int *ks, double *cost = nullptr) {
+int dma_tile(bool w_u8, int64_t T, int nk, int n, const int64_t *M, size_t ws_bytes, int *ks, double *cost = nullptr) {
     int best = TILE_S;
     double best_cost = 1e30;
     int64_t outs = 0;
@@ -1970,7 +2042,7 @@ int dma_tile(CostOf of, int64_t T, int nk, int n, const int64_t *M, size_t ws_by
         int64_t tiles = 0;
         for (int i = 0; i < n; ++i) tiles += ((T + d.tm - 1) / d.tm) * ((M[i] + d.tn - 1) / d.tn);
         double c;
-        const int k = dma_split(of, tile, T, tiles, nk, (size_t)(T * outs) * sizeof(float), ws_bytes, &c);
+        const int k = dma_split(w_u8, tile, T, tiles, nk, (size_t)(T * outs) * sizeof(float), ws_bytes, &c);
         if (c < best_cost) { best_cost = c; best = tile; *ks = k; }
     }
     if (cost) *cost = best_cost;
@@ -1988,39 +2060,27 @@ int launch_splitk_epilogue(int ks, int64_t T, int64_t M, void *Y, int64_t ldy, c
     return RWKV_OK;
 }
 
-// gemm_dma_kernel with K split ks ways (slabs as in launch_cfg).
-template <bool W_U8, int TM, int TN, int NW, int NSTG>
-int launch_dma(int ks, int64_t T, int64_t N, int64_t M, const rwkv_half *A, int64_t lda, const void *W, int64_t ldw, void *Y,
-               int64_t ldy, GemmEpi ep, hipStream_t st) {
-    constexpr size_t lds = DmaCfg<W_U8, TM, TN, NW, NSTG>::LDS;
-    constexpr int FOURS = TM == 256 ? 1 : -1, EIGHTS = TM == 256 ? 0 : -1;
-    static PerDeviceOnce once;
-    bool *attr_done = once.slot();
-    if (!attr_done || !*attr_done) {
-        hipError_t e = hipFuncSetAttribute((const void *)gemm_dma_kernel<W_U8, false, TM, TN, NW, NSTG, EIGHTS>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (e == hipSuccess)
-            e = hipFuncSetAttribute((const void *)gemm_dma_kernel<W_U8, false, TM, TN, NW, NSTG, FOURS>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (e == hipSuccess)
-            e = hipFuncSetAttribute((const void *)gemm_dma_kernel<W_U8, true, TM, TN, NW, NSTG, -1>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (e != hipSuccess) return (int)e;
-        if (attr_done) *attr_done = true;
+// A launch of tile `tile` with K split ks ways, its slabs in g.part.
+template <bool W_U8>
+int launch_tile(int tile, GemmGroup &g, int n, int64_t T, int64_t N, int ks, hipStream_t st) {
+    switch (tile) {
+        case TILE_256x256: return launch_dma<W_U8, 256, 256, 8, 0>(g, n, T, N, ks, st);
+        case TILE_S: return launch_dma<W_U8, 128, 128, 8, 0>(g, n, T, N, ks, st);
+        case TILE_S4: return launch_dma<W_U8, 128, 128, 8, 4>(g, n, T, N, ks, st);
+        case TILE_N: return launch_dma<W_U8, 64, 128, 4, 4>(g, n, T, N, ks, st);
+        case TILE_K8: return launch_kg<W_U8, 64, 64>(g, n, T, N, ks, st);
+        case TILE_K4: return launch_kg<W_U8, 64, 128>(g, n, T, N, ks, st);
+        case TILE_256x192: return launch_dma<W_U8, 256, 192, 8, 0>(g, n, T, N, ks, st);
+        case TILE_224x256: return launch_dma<W_U8, 224, 256, 8, 0>(g, n, T, N, ks, st);
+        case TILE_224x192: return launch_dma<W_U8, 224, 192, 8, 0>(g, n, T, N, ks, st);
+        case TILE_192x256: return launch_dma<W_U8, 192, 256, 8, 0>(g, n, T, N, ks, st);
+        case TILE_192x192: return launch_dma<W_U8, 192, 192, 8, 0>(g, n, T, N, ks, st);
+        case TILE_160x256: return launch_dma<W_U8, 160, 256, 8, 0>(g, n, T, N, ks, st);
+        case TILE_160x192: return launch_dma<W_U8, 160, 192, 8, 0>(g, n, T, N, ks, st);
+        case TILE_128x256: return launch_dma<W_U8, 128, 256, 8, 0>(g, n, T, N, ks, st);
+        case TILE_128x192: return launch_dma<W_U8, 128, 192, 8, 0>(g, n, T, N, ks, st);
+        default: return RWKV_E_DTYPE;
     }
-    if (!dma_ok(W_U8, N, M, A, lda, W, ldw, Y, ldy, ep)) return RWKV_E_LAYOUT;
-    ep.walk_m = walks_m(W_U8, T, N, M);
-    const int64_t tiles = ((T + TM - 1) / TM) * ((M + TN - 1) / TN);
-    const int nk = (int)(N / BK);
-    if (ks > 1) {
-        hipLaunchKernelGGL((gemm_dma_kernel<W_U8, true, TM, TN, NW, NSTG, -1>), dim3((unsigned)tiles, (unsigned)ks), dim3(64 * NW), lds, st, (int)T, (int)N,
-                           (int)M, (const h16 *)A, lda, W, ldw, Y, ldy, ep, nk / ks, ep.splitk_ws);
-        return launch_splitk_epilogue(ks, T, M, Y, ldy, ep, st);
-    } else {
-        const auto kernel = by_four((int)M, ldy, Y, ep) ? gemm_dma_kernel<W_U8, false, TM, TN, NW, NSTG, FOURS>
-                                                       : gemm_dma_kernel<W_U8, false, TM, TN, NW, NSTG, EIGHTS>;
-        hipLaunchKernelGGL(kernel, dim3((unsigned)tiles), dim3(64 * NW), lds, st, (int)T, (int)N, (int)M, (const h16 *)A, lda, W, ldw,
-                           Y, ldy, ep, nk, (float *)nullptr);
-    }
-    RWKV_LAUNCH_CHECK();
-    return RWKV_OK;
 }
 
 constexpr int CFG_DMA = 16;   // + TILE_*
@@ -2032,28 +2092,21 @@ int launch_pick(int cfg, int ks, int64_t T, int64_t N, int64_t M, const rwkv_hal
         case 9:
             if constexpr (W_U8) return launch_cfg<true, 256, 256, 4, 4, 2>(T, N, M, A, lda, W, ldw, Y, ldy, ep, st);
             return RWKV_E_DTYPE;
-        case CFG_DMA + TILE_L: return launch_dma<W_U8, 256, 256, 8, 0>(ks, T, N, M, A, lda, W, ldw, Y, ldy, ep, st);
-        case CFG_DMA + TILE_S: return launch_dma<W_U8, 128, 128, 8, 0>(ks, T, N, M, A, lda, W, ldw, Y, ldy, ep, st);
-        case CFG_DMA + TILE_S4: return launch_dma<W_U8, 128, 128, 8, 4>(ks, T, N, M, A, lda, W, ldw, Y, ldy, ep, st);
-        case CFG_DMA + TILE_N: return launch_dma<W_U8, 64, 128, 4, 4>(ks, T, N, M, A, lda, W, ldw, Y, ldy, ep, st);
-        case CFG_DMA + TILE_K8:
-        case CFG_DMA + TILE_K4: {
-            if (!dma_ok(W_U8, N, M, A, lda, W, ldw, Y, ldy, ep)) return RWKV_E_LAYOUT;
-            GemmGroup g{};
-            g.A[0] = (const h16 *)A; g.W[0] = W; g.Y[0] = Y; g.lda = lda; g.ldw[0] = ldw; g.ldy[0] = ldy; g.M[0] = (int)M; g.ep[0] = ep;
-            g.nk_split = (int)(N / BK) / ks;
-            g.part[0] = ep.splitk_ws;
-            const int rc = cfg == CFG_DMA + TILE_K8 ? launch_kg<W_U8, 64, 64>(g, 1, T, N, ks, st) : launch_kg<W_U8, 64, 128>(g, 1, T, N, ks, st);
-            if (rc || ks == 1) return rc;
-            return launch_splitk_epilogue(ks, T, M, Y, ldy, ep, st);
-        }
-        default: return RWKV_E_DTYPE;
+        default: break;
     }
+    if (cfg < CFG_DMA || cfg >= CFG_DMA + TILES) return RWKV_E_DTYPE;
+    if (!dma_ok(W_U8, N, M, A, lda, W, ldw, Y, ldy, ep)) return RWKV_E_LAYOUT;
+    GemmGroup g{};
+    g.A[0] = (const h16 *)A; g.W[0] = W; g.Y[0] = Y; g.lda = lda; g.ldw[0] = ldw; g.ldy[0] = ldy; g.M[0] = (int)M; g.ep[0] = ep;
+    g.nk_split = (int)(N / BK) / ks;
+    g.part[0] = ep.splitk_ws;
+    const int rc = launch_tile<W_U8>(cfg - CFG_DMA, g, 1, T, N, ks, st);
+    if (rc || ks == 1) return rc;
+    return launch_splitk_epilogue(ks, T, M, Y, ldy, ep, st);
 }
 
-// Tile choice (RWKV_GEMM_CFG = 3, 9, 14, 15, 20 or 21 overrides it for tuning sweeps: the register-staged tiles by their
-// number here, the direct-to-LDS 256 x 256 and 128 x 128 tiles and gemm_kg_kernel's 64 x 64 and 64 x 128 ones with the K split
-// of least cost).
+// Tile choice (RWKV_GEMM_CFG overrides it for tuning sweeps: 3 and 9 the register-staged tiles by their number here, 14 and 15 the
+// direct-to-LDS 256 x 256 and 128 x 128 ones, 18 to 30 the others, CFG_DMA + TILE_*, with the K split of least cost).
 //   CFG_DMA +  operands laid out for 16-byte loads: the direct-to-LDS kernel with the tile and K split that the cost
 //              model puts first (128 x 128 tiles at full depth when another product runs beside this one: a 256 x 256
 //              tile's LDS leaves no room beside it on the CU, two small ones fit)
@@ -2066,20 +2119,19 @@ int pick_cfg(int64_t T, int64_t N, int64_t M, bool w_u8, const GemmEpi &ep, bool
     // The reduction pass takes eight outputs at a time, or four.  Not splitting widths that are no multiple of eight cost
     // [100 x 16384] x [16384 x 1004] 45.7 us against 28.2, [300 x 16384] x [16384 x 1004] 48.8 against 33.4.
     const size_t ws = !(M & 3) && ep.splitk_ws ? ep.splitk_bytes : 0;
-    const CostOf of = {w_u8, slow_epilogue(ep)};
     auto with_split = [&](int tile) {
         const TileDim d = tile_dim[tile];
-        *ks = dma_split(of, tile, T, ((T + d.tm - 1) / d.tm) * ((M + d.tn - 1) / d.tn), (int)(N / BK), (size_t)(T * M) * sizeof(float), ws);
+        *ks = dma_split(w_u8, tile, T, ((T + d.tm - 1) / d.tm) * ((M + d.tn - 1) / d.tn), (int)(N / BK), (size_t)(T * M) * sizeof(float), ws);
         return CFG_DMA + tile;
     };
     const char *e = getenv("RWKV_GEMM_CFG");
     if (e && *e) {
         const int cfg = atoi(e);
-        return cfg == 14 ? with_split(TILE_L) : cfg == 15 ? with_split(TILE_S) : cfg == CFG_DMA + TILE_K8 ? with_split(TILE_K8)
-             : cfg == CFG_DMA + TILE_K4 ? with_split(TILE_K4) : cfg < CFG_DMA ? cfg : -1;
+        return cfg == 14 ? with_split(TILE_256x256) : cfg == 15 ? with_split(TILE_S)
+             : cfg >= CFG_DMA + TILE_S4 && cfg < CFG_DMA + TILES ? with_split(cfg - CFG_DMA) : cfg < CFG_DMA ? cfg : -1;
     }
     if (dma && !alone) return with_split(TILE_S);
-    if (dma) return CFG_DMA + dma_tile(of, T, (int)(N / BK), 1, &M, ws, ks);
+    if (dma) return CFG_DMA + dma_tile(w_u8, T, (int)(N / BK), 1, &M, ws, ks);
     if (!alone) return 3;
     const int64_t big = ((T + 255) / 256) * ((M + 255) / 256), rounds = (big + 255) / 256;
     return w_u8 && big * 10 >= rounds * 256 * 7 ? 9 : 3;   // fp16 weight tiles are twice the bytes: the large tile spills
@@ -2096,7 +2148,7 @@ GemmPlan gemm_plan(bool w_u8, int64_t T, int64_t N, int64_t M, const rwkv_half *
     const TileDim d = tile_dim[cfg - CFG_DMA];
     const int64_t tiles = ((T + d.tm - 1) / d.tm) * ((M + d.tn - 1) / d.tn);
     return GemmPlan{2, d.tm, d.tn, ks,
-                    dma_cost({w_u8, slow_epilogue(ep)}, cfg - CFG_DMA, T, tiles, (int)(N / BK), ks, (size_t)(T * M) * sizeof(float))};
+                    dma_cost(w_u8, cfg - CFG_DMA, T, tiles, (int)(N / BK), ks, (size_t)(T * M) * sizeof(float))};
 }
 
 int gemm_launch(bool w_u8, int64_t T, int64_t N, int64_t M, const rwkv_half *A, int64_t lda, const void *W,
@@ -2140,7 +2192,7 @@ static int group_tile(bool w_u8, int n, int64_t T, int64_t N, const rwkv_mat *co
         outs[i] = mats[i]->M;
         m8 = m8 && !(mats[i]->M & 7);
     }
-    return dma_tile({w_u8, false}, T, (int)(N / BK), n, outs, may_split && m8 ? RWKV_SPLITK_WS_BYTES : 0, ks, us);
+    return dma_tile(w_u8, T, (int)(N / BK), n, outs, may_split && m8 ? RWKV_SPLITK_WS_BYTES : 0, ks, us);
 }
 GemmPlan gemm_group_plan(bool w_u8, int n, int64_t T, int64_t N, const rwkv_half *const *x, const rwkv_mat *const *mats,
                          void *const *Y, bool may_split) {
@@ -2232,15 +2284,7 @@ int gemm_group_launch(bool w_u8, int n, int64_t T, int64_t N, const rwkv_half *c
             float *p = splitk_ws;
             for (int i = 0; i < n; ++i) { g.part[i] = p; p += (size_t)ks * T * mats[i]->M; }
         }
-        int rc;
-        switch (tile) {
-            case TILE_L: rc = w_u8 ? launch_dma_group<true, 256, 256, 8, 0>(g, n, T, N, ks, st) : launch_dma_group<false, 256, 256, 8, 0>(g, n, T, N, ks, st); break;
-            case TILE_S: rc = w_u8 ? launch_dma_group<true, 128, 128, 8, 0>(g, n, T, N, ks, st) : launch_dma_group<false, 128, 128, 8, 0>(g, n, T, N, ks, st); break;
-            case TILE_S4: rc = w_u8 ? launch_dma_group<true, 128, 128, 8, 4>(g, n, T, N, ks, st) : launch_dma_group<false, 128, 128, 8, 4>(g, n, T, N, ks, st); break;
-            case TILE_K8: rc = w_u8 ? launch_kg<true, 64, 64>(g, n, T, N, ks, st) : launch_kg<false, 64, 64>(g, n, T, N, ks, st); break;
-            case TILE_K4: rc = w_u8 ? launch_kg<true, 64, 128>(g, n, T, N, ks, st) : launch_kg<false, 64, 128>(g, n, T, N, ks, st); break;
-            default: rc = w_u8 ? launch_dma_group<true, 64, 128, 4, 4>(g, n, T, N, ks, st) : launch_dma_group<false, 64, 128, 4, 4>(g, n, T, N, ks, st); break;
-        }
+        const int rc = w_u8 ? launch_tile<true>(tile, g, n, T, N, ks, st) : launch_tile<false>(tile, g, n, T, N, ks, st);
         if (rc) return rc;
         if (ks > 1) {
             const unsigned blocks = (unsigned)std::min<int64_t>((max_out + 2047) / 2048, 16384);

@@ -33,7 +33,7 @@ struct GemmEpi {
     // says which launches those are).
     // Producer: emit_ry != NULL: the output y is stored as fp16(y * emit_ry[m]), already scaled for the next
     //   product, and the sums of y and of y * emit_my over the columns of each tile go to
-    //   emit_s0 / emit_s2 [T][ceil(M / tile width)].
+    //   emit_s0 / emit_s2 [T][emitted_parts(M, tile width)].
     // Consumer: parts > 1: p0 / p2 [T][parts] hold such partial row sums; a row's totals are formed in index order
     //   by the launch itself (the K-split form writes them to s0 / s2 for its second pass, so these name scratch).
     const rwkv_half *emit_ry, *emit_my;
@@ -42,6 +42,9 @@ struct GemmEpi {
     const float *p0, *p2;
     int walk_m;                    // set by the launch: consecutive tiles walk along M first (direct-to-LDS launches)
 };
+
+// Partial row sums that a launch of tiles tn columns wide emits per row of M outputs: one per tile, and zeros up to a multiple of four.
+__host__ __device__ inline int emitted_parts(int M, int tn) { return ((M + tn - 1) / tn + 3) & ~3; }
 
 // How gemm_launch would run a product: kind 0 = the 2..16-row kernel, 1 = register-staged tiles, 2 = direct-to-LDS
 // tiles of tm x tn with K split ks ways; us: what the cost model says of the latter.
