@@ -18,6 +18,7 @@ OUT = os.path.join(HERE, "librwkv_hip.so")
 FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+    "-mllvm", "-amdgpu-kernarg-preload-count=16",   # leading scalar arguments arrive in registers
     "-Wall", "-Wno-unused-function",
 ]
 

@@ -503,9 +503,9 @@ DEV void emit_parts(const GemmEpi &ep, int t, int m0, int M, int TN, float a0, f
 }
 // This workgroup's tile: the hardware deals consecutive workgroup ids round-robin to the 8 XCDs; undone here, so that
 // each XCD gets a contiguous range of tiles (those walk the T direction first, and share weight tiles in its L2).
-DEV int xcd_tile() {
+DEV int xcd_tile(int tiles) {
     const int bid = blockIdx.x;
-    return (gridDim.x & 7) == 0 ? (bid & 7) * (gridDim.x >> 3) + (bid >> 3) : bid;
+    return (tiles & 7) == 0 ? (bid & 7) * (tiles >> 3) + (bid >> 3) : bid;
 }
 // Its place.  The walk goes along T, so that an XCD reads all activations and its own part of the weights, unless the activations
 // are the larger operand and more than its 4 MB of L2 hold: then along M.  us, uint8, T -> M: 64 x 64 tile, [2048 x 4096] x [4096 x
@@ -524,7 +524,7 @@ constexpr int vm_lgkm0(int n) { return 0x0070 | (n & 15) | ((n >> 4) << 14); }
 constexpr int lgkm_only(int n) { return 0xC07F | (n << 8); }
 
 template <bool W_U8, bool SPLIT, int TM, int TN, int NW, int NSTG>
-DEV void gemm_dma_body(int bid, int T, int N, int M, const h16 *__restrict__ A, int64_t lda, const void *__restrict__ Wv,
+DEV void gemm_dma_body(int bid, int T, int N, int M, int walk_m, const h16 *__restrict__ A, int64_t lda, const void *__restrict__ Wv,
                        int64_t ldw, void *__restrict__ Y, int64_t ldy, const GemmEpi &ep, int nk_split,
                        float *__restrict__ part, int split) {
     using Cfg = DmaCfg<W_U8, TM, TN, NW, NSTG>;
@@ -533,9 +533,9 @@ DEV void gemm_dma_body(int bid, int T, int N, int M, const h16 *__restrict__ A, 
     extern __shared__ __align__(1024) unsigned char smem[];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int grp = wave / (Cfg::WR * Cfg::WC), wr = wave / Cfg::WC % Cfg::WR, wc = wave % Cfg::WC;
-    const TileAt at = tile_at<TM, TN>(bid, T, M, ep.walk_m);
+    const TileAt at = tile_at<TM, TN>(bid, T, M, walk_m);
     const int t0 = at.t0, m0 = at.m0;
-    const int kbase = SPLIT ? split * nk_split : 0, nk = SPLIT ? nk_split : N / BK;
+    const int kbase = SPLIT ? split * nk_split : 0, nk = nk_split;
 
     // load sources; rows past the end re-read the last row (never stored)
     auto a_piece = [&](int i) { return min(wave * AL + i, Cfg::AP - 1); };
@@ -1001,47 +1001,63 @@ DEV void gemm_dma_body(int bid, int T, int N, int M, const h16 *__restrict__ A, 
 // Direct-to-LDS tiles: blockIdx.x runs over the tiles of all members, first[i] being member i's first.  (With a grid
 // for the widest member the tiles of the narrow ones all fell on the first XCDs: four first LoRA stages of 128, 128,
 // 128 and 512 outputs took two rounds on two XCDs with the others idle, 41 us instead of 23 with the 64 x 64 tile.)
-struct GemmGroup {
-    const h16 *A[4];
-    const void *W[4];
-    void *Y[4];
-    int64_t lda, ldw[4], ldy[4];
-    int M[4];
-    float *part[4];   // split-K slabs of member i, [splits][T][M_i] (direct-to-LDS group only)
+struct GemmMember {
+    const h16 *A;     // what the first loads need, 32 bytes
+    const void *W;
+    int64_t ldw;
+    int M, walk_m;    // walk_m: consecutive tiles walk along M first (direct-to-LDS launches)
+    void *Y;
+    int64_t ldy;
+    float *part;      // split-K slabs, [splits][T][M] (direct-to-LDS launches only)
+    GemmEpi ep;
+};
+struct GemmMembers { GemmMember m[4]; };
+struct GemmGroup : GemmMembers {
+    int64_t lda;
     int first[4];     // members that are not there: INT_MAX
     int nk_split;
-    GemmEpi ep[4];
 };
 
 // register-staged 128 x 128 tiles: uint8 matrices whose mx or rx lie on no 16-byte boundary
 __global__ __launch_bounds__(256) void gemm_group_kernel(int T, int N, GemmGroup g) {
-    const int gi = blockIdx.y, M = g.M[gi];
-    gemm_body<true, 128, 128, 2, 2, 4, false>(T, N, M, g.A[gi], g.lda, g.W[gi], g.ldw[gi], g.Y[gi], M, g.ep[gi], N / BK, nullptr);
+    const int gi = blockIdx.y, M = g.m[gi].M;
+    gemm_body<true, 128, 128, 2, 2, 4, false>(T, N, M, g.m[gi].A, g.lda, g.m[gi].W, g.m[gi].ldw, g.m[gi].Y, M, g.m[gi].ep, N / BK, nullptr);
 }
 
-DEV int group_member(const GemmGroup &g, int &tile) {
-    const int gi = (tile >= g.first[1]) + (tile >= g.first[2]) + (tile >= g.first[3]);
-    tile -= g.first[gi];
+// The member that a tile belongs to, and its tile of it.  first1 .. first3 are kernel arguments of their own ahead of the members:
+// such ones are in scalar registers when a wave starts.  What the first loads need of a member is read at once: left alone, the compiler
+// reads M, waits, and then reads the pointers.
+DEV int group_member(int first1, int first2, int first3, int &tile) {
+    const int gi = (tile >= first1) + (tile >= first2) + (tile >= first3);
+    tile -= tile >= first3 ? first3 : tile >= first2 ? first2 : tile >= first1 ? first1 : 0;
     return gi;
+}
+struct GemmIn { const h16 *A; const void *W; int64_t ldw; int M, walk_m; };
+DEV GemmIn gemm_in(const GemmMember &m) {
+    GemmIn in = {m.A, m.W, m.ldw, m.M, m.walk_m};
+    asm volatile("" : "+s"(in.A), "+s"(in.W), "+s"(in.ldw), "+s"(in.M), "+s"(in.walk_m));
+    return in;
 }
 // fills `first` and the walks for tiles of tm x tn; returns the tiles of the launch
 int64_t group_tiles(bool w_u8, GemmGroup &g, int n, int64_t T, int64_t N, int tm, int tn) {
     int64_t tiles = 0;
-    for (int i = 0; i < n; ++i) g.ep[i].walk_m = walks_m(w_u8, T, N, g.M[i]);
+    for (int i = 0; i < n; ++i) g.m[i].walk_m = walks_m(w_u8, T, N, g.m[i].M);
     for (int i = 0; i < 4; ++i) {
         g.first[i] = i < n ? (int)tiles : 0x7fffffff;
-        if (i < n) tiles += ((T + tm - 1) / tm) * ((g.M[i] + tn - 1) / tn);
+        if (i < n) tiles += ((T + tm - 1) / tm) * ((g.m[i].M + tn - 1) / tn);
     }
     return tiles;
 }
 
 // the direct-to-LDS kernel; blockIdx.y is the K split
 template <bool W_U8, bool SPLIT, int TM, int TN, int NW, int NSTG>
-__global__ __launch_bounds__(64 * NW) void gemm_dma_kernel(int T, int N, GemmGroup g) {
-    int tile = xcd_tile();
-    const int gi = group_member(g, tile), M = g.M[gi];
-    gemm_dma_body<W_U8, SPLIT, TM, TN, NW, NSTG>(tile, T, N, M, g.A[gi], g.lda, g.W[gi], g.ldw[gi], g.Y[gi], g.ldy[gi], g.ep[gi],
-                                                 SPLIT ? g.nk_split : N / BK, g.part[gi], SPLIT ? blockIdx.y : 0);
+__global__ __launch_bounds__(64 * NW) void gemm_dma_kernel(int T, int N, int tiles, int first1, int first2, int first3, int nk_split,
+                                                           int64_t lda, GemmMembers g) {
+    int tile = xcd_tile(tiles);
+    const GemmMember &m = g.m[group_member(first1, first2, first3, tile)];
+    const GemmIn in = gemm_in(m);
+    gemm_dma_body<W_U8, SPLIT, TM, TN, NW, NSTG>(tile, T, N, in.M, in.walk_m, in.A, lda, in.W, in.ldw, m.Y, m.ldy, m.ep, nk_split, m.part,
+                                                 SPLIT ? blockIdx.y : 0);
 }
 
 template <bool W_U8, int TM, int TN, int NW, int NSTG>
@@ -1059,8 +1075,9 @@ int launch_dma(GemmGroup &g, int n, int64_t T, int64_t N, int ks, hipStream_t st
         if (attr_done) *attr_done = true;
     }
     const dim3 grid((unsigned)group_tiles(W_U8, g, n, T, N, TM, TN), (unsigned)ks);
-    if (ks > 1) hipLaunchKernelGGL((gemm_dma_kernel<W_U8, true, TM, TN, NW, NSTG>), grid, dim3(64 * NW), lds, st, (int)T, (int)N, g);
-    else hipLaunchKernelGGL((gemm_dma_kernel<W_U8, false, TM, TN, NW, NSTG>), grid, dim3(64 * NW), lds, st, (int)T, (int)N, g);
+    const auto kernel = ks > 1 ? gemm_dma_kernel<W_U8, true, TM, TN, NW, NSTG> : gemm_dma_kernel<W_U8, false, TM, TN, NW, NSTG>;
+    hipLaunchKernelGGL(kernel, grid, dim3(64 * NW), lds, st, (int)T, (int)N, (int)grid.x, g.first[1], g.first[2], g.first[3], g.nk_split, g.lda,
+                       (const GemmMembers &)g);
     RWKV_LAUNCH_CHECK();
     return RWKV_OK;
 }
@@ -1101,7 +1118,7 @@ template <int RBYTES> DEV int kg_key(int row) {
     return (row / RPB) & (CH - 1);
 }
 template <bool W_U8, bool SPLIT, int TM, int TN>
-DEV void gemm_kg_body(int bid, int T, int N, int M, const h16 *__restrict__ A, int64_t lda, const void *__restrict__ Wv, int64_t ldw,
+DEV void gemm_kg_body(int bid, int T, int N, int M, int walk_m, const h16 *__restrict__ A, int64_t lda, const void *__restrict__ Wv, int64_t ldw,
                       void *__restrict__ Y, int64_t ldy, const GemmEpi &ep, int nk_split, float *__restrict__ part, int split) {
     using Cfg = KgCfg<W_U8, TM, TN>;
     constexpr int NST = Cfg::NST, STAGE = Cfg::STAGE, AL = Cfg::AL, WL = Cfg::WL, BKS = Cfg::BKS, KW = Cfg::KW, US = Cfg::US;
@@ -1109,9 +1126,9 @@ DEV void gemm_kg_body(int bid, int T, int N, int M, const h16 *__restrict__ A, i
     extern __shared__ __align__(1024) unsigned char smem[];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int blk = wave % (RA * RB), grp = wave / (RA * RB), wr = blk / RB, wc = blk % RB;
-    const TileAt at = tile_at<TM, TN>(bid, T, M, ep.walk_m);
+    const TileAt at = tile_at<TM, TN>(bid, T, M, walk_m);
     const int t0 = at.t0, m0 = at.m0;
-    const int kbase = SPLIT ? split * nk_split * BK : 0, K = SPLIT ? nk_split * BK : N;   // this workgroup's k's (a multiple of 64)
+    const int kbase = SPLIT ? split * nk_split * BK : 0, K = nk_split * BK;   // this workgroup's k's (a multiple of 64)
     const int nk = (K + BKS - 1) / BKS;
 
     // load sources; rows past the end re-read the last row (never stored).  Load i of a wave fills 1 KB: the rows
@@ -1381,11 +1398,13 @@ DEV void gemm_kg_body(int bid, int T, int N, int M, const h16 *__restrict__ A, i
 }
 
 template <bool W_U8, bool SPLIT, int TM, int TN>
-__global__ __launch_bounds__(512) void gemm_kg_kernel(int T, int N, GemmGroup g) {
-    int tile = xcd_tile();
-    const int gi = group_member(g, tile), M = g.M[gi];
-    gemm_kg_body<W_U8, SPLIT, TM, TN>(tile, T, N, M, g.A[gi], g.lda, g.W[gi], g.ldw[gi], g.Y[gi], g.ldy[gi], g.ep[gi],
-                                      SPLIT ? g.nk_split : N / BK, g.part[gi], SPLIT ? blockIdx.y : 0);
+__global__ __launch_bounds__(512) void gemm_kg_kernel(int T, int N, int tiles, int first1, int first2, int first3, int nk_split, int64_t lda,
+                                                      GemmMembers g) {
+    int tile = xcd_tile(tiles);
+    const GemmMember &m = g.m[group_member(first1, first2, first3, tile)];
+    const GemmIn in = gemm_in(m);
+    gemm_kg_body<W_U8, SPLIT, TM, TN>(tile, T, N, in.M, in.walk_m, in.A, lda, in.W, in.ldw, m.Y, m.ldy, m.ep, nk_split, m.part,
+                                      SPLIT ? blockIdx.y : 0);
 }
 
 template <bool W_U8, int TM, int TN>
@@ -1400,8 +1419,9 @@ int launch_kg(GemmGroup &g, int n, int64_t T, int64_t N, int ks, hipStream_t st)
         if (attr_done) *attr_done = true;
     }
     const dim3 grid((unsigned)group_tiles(W_U8, g, n, T, N, TM, TN), (unsigned)ks);
-    if (ks > 1) hipLaunchKernelGGL((gemm_kg_kernel<W_U8, true, TM, TN>), grid, dim3(512), lds, st, (int)T, (int)N, g);
-    else hipLaunchKernelGGL((gemm_kg_kernel<W_U8, false, TM, TN>), grid, dim3(512), lds, st, (int)T, (int)N, g);
+    const auto kernel = ks > 1 ? gemm_kg_kernel<W_U8, true, TM, TN> : gemm_kg_kernel<W_U8, false, TM, TN>;
+    hipLaunchKernelGGL(kernel, grid, dim3(512), lds, st, (int)T, (int)N, (int)grid.x, g.first[1], g.first[2], g.first[3], g.nk_split, g.lda,
+                       (const GemmMembers &)g);
     RWKV_LAUNCH_CHECK();
     return RWKV_OK;
 }
@@ -1409,7 +1429,7 @@ int launch_kg(GemmGroup &g, int n, int64_t T, int64_t N, int ks, hipStream_t st)
 // second pass of a split group launch: member blockIdx.y, as splitk_epilogue8_kernel
 __global__ __launch_bounds__(256) void splitk_group_epilogue8_kernel(int T, int KS, GemmGroup g) {
     const int gi = blockIdx.y;
-    splitk_rows8(T, g.M[gi], KS, g.part[gi], g.Y[gi], g.M[gi], g.ep[gi], (int64_t)blockIdx.x * 256 + threadIdx.x,
+    splitk_rows8(T, g.m[gi].M, KS, g.m[gi].part, g.m[gi].Y, g.m[gi].M, g.m[gi].ep, (int64_t)blockIdx.x * 256 + threadIdx.x,
                      (int64_t)gridDim.x * 256);
 }
 
@@ -1501,12 +1521,8 @@ __global__ __launch_bounds__(256) void mm8_prepare_group_kernel(int T, int N, Pr
 // outputs 18.7 -> 16.8, [8 x 16384] x [16384 x 4096] 22.9 -> 21.4, three of 5120 at 5120 wide 45.3 -> 28.9, [8 x 20480] x
 // [20480 x 5120] 51.9 -> 46.6 (320 row groups on 256 CUs).  The same sums in the same order.
 struct SkinnyGroup {
-    const h16 *A[4];
-    const void *W[4];
-    void *Y[4];
-    int64_t lda, ldw[4], ldy[4];
-    int M[4];
-    GemmEpi ep[4];
+    int64_t lda;
+    GemmMember m[4];
 };
 
 template <int NU>
@@ -1539,14 +1555,14 @@ __global__ __launch_bounds__(1024) void skinny_u8_kernel(int T, int N, int n, in
     };
     int base = 0, count = 0;                                    // row groups of the members before; done by this workgroup
     for (int gi = 0; gi < n; ++gi) {
-        const int M = g.M[gi], groups = (M + 15) >> 4;
+        const int M = g.m[gi].M, groups = (M + 15) >> 4;
         const int lo = max(b0, base) - base, hi = min(b1, base + groups) - base;
         base += groups;
         if (lo >= hi) continue;
-        const GemmEpi &ep = g.ep[gi];
-        const h16 *A = g.A[gi];
-        const unsigned char *W = (const unsigned char *)g.W[gi];
-        const int64_t ldw = g.ldw[gi];
+        const GemmEpi &ep = g.m[gi].ep;
+        const h16 *A = g.m[gi].A;
+        const unsigned char *W = (const unsigned char *)g.m[gi].W;
+        const int64_t ldw = g.m[gi].ldw;
         // In place of a unit past the end of the row, and of every unit past the share's last row group, all lanes load the
         // first bytes of the matrix, which nothing uses: a branch around a load would make the waits for those before it longer.
         struct Step { u32x4 w[UB]; h16x8 x[HELD ? 1 : UB][2]; };
@@ -1587,16 +1603,16 @@ __global__ __launch_bounds__(1024) void skinny_u8_kernel(int T, int N, int n, in
                 for (int w = 0; w < 16; ++w) v += red[buf][w][RQ * (fm >> 2) + 4 * ft + (fm & 3)];
                 const int m = 16 * grp + fm;
                 if (m < M && ft < T) {
-                    const size_t at = (size_t)ft * g.ldy[gi] + m;
+                    const size_t at = (size_t)ft * g.m[gi].ldy + m;
                     v = epi_affine(v, h2f(o.rx), h2f(o.mx), o.s0, o.s2);
                     if (ep.raw_f32) {
-                        ((float *)g.Y[gi])[at] = v;
+                        ((float *)g.m[gi].Y)[at] = v;
                     } else {
                         float r[1] = {v};
                         h16 res[1] = {__builtin_bit_cast(h16, o.res)}, gate[1] = {__builtin_bit_cast(h16, o.gate)};
                         epi_act<1, const h16 *>(r, res, gate, ep);
-                        if (ep.out_dtype == RWKV_DT_F32) ((float *)g.Y[gi])[at] = round_h(r[0]);
-                        else ((rwkv_half *)g.Y[gi])[at] = f2h(r[0]);
+                        if (ep.out_dtype == RWKV_DT_F32) ((float *)g.m[gi].Y)[at] = round_h(r[0]);
+                        else ((rwkv_half *)g.m[gi].Y)[at] = f2h(r[0]);
                     }
                 }
                 if (NB == 1) __builtin_amdgcn_s_waitcnt(0xC07F);
@@ -1692,10 +1708,10 @@ __global__ __launch_bounds__(1024) void skinny_u8_kernel(int T, int N, int n, in
 template <int NCI>
 __global__ __launch_bounds__(1024) void skinny_f16_kernel(int T, int N, SkinnyGroup g) {
     __shared__ float red[16][64][4];
-    const int gi = blockIdx.y, M = g.M[gi];
-    const h16 *__restrict__ A = g.A[gi];
-    const unsigned char *__restrict__ W = (const unsigned char *)g.W[gi];
-    const int64_t lda = g.lda, ldw = g.ldw[gi];
+    const int gi = blockIdx.y, M = g.m[gi].M;
+    const h16 *__restrict__ A = g.m[gi].A;
+    const unsigned char *__restrict__ W = (const unsigned char *)g.m[gi].W;
+    const int64_t lda = g.lda, ldw = g.m[gi].ldw;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int sub = lane & 15, q = lane >> 4;
     const int nchunks = N / 32;
@@ -1755,7 +1771,7 @@ __global__ __launch_bounds__(1024) void skinny_f16_kernel(int T, int N, SkinnyGr
 #pragma unroll
             for (int w = 0; w < 16; ++w) v += red[w][l][r];
             const int m = m0 + 4 * (l >> 4) + r, t = l & 15;
-            if (m < M && t < T) gemm_epilogue(v, t, m, 1.f, 0.f, g.ep[gi], g.Y[gi], g.ldy[gi]);
+            if (m < M && t < T) gemm_epilogue(v, t, m, 1.f, 0.f, g.m[gi].ep, g.m[gi].Y, g.m[gi].ldy);
         }
     }
 }
@@ -1776,8 +1792,8 @@ bool skinny_ok(bool w_u8, int64_t T, int64_t N, const void *A, int64_t lda, cons
 int skinny_launch(bool w_u8, int n, int64_t T, int64_t N, const SkinnyGroup &g, hipStream_t st) {
     int total = 0, maxg = 1;
     for (int i = 0; i < n; ++i) {
-        total += (g.M[i] + 15) / 16;
-        maxg = std::max(maxg, (g.M[i] + 15) / 16);
+        total += (g.m[i].M + 15) / 16;
+        maxg = std::max(maxg, (g.m[i].M + 15) / 16);
     }
     const int64_t per_wave = (N / (w_u8 ? 64 : 32) + 15) / 16;    // chunks a wave owns
 #define RWKV_SKINNY(NC)                                                                                                              \
@@ -2097,9 +2113,9 @@ int launch_pick(int cfg, int ks, int64_t T, int64_t N, int64_t M, const rwkv_hal
     if (cfg < CFG_DMA || cfg >= CFG_DMA + TILES) return RWKV_E_DTYPE;
     if (!dma_ok(W_U8, N, M, A, lda, W, ldw, Y, ldy, ep)) return RWKV_E_LAYOUT;
     GemmGroup g{};
-    g.A[0] = (const h16 *)A; g.W[0] = W; g.Y[0] = Y; g.lda = lda; g.ldw[0] = ldw; g.ldy[0] = ldy; g.M[0] = (int)M; g.ep[0] = ep;
+    g.m[0].A = (const h16 *)A; g.m[0].W = W; g.m[0].Y = Y; g.lda = lda; g.m[0].ldw = ldw; g.m[0].ldy = ldy; g.m[0].M = (int)M; g.m[0].ep = ep;
     g.nk_split = (int)(N / BK) / ks;
-    g.part[0] = ep.splitk_ws;
+    g.m[0].part = ep.splitk_ws;
     const int rc = launch_tile<W_U8>(cfg - CFG_DMA, g, 1, T, N, ks, st);
     if (rc || ks == 1) return rc;
     return launch_splitk_epilogue(ks, T, M, Y, ldy, ep, st);
@@ -2155,7 +2171,7 @@ int gemm_launch(bool w_u8, int64_t T, int64_t N, int64_t M, const rwkv_half *A, 
                 int64_t ldw, void *Y, int64_t ldy, const GemmEpi &ep, hipStream_t st) {
     if (skinny_ok(w_u8, T, N, A, lda, W, ldw, ep)) {
         SkinnyGroup g{};
-        g.A[0] = (const h16 *)A; g.W[0] = W; g.Y[0] = Y; g.lda = lda; g.ldw[0] = ldw; g.ldy[0] = ldy; g.M[0] = (int)M; g.ep[0] = ep;
+        g.m[0].A = (const h16 *)A; g.m[0].W = W; g.m[0].Y = Y; g.lda = lda; g.m[0].ldw = ldw; g.m[0].ldy = ldy; g.m[0].M = (int)M; g.m[0].ep = ep;
         return skinny_launch(w_u8, 1, T, N, g, st);
     }
     if (narrow_ok(w_u8, T, N, M, A, lda, W, ldw, Y, ldy, ep)) {
@@ -2250,26 +2266,26 @@ int gemm_group_launch(bool w_u8, int n, int64_t T, int64_t N, const rwkv_half *c
     bool dma = true;
     for (int i = 0; i < n; ++i) {
         if (mats[i]->N != N) return RWKV_E_SHAPE;
-        g.A[i] = (const h16 *)(prep ? xs[i] : x[i]);
-        g.W[i] = mats[i]->w; g.ldw[i] = mats[i]->ld; g.Y[i] = Y[i]; g.ldy[i] = mats[i]->M; g.M[i] = (int)mats[i]->M;
-        g.ep[i] = eps[i];
-        g.ep[i].ldres = g.ep[i].ldgate = mats[i]->M;
-        if (w_u8) { g.ep[i].mx = mats[i]->mx; g.ep[i].rx = mats[i]->rx; g.ep[i].s0 = sums[i]; g.ep[i].s2 = sums[i] + T; }
-        if (parts > 1) { g.ep[i].parts = parts; g.ep[i].p0 = sums[i] + 2 * T; g.ep[i].p2 = sums[i] + 2 * T + (size_t)T * parts; }
+        g.m[i].A = (const h16 *)(prep ? xs[i] : x[i]);
+        g.m[i].W = mats[i]->w; g.m[i].ldw = mats[i]->ld; g.m[i].Y = Y[i]; g.m[i].ldy = mats[i]->M; g.m[i].M = (int)mats[i]->M;
+        g.m[i].ep = eps[i];
+        g.m[i].ep.ldres = g.m[i].ep.ldgate = mats[i]->M;
+        if (w_u8) { g.m[i].ep.mx = mats[i]->mx; g.m[i].ep.rx = mats[i]->rx; g.m[i].ep.s0 = sums[i]; g.m[i].ep.s2 = sums[i] + T; }
+        if (parts > 1) { g.m[i].ep.parts = parts; g.m[i].ep.p0 = sums[i] + 2 * T; g.m[i].ep.p2 = sums[i] + 2 * T + (size_t)T * parts; }
         tiles = std::max<int64_t>(tiles, ((T + 127) / 128) * ((mats[i]->M + 127) / 128));
         max_out = std::max<int64_t>(max_out, T * mats[i]->M);
-        dma = dma && dma_ok(w_u8, N, mats[i]->M, g.A[i], N, g.W[i], g.ldw[i], g.Y[i], mats[i]->M, g.ep[i]);
+        dma = dma && dma_ok(w_u8, N, mats[i]->M, g.m[i].A, N, g.m[i].W, g.m[i].ldw, g.m[i].Y, mats[i]->M, g.m[i].ep);
     }
     {
         bool skinny = true;
-        for (int i = 0; i < n; ++i) skinny = skinny && skinny_ok(w_u8, T, N, g.A[i], N, g.W[i], g.ldw[i], g.ep[i]);
+        for (int i = 0; i < n; ++i) skinny = skinny && skinny_ok(w_u8, T, N, g.m[i].A, N, g.m[i].W, g.m[i].ldw, g.m[i].ep);
         if (skinny) {
             if (parts > 1) return RWKV_E_LAYOUT;
             SkinnyGroup sg{};
             sg.lda = N;
             for (int i = 0; i < n; ++i) {
-                sg.A[i] = g.A[i]; sg.W[i] = g.W[i]; sg.Y[i] = g.Y[i]; sg.ldw[i] = g.ldw[i]; sg.ldy[i] = g.M[i]; sg.M[i] = g.M[i];
-                sg.ep[i] = g.ep[i];
+                sg.m[i].A = g.m[i].A; sg.m[i].W = g.m[i].W; sg.m[i].Y = g.m[i].Y; sg.m[i].ldw = g.m[i].ldw; sg.m[i].ldy = g.m[i].M; sg.m[i].M = g.m[i].M;
+                sg.m[i].ep = g.m[i].ep;
             }
             return skinny_launch(w_u8, n, T, N, sg, st);
         }
@@ -2282,7 +2298,7 @@ int gemm_group_launch(bool w_u8, int n, int64_t T, int64_t N, const rwkv_half *c
         g.nk_split = nk / ks;
         if (ks > 1) {
             float *p = splitk_ws;
-            for (int i = 0; i < n; ++i) { g.part[i] = p; p += (size_t)ks * T * mats[i]->M; }
+            for (int i = 0; i < n; ++i) { g.m[i].part = p; p += (size_t)ks * T * mats[i]->M; }
         }
         const int rc = w_u8 ? launch_tile<true>(tile, g, n, T, N, ks, st) : launch_tile<false>(tile, g, n, T, N, ks, st);
         if (rc) return rc;

@@ -40,7 +40,6 @@ struct GemmEpi {
     float *emit_s0, *emit_s2;
     int parts;
     const float *p0, *p2;
-    int walk_m;                    // set by the launch: consecutive tiles walk along M first (direct-to-LDS launches)
 };
 
 // Partial row sums that a launch of tiles tn columns wide emits per row of M outputs: one per tile, and zeros up to a multiple of four.
