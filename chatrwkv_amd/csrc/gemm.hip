@@ -501,11 +501,14 @@ DEV void emit_parts(const GemmEpi &ep, int t, int m0, int M, int TN, float a0, f
     if (m0 + TN >= M)
         for (int j = i + 1; j < parts; ++j) p0[j] = p2[j] = 0.f;
 }
-// This workgroup's tile: the hardware deals consecutive workgroup ids round-robin to the 8 XCDs; undone here, so that
-// each XCD gets a contiguous range of tiles (those walk the T direction first, and share weight tiles in its L2).
-DEV int xcd_tile(int tiles) {
-    const int bid = blockIdx.x;
-    return (tiles & 7) == 0 ? (bid & 7) * (tiles >> 3) + (bid >> 3) : bid;
+// This workgroup's place in a launch of `units` workgroups.  The hardware deals consecutive workgroup ids round-robin to the 8 XCDs;
+// undone here, so that each XCD gets a contiguous range of the units: tiles that walk the T direction first and share weight tiles in
+// its L2, each with all of its K splits.  Dealt as the hardware does wherever the tiles were no multiple of eight, every XCD read
+// all of both operands: fp16, us, [300 x 3200] x [3200 x 3200] 20.5 -> 14.4, [333 x 1280] x [1280 x 3840] 14.1 -> 10.8.  With one split
+// after the other instead of one tile after the other an XCD reads a part of every row of the weights: 1 to 2 % slower over 5000 launches.
+DEV int xcd_unit(int units) {
+    const int x = blockIdx.x & 7, each = units >> 3;
+    return x * each + min(x, units & 7) + ((int)blockIdx.x >> 3);
 }
 // Its place.  The walk goes along T, so that an XCD reads all activations and its own part of the weights, unless the activations
 // are the larger operand and more than its 4 MB of L2 hold: then along M.  us, uint8, T -> M: 64 x 64 tile, [2048 x 4096] x [4096 x
@@ -998,7 +1001,7 @@ DEV void gemm_dma_body(int bid, int T, int N, int M, int walk_m, const h16 *__re
 
 // One to four contractions [T, N] x [N, M_i] in one launch: short calls, where each of them alone would split K and need
 // a reduction pass.  Register-staged tiles: blockIdx.y picks the member, the grid is as wide as the widest one.
-// Direct-to-LDS tiles: blockIdx.x runs over the tiles of all members, first[i] being member i's first.  (With a grid
+// Direct-to-LDS tiles: the units run over the tiles of all members, first[i] being member i's first, and the K splits.  (With a grid
 // for the widest member the tiles of the narrow ones all fell on the first XCDs: four first LoRA stages of 128, 128,
 // 128 and 512 outputs took two rounds on two XCDs with the others idle, 41 us instead of 23 with the 64 x 64 tile.)
 struct GemmMember {
@@ -1049,15 +1052,17 @@ int64_t group_tiles(bool w_u8, GemmGroup &g, int n, int64_t T, int64_t N, int tm
     return tiles;
 }
 
-// the direct-to-LDS kernel; blockIdx.y is the K split
+// the direct-to-LDS kernel
 template <bool W_U8, bool SPLIT, int TM, int TN, int NW, int NSTG>
-__global__ __launch_bounds__(64 * NW) void gemm_dma_kernel(int T, int N, int tiles, int first1, int first2, int first3, int nk_split,
+__global__ __launch_bounds__(64 * NW) void gemm_dma_kernel(int T, int N, int units, int splits, int first1, int first2, int first3, int nk_split,
                                                            int64_t lda, GemmMembers g) {
-    int tile = xcd_tile(tiles);
+    const int unit = xcd_unit(units);
+    int tile = SPLIT ? unit / splits : unit;
+    const int split = SPLIT ? unit - tile * splits : 0;
     const GemmMember &m = g.m[group_member(first1, first2, first3, tile)];
     const GemmIn in = gemm_in(m);
     gemm_dma_body<W_U8, SPLIT, TM, TN, NW, NSTG>(tile, T, N, in.M, in.walk_m, in.A, lda, in.W, in.ldw, m.Y, m.ldy, m.ep, nk_split, m.part,
-                                                 SPLIT ? blockIdx.y : 0);
+                                                 split);
 }
 
 template <bool W_U8, int TM, int TN, int NW, int NSTG>
@@ -1074,9 +1079,9 @@ int launch_dma(GemmGroup &g, int n, int64_t T, int64_t N, int ks, hipStream_t st
         if (e != hipSuccess) return (int)e;
         if (attr_done) *attr_done = true;
     }
-    const dim3 grid((unsigned)group_tiles(W_U8, g, n, T, N, TM, TN), (unsigned)ks);
+    const int units = (int)group_tiles(W_U8, g, n, T, N, TM, TN) * ks;
     const auto kernel = ks > 1 ? gemm_dma_kernel<W_U8, true, TM, TN, NW, NSTG> : gemm_dma_kernel<W_U8, false, TM, TN, NW, NSTG>;
-    hipLaunchKernelGGL(kernel, grid, dim3(64 * NW), lds, st, (int)T, (int)N, (int)grid.x, g.first[1], g.first[2], g.first[3], g.nk_split, g.lda,
+    hipLaunchKernelGGL(kernel, dim3((unsigned)units), dim3(64 * NW), lds, st, (int)T, (int)N, units, ks, g.first[1], g.first[2], g.first[3], g.nk_split, g.lda,
                        (const GemmMembers &)g);
     RWKV_LAUNCH_CHECK();
     return RWKV_OK;
@@ -1398,13 +1403,15 @@ DEV void gemm_kg_body(int bid, int T, int N, int M, int walk_m, const h16 *__res
 }
 
 template <bool W_U8, bool SPLIT, int TM, int TN>
-__global__ __launch_bounds__(512) void gemm_kg_kernel(int T, int N, int tiles, int first1, int first2, int first3, int nk_split, int64_t lda,
+__global__ __launch_bounds__(512) void gemm_kg_kernel(int T, int N, int units, int splits, int first1, int first2, int first3, int nk_split, int64_t lda,
                                                       GemmMembers g) {
-    int tile = xcd_tile(tiles);
+    const int unit = xcd_unit(units);
+    int tile = SPLIT ? unit / splits : unit;
+    const int split = SPLIT ? unit - tile * splits : 0;
     const GemmMember &m = g.m[group_member(first1, first2, first3, tile)];
     const GemmIn in = gemm_in(m);
     gemm_kg_body<W_U8, SPLIT, TM, TN>(tile, T, N, in.M, in.walk_m, in.A, lda, in.W, in.ldw, m.Y, m.ldy, m.ep, nk_split, m.part,
-                                      SPLIT ? blockIdx.y : 0);
+                                      split);
 }
 
 template <bool W_U8, int TM, int TN>
@@ -1418,9 +1425,9 @@ int launch_kg(GemmGroup &g, int n, int64_t T, int64_t N, int ks, hipStream_t st)
         if (e != hipSuccess) return (int)e;
         if (attr_done) *attr_done = true;
     }
-    const dim3 grid((unsigned)group_tiles(W_U8, g, n, T, N, TM, TN), (unsigned)ks);
+    const int units = (int)group_tiles(W_U8, g, n, T, N, TM, TN) * ks;
     const auto kernel = ks > 1 ? gemm_kg_kernel<W_U8, true, TM, TN> : gemm_kg_kernel<W_U8, false, TM, TN>;
-    hipLaunchKernelGGL(kernel, grid, dim3(512), lds, st, (int)T, (int)N, (int)grid.x, g.first[1], g.first[2], g.first[3], g.nk_split, g.lda,
+    hipLaunchKernelGGL(kernel, dim3((unsigned)units), dim3(512), lds, st, (int)T, (int)N, units, ks, g.first[1], g.first[2], g.first[3], g.nk_split, g.lda,
                        (const GemmMembers &)g);
     RWKV_LAUNCH_CHECK();
     return RWKV_OK;
@@ -1981,8 +1988,8 @@ constexpr TileDim tile_dim[TILES] = {{256, 256}, {128, 128}, {128, 128}, {64, 12
 //                       extra for what exceeds one round)
 //          + with a split, slab per 16 MB of fp32 slabs written and read and split per slab.
 // One fit per tile and type, over launches within 1.6 times the best one of 342 products each (18 lengths from 24 to 2048 rows, 19 widths
-// from 512 to 16384; weights from HBM; the chip under load before): the tile and split it picks takes 0.5 % (uint8) and 1.2 %
-// (fp16) longer than the best of all on average, 13 and 25 % at most.  A tile per round costs between 5 and 13 us whatever K is, so
+// from 512 to 16384; weights from HBM; the chip under load before): the tile and split it picks takes 0.6 % (uint8) and 1.1 %
+// (fp16) longer than the best of all on average.  A tile per round costs between 5 and 13 us whatever K is, so
 // tiles of many sizes pay: each of these is the best one somewhere, the ones with sides of 160, 192 and 224 where 256 x 256 or 128 x
 // 128 leave CUs idle or rows empty.  us, uint8 / fp16 weights: [1024 x 4096] x [4096 x 12288] three rounds of 128 x 128 115.7 / 132.5,
 // one of 256 x 192 90 / 97; [777 x 4096] x [4096 x 16384] 256 x 256 126 / 130, 224 x 256 100 / 107; [768 x 4096] x [4096 x 12288]
@@ -1990,37 +1997,37 @@ constexpr TileDim tile_dim[TILES] = {{256, 256}, {128, 128}, {128, 128}, {64, 12
 struct TilePrice { float launch, round, split_round, step_0, step_1, extra, slab, split; };
 constexpr TilePrice tile_price[2][TILES] = {
     {   // fp16 weights
-        {3.708f, 9.540f, 10.123f, 1.082f, 1.646f, -0.034f, 3.361f, 0.187f},   // 256x256
-        {3.602f, 2.757f, 3.837f, 0.442f, 0.611f, 0.008f, 5.384f, 0.127f},   // S
-        {2.318f, 4.510f, 4.717f, 0.327f, 0.562f, -0.021f, 7.471f, 0.249f},   // S4
-        {3.693f, 1.904f, 2.695f, 0.368f, 0.662f, 0.050f, 6.663f, 0.f},   // N
-        {2.217f, 2.471f, 4.018f, 0.151f, 0.255f, -0.038f, 6.035f, 0.232f},   // K8
-        {2.313f, 2.916f, 3.938f, 0.236f, 0.421f, -0.066f, 7.570f, 0.214f},   // K4
-        {2.492f, 11.106f, 9.222f, 0.863f, 1.307f, -0.029f, 3.933f, 0.054f},   // 256x192
-        {5.828f, 7.739f, 7.996f, 1.014f, 1.453f, -0.058f, 3.693f, 0.052f},   // 224x256
-        {1.500f, 9.906f, 8.848f, 0.769f, 1.229f, -0.063f, 3.795f, 0.134f},   // 224x192
-        {2.319f, 8.198f, 9.022f, 0.924f, 1.341f, -0.100f, 4.147f, 0.119f},   // 192x256
-        {1.500f, 7.879f, 8.029f, 0.677f, 1.136f, -0.093f, 4.020f, 0.115f},   // 192x192
-        {1.500f, 7.941f, 8.551f, 0.744f, 1.251f, -0.211f, 4.156f, 0.262f},   // 160x256
-        {3.484f, 4.923f, 5.617f, 0.601f, 1.136f, -0.080f, 3.797f, 0.106f},   // 160x192
-        {5.276f, 4.061f, 5.783f, 0.703f, 1.013f, 0.007f, 3.958f, 0.064f},   // 128x256
-        {3.435f, 5.320f, 4.890f, 0.556f, 0.818f, -0.009f, 6.064f, 0.088f},   // 128x192
+        {5.831f, 8.813f, 6.274f, 0.999f, 1.721f, 0.057f, 4.252f, 0.121f},   // 256x256
+        {2.012f, 3.875f, 4.591f, 0.415f, 0.619f, 0.008f, 5.344f, 0.221f},   // S
+        {1.500f, 4.656f, 4.697f, 0.295f, 0.569f, 0.f, 8.799f, 0.192f},   // S4
+        {3.105f, 1.893f, 2.537f, 0.343f, 0.679f, 0.f, 5.957f, 0.f},   // N
+        {1.794f, 2.270f, 3.851f, 0.149f, 0.240f, 0.f, 5.660f, 0.286f},   // K8
+        {1.905f, 2.896f, 3.736f, 0.230f, 0.387f, 0.f, 8.168f, 0.240f},   // K4
+        {3.022f, 10.904f, 7.859f, 0.832f, 1.358f, 0.f, 4.391f, 0.f},   // 256x192
+        {5.969f, 8.112f, 7.071f, 0.932f, 1.539f, 0.f, 3.668f, 0.091f},   // 224x256
+        {4.430f, 7.532f, 4.378f, 0.755f, 1.210f, 0.f, 4.956f, 0.152f},   // 224x192
+        {4.085f, 7.060f, 6.380f, 0.874f, 1.374f, 0.f, 4.356f, 0.188f},   // 192x256
+        {3.593f, 5.714f, 3.553f, 0.666f, 1.112f, 0.f, 5.118f, 0.311f},   // 192x192
+        {3.679f, 5.143f, 5.127f, 0.739f, 1.260f, 0.f, 4.542f, 0.330f},   // 160x256
+        {5.327f, 3.260f, 2.487f, 0.560f, 1.102f, 0.f, 4.280f, 0.251f},   // 160x192
+        {4.914f, 4.682f, 4.923f, 0.666f, 1.069f, 0.011f, 4.250f, 0.094f},   // 128x256
+        {3.239f, 5.415f, 4.335f, 0.532f, 0.829f, 0.006f, 5.058f, 0.207f},   // 128x192
     }, {   // uint8
-        {5.421f, 9.020f, 8.769f, 1.060f, 1.557f, 0.035f, 3.401f, 0.f},   // 256x256
-        {6.865f, 0.f, 1.265f, 0.368f, 0.545f, -0.069f, 4.173f, 0.112f},   // S
-        {5.254f, 3.096f, 3.291f, 0.325f, 0.487f, 0.080f, 4.998f, 0.145f},   // S4
-        {5.979f, 0.f, 0.f, 0.385f, 0.448f, -0.153f, 8.262f, 0.100f},   // N
-        {2.896f, 3.047f, 4.100f, 0.118f, 0.178f, 0.011f, 5.349f, 0.166f},   // K8
-        {3.277f, 2.970f, 3.735f, 0.204f, 0.297f, 0.032f, 7.355f, 0.128f},   // K4
-        {5.830f, 10.148f, 5.253f, 0.816f, 1.178f, 0.103f, 4.239f, 0.f},   // 256x192
-        {5.115f, 10.229f, 9.416f, 0.904f, 1.400f, -0.089f, 2.933f, 0.f},   // 224x256
-        {6.133f, 8.038f, 5.055f, 0.749f, 1.082f, 0.098f, 4.030f, 0.f},   // 224x192
-        {6.073f, 6.623f, 6.623f, 0.846f, 1.216f, 0.047f, 3.270f, 0.087f},   // 192x256
-        {6.485f, 6.782f, 3.426f, 0.603f, 0.936f, 0.129f, 4.279f, 0.044f},   // 192x192
-        {6.755f, 5.550f, 5.237f, 0.764f, 1.092f, 0.061f, 3.441f, 0.023f},   // 160x256
-        {6.725f, 5.622f, 3.040f, 0.535f, 0.854f, 0.116f, 4.004f, 0.077f},   // 160x192
-        {6.404f, 4.079f, 3.566f, 0.619f, 0.886f, 0.093f, 4.419f, 0.120f},   // 128x256
-        {6.151f, 3.907f, 2.421f, 0.540f, 0.721f, 0.089f, 5.413f, 0.129f},   // 128x192
+        {7.170f, 10.217f, 5.543f, 0.968f, 1.566f, 0.135f, 3.946f, 0.041f},   // 256x256
+        {6.880f, 0.f, 0.706f, 0.350f, 0.540f, 0.f, 4.587f, 0.162f},   // S
+        {4.450f, 3.447f, 2.539f, 0.315f, 0.506f, 0.078f, 6.311f, 0.207f},   // S4
+        {5.812f, 0.f, 0.f, 0.366f, 0.434f, 0.f, 7.064f, 0.099f},   // N
+        {2.045f, 2.974f, 4.338f, 0.117f, 0.181f, 0.011f, 4.108f, 0.195f},   // K8
+        {2.545f, 2.923f, 3.674f, 0.204f, 0.308f, 0.040f, 7.536f, 0.156f},   // K4
+        {6.193f, 9.593f, 4.232f, 0.804f, 1.215f, 0.128f, 4.631f, 0.f},   // 256x192
+        {7.017f, 9.153f, 6.790f, 0.867f, 1.441f, 0.065f, 3.205f, 0.f},   // 224x256
+        {5.264f, 9.053f, 5.484f, 0.692f, 1.136f, 0.036f, 4.223f, 0.f},   // 224x192
+        {5.750f, 7.695f, 7.373f, 0.748f, 1.266f, 0.077f, 3.127f, 0.016f},   // 192x256
+        {5.691f, 6.511f, 4.394f, 0.609f, 1.021f, 0.070f, 4.032f, 0.017f},   // 192x192
+        {5.144f, 6.870f, 6.213f, 0.706f, 1.125f, 0.046f, 3.505f, 0.076f},   // 160x256
+        {4.537f, 6.501f, 4.429f, 0.518f, 0.869f, 0.050f, 4.330f, 0.101f},   // 160x192
+        {7.339f, 3.059f, 2.299f, 0.598f, 0.967f, 0.109f, 4.353f, 0.040f},   // 128x256
+        {6.131f, 3.390f, 2.807f, 0.530f, 0.755f, 0.111f, 4.612f, 0.060f},   // 128x192
     }};
 double dma_cost(bool w_u8, int tile, int64_t T, int64_t tiles, int nk, int c, size_t out_bytes) {
     if (tile == TILE_N && T > 64) return 1e30;
