@@ -18,11 +18,11 @@ constexpr int DTHREADS = 1024;
 constexpr int DWAVES = DTHREADS / 64;
 constexpr int VP = 4;  // most 8-element groups per thread the vector prologue keeps in registers (N <= 32768)
 
-// x for this step: the embedding row of the token (first layer) or the running activation.  The id comes
+// x of the first layer: the embedding row of the token.  The id comes
 // from device memory (it may be the output of a sampling kernel); one outside [0, vocab) is clamped to the
 // nearest valid row, so a bad id can never become an out-of-bounds read.
-DEV const rwkv_half *resolve_x(const rwkv_half *x, const rwkv_half *emb, const int32_t *token, int C, int vocab) {
-    return token ? emb + (size_t)min(max(*token, 0), vocab - 1) * C : x;
+DEV const rwkv_half *token_row(const rwkv_half *emb, const int32_t *token, int C, int vocab) {
+    return emb + (size_t)min(max(*token, 0), vocab - 1) * C;
 }
 
 // LDS item (16 bytes = 8 halves) index of the 8-element group j8 of an activation vector.
@@ -34,6 +34,43 @@ struct MatDev {
     int64_t ld;
     const rwkv_half *mx, *rx, *my, *ry;
 };
+
+// Kernel arguments.  A wave's first loads wait for the addresses in them, and a read of the arguments is a trip to memory of its own:
+// left to the compiler these kernels read the sizes, waited, divided, read the matrices, waited, read the operands' addresses and
+// waited again, about 1 us of a launch of 5 to 18.  So the scalars and addresses needed first are leading arguments of their own, which
+// are in registers when a wave starts (-amdgpu-kernarg-preload-count), and the others are read together (`at_once`).  us a token, with
+// the division below taken out: RWKV-4 7B uint8 1836 -> 1740, RWKV-6 7B uint8 2500 -> 2349, RWKV-7 7B fp16 3054 -> 2920.
+template <int N>
+DEV void at_once(const void *(&p)[N]) {
+    static_assert(N == 2 || N == 3 || N == 4 || N == 6 || N == 8 || N == 9 || N == 12, "written out");
+    if constexpr (N == 2) asm volatile("" : "+s"(p[0]), "+s"(p[1]));
+    if constexpr (N == 3) asm volatile("" : "+s"(p[0]), "+s"(p[1]), "+s"(p[2]));
+    if constexpr (N == 4) asm volatile("" : "+s"(p[0]), "+s"(p[1]), "+s"(p[2]), "+s"(p[3]));
+    if constexpr (N == 6) asm volatile("" : "+s"(p[0]), "+s"(p[1]), "+s"(p[2]), "+s"(p[3]), "+s"(p[4]), "+s"(p[5]));
+    if constexpr (N == 8)
+        asm volatile("" : "+s"(p[0]), "+s"(p[1]), "+s"(p[2]), "+s"(p[3]), "+s"(p[4]), "+s"(p[5]), "+s"(p[6]), "+s"(p[7]));
+    if constexpr (N == 9)
+        asm volatile("" : "+s"(p[0]), "+s"(p[1]), "+s"(p[2]), "+s"(p[3]), "+s"(p[4]), "+s"(p[5]), "+s"(p[6]), "+s"(p[7]), "+s"(p[8]));
+    if constexpr (N == 12)
+        asm volatile("" : "+s"(p[0]), "+s"(p[1]), "+s"(p[2]), "+s"(p[3]), "+s"(p[4]), "+s"(p[5]), "+s"(p[6]), "+s"(p[7]), "+s"(p[8]),
+                     "+s"(p[9]), "+s"(p[10]), "+s"(p[11]));
+}
+
+// eight values through such an address, which the compiler no longer knows to be one of global memory
+DEV h16x8 load8(const void *p, int i) { return ((const __attribute__((address_space(1))) h16x8 *)p)[i]; }
+
+// The rows of a launch over its waves: wave w takes the groups [split_at(w), split_at(w + 1)), floor or ceil of ngroups / nwaves of
+// them, i.e. floor(w * ngroups / nwaves) = w q + floor(w r / nwaves), and the division is a multiplication (exact for w r < 2^26:
+// the factor is at most nwaves <= 2^13 too large in 2^40).  Two 64-bit divisions stood here, 250 instructions ahead of a wave's first load.
+struct RowSplit { uint64_t magic; int q, r; };
+inline RowSplit row_split(int64_t ngroups, int grid) {
+    const int64_t nwaves = (int64_t)grid * DWAVES;
+    return RowSplit{((uint64_t)1 << 40) / (uint64_t)nwaves + 1, (int)(ngroups / nwaves), (int)(ngroups % nwaves)};
+}
+#define RWKV_SPLIT_ARGS uint64_t split_magic, int split_q, int split_r
+#define RWKV_SPLIT (RowSplit{split_magic, split_q, split_r})
+#define RWKV_SPLIT_PASS(sp) (sp).magic, (sp).q, (sp).r
+DEV int split_at(const RowSplit &s, int wave) { return wave * s.q + (int)(((uint64_t)(uint32_t)(wave * s.r) * s.magic) >> 40); }
 
 // Sums of K values over the first `npw` waves of the workgroup (the waves that run a prologue), in two
 // halves with a synchronisation between them, which the caller places: `put` by each of those waves
@@ -118,17 +155,28 @@ struct LnMixPro {
         x = lw = lb = sx = h16x8{};
 #pragma unroll
         for (int j = 0; j < NJ; ++j) mix[j] = ry[j] = my[j] = h16x8{};
-        if (!own) return;
-        x = *(const h16x8 *)(xp + 8 * j8);
-        lw = *(const h16x8 *)(ln_w + 8 * j8);
-        lb = *(const h16x8 *)(ln_b + 8 * j8);
-        sx = *(const h16x8 *)((sxp ? sxp : ln_w) + 8 * j8);
+        if (own) {
+            x = *(const h16x8 *)(xp + 8 * j8);
+            lw = *(const h16x8 *)(ln_w + 8 * j8);
+            lb = *(const h16x8 *)(ln_b + 8 * j8);
+            sx = *(const h16x8 *)((sxp ? sxp : ln_w) + 8 * j8);
+        }
+        constexpr int NP = U8 ? 3 : 1;
+        const void *p[NP * NJ];
 #pragma unroll
         for (int j = 0; j < NJ; ++j) {
-            mix[j] = *(const h16x8 *)((mixp[j] ? mixp[j] : ln_w) + 8 * j8);
-            if (U8) {
-                ry[j] = *(const h16x8 *)(mat[j].ry + 8 * j8);
-                my[j] = *(const h16x8 *)(mat[j].my + 8 * j8);
+            p[NP * j] = mixp[j];
+            if (U8) { p[NP * j + 1] = mat[j].ry; p[NP * j + 2] = mat[j].my; }
+        }
+        if constexpr (NP * NJ > 1) at_once(p);
+        if (own) {
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) {
+                mix[j] = load8(p[NP * j] ? p[NP * j] : ln_w, j8);
+                if (U8) {
+                    ry[j] = load8(p[NP * j + 1], j8);
+                    my[j] = load8(p[NP * j + 2], j8);
+                }
             }
         }
     }
@@ -244,49 +292,55 @@ DEV float finish(float dot, const VecSums &S, float rx, float mx) {
 // per group batch), and read back when its last segment batch has been reduced.
 template <bool U8, int G, int K, int U, class E, bool PRO, class ProLoad, class ProCompute, class ProFinish, class RowFn,
           class EpiLoad, class EpiFn>
-DEV void stream_rows(int ngroups, int nseg, int npw, unsigned *sync, ProLoad pro_load, ProCompute pro_compute,
+DEV void stream_rows(const RowSplit &sp, int nseg, int npw, unsigned *sync, ProLoad pro_load, ProCompute pro_compute,
                      ProFinish pro_finish, RowFn rowf, EpiLoad epi_load, EpiFn epi) {
     constexpr int R = G * K;
     const int lane = threadIdx.x & 63;
     // the wave index through readfirstlane: the compiler then knows that everything derived from it (row
     // ranges, batch counters, loop control) is wave-uniform and keeps it in scalar registers
-    const int wave = blockIdx.x * DWAVES + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nwaves = gridDim.x * DWAVES;
-    // balanced split: every wave gets floor or ceil of ngroups / nwaves groups
-    const int g0 = (int)((int64_t)wave * ngroups / nwaves), g1 = (int)((int64_t)(wave + 1) * ngroups / nwaves);
-    const int glast = g1 > g0 ? g1 - 1 : min(g0, ngroups - 1);
+    const int wave = blockIdx.x * DWAVES + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int g0 = split_at(sp, wave), g1 = split_at(sp, wave + 1);
+    const int glast = g1 > g0 ? g1 - 1 : 0;
     const int nsb = (nseg + 64 * U - 1) / (64 * U);             // segment batches per group batch
-    const int nb = ((g1 - g0 + G - 1) / G) * nsb;               // batches of this wave
     const int sb_epi = nsb > 1 ? 1 : 0;                         // segment batch that carries the epilogue operands
+    const int odd_epi = (nsb - 1 + sb_epi) & 1;                 // 1: it and the last segment batch are in different tiles
     RowTile<U8, R, U> t0, t1;
     E e0{}, e1{};
-    auto load = [&](RowTile<U8, R, U> &t, E &e, int q) {
-        const bool real = q < nb;
-        const int gbi = q / nsb, gb = g0 + gbi * G, sb = q - gbi * nsb;
-        const uint8_t *rows[R];
+    struct Cursor { int gb, sb; };                              // first group and segment batch of a batch
+    Cursor lc = {g0, 0}, pc = {g0, 0};                          // of the next one to load, to process
+    auto next = [&](Cursor &c) {
+        if (++c.sb == nsb) { c.sb = 0; c.gb += G; }
+    };
+    auto rows_of = [&](const uint8_t *(&rows)[R]) {
         const h16 *xs_unused;
 #pragma unroll
         for (int i = 0; i < G; ++i)
 #pragma unroll
-            for (int k = 0; k < K; ++k) rowf(min(gb + i, glast), k, rows[i * K + k], xs_unused);
-        if (real && sb == sb_epi) e = epi_load(min(gb + min(lane, G - 1), glast));
-        t.load(rows, sb * 64 * U, nseg, real);
+            for (int k = 0; k < K; ++k) rowf(min(lc.gb + i, glast), k, rows[i * K + k], xs_unused);
+    };
+    auto load = [&](RowTile<U8, R, U> &t, E &e) {
+        const bool real = lc.gb < g1;
+        const uint8_t *rows[R];
+        rows_of(rows);
+        if (real && lc.sb == sb_epi) e = epi_load(min(lc.gb + min(lane, G - 1), glast));
+        t.load(rows, lc.sb * 64 * U, nseg, real);
+        next(lc);
     };
     float acc[R];
 #pragma unroll
     for (int r = 0; r < R; ++r) acc[r] = 0.f;
-    auto process = [&](const RowTile<U8, R, U> &t, int q) {
-        const int gbi = q / nsb, sb = q - gbi * nsb, gb = g0 + gbi * G;
+    auto process = [&](const RowTile<U8, R, U> &t, int odd) {
         const uint8_t *row_unused;
         const h16 *xs[R];
 #pragma unroll
         for (int i = 0; i < G; ++i)
 #pragma unroll
-            for (int k = 0; k < K; ++k) rowf(min(gb + i, glast), k, row_unused, xs[i * K + k]);
-        t.consume(xs, sb * 64 * U, nseg, acc);
-        if (sb == nsb - 1) {
+            for (int k = 0; k < K; ++k) rowf(min(pc.gb + i, glast), k, row_unused, xs[i * K + k]);
+        t.consume(xs, pc.sb * 64 * U, nseg, acc);
+        if (pc.sb == nsb - 1) {
 #pragma unroll
             for (int r = 0; r < R; ++r) acc[r] = wave_sum(acc[r]);
-            if (lane < G && gb + lane < g1) {
+            if (lane < G && pc.gb + lane < g1) {
                 float d[K];
 #pragma unroll
                 for (int k = 0; k < K; ++k) {
@@ -294,11 +348,12 @@ DEV void stream_rows(int ngroups, int nseg, int npw, unsigned *sync, ProLoad pro
 #pragma unroll
                     for (int i = 1; i < G; ++i) d[k] = (lane == i) ? acc[i * K + k] : d[k];
                 }
-                epi(gb + lane, d, ((q - (nsb - 1) + sb_epi) & 1) ? e1 : e0);
+                epi(pc.gb + lane, d, odd ^ odd_epi ? e1 : e0);
             }
 #pragma unroll
             for (int r = 0; r < R; ++r) acc[r] = 0.f;
         }
+        next(pc);
     };
     // Waves whose threads hold prologue operands request them, run the prologue and fetch their first tile
     // after it.  The other waves request their first tile at once, which keeps HBM busy meanwhile, and then
@@ -321,35 +376,37 @@ DEV void stream_rows(int ngroups, int nseg, int npw, unsigned *sync, ProLoad pro
         if (threadIdx.x == 0) { sync[0] = 0; sync[1] = 0; }
         if (pro_wave) {
             pro_load();
+            __builtin_amdgcn_sched_barrier(0);   // nothing that waits for an operand goes ahead of the barrier
             __syncthreads();
+            __builtin_amdgcn_sched_barrier(0);
             pro_compute();
-            load(t0, e0, 0);
+            load(t0, e0);
         } else {
             __syncthreads();
-            load(t0, e0, 0);
+            load(t0, e0);
         }
         pro_wait(&sync[1], (unsigned)npw);
         pro_finish();
     } else {
-        load(t0, e0, 0);
+        load(t0, e0);
     }
-    for (int q = 0; q < nb; q += 2) {
-        load(t1, e1, q + 1);
-        process(t0, q);
-        load(t0, e0, q + 2);
-        if (q + 1 < nb) process(t1, q + 1);
+    while (pc.gb < g1) {
+        load(t1, e1);
+        process(t0, 0);
+        load(t0, e0);
+        if (pc.gb < g1) process(t1, 1);
     }
 }
 
 // ------------------------------------------------------------------------------------------
 struct AttArgs {
-    const rwkv_half *x, *emb;
-    const int32_t *token;
-    int C, vocab;
-    const rwkv_half *ln_w, *ln_b, *sx;
-    rwkv_half *xx_tmp;
     const rwkv_half *mix[3];  // k, v, r
     MatDev mat[3];            // key, value, receptance
+    rwkv_half *xx_tmp;
+    const rwkv_half *x, *ln_w, *ln_b, *sx, *emb;
+    const int32_t *token;
+    rwkv_half *x_out;         // FIRST: x, for the launches that follow
+    int C, vocab;
     const float *decay, *first;
     float *aa, *bb, *pp;
     rwkv_half *rwkv;          // out: r * wkv, fp16 [C]
@@ -360,19 +417,23 @@ struct AttEpi {
     float u, w, aa, bb, pp;
 };
 
-template <bool U8, int G>
-__global__ __launch_bounds__(DTHREADS) void att_kernel(AttArgs a) {
+// FIRST: the first layer, whose x is the token's embedding row
+template <bool U8, int G, bool FIRST>
+__global__ __launch_bounds__(DTHREADS) void att_kernel(const rwkv_half *x, const rwkv_half *ln_w, const rwkv_half *ln_b, const rwkv_half *sx,
+                                                       RWKV_SPLIT_ARGS, int C, AttArgs a) {
     extern __shared__ __align__(16) unsigned char smem[];
     __shared__ float red[(2 + 9) * DWAVES];
     __shared__ unsigned sync[2];
-    const int C = a.C;
     h16 *xs[3] = {(h16 *)smem, (h16 *)smem + C, (h16 *)smem + 2 * C};
     VecSums S[3];
     LnMixPro<U8, 3> pro;
     auto pro_load = [&]() {
-        pro.load(resolve_x(a.x, a.emb, a.token, C, a.vocab), C, a.ln_w, a.ln_b, a.sx, a.mix, a.mat);
+        pro.load(FIRST ? token_row(a.emb, a.token, C, a.vocab) : x, C, ln_w, ln_b, sx, a.mix, a.mat);
     };
-    auto pro_compute = [&]() { pro.compute(C, a.sx != nullptr, a.mix, xs, a.xx_tmp, red, sync); };
+    auto pro_compute = [&]() {
+        pro.compute(C, sx != nullptr, a.mix, xs, a.xx_tmp, red, sync);
+        if (FIRST && pro.own && blockIdx.x == 0) *(h16x8 *)(a.x_out + 8 * threadIdx.x) = pro.x;   // the residual of the launches that follow
+    };
     auto pro_finish = [&]() { LnMixPro<U8, 3>::finish(C, S, red); };
     auto rowf = [&](int c, int k, const uint8_t *&row, const h16 *&xv) {
         row = row_ptr<U8>(a.mat[k], c);
@@ -406,7 +467,7 @@ __global__ __launch_bounds__(DTHREADS) void att_kernel(AttArgs a) {
         a.pp[c] = p;
         a.rwkv[c] = f2h(r * round_h(wkv));
     };
-    stream_rows<U8, G, 3, 2, AttEpi, true>(C, (C * (U8 ? 1 : 2)) >> 4, pro_waves(C >> 3), sync, pro_load, pro_compute, pro_finish,
+    stream_rows<U8, G, 3, 2, AttEpi, true>(RWKV_SPLIT, (C * (U8 ? 1 : 2)) >> 4, pro_waves(C >> 3), sync, pro_load, pro_compute, pro_finish,
                                            rowf, epi_load, epi);
 }
 
@@ -414,12 +475,11 @@ __global__ __launch_bounds__(DTHREADS) void att_kernel(AttArgs a) {
 enum { EPI_SIGMOID = 0, EPI_RELU_SQ = 1, EPI_LOGITS = 2, EPI_TANH = 3 };
 
 struct LnMixArgs {
-    const rwkv_half *x;
-    int C;
-    const rwkv_half *ln_w, *ln_b, *sx;
-    rwkv_half *xx_tmp;
     const rwkv_half *mix[2];
     MatDev mat[2];
+    rwkv_half *xx_tmp;
+    const rwkv_half *x, *ln_w, *ln_b, *sx;
+    int C;
     int M[2];
     int epi[2];
     void *out[2];
@@ -431,21 +491,20 @@ struct ScaleEpi {
 };
 
 template <bool U8, int NJ, int G>
-__global__ __launch_bounds__(DTHREADS) void lnmix_kernel(LnMixArgs a) {
+__global__ __launch_bounds__(DTHREADS) void lnmix_kernel(const rwkv_half *x, const rwkv_half *ln_w, const rwkv_half *ln_b, const rwkv_half *sx,
+                                                         RWKV_SPLIT_ARGS, int C, int M0, LnMixArgs a) {
     extern __shared__ __align__(16) unsigned char smem[];
     __shared__ float red[(2 + 3 * NJ) * DWAVES];
     __shared__ unsigned sync[2];
-    const int C = a.C;
     h16 *xs[NJ];
     const rwkv_half *mix[NJ];
     MatDev mat[NJ];
 #pragma unroll
     for (int j = 0; j < NJ; ++j) { xs[j] = (h16 *)smem + j * C; mix[j] = a.mix[j]; mat[j] = a.mat[j]; }
     VecSums S[NJ];
-    const int M0 = a.M[0];
     LnMixPro<U8, NJ> pro;
-    auto pro_load = [&]() { pro.load(a.x, C, a.ln_w, a.ln_b, a.sx, mix, mat); };
-    auto pro_compute = [&]() { pro.compute(C, a.sx != nullptr, mix, xs, a.xx_tmp, red, sync, a.maa_form != 0); };
+    auto pro_load = [&]() { pro.load(x, C, ln_w, ln_b, sx, mix, mat); };
+    auto pro_compute = [&]() { pro.compute(C, sx != nullptr, mix, xs, a.xx_tmp, red, sync, a.maa_form != 0); };
     auto pro_finish = [&]() { LnMixPro<U8, NJ>::finish(C, S, red); };
     auto rowf = [&](int g, int, const uint8_t *&row, const h16 *&xv) {
         const int j = (NJ > 1 && g >= M0) ? 1 : 0;
@@ -475,19 +534,18 @@ __global__ __launch_bounds__(DTHREADS) void lnmix_kernel(LnMixArgs a) {
             ((rwkv_half *)a.out[j])[m] = f2h(t * t);
         }
     };
-    stream_rows<U8, G, 1, (G >= 4 ? 1 : 2), ScaleEpi, true>(M0 + (NJ > 1 ? a.M[1] : 0), (C * (U8 ? 1 : 2)) >> 4,
+    stream_rows<U8, G, 1, (G >= 4 ? 1 : 2), ScaleEpi, true>(RWKV_SPLIT, (C * (U8 ? 1 : 2)) >> 4,
                                                             pro_waves(C >> 3), sync, pro_load, pro_compute, pro_finish, rowf,
                                                             epi_load, epi);
 }
 
 // ------------------------------------------------------------------------------------------
 struct VecArgs {
+    MatDev mat;
     const rwkv_half *vin;   // [N] fp16 input vector
     int N, M;
-    MatDev mat;
-    const rwkv_half *x_in, *emb;  // residual source (emb row when token != NULL)
-    const int32_t *token;
-    int C, vocab;
+    const rwkv_half *x_in;  // residual source
+    int C;
     const rwkv_half *gate;  // [M] or NULL
     rwkv_half *x_out;       // [M]
     float out_scale;
@@ -509,11 +567,11 @@ struct VecEpi {
 // The prologue is done by the first OW waves, VPN 8-element groups of the input vector per thread
 // (N <= 512 * OW * VPN); the other waves already stream weights meanwhile.
 template <bool U8, int U, int VPN, int OW>
-__global__ __launch_bounds__(DTHREADS) void vec_kernel(VecArgs a) {
+__global__ __launch_bounds__(DTHREADS) void vec_kernel(const rwkv_half *vin, const rwkv_half *ry, const rwkv_half *my, const void *w,
+                                                       RWKV_SPLIT_ARGS, int N, int M, VecArgs a) {
     extern __shared__ __align__(16) unsigned char smem[];
     __shared__ float red[3 * DWAVES];
     __shared__ unsigned sync[2];
-    const int N = a.N;
     h16 *xs = (h16 *)smem;
     VecSums S;
     h16x8 pv[VPN], pr[VPN], pm[VPN];
@@ -522,10 +580,10 @@ __global__ __launch_bounds__(DTHREADS) void vec_kernel(VecArgs a) {
         for (int i = 0; i < VPN; ++i) {
             const int j8 = threadIdx.x + i * 64 * OW;
             if ((int)threadIdx.x < 64 * OW && j8 < (N >> 3)) {
-                pv[i] = *(const h16x8 *)(a.vin + 8 * j8);
+                pv[i] = *(const h16x8 *)(vin + 8 * j8);
                 if (U8) {
-                    pr[i] = *(const h16x8 *)(a.mat.ry + 8 * j8);
-                    pm[i] = *(const h16x8 *)(a.mat.my + 8 * j8);
+                    pr[i] = *(const h16x8 *)(ry + 8 * j8);
+                    pm[i] = *(const h16x8 *)(my + 8 * j8);
                 }
             }
         }
@@ -562,14 +620,15 @@ __global__ __launch_bounds__(DTHREADS) void vec_kernel(VecArgs a) {
         wave_sums_get<3>(acc, red, npw);
         S.s0 = acc[0]; S.s1 = acc[1]; S.s2 = acc[2];
     };
+    const MatDev mat = {w, a.mat.ld, a.mat.mx, a.mat.rx, my, ry};
     auto rowf = [&](int m, int, const uint8_t *&row, const h16 *&xv) {
-        row = row_ptr<U8>(a.mat, m);
+        row = row_ptr<U8>(mat, m);
         xv = xs;
     };
     auto epi_load = [&](int m) {
         VecEpi e{};
         if (U8) { e.rx = a.mat.rx[m]; e.mx = a.mat.mx[m]; }
-        if (a.act == VACT_RESIDUAL) e.xin = resolve_x(a.x_in, a.emb, a.token, a.C, a.vocab)[m];
+        if (a.act == VACT_RESIDUAL) e.xin = a.x_in[m];
         if (a.gate) e.gate = a.gate[m];
         return e;
     };
@@ -592,7 +651,7 @@ __global__ __launch_bounds__(DTHREADS) void vec_kernel(VecArgs a) {
         }
         ((rwkv_half *)a.out)[m] = f2h(o);
     };
-    stream_rows<U8, 1, 1, U, VecEpi, true>(a.M, (N * (U8 ? 1 : 2)) >> 4, npw, sync, pro_load, pro_compute, pro_finish, rowf, epi_load,
+    stream_rows<U8, 1, 1, U, VecEpi, true>(RWKV_SPLIT, (N * (U8 ? 1 : 2)) >> 4, npw, sync, pro_load, pro_compute, pro_finish, rowf, epi_load,
                                            epi);
     // the token-shift state every workgroup of the previous launch read: committed after this workgroup's
     // rows, so that the copy's load -> store dependency does not sit in front of the weight stream
@@ -605,9 +664,9 @@ __global__ __launch_bounds__(DTHREADS) void vec_kernel(VecArgs a) {
 // Several GEMVs of the same shape [N -> M] in one launch, each with its own input vector
 // (RWKV-5/6 time mix: receptance, key, value and gate rows over the r/k/v/g mixes).
 struct MultiVecArgs {
-    int N, M, nm;                // nm matrices (<= 4)
     const rwkv_half *vin[4];     // [N] fp16 each
     MatDev mat[4];
+    int N, M, nm;                // nm matrices (<= 4)
     int act[4];                  // VACT_F16 / VACT_SILU / VACT_SIGMOID ...
     rwkv_half *out[4];           // [M] fp16 each
     const rwkv_half *commit_src; // scratch xx -> token-shift state, done by workgroup 0
@@ -617,6 +676,7 @@ struct MultiVecArgs {
     // (RWKV-6: the first decay-LoRA stage), NULL = none
     const rwkv_half *xin, *xmat;
     int xm;
+    RowSplit xsplit;             // set by the launch
     rwkv_half *xout;             // [xm]
 };
 
@@ -624,11 +684,11 @@ struct NoEpi {};
 
 // NM input vectors of N <= 4096 elements (one 8-element group per thread of the first 8 waves).
 template <bool U8, int NM>
-__global__ __launch_bounds__(DTHREADS) void multi_vec_kernel(MultiVecArgs a) {
+__global__ __launch_bounds__(DTHREADS) void multi_vec_kernel(const rwkv_half *v0, const rwkv_half *v1, const rwkv_half *v2, const rwkv_half *v3,
+                                                             RWKV_SPLIT_ARGS, int N, int M, MultiVecArgs a) {
     extern __shared__ __align__(16) unsigned char smem[];
     __shared__ float red[3 * NM * DWAVES];
     __shared__ unsigned sync[2];
-    const int N = a.N, M = a.M;
     h16 *xs[NM];
 #pragma unroll
     for (int j = 0; j < NM; ++j) xs[j] = (h16 *)smem + (size_t)j * N;
@@ -640,15 +700,21 @@ __global__ __launch_bounds__(DTHREADS) void multi_vec_kernel(MultiVecArgs a) {
 #pragma unroll
         for (int j = 0; j < NM; ++j) pv[j] = pr[j] = pm[j] = h16x8{};
         if (!own) return;
-        px = *(const h16x8 *)((a.xin ? a.xin : a.vin[0]) + 8 * threadIdx.x);
+        const rwkv_half *const vin[4] = {v0, v1, v2, v3};
 #pragma unroll
-        for (int j = 0; j < NM; ++j) {
-            pv[j] = *(const h16x8 *)(a.vin[j] + 8 * threadIdx.x);
-            if (U8) {
-                pr[j] = *(const h16x8 *)(a.mat[j].ry + 8 * threadIdx.x);
-                pm[j] = *(const h16x8 *)(a.mat[j].my + 8 * threadIdx.x);
+        for (int j = 0; j < NM; ++j) pv[j] = *(const h16x8 *)(vin[j] + 8 * threadIdx.x);
+        if (U8) {
+            const void *p[2 * NM];
+#pragma unroll
+            for (int j = 0; j < NM; ++j) { p[2 * j] = a.mat[j].ry; p[2 * j + 1] = a.mat[j].my; }
+            at_once(p);
+#pragma unroll
+            for (int j = 0; j < NM; ++j) {
+                pr[j] = load8(p[2 * j], threadIdx.x);
+                pm[j] = load8(p[2 * j + 1], threadIdx.x);
             }
         }
+        px = *(const h16x8 *)((a.xin ? a.xin : v0) + 8 * threadIdx.x);
     };
     auto pro_compute = [&]() {
         const int nseg = N >> 4;
@@ -710,7 +776,7 @@ __global__ __launch_bounds__(DTHREADS) void multi_vec_kernel(MultiVecArgs a) {
             a.out[k][m] = f2h(o);
         }
     };
-    stream_rows<U8, 1, NM, 2, Epi, true>(M, (N * (U8 ? 1 : 2)) >> 4, pro_waves(N >> 3), sync, pro_load, pro_compute, pro_finish, rowf,
+    stream_rows<U8, 1, NM, 2, Epi, true>(RWKV_SPLIT, (N * (U8 ? 1 : 2)) >> 4, pro_waves(N >> 3), sync, pro_load, pro_compute, pro_finish, rowf,
                                          epi_load, epi);
     if (a.xmat) {
         auto rowf2 = [&](int g, int, const uint8_t *&row, const h16 *&xv) {
@@ -719,38 +785,49 @@ __global__ __launch_bounds__(DTHREADS) void multi_vec_kernel(MultiVecArgs a) {
         };
         auto epi_load2 = [&](int) { return NoEpi{}; };
         auto epi2 = [&](int g, const float (&d)[1], const NoEpi &) { a.xout[g] = f2h(tanhf(round_h(d[0]))); };
-        stream_rows<false, 1, 1, 2, NoEpi, false>(a.xm, (N * 2) >> 4, 0, nullptr, [] {}, [] {}, [] {}, rowf2, epi_load2, epi2);
+        stream_rows<false, 1, 1, 2, NoEpi, false>(a.xsplit, (N * 2) >> 4, 0, nullptr, [] {}, [] {}, [] {}, rowf2, epi_load2, epi2);
     }
     if (blockIdx.x == 0 && a.commit_dst)
         for (int j8 = threadIdx.x; j8 < (a.commit_n >> 3); j8 += blockDim.x)
             *(u32x4 *)(a.commit_dst + 8 * j8) = *(const u32x4 *)(a.commit_src + 8 * j8);
 }
 
-inline void multi_vec_launch(bool u8, const MultiVecArgs &a, int grid, hipStream_t st) {
+#define RWKV_MULTI_VEC(U8, NM)                                                                                                       \
+    hipLaunchKernelGGL((multi_vec_kernel<U8, NM>), dim3(grid), dim3(DTHREADS), lds, st, a.vin[0], a.vin[1], a.vin[2], a.vin[3],      \
+                       RWKV_SPLIT_PASS(sp), a.N, a.M, a)
+inline void multi_vec_launch(bool u8, MultiVecArgs a, int grid, hipStream_t st) {
     const size_t lds = (size_t)(a.nm + 1) * a.N * 2;
+    const RowSplit sp = row_split(a.M, grid);
+    a.xsplit = row_split(a.xm, grid);
     if (a.nm == 4) {
-        if (u8) hipLaunchKernelGGL((multi_vec_kernel<true, 4>), dim3(grid), dim3(DTHREADS), lds, st, a);
-        else hipLaunchKernelGGL((multi_vec_kernel<false, 4>), dim3(grid), dim3(DTHREADS), lds, st, a);
+        if (u8) RWKV_MULTI_VEC(true, 4);
+        else RWKV_MULTI_VEC(false, 4);
     } else {
-        if (u8) hipLaunchKernelGGL((multi_vec_kernel<true, 3>), dim3(grid), dim3(DTHREADS), lds, st, a);
-        else hipLaunchKernelGGL((multi_vec_kernel<false, 3>), dim3(grid), dim3(DTHREADS), lds, st, a);
+        if (u8) RWKV_MULTI_VEC(true, 3);
+        else RWKV_MULTI_VEC(false, 3);
     }
+}
+
+template <bool U8, int NJ, int G>
+inline void lnmix_start(const LnMixArgs &a, int grid, hipStream_t st) {
+    const RowSplit sp = row_split((int64_t)a.M[0] + (NJ > 1 ? a.M[1] : 0), grid);
+    hipLaunchKernelGGL((lnmix_kernel<U8, NJ, G>), dim3(grid), dim3(DTHREADS), NJ * (size_t)a.C * 2, st, a.x, a.ln_w, a.ln_b, a.sx,
+                       RWKV_SPLIT_PASS(sp), a.C, a.M[0], a);
 }
 
 // LN + token shift + two GEMVs (channel-mix receptance and key) in one launch; picks the tile depth that
 // divides a wave's share of the rows.
 inline void lnmix2_launch(bool u8, const LnMixArgs &a, int grid, hipStream_t st) {
-    const size_t lds = 2 * (size_t)a.C * 2;
     const int per = (a.M[0] + a.M[1] + grid * DWAVES - 1) / (grid * DWAVES);
     if (per % 5 == 0) {
-        if (u8) hipLaunchKernelGGL((lnmix_kernel<true, 2, 5>), dim3(grid), dim3(DTHREADS), lds, st, a);
-        else hipLaunchKernelGGL((lnmix_kernel<false, 2, 5>), dim3(grid), dim3(DTHREADS), lds, st, a);
+        if (u8) lnmix_start<true, 2, 5>(a, grid, st);
+        else lnmix_start<false, 2, 5>(a, grid, st);
     } else if (per >= 4) {
-        if (u8) hipLaunchKernelGGL((lnmix_kernel<true, 2, 4>), dim3(grid), dim3(DTHREADS), lds, st, a);
-        else hipLaunchKernelGGL((lnmix_kernel<false, 2, 4>), dim3(grid), dim3(DTHREADS), lds, st, a);
+        if (u8) lnmix_start<true, 2, 4>(a, grid, st);
+        else lnmix_start<false, 2, 4>(a, grid, st);
     } else {
-        if (u8) hipLaunchKernelGGL((lnmix_kernel<true, 2, 2>), dim3(grid), dim3(DTHREADS), lds, st, a);
-        else hipLaunchKernelGGL((lnmix_kernel<false, 2, 2>), dim3(grid), dim3(DTHREADS), lds, st, a);
+        if (u8) lnmix_start<true, 2, 2>(a, grid, st);
+        else lnmix_start<false, 2, 2>(a, grid, st);
     }
 }
 
@@ -758,14 +835,13 @@ inline void lnmix2_launch(bool u8, const LnMixArgs &a, int grid, hipStream_t st)
 // the data-dependent mixes), one row per wave.
 inline void lnmix1_small_launch(const LnMixArgs &a, hipStream_t st) {
     const int grid = (a.M[0] + DWAVES - 1) / DWAVES;
-    hipLaunchKernelGGL((lnmix_kernel<false, 1, 1>), dim3(grid), dim3(DTHREADS), (size_t)a.C * 2, st, a);
+    lnmix_start<false, 1, 1>(a, grid, st);
 }
 
 // LN + token shift + one mix + a GEMV over the rows of one large matrix.
 inline void lnmix1_launch(bool u8, const LnMixArgs &a, int grid, hipStream_t st) {
-    const size_t lds = (size_t)a.C * 2;
-    if (u8) hipLaunchKernelGGL((lnmix_kernel<true, 1, 4>), dim3(grid), dim3(DTHREADS), lds, st, a);
-    else hipLaunchKernelGGL((lnmix_kernel<false, 1, 4>), dim3(grid), dim3(DTHREADS), lds, st, a);
+    if (u8) lnmix_start<true, 1, 4>(a, grid, st);
+    else lnmix_start<false, 1, 4>(a, grid, st);
 }
 
 // LN_out(x) @ head -> fp32 logits (fp16-rounded values) in one launch.
@@ -774,20 +850,21 @@ inline void lnhead_launch(bool u8, const rwkv_half *x, int C, const rwkv_half *l
     LnMixArgs h{};
     h.x = x; h.C = C; h.ln_w = ln_w; h.ln_b = ln_b; h.sx = nullptr; h.xx_tmp = nullptr;
     h.mix[0] = nullptr; h.mat[0] = head; h.M[0] = vocab; h.epi[0] = EPI_LOGITS; h.out[0] = logits;
-    const size_t lds = (size_t)C * 2;
-    if (u8) hipLaunchKernelGGL((lnmix_kernel<true, 1, 4>), dim3(grid), dim3(DTHREADS), lds, st, h);
-    else hipLaunchKernelGGL((lnmix_kernel<false, 1, 4>), dim3(grid), dim3(DTHREADS), lds, st, h);
+    if (u8) lnmix_start<true, 1, 4>(h, grid, st);
+    else lnmix_start<false, 1, 4>(h, grid, st);
 }
 
 // Launches the vector GEMV with the tile depth and prologue shape that fit N (N <= 8192 * VP).
 #define RWKV_VEC_CASE(U, VPN, OW)                                                                              \
     do {                                                                                                       \
-        if (u8) hipLaunchKernelGGL((vec_kernel<true, U, VPN, OW>), dim3(grid), dim3(DTHREADS), lds, st, a);    \
-        else hipLaunchKernelGGL((vec_kernel<false, U, VPN, OW>), dim3(grid), dim3(DTHREADS), lds, st, a);     \
+        const auto kernel = u8 ? vec_kernel<true, U, VPN, OW> : vec_kernel<false, U, VPN, OW>;                 \
+        hipLaunchKernelGGL(kernel, dim3(grid), dim3(DTHREADS), lds, st, a.vin, a.mat.ry, a.mat.my, a.mat.w,    \
+                           RWKV_SPLIT_PASS(sp), a.N, a.M, a);                                                  \
     } while (0)
 inline void vec_launch(bool u8, const VecArgs &a, int grid, hipStream_t st) {
     const size_t lds = (size_t)a.N * 2;
     const int groups = a.N >> 3;
+    const RowSplit sp = row_split(a.M, grid);
     if (groups <= 512) RWKV_VEC_CASE(4, 1, 8);
     else if (groups <= 1024) RWKV_VEC_CASE(4, 2, 8);
     else if (groups <= 2048) RWKV_VEC_CASE(8, 4, 8);

@@ -136,21 +136,23 @@ static int v4_one_impl(const rwkv_v4_model *m, const rwkv_v4_layer_state *states
         const bool u8 = mat_is_u8(m->weights_u8, l.att_key);
         if (only_phase < 0 || only_phase == 0) {
             AttArgs a{};
-            a.x = ws.x; a.emb = m->emb; a.token = tok; a.C = C; a.vocab = m->vocab;
+            a.x = ws.x; a.emb = m->emb; a.token = tok; a.x_out = ws.x; a.C = C; a.vocab = m->vocab;
             a.ln_w = l.ln1_w; a.ln_b = l.ln1_b; a.sx = s.att_xx; a.xx_tmp = ws.xx_att;
             a.mix[0] = l.att_mix_k; a.mix[1] = l.att_mix_v; a.mix[2] = l.att_mix_r;
             a.mat[0] = to_dev(l.att_key); a.mat[1] = to_dev(l.att_value); a.mat[2] = to_dev(l.att_receptance);
             a.decay = l.time_decay; a.first = l.time_first; a.aa = s.aa; a.bb = s.bb; a.pp = s.pp;
             a.rwkv = ws.rwkv;
             const size_t lds = 3 * (size_t)C * 2;
-            if (u8) hipLaunchKernelGGL((att_kernel<true, 1>), dim3(grid), dim3(DTHREADS), lds, st, a);
-            else hipLaunchKernelGGL((att_kernel<false, 1>), dim3(grid), dim3(DTHREADS), lds, st, a);
+            const RowSplit sp = row_split(C, grid);
+            const auto kernel = u8 ? (tok ? att_kernel<true, 1, true> : att_kernel<true, 1, false>)
+                                   : (tok ? att_kernel<false, 1, true> : att_kernel<false, 1, false>);
+            hipLaunchKernelGGL(kernel, dim3(grid), dim3(DTHREADS), lds, st, a.x, a.ln_w, a.ln_b, a.sx, RWKV_SPLIT_PASS(sp), C, a);
             mark();
         }
         if (only_phase < 0 || only_phase == 1) {
             VecArgs a{};
             a.vin = ws.rwkv; a.N = C; a.M = C; a.mat = to_dev(l.att_output);
-            a.x_in = ws.x; a.emb = m->emb; a.token = tok; a.C = C; a.vocab = m->vocab; a.gate = nullptr; a.x_out = ws.x;
+            a.x_in = ws.x; a.C = C; a.gate = nullptr; a.x_out = ws.x;
             a.out_scale = 1.f; a.commit_src = ws.xx_att; a.commit_dst = s.att_xx; a.act = VACT_RESIDUAL;
             vec_launch(u8, a, grid, st);
             mark();
@@ -168,7 +170,7 @@ static int v4_one_impl(const rwkv_v4_model *m, const rwkv_v4_layer_state *states
         if (only_phase < 0 || only_phase == 3) {
             VecArgs a{};
             a.vin = ws.vx; a.N = F; a.M = C; a.mat = to_dev(l.ffn_value);
-            a.x_in = ws.x; a.emb = nullptr; a.token = nullptr; a.C = C; a.gate = ws.r_ffn; a.x_out = ws.x;
+            a.x_in = ws.x; a.C = C; a.gate = ws.r_ffn; a.x_out = ws.x;
             a.out_scale = (m->rescale_layer > 0 && (i + 1) % m->rescale_layer == 0) ? 0.5f : 1.f;
             a.commit_src = ws.xx_ffn; a.commit_dst = s.ffn_xx; a.act = VACT_RESIDUAL;
             vec_launch(u8, a, grid, st);

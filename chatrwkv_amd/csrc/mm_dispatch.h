@@ -28,7 +28,7 @@ inline int mm(const Ctx &c, const rwkv_mat &m, bool mat_u8, const rwkv_half *x, 
     if (c.T == 1) {
         VecArgs a{};
         a.vin = x; a.N = N; a.M = M; a.mat = to_dev56(m);
-        a.x_in = res; a.emb = nullptr; a.token = nullptr; a.C = commit_n; a.gate = gate; a.x_out = out;
+        a.x_in = res; a.C = commit_n; a.gate = gate; a.x_out = out;
         a.out_scale = out_scale; a.commit_src = commit_src; a.commit_dst = commit_dst; a.out = out;
         switch (act) {
             case ACT_NONE: a.act = VACT_F16; break;

@@ -673,30 +673,30 @@ __global__ __launch_bounds__(256) void gn7_kernel(int T, int C, const float *__r
 
 // ---- one-token kernels ---------------------------------------------------------------------
 struct Att7Args {
-    const rwkv_half *x;
-    int C;
-    const rwkv_half *ln_w, *ln_b, *sx;
-    rwkv_half *xx_tmp;
     const rwkv_half *mix[6];   // r, w, k, v, a, g
     MatDev mat[3];             // receptance, key, value
+    rwkv_half *xx_tmp;
+    const rwkv_half *x, *ln_w, *ln_b, *sx;
+    int C;
+    RowSplit lsplit;           // of the rtot rows
     rwkv_half *out[3];         // r, k, v  [C]
     const rwkv_half *lora1;    // [rtot][C]
     int rtot, o_a, o_v, o_g;   // rows, first row of the a / v / g blocks
     rwkv_half *l1;             // [rtot] activated first-stage outputs
 };
 
-__global__ __launch_bounds__(DTHREADS) void att7_kernel(Att7Args a) {
+__global__ __launch_bounds__(DTHREADS) void att7_kernel(const rwkv_half *x, const rwkv_half *ln_w, const rwkv_half *ln_b, const rwkv_half *sx,
+                                                        RWKV_SPLIT_ARGS, int C, Att7Args a) {
     extern __shared__ __align__(16) unsigned char smem[];
     __shared__ float red[(2 + 3 * 6) * DWAVES];
     __shared__ unsigned sync[2];
-    const int C = a.C;
     h16 *xs[6];
     const rwkv_half *mix[6];
     MatDev nomat[6] = {};
 #pragma unroll
     for (int j = 0; j < 6; ++j) { xs[j] = (h16 *)smem + j * C; mix[j] = a.mix[j]; }
     LnMixPro<false, 6> pro;
-    auto pro_load = [&]() { pro.load(a.x, C, a.ln_w, a.ln_b, a.sx, mix, nomat); };
+    auto pro_load = [&]() { pro.load(x, C, ln_w, ln_b, sx, mix, nomat); };
     auto pro_compute = [&]() { pro.compute(C, true, mix, xs, a.xx_tmp, red, sync, true); };
     auto rowf = [&](int c, int k, const uint8_t *&row, const h16 *&xv) {
         row = row_ptr<false>(a.mat[k], c);
@@ -708,7 +708,7 @@ __global__ __launch_bounds__(DTHREADS) void att7_kernel(Att7Args a) {
         for (int k = 0; k < 3; ++k) a.out[k][c] = f2h(d[k]);
     };
     const int nseg = (C * 2) >> 4;
-    stream_rows<false, 1, 3, 2, NoEpi, true>(C, nseg, pro_waves(C >> 3), sync, pro_load, pro_compute, [] {}, rowf, epi_load, epi);
+    stream_rows<false, 1, 3, 2, NoEpi, true>(RWKV_SPLIT, nseg, pro_waves(C >> 3), sync, pro_load, pro_compute, [] {}, rowf, epi_load, epi);
     // first LoRA stages: row g of the stacked matrix belongs to block j = w, a, v, g
     auto block_of = [&](int g) { return (g >= a.o_a ? 1 : 0) + (g >= a.o_v ? 1 : 0) + (g >= a.o_g ? 1 : 0); };
     auto rowf2 = [&](int g, int, const uint8_t *&row, const h16 *&xv) {
@@ -723,7 +723,7 @@ __global__ __launch_bounds__(DTHREADS) void att7_kernel(Att7Args a) {
         v = j == 0 ? tanhf(v) : (j == 3 ? sigmoidf_(v) : v);
         a.l1[g] = f2h(v);
     };
-    stream_rows<false, 1, 1, 2, NoEpi, false>(a.rtot, nseg, 0, nullptr, [] {}, [] {}, [] {}, rowf2, epi_load, epi2);
+    stream_rows<false, 1, 1, 2, NoEpi, false>(a.lsplit, nseg, 0, nullptr, [] {}, [] {}, [] {}, rowf2, epi_load, epi2);
 }
 
 struct Tmix7Args {
@@ -1054,7 +1054,10 @@ extern "C" int rwkv_v7_forward(const rwkv_v7_model *m, const rwkv_v56_layer_stat
                 a.mat[0] = to_dev56(l.att_receptance); a.mat[1] = to_dev56(l.att_key); a.mat[2] = to_dev56(l.att_value);
                 a.out[0] = ws.r; a.out[1] = ws.k; a.out[2] = v1;
                 a.lora1 = l.lora1; a.rtot = rtot; a.o_a = o_a; a.o_v = o_v; a.o_g = o_g; a.l1 = ws.l1;
-                hipLaunchKernelGGL(att7_kernel, dim3(c.grid), dim3(DTHREADS), 6 * (size_t)C * 2, st, a);
+                a.lsplit = row_split(rtot, c.grid);
+                const RowSplit sp = row_split(C, c.grid);
+                hipLaunchKernelGGL(att7_kernel, dim3(c.grid), dim3(DTHREADS), 6 * (size_t)C * 2, st, a.x, a.ln_w, a.ln_b, a.sx, RWKV_SPLIT_PASS(sp),
+                                   C, a);
             }
             {
                 Tmix7Args a{};
