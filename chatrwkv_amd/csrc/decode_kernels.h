@@ -35,42 +35,14 @@ struct MatDev {
     const rwkv_half *mx, *rx, *my, *ry;
 };
 
-// Kernel arguments.  A wave's first loads wait for the addresses in them, and a read of the arguments is a trip to memory of its own:
-// left to the compiler these kernels read the sizes, waited, divided, read the matrices, waited, read the operands' addresses and
-// waited again, about 1 us of a launch of 5 to 18.  So the scalars and addresses needed first are leading arguments of their own, which
-// are in registers when a wave starts (-amdgpu-kernarg-preload-count), and the others are read together (`at_once`).  us a token, with
-// the division below taken out: RWKV-4 7B uint8 1836 -> 1740, RWKV-6 7B uint8 2500 -> 2349, RWKV-7 7B fp16 3054 -> 2920.
-template <int N>
-DEV void at_once(const void *(&p)[N]) {
-    static_assert(N == 2 || N == 3 || N == 4 || N == 6 || N == 8 || N == 9 || N == 12, "written out");
-    if constexpr (N == 2) asm volatile("" : "+s"(p[0]), "+s"(p[1]));
-    if constexpr (N == 3) asm volatile("" : "+s"(p[0]), "+s"(p[1]), "+s"(p[2]));
-    if constexpr (N == 4) asm volatile("" : "+s"(p[0]), "+s"(p[1]), "+s"(p[2]), "+s"(p[3]));
-    if constexpr (N == 6) asm volatile("" : "+s"(p[0]), "+s"(p[1]), "+s"(p[2]), "+s"(p[3]), "+s"(p[4]), "+s"(p[5]));
-    if constexpr (N == 8)
-        asm volatile("" : "+s"(p[0]), "+s"(p[1]), "+s"(p[2]), "+s"(p[3]), "+s"(p[4]), "+s"(p[5]), "+s"(p[6]), "+s"(p[7]));
-    if constexpr (N == 9)
-        asm volatile("" : "+s"(p[0]), "+s"(p[1]), "+s"(p[2]), "+s"(p[3]), "+s"(p[4]), "+s"(p[5]), "+s"(p[6]), "+s"(p[7]), "+s"(p[8]));
-    if constexpr (N == 12)
-        asm volatile("" : "+s"(p[0]), "+s"(p[1]), "+s"(p[2]), "+s"(p[3]), "+s"(p[4]), "+s"(p[5]), "+s"(p[6]), "+s"(p[7]), "+s"(p[8]),
-                     "+s"(p[9]), "+s"(p[10]), "+s"(p[11]));
-}
-
-// eight values through such an address, which the compiler no longer knows to be one of global memory
-DEV h16x8 load8(const void *p, int i) { return ((const __attribute__((address_space(1))) h16x8 *)p)[i]; }
-
-// The rows of a launch over its waves: wave w takes the groups [split_at(w), split_at(w + 1)), floor or ceil of ngroups / nwaves of
-// them, i.e. floor(w * ngroups / nwaves) = w q + floor(w r / nwaves), and the division is a multiplication (exact for w r < 2^26:
-// the factor is at most nwaves <= 2^13 too large in 2^40).  Two 64-bit divisions stood here, 250 instructions ahead of a wave's first load.
-struct RowSplit { uint64_t magic; int q, r; };
-inline RowSplit row_split(int64_t ngroups, int grid) {
-    const int64_t nwaves = (int64_t)grid * DWAVES;
-    return RowSplit{((uint64_t)1 << 40) / (uint64_t)nwaves + 1, (int)(ngroups / nwaves), (int)(ngroups % nwaves)};
-}
-#define RWKV_SPLIT_ARGS uint64_t split_magic, int split_q, int split_r
-#define RWKV_SPLIT (RowSplit{split_magic, split_q, split_r})
-#define RWKV_SPLIT_PASS(sp) (sp).magic, (sp).q, (sp).r
-DEV int split_at(const RowSplit &s, int wave) { return wave * s.q + (int)(((uint64_t)(uint32_t)(wave * s.r) * s.magic) >> 40); }
+// The arguments of these kernels (kernels.h): the prologue's first operands and the split of the rows over the waves come first.  Before,
+// they read the sizes, waited, divided twice in 64 bits, read the matrices, waited, read the operands' addresses and waited again, and
+// a barrier that is there for the order of requests came after the wait for the first operand.  us a token: RWKV-4 7B uint8 1836 ->
+// 1740, RWKV-6 7B uint8 2500 -> 2349, RWKV-7 7B fp16 3054 -> 2920.
+#define RWKV_SPLIT_ARGS uint64_t split_factor, int split_q, int split_r
+#define RWKV_SPLIT (RowSplit{split_factor, split_q, split_r})
+#define RWKV_SPLIT_PASS(sp) (sp).factor, (sp).q, (sp).r
+inline RowSplit wave_split(int64_t rows, int grid) { return row_split(rows, (int64_t)grid * DWAVES); }
 
 // Sums of K values over the first `npw` waves of the workgroup (the waves that run a prologue), in two
 // halves with a synchronisation between them, which the caller places: `put` by each of those waves
@@ -751,6 +723,12 @@ __global__ __launch_bounds__(DTHREADS) void multi_vec_kernel(const rwkv_half *v0
     // a group is one output index m with its NM rows (row m of every matrix), so the matrix number is a
     // compile-time constant everywhere (an array of per-matrix fields indexed at run time would go to scratch)
     struct Epi { rwkv_half rx[NM], mx[NM]; };
+    {
+        const void *wl[2 * NM];   // the matrices and their strides
+#pragma unroll
+        for (int k = 0; k < NM; ++k) { wl[2 * k] = a.mat[k].w; wl[2 * k + 1] = (const void *)a.mat[k].ld; }
+        at_once(wl);
+    }
     auto rowf = [&](int m, int k, const uint8_t *&row, const h16 *&xv) {
         row = row_ptr<U8>(a.mat[k], m);
         xv = xs[k];
@@ -797,8 +775,8 @@ __global__ __launch_bounds__(DTHREADS) void multi_vec_kernel(const rwkv_half *v0
                        RWKV_SPLIT_PASS(sp), a.N, a.M, a)
 inline void multi_vec_launch(bool u8, MultiVecArgs a, int grid, hipStream_t st) {
     const size_t lds = (size_t)(a.nm + 1) * a.N * 2;
-    const RowSplit sp = row_split(a.M, grid);
-    a.xsplit = row_split(a.xm, grid);
+    const RowSplit sp = wave_split(a.M, grid);
+    a.xsplit = wave_split(a.xm, grid);
     if (a.nm == 4) {
         if (u8) RWKV_MULTI_VEC(true, 4);
         else RWKV_MULTI_VEC(false, 4);
@@ -810,7 +788,7 @@ inline void multi_vec_launch(bool u8, MultiVecArgs a, int grid, hipStream_t st) 
 
 template <bool U8, int NJ, int G>
 inline void lnmix_start(const LnMixArgs &a, int grid, hipStream_t st) {
-    const RowSplit sp = row_split((int64_t)a.M[0] + (NJ > 1 ? a.M[1] : 0), grid);
+    const RowSplit sp = wave_split((int64_t)a.M[0] + (NJ > 1 ? a.M[1] : 0), grid);
     hipLaunchKernelGGL((lnmix_kernel<U8, NJ, G>), dim3(grid), dim3(DTHREADS), NJ * (size_t)a.C * 2, st, a.x, a.ln_w, a.ln_b, a.sx,
                        RWKV_SPLIT_PASS(sp), a.C, a.M[0], a);
 }
@@ -864,7 +842,7 @@ inline void lnhead_launch(bool u8, const rwkv_half *x, int C, const rwkv_half *l
 inline void vec_launch(bool u8, const VecArgs &a, int grid, hipStream_t st) {
     const size_t lds = (size_t)a.N * 2;
     const int groups = a.N >> 3;
-    const RowSplit sp = row_split(a.M, grid);
+    const RowSplit sp = wave_split(a.M, grid);
     if (groups <= 512) RWKV_VEC_CASE(4, 1, 8);
     else if (groups <= 1024) RWKV_VEC_CASE(4, 2, 8);
     else if (groups <= 2048) RWKV_VEC_CASE(8, 4, 8);

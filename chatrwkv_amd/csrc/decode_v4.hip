@@ -143,7 +143,7 @@ static int v4_one_impl(const rwkv_v4_model *m, const rwkv_v4_layer_state *states
             a.decay = l.time_decay; a.first = l.time_first; a.aa = s.aa; a.bb = s.bb; a.pp = s.pp;
             a.rwkv = ws.rwkv;
             const size_t lds = 3 * (size_t)C * 2;
-            const RowSplit sp = row_split(C, grid);
+            const RowSplit sp = wave_split(C, grid);
             const auto kernel = u8 ? (tok ? att_kernel<true, 1, true> : att_kernel<true, 1, false>)
                                    : (tok ? att_kernel<false, 1, true> : att_kernel<false, 1, false>);
             hipLaunchKernelGGL(kernel, dim3(grid), dim3(DTHREADS), lds, st, a.x, a.ln_w, a.ln_b, a.sx, RWKV_SPLIT_PASS(sp), C, a);

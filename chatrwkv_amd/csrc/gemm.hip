@@ -230,13 +230,13 @@ DEV void slab_sum8(size_t n, const float *__restrict__ p, f32x4 &lo, f32x4 &hi) 
 #pragma unroll
     for (int k = 1; k < KS; ++k) { lo += pl[k]; hi += ph[k]; }
 }
-DEV void splitk_rows8(int T, int M, int ks, const float *__restrict__ part, void *Y, int64_t ldy, const GemmEpi &ep,
-                      int64_t first, int64_t stride) {
-    const int64_t n8 = (int64_t)T * M / 8, n = (int64_t)T * M;
-    const int m8 = M / 8;
+// Chunk i of eight outputs, i < n8; factor: div_factor of a row's chunks (n8 < 2^20: the slabs fit 64 MB).
+DEV void splitk_chunk8(int i, int n8, int M, uint64_t factor, int ks, const float *__restrict__ part, void *Y, int64_t ldy, const GemmEpi &ep) {
+    if (i >= n8) return;
+    const size_t n = (size_t)n8 * 8;
     const bool four = by_four(M, ldy, Y, ep);
-    for (int64_t i = first; i < n8; i += stride) {
-        const int t = (int)(i / m8), col = (int)(i - (int64_t)t * m8) * 8;
+    {
+        const int t = div_by((uint32_t)i, factor), col = (i - t * (M / 8)) * 8;
         EpiIn in = {};
         h16x8 rx8 = {}, mx8 = {};
         if (!four) in = epi_in(ep, t, col, true, false);
@@ -248,29 +248,29 @@ DEV void splitk_rows8(int T, int M, int ks, const float *__restrict__ part, void
         }
         f32x4 lo, hi;
         switch (ks) {
-            case 2: slab_sum8<2>(n, part + 8 * i, lo, hi); break;
-            case 3: slab_sum8<3>(n, part + 8 * i, lo, hi); break;
-            case 4: slab_sum8<4>(n, part + 8 * i, lo, hi); break;
-            case 5: slab_sum8<5>(n, part + 8 * i, lo, hi); break;
-            case 6: slab_sum8<6>(n, part + 8 * i, lo, hi); break;
-            case 7: slab_sum8<7>(n, part + 8 * i, lo, hi); break;
-            default: slab_sum8<8>(n, part + 8 * i, lo, hi); break;   // dma_split: at most eight
+            case 2: slab_sum8<2>(n, part + 8 * (size_t)i, lo, hi); break;
+            case 3: slab_sum8<3>(n, part + 8 * (size_t)i, lo, hi); break;
+            case 4: slab_sum8<4>(n, part + 8 * (size_t)i, lo, hi); break;
+            case 5: slab_sum8<5>(n, part + 8 * (size_t)i, lo, hi); break;
+            case 6: slab_sum8<6>(n, part + 8 * (size_t)i, lo, hi); break;
+            case 7: slab_sum8<7>(n, part + 8 * (size_t)i, lo, hi); break;
+            default: slab_sum8<8>(n, part + 8 * (size_t)i, lo, hi); break;   // dma_split: at most eight
         }
         float v[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
         if (ep.rx) affine8(v, rx8, mx8, in.s0, in.s2);
         if (four) {
 #pragma unroll 1
             for (int g = 0; g < 2; ++g) finish_row4(g ? f32x4{v[4], v[5], v[6], v[7]} : f32x4{v[0], v[1], v[2], v[3]}, t, col + 4 * g, M, ep, Y, ldy);
-            continue;
+            return;
         }
         float a0 = 0.f, a2 = 0.f;   // a product that emits row sums does not split K
         finish_row8<false>(v, in, t, col, ep, Y, ldy, Emit8{}, a0, a2);
     }
 }
 
-__global__ __launch_bounds__(256) void splitk_epilogue8_kernel(int T, int M, int KS, const float *__restrict__ part, void *Y,
+__global__ __launch_bounds__(256) void splitk_epilogue8_kernel(const float *__restrict__ part, uint64_t factor, int n8, int M, int KS, void *Y,
                                                                int64_t ldy, GemmEpi ep) {
-    splitk_rows8(T, M, KS, part, Y, ldy, ep, (int64_t)blockIdx.x * 256 + threadIdx.x, (int64_t)gridDim.x * 256);
+    splitk_chunk8((int)blockIdx.x * 256 + threadIdx.x, n8, M, factor, KS, part, Y, ldy, ep);
 }
 
 template <bool W_U8, int BT, int BM, int WT, int WM, int PF, bool SPLIT>
@@ -1038,7 +1038,7 @@ DEV int group_member(int first1, int first2, int first3, int &tile) {
 struct GemmIn { const h16 *A; const void *W; int64_t ldw; int M, walk_m; };
 DEV GemmIn gemm_in(const GemmMember &m) {
     GemmIn in = {m.A, m.W, m.ldw, m.M, m.walk_m};
-    asm volatile("" : "+s"(in.A), "+s"(in.W), "+s"(in.ldw), "+s"(in.M), "+s"(in.walk_m));
+    asm volatile("" ::"s"(in.A), "s"(in.W), "s"(in.ldw), "s"(in.M), "s"(in.walk_m));
     return in;
 }
 // fills `first` and the walks for tiles of tm x tn; returns the tiles of the launch
@@ -1434,10 +1434,10 @@ int launch_kg(GemmGroup &g, int n, int64_t T, int64_t N, int ks, hipStream_t st)
 }
 
 // second pass of a split group launch: member blockIdx.y, as splitk_epilogue8_kernel
-__global__ __launch_bounds__(256) void splitk_group_epilogue8_kernel(int T, int KS, GemmGroup g) {
-    const int gi = blockIdx.y;
-    splitk_rows8(T, g.m[gi].M, KS, g.m[gi].part, g.m[gi].Y, g.m[gi].M, g.m[gi].ep, (int64_t)blockIdx.x * 256 + threadIdx.x,
-                     (int64_t)gridDim.x * 256);
+struct SplitFactors { uint64_t f[4]; };
+__global__ __launch_bounds__(256) void splitk_group_epilogue8_kernel(int T, int KS, SplitFactors rows, GemmMembers g) {
+    const GemmMember &m = g.m[blockIdx.y];
+    splitk_chunk8((int)blockIdx.x * 256 + threadIdx.x, T * (m.M / 8), m.M, rows.f[blockIdx.y], KS, m.part, m.Y, m.ldy, m.ep);
 }
 
 struct PrepGroup {
@@ -1533,7 +1533,7 @@ struct SkinnyGroup {
 };
 
 template <int NU>
-__global__ __launch_bounds__(1024) void skinny_u8_kernel(int T, int N, int n, int total, SkinnyGroup g) {
+__global__ __launch_bounds__(1024) void skinny_u8_kernel(uint64_t factor, int share, int rest, int T, int N, int n, SkinnyGroup g) {
     constexpr bool HELD = NU > 0;
     constexpr int UB = NU == 1 ? 1 : NU == 4 ? 4 : 2;           // units of a step
     constexpr int NS = HELD ? NU / UB : 2;                      // steps of a row group; NU == 0: of a pass of its loop
@@ -1545,7 +1545,8 @@ __global__ __launch_bounds__(1024) void skinny_u8_kernel(int T, int N, int n, in
     const int sub = lane & 15, q = lane >> 4;
     const int nunits = N / 64;
     const h16x2 off = {(h16)1023.5f, (h16)1023.5f};
-    const int b0 = (int)((int64_t)total * blockIdx.x / gridDim.x), b1 = (int)((int64_t)total * (blockIdx.x + 1) / gridDim.x);
+    const RowSplit sp = {factor, share, rest};
+    const int b0 = split_at(sp, blockIdx.x), b1 = split_at(sp, blockIdx.x + 1);
     auto fence = [] {                                           // loads are used in the order of their issue (v7.hip)
         asm volatile("" ::: "memory");
         __builtin_amdgcn_sched_barrier(0);
@@ -1562,14 +1563,15 @@ __global__ __launch_bounds__(1024) void skinny_u8_kernel(int T, int N, int n, in
     };
     int base = 0, count = 0;                                    // row groups of the members before; done by this workgroup
     for (int gi = 0; gi < n; ++gi) {
-        const int M = g.m[gi].M, groups = (M + 15) >> 4;
+        const GemmIn in = gemm_in(g.m[gi]);
+        const int M = in.M, groups = (M + 15) >> 4;
         const int lo = max(b0, base) - base, hi = min(b1, base + groups) - base;
         base += groups;
         if (lo >= hi) continue;
         const GemmEpi &ep = g.m[gi].ep;
-        const h16 *A = g.m[gi].A;
-        const unsigned char *W = (const unsigned char *)g.m[gi].W;
-        const int64_t ldw = g.m[gi].ldw;
+        const h16 *A = in.A;
+        const unsigned char *W = (const unsigned char *)in.W;
+        const int64_t ldw = in.ldw;
         // In place of a unit past the end of the row, and of every unit past the share's last row group, all lanes load the
         // first bytes of the matrix, which nothing uses: a branch around a load would make the waits for those before it longer.
         struct Step { u32x4 w[UB]; h16x8 x[HELD ? 1 : UB][2]; };
@@ -1715,10 +1717,12 @@ __global__ __launch_bounds__(1024) void skinny_u8_kernel(int T, int N, int n, in
 template <int NCI>
 __global__ __launch_bounds__(1024) void skinny_f16_kernel(int T, int N, SkinnyGroup g) {
     __shared__ float red[16][64][4];
-    const int gi = blockIdx.y, M = g.m[gi].M;
-    const h16 *__restrict__ A = g.m[gi].A;
-    const unsigned char *__restrict__ W = (const unsigned char *)g.m[gi].W;
-    const int64_t lda = g.lda, ldw = g.m[gi].ldw;
+    const int gi = blockIdx.y;
+    const GemmIn gin = gemm_in(g.m[gi]);
+    const int M = gin.M;
+    const h16 *__restrict__ A = gin.A;
+    const unsigned char *__restrict__ W = (const unsigned char *)gin.W;
+    const int64_t lda = g.lda, ldw = gin.ldw;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int sub = lane & 15, q = lane >> 4;
     const int nchunks = N / 32;
@@ -1803,10 +1807,12 @@ int skinny_launch(bool w_u8, int n, int64_t T, int64_t N, const SkinnyGroup &g, 
         maxg = std::max(maxg, (g.m[i].M + 15) / 16);
     }
     const int64_t per_wave = (N / (w_u8 ? 64 : 32) + 15) / 16;    // chunks a wave owns
+    const int grid = std::min(total, num_cu());
+    const RowSplit sp = row_split(total, grid);
 #define RWKV_SKINNY(NC)                                                                                                              \
     do {                                                                                                                             \
-        if (w_u8) hipLaunchKernelGGL((skinny_u8_kernel<NC>), dim3((unsigned)std::min(total, num_cu())), dim3(1024), 0, st, (int)T,   \
-                                     (int)N, n, total, g);                                                                           \
+        if (w_u8) hipLaunchKernelGGL((skinny_u8_kernel<NC>), dim3((unsigned)grid), dim3(1024), 0, st, sp.factor, sp.q, sp.r, (int)T, \
+                                     (int)N, n, g);                                                                                  \
         else hipLaunchKernelGGL((skinny_f16_kernel<NC>), dim3((unsigned)std::min(maxg, 2 * num_cu()), (unsigned)n), dim3(1024), 0,   \
                                 st, (int)T, (int)N, g);                                                                              \
     } while (0)
@@ -2075,10 +2081,13 @@ int dma_tile(bool w_u8, int64_t T, int nk, int n, const int64_t *M, size_t ws_by
 // The second pass of a direct-to-LDS launch with K split ks ways: eight outputs wide where M is a multiple.
 int launch_splitk_epilogue(int ks, int64_t T, int64_t M, void *Y, int64_t ldy, const GemmEpi &ep, hipStream_t st) {
     const int64_t n = T * M;
-    const int per_block = M & 7 ? 1024 : 2048;
-    const unsigned blocks = (unsigned)std::min<int64_t>((n + per_block - 1) / per_block, 16384);
-    if (M & 7) hipLaunchKernelGGL(splitk_epilogue_kernel, dim3(blocks), dim3(256), 0, st, (int)T, (int)M, ks, ep.splitk_ws, Y, ldy, ep);
-    else hipLaunchKernelGGL(splitk_epilogue8_kernel, dim3(blocks), dim3(256), 0, st, (int)T, (int)M, ks, ep.splitk_ws, Y, ldy, ep);
+    if (M & 7) {
+        hipLaunchKernelGGL(splitk_epilogue_kernel, dim3((unsigned)std::min<int64_t>((n + 1023) / 1024, 16384)), dim3(256), 0, st, (int)T, (int)M, ks,
+                           ep.splitk_ws, Y, ldy, ep);
+    } else {
+        hipLaunchKernelGGL(splitk_epilogue8_kernel, dim3((unsigned)((n / 8 + 255) / 256)), dim3(256), 0, st, ep.splitk_ws, div_factor(M / 8),
+                           (int)(n / 8), (int)M, ks, Y, ldy, ep);
+    }
     RWKV_LAUNCH_CHECK();
     return RWKV_OK;
 }
@@ -2310,8 +2319,10 @@ int gemm_group_launch(bool w_u8, int n, int64_t T, int64_t N, const rwkv_half *c
         const int rc = w_u8 ? launch_tile<true>(tile, g, n, T, N, ks, st) : launch_tile<false>(tile, g, n, T, N, ks, st);
         if (rc) return rc;
         if (ks > 1) {
-            const unsigned blocks = (unsigned)std::min<int64_t>((max_out + 2047) / 2048, 16384);
-            hipLaunchKernelGGL(splitk_group_epilogue8_kernel, dim3(blocks, (unsigned)n), dim3(256), 0, st, (int)T, ks, g);
+            SplitFactors rows{};
+            for (int i = 0; i < n; ++i) rows.f[i] = div_factor(g.m[i].M / 8);
+            hipLaunchKernelGGL(splitk_group_epilogue8_kernel, dim3((unsigned)((max_out + 2047) / 2048), (unsigned)n), dim3(256), 0, st, (int)T, ks, rows,
+                               (const GemmMembers &)g);
         }
         RWKV_LAUNCH_CHECK();
         return RWKV_OK;

@@ -13,6 +13,37 @@ struct PerDeviceOnce {
     }
 };
 
+// Kernel arguments.  A wave's first loads wait for the addresses in them, and a read of the arguments is a trip to memory of its own;
+// left to the compiler a kernel reads the sizes, waits, reads a few addresses, waits, and so on.  So what is needed first are leading
+// scalar arguments, which are in registers when a wave starts (up to 14 words, -amdgpu-kernarg-preload-count), and others are read
+// together: at_once makes all of these addresses be there from here on.
+template <int N>
+DEV void at_once(const void *const (&p)[N]) {
+    static_assert(N == 2 || N == 3 || N == 4 || N == 6 || N == 8 || N == 9 || N == 12, "written out");
+    if constexpr (N == 2) asm volatile("" ::"s"(p[0]), "s"(p[1]));
+    if constexpr (N == 3) asm volatile("" ::"s"(p[0]), "s"(p[1]), "s"(p[2]));
+    if constexpr (N == 4) asm volatile("" ::"s"(p[0]), "s"(p[1]), "s"(p[2]), "s"(p[3]));
+    if constexpr (N == 6) asm volatile("" ::"s"(p[0]), "s"(p[1]), "s"(p[2]), "s"(p[3]), "s"(p[4]), "s"(p[5]));
+    if constexpr (N == 8) asm volatile("" ::"s"(p[0]), "s"(p[1]), "s"(p[2]), "s"(p[3]), "s"(p[4]), "s"(p[5]), "s"(p[6]), "s"(p[7]));
+    if constexpr (N == 9)
+        asm volatile("" ::"s"(p[0]), "s"(p[1]), "s"(p[2]), "s"(p[3]), "s"(p[4]), "s"(p[5]), "s"(p[6]), "s"(p[7]), "s"(p[8]));
+    if constexpr (N == 12)
+        asm volatile("" ::"s"(p[0]), "s"(p[1]), "s"(p[2]), "s"(p[3]), "s"(p[4]), "s"(p[5]), "s"(p[6]), "s"(p[7]), "s"(p[8]), "s"(p[9]),
+                     "s"(p[10]), "s"(p[11]));
+}
+DEV h16x8 load8(const void *p, int i) { return ((const h16x8 *)p)[i]; }
+
+// n / d as a multiplication with a factor from the host, exact for n (d - 1) < 2^40: the factor is at most d too large in 2^40.
+// (A 64-bit division is 120 instructions, and stood ahead of the first load of the kernels that have one of these.)
+inline uint64_t div_factor(int64_t d) { return ((uint64_t)1 << 40) / (uint64_t)d + 1; }
+DEV int div_by(uint32_t n, uint64_t factor) { return (int)(((uint64_t)n * factor) >> 40); }
+
+// `n` things over `parts`: part w takes [split_at(w), split_at(w + 1)), floor or ceil of n / parts of them, i.e. floor(w n / parts) =
+// w q + floor(w r / parts); parts <= 2^13.
+struct RowSplit { uint64_t factor; int q, r; };
+inline RowSplit row_split(int64_t n, int64_t parts) { return RowSplit{div_factor(parts), (int)(n / parts), (int)(n % parts)}; }
+DEV int split_at(const RowSplit &s, int w) { return w * s.q + div_by((uint32_t)(w * s.r), s.factor); }
+
 enum { ACT_NONE = 0, ACT_SIGMOID = 1, ACT_RELU_SQ = 2, ACT_RESIDUAL = 3, ACT_GATED_RESIDUAL = 4, ACT_SILU = 5, ACT_TANH = 6 };
 
 // Epilogue of the MFMA contraction (gemm.hip).

@@ -52,19 +52,20 @@ __global__ __launch_bounds__(256) void ln_f32_f16_kernel(int C, const float *__r
 // PRE: the mix / scale vectors too are requested at the top (3 NJ CH more registers per thread: shorter chain, fewer
 // workgroups per CU -- for short calls, where a CU has one or two rows anyway).
 template <int NJ, int CH, bool PRE, int NT>
-__global__ __launch_bounds__(NT) void lnmix_seq_fast_kernel(SeqMixArgs a) {
+__global__ __launch_bounds__(NT) void lnmix_seq_fast_kernel(const rwkv_half *x0, const rwkv_half *ln_w, const rwkv_half *ln_b, const rwkv_half *sx,
+                                                            rwkv_half *state_out, int C, int T, SeqMixArgs a) {
     constexpr int NSUM = 2 * NJ > 3 ? 2 * NJ : 3;
     __shared__ __align__(16) float red[24 + 8 * NJ];
     __shared__ float hop[NT == 512 ? 256 * NSUM : 1];
-    const int t = blockIdx.x, C = a.C, nch = C >> 3;
+    const int t = blockIdx.x, nch = C >> 3;
     // this thread's chunk c: tid + 256 c, or with 512 threads the first CH and the last CH of a chain's 2 CH
     const int j8_0 = NT == 256 ? (int)threadIdx.x : (int)(threadIdx.x & 255) + 256 * CH * (int)(threadIdx.x >> 8);
-    const rwkv_half *x = a.x + (size_t)t * C;
-    const bool shift = a.sx != nullptr, prev_row = shift && t > 0;
+    const rwkv_half *x = x0 + (size_t)t * C;
+    const bool shift = sx != nullptr, prev_row = shift && t > 0;
     const rwkv_half *xp = prev_row ? x - C : x;
     // Row 0's workgroup also forms the new token-shift state LN(x[T-1]): its statistics ride in the same barriers
-    const bool commit = a.state_out && t == 0;
-    const rwkv_half *xl = commit ? a.x + (size_t)(a.T - 1) * C : x;
+    const bool commit = state_out && t == 0;
+    const rwkv_half *xl = commit ? x0 + (size_t)(T - 1) * C : x;
     h16x8 xv[CH], pxv[CH], lv[CH], wv[CH], bv[CH], mv[PRE ? NJ : 1][CH], rv[PRE ? NJ : 1][CH], yv[PRE ? NJ : 1][CH];
 #pragma unroll
     for (int c = 0; c < CH; ++c) {
@@ -72,13 +73,21 @@ __global__ __launch_bounds__(NT) void lnmix_seq_fast_kernel(SeqMixArgs a) {
         xv[c] = *(const h16x8 *)(x + 8 * j8);
         pxv[c] = *(const h16x8 *)(xp + 8 * j8);
         lv[c] = *(const h16x8 *)(xl + 8 * j8);
-        wv[c] = *(const h16x8 *)(a.ln_w + 8 * j8);
-        bv[c] = *(const h16x8 *)(a.ln_b + 8 * j8);
-        if constexpr (PRE) {
+        wv[c] = *(const h16x8 *)(ln_w + 8 * j8);
+        bv[c] = *(const h16x8 *)(ln_b + 8 * j8);
+    }
+    const void *vec[3 * NJ];   // mix, ry, my
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) { vec[3 * j] = a.mix[j]; vec[3 * j + 1] = a.ry[j]; vec[3 * j + 2] = a.my[j]; }
+    if constexpr (PRE) {
+        if constexpr (NJ <= 4) at_once(vec);
+#pragma unroll
+        for (int c = 0; c < CH; ++c) {
+            const int j8 = min(j8_0 + c * 256, nch - 1);
 #pragma unroll
             for (int j = 0; j < NJ; ++j) {
-                mv[j][c] = *(const h16x8 *)((a.mix[j] ? a.mix[j] : a.ln_w) + 8 * j8);
-                if (a.ry[j]) { rv[j][c] = *(const h16x8 *)(a.ry[j] + 8 * j8); yv[j][c] = *(const h16x8 *)(a.my[j] + 8 * j8); }
+                mv[j][c] = load8(vec[3 * j] ? vec[3 * j] : ln_w, j8);
+                if (vec[3 * j + 1]) { rv[j][c] = load8(vec[3 * j + 1], j8); yv[j][c] = load8(vec[3 * j + 2], j8); }
             }
         }
     }
@@ -133,22 +142,22 @@ __global__ __launch_bounds__(NT) void lnmix_seq_fast_kernel(SeqMixArgs a) {
         h16x8 pv = xx;
         if (shift) {
             if (t > 0) pv = norm8(dp[c], prstd, wv[c], bv[c]);
-            else pv = *(const h16x8 *)(a.sx + 8 * j8);
+            else pv = *(const h16x8 *)(sx + 8 * j8);
         }
-        if (a.xx_last && t == a.T - 1) *(h16x8 *)(a.xx_last + 8 * j8) = xx;
+        if (a.xx_last && t == T - 1) *(h16x8 *)(a.xx_last + 8 * j8) = xx;
 #pragma unroll
         for (int j = 0; j < NJ; ++j) {
             h16x8 kx = xx;
-            if (a.mix[j]) {
+            if (vec[3 * j]) {
                 h16x8 m8;
-                if constexpr (PRE) m8 = mv[j][c]; else m8 = *(const h16x8 *)(a.mix[j] + 8 * j8);
+                if constexpr (PRE) m8 = mv[j][c]; else m8 = load8(vec[3 * j], j8);
                 kx = mix8(xx, pv, m8, a.maa_form);
             }
             h16x8 o = kx;
-            if (a.ry[j]) {
+            if (vec[3 * j + 1]) {
                 h16x8 r8, y8;
                 if constexpr (PRE) { r8 = rv[j][c]; y8 = yv[j][c]; }
-                else { r8 = *(const h16x8 *)(a.ry[j] + 8 * j8); y8 = *(const h16x8 *)(a.my[j] + 8 * j8); }
+                else { r8 = load8(vec[3 * j + 1], j8); y8 = load8(vec[3 * j + 2], j8); }
                 o = kx * r8;
                 if constexpr (NT == 256) add_mix(acc, j, kx, y8);
                 else { kv[c][j] = kx; sv[c][j] = y8; }
@@ -160,12 +169,12 @@ __global__ __launch_bounds__(NT) void lnmix_seq_fast_kernel(SeqMixArgs a) {
         if (commit) {
             float dl[8];
             less_mean8(lv[c], lmean, dl);
-            *(h16x8 *)(a.state_out + 8 * j8) = norm8(dl, lrstd, wv[c], bv[c]);
+            *(h16x8 *)(state_out + 8 * j8) = norm8(dl, lrstd, wv[c], bv[c]);
         }
     }
     bool any = false;
 #pragma unroll
-    for (int j = 0; j < NJ; ++j) any = any || a.ry[j];
+    for (int j = 0; j < NJ; ++j) any = any || vec[3 * j + 1];
     if (any) {
         row_sums<2 * NJ, NT>(acc, red + 24, hop, [&](float (&v)[2 * NJ], auto) {
             if constexpr (NT > 256)
@@ -174,12 +183,12 @@ __global__ __launch_bounds__(NT) void lnmix_seq_fast_kernel(SeqMixArgs a) {
                     if (j8_0 + c * 256 < nch)
 #pragma unroll
                         for (int j = 0; j < NJ; ++j)
-                            if (a.ry[j]) add_mix(v, j, kv[c][j], sv[c][j]);
+                            if (vec[3 * j + 1]) add_mix(v, j, kv[c][j], sv[c][j]);
         });
         if (threadIdx.x == 0)
 #pragma unroll
             for (int j = 0; j < NJ; ++j)
-                if (a.ry[j]) { a.s0[j][t] = acc[2 * j]; a.s2[j][t] = acc[2 * j + 1]; }
+                if (vec[3 * j + 1]) { a.s0[j][t] = acc[2 * j]; a.s2[j][t] = acc[2 * j + 1]; }
     }
 }
 
@@ -189,11 +198,11 @@ template <int CH, bool PRE, int NT>
 static bool lnmix_seq_fast_launch(const SeqMixArgs &a, int nj, hipStream_t st) {
     const dim3 grid((unsigned)a.T), block(NT);
     switch (nj) {
-        case 1: hipLaunchKernelGGL((lnmix_seq_fast_kernel<1, CH, PRE, NT>), grid, block, 0, st, a); break;
-        case 2: hipLaunchKernelGGL((lnmix_seq_fast_kernel<2, CH, PRE, NT>), grid, block, 0, st, a); break;
-        case 3: hipLaunchKernelGGL((lnmix_seq_fast_kernel<3, CH, PRE, NT>), grid, block, 0, st, a); break;
-        case 4: hipLaunchKernelGGL((lnmix_seq_fast_kernel<4, CH, PRE, NT>), grid, block, 0, st, a); break;
-        case 6: hipLaunchKernelGGL((lnmix_seq_fast_kernel<6, CH, PRE && NT == 256, NT>), grid, block, 0, st, a); break;
+        case 1: hipLaunchKernelGGL((lnmix_seq_fast_kernel<1, CH, PRE, NT>), grid, block, 0, st, a.x, a.ln_w, a.ln_b, a.sx, a.state_out, a.C, a.T, a); break;
+        case 2: hipLaunchKernelGGL((lnmix_seq_fast_kernel<2, CH, PRE, NT>), grid, block, 0, st, a.x, a.ln_w, a.ln_b, a.sx, a.state_out, a.C, a.T, a); break;
+        case 3: hipLaunchKernelGGL((lnmix_seq_fast_kernel<3, CH, PRE, NT>), grid, block, 0, st, a.x, a.ln_w, a.ln_b, a.sx, a.state_out, a.C, a.T, a); break;
+        case 4: hipLaunchKernelGGL((lnmix_seq_fast_kernel<4, CH, PRE, NT>), grid, block, 0, st, a.x, a.ln_w, a.ln_b, a.sx, a.state_out, a.C, a.T, a); break;
+        case 6: hipLaunchKernelGGL((lnmix_seq_fast_kernel<6, CH, PRE && NT == 256, NT>), grid, block, 0, st, a.x, a.ln_w, a.ln_b, a.sx, a.state_out, a.C, a.T, a); break;
         default: return false;
     }
     return true;

@@ -25,16 +25,17 @@ struct Mix1Args {
 // chunks of the row and of the previous row stay in registers from one round of loads, and the four sums of the two rows'
 // statistics share their barriers.
 template <int CH, int NT>
-__global__ __launch_bounds__(NT) void v6_mix1_kernel(Mix1Args a) {
+__global__ __launch_bounds__(NT) void v6_mix1_kernel(const rwkv_half *x0, const rwkv_half *ln_w, const rwkv_half *ln_b, const rwkv_half *maa_x,
+                                                     const rwkv_half *sx, int C, int T, Mix1Args a) {
     __shared__ __align__(16) float red[24];
     __shared__ float hop[NT == 512 ? 256 * 6 : 1];
-    const int t = blockIdx.x, C = a.C, nch = C >> 3;
+    const int t = blockIdx.x, nch = C >> 3;
     const int j8_0 = NT == 256 ? (int)threadIdx.x : (int)(threadIdx.x & 255) + 256 * CH * (int)(threadIdx.x >> 8);
-    const rwkv_half *x = a.x + (size_t)t * C;
+    const rwkv_half *x = x0 + (size_t)t * C;
     const rwkv_half *xp = t > 0 ? x - C : x;
     // row 0's workgroup also forms the new token-shift state LN1(x[T-1]); its statistics ride in the same barriers
     const bool commit = t == 0;
-    const rwkv_half *xl = commit ? a.x + (size_t)(a.T - 1) * C : x;
+    const rwkv_half *xl = commit ? x0 + (size_t)(T - 1) * C : x;
     h16x8 xv[CH], pxv[CH], lv[CH], wv[CH], bv[CH], mv[CH];
 #pragma unroll
     for (int c = 0; c < CH; ++c) {
@@ -42,9 +43,9 @@ __global__ __launch_bounds__(NT) void v6_mix1_kernel(Mix1Args a) {
         xv[c] = *(const h16x8 *)(x + 8 * j8);
         pxv[c] = *(const h16x8 *)(xp + 8 * j8);
         lv[c] = *(const h16x8 *)(xl + 8 * j8);
-        wv[c] = *(const h16x8 *)(a.ln_w + 8 * j8);
-        bv[c] = *(const h16x8 *)(a.ln_b + 8 * j8);
-        mv[c] = *(const h16x8 *)(a.maa_x + 8 * j8);
+        wv[c] = *(const h16x8 *)(ln_w + 8 * j8);
+        bv[c] = *(const h16x8 *)(ln_b + 8 * j8);
+        mv[c] = *(const h16x8 *)(maa_x + 8 * j8);
     }
     float sq[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};   // sum and sum of squares of the row, the previous row, the last row
     row_sums<6, NT>(sq, red, hop, [&](float (&v)[6], auto) {
@@ -71,7 +72,7 @@ __global__ __launch_bounds__(NT) void v6_mix1_kernel(Mix1Args a) {
             less_mean8(pxv[c], pmean, d);
             pv = norm8(d, prstd, wv[c], bv[c]);
         } else {
-            pv = *(const h16x8 *)(a.sx + 8 * j8);
+            pv = *(const h16x8 *)(sx + 8 * j8);
         }
         const size_t o = (size_t)t * C + 8 * j8;
         *(h16x8 *)(a.xx + o) = xx;
@@ -92,7 +93,7 @@ void v6_mix1_launch(const Mix1Args &a, hipStream_t st) {
     const auto kernel = a.C <= 2048   ? v6_mix1_kernel<1, 256>
                         : a.C <= 4096 ? (few ? v6_mix1_kernel<1, 512> : v6_mix1_kernel<2, 256>)
                                       : (few ? v6_mix1_kernel<2, 512> : v6_mix1_kernel<4, 256>);
-    hipLaunchKernelGGL(kernel, dim3((unsigned)a.T), dim3(few && a.C > 2048 ? 512 : 256), 0, st, a);
+    hipLaunchKernelGGL(kernel, dim3((unsigned)a.T), dim3(few && a.C > 2048 ? 512 : 256), 0, st, a.x, a.ln_w, a.ln_b, a.maa_x, a.sx, a.C, a.T, a);
 }
 
 struct Mix2Args {

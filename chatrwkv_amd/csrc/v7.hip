@@ -50,16 +50,13 @@ DEV float head8_sum(float v) {
     return v;
 }
 
-__global__ __launch_bounds__(256) void prep7_kernel(Prep7Args a) {
-    const int64_t nchunk = (int64_t)a.T * a.C / 8;
+__global__ __launch_bounds__(256) void prep7_kernel(int per_row, uint64_t factor, Prep7Args a) {
     const int cpr = a.C / 8;   // chunks per token row
-    // whole waves take part in the DPP sums: chunks past the end repeat the last one and store nothing
-    for (int64_t i0 = (int64_t)blockIdx.x * 256; i0 < nchunk; i0 += (int64_t)gridDim.x * 256) {
-        const int64_t i = i0 + threadIdx.x;
-        const bool live = i < nchunk;
-        const int64_t ic = live ? i : nchunk - 1;
-        const int64_t t = ic / cpr;
-        const int c = (int)(ic - t * cpr) * 8;
+    {
+        // whole waves take part in the DPP sums: chunks past the end of the row repeat its last one and store nothing
+        const int t = div_by(blockIdx.x, factor), i = ((int)blockIdx.x - t * per_row) * 256 + threadIdx.x;
+        const bool live = i < cpr;
+        const int c = min(i, cpr - 1) * 8;
         const size_t o = (size_t)t * a.C + c;
         const h16x8 r8 = *(const h16x8 *)(a.r + o), k8 = *(const h16x8 *)(a.k + o), v8 = *(const h16x8 *)(a.v + o);
         const h16x8 ar8 = *(const h16x8 *)(a.a_raw + o), wr8 = *(const h16x8 *)(a.w_raw + o);
@@ -634,19 +631,16 @@ __global__ __launch_bounds__(256, 2) void wkv7_apply_kernel(int H, int C, float 
 // GroupNorm over each head's 64 outputs (eps 64e-5) on the fp16-rounded read-out, + bonus * v, * g.  Four adjacent
 // channels per lane (16-byte loads of y, 8-byte accesses to v, g and the output): a row of 16 lanes owns one head
 // of one token, its two sums are DPP row sums; grid-stride over the T * C / 4 chunks.
-__global__ __launch_bounds__(256) void gn7_kernel(int T, int C, const float *__restrict__ y,
+__global__ __launch_bounds__(256) void gn7_kernel(int per_row, uint64_t factor, int C, const float *__restrict__ y,
                                                   const rwkv_half *__restrict__ lnx_w,
                                                   const rwkv_half *__restrict__ lnx_b, const float *__restrict__ rk,
                                                   const rwkv_half *__restrict__ v, const rwkv_half *__restrict__ gate,
                                                   rwkv_half *__restrict__ out) {
-    const int64_t nchunk = (int64_t)T * C / 4;   // a multiple of 16: whole rows of lanes are live or idle together
-    const int cpr = C / 4, H = C / HS7;
-    for (int64_t i0 = (int64_t)blockIdx.x * 256; i0 < nchunk; i0 += (int64_t)gridDim.x * 256) {
-        const int64_t i = i0 + threadIdx.x;
-        const bool live = i < nchunk;
-        const int64_t ic = live ? i : nchunk - 1;
-        const int64_t t = ic / cpr;
-        const int c = (int)(ic - t * cpr) * 4;
+    const int cpr = C / 4, H = C / HS7;   // cpr % 16 == 0: whole rows of lanes are live or idle together
+    {
+        const int t = div_by(blockIdx.x, factor), i = ((int)blockIdx.x - t * per_row) * 256 + threadIdx.x;
+        const bool live = i < cpr;
+        const int c = min(i, cpr - 1) * 4;
         const size_t o = (size_t)t * C + c;
         const f32x4 y4 = *(const f32x4 *)(y + o);
         const h16x4 w4 = *(const h16x4 *)(lnx_w + c), b4 = *(const h16x4 *)(lnx_b + c);
@@ -726,14 +720,11 @@ __global__ __launch_bounds__(DTHREADS) void att7_kernel(const rwkv_half *x, cons
     stream_rows<false, 1, 1, 2, NoEpi, false>(a.lsplit, nseg, 0, nullptr, [] {}, [] {}, [] {}, rowf2, epi_load, epi2);
 }
 
+// besides the leading arguments l1 [rtot], lora2 [C][rtot], state [H][64][64], the stacked rows' total, offsets and ranks
 struct Tmix7Args {
-    int C, rtot, o_a, o_v, o_g, d_w, d_a, d_v, d_g;
-    int first_layer;
-    const rwkv_half *l1;       // [rtot]
-    const rwkv_half *lora2;    // [C][rtot]
+    int C, first_layer;
     const rwkv_half *r, *k, *v, *v_first;   // [C]; v_first unused in layer 0 (there v is the layer-0 value itself)
     const rwkv_half *w0, *a0, *v0, *k_k, *k_a, *r_k, *lnx_w, *lnx_b;
-    float *state;              // [H][64][64]
     rwkv_half *out;            // [C]
     const rwkv_half *commit_src;   // scratch xx -> token-shift state, done by workgroup 0
     rwkv_half *commit_dst;
@@ -745,7 +736,8 @@ struct Tmix7Args {
 // state, wave 0 also the head's vectors.  Then: row sums -> LDS; wave 0 prepares the step; threads 0..255
 // (value rows il + 16 m, key group g = lane & 15, holding S[i][4g..4g+3] of their four rows) advance the
 // state, the sums over a row's key groups being DPP row sums; wave 0 normalises and gates.
-__global__ __launch_bounds__(1024) void tmix7_kernel(Tmix7Args a) {
+__global__ __launch_bounds__(1024) void tmix7_kernel(const rwkv_half *l1, const rwkv_half *lora2, float *state, int rtot, int o_a, int o_v, int o_g,
+                                                    int d_w, int d_a, int d_v, int d_g, Tmix7Args a) {
     __shared__ float lo[4][HS7];
     __shared__ __align__(16) float sr[HS7], sk[HS7], sw[HS7], sa[HS7], sb[HS7];
     __shared__ float sv[HS7], sy[HS7], srk;
@@ -753,17 +745,17 @@ __global__ __launch_bounds__(1024) void tmix7_kernel(Tmix7Args a) {
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int il = (tid >> 4) & 15, g = tid & 15;
     const int c = h * HS7 + lane;
-    float *S = a.state + (size_t)h * HS7 * HS7;
+    float *S = state + (size_t)h * HS7 * HS7;
     // ---- loads
     const int q = w >> 2;
-    const int off = q == 0 ? 0 : (q == 1 ? a.o_a : (q == 2 ? a.o_v : a.o_g));
-    const int d8 = (q == 0 ? a.d_w : (q == 1 ? a.d_a : (q == 2 ? (a.first_layer ? 0 : a.d_v) : a.d_g))) >> 3;
+    const int off = q == 0 ? 0 : (q == 1 ? o_a : (q == 2 ? o_v : o_g));
+    const int d8 = (q == 0 ? d_w : (q == 1 ? d_a : (q == 2 ? d_v : d_g))) >> 3;   // d_v: 0 in the first layer
     const int seg = lane < d8 ? lane : 0;
-    const h16x8 xv = *(const h16x8 *)(a.l1 + off + 8 * seg);
+    const h16x8 xv = *(const h16x8 *)(l1 + off + 8 * seg);
     u32x4 wv[16];
 #pragma unroll
     for (int jj = 0; jj < 16; ++jj)
-        wv[jj] = *(const u32x4 *)(a.lora2 + (size_t)(h * HS7 + (w & 3) * 16 + jj) * a.rtot + off + 8 * seg);
+        wv[jj] = *(const u32x4 *)(lora2 + (size_t)(h * HS7 + (w & 3) * 16 + jj) * rtot + off + 8 * seg);
     f32x4 s[4] = {};
     if (w < 4)
 #pragma unroll
@@ -1054,21 +1046,20 @@ extern "C" int rwkv_v7_forward(const rwkv_v7_model *m, const rwkv_v56_layer_stat
                 a.mat[0] = to_dev56(l.att_receptance); a.mat[1] = to_dev56(l.att_key); a.mat[2] = to_dev56(l.att_value);
                 a.out[0] = ws.r; a.out[1] = ws.k; a.out[2] = v1;
                 a.lora1 = l.lora1; a.rtot = rtot; a.o_a = o_a; a.o_v = o_v; a.o_g = o_g; a.l1 = ws.l1;
-                a.lsplit = row_split(rtot, c.grid);
-                const RowSplit sp = row_split(C, c.grid);
+                a.lsplit = wave_split(rtot, c.grid);
+                const RowSplit sp = wave_split(C, c.grid);
                 hipLaunchKernelGGL(att7_kernel, dim3(c.grid), dim3(DTHREADS), 6 * (size_t)C * 2, st, a.x, a.ln_w, a.ln_b, a.sx, RWKV_SPLIT_PASS(sp),
                                    C, a);
             }
             {
                 Tmix7Args a{};
-                a.C = C; a.rtot = rtot; a.o_a = o_a; a.o_v = o_v; a.o_g = o_g;
-                a.d_w = m->lora_w; a.d_a = m->lora_a; a.d_v = m->lora_v; a.d_g = m->lora_g;
-                a.first_layer = i == 0; a.l1 = ws.l1; a.lora2 = l.lora2;
+                a.C = C; a.first_layer = i == 0;
                 a.r = ws.r; a.k = ws.k; a.v = v1; a.v_first = ws.v_first;
                 a.w0 = l.w0; a.a0 = l.a0; a.v0 = l.v0; a.k_k = l.k_k; a.k_a = l.k_a; a.r_k = l.r_k;
-                a.lnx_w = l.lnx_w; a.lnx_b = l.lnx_b; a.state = s.att_kv; a.out = ws.att;
+                a.lnx_w = l.lnx_w; a.lnx_b = l.lnx_b; a.out = ws.att;
                 a.commit_src = ws.xx_att; a.commit_dst = s.att_xx;
-                hipLaunchKernelGGL(tmix7_kernel, dim3((unsigned)H), dim3(1024), 0, st, a);
+                hipLaunchKernelGGL(tmix7_kernel, dim3((unsigned)H), dim3(1024), 0, st, ws.l1, l.lora2, s.att_kv, rtot, o_a, o_v, o_g, (int)m->lora_w,
+                                   (int)m->lora_a, i == 0 ? 0 : (int)m->lora_v, (int)m->lora_g, a);
             }
             if ((rc = mm(c, l.att_output, false, ws.att, ACT_RESIDUAL, ws.x, nullptr, 1.f, ws.x))) return rc;
             {
@@ -1189,14 +1180,15 @@ extern "C" int rwkv_v7_forward(const rwkv_v7_model *m, const rwkv_v56_layer_stat
                     hipLaunchKernelGGL(wkv7_apply_kernel, dim3((unsigned)(4 * H)), dim3(256), 0, st, H, C, s.att_kv, ws.y32, (int)t0, nchunk, ws.chunks);
                 }
             } else {
-                const int64_t blocks = ((int64_t)T * C / 8 + 255) / 256;
-                hipLaunchKernelGGL(prep7_kernel, dim3((unsigned)std::min<int64_t>(blocks, 65535)), dim3(256), 0, st, a);
+                const int per_row = (C / 8 + 255) / 256;
+                hipLaunchKernelGGL(prep7_kernel, dim3((unsigned)(T * per_row)), dim3(256), 0, st, per_row, div_factor(per_row), a);
                 Wkv7Args q{(int)T, C, s.att_kv, ws.r, ws.dec, ws.k, v, ws.an, ws.b, ws.y32};
                 hipLaunchKernelGGL((wkv7_kernel<RWKV_DT_F16, true>), dim3((unsigned)(4 * H)), dim3(256), 0, st, q);
             }
         }
-        hipLaunchKernelGGL(gn7_kernel, dim3((unsigned)std::min<int64_t>(((int64_t)T * C / 4 + 255) / 256, 65535)), dim3(256), 0, st, (int)T, C, ws.y32 + (T >= CHUNKED7 ? (size_t)CL * C : 0), l.lnx_w, l.lnx_b, ws.rk, v,
-                           ws.g, ws.att);
+        const int per_row = (C / 4 + 255) / 256;
+        hipLaunchKernelGGL(gn7_kernel, dim3((unsigned)(T * per_row)), dim3(256), 0, st, per_row, div_factor(per_row), C,
+                           ws.y32 + (T >= CHUNKED7 ? (size_t)CL * C : 0), l.lnx_w, l.lnx_b, ws.rk, v, ws.g, ws.att);
         if ((rc = mm(c, l.att_output, false, ws.att, ACT_RESIDUAL, ws.x, nullptr, 1.f, ws.x))) return rc;
         // ---- channel mix
         {

@@ -683,17 +683,14 @@ __global__ __launch_bounds__(256, 2) void wkv56_apply_kernel(Wkv56Args a, int H,
 // GroupNorm over each head's 64 outputs (eps 64e-5), affine, fp16 rounding, gate.  Four adjacent channels per lane
 // (16-byte loads of y and of the affine vectors, 8-byte accesses to the gate and the output): a row of 16 lanes owns
 // one head of one token, its two sums are DPP row sums; grid-stride over the T * C / 4 chunks.
-__global__ __launch_bounds__(256) void wkv56_gn_kernel(int T, int C, const float *__restrict__ y,
+__global__ __launch_bounds__(256) void wkv56_gn_kernel(int per_row, uint64_t factor, int C, const float *__restrict__ y,
                                                        const float *__restrict__ lnx_w, const float *__restrict__ lnx_b,
                                                        const rwkv_half *__restrict__ gate, rwkv_half *__restrict__ out) {
-    const int64_t nchunk = (int64_t)T * C / 4;   // a multiple of 16: whole rows of lanes are live or idle together
-    const int cpr = C / 4;
-    for (int64_t i0 = (int64_t)blockIdx.x * 256; i0 < nchunk; i0 += (int64_t)gridDim.x * 256) {
-        const int64_t i = i0 + threadIdx.x;
-        const bool live = i < nchunk;
-        const int64_t ic = live ? i : nchunk - 1;
-        const int64_t t = ic / cpr;
-        const int c = (int)(ic - t * cpr) * 4;
+    const int cpr = C / 4;   // a multiple of 16: whole rows of lanes are live or idle together
+    {
+        const int t = div_by(blockIdx.x, factor), i = ((int)blockIdx.x - t * per_row) * 256 + threadIdx.x;
+        const bool live = i < cpr;
+        const int c = min(i, cpr - 1) * 4;
         const size_t o = (size_t)t * C + c;
         const f32x4 y4 = *(const f32x4 *)(y + o), w4 = *(const f32x4 *)(lnx_w + c), b4 = *(const f32x4 *)(lnx_b + c);
         h16x4 g4 = {};
@@ -796,8 +793,9 @@ int wkv56_fused_launch(bool v6, int T, int C, int H, float *state, const rwkv_ha
             else hipLaunchKernelGGL((wkv56_chunk_kernel<0>), grid, dim3(256), 0, st, a, H, t0, chunks);
             hipLaunchKernelGGL(wkv56_apply_kernel, dim3((unsigned)(4 * H)), dim3(256), 0, st, a, H, t0, nchunk, chunks);
         }
-        hipLaunchKernelGGL(wkv56_gn_kernel, dim3((unsigned)std::min<int64_t>(((int64_t)T * C / 4 + 255) / 256, 65535)), dim3(256), 0, st,
-                           T, C, y32, lnx_w, lnx_b, gate, out);
+        const int per_row = (C / 4 + 255) / 256;
+        hipLaunchKernelGGL(wkv56_gn_kernel, dim3((unsigned)(T * per_row)), dim3(256), 0, st, per_row, div_factor(per_row), C, y32, lnx_w, lnx_b,
+                           gate, out);
     } else if (v6 && dw2) {
         if (ld <= 0 || (ld & 7)) return RWKV_E_SHAPE;
         hipLaunchKernelGGL((wkv56_kernel<true, 3, true>), dim3((unsigned)H), dim3(256), 0, st, a);
