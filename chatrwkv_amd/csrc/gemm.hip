@@ -1433,6 +1433,302 @@ int launch_kg(GemmGroup &g, int n, int64_t T, int64_t N, int ks, hipStream_t st)
     return RWKV_OK;
 }
 
+// ---- few rows: tiles of 32, 48 or 64 rows and 16 to 96 columns ----------------------------------------------------
+// Calls of 17 to 64 rows are bound by how fast a CU takes its operands, 50 GB/s with a tile's activations at twice the bytes of its
+// uint8 weights, so what counts is that every CU has the same share and no rows past the end: 12288 outputs are 192 tiles of 64 x 64
+// and 256 of 48 x 48.  The form is that of gemm_kg_kernel (the waves share K, partial blocks meet in LDS and are added in group order)
+// with v_mfma_f32_16x16x32_f16, whose blocks make sides of any multiple of 16: KG = 8 groups of one wave, or four of two waves side by
+// side, and 32 k's a wave and stage, so that a stage is one MFMA step.  A stage's 1 KB loads are dealt to the waves, activations
+// and weights alike; the last ones repeat where they do not divide.
+template <bool W_U8, int TM, int TN> struct FewCfg {
+    static constexpr int RB = TN == 16 || TN == 48 ? 1 : 2, KG = 8 / RB, BKS = 32 * KG;   // waves side by side, groups that share K, k's of a stage
+    static constexpr int AB = BKS * 2, WB = BKS * (W_U8 ? 1 : 2);                         // bytes of a row
+    static constexpr int A = TM * AB, STAGE = A + TN * WB, AP = A / 1024, PIECES = STAGE / 1024, LOADS = (PIECES + 7) / 8;
+    static constexpr int NST = (160 * 1024 - 2 * TM * 4) / STAGE < 4 ? (160 * 1024 - 2 * TM * 4) / STAGE : 4;
+    static constexpr int MI = TM / 16, NI = TN / (16 * RB);                               // 16 x 16 blocks of a wave
+    static constexpr int SW = TN / RB + 4, REGION = TM * SW * 4;                          // partial tile of a wave: row stride (floats), bytes
+    static constexpr int BODY = NST * STAGE > 8 * REGION ? NST * STAGE : 8 * REGION, LDS = BODY + (W_U8 ? 2 * TM * 4 : 0);
+    static constexpr int CPR = TN <= 16 ? 2 : TN <= 32 ? 4 : TN <= 64 ? 8 : 16;           // threads that finish a row, eight outputs each
+    static_assert(TM % 16 == 0 && TN % (16 * RB) == 0 && A % 1024 == 0 && STAGE % 1024 == 0 && NST >= 2 && LDS <= 160 * 1024, "tile");
+};
+template <bool W_U8, int TM, int TN>
+__global__ __launch_bounds__(512) void gemm_few_kernel(int T, int units, int splits, int first1, int first2, int first3, int nk_split, int64_t lda,
+                                                       GemmMembers g) {
+    using Cfg = FewCfg<W_U8, TM, TN>;
+    constexpr int NST = Cfg::NST, STAGE = Cfg::STAGE, LOADS = Cfg::LOADS, BKS = Cfg::BKS, AB = Cfg::AB, WB = Cfg::WB, MI = Cfg::MI, NI = Cfg::NI;
+    constexpr int KG = Cfg::KG, RB = Cfg::RB, SW = Cfg::SW, REGION = Cfg::REGION, CPR = Cfg::CPR;
+    extern __shared__ __align__(1024) unsigned char smem[];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int grp = wave / RB, wc = wave % RB;
+    const int unit = xcd_unit(units);
+    int tile = splits > 1 ? unit / splits : unit;
+    const int split = splits > 1 ? unit - tile * splits : 0;
+    const GemmMember &mb = g.m[group_member(first1, first2, first3, tile)];
+    const GemmIn in = gemm_in(mb);
+    const int M = in.M;
+    const TileAt at = tile_at<TM, TN>(tile, T, M, in.walk_m);
+    const int t0 = at.t0, m0 = at.m0;
+    const int kbase = split * nk_split * BK, K = nk_split * BK, nk = (K + BKS - 1) / BKS;
+
+    // load i of this wave: 1 KB of a stage, whole rows; rows past the end re-read the last row (never stored).  The lane that fills
+    // slot p of row r fetches chunk p ^ key(r).
+    const unsigned char *src[LOADS];
+    int klane[LOADS], kb[LOADS];   // this lane's first k of a stage; bytes per k
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) {
+        const int p = min(wave + 8 * i, Cfg::PIECES - 1);
+        if (p < Cfg::AP) {
+            const int r = p * (1024 / AB) + lane / (AB / 16), c = (lane % (AB / 16)) ^ kg_key<AB>(r);
+            klane[i] = c * 8;
+            kb[i] = 2;
+            src[i] = (const unsigned char *)(in.A + (size_t)min(t0 + r, T - 1) * lda + kbase + klane[i]);
+        } else {
+            const int r = (p - Cfg::AP) * (1024 / WB) + lane / (WB / 16), c = (lane % (WB / 16)) ^ kg_key<WB>(r);
+            klane[i] = c * (W_U8 ? 16 : 8);
+            kb[i] = W_U8 ? 1 : 2;
+            src[i] = (const unsigned char *)in.W + ((size_t)min(m0 + r, M - 1) * in.ldw + kbase + klane[i]) * (W_U8 ? 1 : 2);
+        }
+    }
+    typedef __attribute__((address_space(1))) const void *gptr;
+    typedef __attribute__((address_space(3))) void *lptr;
+    auto issue = [&](int kt, int so) {
+#pragma unroll
+        for (int i = 0; i < LOADS; ++i)
+            __builtin_amdgcn_global_load_lds((gptr)(src[i] + kt * BKS * kb[i]), (lptr)(smem + so + min(wave + 8 * i, Cfg::PIECES - 1) * 1024), 16, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto issue_any = [&](int kt, int so) {
+        if (kt * BKS + BKS <= K) { issue(kt, so); return; }
+        // the last stage of a K that is no multiple of BKS: chunks past the end fetch k's 0 .. 63 (never multiplied)
+#pragma unroll
+        for (int i = 0; i < LOADS; ++i) {
+            const int d = kt * BKS + klane[i] < K ? kt * BKS : (klane[i] & 63) - klane[i];
+            __builtin_amdgcn_global_load_lds((gptr)(src[i] + d * kb[i]), (lptr)(smem + so + min(wave + 8 * i, Cfg::PIECES - 1) * 1024), 16, 0, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+
+    f32x4 acc[MI][NI];
+#pragma unroll
+    for (int a = 0; a < MI; ++a)
+#pragma unroll
+        for (int b = 0; b < NI; ++b) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+    // fragments: lane (row, q) of group g takes the k's 32 g + 8 q .. + 7 of the stage, for both operands
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)smem;
+    const int row = lane & 15, q = lane >> 4;
+    uint32_t vA[MI], vW[NI];   // the swizzle keys of a block's rows depend on the block where a row is 256 bytes or more
+#pragma unroll
+    for (int a = 0; a < MI; ++a) vA[a] = lds0 + (a * 16 + row) * AB + (((4 * grp + q) ^ kg_key<AB>(a * 16 + row)) << 4);
+#pragma unroll
+    for (int b = 0; b < NI; ++b) {
+        const int r = wc * 16 * NI + b * 16 + row;
+        vW[b] = lds0 + Cfg::A + r * WB + (((W_U8 ? 2 * grp + (q >> 1) : 4 * grp + q) ^ kg_key<WB>(r)) << 4) + (W_U8 ? (q & 1) * 8 : 0);
+    }
+    h16x8 fa[2][MI], fb[2][NI];
+    u32x2 raw[2][NI];
+    auto ldstage = [&](int set, int so) {
+#pragma unroll
+        for (int b = 0; b < NI; ++b) {
+            if constexpr (W_U8) asm volatile("ds_read_b64 %0, %1" : "=v"(raw[set][b]) : "v"(vW[b] + so));
+            else asm volatile("ds_read_b128 %0, %1" : "=v"(fb[set][b]) : "v"(vW[b] + so));
+        }
+#pragma unroll
+        for (int a = 0; a < MI; ++a) asm volatile("ds_read_b128 %0, %1" : "=v"(fa[set][a]) : "v"(vA[a] + so));
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    const h16x2 off = {(h16)1023.5f, (h16)1023.5f};
+    auto mul = [&](int set) {
+#pragma unroll
+        for (int b = 0; b < NI; ++b) {
+            h16x8 w;
+            if constexpr (W_U8) {
+                const u32x2 v = raw[set][b];
+                const h16x2 q0 = u8pair_lo_1024(v.x) - off, q1 = u8pair_hi_1024(v.x) - off, q2 = u8pair_lo_1024(v.y) - off, q3 = u8pair_hi_1024(v.y) - off;
+                w = h16x8{q0.x, q0.y, q1.x, q1.y, q2.x, q2.y, q3.x, q3.y};
+            } else {
+                w = fb[set][b];
+            }
+#pragma unroll
+            for (int a = 0; a < MI; ++a) acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w, fa[set][a], acc[a][b], 0, 0, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto reads_done = [&]() {
+        __builtin_amdgcn_s_waitcnt(lgkm_only(0));
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    const GemmEpi &ep = mb.ep;
+#pragma unroll
+    for (int s = 0; s < NST; ++s)
+        if (s < nk) issue_any(s, s * STAGE);
+    bool lds_sums = false;
+    float *lsum = (float *)(smem + Cfg::BODY);
+    if constexpr (W_U8) {
+        if (ep.parts > 1 && (splits == 1 || (m0 == 0 && split == 0))) {   // as in gemm_dma_body
+            lds_sums = splits == 1;
+            if (tid < 2 * TM) {
+                const int r = tid % TM, which = tid / TM, t = min(t0 + r, T - 1);
+                const float *p = (which ? ep.p2 : ep.p0) + (size_t)t * ep.parts;
+                float tot = 0.f;
+                for (int j = 0; j < ep.parts; j += 64) {
+                    f32x4 v[16];
+#pragma unroll
+                    for (int u = 0; u < 16; ++u) v[u] = j + 4 * u < ep.parts ? *(const f32x4 *)(p + j + 4 * u) : f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                    for (int u = 0; u < 16; ++u) tot = (((tot + v[u][0]) + v[u][1]) + v[u][2]) + v[u][3];
+                }
+                if (splits > 1) {
+                    if (t0 + r < T) (which ? (float *)ep.s2 : (float *)ep.s0)[t] = tot;
+                } else {
+                    lsum[tid] = tot;
+                }
+            }
+        }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    if (nk >= NST) __builtin_amdgcn_s_waitcnt(vm_lgkm0((NST - 1) * LOADS));   // my part of stage 0 has landed
+    else __builtin_amdgcn_s_waitcnt(vm_lgkm0(0));
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    int so = 0;
+    ldstage(0, 0);
+    reads_done();
+    // One stage: past its barrier stage kt + 1 has landed for every wave and nobody reads stage kt any more, so stage kt + NST goes
+    // where it was.  STEADY: that one is there and whole.
+    auto stage = [&](auto steady, int kt, int set) {
+        constexpr bool STEADY = decltype(steady)::value;
+        const int sn = so + STAGE >= NST * STAGE ? 0 : so + STAGE;
+        if (STEADY || kt + NST <= nk) __builtin_amdgcn_s_waitcnt(vm_only((NST - 2) * LOADS));
+        else __builtin_amdgcn_s_waitcnt(vm_only(0));
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+        ldstage(set ^ 1, sn);
+        if constexpr (STEADY) issue(kt + NST, so);
+        else if (kt + NST < nk) issue_any(kt + NST, so);
+        if (STEADY || kt * BKS + grp * 32 < K) mul(set);   // the wave's k's of the last stage may be past the end
+        reads_done();
+        so = sn;
+    };
+    int kt = 0;
+    const int steady = max(K / BKS - NST, 0) & ~1;   // stage kt + NST is whole for kt < K / BKS - NST
+    for (; kt < steady; kt += 2) {
+        stage(std::true_type{}, kt, 0);
+        stage(std::true_type{}, kt + 1, 1);
+    }
+    for (; kt < nk; kt += 2) {   // an odd number of stages ends with one in which nobody multiplies
+        stage(std::false_type{}, kt, 0);
+        stage(std::false_type{}, kt + 1, 1);
+    }
+    // nothing may land in LDS or in a fragment register after this point (see gemm_dma_body)
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_waitcnt(0x0070);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int set = 0; set < 2; ++set) {
+#pragma unroll
+        for (int b = 0; b < NI; ++b) {
+            if constexpr (W_U8) asm volatile("" ::"v"(raw[set][b]));
+            else asm volatile("" ::"v"(fb[set][b]));
+        }
+#pragma unroll
+        for (int a = 0; a < MI; ++a) asm volatile("" ::"v"(fa[set][a]));
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    __syncthreads();   // every wave has read its last fragments: the partial tiles go where the stages were
+    float *mypart = (float *)(smem + wave * REGION);
+#pragma unroll
+    for (int a = 0; a < MI; ++a)
+#pragma unroll
+        for (int b = 0; b < NI; ++b) *(f32x4 *)(mypart + (a * 16 + row) * SW + b * 16 + 4 * q) = acc[a][b];
+    auto tile_sum = [&](int r, int c) {   // four values at tile row r, column c: the groups' in group order
+        const int half = RB == 2 && c >= TN / 2 ? 1 : 0;
+        const float *p = (const float *)(smem + half * REGION) + r * SW + c - half * (TN / 2);
+        f32x4 v = *(const f32x4 *)p;
+#pragma unroll
+        for (int k = 1; k < KG; ++k) v += *(const f32x4 *)(p + k * (RB * REGION / 4));
+        return v;
+    };
+    constexpr int RPI = 512 / CPR, ITS = (TM + RPI - 1) / RPI;   // rows of a pass, passes
+    const int cq = tid % CPR, col = m0 + cq * 8;
+    const bool in_tile = cq * 8 < TN, col_ok = in_tile && col < M;
+    if (splits > 1) {
+        __syncthreads();
+        float *slab = mb.part + (size_t)split * T * M;
+#pragma unroll
+        for (int it = 0; it < ITS; ++it) {
+            const int r = it * RPI + tid / CPR, t = t0 + r;
+            if (r >= TM || t >= T || !col_ok) continue;
+            *(f32x4 *)(slab + (size_t)t * M + col) = tile_sum(r, cq * 8);                                   // M % 4 == 0
+            if (col + 4 < M) *(f32x4 *)(slab + (size_t)t * M + col + 4) = tile_sum(r, cq * 8 + 4);
+        }
+        return;
+    }
+    if (by_four(M, mb.ldy, mb.Y, ep)) {   // a loop of its own, as in gemm_dma_body
+        __syncthreads();
+#pragma unroll 1
+        for (int it = 0; it < ITS; ++it) {
+            const int r = it * RPI + tid / CPR, t = t0 + r;
+            if (r >= TM || t >= T) break;
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                const int c = e * (TN / 2) + cq * 4;
+                if (!in_tile || m0 + c >= M) continue;
+                f32x4 v = tile_sum(r, c);
+                if constexpr (W_U8) affine4(v, m0 + c, M, lds_sums ? lsum[r] : ep.s0[t], lds_sums ? lsum[TM + r] : ep.s2[t], ep);
+                finish_row4(v, t, m0 + c, M, ep, mb.Y, mb.ldy);
+            }
+        }
+        return;
+    }
+    h16x8 rx8 = {}, mx8 = {};
+    EpiIn ein[ITS] = {};
+    if (W_U8 && col_ok) { rx8 = load_n<h16x8, 8>(ep.rx + col, M - col); mx8 = load_n<h16x8, 8>(ep.mx + col, M - col); }
+    const Emit8 em = emit8(ep, col, col_ok);
+#pragma unroll
+    for (int it = 0; it < ITS; ++it) {
+        const int r = it * RPI + tid / CPR, t = t0 + r;
+        ein[it] = epi_in(ep, t, col, r < TM && t < T && col_ok, W_U8 && !lds_sums);
+    }
+    __syncthreads();   // the partial tiles are in LDS
+#pragma unroll 1
+    for (int it = 0; it < ITS; ++it) {
+        const EpiIn cur = ein[0];
+#pragma unroll
+        for (int i = 0; i + 1 < ITS; ++i) ein[i] = ein[i + 1];
+        const int r = it * RPI + tid / CPR, t = t0 + r;
+        const bool valid = r < TM && t < T && col_ok;
+        float a0 = 0.f, a2 = 0.f;
+        if (valid) {
+            const f32x4 lo = tile_sum(r, cq * 8), hi = tile_sum(r, cq * 8 + 4);
+            float v[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+            if constexpr (W_U8) affine8(v, rx8, mx8, lds_sums ? lsum[r] : cur.s0, lds_sums ? lsum[TM + r] : cur.s2);
+            finish_row8<true>(v, cur, t, col, ep, mb.Y, mb.ldy, em, a0, a2);
+        }
+        if (ep.emit_ry) {   // the CPR threads of a row are neighbours in one wave; every lane takes part
+#pragma unroll
+            for (int o = 1; o < CPR; o <<= 1) { a0 += __shfl_xor(a0, o, WAVE); a2 += __shfl_xor(a2, o, WAVE); }
+            if (valid && cq == 0) emit_parts(ep, t, m0, M, TN, a0, a2);
+        }
+    }
+}
+
+template <bool W_U8, int TM, int TN>
+int launch_few(GemmGroup &g, int n, int64_t T, int64_t N, int ks, hipStream_t st) {
+    constexpr int lds = FewCfg<W_U8, TM, TN>::LDS;
+    static PerDeviceOnce once;
+    bool *attr_done = once.slot();
+    if (!attr_done || !*attr_done) {
+        const hipError_t e = hipFuncSetAttribute((const void *)gemm_few_kernel<W_U8, TM, TN>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+        if (e != hipSuccess) return (int)e;
+        if (attr_done) *attr_done = true;
+    }
+    const int units = (int)group_tiles(W_U8, g, n, T, N, TM, TN) * ks;
+    hipLaunchKernelGGL((gemm_few_kernel<W_U8, TM, TN>), dim3((unsigned)units), dim3(512), lds, st, (int)T, units, ks, g.first[1], g.first[2], g.first[3],
+                       g.nk_split, g.lda, (const GemmMembers &)g);
+    RWKV_LAUNCH_CHECK();
+    return RWKV_OK;
+}
+
 // second pass of a split group launch: member blockIdx.y, as splitk_epilogue8_kernel
 struct SplitFactors { uint64_t f[4]; };
 __global__ __launch_bounds__(256) void splitk_group_epilogue8_kernel(int T, int KS, SplitFactors rows, GemmMembers g) {
@@ -1982,61 +2278,95 @@ bool dma_ok(bool w_u8, int64_t N, int64_t M, const void *A, int64_t lda, const v
 // and K over two groups, TILE_N 64 x 128 with four waves, TILE_K8 and TILE_K4 gemm_kg_kernel with eight and four groups.
 enum {
     TILE_256x256, TILE_S, TILE_S4, TILE_N, TILE_K8, TILE_K4, TILE_256x192, TILE_224x256, TILE_224x192, TILE_192x256, TILE_192x192,
-    TILE_160x256, TILE_160x192, TILE_128x256, TILE_128x192, TILES
+    TILE_160x256, TILE_160x192, TILE_128x256, TILE_128x192,
+    TILE_32x16, TILE_32x32, TILE_32x48, TILE_32x64, TILE_32x96, TILE_48x16, TILE_48x32, TILE_48x48, TILE_48x64, TILE_48x96, TILE_64x16, TILE_64x32, TILE_64x48, TILE_64x64, TILE_64x96, TILES
 };
 struct TileDim { int tm, tn; };
 constexpr TileDim tile_dim[TILES] = {{256, 256}, {128, 128}, {128, 128}, {64, 128}, {64, 64}, {64, 128}, {256, 192}, {224, 256}, {224, 192},
-                                     {192, 256}, {192, 192}, {160, 256}, {160, 192}, {128, 256}, {128, 192}};
+                                     {192, 256}, {192, 192}, {160, 256}, {160, 192}, {128, 256}, {128, 192},
+                                     {32, 16}, {32, 32}, {32, 48}, {32, 64}, {32, 96}, {48, 16}, {48, 32}, {48, 48}, {48, 64}, {48, 96}, {64, 16}, {64, 32}, {64, 48}, {64, 64}, {64, 96}};
 
 // Cost model of a direct-to-LDS launch in microseconds.  `tiles` tiles of nk k-tiles split c ways run in rounds over the 256 CUs:
 //   launch + rounds * (round, or split_round, which leaves the epilogue to the second pass)
 //          + k-tiles * (step_1 for every full round, between step_0 and step_1 for the last one by the CUs busy,
 //                       extra for what exceeds one round)
 //          + with a split, slab per 16 MB of fp32 slabs written and read and split per slab.
-// One fit per tile and type, over launches within 1.6 times the best one of 342 products each (18 lengths from 24 to 2048 rows, 19 widths
-// from 512 to 16384; weights from HBM; the chip under load before): the tile and split it picks takes 0.6 % (uint8) and 1.1 %
-// (fp16) longer than the best of all on average.  A tile per round costs between 5 and 13 us whatever K is, so
-// tiles of many sizes pay: each of these is the best one somewhere, the ones with sides of 160, 192 and 224 where 256 x 256 or 128 x
-// 128 leave CUs idle or rows empty.  us, uint8 / fp16 weights: [1024 x 4096] x [4096 x 12288] three rounds of 128 x 128 115.7 / 132.5,
-// one of 256 x 192 90 / 97; [777 x 4096] x [4096 x 16384] 256 x 256 126 / 130, 224 x 256 100 / 107; [768 x 4096] x [4096 x 12288]
-// 104 / 109, 192 x 192 71 / 80.
+// One fit per tile and type, over launches within 1.6 times the best one of 648 products each (24 lengths from 17 to 2048 rows, 27 widths
+// from 64 to 20480; weights from HBM; the chip under load before): the tile and split it picks takes 1 % (uint8) and 2 %
+// (fp16) longer than the best of all on average, with products that the host launches no faster counted in.  A tile per round costs
+// between 3 and 15 us whatever K is, so tiles of many sizes pay: each of these is the best one somewhere, the large ones with sides of
+// 160, 192 and 224 where 256 x 256 or 128 x 128 leave CUs idle or rows empty, those of 32, 48 and 64 rows in calls of up to 128 rows.
+// us, uint8 / fp16 weights: [1024 x 4096] x [4096 x 12288] three rounds of 128 x 128 115.7 / 132.5, one of 256 x 192 90 / 97; [777 x
+// 4096] x [4096 x 16384] 256 x 256 126 / 130, 224 x 256 100 / 107; [768 x 4096] x [4096 x 12288] 104 / 109, 192 x 192 71 / 80;
+// [45 x 4096] x [4096 x 4096] four splits of 64 x 64 11.0 / 12.4, 48 x 16 8.7 / 10.6; [45 x 4096] x [4096 x 20480] 64 x 128 26.5 /
+// 40.6, 48 x 96 23.8 / 37.9; [24 x 2048] x [2048 x 2048] 8.1 / 8.1, 32 x 16 5.6 / 5.5.
 struct TilePrice { float launch, round, split_round, step_0, step_1, extra, slab, split; };
 constexpr TilePrice tile_price[2][TILES] = {
     {   // fp16 weights
-        {5.831f, 8.813f, 6.274f, 0.999f, 1.721f, 0.057f, 4.252f, 0.121f},   // 256x256
-        {2.012f, 3.875f, 4.591f, 0.415f, 0.619f, 0.008f, 5.344f, 0.221f},   // S
-        {1.500f, 4.656f, 4.697f, 0.295f, 0.569f, 0.f, 8.799f, 0.192f},   // S4
-        {3.105f, 1.893f, 2.537f, 0.343f, 0.679f, 0.f, 5.957f, 0.f},   // N
-        {1.794f, 2.270f, 3.851f, 0.149f, 0.240f, 0.f, 5.660f, 0.286f},   // K8
-        {1.905f, 2.896f, 3.736f, 0.230f, 0.387f, 0.f, 8.168f, 0.240f},   // K4
-        {3.022f, 10.904f, 7.859f, 0.832f, 1.358f, 0.f, 4.391f, 0.f},   // 256x192
-        {5.969f, 8.112f, 7.071f, 0.932f, 1.539f, 0.f, 3.668f, 0.091f},   // 224x256
-        {4.430f, 7.532f, 4.378f, 0.755f, 1.210f, 0.f, 4.956f, 0.152f},   // 224x192
-        {4.085f, 7.060f, 6.380f, 0.874f, 1.374f, 0.f, 4.356f, 0.188f},   // 192x256
-        {3.593f, 5.714f, 3.553f, 0.666f, 1.112f, 0.f, 5.118f, 0.311f},   // 192x192
-        {3.679f, 5.143f, 5.127f, 0.739f, 1.260f, 0.f, 4.542f, 0.330f},   // 160x256
-        {5.327f, 3.260f, 2.487f, 0.560f, 1.102f, 0.f, 4.280f, 0.251f},   // 160x192
-        {4.914f, 4.682f, 4.923f, 0.666f, 1.069f, 0.011f, 4.250f, 0.094f},   // 128x256
-        {3.239f, 5.415f, 4.335f, 0.532f, 0.829f, 0.006f, 5.058f, 0.207f},   // 128x192
+        {4.549f, 9.813f, 10.035f, 0.941f, 1.721f, 0.081f, 3.477f, 0.f},   // 256x256
+        {2.456f, 3.248f, 4.838f, 0.423f, 0.631f, 0.f, 4.568f, 0.076f},   // S
+        {1.871f, 4.556f, 4.704f, 0.298f, 0.575f, 0.f, 7.450f, 0.136f},   // S4
+        {2.546f, 2.311f, 1.782f, 0.363f, 0.699f, 0.f, 8.143f, 0.073f},   // N
+        {1.987f, 2.281f, 4.023f, 0.141f, 0.253f, 0.f, 4.754f, 0.175f},   // K8
+        {1.808f, 3.209f, 4.405f, 0.217f, 0.391f, 0.f, 7.476f, 0.162f},   // K4
+        {4.715f, 8.832f, 6.523f, 0.825f, 1.348f, 0.067f, 4.078f, 0.019f},   // 256x192
+        {5.750f, 7.778f, 9.926f, 0.869f, 1.545f, 0.f, 2.620f, 0.f},   // 224x256
+        {5.169f, 7.209f, 5.179f, 0.704f, 1.218f, 0.005f, 4.432f, 0.f},   // 224x192
+        {5.462f, 5.451f, 8.367f, 0.833f, 1.404f, 0.034f, 2.485f, 0.067f},   // 192x256
+        {6.233f, 4.192f, 4.042f, 0.576f, 1.135f, 0.013f, 3.789f, 0.014f},   // 192x192
+        {5.662f, 4.463f, 7.448f, 0.729f, 1.266f, 0.f, 2.506f, 0.064f},   // 160x256
+        {6.807f, 2.897f, 4.219f, 0.444f, 1.116f, 0.f, 2.900f, 0.f},   // 160x192
+        {3.811f, 5.068f, 6.800f, 0.674f, 1.048f, 0.f, 4.031f, 0.006f},   // 128x256
+        {3.662f, 4.895f, 5.956f, 0.520f, 0.831f, 0.015f, 3.948f, 0.f},   // 128x192
+        {2.064f, 1.754f, 1.770f, 0.045f, 0.071f, 0.029f, 8.577f, 0.499f},   // 32x16
+        {3.459f, 0.f, 0.708f, 0.075f, 0.127f, 0.004f, 0.f, 0.356f},   // 32x32
+        {2.995f, 1.030f, 2.668f, 0.077f, 0.169f, 0.031f, 0.f, 0.107f},   // 32x48
+        {2.020f, 1.586f, 3.023f, 0.107f, 0.209f, 0.002f, 0.f, 0.249f},   // 32x64
+        {2.242f, 1.739f, 3.490f, 0.122f, 0.309f, 0.f, 1.050f, 0.125f},   // 32x96
+        {2.035f, 1.839f, 2.184f, 0.066f, 0.101f, 0.019f, 5.215f, 0.412f},   // 48x16
+        {3.611f, 0.f, 0.981f, 0.097f, 0.180f, 0.f, 0.f, 0.295f},   // 48x32
+        {3.170f, 1.064f, 2.539f, 0.091f, 0.237f, 0.019f, 6.597f, 0.109f},   // 48x48
+        {2.941f, 0.957f, 2.587f, 0.118f, 0.329f, 0.f, 2.137f, 0.100f},   // 48x64
+        {3.241f, 1.435f, 2.964f, 0.140f, 0.488f, 0.f, 2.435f, 0.047f},   // 48x96
+        {3.061f, 0.871f, 1.378f, 0.080f, 0.124f, 0.043f, 0.f, 0.407f},   // 64x16
+        {3.389f, 0.364f, 1.904f, 0.101f, 0.197f, 0.061f, 0.317f, 0.153f},   // 64x32
+        {4.503f, 0.040f, 1.948f, 0.095f, 0.337f, 0.117f, 0.f, 0.027f},   // 64x48
+        {2.451f, 1.661f, 3.319f, 0.136f, 0.330f, 0.f, 4.174f, 0.119f},   // 64x64
+        {2.816f, 2.220f, 3.033f, 0.188f, 0.429f, 0.f, 7.091f, 0.094f},   // 64x96
     }, {   // uint8
-        {7.170f, 10.217f, 5.543f, 0.968f, 1.566f, 0.135f, 3.946f, 0.041f},   // 256x256
-        {6.880f, 0.f, 0.706f, 0.350f, 0.540f, 0.f, 4.587f, 0.162f},   // S
-        {4.450f, 3.447f, 2.539f, 0.315f, 0.506f, 0.078f, 6.311f, 0.207f},   // S4
-        {5.812f, 0.f, 0.f, 0.366f, 0.434f, 0.f, 7.064f, 0.099f},   // N
-        {2.045f, 2.974f, 4.338f, 0.117f, 0.181f, 0.011f, 4.108f, 0.195f},   // K8
-        {2.545f, 2.923f, 3.674f, 0.204f, 0.308f, 0.040f, 7.536f, 0.156f},   // K4
-        {6.193f, 9.593f, 4.232f, 0.804f, 1.215f, 0.128f, 4.631f, 0.f},   // 256x192
-        {7.017f, 9.153f, 6.790f, 0.867f, 1.441f, 0.065f, 3.205f, 0.f},   // 224x256
-        {5.264f, 9.053f, 5.484f, 0.692f, 1.136f, 0.036f, 4.223f, 0.f},   // 224x192
-        {5.750f, 7.695f, 7.373f, 0.748f, 1.266f, 0.077f, 3.127f, 0.016f},   // 192x256
-        {5.691f, 6.511f, 4.394f, 0.609f, 1.021f, 0.070f, 4.032f, 0.017f},   // 192x192
-        {5.144f, 6.870f, 6.213f, 0.706f, 1.125f, 0.046f, 3.505f, 0.076f},   // 160x256
-        {4.537f, 6.501f, 4.429f, 0.518f, 0.869f, 0.050f, 4.330f, 0.101f},   // 160x192
-        {7.339f, 3.059f, 2.299f, 0.598f, 0.967f, 0.109f, 4.353f, 0.040f},   // 128x256
-        {6.131f, 3.390f, 2.807f, 0.530f, 0.755f, 0.111f, 4.612f, 0.060f},   // 128x192
+        {5.336f, 9.067f, 8.377f, 0.949f, 1.642f, 0.022f, 3.336f, 0.f},   // 256x256
+        {6.522f, 0.f, 0.599f, 0.349f, 0.546f, 0.f, 4.631f, 0.085f},   // S
+        {3.456f, 3.989f, 3.830f, 0.317f, 0.523f, 0.041f, 5.040f, 0.081f},   // S4
+        {5.441f, 0.f, 0.f, 0.346f, 0.468f, 0.f, 6.072f, 0.143f},   // N
+        {1.922f, 3.185f, 4.514f, 0.115f, 0.176f, 0.013f, 6.113f, 0.121f},   // K8
+        {1.799f, 3.765f, 4.212f, 0.200f, 0.305f, 0.021f, 7.262f, 0.149f},   // K4
+        {5.813f, 9.209f, 4.665f, 0.786f, 1.222f, 0.067f, 4.361f, 0.f},   // 256x192
+        {6.485f, 8.992f, 8.275f, 0.837f, 1.443f, 0.027f, 2.592f, 0.f},   // 224x256
+        {5.976f, 8.521f, 5.926f, 0.677f, 1.123f, 0.072f, 3.349f, 0.f},   // 224x192
+        {5.631f, 7.400f, 8.116f, 0.702f, 1.282f, 0.041f, 2.417f, 0.089f},   // 192x256
+        {5.123f, 7.379f, 3.369f, 0.573f, 0.988f, 0.088f, 4.369f, 0.092f},   // 192x192
+        {5.432f, 6.626f, 6.901f, 0.678f, 1.133f, 0.029f, 2.803f, 0.050f},   // 160x256
+        {6.671f, 4.130f, 4.142f, 0.495f, 0.891f, 0.104f, 3.467f, 0.f},   // 160x192
+        {6.383f, 3.449f, 3.229f, 0.589f, 0.939f, 0.128f, 3.964f, 0.092f},   // 128x256
+        {6.019f, 3.214f, 3.148f, 0.518f, 0.752f, 0.093f, 4.309f, 0.040f},   // 128x192
+        {1.699f, 2.323f, 2.288f, 0.041f, 0.055f, 0.f, 12.951f, 0.432f},   // 32x16
+        {3.999f, 0.f, 0.899f, 0.066f, 0.083f, 0.004f, 2.289f, 0.215f},   // 32x32
+        {2.913f, 1.532f, 3.101f, 0.071f, 0.098f, 0.023f, 2.608f, 0.078f},   // 32x48
+        {4.114f, 0.f, 1.196f, 0.086f, 0.112f, 0.015f, 3.985f, 0.176f},   // 32x64
+        {3.385f, 1.010f, 2.444f, 0.122f, 0.163f, 0.054f, 6.361f, 0.100f},   // 32x96
+        {4.058f, 0.069f, 1.352f, 0.059f, 0.074f, 0.028f, 8.241f, 0.155f},   // 48x16
+        {4.037f, 0.f, 0.851f, 0.079f, 0.097f, 0.028f, 2.529f, 0.277f},   // 48x32
+        {4.127f, 0.628f, 2.240f, 0.092f, 0.127f, 0.097f, 5.425f, 0.035f},   // 48x48
+        {4.308f, 0.f, 1.565f, 0.115f, 0.151f, 0.106f, 7.660f, 0.069f},   // 48x64
+        {4.278f, 0.820f, 2.197f, 0.129f, 0.229f, 0.081f, 5.005f, 0.020f},   // 48x96
+        {4.043f, 0.282f, 1.457f, 0.076f, 0.091f, 0.003f, 12.132f, 0.137f},   // 64x16
+        {4.251f, 0.f, 1.418f, 0.100f, 0.124f, 0.088f, 6.335f, 0.096f},   // 64x32
+        {4.608f, 0.525f, 1.966f, 0.106f, 0.147f, 0.088f, 4.921f, 0.074f},   // 64x48
+        {4.535f, 0.f, 1.492f, 0.129f, 0.173f, 0.093f, 8.795f, 0.060f},   // 64x64
+        {5.097f, 0.529f, 1.525f, 0.160f, 0.257f, 0.103f, 6.215f, 0.071f},   // 64x96
     }};
 double dma_cost(bool w_u8, int tile, int64_t T, int64_t tiles, int nk, int c, size_t out_bytes) {
-    if (tile == TILE_N && T > 64) return 1e30;
+    if (T > (tile == TILE_N ? 64 : tile < TILE_32x16 ? T : tile_dim[tile].tn <= 32 ? 128 : 256)) return 1e30;   // not measured there: never the best
     const TilePrice &p = tile_price[w_u8][tile];
     const int64_t wgs = tiles * c, full = wgs / 256;
     const float n = (float)(nk / c), last = (float)(wgs % 256) / 256.f;
@@ -2111,6 +2441,21 @@ int launch_tile(int tile, GemmGroup &g, int n, int64_t T, int64_t N, int ks, hip
         case TILE_160x192: return launch_dma<W_U8, 160, 192, 8, 0>(g, n, T, N, ks, st);
         case TILE_128x256: return launch_dma<W_U8, 128, 256, 8, 0>(g, n, T, N, ks, st);
         case TILE_128x192: return launch_dma<W_U8, 128, 192, 8, 0>(g, n, T, N, ks, st);
+        case TILE_32x16: return launch_few<W_U8, 32, 16>(g, n, T, N, ks, st);
+        case TILE_32x32: return launch_few<W_U8, 32, 32>(g, n, T, N, ks, st);
+        case TILE_32x48: return launch_few<W_U8, 32, 48>(g, n, T, N, ks, st);
+        case TILE_32x64: return launch_few<W_U8, 32, 64>(g, n, T, N, ks, st);
+        case TILE_32x96: return launch_few<W_U8, 32, 96>(g, n, T, N, ks, st);
+        case TILE_48x16: return launch_few<W_U8, 48, 16>(g, n, T, N, ks, st);
+        case TILE_48x32: return launch_few<W_U8, 48, 32>(g, n, T, N, ks, st);
+        case TILE_48x48: return launch_few<W_U8, 48, 48>(g, n, T, N, ks, st);
+        case TILE_48x64: return launch_few<W_U8, 48, 64>(g, n, T, N, ks, st);
+        case TILE_48x96: return launch_few<W_U8, 48, 96>(g, n, T, N, ks, st);
+        case TILE_64x16: return launch_few<W_U8, 64, 16>(g, n, T, N, ks, st);
+        case TILE_64x32: return launch_few<W_U8, 64, 32>(g, n, T, N, ks, st);
+        case TILE_64x48: return launch_few<W_U8, 64, 48>(g, n, T, N, ks, st);
+        case TILE_64x64: return launch_few<W_U8, 64, 64>(g, n, T, N, ks, st);
+        case TILE_64x96: return launch_few<W_U8, 64, 96>(g, n, T, N, ks, st);
         default: return RWKV_E_DTYPE;
     }
 }
@@ -2138,7 +2483,7 @@ int launch_pick(int cfg, int ks, int64_t T, int64_t N, int64_t M, const rwkv_hal
 }
 
 // Tile choice (RWKV_GEMM_CFG overrides it for tuning sweeps: 3 and 9 the register-staged tiles by their number here, 14 and 15 the
-// direct-to-LDS 256 x 256 and 128 x 128 ones, 18 to 30 the others, CFG_DMA + TILE_*, with the K split of least cost).
+// direct-to-LDS 256 x 256 and 128 x 128 ones, 18 to 45 the others, CFG_DMA + TILE_*, with the K split of least cost).
 //   CFG_DMA +  operands laid out for 16-byte loads: the direct-to-LDS kernel with the tile and K split that the cost
 //              model puts first (128 x 128 tiles at full depth when another product runs beside this one: a 256 x 256
 //              tile's LDS leaves no room beside it on the CU, two small ones fit)

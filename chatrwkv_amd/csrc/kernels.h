@@ -74,6 +74,7 @@ struct GemmEpi {
 };
 
 // Partial row sums that a launch of tiles tn columns wide emits per row of M outputs: one per tile, and zeros up to a multiple of four.
+constexpr int EMIT_MIN_TN = 48;   // narrower tiles hand nothing over: too many sums per row
 __host__ __device__ inline int emitted_parts(int M, int tn) { return ((M + tn - 1) / tn + 3) & ~3; }
 
 // How gemm_launch would run a product: kind 0 = the 2..16-row kernel, 1 = register-staged tiles, 2 = direct-to-LDS

@@ -99,7 +99,7 @@ inline int mm_pair_parts(const GemmPlan &p1, const Ctx &c2, const rwkv_mat &m1, 
     e2.small_tiles = c2.small_tiles;
     e2.mx = m2.mx; e2.rx = m2.rx; e2.s0 = c2.s0; e2.s2 = c2.s2;
     const GemmPlan p2 = gemm_plan(true, c2.T, M1, M2, c2.xs, M1, m2.w, m2.ld, out, M2, e2);
-    return p2.kind == 2 ? emitted_parts(M1, p1.tn) : 0;
+    return p2.kind == 2 && p1.tn >= EMIT_MIN_TN ? emitted_parts(M1, p1.tn) : 0;
 }
 
 inline int mm_pair_first(const Ctx &c1, const Ctx &c2, const rwkv_mat &m1, const rwkv_mat &m2, bool mat_u8,

@@ -261,8 +261,8 @@ struct SeqWs {
     size_t total;
 };
 
-// most partial sums a row can have: tiles of 64 columns of the channel-mix key product
-int64_t parts_max(int64_t F) { return emitted_parts((int)F, 64); }
+// most partial sums a row can have
+int64_t parts_max(int64_t F) { return emitted_parts((int)F, EMIT_MIN_TN); }
 
 SeqWs carve(void *base, int64_t T, int64_t C, int64_t F) {
     SeqWs w;
@@ -501,7 +501,7 @@ extern "C" int rwkv_v4_forward_seq(const rwkv_v4_model *m, const rwkv_v4_layer_s
             ev.out_scale = 1.f; ev.out_dtype = RWKV_DT_F16;
             ev.act = ACT_GATED_RESIDUAL; ev.gate = ws.r; ev.ldgate = C; ev.res = ws.x; ev.ldres = C;
             const GemmPlan pv = plan_gemm(l.ffn_value, true, T, ws.xsv, s0v, s2v, ws.x, C, ev, ws.splitk);
-            return pv.kind == 2 ? emitted_parts(F, pk.tn) : 0;
+            return pv.kind == 2 && pk.tn >= EMIT_MIN_TN ? emitted_parts(F, pk.tn) : 0;
         };
         auto emit = [&](GemmEpi &k, int np) {
             if (!np) return;

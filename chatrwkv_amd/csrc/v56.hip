@@ -289,7 +289,7 @@ Ws56 carve56(void *base, int64_t T, int64_t C, int64_t F, int64_t lm, int64_t ld
     }
     w.splitk = (float *)take(RWKV_SPLITK_WS_BYTES);
     w.y32 = (float *)take(wkv56_scratch_bytes(T, C));
-    w.parts = (float *)take(T > 1 ? (size_t)T * 2 * emitted_parts((int)F, 64) * sizeof(float) : 256);
+    w.parts = (float *)take(T > 1 ? (size_t)T * 2 * emitted_parts((int)F, EMIT_MIN_TN) * sizeof(float) : 256);
     for (int j = 0; j < 4; ++j) w.att_parts[j] = (float *)take(T > 1 ? (size_t)T * (2 + 2 * mix_parts(C)) * sizeof(float) : 256);
     w.total = (size_t)(p - (unsigned char *)base);
     return w;

@@ -252,6 +252,24 @@ def test_tiles_with_sides_of_128_to_256(N, M, B, cfg, monkeypatch):
         assert np.array_equal(ops.matmul_float(xt, _to_dev_ic(w), output_dtype=dtype).cpu().numpy(), exact.astype(np_dtype))
 
 
+@pytest.mark.parametrize("cfg", [str(c) for c in range(31, 46)])
+@pytest.mark.parametrize("N,M,B", [(64, 200, 17), (192, 1000, 50), (320, 264, 97), (4096, 520, 33), (8192, 96, 64), (1088, 1003, 65)])
+def test_tiles_of_few_rows(N, M, B, cfg, monkeypatch):
+    """The tiles of 32, 48 and 64 rows and 16 to 96 columns, both weight types: K shorter than a stage, a last stage that is there in
+    part, odd and even numbers of stages, ragged rows and columns, K splits (4096 and 8192 inputs), outputs that leave four at a time
+    (fp32, and 1003 of them).  The sums are exact, so the results are equal bit for bit."""
+    ops = _ops()
+    x, (q, mx, rx, my, ry), want, _ = _affine_case(N, M, B, N + M + B)
+    xt = torch.from_numpy(x).to(DEV)
+    monkeypatch.setenv("RWKV_GEMM_CFG", cfg)
+    y = ops.cuda_mm8_seq(B, N, M, xt, _to_dev_ic(q), *(torch.from_numpy(a).to(DEV) for a in (mx, rx, my, ry)))
+    assert np.array_equal(y.cpu().numpy(), want)
+    w = (_rng(N).integers(-64, 65, (N, M)) / 64).astype(np.float16)
+    exact = x.astype(np.float64) @ w.astype(np.float64)
+    for dtype, np_dtype in ((torch.float32, np.float64), (torch.float16, np.float16)):
+        assert np.array_equal(ops.matmul_float(xt, _to_dev_ic(w), output_dtype=dtype).cpu().numpy(), exact.astype(np_dtype))
+
+
 @pytest.mark.parametrize("u8,N,M,B", [(False, 16384, 1000, 48), (False, 8192, 66, 100), (False, 11520, 78, 29), (False, 4096, 512, 64),
                                       (True, 3904, 2880, 1922), (True, 3584, 7042, 663)])
 def test_tile_that_the_cost_model_puts_first(u8, N, M, B, monkeypatch):
