@@ -466,7 +466,7 @@ __global__ __launch_bounds__(64 * WT * WM) void gemm_kernel(int T, int N, int M,
 //              and with three stages the loads of tile kt + 2 are issued in three parts between the halves.
 //   HS = 1     (64 rows a wave) a step's fragments are read while the other step multiplies; the barrier follows the first step, and
 //              the loads of the tile NST ahead go into the stage that has just been read.
-//   KG = 2     (128 x 128 with four stages, one workgroup to a CU) the waves are two groups of 2 x 2, group g takes step g: 64 x 64 a
+//   KG = 2     (128 x 128 with four stages, one workgroup to a CU, and the tiles with a side of 96) the waves are two groups of 2 x 2, group g takes step g: 64 x 64 a
 //              wave instead of 64 x 32, two fifths fewer fragment bytes; all fragments of a tile are read while the one before
 //              multiplies.  us, one step after the other / two groups / as HS = 1: uint8 [256 x 4096] x [4096 x 12288] 38.8 / 37.5 /
 //              40.4, [1024 x 4096] x [4096 x 4096] 40.7 / 39.5 / 41.8; fp16 [333 x 2048] x [2048 x 8192] 21.6 / 21.5 / 23.5.
@@ -479,19 +479,20 @@ template <bool W_U8, int TM, int TN, int NW = 8, int NSTG = 0> struct DmaCfg {
     static constexpr int NST = NSTG ? NSTG : 3 * STAGE + (W_U8 ? 2 * TM * 4 + 2 * TN * 2 : 0) <= 160 * 1024 ? 3 : 2;
     static constexpr int AP = A / 1024, WP = W / 1024;                                        // 1 KB loads of a stage
     static constexpr int AL = (AP + NW - 1) / NW, WL = (WP + NW - 1) / NW, LOADS = AL + WL;   // per wave; past the end the last one again
-    static constexpr int KG = TM == 128 && NST == 4 ? 2 : 1;                                  // groups of waves that share K
-    static constexpr int WR = TM >= 128 ? 2 : 1, WC = NW / WR / KG;                           // waves: 2 rows x 4 columns; 64-row tile: 1 x 4
+    static constexpr int KG = NW == 8 && NST == 4 ? 2 : 1;                                    // groups of waves that share K
+    static constexpr bool SPLITS = TM != 96 && TN != 96;                                      // K split over workgroups: see dma_split
+    static constexpr int WR = TM > 64 ? 2 : 1, WC = NW / WR / KG;                             // waves: 2 rows x 4 columns; 64-row tile: 1 x 4
     static constexpr int MI = TM / (16 * WR), NI = TN / (16 * WC);                            // 16 x 16 blocks per wave
     static constexpr int HS = MI > 4 ? 2 : 1, H0 = HS == 2 ? (MI + 1) / 2 : MI;               // row blocks in one or two halves
     static constexpr int STG_STRIDE = TN + 4;   // epilogue staging, floats: 16 bytes apart, so 16 rows fill all banks
     static constexpr int HSTRIDE = TN + 8;      // the same for fp16 outputs
     static constexpr int FROWS = TM > 128 ? TM / 2 : TM;                                      // rows of a pass of the former
-    static constexpr int CPR = TN == 192 ? 32 : TN / 8;                                       // threads that finish a row, eight outputs each
+    static constexpr int CPR = TN > 128 ? 32 : 16;                                            // threads that finish a row, eight outputs each
     static constexpr size_t max3(size_t a, size_t b, size_t c) { return a > b ? (a > c ? a : c) : (b > c ? b : c); }
     static constexpr size_t BODY = max3((size_t)NST * STAGE, (size_t)KG * FROWS * STG_STRIDE * 4, (size_t)TM * HSTRIDE * 2);
     static constexpr size_t LDS = BODY + (W_U8 ? 2 * TM * 4 + 2 * TN * 2 : 0);   // uint8: past the stages the rows' sums s0, s2 and the columns' rx, mx
     static_assert(TM % (16 * WR) == 0 && TN % (16 * WC) == 0 && MI <= 8 && NI <= 4 && H0 <= 4 && 2 * TM <= 64 * NW, "waves");
-    static_assert((NST - 1) * LOADS < 64 && LDS <= 160 * 1024 && (TN == 64 || TN == 128 || TN == 192 || TN == 256), "tile");
+    static_assert((NST - 1) * LOADS < 64 && LDS <= 160 * 1024 && TN > 64 && TN <= 256, "tile");
 };
 DEV void emit_parts(const GemmEpi &ep, int t, int m0, int M, int TN, float a0, float a2) {
     const int parts = emitted_parts(M, TN), i = m0 / TN;
@@ -825,7 +826,7 @@ DEV void gemm_dma_body(int bid, int T, int N, int M, int walk_m, const h16 *__re
     const bool in_tile = cq * 8 < TN, col_ok = in_tile && col < M;
     constexpr int SW = Cfg::STG_STRIDE;                  // row stride of fp32 in LDS, in floats
     float *const stg = (float *)smem;
-    constexpr int ITS = TM / RPI, AHEAD_ROWS = ITS % 4 ? 2 : 4;      // rows of a thread; rows requested together
+    constexpr int ITS = TM / RPI, AHEAD_ROWS = KG == 2 ? ITS : ITS % 4 ? 2 : 4;      // rows of a thread; rows requested together
     static_assert(ITS % AHEAD_ROWS == 0 && TM % RPI == 0 && Cfg::FROWS % RPI == 0, "rows");
     // the sums of a row of the tile that the CPR threads finishing it hold, neighbours in one wave: every lane takes part
     auto emit_row = [&](int t, bool valid, float a0, float a2) {
@@ -858,8 +859,8 @@ DEV void gemm_dma_body(int bid, int T, int N, int M, int walk_m, const h16 *__re
 #pragma unroll
             for (int it = 0; it < ITS; ++it) {
                 const int r = it * RPI + tid / CPR, t = t0 + r;
-                if (t < T && col < M) *(f32x4 *)(slab + (size_t)t * M + col) = sum4(r, cq * 8);           // M % 4 == 0
-                if (t < T && col + 4 < M) *(f32x4 *)(slab + (size_t)t * M + col + 4) = sum4(r, cq * 8 + 4);
+                if (t < T && col_ok) *(f32x4 *)(slab + (size_t)t * M + col) = sum4(r, cq * 8);           // M % 4 == 0
+                if (t < T && col_ok && col + 4 < M) *(f32x4 *)(slab + (size_t)t * M + col + 4) = sum4(r, cq * 8 + 4);
             }
         } else if (by_four(M, ldy, Y, ep)) {
             __syncthreads();
@@ -870,7 +871,7 @@ DEV void gemm_dma_body(int bid, int T, int N, int M, int walk_m, const h16 *__re
 #pragma unroll
                 for (int g = 0; g < 2; ++g) {
                     const int c = g * (TN / 2) + cq * 4;
-                    if (m0 + c >= M) continue;
+                    if (!in_tile || m0 + c >= M) continue;
                     f32x4 v = sum4(r, c);
                     if constexpr (W_U8) affine4(v, m0 + c, M, lsum[r], lsum[TM + r], ep);
                     finish_row4(v, t, m0 + c, M, ep, Y, ldy);
@@ -1067,20 +1068,24 @@ __global__ __launch_bounds__(64 * NW) void gemm_dma_kernel(int T, int N, int uni
 
 template <bool W_U8, int TM, int TN, int NW, int NSTG>
 int launch_dma(GemmGroup &g, int n, int64_t T, int64_t N, int ks, hipStream_t st) {
-    constexpr size_t lds = DmaCfg<W_U8, TM, TN, NW, NSTG>::LDS;
+    using Cfg = DmaCfg<W_U8, TM, TN, NW, NSTG>;
+    constexpr size_t lds = Cfg::LDS;
+    if (ks > 1 && !Cfg::SPLITS) return RWKV_E_DTYPE;
     static PerDeviceOnce once;
     bool *attr_done = once.slot();
     if (!attr_done || !*attr_done) {
         hipError_t e = hipFuncSetAttribute((const void *)gemm_dma_kernel<W_U8, false, TM, TN, NW, NSTG>,
                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (e == hipSuccess)
-            e = hipFuncSetAttribute((const void *)gemm_dma_kernel<W_U8, true, TM, TN, NW, NSTG>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                    (int)lds);
+        if constexpr (Cfg::SPLITS) {
+            if (e == hipSuccess)
+                e = hipFuncSetAttribute((const void *)gemm_dma_kernel<W_U8, true, TM, TN, NW, NSTG>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                        (int)lds);
+        }
         if (e != hipSuccess) return (int)e;
         if (attr_done) *attr_done = true;
     }
     const int units = (int)group_tiles(W_U8, g, n, T, N, TM, TN) * ks;
-    const auto kernel = ks > 1 ? gemm_dma_kernel<W_U8, true, TM, TN, NW, NSTG> : gemm_dma_kernel<W_U8, false, TM, TN, NW, NSTG>;
+    const auto kernel = Cfg::SPLITS && ks > 1 ? gemm_dma_kernel<W_U8, Cfg::SPLITS, TM, TN, NW, NSTG> : gemm_dma_kernel<W_U8, false, TM, TN, NW, NSTG>;
     hipLaunchKernelGGL(kernel, dim3((unsigned)units), dim3(64 * NW), lds, st, (int)T, (int)N, units, ks, g.first[1], g.first[2], g.first[3], g.nk_split, g.lda,
                        (const GemmMembers &)g);
     RWKV_LAUNCH_CHECK();
@@ -2279,12 +2284,14 @@ bool dma_ok(bool w_u8, int64_t N, int64_t M, const void *A, int64_t lda, const v
 enum {
     TILE_256x256, TILE_S, TILE_S4, TILE_N, TILE_K8, TILE_K4, TILE_256x192, TILE_224x256, TILE_224x192, TILE_192x256, TILE_192x192,
     TILE_160x256, TILE_160x192, TILE_128x256, TILE_128x192,
-    TILE_32x16, TILE_32x32, TILE_32x48, TILE_32x64, TILE_32x96, TILE_48x16, TILE_48x32, TILE_48x48, TILE_48x64, TILE_48x96, TILE_64x16, TILE_64x32, TILE_64x48, TILE_64x64, TILE_64x96, TILES
+    TILE_32x16, TILE_32x32, TILE_32x48, TILE_32x64, TILE_32x96, TILE_48x16, TILE_48x32, TILE_48x48, TILE_48x64, TILE_48x96, TILE_64x16, TILE_64x32, TILE_64x48, TILE_64x64, TILE_64x96,
+    TILE_96x128, TILE_128x96, TILE_96x96, TILES
 };
 struct TileDim { int tm, tn; };
 constexpr TileDim tile_dim[TILES] = {{256, 256}, {128, 128}, {128, 128}, {64, 128}, {64, 64}, {64, 128}, {256, 192}, {224, 256}, {224, 192},
                                      {192, 256}, {192, 192}, {160, 256}, {160, 192}, {128, 256}, {128, 192},
-                                     {32, 16}, {32, 32}, {32, 48}, {32, 64}, {32, 96}, {48, 16}, {48, 32}, {48, 48}, {48, 64}, {48, 96}, {64, 16}, {64, 32}, {64, 48}, {64, 64}, {64, 96}};
+                                     {32, 16}, {32, 32}, {32, 48}, {32, 64}, {32, 96}, {48, 16}, {48, 32}, {48, 48}, {48, 64}, {48, 96}, {64, 16}, {64, 32}, {64, 48}, {64, 64}, {64, 96},
+                                     {96, 128}, {128, 96}, {96, 96}};
 
 // Cost model of a direct-to-LDS launch in microseconds.  `tiles` tiles of nk k-tiles split c ways run in rounds over the 256 CUs:
 //   launch + rounds * (round, or split_round, which leaves the epilogue to the second pass)
@@ -2295,11 +2302,14 @@ constexpr TileDim tile_dim[TILES] = {{256, 256}, {128, 128}, {128, 128}, {64, 12
 // from 64 to 20480; weights from HBM; the chip under load before): the tile and split it picks takes 1 % (uint8) and 2 %
 // (fp16) longer than the best of all on average, with products that the host launches no faster counted in.  A tile per round costs
 // between 3 and 15 us whatever K is, so tiles of many sizes pay: each of these is the best one somewhere, the large ones with sides of
-// 160, 192 and 224 where 256 x 256 or 128 x 128 leave CUs idle or rows empty, those of 32, 48 and 64 rows in calls of up to 128 rows.
+// 160, 192 and 224 where 256 x 256 or 128 x 128 leave CUs idle or rows empty, those of 32, 48 and 64 rows in calls of up to 128 rows, those with a side of
+// 96 where a round of 128 x 128 leaves CUs idle (fitted apart, at full depth, 97 rows and more).
 // us, uint8 / fp16 weights: [1024 x 4096] x [4096 x 12288] three rounds of 128 x 128 115.7 / 132.5, one of 256 x 192 90 / 97; [777 x
 // 4096] x [4096 x 16384] 256 x 256 126 / 130, 224 x 256 100 / 107; [768 x 4096] x [4096 x 12288] 104 / 109, 192 x 192 71 / 80;
 // [45 x 4096] x [4096 x 4096] four splits of 64 x 64 11.0 / 12.4, 48 x 16 8.7 / 10.6; [45 x 4096] x [4096 x 20480] 64 x 128 26.5 /
-// 40.6, 48 x 96 23.8 / 37.9; [24 x 2048] x [2048 x 2048] 8.1 / 8.1, 32 x 16 5.6 / 5.5.
+// 40.6, 48 x 96 23.8 / 37.9; [24 x 2048] x [2048 x 2048] 8.1 / 8.1, 32 x 16 5.6 / 5.5; [333 x 2048]
+// x [2048 x 8192] four-stage 128 x 128 21.5 / 22.8, 96 x 128 19.1 / 20.2; [160 x 4096] x [4096 x 16384] 40.5 / 44.0, 33.5 / 42.7; [513 x
+// 4096] x [4096 x 4096] 33.0 / 31.8, 128 x 96 28.9 / 29.7; [513 x 1280] x [1280 x 3840] 16.1 / 14.3, 96 x 96 12.4 / 12.0.
 struct TilePrice { float launch, round, split_round, step_0, step_1, extra, slab, split; };
 constexpr TilePrice tile_price[2][TILES] = {
     {   // fp16 weights
@@ -2333,6 +2343,9 @@ constexpr TilePrice tile_price[2][TILES] = {
         {4.503f, 0.040f, 1.948f, 0.095f, 0.337f, 0.117f, 0.f, 0.027f},   // 64x48
         {2.451f, 1.661f, 3.319f, 0.136f, 0.330f, 0.f, 4.174f, 0.119f},   // 64x64
         {2.816f, 2.220f, 3.033f, 0.188f, 0.429f, 0.f, 7.091f, 0.094f},   // 64x96
+        {1.795f, 4.124f, 4.124f, 0.260f, 0.484f, 0.002f, 0.f, 0.f},   // 96x128
+        {1.738f, 4.854f, 4.854f, 0.263f, 0.457f, 0.039f, 0.f, 0.f},   // 128x96
+        {1.881f, 4.025f, 4.025f, 0.246f, 0.404f, 0.029f, 0.f, 0.f},   // 96x96
     }, {   // uint8
         {5.336f, 9.067f, 8.377f, 0.949f, 1.642f, 0.022f, 3.336f, 0.f},   // 256x256
         {6.522f, 0.f, 0.599f, 0.349f, 0.546f, 0.f, 4.631f, 0.085f},   // S
@@ -2364,9 +2377,13 @@ constexpr TilePrice tile_price[2][TILES] = {
         {4.608f, 0.525f, 1.966f, 0.106f, 0.147f, 0.088f, 4.921f, 0.074f},   // 64x48
         {4.535f, 0.f, 1.492f, 0.129f, 0.173f, 0.093f, 8.795f, 0.060f},   // 64x64
         {5.097f, 0.529f, 1.525f, 0.160f, 0.257f, 0.103f, 6.215f, 0.071f},   // 64x96
+        {1.500f, 4.811f, 4.811f, 0.295f, 0.412f, 0.026f, 0.f, 0.f},   // 96x128
+        {1.500f, 5.567f, 5.567f, 0.284f, 0.397f, 0.026f, 0.f, 0.f},   // 128x96
+        {4.415f, 1.814f, 1.814f, 0.238f, 0.325f, 0.016f, 0.f, 0.f},   // 96x96
     }};
 double dma_cost(bool w_u8, int tile, int64_t T, int64_t tiles, int nk, int c, size_t out_bytes) {
-    if (T > (tile == TILE_N ? 64 : tile < TILE_32x16 ? T : tile_dim[tile].tn <= 32 ? 128 : 256)) return 1e30;   // not measured there: never the best
+    // not measured there: never the best
+    if (tile >= TILE_96x128 ? T <= 96 : T > (tile == TILE_N ? 64 : tile < TILE_32x16 ? T : tile_dim[tile].tn <= 32 ? 128 : 256)) return 1e30;
     const TilePrice &p = tile_price[w_u8][tile];
     const int64_t wgs = tiles * c, full = wgs / 256;
     const float n = (float)(nk / c), last = (float)(wgs % 256) / 256.f;
@@ -2377,12 +2394,14 @@ double dma_cost(bool w_u8, int tile, int64_t T, int64_t tiles, int nk, int c, si
     return us;
 }
 
-// the K split (1..8, whole k-tiles, at least 8 per split, slabs within ws_bytes) of least cost
+// the K split (1..8, whole k-tiles, at least 8 per split, slabs within ws_bytes) of least cost.  The tiles with a side of 96 run at full
+// depth only: split they were the best of all, by 5 % at most, for 6 of 560 products, and priced for it they took others where they are 10 to 15 %
+// slower.
 int dma_split(bool w_u8, int tile, int64_t T, int64_t tiles, int nk, size_t out_bytes, size_t ws_bytes, double *cost = nullptr) {
     int best = 1;
     double best_cost = 1e30;
     for (int c = 1; c <= 8; ++c) {
-        if (nk % c || (c > 1 && nk / c < 8) || (c > 1 && c * out_bytes > ws_bytes)) continue;
+        if (nk % c || (c > 1 && (nk / c < 8 || c * out_bytes > ws_bytes || tile >= TILE_96x128))) continue;
         const double k = dma_cost(w_u8, tile, T, tiles, nk, c, out_bytes);
         if (k < best_cost) { best_cost = k; best = c; }
     }
@@ -2441,6 +2460,9 @@ int launch_tile(int tile, GemmGroup &g, int n, int64_t T, int64_t N, int ks, hip
         case TILE_160x192: return launch_dma<W_U8, 160, 192, 8, 0>(g, n, T, N, ks, st);
         case TILE_128x256: return launch_dma<W_U8, 128, 256, 8, 0>(g, n, T, N, ks, st);
         case TILE_128x192: return launch_dma<W_U8, 128, 192, 8, 0>(g, n, T, N, ks, st);
+        case TILE_96x128: return launch_dma<W_U8, 96, 128, 8, 4>(g, n, T, N, ks, st);
+        case TILE_128x96: return launch_dma<W_U8, 128, 96, 8, 4>(g, n, T, N, ks, st);
+        case TILE_96x96: return launch_dma<W_U8, 96, 96, 8, 4>(g, n, T, N, ks, st);
         case TILE_32x16: return launch_few<W_U8, 32, 16>(g, n, T, N, ks, st);
         case TILE_32x32: return launch_few<W_U8, 32, 32>(g, n, T, N, ks, st);
         case TILE_32x48: return launch_few<W_U8, 32, 48>(g, n, T, N, ks, st);
@@ -2483,7 +2505,7 @@ int launch_pick(int cfg, int ks, int64_t T, int64_t N, int64_t M, const rwkv_hal
 }
 
 // Tile choice (RWKV_GEMM_CFG overrides it for tuning sweeps: 3 and 9 the register-staged tiles by their number here, 14 and 15 the
-// direct-to-LDS 256 x 256 and 128 x 128 ones, 18 to 45 the others, CFG_DMA + TILE_*, with the K split of least cost).
+// direct-to-LDS 256 x 256 and 128 x 128 ones, 18 to 48 the others, CFG_DMA + TILE_*, with the K split of least cost).
 //   CFG_DMA +  operands laid out for 16-byte loads: the direct-to-LDS kernel with the tile and K split that the cost
 //              model puts first (128 x 128 tiles at full depth when another product runs beside this one: a 256 x 256
 //              tile's LDS leaves no room beside it on the CU, two small ones fit)

@@ -270,6 +270,13 @@ def test_tiles_of_few_rows(N, M, B, cfg, monkeypatch):
         assert np.array_equal(ops.matmul_float(xt, _to_dev_ic(w), output_dtype=dtype).cpu().numpy(), exact.astype(np_dtype))
 
 
+@pytest.mark.parametrize("cfg", [str(c) for c in range(46, 49)])
+@pytest.mark.parametrize("N,M,B", [(64, 200, 17), (192, 1000, 257), (448, 264, 600), (4096, 520, 97), (128, 1003, 160), (320, 97, 96)])
+def test_tiles_with_a_side_of_96(N, M, B, cfg, monkeypatch):
+    """As above for 96 x 128, 128 x 96 and 96 x 96: rows of outputs that are no power of two, and the last column tile one wide."""
+    test_tiles_with_sides_of_128_to_256(N, M, B, cfg, monkeypatch)
+
+
 @pytest.mark.parametrize("u8,N,M,B", [(False, 16384, 1000, 48), (False, 8192, 66, 100), (False, 11520, 78, 29), (False, 4096, 512, 64),
                                       (True, 3904, 2880, 1922), (True, 3584, 7042, 663)])
 def test_tile_that_the_cost_model_puts_first(u8, N, M, B, monkeypatch):
