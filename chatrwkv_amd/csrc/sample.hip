@@ -453,10 +453,15 @@ __global__ __launch_bounds__(STHREADS) void sample_kernel(SampleArgs a) {
 //           probabilities and the occurrence counts of its segment.
 // Sums are added in a fixed order throughout.  Where the total is no positive number (a NaN, an infinity or nothing but masks
 // among the logits) nothing is kept and id 0 is drawn, which is what the kernel above makes of such logits.
-// Bound by the latency of the three launches.  Measured as above, V = 65536: 20 us a draw (2.9 + 4.3 + 10.8 and the gaps), 38 with one
+// Bound by the latency of the three launches.  Measured as above, V = 65536: 16.4 us a draw (2.9 + 4.4 + 7.7 and the gaps), 38 with one
 // workgroup; with the lists in LDS and the bracket searched by search_list 25.8, 5 us of it in the search.
+// The draw's workgroups each take in the candidates of all segments, 64 bytes a clock and less, and issue every comparison with
+// them 16 waves deep.  So there are two lists: of N(0, 3) 40 % of the entries are candidates at top_p 0.7, and 10 % reach bound HIGH, which has the whole
+// nucleus.  us a draw, one list / two: 65536 entries, top_p 0.7 17.0 / 16.4, 0.85 20.9 / 16.4 (with the sort below), top_k 50 25.5 / 19.9; 50277 from
+// N(0, 0.3), which need the long one a trip to memory later, 39.9 / 36.9.
 constexpr int SEG = 1024, SEGS_MAX = 64, BOUNDS = 32;
 constexpr int FEW = 256;                      // entries of a bracket that are compared with each other at once
+constexpr int HIGH = 25;                      // a bound 2^-13 below the largest probability
 constexpr int PART = 2 * BOUNDS + 3;          // per segment: sums and counts at the bounds, sum of all, length of the list, its smallest entry
 
 struct SampleWs {
@@ -464,6 +469,8 @@ struct SampleWs {
     float *list;       // [segments][SEG] candidates in index order
     float *pow;        // [segments][SEG] the same to the power 1 / temperature, at temperatures other than 0 and 1
     uint16_t *idx;     // [segments][SEG] their places in the segment
+    float *high, *high_pow;   // list, pow and idx of the entries that reach bound HIGH alone
+    uint16_t *high_idx;
     float *soft;       // [segments][2] largest logit, sum of exponentials
     float *part;       // [segments][PART]
 };
@@ -471,25 +478,36 @@ struct SampleWs {
 __global__ __launch_bounds__(256) void sample_adjust_kernel(SampleArgs a, SampleWs ws) {
     __shared__ float red[8];
     const int V = a.V, i0 = blockIdx.x * SEG + 4 * threadIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    f32x4 x;
+    at_once({a.logits, a.seen, a.occ, a.ban, ws.p, ws.soft});
+    // everything is requested before anything is looked at, whether an entry has been seen or not
+    f32x4 x, occ = {0.f, 0.f, 0.f, 0.f};
     uint32_t flag = 0;
-    if (i0 + 3 < V && (((uintptr_t)a.logits) & 15) == 0 && (((uintptr_t)a.seen) & 3) == 0) {
+    const int banned = lane < a.n_ban ? a.ban[lane] : 0;
+    if (i0 + 3 < V && ((((uintptr_t)a.logits) | ((uintptr_t)a.occ)) & 15) == 0 && (((uintptr_t)a.seen) & 3) == 0) {
         x = *(const f32x4 *)(a.logits + i0);
-        if (a.seen) flag = *(const uint32_t *)(a.seen + i0);
+        if (a.seen) {
+            flag = *(const uint32_t *)(a.seen + i0);
+            occ = *(const f32x4 *)(a.occ + i0);
+        }
     } else {
+        uint8_t f[4] = {};
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            x[e] = i0 + e < V ? a.logits[i0 + e] : -INFINITY;
-            if (a.seen && i0 + e < V) flag |= (uint32_t)a.seen[i0 + e] << (8 * e);
+            const int i = min(i0 + e, V - 1);
+            x[e] = a.logits[i];
+            if (a.seen) { f[e] = a.seen[i]; occ[e] = a.occ[i]; }
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            x[e] = i0 + e < V ? x[e] : -INFINITY;
+            flag |= (i0 + e < V ? (uint32_t)f[e] : 0u) << (8 * e);
         }
     }
-    if (flag) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
-            if ((flag >> (8 * e)) & 0xff) x[e] -= a.presence + a.occ[i0 + e] * a.frequency;
-    }
+    for (int e = 0; e < 4; ++e)
+        if ((flag >> (8 * e)) & 0xff) x[e] -= a.presence + occ[e] * a.frequency;
     for (int b = 0; b < a.n_ban; ++b) {
-        const int k = a.ban[b] - i0;
+        const int k = (b < 64 ? __builtin_amdgcn_readlane(banned, b) : a.ban[b]) - i0;
 #pragma unroll
         for (int e = 0; e < 4; ++e)
             if (e == k) x[e] = -INFINITY;
@@ -513,9 +531,10 @@ __global__ __launch_bounds__(256) void sample_adjust_kernel(SampleArgs a, Sample
 
 // The largest logit and the sum of the exponentials from the segments'; every lane gets both.
 struct Soft { float mx, sum; };
-DEV Soft soft_total(const float *soft, int segs) {
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+DEV Soft soft_total(f32x2 own, int segs) {   // own: those of segment `lane`
     const int lane = threadIdx.x & 63;
-    const float m = lane < segs ? soft[2 * lane] : -INFINITY, s = lane < segs ? soft[2 * lane + 1] : 0.f;
+    const float m = lane < segs ? own[0] : -INFINITY, s = lane < segs ? own[1] : 0.f;
     const float mx = wave_max(m);
     return {mx, wave_sum(m == -INFINITY ? 0.f : s * expf(m - mx))};
 }
@@ -554,10 +573,12 @@ __global__ __launch_bounds__(256) void sample_probs_kernel(SampleArgs a, SampleW
     __shared__ unsigned long long bin_s[BOUNDS];   // sums in fixed point
     __shared__ unsigned bin_n[BOUNDS];
     __shared__ float red[4][2], least[4];
+    __shared__ int highs[4];
     if (threadIdx.x < BOUNDS) { bin_s[threadIdx.x] = 0; bin_n[threadIdx.x] = 0; }
     const int i0 = blockIdx.x * SEG + 4 * threadIdx.x, lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int segs = (a.V + SEG - 1) / SEG;
     f32x4 p = *(const f32x4 *)(ws.p + i0);
-    const Soft st = soft_total(ws.soft, gridDim.x);
+    const Soft st = soft_total(*(const f32x2 *)(ws.soft + 2 * min(lane, segs - 1)), segs);
     const float inv = 1.f / st.sum;   // of the largest entry: its exponential is 1
 #pragma unroll
     for (int e = 0; e < 4; ++e) p[e] = p[e] == -INFINITY ? 0.f : expf(p[e] - st.mx) * inv;
@@ -575,30 +596,43 @@ __global__ __launch_bounds__(256) void sample_probs_kernel(SampleArgs a, SampleW
         }
     }
     const float total = wave_sum((p[0] + p[1]) + (p[2] + p[3]));
-    unsigned long long in[4];
-    int before = 0, n_wave = 0;
+    unsigned long long in[4], in_high[4];
+    int before = 0, n_wave = 0, before_high = 0, n_high = 0;
     float small = INFINITY;
+    const float high = top_p > 0.f ? bound_at(inv, HIGH) : INFINITY;   // temperature 0: `list` has the largest entries alone
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
         in[e] = __ballot(p[e] >= floor_);
         small = p[e] >= floor_ ? fminf(small, p[e]) : small;
         before += (int)__popcll(in[e] & ((1ull << lane) - 1));
         n_wave += (int)__popcll(in[e]);
+        in_high[e] = __ballot(p[e] >= high);
+        before_high += (int)__popcll(in_high[e] & ((1ull << lane) - 1));
+        n_high += (int)__popcll(in_high[e]);
     }
     small = -wave_max(-small);
-    if (lane == 0) { red[wave][0] = total; red[wave][1] = (float)n_wave; least[wave] = small; }
+    if (lane == 0) { red[wave][0] = total; red[wave][1] = (float)n_wave; least[wave] = small; highs[wave] = n_high; }
     __syncthreads();
-    int at = blockIdx.x * SEG + before;
+    int at = blockIdx.x * SEG + before, at_high = blockIdx.x * SEG + before_high;
 #pragma unroll
     for (int w = 0; w < 3; ++w)
-        if (w < wave) at += (int)red[w][1];
+        if (w < wave) { at += (int)red[w][1]; at_high += highs[w]; }
 #pragma unroll
-    for (int e = 0; e < 4; ++e)
-        if ((in[e] >> lane) & 1) {
+    for (int e = 0; e < 4; ++e) {
+        const bool one = (in[e] >> lane) & 1, two = (in_high[e] >> lane) & 1;
+        float power = 0.f;
+        if (POW && (one || two)) power = powf(p[e], 1.f / a.temperature);
+        if (one) {
             ws.list[at] = p[e];
-            if (POW) ws.pow[at] = powf(p[e], 1.f / a.temperature);
+            if (POW) ws.pow[at] = power;
             ws.idx[at++] = (uint16_t)(4 * threadIdx.x + e);
         }
+        if (two) {
+            ws.high[at_high] = p[e];
+            if (POW) ws.high_pow[at_high] = power;
+            ws.high_idx[at_high++] = (uint16_t)(4 * threadIdx.x + e);
+        }
+    }
     float *part = ws.part + blockIdx.x * PART;
     if (threadIdx.x == 2) part[2 * BOUNDS + 2] = fminf(fminf(least[0], least[1]), fminf(least[2], least[3]));
     if (threadIdx.x < 2) part[2 * BOUNDS + threadIdx.x] = (red[0][threadIdx.x] + red[1][threadIdx.x]) + (red[2][threadIdx.x] + red[3][threadIdx.x]);
@@ -623,33 +657,47 @@ __global__ __launch_bounds__(STHREADS) void sample_draw_kernel(SampleArgs a, Sam
     __shared__ unsigned part_n[64 * COPIES], total_n[64];
     __shared__ __align__(16) float cols[2 * BOUNDS][SWAVES + 4], few[FEW], sorted[FEW];
     __shared__ int pick, n_few[2];
-    const int V = a.V, tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), segs = gridDim.x;
+    const int V = a.V, tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), segs = (V + SEG - 1) / SEG;
     const int own = blockIdx.x * SEG + tid;                 // this thread's entry
+    at_once({a.seen, a.occ, a.u, a.weight, a.probs, ws.p, ws.high, ws.soft, ws.part});
+    // All that does not depend on the cut is requested first and together.  Read where it is used, it was eight trips to memory one
+    // after the other, the four parts below among them: 20.7 us a draw, 18.7 now.
     const float p_own = ws.p[own];
-    const uint8_t seen_own = a.seen && own < V ? a.seen[own] : 0;
+    uint8_t seen_own = 0;
+    float occ_own = 0.f;
+    if (a.seen) {
+        seen_own = a.seen[min(own, V - 1)];
+        occ_own = a.occ[min(own, V - 1)];
+    }
     const float target_u = *a.u;
+    const f32x2 soft_own = *(const f32x2 *)(ws.soft + 2 * min(lane, segs - 1));
+    float col[SEGS_MAX / SWAVES];
+#pragma unroll
+    for (int j = 0; j < SEGS_MAX / SWAVES; ++j) col[j] = ws.part[min(wave * (SEGS_MAX / SWAVES) + j, segs - 1) * PART + lane];
+    const float *const rest = ws.part + min(lane, segs - 1) * PART + 2 * BOUNDS;   // sum of all, candidates, the smallest of segment `lane`
+    const float all_own = rest[0], len_own = rest[1], small_own = rest[2], high_own = rest[HIGH - BOUNDS];
     const float top_p = a.temperature == 0.f ? 0.f : a.top_p;
-    // 16 threads a segment hold its list: thread r the entries 64 j + 4 r .. + 3.  The first rounds are requested before the
-    // lengths are known
-    constexpr int EARLY = 4;
+    // 16 threads a segment hold its list: thread r the entries 64 j + 4 r .. + 3.  The first rounds of the short one are requested
+    // before the lengths are known and which list it is to be
+    constexpr int EARLY = 2;
     const int sg = tid >> 4, r = tid & 15;
     f32x4 v[SEG / 64];
 #pragma unroll
-    for (int j = 0; j < EARLY; ++j) v[j] = *(const f32x4 *)(ws.list + min(sg, segs - 1) * SEG + 64 * j + 4 * r);
+    for (int j = 0; j < EARLY; ++j) v[j] = *(const f32x4 *)(ws.high + min(sg, segs - 1) * SEG + 64 * j + 4 * r);
     if (tid < 2) n_few[tid] = 0;
+    if (tid < FEW) few[tid] = 0.f;
     // ---- totals of the segments
     {
         float c = 0.f;
 #pragma unroll
         for (int j = 0; j < SEGS_MAX / SWAVES; ++j) {
-            const int sg = wave * (SEGS_MAX / SWAVES) + j;
-            if (sg < segs) c += ws.part[sg * PART + lane];
+            if (wave * (SEGS_MAX / SWAVES) + j < segs) c += col[j];
         }
         cols[lane][wave] = c;
     }
-    const Soft st = soft_total(ws.soft, segs);
+    const Soft st = soft_total(soft_own, segs);
     const float pmax = 1.f / st.sum;
-    const float all = wave_sum(lane < segs ? ws.part[lane * PART + 2 * BOUNDS] : 0.f);
+    const float all = wave_sum(lane < segs ? all_own : 0.f);
     // token, and the occurrence table: decay, then add the drawn token's weight
     auto store = [&](int tok) {
         if (blockIdx.x == 0 && tid == 0) *a.token = tok;
@@ -657,7 +705,7 @@ __global__ __launch_bounds__(STHREADS) void sample_draw_kernel(SampleArgs a, Sam
             const float w = own == tok ? (a.weight ? a.weight[tok] : 1.f) : 0.f;
             float o = w;
             if (seen_own) {
-                o = a.occ[own] * a.decay;
+                o = occ_own * a.decay;
                 if (own == tok) o += w;
             } else {
                 a.seen[own] = 1;
@@ -671,19 +719,32 @@ __global__ __launch_bounds__(STHREADS) void sample_draw_kernel(SampleArgs a, Sam
         store(0);
         return;
     }
-    const float len = lane < segs ? ws.part[lane * PART + 2 * BOUNDS + 1] : 0.f;
-    const float n = wave_sum(len);                          // candidates
+    __syncthreads();
+    // ---- which half octave holds the cut: lane k has the sum and the count at bound k
+    SumCount at_k = {0.f, 0.f};
+#pragma unroll
+    for (int w = 0; w < SWAVES; w += 4) {
+        const f32x4 x = *(const f32x4 *)&cols[lane & (BOUNDS - 1)][w], y = *(const f32x4 *)&cols[BOUNDS + (lane & (BOUNDS - 1))][w];
+        at_k.s += (x[0] + x[1]) + (x[2] + x[3]);
+        at_k.n += (y[0] + y[1]) + (y[2] + y[3]);
+    }
+    // ---- where the nucleus ends at bound HIGH or above it, or is the largest entry alone, the short list has all of it
+    const bool nucleus = top_p > 0.f && all >= top_p;
+    const bool high = top_p > 0.f && (!nucleus || __ballot(lane <= HIGH && enough(at_k, top_p, -1)) != 0);
+    const float *const list = high ? ws.high : ws.list, *const powers = high ? ws.high_pow : ws.pow;
+    const uint16_t *const idx = high ? ws.high_idx : ws.idx;
+    const float n = wave_sum(lane < segs ? len_own : 0.f);  // candidates
+    const float len = lane < segs ? (high ? high_own : len_own) : 0.f;
     const int n_seg = (int)__shfl(len, sg, WAVE), rounds = ((int)wave_max(len) + 63) >> 6;   // rounds: those that any segment has
 #pragma unroll
-    for (int j = EARLY; j < SEG / 64; ++j)
-        if (j < rounds) v[j] = *(const f32x4 *)(ws.list + min(sg, segs - 1) * SEG + 64 * j + 4 * r);
+    for (int j = 0; j < SEG / 64; ++j)
+        if (j < rounds && (j >= EARLY || !high)) v[j] = *(const f32x4 *)(list + min(sg, segs - 1) * SEG + 64 * j + 4 * r);
 #pragma unroll
     for (int j = 0; j < SEG / 64; ++j)
         if (j < rounds) {
 #pragma unroll
             for (int e = 0; e < 4; ++e) v[j][e] = 64 * j + 4 * r + e < n_seg ? v[j][e] : 0.f;
         }
-    __syncthreads();
     // calls f for every candidate that this thread holds (zeros fill the last round)
     auto each = [&](auto f) {
 #pragma unroll
@@ -693,14 +754,6 @@ __global__ __launch_bounds__(STHREADS) void sample_draw_kernel(SampleArgs a, Sam
                 for (int e = 0; e < 4; ++e) f(v[j][e]);
             }
     };
-    // ---- which half octave holds the cut: lane k has the sum and the count at bound k
-    SumCount at_k = {0.f, 0.f};
-#pragma unroll
-    for (int w = 0; w < SWAVES; w += 4) {
-        const f32x4 x = *(const f32x4 *)&cols[lane & (BOUNDS - 1)][w], y = *(const f32x4 *)&cols[BOUNDS + (lane & (BOUNDS - 1))][w];
-        at_k.s += (x[0] + x[1]) + (x[2] + x[3]);
-        at_k.n += (y[0] + y[1]) + (y[2] + y[3]);
-    }
     int turn = 0;
     auto above = [&](float c) {   // c > 0
         float sc = 0.f;
@@ -719,7 +772,7 @@ __global__ __launch_bounds__(STHREADS) void sample_draw_kernel(SampleArgs a, Sam
         unsigned lo, hi = __float_as_uint(pmax) + 1;
         SumCount at_lo, at_hi = {0.f, 0.f};
         if (!counts) {
-            if (!(top_p > 0.f && all >= top_p)) continue;
+            if (!nucleus) continue;
             lo = __float_as_uint(list_floor(top_p, V));
             at_lo = {all, n};
         } else {
@@ -739,7 +792,7 @@ __global__ __launch_bounds__(STHREADS) void sample_draw_kernel(SampleArgs a, Sam
             at_hi = {__shfl(at_k.s, k - 1, WAVE), __shfl(at_k.n, k - 1, WAVE)};
         }
         if (!counts && at_lo.n == n && n - at_hi.n > (float)FEW)   // all candidates reach lo: begin at the smallest of them
-            lo = max(lo, __float_as_uint(-wave_max(lane < segs ? -ws.part[lane * PART + 2 * BOUNDS + 2] : -INFINITY)));
+            lo = max(lo, __float_as_uint(-wave_max(lane < segs ? -small_own : -INFINITY)));
         while (hi - lo > 1 && at_lo.n - at_hi.n > (float)FEW) {
             // Sums and counts of up to 64 equal parts of the interval.  us a draw, one workgroup / bisection down to 1024 entries and a
             // list of these / this: 65536 equal logits, top_p 0.7 67 / 68 / 34, 50277 of them 58 / 67 / 33; 50277 from N(0, 3),
@@ -785,26 +838,51 @@ __global__ __launch_bounds__(STHREADS) void sample_draw_kernel(SampleArgs a, Sam
             lo += (unsigned)(63 - i) << shift;
             __syncthreads();   // the parts have been read
         }
-        const float flo = __uint_as_float(max(lo, 1u)), fhi = __uint_as_float(hi);
         if (hi - lo > 1) {
             // the entries of the interval, at most FEW, in any order at first
-            each([&](float x) {
-                if (x >= flo && x < fhi) few[min(atomicAdd(&n_few[counts], 1), FEW - 1)] = x;
-            });
+            unsigned ulo = max(lo, 1u);
+            const unsigned span = hi - ulo;   // positive floats order like their bits, and 0 falls out
+            auto inside = [&](float x) { return __float_as_uint(x) - ulo < span; };
+            int mine = 0;
+            each([&](float x) { mine += inside(x) ? 1 : 0; });
+            const float upto = wave_scan((float)mine);
+            const int of_wave = (int)last_lane(upto);
+            if (of_wave) {
+                int at = 0;
+                if (lane == 0) at = atomicAdd(&n_few[counts], of_wave);
+                at = __builtin_amdgcn_readfirstlane(at) + (int)upto - mine;
+                asm volatile("" : "+v"(ulo));   // 64 masks kept from the count would not fit the scalar registers
+#pragma unroll
+                for (int j = 0; j < SEG / 64; ++j)
+                    if (j < rounds && (inside(v[j][0]) || inside(v[j][1]) || inside(v[j][2]) || inside(v[j][3]))) {
+#pragma unroll
+                        for (int e = 0; e < 4; ++e)
+                            if (inside(v[j][e])) few[min(at++, FEW - 1)] = v[j][e];
+                    }
+            }
             __syncthreads();
             // sorted by counting the larger ones (four threads an entry), then added from the largest down
             const int m = min(n_few[counts], FEW), own_few = tid >> 2, q4 = tid & 3;
             if (16 * wave < m) {
-                const float x = few[own_few];
+                // A place is the number of larger entries and of equal ones ahead of it: y >= x is y > x - 1 in bits, for the groups of
+                // four ahead of its own.  Two instructions a comparison; places from m on hold zeros, which are never larger.
+                typedef int i32x4 __attribute__((ext_vector_type(4)));
+                const int x = __float_as_int(few[own_few]), group = own_few & ~3;
                 int rank = 0;
+#pragma unroll 4
                 for (int i = 4 * q4; i < m; i += 16) {
-                    const f32x4 y = *(const f32x4 *)&few[i];
+                    const i32x4 y = *(const i32x4 *)&few[i];
+                    const int than = i < group ? x - 1 : x;
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) rank += (i + e < m && (y[e] > x || (y[e] == x && i + e < own_few))) ? 1 : 0;
+                    for (int e = 0; e < 4; ++e) rank += y[e] > than ? 1 : 0;
+                }
+                if (group % 16 == 4 * q4) {
+#pragma unroll
+                    for (int e = 0; e < 3; ++e) rank += e < own_few - group && __float_as_int(few[group + e]) == x ? 1 : 0;
                 }
                 rank += __builtin_amdgcn_update_dpp(0, rank, 0xB1, 0xf, 0xf, true);
                 rank += __builtin_amdgcn_update_dpp(0, rank, 0x4E, 0xf, 0xf, true);
-                if (q4 == 0 && own_few < m) sorted[rank] = x;
+                if (q4 == 0 && own_few < m) sorted[rank] = __int_as_float(x);
             }
             __syncthreads();
             const f32x4 y = *(const f32x4 *)&sorted[4 * lane];
@@ -822,6 +900,7 @@ __global__ __launch_bounds__(STHREADS) void sample_draw_kernel(SampleArgs a, Sam
             }
             const unsigned long long good = __ballot(at > 0.f);
             if (good) lo = (unsigned)__builtin_amdgcn_readlane(__builtin_bit_cast(int, at), __builtin_ctzll(good));
+            if (!counts && tid < FEW) few[tid] = 0.f;   // read ahead of the last barrier, written past the next one
         }
         cut = __uint_as_float(lo);
     }
@@ -833,7 +912,7 @@ __global__ __launch_bounds__(STHREADS) void sample_draw_kernel(SampleArgs a, Sam
         for (int j = 0; j < SEG / 64; ++j)
             if (j < rounds) {
                 f32x4 q = v[j];
-                if (POW) q = *(const f32x4 *)(ws.pow + min(sg, segs - 1) * SEG + 64 * j + 4 * r);
+                if (POW) q = *(const f32x4 *)(powers + min(sg, segs - 1) * SEG + 64 * j + 4 * r);
 #pragma unroll
                 for (int e = 0; e < 4; ++e) sum += keep(v[j][e]) ? q[e] : 0.f;
             }
@@ -852,9 +931,9 @@ __global__ __launch_bounds__(STHREADS) void sample_draw_kernel(SampleArgs a, Sam
         int found = -1, last = 0;                 // places in the segment
         for (int i0 = 0; i0 < end && found < 0; i0 += 256) {   // four entries a lane
             const int i = i0 + 4 * lane;
-            f32x4 q = *(const f32x4 *)(ws.list + from * SEG + i), w = q;
-            if (POW) w = *(const f32x4 *)(ws.pow + from * SEG + i);
-            const uint2 id = *(const uint2 *)(ws.idx + from * SEG + i);
+            f32x4 q = *(const f32x4 *)(list + from * SEG + i), w = q;
+            if (POW) w = *(const f32x4 *)(powers + from * SEG + i);
+            const uint2 id = *(const uint2 *)(idx + from * SEG + i);
             const int ids[4] = {(int)(id.x & 0xffff), (int)(id.x >> 16), (int)(id.y & 0xffff), (int)(id.y >> 16)};
 #pragma unroll
             for (int e = 0; e < 4; ++e) q[e] = i + e < end && keep(q[e]) ? w[e] : 0.f;
@@ -969,10 +1048,13 @@ static size_t sample_ws(SampleWs &ws, void *base, int64_t V) {
     ws.p = (float *)base;
     ws.list = ws.p + n;
     ws.pow = ws.list + n;
-    ws.part = ws.pow + n;
-    ws.soft = ws.part + segs * PART;
-    ws.idx = (uint16_t *)(ws.soft + 2 * segs);
-    return (3 * n + segs * (PART + 2)) * sizeof(float) + n * sizeof(uint16_t);
+    ws.high = ws.pow + n;
+    ws.high_pow = ws.high + n;
+    ws.idx = (uint16_t *)(ws.high_pow + n);
+    ws.high_idx = ws.idx + n;
+    ws.soft = (float *)(ws.high_idx + n);
+    ws.part = ws.soft + 2 * segs;
+    return (5 * n + segs * (PART + 2)) * sizeof(float) + 2 * n * sizeof(uint16_t);
 }
 
 extern "C" size_t rwkv_sample_workspace(int64_t V) {

@@ -411,6 +411,39 @@ def test_draw_from_logits_close_to_each_other(V, kind):
 
 
 @pytest.mark.parametrize("V", [16388, 50277, 65536])
+@pytest.mark.parametrize("temp,top_k", [(1.0, 0), (0.8, 0), (1.0, 30)])
+def test_draw_whose_cut_is_at_the_end_of_the_short_list(V, temp, top_k):
+    """Cuts in ties at 2^-12.4 to 2^-13.6 of the largest probability, around the 2^-13 that the short list of candidates ends at: the
+    same entries, ids and (up to two roundings and the order of the sum) probabilities as with one workgroup."""
+    from chatrwkv_amd import lib
+    from chatrwkv_amd.sampling import Sampler
+    L = lib.load()
+    rng = np.random.Generator(np.random.PCG64([V, 13]))
+    levels = [0.0, 12.4, 12.9, 13.0, 13.1, 13.6]
+    sizes = [40, 600, 600, 600, 600, 600]
+    x = np.full(V, -30.0, np.float32)
+    at = rng.permutation(V)
+    for d, n in zip(levels, sizes):
+        x[at[:n]] = -d * np.log(2.0)
+        at = at[n:]
+    mass = np.array([n * 2.0 ** -d for d, n in zip(levels, sizes)])
+    s, xt = Sampler(V, device=DEV), torch.from_numpy(x).to(DEV)
+    probs, token = torch.empty_like(s.probs), torch.zeros_like(s.token)
+    for i in range(len(levels)):
+        top_p = float((mass[:i].sum() + 0.5 * mass[i]) / mass.sum())   # half a level is 1e-3: far from any rounding
+        u = torch.tensor([float(rng.random())], device=DEV)
+        s.sample(xt, temp, top_p, top_k, u=u, penalties=False)
+        _one_workgroup(L, xt, temp, top_p, top_k, u, probs, token)
+        got, ref = s.probs.cpu().numpy().astype(np.float64), probs.cpu().numpy().astype(np.float64)
+        kept = sum(sizes[:1 if top_k else i + 1])
+        assert (got > 0).sum() == kept and np.array_equal(got > 0, ref > 0), (i, temp, top_k)
+        assert np.abs(got - ref).max() <= 2e-6 * ref.max()
+        cdf = np.cumsum(ref)
+        if np.abs(cdf / cdf[-1] - float(u)).min() > 1e-5:
+            assert int(s.token) == int(token), (i, temp, top_k)
+
+
+@pytest.mark.parametrize("V", [16388, 50277, 65536])
 @pytest.mark.parametrize("kind,top_p,temp", [("equal", 0.7, 1.0), ("close", 0.7, 1.0), ("slope", 0.85, 0.8), ("normal", 0.999, 1.0), ("normal", 0.999, 0.8)])
 def test_draws_over_the_chip_are_not_slower(V, kind, top_p, temp):
     """Draws that keep or search thousands of entries: the three launches take no longer than the one-workgroup kernel on the
