@@ -49,9 +49,11 @@ __global__ __launch_bounds__(256) void ln_f32_f16_kernel(int C, const float *__r
 // top and kept in registers, the statistics of the two rows share their barriers, and so do the 2 NJ sums at the end: two global
 // round trips and three rounds of barriers.  256 threads per row and 512 form every value with the same operations in the same
 // order (row_sums), so both agree bit for bit.
-// PRE: the mix / scale vectors too are requested at the top (3 NJ CH more registers per thread: shorter chain, fewer
-// workgroups per CU -- for short calls, where a CU has one or two rows anyway).
-template <int NJ, int CH, bool PRE, int NT>
+// The first chunk's mix and scale vectors are requested at the top too, together, and the next chunk's ahead of this one's stores: a wait for a
+// load is one for every older store as well.  Requested mix by mix they were two trips to memory and a store's way there for each mix, one
+// after the other.
+// Q: some of the mixes are scaled and summed.
+template <int NJ, int CH, int NT, bool Q>
 __global__ __launch_bounds__(NT) void lnmix_seq_fast_kernel(const rwkv_half *x0, const rwkv_half *ln_w, const rwkv_half *ln_b, const rwkv_half *sx,
                                                             rwkv_half *state_out, int C, int T, SeqMixArgs a) {
     constexpr int NSUM = 2 * NJ > 3 ? 2 * NJ : 3;
@@ -66,7 +68,7 @@ __global__ __launch_bounds__(NT) void lnmix_seq_fast_kernel(const rwkv_half *x0,
     // Row 0's workgroup also forms the new token-shift state LN(x[T-1]): its statistics ride in the same barriers
     const bool commit = state_out && t == 0;
     const rwkv_half *xl = commit ? x0 + (size_t)(T - 1) * C : x;
-    h16x8 xv[CH], pxv[CH], lv[CH], wv[CH], bv[CH], mv[PRE ? NJ : 1][CH], rv[PRE ? NJ : 1][CH], yv[PRE ? NJ : 1][CH];
+    h16x8 xv[CH], pxv[CH], lv[CH], wv[CH], bv[CH], mv[NJ], rv[Q ? NJ : 1], yv[Q ? NJ : 1];
 #pragma unroll
     for (int c = 0; c < CH; ++c) {
         const int j8 = min(j8_0 + c * 256, nch - 1);   // chunks past the end repeat the last one (unused)
@@ -79,18 +81,19 @@ __global__ __launch_bounds__(NT) void lnmix_seq_fast_kernel(const rwkv_half *x0,
     const void *vec[3 * NJ];   // mix, ry, my
 #pragma unroll
     for (int j = 0; j < NJ; ++j) { vec[3 * j] = a.mix[j]; vec[3 * j + 1] = a.ry[j]; vec[3 * j + 2] = a.my[j]; }
-    if constexpr (PRE) {
-        if constexpr (NJ <= 4) at_once(vec);
+    auto request = [&](int c) {
+        const int j8 = min(j8_0 + c * 256, nch - 1);
 #pragma unroll
-        for (int c = 0; c < CH; ++c) {
-            const int j8 = min(j8_0 + c * 256, nch - 1);
-#pragma unroll
-            for (int j = 0; j < NJ; ++j) {
-                mv[j][c] = load8(vec[3 * j] ? vec[3 * j] : ln_w, j8);
-                if (vec[3 * j + 1]) { rv[j][c] = load8(vec[3 * j + 1], j8); yv[j][c] = load8(vec[3 * j + 2], j8); }
+        for (int j = 0; j < NJ; ++j) {
+            mv[j] = load8(vec[3 * j] ? vec[3 * j] : ln_w, j8);
+            if constexpr (Q) {
+                rv[j] = load8(vec[3 * j + 1] ? vec[3 * j + 1] : ln_w, j8);
+                yv[j] = load8(vec[3 * j + 1] ? vec[3 * j + 2] : ln_w, j8);
             }
         }
-    }
+    };
+    if constexpr (NJ <= 4) at_once(vec);
+    request(0);
     float st[3] = {0.f, 0.f, 0.f};
     row_sums<3, NT>(st, red, hop, [&](float (&v)[3], auto) {
 #pragma unroll
@@ -145,25 +148,20 @@ __global__ __launch_bounds__(NT) void lnmix_seq_fast_kernel(const rwkv_half *x0,
             else pv = *(const h16x8 *)(sx + 8 * j8);
         }
         if (a.xx_last && t == T - 1) *(h16x8 *)(a.xx_last + 8 * j8) = xx;
+        h16x8 o[NJ];
 #pragma unroll
         for (int j = 0; j < NJ; ++j) {
-            h16x8 kx = xx;
-            if (vec[3 * j]) {
-                h16x8 m8;
-                if constexpr (PRE) m8 = mv[j][c]; else m8 = load8(vec[3 * j], j8);
-                kx = mix8(xx, pv, m8, a.maa_form);
+            const h16x8 kx = vec[3 * j] ? mix8(xx, pv, mv[j], a.maa_form) : xx;
+            o[j] = kx;
+            if (Q && vec[3 * j + 1]) {
+                o[j] = kx * rv[j];
+                if constexpr (NT == 256) add_mix(acc, j, kx, yv[j]);
+                else { kv[c][j] = kx; sv[c][j] = yv[j]; }
             }
-            h16x8 o = kx;
-            if (vec[3 * j + 1]) {
-                h16x8 r8, y8;
-                if constexpr (PRE) { r8 = rv[j][c]; y8 = yv[j][c]; }
-                else { r8 = load8(vec[3 * j + 1], j8); y8 = load8(vec[3 * j + 2], j8); }
-                o = kx * r8;
-                if constexpr (NT == 256) add_mix(acc, j, kx, y8);
-                else { kv[c][j] = kx; sv[c][j] = y8; }
-            }
-            *(h16x8 *)(a.xs[j] + (size_t)t * C + 8 * j8) = o;
         }
+        if (c + 1 < CH) request(c + 1);
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) *(h16x8 *)(a.xs[j] + (size_t)t * C + 8 * j8) = o[j];
         // Only row 0 reads the old state, so row 0's workgroup writes the new one, each thread exactly the chunk it
         // has just read: no second launch.
         if (commit) {
@@ -172,10 +170,7 @@ __global__ __launch_bounds__(NT) void lnmix_seq_fast_kernel(const rwkv_half *x0,
             *(h16x8 *)(state_out + 8 * j8) = norm8(dl, lrstd, wv[c], bv[c]);
         }
     }
-    bool any = false;
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) any = any || vec[3 * j + 1];
-    if (any) {
+    if constexpr (Q) {
         row_sums<2 * NJ, NT>(acc, red + 24, hop, [&](float (&v)[2 * NJ], auto) {
             if constexpr (NT > 256)
 #pragma unroll
@@ -194,18 +189,26 @@ __global__ __launch_bounds__(NT) void lnmix_seq_fast_kernel(const rwkv_half *x0,
 
 }  // namespace
 
-template <int CH, bool PRE, int NT>
+template <int CH, int NT, bool Q>
 static bool lnmix_seq_fast_launch(const SeqMixArgs &a, int nj, hipStream_t st) {
     const dim3 grid((unsigned)a.T), block(NT);
     switch (nj) {
-        case 1: hipLaunchKernelGGL((lnmix_seq_fast_kernel<1, CH, PRE, NT>), grid, block, 0, st, a.x, a.ln_w, a.ln_b, a.sx, a.state_out, a.C, a.T, a); break;
-        case 2: hipLaunchKernelGGL((lnmix_seq_fast_kernel<2, CH, PRE, NT>), grid, block, 0, st, a.x, a.ln_w, a.ln_b, a.sx, a.state_out, a.C, a.T, a); break;
-        case 3: hipLaunchKernelGGL((lnmix_seq_fast_kernel<3, CH, PRE, NT>), grid, block, 0, st, a.x, a.ln_w, a.ln_b, a.sx, a.state_out, a.C, a.T, a); break;
-        case 4: hipLaunchKernelGGL((lnmix_seq_fast_kernel<4, CH, PRE, NT>), grid, block, 0, st, a.x, a.ln_w, a.ln_b, a.sx, a.state_out, a.C, a.T, a); break;
-        case 6: hipLaunchKernelGGL((lnmix_seq_fast_kernel<6, CH, PRE && NT == 256, NT>), grid, block, 0, st, a.x, a.ln_w, a.ln_b, a.sx, a.state_out, a.C, a.T, a); break;
+        case 1: hipLaunchKernelGGL((lnmix_seq_fast_kernel<1, CH, NT, Q>), grid, block, 0, st, a.x, a.ln_w, a.ln_b, a.sx, a.state_out, a.C, a.T, a); break;
+        case 2: hipLaunchKernelGGL((lnmix_seq_fast_kernel<2, CH, NT, Q>), grid, block, 0, st, a.x, a.ln_w, a.ln_b, a.sx, a.state_out, a.C, a.T, a); break;
+        case 3: hipLaunchKernelGGL((lnmix_seq_fast_kernel<3, CH, NT, Q>), grid, block, 0, st, a.x, a.ln_w, a.ln_b, a.sx, a.state_out, a.C, a.T, a); break;
+        case 4: hipLaunchKernelGGL((lnmix_seq_fast_kernel<4, CH, NT, Q>), grid, block, 0, st, a.x, a.ln_w, a.ln_b, a.sx, a.state_out, a.C, a.T, a); break;
+        case 6: hipLaunchKernelGGL((lnmix_seq_fast_kernel<6, CH, NT, Q>), grid, block, 0, st, a.x, a.ln_w, a.ln_b, a.sx, a.state_out, a.C, a.T, a); break;
         default: return false;
     }
     return true;
+}
+
+template <bool Q>
+static bool lnmix_seq_fast_width(const SeqMixArgs &a, int nj, hipStream_t st) {
+    const bool few = a.T <= 512;
+    if (a.C <= 2048) return lnmix_seq_fast_launch<1, 256, Q>(a, nj, st);
+    if (a.C <= 4096) return few ? lnmix_seq_fast_launch<1, 512, Q>(a, nj, st) : lnmix_seq_fast_launch<2, 256, Q>(a, nj, st);
+    return few ? lnmix_seq_fast_launch<2, 512, Q>(a, nj, st) : lnmix_seq_fast_launch<4, 256, Q>(a, nj, st);
 }
 
 int lnmix_seq_launch(const SeqMixArgs &a, int nj, hipStream_t st) {
@@ -215,21 +218,19 @@ int lnmix_seq_launch(const SeqMixArgs &a, int nj, hipStream_t st) {
     // 256 -> 512 threads at 45 / 256 / 512 / 600 / 1024 rows: one mix 4.2 -> 3.4, 4.4 -> 3.6, 4.7 -> 4.8, 5.4 -> 5.7, 6.6 -> 7.1;
     // three mixes with scaling 6.7 -> 5.4, 7.4 -> 6.1, 8.4 -> 7.9, 9.4 -> 10.4, 11.7 -> 12.6; six mixes without 6.7 -> 5.5, 8.0 ->
     // 6.8, 9.1 -> 8.5, 10.0 -> 11.7, 12.8 -> 14.5 (5120 channels, three mixes: 512 rows 10.6 -> 10.2, 600 rows 11.8 -> 14.6).
-    // Up to 4096 channels the mix and scale vectors of these calls are requested at the top too, except for six mixes.
     // These are launches one after the other on the same rows.  Within a call, whose products have used the caches since, us
     // before the element code of rows.h was written out (three to four instructions per step) and now: three scaled mixes of 4096
     // channels at 45 / 1024 rows 7.3 / 20.5 -> 5.9 / 16.1, two 6.3 / 16.5 -> 5.6 / 12.7; at 777 rows six 20.3 -> 16.7, one 9.5 ->
-    // 7.0; four of 2048 channels at 333 rows 7.1 -> 5.3; three of 768 at 513 rows 6.7 -> 4.9.  An empty launch is 3.2; at 1024 rows
+    // 7.0; four of 2048 channels at 333 rows 7.1 -> 5.3; three of 768 at 513 rows 6.7 -> 4.9.  With the vectors requested together, before ->
+    // now: three scaled mixes of 4096 channels at 1024 / 2048 rows 16.5 / 26.3 -> 14.5 / 22.3, of 5120 at 1024 26.2 -> 21.7; six of 4096 at 300 / 777 /
+    // 2048 9.7 / 16.9 / 30.2 -> 8.0 / 12.2 / 23.3; two scaled ones of 768 at 300 5.3 -> 4.5.  An empty launch is 3.2; at 1024 rows
     // it is the 130 KB per row through a CU's L1 and the 24 MB of stores.
     // Several rows per workgroup, sharing vectors and the previous row's statistics, measured with the element code before: slower
     // at every length (1024 rows 21.8 with two, 33 with four, 20.7 with one).
     if (a.C > 8192) return RWKV_E_SHAPE;
-    const bool few = a.T <= 512;
-    bool known;
-    if (a.C <= 2048) known = few ? lnmix_seq_fast_launch<1, true, 256>(a, nj, st) : lnmix_seq_fast_launch<1, false, 256>(a, nj, st);
-    else if (a.C <= 4096) known = few ? lnmix_seq_fast_launch<1, true, 512>(a, nj, st) : lnmix_seq_fast_launch<2, false, 256>(a, nj, st);
-    else known = few ? lnmix_seq_fast_launch<2, false, 512>(a, nj, st) : lnmix_seq_fast_launch<4, false, 256>(a, nj, st);
-    if (!known) return RWKV_E_SHAPE;
+    bool scaled = false;
+    for (int j = 0; j < nj; ++j) scaled = scaled || a.ry[j];
+    if (!(scaled ? lnmix_seq_fast_width<true>(a, nj, st) : lnmix_seq_fast_width<false>(a, nj, st))) return RWKV_E_SHAPE;
     RWKV_LAUNCH_CHECK();
     return RWKV_OK;
 }
