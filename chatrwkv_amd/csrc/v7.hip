@@ -312,7 +312,8 @@ __global__ __launch_bounds__(256) void wkv7_kernel(Wkv7Args a) {
 // 20 KB of fp32 operands pass from one to the other per head and chunk.  The first kernel moves them at 3.0 TB/s of a
 // copy's 4.8: about 1000 vector instructions a wave, a third of them the five exact divisions per element, six barriers and
 // the forward substitution of one wave beside three that wait.  Six workgroups a CU, by its 78 registers, against five by 30 KB
-// of LDS, and no chunks past the last: 777 tokens 39.3 -> 37 us.  The second is a chain of one exchange per chunk (35 us, 0.72 a chunk).  A
+// of LDS, and no chunks past the last: 777 tokens 39.3 -> 37 us (and 32 since the vectors
+// are requested together).  The second is a chain of one exchange per chunk (35 us, 0.72 a chunk).  A
 // 4096-wide layer, both together: 260 tokens 321 -> 314.5 us, 777 561.5 -> 557, 1024 the same.  Per layer at 64 heads,
 // preparation and recurrence, token by token -> chunks: 1024 tokens 152 -> 89 us, 777 tokens 116 -> 72, 256 tokens 42 -> 31,
 // 100 tokens 21 -> 19; at 64 tokens the two launches take as long as prep7_kernel and wkv7_kernel: CHUNKED7.
@@ -346,17 +347,22 @@ __global__ __launch_bounds__(256) void wkv7_chunk_kernel(Prep7Args a, int t_begi
     // ---- preparation, rounding by rounding as in prep7_kernel
     const h16x4 r4 = *(const h16x4 *)(a.r + o), k4 = *(const h16x4 *)(a.k + o), v4 = *(const h16x4 *)(a.v + o);
     const h16x4 ar4 = *(const h16x4 *)(a.a_raw + o), wr4 = *(const h16x4 *)(a.w_raw + o);
+    // The vectors, on any boundary of two bytes, are requested here too: read where they are used, in branches, eight of the reads were a trip
+    // to memory each, one after the other: 777 tokens of 4096 channels 36.4 -> 32.3 us, 1024 46.3 -> 40.3, 300 17.8 -> 16.2.
+    typedef h16x4 h16x4_any __attribute__((aligned(2)));
+    auto vec4 = [&](const rwkv_half *p) -> h16x4 { return *(const h16x4_any *)(p + ch); };
+    const h16x4 a04 = vec4(a.a0), kk4 = vec4(a.k_k), ka4 = vec4(a.k_a), rk4 = vec4(a.r_k), w04 = vec4(a.w0), v04 = vec4(a.vg_raw ? a.v0 : a.a0);
     h16x4 vg4 = {}, vf4 = {};
     if (a.vg_raw) { vg4 = *(const h16x4 *)(a.vg_raw + o); vf4 = *(const h16x4 *)(a.v_first + o); }
     float kku[4], av[4], k2[4], ss = 0.f, rks = 0.f;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
         const float k = (float)k4[e];
-        av[e] = round_h(sigmoidf_(round_h(h2f(a.a0[ch + e]) + (float)ar4[e])));
-        kku[e] = round_h(k * h2f(a.k_k[ch + e]));
+        av[e] = round_h(sigmoidf_(round_h((float)a04[e] + (float)ar4[e])));
+        kku[e] = round_h(k * (float)kk4[e]);
         ss += kku[e] * kku[e];
-        k2[e] = round_h(k * round_h(1.f + round_h(round_h(av[e] - 1.f) * h2f(a.k_a[ch + e]))));
-        rks += round_h(round_h((float)r4[e] * k2[e]) * h2f(a.r_k[ch + e]));
+        k2[e] = round_h(k * round_h(1.f + round_h(round_h(av[e] - 1.f) * (float)ka4[e])));
+        rks += round_h(round_h((float)r4[e] * k2[e]) * (float)rk4[e]);
     }
     const float nrm = fmaxf(round_h(sqrtf(row16_sum(ss))), 1e-12f);
     rks = row16_sum(rks);
@@ -367,10 +373,10 @@ __global__ __launch_bounds__(256) void wkv7_chunk_kernel(Prep7Args a, int t_begi
         const float kk = round_h(kku[e] / nrm);
         if (a.vg_raw) {
             const float v = (float)v4[e];
-            const float sg = round_h(sigmoidf_(round_h(h2f(a.v0[ch + e]) + (float)vg4[e])));
+            const float sg = round_h(sigmoidf_(round_h((float)v04[e] + (float)vg4[e])));
             vo[e] = (h16)(v + round_h(round_h((float)vf4[e] - v) * sg));
         }
-        w[e] = live ? __expf(-0.606531f * sigmoidf_(round_h(h2f(a.w0[ch + e]) + (float)wr4[e]))) : 1.f;
+        w[e] = live ? __expf(-0.606531f * sigmoidf_(round_h((float)w04[e] + (float)wr4[e]))) : 1.f;
         rr[e] = live ? (float)r4[e] : 0.f;
         kk2[e] = live ? k2[e] : 0.f;
         aa[e] = live ? -kk : 0.f;
