@@ -272,7 +272,7 @@ DEV void stream_rows(const RowSplit &sp, int nseg, int npw, unsigned *sync, ProL
     // ranges, batch counters, loop control) is wave-uniform and keeps it in scalar registers
     const int wave = blockIdx.x * DWAVES + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int g0 = split_at(sp, wave), g1 = split_at(sp, wave + 1);
-    const int glast = g1 > g0 ? g1 - 1 : 0;
+    const int glast = g1 > g0 ? g1 - 1 : g0;                    // without rows of its own (loads that are never used): the next row, not one for all such waves
     const int nsb = (nseg + 64 * U - 1) / (64 * U);             // segment batches per group batch
     const int sb_epi = nsb > 1 ? 1 : 0;                         // segment batch that carries the epilogue operands
     const int odd_epi = (nsb - 1 + sb_epi) & 1;                 // 1: it and the last segment batch are in different tiles
