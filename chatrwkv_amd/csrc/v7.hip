@@ -40,7 +40,7 @@ struct Prep7Args {
 };
 
 // Eight adjacent channels per lane (16-byte accesses), so the eight lanes of a row of eight own one head of one
-// token: grid-stride over the T * C / 8 chunks.  Every step rounds to fp16 where an fp16 tensor operation of the
+// token: a workgroup has 256 of the C / 8 chunks of one row.  Every step rounds to fp16 where an fp16 tensor operation of the
 // reference does; the two sums over a head run over a lane's eight channels in index order and then over the
 // eight lanes in three DPP steps.
 DEV float head8_sum(float v) {
@@ -636,7 +636,7 @@ __global__ __launch_bounds__(256, 2) void wkv7_apply_kernel(int H, int C, float 
 
 // GroupNorm over each head's 64 outputs (eps 64e-5) on the fp16-rounded read-out, + bonus * v, * g.  Four adjacent
 // channels per lane (16-byte loads of y, 8-byte accesses to v, g and the output): a row of 16 lanes owns one head
-// of one token, its two sums are DPP row sums; grid-stride over the T * C / 4 chunks.
+// of one token, its two sums are DPP row sums; a workgroup has 256 of the C / 4 chunks of one row.
 __global__ __launch_bounds__(256) void gn7_kernel(int per_row, uint64_t factor, int C, const float *__restrict__ y,
                                                   const rwkv_half *__restrict__ lnx_w,
                                                   const rwkv_half *__restrict__ lnx_b, const float *__restrict__ rk,

@@ -682,7 +682,7 @@ __global__ __launch_bounds__(256, 2) void wkv56_apply_kernel(Wkv56Args a, int H,
 
 // GroupNorm over each head's 64 outputs (eps 64e-5), affine, fp16 rounding, gate.  Four adjacent channels per lane
 // (16-byte loads of y and of the affine vectors, 8-byte accesses to the gate and the output): a row of 16 lanes owns
-// one head of one token, its two sums are DPP row sums; grid-stride over the T * C / 4 chunks.
+// one head of one token, its two sums are DPP row sums; a workgroup has 256 of the C / 4 chunks of one row.
 __global__ __launch_bounds__(256) void wkv56_gn_kernel(int per_row, uint64_t factor, int C, const float *__restrict__ y,
                                                        const float *__restrict__ lnx_w, const float *__restrict__ lnx_b,
                                                        const rwkv_half *__restrict__ gate, rwkv_half *__restrict__ out) {
