@@ -220,7 +220,7 @@ def gemm_roofline(T, N, M, u8, reps=20):
         ms = ctypes.c_float(0.0)
         lib.check(L.rwkv_mm8_seq_time_kernel(*args, reps, ctypes.byref(ms)), "rwkv_mm8_seq_time_kernel")
         t = ms.value * 1e-3
-        name = "gemm_dma_kernel<uint8 weights> (direct-to-LDS loads; 256x256 or 128x128 tile by the launch cost model)"
+        name = "gemm_dma_kernel<uint8 weights> (direct-to-LDS loads; tile by the launch cost model)"
         extra = {"with_scaling_pass": {"kernel": "mm8_prepare_kernel + " + name.split(" (")[0],
                                        "ms_per_call": t_op * 1e3, "achieved": flops / t_op / 1e12,
                                        "frac": flops / t_op / MFMA_F16_PEAK}}
@@ -230,7 +230,7 @@ def gemm_roofline(T, N, M, u8, reps=20):
         def run():
             lib.check(L.rwkv_gemm_f16(T, N, M, x.data_ptr(), N, w.data_ptr(), 1, N, y.data_ptr(), M, lib.RWKV_DT_F16, st),
                       "rwkv_gemm_f16")
-        name = "gemm_dma_kernel<fp16 weights> (direct-to-LDS loads; 256x256 or 128x128 tile by the launch cost model)"
+        name = "gemm_dma_kernel<fp16 weights> (direct-to-LDS loads; tile by the launch cost model)"
         t = timed(run)
     return {"bound": "mfma", "kernel": f"{name}, [{T} x {N}] x [{N} x {M}]", "achieved": flops / t / 1e12,
             "peak": MFMA_F16_PEAK / 1e12, "unit": "TFLOP/s", "frac": flops / t / MFMA_F16_PEAK,
