@@ -23,7 +23,7 @@ constexpr TileDim tile_dim[TILES] = {{256, 256}, {128, 128}, {128, 128}, {64, 12
 //   launch + rounds * (round, or split_round, which leaves the epilogue to the second pass)
 //          + k-tiles * (step_1 for every full round, between step_0 and step_1 for the last one by the CUs busy,
 //                       extra for what exceeds one round)
-//          + with a split, slab per 16 MB of fp32 slabs written and read and split per slab.
+//          + with a split, slab per 16 MB of fp32 slabs written and read, split per slab, and SECOND_LAUNCH.
 // One fit per tile and type, over launches within 1.6 times the best one of 648 products each (24 lengths from 17 to 2048 rows, 27 widths
 // from 64 to 20480; weights from HBM; the chip under load before): the tile and split it picks takes 1 % (uint8) and 2 %
 // (fp16) longer than the best of all on average, with products that the host launches no faster counted in.  A tile per round costs
@@ -32,10 +32,17 @@ constexpr TileDim tile_dim[TILES] = {{256, 256}, {128, 128}, {128, 128}, {64, 12
 // 96 where a round of 128 x 128 leaves CUs idle (fitted apart, at full depth, 97 rows and more).
 // us, uint8 / fp16 weights: [1024 x 4096] x [4096 x 12288] three rounds of 128 x 128 115.7 / 132.5, one of 256 x 192 90 / 97; [777 x
 // 4096] x [4096 x 16384] 256 x 256 126 / 130, 224 x 256 100 / 107; [768 x 4096] x [4096 x 12288] 104 / 109, 192 x 192 71 / 80;
-// [45 x 4096] x [4096 x 4096] four splits of 64 x 64 11.0 / 12.4, 48 x 16 8.7 / 10.6; [45 x 4096] x [4096 x 20480] 64 x 128 26.5 /
+// [45 x 4096] x [4096 x 4096] four splits of 64 x 64 11.0 / 12.4, 48 x 16 at full depth 8.7 / 10.6; [45 x 4096] x [4096 x 20480] 64 x 128 26.5 /
 // 40.6, 48 x 96 23.8 / 37.9; [24 x 2048] x [2048 x 2048] 8.1 / 8.1, 32 x 16 5.6 / 5.5; [333 x 2048]
 // x [2048 x 8192] four-stage 128 x 128 21.5 / 22.8, 96 x 128 19.1 / 20.2; [160 x 4096] x [4096 x 16384] 40.5 / 44.0, 33.5 / 42.7; [513 x
 // 4096] x [4096 x 4096] 33.0 / 31.8, 128 x 96 28.9 / 29.7; [513 x 1280] x [1280 x 3840] 16.1 / 14.3, 96 x 96 12.4 / 12.0.
+// A split's second launch was measured again as part of a chain of launches (graphs of 4 to 24 of them, each on weights of its own; 952 products of
+// 17 to 513 rows per type, up to 16 candidates each): the splits of 32 x 16 took 0.9 / 0.55 us more than fitted beside the other
+// tiles, all splits together 0.2.  With both in the prices the choice for those products takes 0.9 / 2.4 % longer than the best candidate,
+// 1.1 / 2.7 before (and 1.0 / 2.5 or 1.5 / 2.8 with 0.5 or 2 us on every split instead).  us, scaling pass included: uint8 [24 x 3072] x [3072
+// x 768] two splits 9.8, full depth 9.0; [17 x 4096] x [4096 x 2048] 10.6, 9.7; [45 x 4096] x [4096 x 4096] 48 x 32 in two splits 14.6, 48 x 16 14.2;
+// fp16 [17 x 3072] x [3072 x 768] 7.1, 6.3.  [513 x 3072] x [3072 x 768], 64 x 64, two splits / full depth: uint8 17.8 both, fp16 12.3 / 12.6.
+constexpr float SECOND_LAUNCH = 0.2f;
 struct TilePrice { float launch, round, split_round, step_0, step_1, extra, slab, split; };
 constexpr TilePrice tile_price[2][TILES] = {
     {   // fp16 weights
@@ -54,7 +61,7 @@ constexpr TilePrice tile_price[2][TILES] = {
         {6.807f, 2.897f, 4.219f, 0.444f, 1.116f, 0.f, 2.900f, 0.f},   // 160x192
         {3.811f, 5.068f, 6.800f, 0.674f, 1.048f, 0.f, 4.031f, 0.006f},   // 128x256
         {3.662f, 4.895f, 5.956f, 0.520f, 0.831f, 0.015f, 3.948f, 0.f},   // 128x192
-        {2.064f, 1.754f, 1.770f, 0.045f, 0.071f, 0.029f, 8.577f, 0.499f},   // 32x16
+        {2.064f, 1.754f, 2.120f, 0.045f, 0.071f, 0.029f, 8.577f, 0.499f},   // 32x16
         {3.459f, 0.f, 0.708f, 0.075f, 0.127f, 0.004f, 0.f, 0.356f},   // 32x32
         {2.995f, 1.030f, 2.668f, 0.077f, 0.169f, 0.031f, 0.f, 0.107f},   // 32x48
         {2.020f, 1.586f, 3.023f, 0.107f, 0.209f, 0.002f, 0.f, 0.249f},   // 32x64
@@ -88,7 +95,7 @@ constexpr TilePrice tile_price[2][TILES] = {
         {6.671f, 4.130f, 4.142f, 0.495f, 0.891f, 0.104f, 3.467f, 0.f},   // 160x192
         {6.383f, 3.449f, 3.229f, 0.589f, 0.939f, 0.128f, 3.964f, 0.092f},   // 128x256
         {6.019f, 3.214f, 3.148f, 0.518f, 0.752f, 0.093f, 4.309f, 0.040f},   // 128x192
-        {1.699f, 2.323f, 2.288f, 0.041f, 0.055f, 0.f, 12.951f, 0.432f},   // 32x16
+        {1.699f, 2.323f, 2.958f, 0.041f, 0.055f, 0.f, 12.951f, 0.432f},   // 32x16
         {3.999f, 0.f, 0.899f, 0.066f, 0.083f, 0.004f, 2.289f, 0.215f},   // 32x32
         {2.913f, 1.532f, 3.101f, 0.071f, 0.098f, 0.023f, 2.608f, 0.078f},   // 32x48
         {4.114f, 0.f, 1.196f, 0.086f, 0.112f, 0.015f, 3.985f, 0.176f},   // 32x64
@@ -189,7 +196,7 @@ class Launch {
             for (int t = from; t < to; ++t) {
                 const float wgs = tiles[t] * c, x = wgs * (1.f / 256.f), rounds = (float)(int)((wgs + 255.f) * (1.f / 256.f));
                 float k = p.launch[t] + rounds * round[t] + d * p.step_1[t] * x + d * p.step_0[t] * (rounds - x) + d * p.extra[t] * (x > 1.f ? x - 1.f : 0.f);
-                k += s ? c * (p.split[t] + p.slab[t] * out16) : 0.f;
+                k += s ? SECOND_LAUNCH + c * (p.split[t] + p.slab[t] * out16) : 0.f;
                 ks[t] = k < us[t] ? c : ks[t];
                 us[t] = k < us[t] ? k : us[t];
             }

@@ -31,7 +31,7 @@ static TilePick one_by_one(bool w_u8, int64_t T, int nk, int n, const int64_t *M
             float us = p.launch + (float)(full + (last > 0.f)) * (c > 1 ? p.split_round : p.round) + depth * p.step_1 * ((float)full + last);
             if (last > 0.f) us += depth * p.step_0 * (1.f - last);
             if (wgs > 256) us += depth * p.extra * ((float)wgs / 256.f - 1.f);
-            if (c > 1) us += (float)c * (p.split + p.slab * (float)(4 * outs) / (float)(16 << 20));
+            if (c > 1) us += SECOND_LAUNCH + (float)c * (p.split + p.slab * (float)(4 * outs) / (float)(16 << 20));
             if (us < best.us) best = {tile, c, us};
         }
     }
@@ -53,7 +53,6 @@ extern "C" double time_choice(int slow, int reps) {
     }
     return std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count() / reps * 1e9;
 }
-extern "C" int tiles() { return TILES; }
 """
 
 
@@ -106,3 +105,13 @@ def test_choice_takes_little_host_time(choice):
     products of 11 to 20 us by the operators up to 8 % slower; well under that here (0.33 of it as measured)."""
     ratio = min(choice.time_choice(0, 20000) / choice.time_choice(1, 20000) for _ in range(5))
     assert ratio < 0.6, ratio
+
+
+@pytest.mark.parametrize("u8,N,M,Ts", [(1, 3072, 768, (17, 24, 32)), (1, 4096, 2048, (17, 24, 32)), (1, 3072, 1280, (17,)),
+                                       (1, 4096, 4096, (45,)), (1, 3072, 768, (513,)), (0, 3072, 768, (17, 24))])
+def test_a_split_pays_for_its_second_launch(choice, u8, N, M, Ts):
+    """Products that are as fast or up to 0.9 us faster at full depth in a chain of launches, and one launch less for the host."""
+    for T in Ts:
+        assert _pick(choice, u8, T, N // 64, [M]).ks == 1, T
+    # and one that gains by it
+    assert _pick(choice, 0, 513, 48, [768]).ks == 2
