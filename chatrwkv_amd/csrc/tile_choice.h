@@ -126,9 +126,14 @@ constexpr Prices by_field(const TilePrice (&p)[TILES]) {
 }
 constexpr Prices prices[2] = {by_field(tile_price[0]), by_field(tile_price[1])};
 
-// The calls that a tile is offered for: those it was measured in.
-inline bool tile_offered(int tile, int64_t T) {
-    if (tile >= TILE_96x128) return T > 96;
+// The launches that a tile is offered for: those it was measured in.  The tiles with a side of 96 in calls of 65 to 96 rows, one row of tiles,
+// where they nearly fill a round: us, scaling pass included, at 80 or 96 rows with them / with the best choice among the others / with the one
+// that was taken, uint8 [4096] x [4096 x 20480], 214 of them, 37.4 / 39.6 / 44.0, [2048] x [2048 x 18432], 192, 22.3 / 24.2 / 25.8, fp16 47.2 / 50.1 / 51.0 and
+// 24.7 / 26.1 / 27.0; the 32768 outputs of 256 of 96 x 128 48.0 / 49.5.  With fewer the others are faster by more than the
+// prices say, uint8 [4096] x [4096 x 14336], 150, 34.7 / 28.7, [4096 x 12288] 34.4 / 26.0, [4096 x 4096] 32.8 / 16.2, and so they are past a
+// round, [2048] x [2048 x 50304] 44.7 / 42.1.  5120 inputs, fp16, 65 rows: up to 3 % slower with them, at 96 rows 8 % faster.
+inline bool tile_offered(int tile, int64_t T, float tiles) {
+    if (tile >= TILE_96x128) return T > 96 || (T > 64 && tiles >= 192.f && tiles <= 256.f);
     if (tile >= TILE_32x16) return T <= (tile_dim[tile].tn <= 32 ? 128 : 256);
     return tile != TILE_N || T <= 64;
 }
@@ -163,7 +168,7 @@ class Launch {
     }
     // `tile` with the K split of least cost, at full depth where it is not offered
     TilePick with(bool w_u8, int tile) const {
-        if (!tile_offered(tile, T)) return {tile, 1, NEVER};
+        if (!tile_offered(tile, T, tiles(tile))) return {tile, 1, NEVER};
         float us[TILES], ks[TILES];
         price(prices[w_u8], tile, tile + 1, us, ks);
         return {tile, (int)ks[tile], us[tile]};
@@ -172,21 +177,23 @@ class Launch {
     TilePick best(bool w_u8) const {
         float us[TILES], ks[TILES];
         const Prices &p = prices[w_u8];
-        price(p, 0, T <= 256 ? TILE_96x128 : TILE_32x16, us, ks);
+        const int few = T <= 256 ? TILE_96x128 : TILE_32x16;
+        price(p, 0, few, us, ks);
         price(p, TILE_96x128, TILES, us, ks);
         TilePick b = {TILE_S, 1, NEVER};
-        for (int t = 0; t < TILES; ++t)
-            if (tile_offered(t, T) && us[t] < b.us) b = {t, (int)ks[t], us[t]};
+        for (int t = 0; t < TILES; t = t + 1 == few ? TILE_96x128 : t + 1)
+            if (us[t] < b.us && tile_offered(t, T, tiles(t))) b = {t, (int)ks[t], us[t]};
         return b;
     }
 
   private:
+    float tiles(int t) const { return (float)rows[tile_dim[t].tm >> 4] * (float)cols[tile_dim[t].tn >> 4]; }
     // prices of the tiles [from, to) with their best K splits.  The tiles with a side of 96 run at full depth only: split they were the
     // best of all, by 5 % at most, for 6 of 560 products, and priced for it they took others where they are 10 to 15 % slower.
     void price(const Prices &p, int from, int to, float *us, float *ks) const {
-        float tiles[TILES];
+        float n[TILES];
         for (int t = from; t < to; ++t) {
-            tiles[t] = (float)rows[tile_dim[t].tm >> 4] * (float)cols[tile_dim[t].tn >> 4];
+            n[t] = tiles(t);
             us[t] = NEVER;
             ks[t] = 1.f;
         }
@@ -194,7 +201,7 @@ class Launch {
             const float c = ways[s], d = depth[s];
             const float *round = s ? p.split_round : p.round;
             for (int t = from; t < to; ++t) {
-                const float wgs = tiles[t] * c, x = wgs * (1.f / 256.f), rounds = (float)(int)((wgs + 255.f) * (1.f / 256.f));
+                const float wgs = n[t] * c, x = wgs * (1.f / 256.f), rounds = (float)(int)((wgs + 255.f) * (1.f / 256.f));
                 float k = p.launch[t] + rounds * round[t] + d * p.step_1[t] * x + d * p.step_0[t] * (rounds - x) + d * p.extra[t] * (x > 1.f ? x - 1.f : 0.f);
                 k += s ? SECOND_LAUNCH + c * (p.split[t] + p.slab[t] * out16) : 0.f;
                 ks[t] = k < us[t] ? c : ks[t];

@@ -19,11 +19,11 @@ SOURCE = r"""
 static TilePick one_by_one(bool w_u8, int64_t T, int nk, int n, const int64_t *M, uint64_t ws) {
     TilePick best = {TILE_S, 1, NEVER};
     for (int tile = 0; tile < TILES; ++tile) {
-        if (!tile_offered(tile, T)) continue;
         const TileDim d = tile_dim[tile];
         const TilePrice &p = tile_price[w_u8][tile];
         int64_t tiles = 0, outs = 0;
         for (int i = 0; i < n; ++i) { tiles += ((T + d.tm - 1) / d.tm) * ((M[i] + d.tn - 1) / d.tn); outs += T * M[i]; }
+        if (!tile_offered(tile, T, (float)tiles)) continue;
         for (int c = 1; c <= 8; ++c) {
             if (nk % c || (c > 1 && (nk / c < 8 || 4 * (uint64_t)outs * c > ws || tile >= TILE_96x128))) continue;
             const int64_t wgs = tiles * c, full = wgs / 256;
@@ -91,7 +91,7 @@ def test_choice_is_the_one_of_least_cost(choice):
     """Against the definition in 64-bit divisions, one tile and one split after the other: the same tile, split and price, bit for bit,
     for 1 to 4 products, at the edges of every side and of what a tile is offered for, and far past the models' sizes."""
     rng = np.random.default_rng(1)
-    edges = [1, 2, 16, 17, 63, 64, 65, 96, 97, 128, 129, 223, 225, 256, 257, 1024, 65535, 1 << 20]
+    edges = [1, 2, 16, 17, 63, 64, 65, 80, 96, 97, 128, 129, 223, 225, 256, 257, 1024, 65535, 1 << 20]
     for i in range(20000):
         T = int(rng.choice(edges)) if i % 3 == 0 else int(np.exp(rng.uniform(0, np.log(70000))))
         M = [int(rng.choice([16, 97, 255, 257, 50277, 64 * int(rng.integers(1, 400)), 8 * int(rng.integers(1, 9000))]))
@@ -115,3 +115,18 @@ def test_a_split_pays_for_its_second_launch(choice, u8, N, M, Ts):
         assert _pick(choice, u8, T, N // 64, [M]).ks == 1, T
     # and one that gains by it
     assert _pick(choice, 0, 513, 48, [768]).ks == 2
+
+
+@pytest.mark.parametrize("u8", [1, 0])
+@pytest.mark.parametrize("N,M", [(4096, [4096, 16384]), (4096, [4096, 14336]), (5120, [20480]), (2048, [18432]), (4096, [24576])])
+def test_tiles_of_96_rows_in_calls_of_65_to_96(choice, u8, N, M):
+    """Launches of 192 to 256 workgroups take them, so that 65 to 96 rows cost no more than 97; others, where they are slower by up to a
+    factor of two, do not."""
+    more = _pick(choice, u8, 97, N // 64, M).us
+    for T in (65, 72, 80, 95, 96):
+        p = _pick(choice, u8, T, N // 64, M)
+        assert p.tm == 96 and p.us <= more, (T, p.key(), more)
+    for T in (64, 65, 80, 96):
+        for few in ([M[0] // 2], [12288], [16384], [4096] * 3, [50304], [65536]):
+            p = _pick(choice, u8, T, N // 64, few)
+            assert p.tm != 96 and (p.tm, p.tn) != (128, 96), (T, few, p.key())
