@@ -447,7 +447,7 @@ __global__ __launch_bounds__(64 * WT * WM) void gemm_kernel(int T, int N, int M,
 }
 
 // ---- operands straight from global memory into LDS ------------------------------------------------------------
-// Tiles of 64 to 256 rows and 128 to 256 columns, eight waves (2 x 4; the 64-row tile four, 1 x 4), stages of one 64-deep k-tile.
+// Tiles of 96 to 256 rows and columns, eight waves (2 x 4, with K over two groups 2 x 2 each), stages of one 64-deep k-tile.
 // The loads are global_load_lds_dwordx4: one wave instruction copies 64 x 16 B into 1 KB of LDS without passing through
 // registers, so no wave spends issue slots on ds_write or on holding prefetched tiles.  A uint8 weight tile stays
 // uint8 in LDS (half the bytes of fp16) and becomes fp16 in the fragments on the way to the matrix cores.
@@ -475,14 +475,15 @@ __global__ __launch_bounds__(64 * WT * WM) void gemm_kernel(int T, int N, int M,
 // first wave and after the last, 2.5 until the first tile is there, 3 until the outputs are in LDS, 7 until they have left (32 MB at once).
 // Four stages instead of three on the 128 x 128 tile [256 x 4096] x [4096 x 12288] 46.0 -> 40.2 us; slower where the tiles take
 // several rounds, as only one workgroup then fits a CU.
-template <bool W_U8, int TM, int TN, int NW = 8, int NSTG = 0> struct DmaCfg {
+template <bool W_U8, int TM, int TN, int NSTG> struct DmaCfg {
+    static constexpr int NW = 8;                                                              // waves
     static constexpr int A = TM * BK * 2, W = W_U8 ? TN * BK : TN * BK * 2, STAGE = A + W;
     static constexpr int NST = NSTG ? NSTG : 3 * STAGE + (W_U8 ? 2 * TM * 4 + 2 * TN * 2 : 0) <= 160 * 1024 ? 3 : 2;
     static constexpr int AP = A / 1024, WP = W / 1024;                                        // 1 KB loads of a stage
     static constexpr int AL = (AP + NW - 1) / NW, WL = (WP + NW - 1) / NW, LOADS = AL + WL;   // per wave; past the end the last one again
-    static constexpr int KG = NW == 8 && NST == 4 ? 2 : 1;                                    // groups of waves that share K
+    static constexpr int KG = NST == 4 ? 2 : 1;                                               // groups of waves that share K
     static constexpr bool SPLITS = TM != 96 && TN != 96;                                      // K split over workgroups: see tile_choice.h
-    static constexpr int WR = TM > 64 ? 2 : 1, WC = NW / WR / KG;                             // waves: 2 rows x 4 columns; 64-row tile: 1 x 4
+    static constexpr int WR = 2, WC = NW / WR / KG;                                           // waves of a group: rows, columns
     static constexpr int MI = TM / (16 * WR), NI = TN / (16 * WC);                            // 16 x 16 blocks per wave
     static constexpr int HS = MI > 4 ? 2 : 1, H0 = HS == 2 ? (MI + 1) / 2 : MI;               // row blocks in one or two halves
     static constexpr int STG_STRIDE = TN + 4;   // epilogue staging, floats: 16 bytes apart, so 16 rows fill all banks
@@ -528,13 +529,13 @@ constexpr int vm_only(int n) { return 0x0F70 | (n & 15) | ((n >> 4) << 14); }
 constexpr int vm_lgkm0(int n) { return 0x0070 | (n & 15) | ((n >> 4) << 14); }
 constexpr int lgkm_only(int n) { return 0xC07F | (n << 8); }
 
-template <bool W_U8, bool SPLIT, int TM, int TN, int NW, int NSTG>
+template <bool W_U8, bool SPLIT, int TM, int TN, int NSTG>
 DEV void gemm_dma_body(int bid, int T, int N, int M, int walk_m, const h16 *__restrict__ A, int64_t lda, const void *__restrict__ Wv,
                        int64_t ldw, void *__restrict__ Y, int64_t ldy, const GemmEpi &ep, int nk_split,
                        float *__restrict__ part, int split) {
-    using Cfg = DmaCfg<W_U8, TM, TN, NW, NSTG>;
+    using Cfg = DmaCfg<W_U8, TM, TN, NSTG>;
     constexpr int D_A = Cfg::A, D_STAGE = Cfg::STAGE, D_NST = Cfg::NST, AL = Cfg::AL, WL = Cfg::WL, MI = Cfg::MI, NI = Cfg::NI;
-    constexpr int HS = Cfg::HS, H0 = Cfg::H0, KG = Cfg::KG;
+    constexpr int HS = Cfg::HS, H0 = Cfg::H0, KG = Cfg::KG, NW = Cfg::NW;
     extern __shared__ __align__(1024) unsigned char smem[];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int grp = wave / (Cfg::WR * Cfg::WC), wr = wave / Cfg::WC % Cfg::WR, wc = wave % Cfg::WC;
@@ -1055,39 +1056,39 @@ int64_t group_tiles(bool w_u8, GemmGroup &g, int n, int64_t T, int64_t N, int tm
 }
 
 // the direct-to-LDS kernel
-template <bool W_U8, bool SPLIT, int TM, int TN, int NW, int NSTG>
-__global__ __launch_bounds__(64 * NW) void gemm_dma_kernel(int T, int N, int units, int splits, int first1, int first2, int first3, int nk_split,
+template <bool W_U8, bool SPLIT, int TM, int TN, int NSTG>
+__global__ __launch_bounds__(512) void gemm_dma_kernel(int T, int N, int units, int splits, int first1, int first2, int first3, int nk_split,
                                                            int64_t lda, GemmMembers g) {
     const int unit = xcd_unit(units);
     int tile = SPLIT ? unit / splits : unit;
     const int split = SPLIT ? unit - tile * splits : 0;
     const GemmMember &m = g.m[group_member(first1, first2, first3, tile)];
     const GemmIn in = gemm_in(m);
-    gemm_dma_body<W_U8, SPLIT, TM, TN, NW, NSTG>(tile, T, N, in.M, in.walk_m, in.A, lda, in.W, in.ldw, m.Y, m.ldy, m.ep, nk_split, m.part,
+    gemm_dma_body<W_U8, SPLIT, TM, TN, NSTG>(tile, T, N, in.M, in.walk_m, in.A, lda, in.W, in.ldw, m.Y, m.ldy, m.ep, nk_split, m.part,
                                                  split);
 }
 
-template <bool W_U8, int TM, int TN, int NW, int NSTG>
+template <bool W_U8, int TM, int TN, int NSTG>
 int launch_dma(GemmGroup &g, int n, int64_t T, int64_t N, int ks, hipStream_t st) {
-    using Cfg = DmaCfg<W_U8, TM, TN, NW, NSTG>;
+    using Cfg = DmaCfg<W_U8, TM, TN, NSTG>;
     constexpr size_t lds = Cfg::LDS;
     if (ks > 1 && !Cfg::SPLITS) return RWKV_E_DTYPE;
     static PerDeviceOnce once;
     bool *attr_done = once.slot();
     if (!attr_done || !*attr_done) {
-        hipError_t e = hipFuncSetAttribute((const void *)gemm_dma_kernel<W_U8, false, TM, TN, NW, NSTG>,
+        hipError_t e = hipFuncSetAttribute((const void *)gemm_dma_kernel<W_U8, false, TM, TN, NSTG>,
                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if constexpr (Cfg::SPLITS) {
             if (e == hipSuccess)
-                e = hipFuncSetAttribute((const void *)gemm_dma_kernel<W_U8, true, TM, TN, NW, NSTG>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                e = hipFuncSetAttribute((const void *)gemm_dma_kernel<W_U8, true, TM, TN, NSTG>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                         (int)lds);
         }
         if (e != hipSuccess) return (int)e;
         if (attr_done) *attr_done = true;
     }
     const int units = (int)group_tiles(W_U8, g, n, T, N, TM, TN) * ks;
-    const auto kernel = Cfg::SPLITS && ks > 1 ? gemm_dma_kernel<W_U8, Cfg::SPLITS, TM, TN, NW, NSTG> : gemm_dma_kernel<W_U8, false, TM, TN, NW, NSTG>;
-    hipLaunchKernelGGL(kernel, dim3((unsigned)units), dim3(64 * NW), lds, st, (int)T, (int)N, units, ks, g.first[1], g.first[2], g.first[3], g.nk_split, g.lda,
+    const auto kernel = Cfg::SPLITS && ks > 1 ? gemm_dma_kernel<W_U8, Cfg::SPLITS, TM, TN, NSTG> : gemm_dma_kernel<W_U8, false, TM, TN, NSTG>;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)units), dim3(64 * Cfg::NW), lds, st, (int)T, (int)N, units, ks, g.first[1], g.first[2], g.first[3], g.nk_split, g.lda,
                        (const GemmMembers &)g);
     RWKV_LAUNCH_CHECK();
     return RWKV_OK;
@@ -2298,24 +2299,23 @@ int launch_splitk_epilogue(int ks, int64_t T, int64_t M, void *Y, int64_t ldy, c
 template <bool W_U8>
 int launch_tile(int tile, GemmGroup &g, int n, int64_t T, int64_t N, int ks, hipStream_t st) {
     switch (tile) {
-        case TILE_256x256: return launch_dma<W_U8, 256, 256, 8, 0>(g, n, T, N, ks, st);
-        case TILE_S: return launch_dma<W_U8, 128, 128, 8, 0>(g, n, T, N, ks, st);
-        case TILE_S4: return launch_dma<W_U8, 128, 128, 8, 4>(g, n, T, N, ks, st);
-        case TILE_N: return launch_dma<W_U8, 64, 128, 4, 4>(g, n, T, N, ks, st);
+        case TILE_256x256: return launch_dma<W_U8, 256, 256, 0>(g, n, T, N, ks, st);
+        case TILE_S: return launch_dma<W_U8, 128, 128, 0>(g, n, T, N, ks, st);
+        case TILE_S4: return launch_dma<W_U8, 128, 128, 4>(g, n, T, N, ks, st);
         case TILE_K8: return launch_kg<W_U8, 64, 64>(g, n, T, N, ks, st);
         case TILE_K4: return launch_kg<W_U8, 64, 128>(g, n, T, N, ks, st);
-        case TILE_256x192: return launch_dma<W_U8, 256, 192, 8, 0>(g, n, T, N, ks, st);
-        case TILE_224x256: return launch_dma<W_U8, 224, 256, 8, 0>(g, n, T, N, ks, st);
-        case TILE_224x192: return launch_dma<W_U8, 224, 192, 8, 0>(g, n, T, N, ks, st);
-        case TILE_192x256: return launch_dma<W_U8, 192, 256, 8, 0>(g, n, T, N, ks, st);
-        case TILE_192x192: return launch_dma<W_U8, 192, 192, 8, 0>(g, n, T, N, ks, st);
-        case TILE_160x256: return launch_dma<W_U8, 160, 256, 8, 0>(g, n, T, N, ks, st);
-        case TILE_160x192: return launch_dma<W_U8, 160, 192, 8, 0>(g, n, T, N, ks, st);
-        case TILE_128x256: return launch_dma<W_U8, 128, 256, 8, 0>(g, n, T, N, ks, st);
-        case TILE_128x192: return launch_dma<W_U8, 128, 192, 8, 0>(g, n, T, N, ks, st);
-        case TILE_96x128: return launch_dma<W_U8, 96, 128, 8, 4>(g, n, T, N, ks, st);
-        case TILE_128x96: return launch_dma<W_U8, 128, 96, 8, 4>(g, n, T, N, ks, st);
-        case TILE_96x96: return launch_dma<W_U8, 96, 96, 8, 4>(g, n, T, N, ks, st);
+        case TILE_256x192: return launch_dma<W_U8, 256, 192, 0>(g, n, T, N, ks, st);
+        case TILE_224x256: return launch_dma<W_U8, 224, 256, 0>(g, n, T, N, ks, st);
+        case TILE_224x192: return launch_dma<W_U8, 224, 192, 0>(g, n, T, N, ks, st);
+        case TILE_192x256: return launch_dma<W_U8, 192, 256, 0>(g, n, T, N, ks, st);
+        case TILE_192x192: return launch_dma<W_U8, 192, 192, 0>(g, n, T, N, ks, st);
+        case TILE_160x256: return launch_dma<W_U8, 160, 256, 0>(g, n, T, N, ks, st);
+        case TILE_160x192: return launch_dma<W_U8, 160, 192, 0>(g, n, T, N, ks, st);
+        case TILE_128x256: return launch_dma<W_U8, 128, 256, 0>(g, n, T, N, ks, st);
+        case TILE_128x192: return launch_dma<W_U8, 128, 192, 0>(g, n, T, N, ks, st);
+        case TILE_96x128: return launch_dma<W_U8, 96, 128, 4>(g, n, T, N, ks, st);
+        case TILE_128x96: return launch_dma<W_U8, 128, 96, 4>(g, n, T, N, ks, st);
+        case TILE_96x96: return launch_dma<W_U8, 96, 96, 4>(g, n, T, N, ks, st);
         case TILE_32x16: return launch_few<W_U8, 32, 16>(g, n, T, N, ks, st);
         case TILE_32x32: return launch_few<W_U8, 32, 32>(g, n, T, N, ks, st);
         case TILE_32x48: return launch_few<W_U8, 32, 48>(g, n, T, N, ks, st);
@@ -2358,7 +2358,8 @@ int launch_pick(int cfg, int ks, int64_t T, int64_t N, int64_t M, const rwkv_hal
 }
 
 // Tile choice (RWKV_GEMM_CFG overrides it for tuning sweeps: 3 and 9 the register-staged tiles by their number here, 14 and 15 the
-// direct-to-LDS 256 x 256 and 128 x 128 ones, 18 to 48 the others, CFG_DMA + TILE_*, with the K split of least cost).
+// direct-to-LDS 256 x 256 and 128 x 128 ones, 18 TILE_S4, 20 to 48 the others in the order of tile_choice.h, with the K split of least
+// cost).
 //   CFG_DMA +  operands laid out for 16-byte loads: the direct-to-LDS kernel with the tile and K split that the cost
 //              model puts first (128 x 128 tiles at full depth when another product runs beside this one: a 256 x 256
 //              tile's LDS leaves no room beside it on the CU, two small ones fit)
@@ -2380,8 +2381,8 @@ int pick_cfg(int64_t T, int64_t N, int64_t M, bool w_u8, const GemmEpi &ep, bool
     const char *e = getenv("RWKV_GEMM_CFG");
     if (e && *e) {
         const int cfg = atoi(e);
-        return cfg == 14 ? with_split(TILE_256x256) : cfg == 15 ? with_split(TILE_S)
-             : cfg >= CFG_DMA + TILE_S4 && cfg < CFG_DMA + TILES ? with_split(cfg - CFG_DMA) : cfg < CFG_DMA ? cfg : -1;
+        return cfg == 14 ? with_split(TILE_256x256) : cfg == 15 ? with_split(TILE_S) : cfg == 18 ? with_split(TILE_S4)
+             : cfg >= 20 && cfg < 20 + TILES - TILE_K8 ? with_split(cfg - 20 + TILE_K8) : cfg < CFG_DMA ? cfg : -1;
     }
     if (dma && !alone) return with_split(TILE_S);
     if (dma) return take(Launch(T, (int)(N / BK), 1, &M, ws).best(w_u8));

@@ -6,15 +6,15 @@
 namespace {
 
 // The direct-to-LDS tiles: rows and columns.  TILE_S is 128 x 128 with three stages (two workgroups fit a CU), TILE_S4 with four
-// and K over two groups, TILE_N 64 x 128 with four waves, TILE_K8 and TILE_K4 gemm_kg_kernel with eight and four groups.
+// and K over two groups, TILE_K8 and TILE_K4 gemm_kg_kernel with eight and four groups.
 enum {
-    TILE_256x256, TILE_S, TILE_S4, TILE_N, TILE_K8, TILE_K4, TILE_256x192, TILE_224x256, TILE_224x192, TILE_192x256, TILE_192x192,
+    TILE_256x256, TILE_S, TILE_S4, TILE_K8, TILE_K4, TILE_256x192, TILE_224x256, TILE_224x192, TILE_192x256, TILE_192x192,
     TILE_160x256, TILE_160x192, TILE_128x256, TILE_128x192,
     TILE_32x16, TILE_32x32, TILE_32x48, TILE_32x64, TILE_32x96, TILE_48x16, TILE_48x32, TILE_48x48, TILE_48x64, TILE_48x96, TILE_64x16, TILE_64x32, TILE_64x48, TILE_64x64, TILE_64x96,
     TILE_96x128, TILE_128x96, TILE_96x96, TILES
 };
 struct TileDim { int tm, tn; };
-constexpr TileDim tile_dim[TILES] = {{256, 256}, {128, 128}, {128, 128}, {64, 128}, {64, 64}, {64, 128}, {256, 192}, {224, 256}, {224, 192},
+constexpr TileDim tile_dim[TILES] = {{256, 256}, {128, 128}, {128, 128}, {64, 64}, {64, 128}, {256, 192}, {224, 256}, {224, 192},
                                      {192, 256}, {192, 192}, {160, 256}, {160, 192}, {128, 256}, {128, 192},
                                      {32, 16}, {32, 32}, {32, 48}, {32, 64}, {32, 96}, {48, 16}, {48, 32}, {48, 48}, {48, 64}, {48, 96}, {64, 16}, {64, 32}, {64, 48}, {64, 64}, {64, 96},
                                      {96, 128}, {128, 96}, {96, 96}};
@@ -27,7 +27,7 @@ constexpr TileDim tile_dim[TILES] = {{256, 256}, {128, 128}, {128, 128}, {64, 12
 // One fit per tile and type, over launches within 1.6 times the best one of 648 products each (24 lengths from 17 to 2048 rows, 27 widths
 // from 64 to 20480; weights from HBM; the chip under load before): the tile and split it picks takes 1 % (uint8) and 2 %
 // (fp16) longer than the best of all on average, with products that the host launches no faster counted in.  A tile per round costs
-// between 3 and 15 us whatever K is, so tiles of many sizes pay: each of these is the best one somewhere, the large ones with sides of
+// between 3 and 15 us whatever K is, so tiles of many sizes pay: each of these is the choice somewhere (64 x 16 with fp16 weights alone), the large ones with sides of
 // 160, 192 and 224 where 256 x 256 or 128 x 128 leave CUs idle or rows empty, those of 32, 48 and 64 rows in calls of up to 128 rows, those with a side of
 // 96 where a round of 128 x 128 leaves CUs idle (fitted apart, at full depth, 97 rows and more).
 // us, uint8 / fp16 weights: [1024 x 4096] x [4096 x 12288] three rounds of 128 x 128 115.7 / 132.5, one of 256 x 192 90 / 97; [777 x
@@ -49,7 +49,6 @@ constexpr TilePrice tile_price[2][TILES] = {
         {4.549f, 9.813f, 10.035f, 0.941f, 1.721f, 0.081f, 3.477f, 0.f},   // 256x256
         {2.456f, 3.248f, 4.838f, 0.423f, 0.631f, 0.f, 4.568f, 0.076f},   // S
         {1.871f, 4.556f, 4.704f, 0.298f, 0.575f, 0.f, 7.450f, 0.136f},   // S4
-        {2.546f, 2.311f, 1.782f, 0.363f, 0.699f, 0.f, 8.143f, 0.073f},   // N
         {1.987f, 2.281f, 4.023f, 0.141f, 0.253f, 0.f, 4.754f, 0.175f},   // K8
         {1.808f, 3.209f, 4.405f, 0.217f, 0.391f, 0.f, 7.476f, 0.162f},   // K4
         {4.715f, 8.832f, 6.523f, 0.825f, 1.348f, 0.067f, 4.078f, 0.019f},   // 256x192
@@ -83,7 +82,6 @@ constexpr TilePrice tile_price[2][TILES] = {
         {5.336f, 9.067f, 8.377f, 0.949f, 1.642f, 0.022f, 3.336f, 0.f},   // 256x256
         {6.522f, 0.f, 0.599f, 0.349f, 0.546f, 0.f, 4.631f, 0.085f},   // S
         {3.456f, 3.989f, 3.830f, 0.317f, 0.523f, 0.041f, 5.040f, 0.081f},   // S4
-        {5.441f, 0.f, 0.f, 0.346f, 0.468f, 0.f, 6.072f, 0.143f},   // N
         {1.922f, 3.185f, 4.514f, 0.115f, 0.176f, 0.013f, 6.113f, 0.121f},   // K8
         {1.799f, 3.765f, 4.212f, 0.200f, 0.305f, 0.021f, 7.262f, 0.149f},   // K4
         {5.813f, 9.209f, 4.665f, 0.786f, 1.222f, 0.067f, 4.361f, 0.f},   // 256x192
@@ -135,7 +133,7 @@ constexpr Prices prices[2] = {by_field(tile_price[0]), by_field(tile_price[1])};
 inline bool tile_offered(int tile, int64_t T, float tiles) {
     if (tile >= TILE_96x128) return T > 96 || (T > 64 && tiles >= 192.f && tiles <= 256.f);
     if (tile >= TILE_32x16) return T <= (tile_dim[tile].tn <= 32 ? 128 : 256);
-    return tile != TILE_N || T <= 64;
+    return true;
 }
 
 struct TilePick { int tile, ks; float us; };

@@ -42,6 +42,15 @@ static Out out(const TilePick &p) { return {p.tile, p.ks, tile_dim[p.tile].tm, t
 extern "C" Out pick(int u8, int64_t T, int nk, int n, const int64_t *M, uint64_t ws) { return out(Launch(T, nk, n, M, ws).best(u8)); }
 extern "C" Out slow_pick(int u8, int64_t T, int nk, int n, const int64_t *M, uint64_t ws) { return out(one_by_one(u8, T, nk, n, M, ws)); }
 extern "C" Out with(int u8, int tile, int64_t T, int nk, int64_t M, uint64_t ws) { return out(Launch(T, nk, 1, &M, ws).with(u8, tile)); }
+// how often each tile is chosen, over single launches of 17 to 2048 rows with and without scratch
+extern "C" int chosen(int u8, int *count) {
+    for (int t = 0; t < TILES; ++t) count[t] = 0;
+    for (int64_t T = 17; T <= 2048; T += T < 128 ? 1 : T < 600 ? 31 : 181)
+        for (int nk = 1; nk <= 320; nk += nk < 16 ? 1 : 5)
+            for (int64_t M = 64; M <= 24576; M += M < 4096 ? 40 : 672)
+                for (uint64_t ws = 0; ws <= 64u << 20; ws += 64 << 20) ++count[Launch(T, nk, 1, &M, ws).best(u8).tile];
+    return TILES;
+}
 // ns a choice, over launches of many sizes
 extern "C" double time_choice(int slow, int reps) {
     volatile int sink = 0;
@@ -130,3 +139,12 @@ def test_tiles_of_96_rows_in_calls_of_65_to_96(choice, u8, N, M):
         for few in ([M[0] // 2], [12288], [16384], [4096] * 3, [50304], [65536]):
             p = _pick(choice, u8, T, N // 64, few)
             assert p.tm != 96 and (p.tm, p.tn) != (128, 96), (T, few, p.key())
+
+
+@pytest.mark.parametrize("u8", [1, 0])
+def test_every_tile_is_chosen_somewhere(choice, u8):
+    """No kernel is built for nothing, but the uint8 64 x 16 tile."""
+    count = (ctypes.c_int * 64)()
+    n = choice.chosen(u8, count)
+    never = [(d.tm, d.tn) for d in (choice.with_(u8, t, 1024, 64, 4096, WS) for t in range(n)) if not count[d.tile]]
+    assert never == ([(64, 16)] if u8 else [])
