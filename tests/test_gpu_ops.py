@@ -327,6 +327,31 @@ def test_forced_tile_configurations(N, M, B, monkeypatch):
             call()
 
 
+# configurations that add the products of a row in one order at full depth
+SAME_ORDER = [(3, 9), (14, 15, *range(22, 31)), (18, 46, 47, 48), (31, 33, 36, 38, 41, 43), (32, 34, 35, 37, 39, 40, 42, 44, 45)]
+
+
+@pytest.mark.parametrize("order", SAME_ORDER, ids=lambda o: str(o[0]))
+@pytest.mark.parametrize("N,M,B", [(960, 1088, 90), (448, 1003, 129)])
+def test_configurations_that_agree_bit_for_bit(N, M, B, order, monkeypatch):
+    """Rows do not depend on the tile's sides, on sums that round: neither with uint8 nor with fp16 weights, nor where outputs leave
+    four at a time (1003 of them, fp32).  960 inputs are too few for a K split."""
+    ops = _ops()
+    x = torch.from_numpy(_rng(N).standard_normal((B, N)).astype(np.float16)).to(DEV)
+    w = torch.from_numpy((_rng(M).standard_normal((M, N)) * 0.02).astype(np.float32)).to(DEV)
+    q, h = ops.quantize_u8(w.t(), scale_dtype=torch.float16, input_contiguous=True), w.half().t()
+    calls = [lambda: ops.mm8(x, *q)]
+    if order != (3, 9):   # 9 is uint8 alone
+        calls += [lambda: ops.matmul_float(x, h), lambda: ops.matmul_float(x, h, output_dtype=torch.float32)]
+    for call in calls:
+        want = None
+        for cfg in order:
+            monkeypatch.setenv("RWKV_GEMM_CFG", str(cfg))
+            y = call()
+            assert want is None or torch.equal(y, want), cfg
+            want = y
+
+
 @pytest.mark.parametrize("cfg", ["", "14", "15", "20", "21"])
 @pytest.mark.parametrize("N,M,B", [(1088, 1000, 2176), (8192, 200, 520), (8192, 516, 600)])
 def test_tiles_that_walk_along_the_outputs(N, M, B, cfg, monkeypatch):
