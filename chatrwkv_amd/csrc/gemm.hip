@@ -1441,7 +1441,7 @@ int launch_kg(GemmGroup &g, int n, int64_t T, int64_t N, int ks, hipStream_t st)
 }
 
 // ---- few rows: tiles of 32, 48 or 64 rows and 16 to 96 columns ----------------------------------------------------
-// Calls of 17 to 64 rows are bound by how fast a CU takes its operands, 50 GB/s with a tile's activations at twice the bytes of its
+// For calls of up to 128 rows (tiles of 16 and 32 columns) and 256.  Those of 17 to 64 rows are bound by how fast a CU takes its operands, 50 GB/s with a tile's activations at twice the bytes of its
 // uint8 weights, so what counts is that every CU has the same share and no rows past the end: 12288 outputs are 192 tiles of 64 x 64
 // and 256 of 48 x 48.  The form is that of gemm_kg_kernel (the waves share K, partial blocks meet in LDS and are added in group order)
 // with v_mfma_f32_16x16x32_f16, whose blocks make sides of any multiple of 16: KG = 8 groups of one wave, or four of two waves side by

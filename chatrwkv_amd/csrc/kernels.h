@@ -33,7 +33,8 @@ DEV void at_once(const void *const (&p)[N]) {
 }
 DEV h16x8 load8(const void *p, int i) { return ((const h16x8 *)p)[i]; }
 
-// n / d as a multiplication with a factor from the host, exact for n (d - 1) < 2^40: the factor is at most d too large in 2^40.
+// n / d as a multiplication with a factor from the host, exact for n (d - 1) < 2^40, the factor being at most d too large in 2^40, and n < 2^24 d,
+// past which the product with it leaves 64 bits.
 // (A 64-bit division is 120 instructions, and stood ahead of the first load of the kernels that have one of these.)
 inline uint64_t div_factor(int64_t d) { return ((uint64_t)1 << 40) / (uint64_t)d + 1; }
 DEV int div_by(uint32_t n, uint64_t factor) { return (int)(((uint64_t)n * factor) >> 40); }

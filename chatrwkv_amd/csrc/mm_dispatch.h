@@ -86,7 +86,7 @@ inline bool handover_enabled() {
 // products -- as two calls, so that the caller can join a side stream in between.  c1 launches the first product,
 // c2 the second (its xs / s0 / s2 scratch is used).  uint8 matrices, both products through the direct-to-LDS kernel
 // and the first at full depth: the first epilogue stores mid already scaled by W2's ry into c2.xs and one partial
-// row sum per column tile into `parts` (2 * T * ceil(M1 / 64) floats), which the second launch adds up itself -- no
+// row sum per column tile into `parts` (up to 2 * T * emitted_parts(M1, EMIT_MIN_TN) floats), which the second launch adds up itself -- no
 // scaling pass, and the unscaled mid is never stored; *np is then the number of partial sums per row.  Otherwise
 // (*np = 0): mm_scaled, then mm.  mm_pair_parts: that number for a first product of plan p1, which may be a grouped launch.
 inline int mm_pair_parts(const GemmPlan &p1, const Ctx &c2, const rwkv_mat &m1, const rwkv_mat &m2, bool mat_u8, int act2,
