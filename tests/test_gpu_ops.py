@@ -309,6 +309,42 @@ def test_tile_that_the_cost_model_puts_first(u8, N, M, B, monkeypatch):
     assert times[""] <= 1.1 * min(times.values()), times
 
 
+@pytest.mark.parametrize("u8,N,M,B", [(True, 16384, 4096, 45), (True, 4096, 20480, 80), (True, 4096, 16384, 160), (True, 4096, 12288, 333),
+                                      (False, 4096, 20480, 80), (False, 16384, 4096, 160), (False, 4096, 8192, 300)])
+def test_choice_among_all_tiles(u8, N, M, B, monkeypatch):
+    """Within 1.15 of the best of all tiles, each with its K split of least price, in a chain of products with weights of their own (from
+    memory, not from a cache): the prices' error there is 1 to 3 % on average and under 10 % for these."""
+    ops = _ops()
+    x = torch.randn(B, N, device=DEV).half()
+    copies = 10
+    if u8:
+        ws = [torch.randint(0, 256, (M, N), dtype=torch.uint8, device=DEV).t() for _ in range(copies)]
+        v = [torch.rand(n, device=DEV).half() for n in ((M,), (M,), (N, 1), (N, 1))]
+        call = lambda w: ops.mm8(x, w, *v)
+    else:
+        ws = [torch.randn(M, N, device=DEV).half().t() for _ in range(copies)]
+        call = lambda w: ops.matmul_float(x, w)
+
+    def best(cfg):
+        monkeypatch.setenv("RWKV_GEMM_CFG", cfg)
+        ms = []
+        for _ in range(6):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            for _ in range(3):
+                for w in ws:
+                    call(w)
+            b.record()
+            torch.cuda.synchronize()
+            ms.append(a.elapsed_time(b))
+        return min(ms)
+
+    cfgs = ["", "14", "15", "18"] + [str(c) for c in range(20, 49)]
+    times = {cfg: best(cfg) for cfg in cfgs}
+    print(f"chosen {times['']:.3f}, best {min(times, key=times.get)} {min(times.values()):.3f}")
+    assert times[""] <= 1.15 * min(times.values()), times
+
+
 @pytest.mark.parametrize("N,M,B", [(4096, 4096, 100), (768, 3072, 513)])
 def test_forced_tile_configurations(N, M, B, monkeypatch):
     """RWKV_GEMM_CFG (tuning): each tile configuration of the uint8 product, with sums that are exact, gives the bits of the
