@@ -452,7 +452,7 @@ __global__ __launch_bounds__(64 * WT * WM) void gemm_kernel(int T, int N, int M,
 // registers, so no wave spends issue slots on ds_write or on holding prefetched tiles.  A uint8 weight tile stays
 // uint8 in LDS (half the bytes of fp16) and becomes fp16 in the fragments on the way to the matrix cores.
 // The MFMA is v_mfma_f32_16x16x32_f16.  A chip full of large tiles is bound by its clock under load, and this one does more for
-// the power: loops of nothing but MFMAs on random operands sustain 1870 TFLOP/s with it and 1600 with v_mfma_f32_32x32x16_f16
+// the power: loops of nothing but MFMAs on random operands sustain 1810 to 1870 TFLOP/s with it and 1600 to 1620 with v_mfma_f32_32x32x16_f16
 // (whose accumulator it reads and writes half as often per product).  [1024 x 4096] x [4096 x 16384] 126 -> 115 us (uint8), 133 ->
 // 119 (fp16).  It also makes sides that are any multiple of 32, see tile_price.
 // LDS layout of a stage: 128-byte rows [row][8 chunks of 16 B], chunk c of row r at slot c ^ ((r >> 1) & 7); uint8 weight rows

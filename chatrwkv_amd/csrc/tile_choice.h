@@ -24,6 +24,7 @@ constexpr TileDim tile_dim[TILES] = {{256, 256}, {128, 128}, {128, 128}, {64, 64
 //          + k-tiles * (step_1 for every full round, between step_0 and step_1 for the last one by the CUs busy,
 //                       extra for what exceeds one round)
 //          + with a split, slab per 16 MB of fp32 slabs written and read, split per slab, and SECOND_LAUNCH.
+// No term is below 0, and they make up for each other: one by itself, several being 0, is no cost of the hardware.
 // One fit per tile and type, over launches within 1.6 times the best one of 648 products each (24 lengths from 17 to 2048 rows, 27 widths
 // from 64 to 20480; weights from HBM; the chip under load before): the tile and split it picks takes 1 % (uint8) and 2 %
 // (fp16) longer than the best of all on average, with products that the host launches no faster counted in.  A tile per round costs
